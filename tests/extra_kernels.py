@@ -1314,3 +1314,62 @@ def scale_rows_on_a_2d_grid(x_ptr, w_ptr, y_ptr, n_rows, n_cols, BLOCK: tl.const
     w = tl.load(w_ptr + c, mask=m, other=0.0).to(tl.float32)
     x = tl.load(x_ptr + (b * n_rows + r) * n_cols + c, mask=m, other=0.0).to(tl.float32)
     tl.store(y_ptr + (b * n_rows + r) * n_cols + c, (x * w + (b - r)).to(y_ptr.dtype.element_ty), mask=m)
+
+
+@triton.jit
+def attention_biased(Q, K, V, B, O, LSE, sm_scale, seq_q, seq_k, stride_h, stride_s, stride_kh, stride_kd, stride_kn, BM: tl.constexpr, BN: tl.constexpr, D: tl.constexpr,
+                     CAUSAL: tl.constexpr):
+    # attention with a bias per key, keys in either layout (the transposed block is loaded as it is when stride_kn == 1), an
+    # optional causal mask, and the log-sum-exp of every row in fp32 beside the 16-bit result
+    pm = tl.program_id(0)
+    ph = tl.program_id(1)
+    rm = pm * BM + tl.arange(0, BM)
+    rd = tl.arange(0, D)
+    q = tl.load(Q + ph * stride_h + rm[:, None] * stride_s + rd[None, :], mask=rm[:, None] < seq_q, other=0.0)
+    m_i = tl.zeros([BM], dtype=tl.float32) - float("inf")
+    l_i = tl.zeros([BM], dtype=tl.float32)
+    acc = tl.zeros([BM, D], dtype=tl.float32)
+    last = seq_k
+    if CAUSAL:
+        last = tl.minimum(seq_k, (pm + 1) * BM)
+    for start in range(0, last, BN):
+        rn = start + tl.arange(0, BN)
+        kt = tl.load(K + ph * stride_kh + rd[:, None] * stride_kd + rn[None, :] * stride_kn, mask=rn[None, :] < seq_k, other=0.0)
+        v = tl.load(V + ph * stride_h + rn[:, None] * stride_s + rd[None, :], mask=rn[:, None] < seq_k, other=0.0)
+        b = tl.load(B + rn, mask=rn < seq_k, other=0.0)
+        qk = tl.dot(q, kt) * sm_scale + b[None, :]
+        ok = rn[None, :] < seq_k
+        if CAUSAL:
+            ok = ok & (rm[:, None] >= rn[None, :])
+        qk = tl.where(ok, qk, -float("inf"))
+        m_new = tl.maximum(m_i, tl.max(qk, axis=1))
+        p = tl.exp(qk - m_new[:, None])
+        alpha = tl.exp(m_i - m_new)
+        l_i = l_i * alpha + tl.sum(p, axis=1)
+        acc = acc * alpha[:, None]
+        acc = tl.dot(p.to(V.dtype.element_ty), v, acc)
+        m_i = m_new
+    acc = acc / l_i[:, None]
+    tl.store(O + ph * stride_h + rm[:, None] * stride_s + rd[None, :], acc.to(O.dtype.element_ty), mask=rm[:, None] < seq_q)
+    tl.store(LSE + ph * seq_q + rm, m_i + tl.log(l_i), mask=rm < seq_q)
+
+
+@triton.jit
+def chained_products(a_ptr, b_ptr, c_ptr, r_ptr, out_ptr, n_rows, k_cols, pitch_b, pitch_c, BM: tl.constexpr, K: tl.constexpr, N: tl.constexpr, P: tl.constexpr, TURNED: tl.constexpr):
+    # out = relu(a @ b + r) @ c^T for a block of rows: the first product's result is the second one's left operand; b and c are
+    # read as they lie or through a transpose, r is added element by element
+    i = tl.program_id(0) * BM + tl.arange(0, BM)
+    k = tl.arange(0, K)
+    n = tl.arange(0, N)
+    p = tl.arange(0, P)
+    a = tl.load(a_ptr + i[:, None] * K + k[None, :], mask=(i[:, None] < n_rows) & (k[None, :] < k_cols), other=0.0)
+    if TURNED:
+        b = tl.trans(tl.load(b_ptr + n[:, None] * pitch_b + k[None, :], mask=k[None, :] < k_cols, other=0.0))
+        c = tl.load(c_ptr + n[:, None] * pitch_c + p[None, :])
+    else:
+        b = tl.load(b_ptr + k[:, None] * pitch_b + n[None, :], mask=k[:, None] < k_cols, other=0.0)
+        c = tl.trans(tl.load(c_ptr + p[:, None] * pitch_c + n[None, :]))
+    r = tl.load(r_ptr + i[:, None] * N + n[None, :], mask=i[:, None] < n_rows, other=0.0).to(tl.float32)
+    h = tl.maximum(tl.dot(a, b) + r, 0.0)
+    out = tl.dot(h.to(a_ptr.dtype.element_ty), c)
+    tl.store(out_ptr + i[:, None] * P + p[None, :], out, mask=i[:, None] < n_rows)

@@ -721,6 +721,56 @@ def test_flash_attention_forward(H, seq, D, BM, BN):
     assert torch.equal(o[H], torch.full((seq, D), 3.0, device=DEV, dtype=torch.float16))
 
 
+@pytest.mark.parametrize("dtype,D,BM,BN,seq,pad,causal,k_columns", [
+    (torch.float16, 64, 128, 64, 1, 0, False, False), (torch.float16, 64, 64, 32, 33, 0, True, False), (torch.bfloat16, 128, 64, 64, 64, 0, True, False),
+    (torch.float16, 128, 32, 64, 65, 8, False, True), (torch.bfloat16, 32, 128, 64, 127, 0, True, True), (torch.float16, 64, 128, 64, 300, 1, True, False),
+    (torch.float16, 64, 64, 64, 257, 3, False, True), (torch.bfloat16, 64, 32, 32, 1000, 0, True, False), (torch.float16, 256, 64, 32, 130, 0, False, False)])
+def test_matrix_program_attention(dtype, D, BM, BN, seq, pad, causal, k_columns):
+    # the matrix layout of the generic family: row counts around the edges of its tiles (32 rows per wavefront, up to four
+    # programs per workgroup), pitches that are not 16-byte aligned (blocks staged through registers), keys in either layout,
+    # masks that cut through blocks, a per-key bias (a vector along the columns) and an fp32 row result
+    import extra_kernels as X
+    torch.manual_seed(seq + D)
+    H = 3
+    q, k, v = (torch.randn(H, seq, D + pad, device=DEV).to(dtype) for _ in range(3))
+    b = torch.randn(seq, device=DEV)
+    o = torch.full((H + 1, seq, D + pad), 3.0, device=DEV, dtype=dtype)
+    lse = torch.full((H + 1, seq), 5.0, device=DEV)
+    kk = k.transpose(1, 2).contiguous() if k_columns else k
+    s_kd, s_kn = (kk.stride(1), 1) if k_columns else (1, kk.stride(1))
+    kern = X.attention_biased[(triton.cdiv(seq, BM), H)](q, kk, v, b, o, lse, D ** -0.5, seq, seq, seq * (D + pad), D + pad, kk.stride(0), s_kd, s_kn, BM=BM, BN=BN, D=D, CAUSAL=causal)
+    torch.cuda.synchronize()
+    assert kern.function.family == "tile_program" and kern.function.last_kernel == "tile_program (hipRTC, matrix layout)"
+    s = torch.matmul(q[:, :, :D].cpu().double(), k[:, :, :D].cpu().double().transpose(1, 2)) * D ** -0.5 + b.cpu().double()
+    if causal:
+        s.masked_fill_(torch.triu(torch.ones(seq, seq, dtype=torch.bool), 1), -float("inf"))
+    want = torch.matmul(torch.softmax(s, -1), v[:, :, :D].cpu().double())
+    # probabilities and results are each rounded once to 16 bits: half an ulp of |v| and of |o| <= max |v|
+    ulp = 2.0 ** -10 if dtype == torch.float16 else 2.0 ** -7
+    assert (o[:H, :, :D].cpu().double() - want).abs().max().item() <= ulp * v.abs().max().item()
+    # fp32: a dot product of D terms, exponentials and a sum of seq terms
+    assert (lse[:H].cpu().double() - torch.logsumexp(s, -1)).abs().max().item() <= 2e-5
+    assert (lse[H] == 5.0).all() and (o[H] == 3.0).all() and (o[:, :, D:] == 3.0).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rows,BM,K,N,P,k_cols,turned", [(1, 32, 32, 32, 32, 32, False), (100, 64, 64, 128, 32, 50, True), (129, 128, 128, 64, 64, 128, False), (70, 32, 256, 32, 128, 200, True)])
+def test_matrix_program_chained_products(dtype, rows, BM, K, N, P, k_cols, turned):
+    # operands of -1 / 0 / 1 keep the first product exact in 16 bits (|sum| <= 256), so the chain's result is exact in fp32
+    import extra_kernels as X
+    g = torch.Generator().manual_seed(rows)
+    ints = lambda *shape: torch.randint(-1, 2, shape, generator=g).to(dtype)
+    a, b, c, r = ints(rows, K), ints(K, N + 8), ints(P, N + 1), ints(rows, N)
+    bb = torch.nn.functional.pad(b[:, :N].t().contiguous(), (0, 8)) if turned else b
+    cc = c[:, :N].t().contiguous() if turned else c
+    out = torch.full((rows + 1, P), 7.0, device=DEV)
+    kern = X.chained_products[(triton.cdiv(rows, BM),)](a.to(DEV), bb.to(DEV), cc.to(DEV), r.to(DEV), out, rows, k_cols, bb.stride(0), cc.stride(0), BM=BM, K=K, N=N, P=P, TURNED=turned)
+    torch.cuda.synchronize()
+    assert kern.function.family == "tile_program" and kern.function.last_kernel == "tile_program (hipRTC, matrix layout)"
+    h = torch.relu(a[:, :k_cols].double() @ b[:k_cols, :N].double() + r.double())
+    assert torch.equal(out[:rows].cpu().double(), h @ c[:, :N].double().t()) and (out[rows] == 7.0).all()
+
+
 def test_softmax_rows_the_row_kernel_declines(K, oracle_cpu):
     import extra_kernels as X
     torch.manual_seed(5)

@@ -982,7 +982,8 @@ bool try_fused_map(Plan &pl) {
 bool try_tile_program(Plan &pl) {
   Matcher m(pl.prog);
   if (m.accesses.empty()) return false;
-  pl.source = tile_program_source(pl.prog);  // throws Unsupported with the reason
+  pl.source = matrix_program_source(pl.prog);
+  if (pl.source.empty()) pl.source = tile_program_source(pl.prog);  // throws Unsupported with the reason
   pl.family = Family::TileProgram;
   return true;
 }

@@ -757,6 +757,16 @@ tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, con
         persistent = tile_program_is_persistent(source) && !(slot == &plan->fused && plan->fused_is_plain);
       }
       kname = "tile_program (hipRTC)";
+      int per_group = 1, group_axis = -1, group_threads = 256;
+      if (tile_program_is_matrix(source, &per_group, &group_axis, &group_threads)) {  // a one-dimensional launch that numbers the programs itself
+        kname = "tile_program (hipRTC, matrix layout)";
+        int64_t e[3] = {gx, gy, gz};
+        int64_t &shared = e[group_axis < 0 ? 0 : group_axis];
+        shared = (shared + per_group - 1) / per_group;
+        a.lgx = gx; a.lgy = gy; a.lgz = gz;
+        err = rtc_launch(*slot, (int)(e[0] * e[1] * e[2]), 1, 1, group_threads, &a, sizeof a, s);
+        return TTS_OK;
+      }
       // the program asks for neighbouring workgroups along program_id(1) (tile_codegen.cpp); grid.y holds 65535 at most
       a.swap_xy = tile_program_swaps_grid(source) && gy > 1 && gx <= 65535 ? 1 : 0;
       if (persistent) {

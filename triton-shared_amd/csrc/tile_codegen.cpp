@@ -2156,6 +2156,8 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
 )SRC";
 
+#include "tile_mma.h"
+
 }  // namespace
 
 namespace {
@@ -2165,6 +2167,7 @@ namespace {
 // the line below, and the launcher swaps the grid's x and y (x + bias[None, :] on [32, 256] tiles of an 8192 x 8192 matrix,
 // row blocks on program_id(0): 119 us; with column blocks there: 100).
 const char *const SWAP_MARK = "// tts: swap_xy\n";
+const char *const MATRIX_MARK = "// tts: matrix ";  // followed by: programs per workgroup, the axis they lie on, threads per workgroup
 const char *const PERSISTENT_MARK = "// tts: persistent\n";  // the launcher starts a few workgroups per CU, which walk the programs
 bool stores_walk_columns_with_pid1(const Program &p) {
   int votes_for = 0, votes_against = 0;
@@ -2264,6 +2267,58 @@ std::string tile_program_source(const Program &p, bool allow_persistent) {
     if (g.all_store_bases.count(b))
       throw Unsupported("tile_program: an argument is both stored to and read by a load that is not of its body's block shape");
   return without_double_barriers(all.str());
+}
+
+std::string matrix_program_source(const Program &p) {
+  if ((int)p.arg_names.size() > TILE_MAX_ARGS) return std::string();
+  MmaGen g(p);
+  try {
+    g.collect_bases(p.body);
+    g.analyse();
+    g.emit_ops(p.body);
+  } catch (const Unsupported &) {
+    return std::string();
+  }
+  std::string pre = TILE_PRELUDE;
+  const std::string n = std::to_string(TILE_MAX_ARGS);
+  for (size_t pos = 0; (pos = pre.find("%N%", pos)) != std::string::npos;) pre.replace(pos, 3, n);
+  const std::string G = std::to_string(g.G), wpp = std::to_string(g.wpp), waves = std::to_string(g.G * g.wpp);
+  std::ostringstream all;
+  all << MATRIX_MARK << g.G << " " << g.axis << " " << MmaGen::WAVES * 64 << "\n" << pre << MMA_PRELUDE;
+  // two workgroups per CU (256 registers a lane) unless the blocks need more
+  all << "extern \"C\" __global__ __launch_bounds__(" << MmaGen::WAVES * 64 << ", " << (mma_registers(g) <= 208 ? 2 : 1)
+      << ") void tile_program(const Args p, const int swap_xy, const int lgx, const int lgy, const int lgz) {\n"
+      << "  __shared__ __attribute__((aligned(1024))) char lds[" << std::max<int64_t>(g.lds_bytes, 16) << "];\n"
+      << "  const unsigned lds0 = (unsigned)(unsigned long long)TTS_LDS(lds);\n"
+      << "  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), l32 = lane & 31, h4 = 4 * (lane >> 5), r16 = lane & 15;\n"
+      << "  const int wrow = (wave % " << wpp << ") * " << 32 * g.R << ";  // this wavefront's first row of its program's block\n"
+      << "  const long long npx = lgx, npy = lgy, npz = lgz;\n";
+  // Workgroup -> programs.  Workgroups are dealt round-robin to the eight XCDs: with the axis whose programs share their
+  // staged blocks as the slow one, and the others dealt so that equal ones meet on one XCD, what they stage comes from
+  // that XCD's L2.  Programs with longer loops at the end of that axis (a causal mask) go first.
+  const int ax = g.axis < 0 ? 0 : g.axis, b1 = ax == 0 ? 1 : 0, b2 = ax == 2 ? 1 : 2;
+  const std::string NP[3] = {"npx", "npy", "npz"}, PD[3] = {"pidx", "pidy", "pidz"};
+  all << "  const unsigned others = (unsigned)(" << NP[b1] << " * " << NP[b2] << "), groups = (unsigned)((" << NP[ax] << " + " << g.G - 1 << ") / " << g.G << ");\n"
+      << "  unsigned other, group;\n"
+      << "  if (others % 8 == 0) { const unsigned j = blockIdx.x / 8, per = others / 8; other = blockIdx.x % 8 + 8 * (j % per); group = j / per; }\n"
+      << "  else { other = blockIdx.x % others; group = blockIdx.x / others; }\n"
+      << "  const long long " << PD[b1] << " = other % (unsigned)" << NP[b1] << ", " << PD[b2] << " = other / (unsigned)" << NP[b1] << ";\n";
+  for (const SOp &s : p.body)
+    if (s.kind == SK::For && g.expr_uses_pid(s.ub, ax)) {
+      all << "  {\n    auto end = [&](long long " << PD[ax] << ") { (void)" << PD[ax] << "; return " << g.ex(s.ub) << "; };\n"
+          << "    if (end(" << NP[ax] << " - 1) > end(0)) group = groups - 1 - group;\n  }\n";
+      break;
+    }
+  all << "  const long long group0 = (long long)group * " << G << ", " << PD[ax] << " = group0 + wave / " << wpp << " % " << G << ";\n"
+      << "  const bool mine = wave < " << waves << " && " << PD[ax] << " < " << NP[ax] << ";  // whether this wavefront has rows\n"
+      << "  (void)pidx; (void)pidy; (void)pidz; (void)npx; (void)npy; (void)npz; (void)swap_xy; (void)lds0; (void)r16; (void)mine; (void)groups;\n"
+      << g.os.str() << "}\n";
+  return all.str();
+}
+
+bool tile_program_is_matrix(const std::string &source, int *programs, int *axis, int *threads) {
+  if (source.compare(0, strlen(MATRIX_MARK), MATRIX_MARK) != 0) return false;
+  return sscanf(source.c_str() + strlen(MATRIX_MARK), "%d %d %d", programs, axis, threads) == 3;
 }
 
 // What a matmul kernel does to its accumulator between the K loop and the store (an activation, a bias, a residual, the
