@@ -1373,3 +1373,25 @@ def chained_products(a_ptr, b_ptr, c_ptr, r_ptr, out_ptr, n_rows, k_cols, pitch_
     h = tl.maximum(tl.dot(a, b) + r, 0.0)
     out = tl.dot(h.to(a_ptr.dtype.element_ty), c)
     tl.store(out_ptr + i[:, None] * P + p[None, :], out, mask=i[:, None] < n_rows)
+
+
+@triton.jit
+def column_moments(x_ptr, s_ptr, out_ptr, n_rows, n_cols, pitch, BR: tl.constexpr, BC: tl.constexpr):
+    # out[0] = sum + 1, out[1] = sum of squares, out[2] = both combined, per column: a block of columns per program walked down
+    # the rows with a carried pointer, next to a scale per row; one accumulator starts at 1 / BR
+    c = tl.program_id(0) * BC + tl.arange(0, BC)
+    r = tl.arange(0, BR)
+    a = tl.zeros((BR, BC), dtype=tl.float32) + 1.0 / BR
+    b = tl.zeros((BR, BC), dtype=tl.float32)
+    px = x_ptr + r[:, None] * pitch + c[None, :]
+    for r0 in range(0, n_rows, BR):
+        x = tl.load(px, mask=(r[:, None] < n_rows - r0) & (c[None, :] < n_cols), other=0.0).to(tl.float32)
+        s = tl.load(s_ptr + r0 + r, mask=r < n_rows - r0, other=0.0)
+        a += x * s[:, None]
+        b += x * x
+        px += BR * pitch
+    sa = tl.sum(a, axis=0)
+    sb = tl.sum(b, axis=0)
+    tl.store(out_ptr + c, sa, mask=c < n_cols)
+    tl.store(out_ptr + n_cols + c, sb, mask=c < n_cols)
+    tl.store(out_ptr + 2 * n_cols + c, sa - 2.0 * sb, mask=c < n_cols)

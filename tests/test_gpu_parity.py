@@ -771,6 +771,32 @@ def test_matrix_program_chained_products(dtype, rows, BM, K, N, P, k_cols, turne
     assert torch.equal(out[:rows].cpu().double(), h @ c[:, :N].double().t()) and (out[rows] == 7.0).all()
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("rows,cols,pitch", [(1, 5, 5), (31, 128, 128), (65, 130, 136), (1000, 300, 301), (5000, 100, 104), (20000, 40, 40)])
+def test_loops_that_only_add_run_in_slices(dtype, rows, cols, pitch):
+    # few programs with long loops: the launcher deals a program's iterations to several workgroups whose sums meet at the end
+    # (one slice for the shortest loops); small integers keep every sum exact, launches repeat and run on two streams
+    import extra_kernels as X
+    g = torch.Generator().manual_seed(rows)
+    x = torch.randint(-3, 4, (rows, pitch), generator=g).to(dtype).to(DEV)
+    s = torch.randint(-2, 3, (rows,), generator=g).float().to(DEV)
+    xc = x[:, :cols].double()
+    a, b = (xc * s[:, None].double()).sum(0) + 1, (xc * xc).sum(0)
+    want = torch.stack([a, b, a - 2 * b])
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    outs = []
+    for i in range(6):
+        with torch.cuda.stream(streams[i % 2]):
+            out = torch.full((4, cols), 9.0, device=DEV)
+            k = X.column_moments[(triton.cdiv(cols, 64),)](x, s, out, rows, cols, pitch, BR=16, BC=64)
+            outs.append(out)
+    torch.cuda.synchronize()
+    assert k.function.family == "tile_program"
+    for out in outs:
+        assert torch.equal(out[:3].double(), want) and (out[3] == 9.0).all()
+
+
 def test_softmax_rows_the_row_kernel_declines(K, oracle_cpu):
     import extra_kernels as X
     torch.manual_seed(5)

@@ -47,6 +47,8 @@ bool tile_program_is_persistent(const std::string &source);  // the kernel walks
 // The same program in the form for programs built around 16-bit matrix products (tile_mma.h); empty if it is not one.
 std::string matrix_program_source(const Program &p);
 bool tile_program_is_matrix(const std::string &source, int *programs, int *axis, int *threads);  // programs per workgroup along which axis (-1: x), threads
+// The program's loop may be dealt to several workgroups per program: the floats of partial sums each needs, the loop's id.
+bool tile_program_is_sliced(const std::string &source, int *floats, int *loop);
 bool tile_program_swaps_grid(const std::string &source);  // the launcher exchanges the grid's x and y for this source (when y fits)
 // Matmul family with ops between the K loop and the store: the source of the functor that applies them to one
 // accumulator value (tile_codegen.cpp), compiled at run time together with the kernels of gemm_device.h.

@@ -69,6 +69,7 @@ struct Bound {
   MapNParams mapn{};
   bool empty = false;  // nothing to do (e.g. zero trip count with nothing stored)
   bool fallback = false;  // the family's kernels do not take this launch; the generic family's kernel for the same program runs it
+  int64_t slice_trips = 0;  // a generic program whose loop may run in slices: iterations of it (at most, over the grid's corners)
   std::string describe;
   // matrix products with a fused epilogue: which program owns which BM x BN tile (device memory, owned by the binding)
   int *tile_pid = nullptr;
@@ -127,6 +128,21 @@ struct tts_plan {
     if (*buf) retired.push_back(*buf);
     *buf = fresh;
     *have = got;
+    return hipSuccess;
+  }
+  // At least `need` arrival counters for a stream; called with `mu` held.  (New counters start at zero; the old ones, which
+  // launches in flight may still be bumping, are retired.)
+  hipError_t grow_counters(SplitK &sk, size_t need) {
+    if (sk.counters_count >= need) return hipSuccess;
+    int *fresh = nullptr;
+    const size_t count = std::max(need, 2 * sk.counters_count);
+    hipError_t e = hipMalloc((void **)&fresh, count * sizeof(int));
+    if (e == hipSuccess) e = hipMemset(fresh, 0, count * sizeof(int));
+    if (e == hipSuccess) e = hipDeviceSynchronize();  // the fill has landed before a launch on any stream reads the counters
+    if (e != hipSuccess) return e;
+    if (sk.counters) retired.push_back(sk.counters);
+    sk.counters = fresh;
+    sk.counters_count = count;
     return hipSuccess;
   }
   RtcModule *fused = nullptr;  // the kernel compiled for this plan at its first launch (fused maps, tile programs)
@@ -542,7 +558,19 @@ std::shared_ptr<Bound> resolve(tts_plan *h, int gx, int gy, int gz, const tts_ar
       }
       break;
     case Family::FusedMap: bind_fused_map(r, *b); break;
-    case Family::TileProgram: b->describe = "kernel=tile_program\n"; break;
+    case Family::TileProgram: {
+      b->describe = "kernel=tile_program\n";
+      int floats = 0, loop = 0;
+      if (tile_program_is_sliced(h->plan.source, &floats, &loop))
+        for (const SOp &s : h->plan.prog.body)
+          if (s.kind == SK::For && s.loop == loop)
+            for (int corner = 0; corner < 2; corner++) {
+              const EvalEnv e = corner ? r.env(gx - 1, gy - 1, gz - 1) : r.env();
+              const int64_t lb = r.X.eval(s.lb, e), ub = r.X.eval(s.ub, e), step = r.X.eval(s.step, e);
+              if (ub > lb && step > 0) b->slice_trips = std::max(b->slice_trips, (ub - lb + step - 1) / step);
+            }
+      break;
+    }
   }
   h->lru.push_front(key);
   h->cache[key] = {b, h->lru.begin()};
@@ -725,7 +753,7 @@ tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, con
     const char *kname = "";
     // one workgroup of 256 threads per Triton program, on the kernel generated for the program (compiled at its first use)
     auto run_tile_program = [&](RtcModule **slot, const std::string &source) -> tts_status {
-      struct { void *ptr[TILE_MAX_ARGS]; long long ival[TILE_MAX_ARGS]; double fval[TILE_MAX_ARGS]; int swap_xy, lgx, lgy, lgz; } a{};
+      struct TileArgs { void *ptr[TILE_MAX_ARGS]; long long ival[TILE_MAX_ARGS]; double fval[TILE_MAX_ARGS]; int swap_xy, lgx, lgy, lgz; } a{};
       for (int i = 0; i < n; i++) {
         if (args[i].kind == TTS_ARG_PTR) a.ptr[i] = args[i].v.ptr;
         else if (args[i].kind == TTS_ARG_INT) a.ival[i] = args[i].v.i;
@@ -765,6 +793,29 @@ tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, con
         shared = (shared + per_group - 1) / per_group;
         a.lgx = gx; a.lgy = gy; a.lgz = gz;
         err = rtc_launch(*slot, (int)(e[0] * e[1] * e[2]), 1, 1, group_threads, &a, sizeof a, s);
+        return TTS_OK;
+      }
+      int slice_floats = 0, slice_loop = 0;
+      if (tile_program_is_sliced(source, &slice_floats, &slice_loop)) {
+        // As many workgroups as the device holds at once, each program's loop dealt to an equal number of them, two
+        // iterations each at least (dw and db of LayerNorm on fp16 [4096, 8192], 64 programs of 128 iterations: 341 us with
+        // one workgroup per program, 43 us in 12 slices).  A launch that may not allocate keeps to one.
+        const int64_t programs = (int64_t)gx * gy * gz;
+        struct { TileArgs t; int slices; float *partial; int *counters; } sa{};
+        a.lgx = gx; a.lgy = gy; a.lgz = gz;
+        sa.t = a;
+        sa.slices = (int)std::max<int64_t>(1, std::min({(int64_t)rtc_resident_workgroups(*slot) * compute_units() / programs, b->slice_trips / 2, (int64_t)1024}));
+        if (no_alloc) sa.slices = 1;
+        if (sa.slices > 1) {
+          std::lock_guard<std::mutex> lock(plan->mu);
+          tts_plan::SplitK &sk = plan->split_k[stream];
+          hipError_t e = plan->grow((void **)&sk.workspace, &sk.workspace_bytes, (size_t)programs * sa.slices * slice_floats * sizeof(float));
+          if (e == hipSuccess) e = plan->grow_counters(sk, (size_t)programs);
+          if (e != hipSuccess) return fail(TTS_HIP_ERROR, std::string("hipMalloc(partial sums): ") + hipGetErrorString(e));
+          sa.partial = sk.workspace;
+          sa.counters = sk.counters;
+        }
+        err = rtc_launch(*slot, (int)(programs * sa.slices), 1, 1, 256, &sa, sizeof sa, s);
         return TTS_OK;
       }
       // the program asks for neighbouring workgroups along program_id(1) (tile_codegen.cpp); grid.y holds 65535 at most
@@ -938,18 +989,8 @@ tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, con
           tts_plan::SplitK &sk = plan->split_k[stream];
           hipError_t e = plan->grow((void **)&sk.workspace, &sk.workspace_bytes, need);
           if (e != hipSuccess) return fail(TTS_HIP_ERROR, std::string("hipMalloc(split-K workspace): ") + hipGetErrorString(e));
-          if (sk.counters_count < ncount) {
-            // (new counters start at zero; the old ones, which launches in flight may still be bumping, are retired)
-            int *fresh = nullptr;
-            const size_t count = std::max(ncount, 2 * sk.counters_count);
-            e = hipMalloc((void **)&fresh, count * sizeof(int));
-            if (e == hipSuccess) e = hipMemset(fresh, 0, count * sizeof(int));
-            if (e == hipSuccess) e = hipDeviceSynchronize();  // the fill has landed before a launch on any stream reads the counters
-            if (e != hipSuccess) return fail(TTS_HIP_ERROR, std::string("hipMalloc(split-K counters): ") + hipGetErrorString(e));
-            if (sk.counters) plan->retired.push_back(sk.counters);
-            sk.counters = fresh;
-            sk.counters_count = count;
-          }
+          e = plan->grow_counters(sk, ncount);
+          if (e != hipSuccess) return fail(TTS_HIP_ERROR, std::string("hipMalloc(split-K counters): ") + hipGetErrorString(e));
           p.workspace = sk.workspace;
           p.counters = sk.counters;
         }

@@ -752,6 +752,137 @@ struct Gen {
     persistent = !hoisted.empty();
     pack_wide = persistent;
   }
+  // A loop that only adds -- every carried block is `arg + x` with x free of carried values, nothing in the body stores, and
+  // after the loop the blocks are only summed along an axis -- may run in slices: a program's iterations are dealt to
+  // several workgroups, whose sums meet before anything after the loop (see slices_meet).  The column sums of a
+  // normalisation's backward pass are such programs: few of them (a block of columns each), thousands of rows long, and
+  // a launch with one workgroup per program leaves most of the chip idle (dw and db of LayerNorm on fp16 [4096, 8192]: 64
+  // workgroups on 256 CUs, 341 us).
+  const SOp *sliced = nullptr;         // that loop, in slice_head
+  std::vector<SOp> slice_head, slice_tail;  // the ops up to the sums of the loop's results, and the ops after them
+  bool reads_value(int v, const std::set<int> &vs, int depth = 0) const {  // does v's definition name one of vs?
+    if (vs.count(v)) return true;
+    auto d = def.find(v);
+    if (d == def.end() || depth > 64) return depth > 64;
+    std::vector<int> o = d->second->operands;
+    for (int x : {d->second->acc.gather, d->second->acc.mask_value, d->second->acc.other_value})
+      if (x >= 0) o.push_back(x);
+    for (int x : o)
+      if (reads_value(x, vs, depth + 1)) return true;
+    return false;
+  }
+  void choose_slices() {
+    const SOp *L = nullptr;
+    size_t at_loop = 0;
+    for (size_t q = 0; q < P.body.size(); q++)
+      if (P.body[q].kind == SK::For) {
+        if (L) return;
+        L = &P.body[q];
+        at_loop = q;
+      }
+    if (!L || L->tile_args.empty() || P.pool.has_data()) return;
+    for (const SOp &s : P.body) {  // (a carried integer's value after the loop is not known to a slice)
+      std::vector<int> es = s.acc.offsets;
+      for (const auto *more : {&s.acc.strides, &s.acc.dims, &s.acc.mods}) es.insert(es.end(), more->begin(), more->end());
+      es.push_back(s.expr);
+      for (int e : es)
+        if (e >= 0 && P.pool.depends_on(e, EK::Result)) return;
+    }
+    for (size_t q = 0; q < at_loop; q++) {
+      const SK k = P.body[q].kind;
+      if (k != SK::Const && k != SK::Splat && k != SK::Iota && k != SK::FromIndex && k != SK::ScalarArg && k != SK::Map && k != SK::ExpandDims && k != SK::Broadcast) return;
+    }
+    for (const SOp &s : L->body)
+      if (s.kind != SK::Load && s.kind != SK::Const && s.kind != SK::Splat && s.kind != SK::Iota && s.kind != SK::FromIndex && s.kind != SK::ScalarArg && s.kind != SK::Map &&
+          s.kind != SK::ExpandDims && s.kind != SK::Broadcast)
+        return;
+    for (const IntIter &it : L->int_iters) {  // carried integers: init + k * step at iteration k
+      if (it.next == it.iter_expr) continue;
+      const Expr &n = P.pool.at(it.next);
+      if (n.k != EK::Add || (n.a != it.iter_expr && n.b != it.iter_expr)) return;
+      const int step = n.a == it.iter_expr ? n.b : n.a;
+      if (P.pool.depends_on(step, EK::IV) || P.pool.depends_on(step, EK::Iter)) return;
+    }
+    std::map<int, const SOp *> saved = def;
+    for (const SOp &s : L->body)
+      if (s.result >= 0) def[s.result] = &s;
+    const std::set<int> args(L->tile_args.begin(), L->tile_args.end());
+    bool ok = true;
+    std::set<int> sums;
+    for (size_t q = 0; q < L->tile_args.size() && ok; q++) {
+      const Value &V = val(L->tile_args[q]);
+      auto d = def.find(L->tile_yields[q]);
+      ok = V.dtype == "f32" && !V.shape.empty() && d != def.end() && d->second->kind == SK::Map && d->second->name == "arith.addf";
+      if (!ok) break;
+      const auto &o = d->second->operands;
+      const int x = o[0] == L->tile_args[q] ? o[1] : o[0];
+      ok = (o[0] == L->tile_args[q]) != (o[1] == L->tile_args[q]) && !reads_value(x, args) && uses[L->tile_args[q]] == 1;
+      if (L->results[q] < 0) continue;
+      for (const SOp *u : users[L->results[q]]) {
+        ok = ok && u->kind == SK::Reduce && u->name == "arith.addf" && u->operands.size() == 1 && val(u->result).shape.size() == 1 && val(u->result).shape[0] <= 4096;
+        sums.insert(u->result);
+      }
+    }
+    def = saved;
+    if (!ok || sums.empty()) return;
+    for (size_t q = 0; q < P.body.size(); q++) {
+      const SOp &s = P.body[q];
+      const bool head = q <= at_loop || (s.kind == SK::Reduce && sums.count(s.result));
+      if (!head && q > at_loop && s.kind != SK::Store && s.kind != SK::Map && s.kind != SK::Load && s.kind != SK::ExpandDims && s.kind != SK::Broadcast && s.kind != SK::Const &&
+          s.kind != SK::Splat && s.kind != SK::Iota && s.kind != SK::FromIndex && s.kind != SK::ScalarArg) {
+        slice_head.clear();
+        slice_tail.clear();
+        return;
+      }
+      (head ? slice_head : slice_tail).push_back(s);
+    }
+    for (const SOp &s : slice_head)
+      if (s.kind == SK::For) sliced = &s;
+  }
+  // The sums of a sliced program's workgroups: each leaves its own in `partial` (written through, complete before its
+  // arrival is counted), and the one that arrives last adds all of them in slice order -- the result does not depend on
+  // who that is -- and goes on with the program.  Nobody waits for anybody.
+  void slices_meet() {
+    int64_t total = 0;
+    for (const SOp &s : slice_head)
+      if (s.kind == SK::Reduce) total += val(s.result).shape[0];
+    os << pad() << "if (slices > 1) {\n";
+    indent++;
+    os << pad() << "__shared__ int arrived;\n" << pad() << "__syncthreads();\n";
+    int64_t off = 0;
+    for (const SOp &s : slice_head)
+      if (s.kind == SK::Reduce) {
+        const int64_t n = val(s.result).shape[0];
+        os << pad() << "for (int c = threadIdx.x; c < " << n << "; c += 256) __hip_atomic_store(&partial[((long long)slice * programs + lin) * " << total << " + " << off << " + c], "
+           << at(s.result, "c", "0") << ", __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);\n";
+        off += n;
+      }
+    os << pad() << "asm volatile(\"s_waitcnt vmcnt(0)\" ::: \"memory\");\n" << pad() << "__syncthreads();\n"
+       << pad() << "if (threadIdx.x == 0) {\n"
+       << pad() << "  arrived = __hip_atomic_fetch_add(&counters[lin], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);\n"
+       << pad() << "  if (arrived == slices - 1) __hip_atomic_store(&counters[lin], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next launch\n"
+       << pad() << "}\n" << pad() << "__syncthreads();\n" << pad() << "if (arrived != slices - 1) return;\n";
+    off = 0;
+    for (const SOp &s : slice_head)
+      if (s.kind == SK::Reduce) {
+        const int64_t n = val(s.result).shape[0];
+        os << pad() << "for (int c = threadIdx.x; c < " << n << "; c += 256) {\n"
+           << pad() << "  float sum = 0.f;\n" << pad() << "#pragma unroll 8\n"
+           << pad() << "  for (int s = 0; s < slices; s++) sum += __hip_atomic_load(&partial[((long long)s * programs + lin) * " << total << " + " << off
+           << " + c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);\n"
+           << pad() << "  " << at(s.result, "c", "0") << " = sum;\n" << pad() << "}\n";
+        off += n;
+      }
+    os << pad() << "__syncthreads();\n";
+    indent--;
+    os << pad() << "}\n";
+  }
+  int64_t slice_floats() const {  // floats of `partial` per program and slice
+    int64_t total = 0;
+    for (const SOp &s : slice_head)
+      if (s.kind == SK::Reduce) total += val(s.result).shape[0];
+    return total;
+  }
   std::string element_of_slot(const std::vector<int64_t> &shape) const {
     return wide(shape) ? "8 * (int)threadIdx.x + (n & 7) + 2048 * (n >> 3)" : "threadIdx.x + 256 * n";
   }
@@ -1429,7 +1560,7 @@ struct Gen {
       open_element_loop(cshape);
       for (size_t q = 0; q < s.tile_args.size(); q++)
         if (val(s.tile_args[q]).shape == cshape) {
-          os << pad() << "car" << L << "_" << q << "[n] = " << at(s.tile_inits[q], idx0(cshape), idx1(cshape)) << ";\n";
+          os << pad() << "car" << L << "_" << q << "[n] = " << (&s == sliced ? "slice ? 0.f : " : "") << at(s.tile_inits[q], idx0(cshape), idx1(cshape)) << ";\n";
           if (!mirrored[q].empty()) os << pad() << mirrored[q] << "[t] = car" << L << "_" << q << "[n];\n";
         }
       close_loop();
@@ -1443,11 +1574,27 @@ struct Gen {
       held[s.tile_args[q]] = {"car" + L + "_" + std::to_string(q), val(s.tile_args[q]).shape};
       if (!mirrored[q].empty()) mirror[s.tile_args[q]] = mirrored[q];
     }
-    for (size_t q = 0; q < s.int_iters.size(); q++)
-      os << pad() << "long long it" << L << "_" << q << " = " << ex(s.int_iters[q].init) << ";\n";
-    // the induction variable wraps at the width of the loop's bounds
+    const std::string narrow = P.pool.at(s.lb).bits == 32 ? "(long long)(int)" : "";  // the induction variable wraps at the width of the loop's bounds
+    if (&s == sliced)
+      os << pad() << "const long long lb" << L << " = " << ex(s.lb) << ", step" << L << " = " << ex(s.step) << ", left" << L << " = " << ex(s.ub) << " - lb" << L << ";\n"
+         << pad() << "const long long trips" << L << " = left" << L << " > 0 && step" << L << " > 0 ? (left" << L << " + step" << L << " - 1) / step" << L << " : 0;\n"
+         << pad() << "const long long first" << L << " = trips" << L << " * slice / slices, end" << L << " = trips" << L << " * (slice + 1) / slices;\n";
+    for (size_t q = 0; q < s.int_iters.size(); q++) {
+      os << pad() << "long long it" << L << "_" << q << " = ";
+      if (&s == sliced && s.int_iters[q].next != s.int_iters[q].iter_expr) {
+        const Expr &n = P.pool.at(s.int_iters[q].next);
+        const std::string moved = ex(s.int_iters[q].init) + " + first" + L + " * " + ex(n.a == s.int_iters[q].iter_expr ? n.b : n.a);
+        os << (n.bits == 32 ? "(long long)(int)(" + moved + ")" : moved) << ";\n";
+      } else {
+        os << ex(s.int_iters[q].init) << ";\n";
+      }
+    }
+    if (&s == sliced)
+      os << pad() << "for (long long k" << L << " = first" << L << "; k" << L << " < end" << L << "; k" << L << "++) {\n"
+         << pad() << "  const long long iv" << L << " = " << narrow << "(lb" << L << " + k" << L << " * step" << L << ");\n";
+    else
     os << pad() << "for (long long iv" << L << " = " << ex(s.lb) << "; iv" << L << " < " << ex(s.ub) << "; iv" << L << " = "
-       << (P.pool.at(s.lb).bits == 32 ? "(long long)(int)" : "") << "(iv" << L << " + " << ex(s.step) << ")) {\n";
+       << narrow << "(iv" << L << " + " << ex(s.step) << ")) {\n";
     indent++;
     std::vector<int> body_held;
     loop_depth++;
@@ -2168,6 +2315,7 @@ namespace {
 // row blocks on program_id(0): 119 us; with column blocks there: 100).
 const char *const SWAP_MARK = "// tts: swap_xy\n";
 const char *const MATRIX_MARK = "// tts: matrix ";  // followed by: programs per workgroup, the axis they lie on, threads per workgroup
+const char *const SLICED_MARK = "// tts: sliced ";  // followed by: floats of partial sums per program and slice, the loop's id
 const char *const PERSISTENT_MARK = "// tts: persistent\n";  // the launcher starts a few workgroups per CU, which walk the programs
 bool stores_walk_columns_with_pid1(const Program &p) {
   int votes_for = 0, votes_against = 0;
@@ -2230,20 +2378,29 @@ std::string tile_program_source(const Program &p, bool allow_persistent) {
   g.collect_bases(p.body);
   g.choose_wide_shape();
   if (allow_persistent) g.choose_persistent();
+  if (!g.persistent) g.choose_slices();
   if (g.persistent) g.indent = 2;
-  g.body(p.body);
+  if (g.sliced) {
+    g.body(g.slice_head);
+    g.slices_meet();
+    g.body(g.slice_tail);
+  } else {
+    g.body(p.body);
+  }
   // (a CU has 160 KB of LDS and the compiler lets one workgroup declare all of it; 128 KB leaves room for a second, small one)
   if (g.pool_bytes + g.out_bytes > 128 * 1024)
     throw Unsupported("tile_program: the reductions of this program need " + std::to_string(g.pool_bytes + g.out_bytes) + " bytes of LDS (limit 131072)");
   std::ostringstream all;
   if (g.persistent) all << PERSISTENT_MARK;
+  else if (g.sliced) all << SLICED_MARK << g.slice_floats() << " " << g.sliced->loop << "\n";
   else if (stores_walk_columns_with_pid1(p)) all << SWAP_MARK;
   all << pre << g.fns.str();
   if (g.uses_dummy) all << "__device__ __attribute__((aligned(16))) unsigned tts_dummy[8];\n";
   // swap_xy: the launcher has exchanged the grid's x and y (see SWAP_MARK)
   // lgx != 0: the launch is one-dimensional and numbers the programs of an lgx x lgy x lgz grid itself, x fastest (the
   // device's grid holds 65535 along y and z; the reference's launcher loops over any extents, backend/driver.py:116-133)
-  all << "extern \"C\" __global__ __launch_bounds__(256) void tile_program(const Args p, const int swap_xy, const int lgx, const int lgy, const int lgz) {\n";
+  all << "extern \"C\" __global__ __launch_bounds__(256) void tile_program(const Args p, const int swap_xy, const int lgx, const int lgy, const int lgz"
+      << (g.sliced ? ", const int slices, float *partial, int *counters" : "") << ") {\n";
   if (g.pool_bytes) all << "  __shared__ __attribute__((aligned(16))) unsigned char pool[" << g.pool_bytes << "];\n";
   all << g.decl.str();
   if (g.persistent) {
@@ -2256,8 +2413,11 @@ std::string tile_program_source(const Program &p, bool allow_persistent) {
         << "    (void)pidx; (void)pidy; (void)pidz; (void)npx; (void)npy; (void)npz; (void)swap_xy;\n"
         << g.loop_top.str() << per_program_thread_index(g.os.str()) << "    __syncthreads();\n  }\n}\n";
   } else {
-    all << "  const long long lin = blockIdx.x;\n"
-        << "  const long long pidx = lgx ? lin % lgx : swap_xy ? blockIdx.y : blockIdx.x, pidy = lgx ? (lin / lgx) % lgy : swap_xy ? blockIdx.x : blockIdx.y,\n"
+    // sliced: the launch is one-dimensional, the slices of a program lie gridDim.x / slices workgroups apart, so that
+    // workgroups that run at the same time read neighbouring blocks
+    if (g.sliced) all << "  const int programs = (int)gridDim.x / slices, slice = (int)blockIdx.x / programs;\n  const long long lin = blockIdx.x - slice * programs;\n";
+    else all << "  const long long lin = blockIdx.x;\n";
+    all << "  const long long pidx = lgx ? lin % lgx : swap_xy ? blockIdx.y : blockIdx.x, pidy = lgx ? (lin / lgx) % lgy : swap_xy ? blockIdx.x : blockIdx.y,\n"
         << "                  pidz = lgx ? lin / ((long long)lgx * lgy) : blockIdx.z;\n"
         << "  const long long npx = lgx ? lgx : swap_xy ? gridDim.y : gridDim.x, npy = lgx ? lgy : swap_xy ? gridDim.x : gridDim.y, npz = lgx ? lgz : gridDim.z;\n"
         << "  (void)pidx; (void)pidy; (void)pidz; (void)npx; (void)npy; (void)npz;\n"
@@ -2267,6 +2427,11 @@ std::string tile_program_source(const Program &p, bool allow_persistent) {
     if (g.all_store_bases.count(b))
       throw Unsupported("tile_program: an argument is both stored to and read by a load that is not of its body's block shape");
   return without_double_barriers(all.str());
+}
+
+bool tile_program_is_sliced(const std::string &source, int *floats, int *loop) {
+  if (source.compare(0, strlen(SLICED_MARK), SLICED_MARK) != 0) return false;
+  return sscanf(source.c_str() + strlen(SLICED_MARK), "%d %d", floats, loop) == 2;
 }
 
 std::string matrix_program_source(const Program &p) {
