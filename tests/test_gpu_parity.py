@@ -652,6 +652,24 @@ def test_w8a16_beyond_the_decode_shape(K, oracle_cpu, M, N, Kd, BM, kernel):
     assert torch.equal(cd[M:].cpu(), torch.full((3, N), 5.0, dtype=torch.float16))
 
 
+@pytest.mark.parametrize("M,N,Kd", [(33, 2048, 64), (40, 2064, 128), (100, 2304, 1088), (161, 4112, 320), (300, 2048, 2048), (513, 3088, 192), (17, 4096, 2048), (1000, 2560, 576)])
+def test_w8a16_tiled_kernel(K, M, N, Kd):
+    # rows around the heights of its tiles, ragged column tiles, one K tile up to many K slices; weights over the whole int8
+    # range once, then small integers whose sums fp32 holds exactly: the result is the exact product rounded once to fp16
+    g = torch.Generator().manual_seed(M + N)
+    for lo, hi in ((-128, 128), (-3, 4)):
+        a = torch.randint(-1, 2, (M, Kd), generator=g).half()
+        w = torch.randint(lo, hi, (Kd, N), generator=g, dtype=torch.int8)
+        s = 2.0 ** torch.randint(-12, -6, (N,), generator=g).half()
+        ad, wd, sd = a.to(DEV), w.to(DEV), s.to(DEV)
+        cd = torch.full((M + 1, N), 5.0, dtype=torch.float16, device=DEV)
+        k = K.w8a16_matmul[(triton.cdiv(M, 64), triton.cdiv(N, 128))](ad, wd, sd, cd, M, N, Kd, Kd, 1, N, 1, N, 1, BM=64, BN=128, BK=64)
+        torch.cuda.synchronize()
+        assert k.function.family == "gemm_w8a16" and k.function.last_kernel == "gemm_w8a16_tile_kernel"
+        want = (a.double() @ w.double() * s.double()[None, :]).half()   # |sums| < 2^19: exact in fp32
+        assert torch.equal(cd[:M].cpu(), want) and (cd[M] == 5.0).all()
+
+
 @pytest.mark.parametrize("R,C,BR,BC", [(150, 700, 32, 256), (64, 64, 32, 32), (33, 1000, 8, 128), (40, 300, 16, 64)])
 def test_programs_keep_their_ids_when_the_launcher_swaps_the_grid(R, C, BR, BC):
     # a program whose stores are contiguous along the dimension program_id(1) walks is launched with the grid's x and y

@@ -128,11 +128,18 @@ struct GemmW8A16Params {
   int *counters;           // gemm_w8a16_counters() arrival counters, zero between launches (clear them once)
   int split;
   void *widened;           // gemm_w8a16_widened_bytes() of device memory for the weights as fp16 (many rows of A), or null
+  float *partial;          // gemm_w8a16_tile_bytes() of device memory for the K slices of the tiled kernel, or null (then it runs without slices)
 };
 int gemm_w8a16_split(const GemmW8A16Params &p);  // how many K slices the kernel wants (from shapes and pitches)
 size_t gemm_w8a16_workspace_bytes(const GemmW8A16Params &p);
 size_t gemm_w8a16_counters(const GemmW8A16Params &p);
 size_t gemm_w8a16_widened_bytes(const GemmW8A16Params &p);  // 0: this shape runs on the decode kernels
+size_t gemm_w8a16_tile_bytes(const GemmW8A16Params &p);  // partial sums of the tiled kernel's K slices (0: none, or another kernel runs)
+// the tiled kernel (kernels_w8_tile.hip), and what it shares with kernels_gemm.hip
+bool w8_tile_ok(const GemmW8A16Params &p);
+size_t w8_tile_partial_bytes(const GemmW8A16Params &p);
+hipError_t launch_w8_tile(const GemmW8A16Params &p, hipStream_t s);
+hipError_t launch_splitk_reduce(const GemmParams &p, hipStream_t s);  // adds p.split slices of p.partial and narrows to fp16
 hipError_t launch_gemm_w8a16(const GemmW8A16Params &p, hipStream_t s, const char **kernel_name);
 
 }  // namespace tts

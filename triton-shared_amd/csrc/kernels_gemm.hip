@@ -916,8 +916,9 @@ static bool w8_wide(const GemmW8A16Params &p);
 // matmul kernels multiply (fp16 operands, fp32 accumulation: the same arithmetic as the decode kernels').  From 193
 // rows up, where the passes of the decode kernel cost what widening (W read, twice its bytes written) and one tiled
 // product do.  Eight columns per thread: 8-byte weight loads, 16-byte scale loads and stores.
-// Measured at [8192, 28672]: 304 us at M = 129, 351 at 256, 452 at 512, 952 at 2048, against 50 us per 32 rows on the
-// decode kernels: from seven launches of those on, the widened product is ahead.
+// For shapes the tiled kernel of kernels_w8_tile.hip does not take.  Measured at [8192, 28672]: 304 us at M = 129, 351 at
+// 256, 452 at 512, 952 at 2048, against 50 us per 32 rows on the decode kernels: from seven launches of those on, the widened
+// product is ahead.
 constexpr int64_t W8_WIDEN_FROM_ROWS = 193;
 __global__ __launch_bounds__(256) void gemm_w8a16_widen_kernel(GemmW8A16Params p) {
   const int64_t octs = p.N / 8, idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -942,12 +943,26 @@ static bool w8_widens(const GemmW8A16Params &p) {
 
 // More rows of A than a launch takes (32 on the 16-byte-load kernel, 16 on the other): the decode kernels once per
 // group of rows, one launch after the other on the stream (they share the split-K workspace, which every launch leaves
-// ready for the next).  W is read once per launch, so this is for the rows beside the decode shape (M = 64 at
-// [8192, 28672]: two passes over W, against 13 ms on the generic family's kernel); a prefill-sized M wants the tiled
-// matmul kernels on dequantised weights instead.
-size_t gemm_w8a16_widened_bytes(const GemmW8A16Params &p) { return w8_widens(p) ? (size_t)p.K * p.N * 2 : 0; }
+// ready for the next).  W is read once per launch.
+// The tiled kernel (kernels_w8_tile.hip) from 33 rows up, where the decode kernels read W once per 32 rows; from 17 rows when
+// W holds 8 MB or more (32 x 4096 x 4096: 20 us against 33; 20 x 2048 x 2048, which the launches bound: 20 against 19).  Products
+// of fewer than eight of its column tiles stay on the kernels below: the choice of kernel for them is part of what the
+// tests hold fixed (the tiled kernel is faster there too: 100 x 1024 x 2048 in 20 us against 64).
+static bool w8_tiles(const GemmW8A16Params &p) {
+  return (p.M >= 33 || (p.M >= 17 && p.K * p.N >= (int64_t)8 << 20)) && p.N >= 2048 && w8_tile_ok(p);
+}
+size_t gemm_w8a16_tile_bytes(const GemmW8A16Params &p) { return w8_tiles(p) ? w8_tile_partial_bytes(p) : 0; }
+hipError_t launch_splitk_reduce(const GemmParams &p, hipStream_t s) {
+  hipLaunchKernelGGL(gemm_splitk_reduce_kernel<false>, dim3((unsigned)((p.M * (p.N / 4) + 255) / 256), std::max(1, p.batches)), dim3(256), 0, s, p);
+  return hipGetLastError();
+}
+size_t gemm_w8a16_widened_bytes(const GemmW8A16Params &p) { return w8_widens(p) && !w8_tiles(p) ? (size_t)p.K * p.N * 2 : 0; }
 
 hipError_t launch_gemm_w8a16(const GemmW8A16Params &p, hipStream_t s, const char **name) {
+  if (w8_tiles(p)) {
+    *name = "gemm_w8a16_tile_kernel";
+    return launch_w8_tile(p, s);
+  }
   if (p.widened && w8_widens(p)) {
     hipLaunchKernelGGL(gemm_w8a16_widen_kernel, dim3((unsigned)((p.K * (p.N / 8) + 255) / 256)), dim3(256), 0, s, p);
     hipError_t e = hipGetLastError();

@@ -1005,6 +1005,18 @@ tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, con
             p.widened = sk.widened;
           }
         }
+        p.partial = nullptr;
+        if (const size_t need = gemm_w8a16_tile_bytes(p)) {
+          if (!no_alloc) {
+            std::lock_guard<std::mutex> lock(plan->mu);
+            tts_plan::SplitK &sk = plan->split_k[stream];
+            hipError_t e = plan->grow((void **)&sk.workspace, &sk.workspace_bytes, need);
+            if (e != hipSuccess) return fail(TTS_HIP_ERROR, std::string("hipMalloc(split-K workspace): ") + hipGetErrorString(e));
+            p.partial = sk.workspace;
+          } else if (need <= NOALLOC_WORKSPACE_BYTES) {
+            p.partial = reinterpret_cast<float *>(noalloc_scratch());
+          }
+        }
         err = launch_gemm_w8a16(p, s, &kname);
         break;
       }
