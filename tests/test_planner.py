@@ -614,3 +614,16 @@ def test_batched_matmul_and_carried_scalars_plan(native):
     s = native.ttir_to_structured(compile_ttir(X.while_sum_until, sig, {"BLOCK": 256}))
     assert "ub=" in s and "2147483647" in s and "ival=2" in s
     assert native.PlanHandle(native.structured_to_plan(s)[0]).family == "tile_program"
+
+
+@pytest.mark.parametrize("dtype", ["fp16", "fp32"])
+def test_loops_end_with_a_barrier_behind_what_an_iteration_staged(native, tmp_path, dtype):
+    """A row's scale is copied to LDS at the top of every iteration and read through a broadcast at its end: without a
+    barrier between that reading and the next iteration's copy, a fast wavefront overwrites what a slow one still reads."""
+    import extra_kernels as X
+    sig = {"x_ptr": "*" + dtype, "s_ptr": "*fp32", "out_ptr": "*fp32", "n_rows": "i32", "n_cols": "i32", "pitch": "i32", "BR": "constexpr", "BC": "constexpr"}
+    src = _generic_source(tmp_path, compile_ttir(X.column_moments, sig, {"BR": 16, "BC": 64}))
+    loop = src[src.index("for (long long k0"):src.index("const long long res0_0")]
+    assert "blk" in loop
+    behind = loop[loop.rindex("blk"):]
+    assert "__syncthreads();" in behind, behind

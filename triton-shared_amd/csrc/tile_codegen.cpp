@@ -1598,8 +1598,10 @@ struct Gen {
     indent++;
     std::vector<int> body_held;
     loop_depth++;
+    const size_t body_at = os.str().size();
     body(s.body, &body_held);
     loop_depth--;
+    const bool staged = os.str().find("__syncthreads", body_at) != std::string::npos;
     // the scalars' new values first, their assignment last: the blocks' new values may be written in terms of the old scalars
     for (size_t q = 0; q < s.tile_args.size(); q++)
       if (scalar(q)) os << pad() << "const " << ctype(val(s.tile_args[q]).dtype) << " nys" << L << "_" << q << " = " << at(s.tile_yields[q], "0", "0") << ";\n";
@@ -1643,6 +1645,9 @@ struct Gen {
     for (size_t q = 0; q < s.int_iters.size(); q++)
       os << pad() << "const long long nx" << L << "_" << q << " = " << ex(s.int_iters[q].next) << ";\n";
     for (size_t q = 0; q < s.int_iters.size(); q++) os << pad() << "it" << L << "_" << q << " = nx" << L << "_" << q << ";\n";
+    // what an iteration staged in LDS is still being read above (a row's scale next to a carried block, say) while the
+    // fastest wavefront could begin the next iteration and stage over it
+    if (staged) os << pad() << "__syncthreads();\n";
     indent--;
     os << pad() << "}\n";
     for (size_t q = 0; q < s.int_iters.size(); q++)
