@@ -396,6 +396,27 @@ def test_matmul_with_wraparound_operands(K, oracle_cpu, M, N, Kd, dtype):
         assert relfro(cd.cpu(), oracle_cpu.matmul_tiles(a, b)) <= 1e-2
 
 
+@pytest.mark.parametrize("M,N,Kd,pad,at,bt", [(2, 3, 5, 0, False, False), (127, 9, 320, 0, False, False), (129, 131, 64, 0, False, False), (130, 257, 321, 3, False, False),
+                                              (64, 7, 449, 0, False, False), (3, 140, 576, 0, False, True), (131, 129, 385, 5, False, True), (200, 130, 384, 0, True, False), (133, 65, 450, 1, True, True)])
+def test_gemm_any_shape_kernel_reads_and_writes_only_its_problem(K, M, N, Kd, pad, at, bt):
+    # one K tile up to more than the pipeline holds, a last tile that is whole or nearly empty, rows at every alignment, each
+    # layout of the operands; what lies between the rows is NaN and reaches no result.  Small integers: exact in any order
+    g = torch.Generator().manual_seed(M + N + Kd)
+    def operand(rows, cols, turned):
+        x = torch.randint(-2, 3, (rows, cols), generator=g).to(torch.float16)
+        full = torch.full((cols, rows + pad) if turned else (rows, cols + pad), float("nan"), dtype=torch.float16)
+        full[:, :rows if turned else cols] = x.t() if turned else x
+        d = full.to(DEV)
+        return x, (d.t()[:rows] if turned else d[:, :cols])
+    (a, ad), (b, bd) = operand(M, Kd, at), operand(Kd, N, bt)
+    cd = torch.full((M + 1, N + 1), 7.0, dtype=torch.float16, device=DEV)
+    k = K.matmul_tiles[(triton.cdiv(M, 128) * triton.cdiv(N, 128),)](ad, bd, cd, M, N, Kd, ad.stride(0), ad.stride(1), bd.stride(0), bd.stride(1), N + 1, 1, BM=128, BN=128, BK=64, GROUP_M=8)
+    torch.cuda.synchronize()
+    assert k.function.last_kernel.startswith("gemm_mfma_kernel")
+    assert torch.equal(cd[:M, :N].cpu().double(), a.double() @ b.double())
+    assert (cd[M] == 7.0).all() and (cd[:, N] == 7.0).all()
+
+
 def test_gemm_with_padded_pitches_and_untouched_border(K):
     torch.manual_seed(3)
     M, N, Kd = 200, 300, 150

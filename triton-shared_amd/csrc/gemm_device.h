@@ -94,13 +94,17 @@ __device__ __forceinline__ uint4 load8(const uint16_t *p, int valid, bool vec) {
 // The kernel for any shape, any alignment, and operands that are row- or column-major.
 // Workgroup: 256 threads = 2 x 2 wavefronts; each wavefront owns TM x TN MFMA tiles of 32 x 32.  An operand tile is
 // R = BM = BN rows (rows of A, columns of B) by BK values of k and is staged through LDS (two buffers) in the form it
-// has in memory, with 16-byte loads and stores where alignment allows:
+// has in memory, with 16-byte loads and stores:
 //   k contiguous (A row-major, B column-major): LDS [r][k], pitch BK + 8 elements; a lane's MFMA operand (8 consecutive
 //     k of row lane % 32) is one 16-byte read, and 32 consecutive rows hit distinct banks;
 //   r contiguous (B row-major, A column-major): LDS [k][r], pitch R + 16 elements; `ds_read_b64_tr_b16` transposes on
 //     the way out -- within 16 lanes, lane i receives element i % 4 of the 8-byte rows addressed by lanes i / 4,
 //     i / 4 + 4, i / 4 + 8, i / 4 + 12, so lane j of a group addresses k row j / 4, elements 4 (j % 4) .. +3 of the
 //     group's 16, and two reads (k 0-3, k 4-7) make one operand.
+// What bounds it on ragged sizes is the way of the operands from memory, a chain of one load per K tile where a shape
+// gives the chip less than one workgroup per CU.  Chunks are therefore 16-byte loads at any alignment (global memory takes
+// them at element addresses), untested in all K tiles but the last, and two tiles are in flight.  1000 x 3001 x 1003 fp16 with
+// a fused activation: 27.8 us; with eight two-byte loads for every chunk that is not 16-byte aligned, each behind a test, 163.
 // Rows of A may be taken through an index vector (p.a_rows) and the base of B may depend on the block of rows
 // (p.b_block): a mixture-of-experts product is this kernel with both set.
 // `ep(acc, row, col)` maps an accumulator value to the value that is stored at (row, col) of C (the identity for a plain
@@ -177,7 +181,6 @@ __device__ __forceinline__ void gemm_mfma_body(const GemmParams &p, int tiles_m,
       b_at[j] = n0 + (c % (BN / 8)) * 8;
     }
   }
-  uint4 ra[CA], rb[CA];
   auto load_operand = [&](uint4 (&reg)[CA], const uint16_t *P, bool r_contiguous, const int64_t (&at)[CA], int64_t ld, int64_t rows, bool vec, int k0) {
 #pragma unroll
     for (int j = 0; j < CA; j++) {
@@ -225,24 +228,48 @@ __device__ __forceinline__ void gemm_mfma_body(const GemmParams &p, int tiles_m,
   const int nk = (K + BK - 1) / BK;
   auto sweep_k = [&](auto a_form, auto b_form) {
     constexpr bool a_r = decltype(a_form)::value, b_r = decltype(b_form)::value;  // r-contiguous in memory and in LDS
-    auto load_tiles = [&](int k0) {
-      load_operand(ra, A, a_r, a_at, p.lda, p.M, a_vec, k0);
-      load_operand(rb, B, b_r, b_at, p.ldb, p.N, b_vec, k0);
+    // K tiles [0, nwide) load 16 bytes a chunk without a test, at any alignment: rows (columns) beyond the problem are
+    // replaced by others, they only reach results nobody stores; a chunk that starts inside a row of an r-contiguous
+    // operand and ends behind it reads into the next row, which the last k row does not have.
+    int nwide = K / BK;
+    if ((a_r && p.lda < 8) || (b_r && p.ldb < 8)) nwide = 0;
+    else if (K % BK == 0 && ((a_r && m0 + BM > p.M) || (b_r && n0 + BN > p.N))) nwide = nk - 1;
+    const uint16_t *a_ptr[CA], *b_ptr[CA];
+    auto first_chunk = [&](const uint16_t *P, bool r_contiguous, const int64_t at, int64_t other, int64_t ld, int64_t rows, int c) {
+      return r_contiguous ? P + (c / (BM / 8)) * ld + (at < rows ? at : 0) : P + (at >= 0 ? at : other) + (c % (BK / 8)) * 8;
     };
-    auto store_tiles = [&](int buf) {
-      uint16_t *As = smem + buf * Lds::BUFFER_ELEMS, *Bs = As + Lds::A_ELEMS;
-      store_operand(ra, As, a_r);
-      store_operand(rb, Bs, b_r);
-    };
-    if (nk > 0) {
-      load_tiles(0);
-      store_tiles(0);
+    // a row beyond the problem: the tile's first, or where rows are gathered the operand's first (store_tiles clears them)
+    const int64_t a_first = a_r || p.a_rows ? 0 : m0 * p.lda;
+#pragma unroll
+    for (int j = 0; j < CA; j++) {
+      a_ptr[j] = first_chunk(A, a_r, a_at[j], a_first, p.lda, p.M, tid + 256 * j);
+      b_ptr[j] = first_chunk(B, b_r, b_at[j], n0 * p.ldb, p.ldb, p.N, tid + 256 * j);
     }
-    __syncthreads();
-    for (int kt = 0; kt < nk; kt++) {
-      const int cur = kt & 1;
-      if (kt + 1 < nk) load_tiles((kt + 1) * BK);
-      const uint16_t *As = smem + cur * Lds::BUFFER_ELEMS, *Bs = As + Lds::A_ELEMS;
+    struct Tiles { uint4 a[CA], b[CA]; };
+    auto load_wide = [&](Tiles &t, int kt) {
+      const int64_t a_k = a_r ? (int64_t)kt * BK * p.lda : (int64_t)kt * BK, b_k = b_r ? (int64_t)kt * BK * p.ldb : (int64_t)kt * BK;
+#pragma unroll
+      for (int j = 0; j < CA; j++) __builtin_memcpy(&t.a[j], a_ptr[j] + a_k, 16);
+#pragma unroll
+      for (int j = 0; j < CA; j++) __builtin_memcpy(&t.b[j], b_ptr[j] + b_k, 16);
+    };
+    auto load_any = [&](Tiles &t, int kt) {
+      if (kt < nwide) load_wide(t, kt);
+      else if (kt < nk) {
+        load_operand(t.a, A, a_r, a_at, p.lda, p.M, a_vec, kt * BK);
+        load_operand(t.b, B, b_r, b_at, p.ldb, p.N, b_vec, kt * BK);
+      }
+    };
+    auto store_tiles = [&](const Tiles &t, int buf) {
+      uint16_t *As = smem + buf * Lds::BUFFER_ELEMS, *Bs = As + Lds::A_ELEMS;
+      uint4 a[CA];
+#pragma unroll
+      for (int j = 0; j < CA; j++) a[j] = a_r || a_at[j] >= 0 ? t.a[j] : make_uint4(0, 0, 0, 0);
+      store_operand(a, As, a_r);
+      store_operand(t.b, Bs, b_r);
+    };
+    auto multiply = [&](int buf) {
+      const uint16_t *As = smem + buf * Lds::BUFFER_ELEMS, *Bs = As + Lds::A_ELEMS;
 #pragma unroll
       for (int ks = 0; ks < BK / 16; ks++) {
         uint4 af[TM], bf[TN];
@@ -255,7 +282,34 @@ __device__ __forceinline__ void gemm_mfma_body(const GemmParams &p, int tiles_m,
 #pragma unroll
           for (int j = 0; j < TN; j++) acc[i][j] = mfma32<BF16>(af[i], bf[j], acc[i][j]);
       }
-      if (kt + 1 < nk) store_tiles(cur ^ 1);
+    };
+    // Two K tiles are in flight in registers beside the two in LDS: a tile's loads are issued two products before they are stored.
+    Tiles even, odd;
+    load_any(even, 0);
+    load_any(odd, 1);
+    if (nk > 0) store_tiles(even, 0);
+    load_any(even, 2);
+    __syncthreads();
+    int kt = 0;
+    for (; kt + 4 < nwide; kt += 2) {  // loads tiles kt + 3 and kt + 4
+      multiply(0);
+      store_tiles(odd, 1);
+      load_wide(odd, kt + 3);
+      __syncthreads();
+      multiply(1);
+      store_tiles(even, 0);
+      load_wide(even, kt + 4);
+      __syncthreads();
+    }
+    for (; kt < nk; kt += 2) {
+      multiply(0);
+      if (kt + 1 >= nk) break;
+      store_tiles(odd, 1);
+      load_any(odd, kt + 3);
+      __syncthreads();
+      multiply(1);
+      if (kt + 2 < nk) store_tiles(even, 0);
+      load_any(even, kt + 4);
       __syncthreads();
     }
   };
