@@ -836,6 +836,33 @@ def test_loops_that_only_add_run_in_slices(dtype, rows, cols, pitch):
         assert torch.equal(out[:3].double(), want) and (out[3] == 9.0).all()
 
 
+def test_loops_that_only_add_can_be_recorded_in_a_graph():
+    # a recorded launch neither allocates nor holds the stream's workspace: it keeps to one workgroup per program.  Replays
+    # between eager launches of the same kernel on the stream that recorded it
+    import extra_kernels as X
+    rows, cols = 5000, 100
+    g = torch.Generator().manual_seed(3)
+    x, s = torch.randint(-3, 4, (rows, cols), generator=g).half().to(DEV), torch.randint(-2, 3, (rows,), generator=g).float().to(DEV)
+    launch = lambda out: X.column_moments[(triton.cdiv(cols, 64),)](x, s, out, rows, cols, cols, BR=16, BC=64)
+    eager, recorded = torch.zeros(3, cols, device=DEV), torch.zeros(3, cols, device=DEV)
+    launch(eager)
+    torch.cuda.synchronize()
+    graph, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    with torch.cuda.graph(graph, stream=side):
+        launch(recorded)
+    for seed in range(3):
+        x.copy_(torch.randint(-3, 4, (rows, cols), generator=g).half())
+        recorded.zero_()
+        eager.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        with torch.cuda.stream(side):
+            launch(eager)
+        torch.cuda.synchronize()
+        a, b = (x.double() * s[:, None].double()).sum(0) + 1, (x.double() ** 2).sum(0)
+        assert torch.equal(eager.double(), torch.stack([a, b, a - 2 * b])) and torch.equal(recorded, eager)
+
+
 def test_softmax_rows_the_row_kernel_declines(K, oracle_cpu):
     import extra_kernels as X
     torch.manual_seed(5)

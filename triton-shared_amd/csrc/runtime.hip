@@ -725,6 +725,15 @@ int compute_units() {  // of the current device (256 when the query fails)
   return cus;
 }
 
+// Whether the stream records a graph: nothing may be allocated then, and a workspace of the stream's would be shared by
+// every replay.
+bool is_capturing(hipStream_t s) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &status) == hipSuccess) return status != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return false;
+}
+
 // tts_launch and tts_launch_noalloc (no_alloc: nothing below may allocate device memory or compile)
 tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, const tts_arg *args, int n, bool no_alloc) {
   if (!plan || (n > 0 && !args)) return fail(TTS_INVALID, "null argument");
@@ -799,13 +808,14 @@ tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, con
       if (tile_program_is_sliced(source, &slice_floats, &slice_loop)) {
         // As many workgroups as the device holds at once, each program's loop dealt to an equal number of them, two
         // iterations each at least (dw and db of LayerNorm on fp16 [4096, 8192], 64 programs of 128 iterations: 341 us with
-        // one workgroup per program, 43 us in 12 slices).  A launch that may not allocate keeps to one.
+        // one workgroup per program, 43 us in 12 slices).  A launch that may not allocate keeps to one, and so does one that
+        // is recorded into a graph: the graph may be replayed beside launches that use the same stream's workspace.
         const int64_t programs = (int64_t)gx * gy * gz;
         struct { TileArgs t; int slices; float *partial; int *counters; } sa{};
         a.lgx = gx; a.lgy = gy; a.lgz = gz;
         sa.t = a;
         sa.slices = (int)std::max<int64_t>(1, std::min({(int64_t)rtc_resident_workgroups(*slot) * compute_units() / programs, b->slice_trips / 2, (int64_t)1024}));
-        if (no_alloc) sa.slices = 1;
+        if (sa.slices > 1 && (no_alloc || is_capturing(s))) sa.slices = 1;
         if (sa.slices > 1) {
           std::lock_guard<std::mutex> lock(plan->mu);
           tts_plan::SplitK &sk = plan->split_k[stream];
@@ -1007,13 +1017,13 @@ tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, con
         }
         p.partial = nullptr;
         if (const size_t need = gemm_w8a16_tile_bytes(p)) {
-          if (!no_alloc) {
+          if (!no_alloc && !is_capturing(s)) {
             std::lock_guard<std::mutex> lock(plan->mu);
             tts_plan::SplitK &sk = plan->split_k[stream];
             hipError_t e = plan->grow((void **)&sk.workspace, &sk.workspace_bytes, need);
             if (e != hipSuccess) return fail(TTS_HIP_ERROR, std::string("hipMalloc(split-K workspace): ") + hipGetErrorString(e));
             p.partial = sk.workspace;
-          } else if (need <= NOALLOC_WORKSPACE_BYTES) {
+          } else if (no_alloc && need <= NOALLOC_WORKSPACE_BYTES) {
             p.partial = reinterpret_cast<float *>(noalloc_scratch());
           }
         }
