@@ -417,6 +417,40 @@ def test_gemm_any_shape_kernel_reads_and_writes_only_its_problem(K, M, N, Kd, pa
     assert (cd[M] == 7.0).all() and (cd[:, N] == 7.0).all()
 
 
+@pytest.mark.parametrize("M,N,Kd,bt,dtype", [(17, 129, 4095, True, torch.bfloat16), (100, 700, 2000, False, torch.float16), (200, 15, 1984, False, torch.bfloat16), (130, 257, 1153, True, torch.float16)])
+def test_gemm_any_shape_kernel_in_k_slices(K, M, N, Kd, bt, dtype):
+    # few tiles and a long K: slices whose sums a second kernel adds, narrow and wide rows; with and without a functor that
+    # looks at the element's position and at what the output held.  Integers: exact in fp32, results of at most 8 bits
+    import extra_kernels as X
+    g = torch.Generator().manual_seed(M + N)
+    a = torch.zeros(M, Kd, dtype=dtype)
+    a.scatter_(1, torch.randint(0, Kd, (M, 40), generator=g), 1.0)
+    b = torch.randint(-2, 3, (Kd, N), generator=g).to(dtype)
+    want = a.double() @ b.double()
+    ad, bd = a.to(DEV), (b.t().contiguous().to(DEV).t() if bt else b.to(DEV))
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    for i in range(4):
+        with torch.cuda.stream(streams[i % 2]):
+            cd = torch.full((M + 1, N + 3), 7.0, dtype=dtype, device=DEV)
+            k = K.matmul_tiles[(triton.cdiv(M, 128) * triton.cdiv(N, 128),)](ad, bd, cd, M, N, Kd, Kd, 1, bd.stride(0), bd.stride(1), N + 3, 1, BM=128, BN=128, BK=64, GROUP_M=8)
+        torch.cuda.synchronize()
+        assert k.function.last_kernel == "gemm_mfma_kernel<128x128x64>, K slices"
+        assert torch.equal(cd[:M, :N].cpu().double(), want) and (cd[M] == 7.0).all() and (cd[:, N:] == 7.0).all()
+    bias = torch.randint(-4, 5, (N,), generator=g).float()
+    held = torch.randint(-8, 9, (M, N), generator=g).to(dtype)
+    run = lambda c, **kw: X.matmul_leaky[(triton.cdiv(M, 128), triton.cdiv(N, 128))](ad, b.to(DEV), c, M, N, Kd, Kd, N, N, 0.5, BM=128, BN=128, BK=64, **kw)
+    c = held.to(DEV)
+    k = run(c, ACT=2, bias_ptr=bias.to(DEV))
+    torch.cuda.synchronize()
+    assert k.function.last_kernel == "gemm_mfma_kernel<128x128x64> + epilogue (hipRTC), K slices"
+    assert torch.equal(c.cpu().double(), torch.nn.functional.leaky_relu(want + bias.double(), 0.5))
+    c = held.to(DEV)
+    run(c, ACT=3)
+    torch.cuda.synchronize()
+    assert torch.equal(c.cpu().double(), want * 0.5 + held.double())
+
+
 def test_gemm_with_padded_pitches_and_untouched_border(K):
     torch.manual_seed(3)
     M, N, Kd = 200, 300, 150

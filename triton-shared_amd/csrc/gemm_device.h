@@ -1,8 +1,8 @@
 // Device code of the 16-bit matrix-product kernels, in a header of its own because it is compiled twice: ahead of
 // time into the library (kernels_gemm.hip, results stored as they are), and at run time with hipRTC when the Triton
 // kernel applies elementwise ops to the accumulator before the store (a fused activation): the generated source
-// defines TTS_GEMM_RTC (which kernel: 0 whole 256 x 256 x 32 tiles, 1 any shape in 128 x 128 x 64 tiles), TTS_GEMM_BF16 and the functor TtsEp (a plain struct, passed as the kernel's last argument) that maps
-// an accumulator value and its position to the value stored, then this file's text.  Nothing here may need a host header.
+// defines TTS_GEMM_RTC (which kernel: 0 whole 256 x 256 x 32 tiles, 1 any shape in 128 x 128 x 64 tiles, 2 the sum of the K
+// slices), TTS_GEMM_BF16 and the functor TtsEp (a plain struct, passed as the kernel's last argument) that maps an accumulator value and its position to the value stored, then this file's text.  Nothing here may need a host header.
 #pragma once
 #ifdef __HIPCC_RTC__
 typedef __INT64_TYPE__ int64_t;
@@ -122,7 +122,10 @@ struct GemmStageLds {
   static constexpr int BYTES = 2 * BUFFER_ELEMS * 2;
 };
 
-template <bool BF16, int TM, int TN, int BK, class Ep>
+//
+// SK: the grid holds p.split workgroups per tile; workgroup (tile, s) walks the s-th share of the K tiles and leaves its fp32
+// sums in p.partial (gemm_splitk_reduce_body adds them and applies the functor).
+template <bool BF16, int TM, int TN, int BK, class Ep, bool SK = false>
 __device__ __forceinline__ void gemm_mfma_body(const GemmParams &p, int tiles_m, int tiles_n, const Ep &ep) {
   constexpr int BM = 2 * TM * 32, BN = 2 * TN * 32;
   constexpr int PK = BK + 8;   // pitch of a k-contiguous tile
@@ -142,6 +145,8 @@ __device__ __forceinline__ void gemm_mfma_body(const GemmParams &p, int tiles_m,
   // round-robin to the 8 XCDs), and within an XCD walk 8-tile-tall column groups
   int bid = blockIdx.x;
   const int nwg = tiles_m * tiles_n;
+  const int slice = SK ? bid / nwg : 0;
+  if (SK) bid -= slice * nwg;
   if (nwg % 8 == 0) bid = (bid % 8) * (nwg / 8) + bid / 8;
   const int group = 8 * tiles_n;
   const int g0 = (bid / group) * 8;
@@ -225,7 +230,9 @@ __device__ __forceinline__ void gemm_mfma_body(const GemmParams &p, int tiles_m,
 
   // The forms of the two operands are fixed for the launch: the loop is compiled once per combination, so that inside
   // it the loads, the LDS traffic and the MFMAs are straight-line code the compiler can overlap.
-  const int nk = (K + BK - 1) / BK;
+  const int nk_all = (K + BK - 1) / BK;
+  const int k_begin = SK ? (int)((int64_t)slice * nk_all / p.split) : 0;
+  const int nk = SK ? (int)((int64_t)(slice + 1) * nk_all / p.split) : nk_all;  // K tiles [k_begin, nk) are this workgroup's
   auto sweep_k = [&](auto a_form, auto b_form) {
     constexpr bool a_r = decltype(a_form)::value, b_r = decltype(b_form)::value;  // r-contiguous in memory and in LDS
     // K tiles [0, nwide) load 16 bytes a chunk without a test, at any alignment: rows (columns) beyond the problem are
@@ -233,7 +240,8 @@ __device__ __forceinline__ void gemm_mfma_body(const GemmParams &p, int tiles_m,
     // operand and ends behind it reads into the next row, which the last k row does not have.
     int nwide = K / BK;
     if ((a_r && p.lda < 8) || (b_r && p.ldb < 8)) nwide = 0;
-    else if (K % BK == 0 && ((a_r && m0 + BM > p.M) || (b_r && n0 + BN > p.N))) nwide = nk - 1;
+    else if (K % BK == 0 && ((a_r && m0 + BM > p.M) || (b_r && n0 + BN > p.N))) nwide = nk_all - 1;
+    nwide = min(nwide, nk);
     const uint16_t *a_ptr[CA], *b_ptr[CA];
     auto first_chunk = [&](const uint16_t *P, bool r_contiguous, const int64_t at, int64_t other, int64_t ld, int64_t rows, int c) {
       return r_contiguous ? P + (c / (BM / 8)) * ld + (at < rows ? at : 0) : P + (at >= 0 ? at : other) + (c % (BK / 8)) * 8;
@@ -285,12 +293,12 @@ __device__ __forceinline__ void gemm_mfma_body(const GemmParams &p, int tiles_m,
     };
     // Two K tiles are in flight in registers beside the two in LDS: a tile's loads are issued two products before they are stored.
     Tiles even, odd;
-    load_any(even, 0);
-    load_any(odd, 1);
-    if (nk > 0) store_tiles(even, 0);
-    load_any(even, 2);
+    load_any(even, k_begin);
+    load_any(odd, k_begin + 1);
+    if (nk > k_begin) store_tiles(even, 0);
+    load_any(even, k_begin + 2);
     __syncthreads();
-    int kt = 0;
+    int kt = k_begin;
     for (; kt + 4 < nwide; kt += 2) {  // loads tiles kt + 3 and kt + 4
       multiply(0);
       store_tiles(odd, 1);
@@ -321,6 +329,21 @@ __device__ __forceinline__ void gemm_mfma_body(const GemmParams &p, int tiles_m,
     else sweep_k(BoolConstant<false>(), BoolConstant<true>());
   }
 
+  if constexpr (SK) {  // (a lane's place in each 32 x 32 tile: see below)
+    float *__restrict__ part = p.partial + (int64_t)slice * p.M * p.N;
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+      for (int j = 0; j < TN; j++) {
+        const int64_t col = n0 + wn * TN * 32 + j * 32 + (lane & 31);
+#pragma unroll
+        for (int v = 0; v < 16; v++) {
+          const int64_t row = m0 + wm * TM * 32 + i * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
+          if (row < p.M && col < p.N) part[row * p.N + col] = acc[i][j][v];
+        }
+      }
+    return;
+  }
   // epilogue: lane holds column (lane % 32), rows 8*(v/4) + 4*(lane/32) + v%4 of each 32x32 tile
   uint16_t *__restrict__ C = (uint16_t *)p.c;
 #pragma unroll
@@ -334,6 +357,22 @@ __device__ __forceinline__ void gemm_mfma_body(const GemmParams &p, int tiles_m,
         if (row < p.M && col < p.N) C[row * p.ldc + col] = BF16 ? f32_to_bf16(ep(acc[i][j][v], row, col)) : f32_to_f16(ep(acc[i][j][v], row, col));
       }
     }
+}
+
+// Adds the K slices' partial sums in slice order, applies the functor and narrows: one element per thread, for any N.  A
+// workgroup's 256 threads are `across` columns (a power of two) of 256 / across rows; the grid is blocks of columns, fastest,
+// by groups of rows.
+template <bool BF16, class Ep>
+__device__ __forceinline__ void gemm_splitk_reduce_body(const GemmParams &p, int across, int col_blocks, const Ep &ep) {
+  const int64_t row = (int64_t)(blockIdx.x / col_blocks) * (256 / across) + threadIdx.x / across;
+  const int64_t col = (int64_t)(blockIdx.x % col_blocks) * across + threadIdx.x % across;
+  if (row >= p.M || col >= p.N) return;
+  const float *__restrict__ src = p.partial + row * p.N + col;
+  float t = src[0];
+#pragma unroll 4
+  for (int sl = 1; sl < p.split; sl++) t += src[(int64_t)sl * p.M * p.N];
+  const float v = ep(t, row, col);
+  ((uint16_t *)p.c)[row * p.ldc + col] = BF16 ? f32_to_bf16(v) : f32_to_f16(v);
 }
 
 // ------------------------------------------- 16-bit GEMM, full-tile fast path
@@ -1025,6 +1064,8 @@ __device__ __forceinline__ void gemm_dma16_body(const GemmParams &p, int tiles_m
 extern "C" __global__ __launch_bounds__(256) void gemm_rtc(TtsGemmParams p, int tiles_m, int tiles_n, TtsEp ep) {
 #if TTS_GEMM_RTC == 0
   tts_gemm_device::gemm_dma16_body<TTS_GEMM_BF16 != 0>(p, tiles_m, tiles_n, ep);
+#elif TTS_GEMM_RTC == 2
+  tts_gemm_device::gemm_splitk_reduce_body<TTS_GEMM_BF16 != 0>(p, tiles_m, tiles_n, ep);  // (across, col_blocks)
 #else
   tts_gemm_device::gemm_mfma_body<TTS_GEMM_BF16 != 0, 2, 2, 64>(p, tiles_m, tiles_n, ep);
 #endif

@@ -25,27 +25,38 @@ struct IdentityEp {
 };
 
 // the kernels' device code is in gemm_device.h (it is also compiled at run time, with a fused epilogue)
-template <bool BF16, int TM, int TN, int BK>
+template <bool BF16, int TM, int TN, int BK, bool SK>
 __global__ __launch_bounds__(256) void gemm_mfma_kernel(GemmParams p, int tiles_m, int tiles_n) {
-  gemm_mfma_body<BF16, TM, TN, BK>(of_batch(p, 2), tiles_m, tiles_n, IdentityEp());
+  gemm_mfma_body<BF16, TM, TN, BK, IdentityEp, SK>(of_batch(p, 2), tiles_m, tiles_n, IdentityEp());
 }
 
-template <bool BF16, int TM, int TN, int BK>
-hipError_t launch_gemm_cfg(const GemmParams &p, hipStream_t s) {
-  constexpr int BM = 2 * TM * 32, BN = 2 * TN * 32;
-  constexpr size_t lds = GemmStageLds<BM, BN, BK>::BYTES;
-  static bool configured = false;
-  auto kern = gemm_mfma_kernel<BF16, TM, TN, BK>;
-  if (!configured) {
-    hipError_t e = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (e != hipSuccess) return e;
-    configured = true;
+template <bool BF16>
+__global__ __launch_bounds__(256) void gemm_splitk_reduce_any_kernel(GemmParams p, int across, int col_blocks) {
+  gemm_splitk_reduce_body<BF16>(of_batch(p, 2), across, col_blocks, IdentityEp());
+}
+
+// the grid of gemm_splitk_reduce_body
+struct ReduceGrid {
+  int across, col_blocks, workgroups;
+  explicit ReduceGrid(const GemmParams &p) {
+    for (across = 16; across < 256 && across < p.N; across *= 2) {}
+    col_blocks = (int)((p.N + across - 1) / across);
+    workgroups = (int)((p.M + 256 / across - 1) / (256 / across)) * col_blocks;
   }
-  int tiles_m = (int)((p.M + BM - 1) / BM), tiles_n = (int)((p.N + BN - 1) / BN);
-  hipLaunchKernelGGL(kern, dim3(tiles_m * tiles_n, std::max(1, p.batches)), dim3(256), lds, s, p, tiles_m, tiles_n);
+};
+
+// p.split > 1: the slices alone; whoever launches it adds them
+template <bool BF16, bool SK>
+hipError_t launch_gemm_any(const GemmParams &p, hipStream_t s) {
+  constexpr size_t lds = GemmStageLds<128, 128, 64>::BYTES;
+  auto kern = gemm_mfma_kernel<BF16, 2, 2, 64, SK>;
+  static const hipError_t attr = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  if (attr != hipSuccess) return attr;
+  const int tiles_m = (int)((p.M + 127) / 128), tiles_n = (int)((p.N + 127) / 128);
+  hipLaunchKernelGGL(kern, dim3(tiles_m * tiles_n * (SK ? p.split : 1), std::max(1, p.batches)), dim3(256), lds, s, p, tiles_m, tiles_n);
   return hipGetLastError();
 }
-
+hipError_t launch_gemm_any_slices(const GemmParams &p, hipStream_t s) { return p.is_bf16 ? launch_gemm_any<true, true>(p, s) : launch_gemm_any<false, true>(p, s); }
 
 // PF: a fifth wavefront that touches B's lines ahead of the four that work (gemm_device.h); the accumulators then sit in
 // the 256 registers two wavefronts of a SIMD can have each, which the 128 x 256 tile fits without spilling.
@@ -779,11 +790,47 @@ DmaChoice choose_dma(const GemmParams &p, int max_split) {
 }
 }  // namespace
 
+namespace {
+// K slices of the any-shape kernel (1: none), at most max_split: where its tiles leave CUs without work, every workgroup
+// would walk all of K alone.  Modelled like choose_dma's: the K tiles of 64 a workgroup walks (two share a CU), the slices'
+// sums through memory and the second launch.  Measured in bf16 with 1 / 2 / 4 / 8 / 16 slices, us: 33 x 4001 x 4001 62 / 40 /
+// 28 / 23 / 23; 600 x 601 x 3001 56 / 40 / 30 / 27 / 33; 100 x 700 x 2000 32 / 22 / 21 / 21 / 21 (19 to 20 is what the calls of
+// that loop took on the host); 1000 x 3001 x 1003 31 / 40 / 48; 64 x 1003 x 517 18.6 / 20.5 / 20.2: the model takes 1 where two lose.
+int any_split(const GemmParams &p, int max_split) {
+  if (p.a_rows || p.b_block) return 1;
+  static const int cus = [] {
+    int dev = 0, n = 0;
+    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
+    return n;
+  }();
+  const int64_t tiles = ((p.M + 127) / 128) * ((p.N + 127) / 128) * std::max(1, p.batches), nk = (p.K + 63) / 64;
+  const double sums = (double)p.M * (double)p.N * std::max(1, p.batches) * 4;
+  auto model = [&](int split) {
+    const double wgs = (double)tiles * split;
+    double t = std::max(1.0, wgs / (1.5 * cus)) * (double)((nk + split - 1) / split) * 1.0e-6 + 5e-6;
+    if (split > 1) t += 2 * split * sums / 4e12 + 6e-6;
+    return t;
+  };
+  static const char *split_env = getenv("TTS_GEMM_SPLIT");  // tuning aid (see choose_dma)
+  if (split_env) return std::max(1, std::min(atoi(split_env), std::min(16, max_split)));
+  int pick = 1;
+  double pick_t = 0.9 * model(1);
+  for (int sp = 2; sp <= std::min<int64_t>(std::min(16, max_split), nk / 3); sp++) {
+    if ((double)sp * sums > (double)((size_t)256 << 20)) break;
+    const double t = model(sp);
+    if (t < pick_t) { pick = sp; pick_t = t; }
+  }
+  return pick;
+}
+}  // namespace
+
 int gemm_split(const GemmParams &p) {
   static const char *tile_env = getenv("TTS_GEMM_TILE");
   if (p.is_f32 || tile_env) return 1;
-  return choose_dma(p, 16).split;
+  const DmaChoice choice = choose_dma(p, 16);
+  return choice.tile ? choice.split : any_split(p, 16);
 }
+bool gemm_any_shape(const GemmParams &p) { return !p.is_f32 && !choose_dma(p, 1).tile; }
 size_t gemm_workspace_bytes(const GemmParams &p) { return p.split > 1 ? (size_t)p.split * p.M * p.N * std::max(1, p.batches) * sizeof(float) : 0; }
 
 // p.split: the most K slices p.partial has room for (what gemm_split(p) said, or fewer; 1: none).
@@ -814,24 +861,41 @@ hipError_t launch_gemm(const GemmParams &p, hipStream_t s, const char **name) {
   }
   // anything else: 128 x 128 x 64 tiles, two workgroups per CU (a 256 x 256 x 32 form of the same kernel measured behind it
   // at every size tried: 4096^3: 202 against 197 us; 4096 x 2048 x 2048: 112 against 56 us)
-  *name = "gemm_mfma_kernel<128x128x64>";
-  return p.is_bf16 ? launch_gemm_cfg<true, 2, 2, 64>(p, s) : launch_gemm_cfg<false, 2, 2, 64>(p, s);
+  GemmParams q = p;
+  q.split = tile_env || !p.partial ? 1 : any_split(p, std::max(1, p.split));
+  if (q.split == 1) {
+    *name = "gemm_mfma_kernel<128x128x64>";
+    return p.is_bf16 ? launch_gemm_any<true, false>(q, s) : launch_gemm_any<false, false>(q, s);
+  }
+  *name = "gemm_mfma_kernel<128x128x64>, K slices";
+  hipError_t e = launch_gemm_any_slices(q, s);
+  if (e != hipSuccess) return e;
+  const ReduceGrid g(q);
+  if (q.is_bf16) hipLaunchKernelGGL(gemm_splitk_reduce_any_kernel<true>, dim3(g.workgroups, std::max(1, q.batches)), dim3(256), 0, s, q, g.across, g.col_blocks);
+  else hipLaunchKernelGGL(gemm_splitk_reduce_any_kernel<false>, dim3(g.workgroups, std::max(1, q.batches)), dim3(256), 0, s, q, g.across, g.col_blocks);
+  return hipGetLastError();
 }
 
 int gemm_epilogue_kernel_index(const GemmParams &p) { return gemm_fast_path_ok(p) ? 0 : 1; }
 
-// Kernel 0: whole 256 x 256 x 32 tiles; 1: any shape in 128 x 128 x 64 tiles -- compiled from gemm_device.h plus the
-// epilogue functor at the first launch that needs it.
+// A launch in K slices only where the any-shape kernel (kernel 1 below) would run it whole.
+int gemm_epilogue_split(const GemmParams &p) { return gemm_epilogue_kernel_index(p) == 1 ? any_split(p, 16) : 1; }
+
+// Kernel 0: whole 256 x 256 x 32 tiles; 1: any shape in 128 x 128 x 64 tiles; 2: the sum of the K slices that the any-shape
+// kernel without a functor leaves (p.split > 1) -- compiled from gemm_device.h plus the epilogue functor at the first launch
+// that needs it.  A launch in slices also compiles the kernel it would be without, so that a later one of the same plan that
+// may not use a workspace finds it.
 hipError_t launch_gemm_epilogue(const GemmParams &p, const std::string &epilogue, RtcModule **modules, const GemmEpilogueArgs &ep,
                                 hipStream_t s, const char **name, std::string *err) {
-  static const char *names[2] = {"gemm_dma_kernel + epilogue (hipRTC)", "gemm_mfma_kernel<128x128x64> + epilogue (hipRTC)"};
-  const int which = gemm_epilogue_kernel_index(p);
-  const int64_t tile = which == 1 ? 128 : 256;
+  static const char *names[3] = {"gemm_dma_kernel + epilogue (hipRTC)", "gemm_mfma_kernel<128x128x64> + epilogue (hipRTC)",
+                                 "gemm_mfma_kernel<128x128x64> + epilogue (hipRTC), K slices"};
+  const int whole = gemm_epilogue_kernel_index(p), which = p.split > 1 ? 2 : whole;
   *name = names[which];
-  if (!modules[which]) {
-    const std::string source = epilogue + "#define TTS_GEMM_RTC " + std::to_string(which) + "\n#define TTS_GEMM_BF16 " + std::to_string(p.is_bf16 ? 1 : 0) +
+  for (int m : {whole, which}) {
+    if (modules[m]) continue;
+    const std::string source = epilogue + "#define TTS_GEMM_RTC " + std::to_string(m) + "\n#define TTS_GEMM_BF16 " + std::to_string(p.is_bf16 ? 1 : 0) +
                                "\n" + gemm_device_source();
-    hipError_t e = rtc_compile(source, "gemm_rtc", &modules[which], err);
+    hipError_t e = rtc_compile(source, "gemm_rtc", &modules[m], err);
     if (e != hipSuccess) {
       if (getenv("TTS_DUMP_RTC_SOURCE")) *err += "\n--- source ---\n" + source;
       return e;
@@ -839,13 +903,22 @@ hipError_t launch_gemm_epilogue(const GemmParams &p, const std::string &epilogue
   }
   struct {
     GemmParams p;
-    int tiles_m, tiles_n;
-    GemmEpilogueArgs ep;  // the functor: same layout as the generated struct TtsEp
+    int tiles_m, tiles_n;  // (kernel 2: columns a workgroup spans, blocks of them)
+    GemmEpilogueArgs ep;   // the functor: same layout as the generated struct TtsEp
   } a;
   a.p = p;
+  a.ep = ep;
+  if (which == 2) {
+    hipError_t e = launch_gemm_any_slices(p, s);
+    if (e != hipSuccess) return e;
+    const ReduceGrid g(p);
+    a.tiles_m = g.across;
+    a.tiles_n = g.col_blocks;
+    return rtc_launch(modules[2], g.workgroups, 1, 1, 256, &a, sizeof a, s);
+  }
+  const int64_t tile = which == 1 ? 128 : 256;
   a.tiles_m = (int)((p.M + tile - 1) / tile);
   a.tiles_n = (int)((p.N + tile - 1) / tile);
-  a.ep = ep;
   return rtc_launch(modules[which], a.tiles_m * a.tiles_n, 1, 1, 256, &a, sizeof a, s);
 }
 

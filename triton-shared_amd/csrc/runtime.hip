@@ -147,7 +147,7 @@ struct tts_plan {
   }
   RtcModule *fused = nullptr;  // the kernel compiled for this plan at its first launch (fused maps, tile programs)
   bool fused_is_plain = false; // a tile program whose source is persistent but whose kernel with a workgroup per program was kept
-  RtcModule *gemm_rtc[2] = {nullptr, nullptr};  // matrix products with a fused epilogue: one kernel per tiling
+  RtcModule *gemm_rtc[3] = {nullptr, nullptr, nullptr};  // matrix products with a fused epilogue: launch_gemm_epilogue's kernels
   RtcModule *fallback = nullptr;  // the generic family's kernel for a matrix-product plan (launches the product kernels decline)
   ~tts_plan() {
     for (auto &kv : split_k) {
@@ -925,8 +925,9 @@ tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, con
           // a product with too few tiles for the chip runs in K slices, whose partial sums need memory: the stream's
           // workspace (as for the int8-weight product), or the static array of the call that may not allocate, when
           // they fit there (else that call runs the product without slices)
+          // (the any-shape kernel keeps to whole products where the launch may not allocate or is recorded into a graph)
           const int want = gemm_split(p);
-          if (want > 1) {
+          if (want > 1 && !(gemm_any_shape(p) && (no_alloc || is_capturing(s)))) {
             p.split = want;
             const size_t need = gemm_workspace_bytes(p);
             if (no_alloc) {  // as many slices as the static array holds
@@ -966,6 +967,14 @@ tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, con
         }
         {
           std::lock_guard<std::mutex> lock(plan->mu);
+          const int want = gemm_epilogue_split(p);
+          if (want > 1 && !no_alloc && !is_capturing(s)) {
+            p.split = want;
+            tts_plan::SplitK &sk = plan->split_k[stream];
+            hipError_t e = plan->grow((void **)&sk.workspace, &sk.workspace_bytes, gemm_workspace_bytes(p));
+            if (e != hipSuccess) return fail(TTS_HIP_ERROR, std::string("hipMalloc(split-K workspace): ") + hipGetErrorString(e));
+            p.partial = sk.workspace;
+          }
           err = launch_gemm_epilogue(p, pl.source, plan->gemm_rtc, a, s, &kname, &why);
         }
         if (err != hipSuccess && !why.empty()) return fail(TTS_HIP_ERROR, "gemm epilogue: " + why);
