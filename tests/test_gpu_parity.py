@@ -657,6 +657,27 @@ def test_gemm_on_fp32_blocks(K, M, N, Kd, at, bt, BM, BN, BK):
     assert (c.cpu().double() - want).abs().max().item() <= 1e-3 and relfro(c.cpu(), want) <= 1e-5
 
 
+@pytest.mark.parametrize("M,N,Kd,at,bt", [(2, 3, 5, False, False), (33, 31, 16, False, False), (100, 65, 79, True, False), (16, 700, 1003, False, True), (1000, 999, 50, False, False),
+                                          (1030, 2000, 83, True, True), (1500, 1501, 65, False, True), (2900, 2999, 35, False, False)])
+def test_gemm_on_fp32_blocks_in_each_tile_size(K, M, N, Kd, at, bt):
+    # 32 x 32 tiles in four groups (down to fewer K tiles than groups), 64 x 64 in two and in one, 128 x 128; rows at every
+    # dword alignment, NaN between the rows; small integers are exact in any order
+    g = torch.Generator().manual_seed(M + Kd)
+    def operand(rows, cols, turned):
+        x = torch.randint(-4, 5, (rows, cols), generator=g).float()
+        full = torch.full((cols, rows + 1) if turned else (rows, cols + 1), float("nan"))
+        full[:, :-1] = x.t() if turned else x
+        d = full.to(DEV)[:, :-1]
+        return x, (d.t() if turned else d)
+    (a, ad), (b, bd) = operand(M, Kd, at), operand(Kd, N, bt)
+    cd = torch.full((M + 1, N + 1), 7.0, device=DEV)
+    k = K.matmul_tiles[(triton.cdiv(M, 32) * triton.cdiv(N, 64),)](ad, bd, cd, M, N, Kd, ad.stride(0), ad.stride(1), bd.stride(0), bd.stride(1), N + 1, 1, BM=32, BN=64, BK=16, GROUP_M=8)
+    torch.cuda.synchronize()
+    assert k.function.last_kernel == "gemm_f32_kernel"
+    assert torch.equal(cd[:M, :N].cpu(), a @ b)
+    assert (cd[M] == 7.0).all() and (cd[:, N] == 7.0).all()
+
+
 def test_gemm_with_column_major_a_and_with_strides_no_kernel_takes(K):
     torch.manual_seed(11)
     M, N, Kd = 300, 260, 136
