@@ -847,6 +847,22 @@ def test_matrix_program_attention(dtype, D, BM, BN, seq, pad, causal, k_columns)
     assert (lse[H] == 5.0).all() and (o[H] == 3.0).all() and (o[:, :, D:] == 3.0).all()
 
 
+@pytest.mark.parametrize("score", [torch.finfo(torch.float32).min, 2.6e38])
+def test_matrix_program_attention_scores_at_the_end_of_fp32(score):
+    # every score of a row is the same number (a finite mask on all keys, for one): the result is the mean of the values
+    import extra_kernels as X
+    torch.manual_seed(5)
+    H, seq, D, BM = 2, 130, 64, 64
+    q, k = torch.ones(H, seq, D, device=DEV, dtype=torch.float16), torch.ones(H, seq, D, device=DEV, dtype=torch.float16)
+    v = torch.randn(H, seq, D, device=DEV).half()
+    o = torch.zeros_like(v)
+    kern = X.attention_fwd[(triton.cdiv(seq, BM), H)](q, k, v, o, score / D, seq, seq * D, D, BM=BM, BN=64, D=D)
+    torch.cuda.synchronize()
+    assert kern.function.last_kernel == "tile_program (hipRTC, matrix layout)"
+    want = v.cpu().double().mean(1, keepdim=True).expand(H, seq, D)
+    assert (o.cpu().double() - want).abs().max().item() <= 2.0 ** -10 * want.abs().max().item()  # every probability is exact: one rounding
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("rows,BM,K,N,P,k_cols,turned", [(1, 32, 32, 32, 32, 32, False), (100, 64, 64, 128, 32, 50, True), (129, 128, 128, 64, 64, 128, False), (70, 32, 256, 32, 128, 200, True)])
 def test_matrix_program_chained_products(dtype, rows, BM, K, N, P, k_cols, turned):

@@ -18,7 +18,7 @@
 //     Blocks that stick out of their tensor or are not 16-byte aligned are staged through registers instead.
 // What the ordinary form of the family spends its time on -- operands, products and every reduced row going through LDS
 // element by element between some twenty barriers per iteration -- does not exist here: causal attention of 32 heads x
-// 4096 x 128 in bf16 (64 x 64 blocks) 12.4 ms -> 174 us, 790 TFLOP/s; 32 x 4096 x 64 in fp16, no mask, 2.7 ms -> 217 us.
+// 4096 x 128 in bf16 (64 x 64 blocks) 12.4 ms -> 171 us, 805 TFLOP/s; 32 x 4096 x 64 in fp16, no mask, 2.7 ms -> 217 us.
 // What bounds it: exponentials and the other elementwise work of the softmax, some nine vector instructions per score
 // (the exponential counts four), against 8 matrix-pipe cycles per score of a wavefront at D = 128; two workgroups per CU
 // (256 registers a lane) run their phases against each other, so that one's products hide the other's exponentials.
@@ -360,8 +360,9 @@ struct MmaGen : Gen {
     }
     return map_expr(s, a);
   }
-  // exp(x - m) with m the same along a row: exp2(x log2e - m log2e), one fma per element.  The
-  // rounding of m log2e is a factor common to all elements of the row that were taken with this m.
+  // exp(x - m) with m the same along a row, the difference written where it is read.  It is taken before the factor log2 e:
+  // with fma(x, log2e, -m log2e) a row of the type's lowest values (all keys masked with a finite number) is infinity minus
+  // infinity, and m log2e rounds by up to |m| 2^-24 of the exponent.
   bool exp_of_difference(const SOp &s, int role, std::string *text) {
     if (!fast_exp || role != TILE || val(s.result).dtype != "f32" || (s.name != "math.exp" && s.name != "math.exp2")) return false;
     const SOp *d = def_of(s.operands[0]);
@@ -371,7 +372,7 @@ struct MmaGen : Gen {
     const bool e2 = s.name == "math.exp2";
     const std::string x = el(d->operands[0], role), m = el(d->operands[1], role);
     if (e2) *text = "__builtin_amdgcn_exp2f(" + x + " - " + m + ")";
-    else *text = "__builtin_amdgcn_exp2f(fmaf(" + x + ", TTS_LOG2E, -(" + m + " * TTS_LOG2E)))";
+    else *text = "__builtin_amdgcn_exp2f((" + x + " - " + m + ") * TTS_LOG2E)";
     return true;
   }
   bool folded_into_exp(const SOp &s) const {  // a difference that only an exponential reads is written there
