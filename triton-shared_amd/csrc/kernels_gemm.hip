@@ -832,11 +832,18 @@ DmaChoice choose_dma(const GemmParams &p, int max_split) {
   // Among the tiles that give every CU a workgroup (128 x 128: always), the one with the least padded work per unit
   // of the tile's measured efficiency at 4096^3 (105 / 136 / 144 / 179 us): a ragged edge counts against a tile that
   // overshoots it by more.
+  // Rows with a weight matrix per block stream their weights from HBM, and the 128 x 256 tile's prefetching wavefront is ahead
+  // from half a workgroup per CU on (us with 128 x 128 / 128 x 256 tiles: 144 of the latter 65 / 58, 160 42.4 / 40.1, 192 57.8 /
+  // 50.8; below, 72 29.0 / 43.9, 28 16.4 / 19.6), but not where they make a second round that is mostly empty (288 73.3 / 79.1, 320
+  // 77.4 / 80.3, 336 74.0 / 78.2, 396 87.4 / 92.0; 504 31.5 / 30.4, 510 47.8 / 45.1; beyond two rounds they are even: 576 110 / 110,
+  // 800 210 / 210).  A few tiles over one round count as one: blocks of rows that pad the last matrix have nothing to do.
+  const bool grouped = p.b_block != nullptr && !p.b_trans;
+  auto grouped_wide = [&](int64_t t) { return 2 * t >= cus && !(10 * t > 11 * cus && 10 * t < 16 * cus); };
   DmaChoice best;
   double best_cost = 0;
   for (const DmaCand &c : DMA_CANDS) {
     if (!gemm_dma_ok(p, c.bm, c.bn)) continue;
-    if (dma_env ? std::string(dma_env) != c.tag : (tiles(c) < cus && c.bm + c.bn != 256)) continue;
+    if (dma_env ? std::string(dma_env) != c.tag : (c.bm + c.bn != 256 && (grouped ? !grouped_wide(tiles(c)) : tiles(c) < cus))) continue;
     const double cost = (double)(tiles(c) * c.bm * c.bn) / c.eff;
     if (!best.tile || cost < best_cost) { best.tile = &c; best_cost = cost; }
   }
