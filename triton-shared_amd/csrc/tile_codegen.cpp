@@ -841,7 +841,8 @@ struct Gen {
   }
   // The sums of a sliced program's workgroups: each leaves its own in `partial` (written through, complete before its
   // arrival is counted), and the one that arrives last adds all of them in slice order -- the result does not depend on
-  // who that is -- and goes on with the program.  Nobody waits for anybody.
+  // who that is -- and goes on with the program.  Nobody waits for anybody.  (The slices' sums are large next to what a
+  // thread of one workgroup adds up: added in fp32, db of LayerNorm on fp32 [3000, 1000] was 1.05e-7 off, 7.1e-8 in one slice.)
   void slices_meet() {
     int64_t total = 0;
     for (const SOp &s : slice_head)
@@ -867,10 +868,10 @@ struct Gen {
       if (s.kind == SK::Reduce) {
         const int64_t n = val(s.result).shape[0];
         os << pad() << "for (int c = threadIdx.x; c < " << n << "; c += 256) {\n"
-           << pad() << "  float sum = 0.f;\n" << pad() << "#pragma unroll 8\n"
+           << pad() << "  double sum = 0;\n" << pad() << "#pragma unroll 8\n"
            << pad() << "  for (int s = 0; s < slices; s++) sum += __hip_atomic_load(&partial[((long long)s * programs + lin) * " << total << " + " << off
            << " + c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);\n"
-           << pad() << "  " << at(s.result, "c", "0") << " = sum;\n" << pad() << "}\n";
+           << pad() << "  " << at(s.result, "c", "0") << " = (float)sum;\n" << pad() << "}\n";
         off += n;
       }
     os << pad() << "__syncthreads();\n";
