@@ -746,6 +746,31 @@ def test_w8a16_tiled_kernel(K, M, N, Kd):
         assert torch.equal(cd[:M].cpu(), want) and (cd[M] == 5.0).all()
 
 
+@pytest.mark.parametrize("M,N,Kd", [(33, 2048, 64), (300, 2064, 576), (17, 4096, 2048)])
+def test_w8a16_tiled_kernel_rounds_weights_as_the_program_does(K, M, N, Kd):
+    # w.to(f16) * scale is rounded to fp16 before the product.  Two terms of one column and opposite sign: their fp16 products
+    # differ by something fp32 holds exactly, and the result is that, rounded once.  Scales over all of fp16 (subnormal ones, zeros
+    # of both signs, the largest whose products stay finite), in the last columns also such as overflow, infinities and NaNs
+    g = torch.Generator().manual_seed(M + N)
+    a = torch.zeros(M, Kd, dtype=torch.float16)
+    rows = torch.arange(M)
+    a[rows, torch.randint(0, Kd // 2, (M,), generator=g)] = 1.0
+    a[rows, torch.randint(Kd // 2, Kd, (M,), generator=g)] = -1.0
+    w = torch.randint(-128, 128, (Kd, N), generator=g, dtype=torch.int8)
+    s = torch.randint(0, 0x6000, (N,), generator=g, dtype=torch.int16)
+    s[torch.rand(N, generator=g) < 0.2] &= 0x3ff
+    s = torch.where(torch.rand(N, generator=g) < 0.5, s, s | -0x8000).view(torch.float16)
+    s[:4] = torch.tensor([0.0, -0.0, 511.75, 2.0 ** -24])
+    s[-8:] = torch.tensor([512.0, -600.0, 65504.0, float("inf"), -float("inf"), float("nan"), 0.001, 2.0 ** -15])
+    cd = torch.full((M + 1, N), 5.0, dtype=torch.float16, device=DEV)
+    k = K.w8a16_matmul[(triton.cdiv(M, 64), triton.cdiv(N, 128))](a.to(DEV), w.to(DEV), s.to(DEV), cd, M, N, Kd, Kd, 1, N, 1, N, 1, BM=64, BN=128, BK=64)
+    torch.cuda.synchronize()
+    assert k.function.last_kernel == "gemm_w8a16_tile_kernel"
+    want = (a.double() @ (w.half() * s).double()).half()   # (0 x infinity is a NaN on both sides)
+    assert torch.equal(want.isnan(), cd[:M].cpu().isnan()) and (cd[M] == 5.0).all()
+    assert torch.equal(torch.nan_to_num(cd[:M].cpu(), nan=1.0), torch.nan_to_num(want, nan=1.0))
+
+
 @pytest.mark.parametrize("R,C,BR,BC", [(150, 700, 32, 256), (64, 64, 32, 32), (33, 1000, 8, 128), (40, 300, 16, 64)])
 def test_programs_keep_their_ids_when_the_launcher_swaps_the_grid(R, C, BR, BC):
     # a program whose stores are contiguous along the dimension program_id(1) walks is launched with the grid's x and y

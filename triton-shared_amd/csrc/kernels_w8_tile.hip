@@ -15,11 +15,13 @@
 //   W stage [64 k rows][256 bytes] of int8; position q of row k holds chunk q ^ (((k >> 3) & 3) << 2), so that the four
 //     k octets of a wavefront's dword reads fall into different banks.
 // A lane reads the dword of its four columns in each of its eight k rows (one octet of k per 16 lanes).  Column c of the four
-// gives one operand of the instruction: byte c of the eight dwords.  Widening two of them is v_perm and one v_pk_fma_f16: the
-// byte with its sign flipped, b + 128, is the fp16 subnormal (b + 128) 2^-24; times 2^15 minus 1/4 is b / 512, exactly.  The
-// columns' scales, times 512, multiply the fp32 sums instead of the weights: one rounding fewer than the source's fp16
-// product of weight and scale, and 40 vector instructions per step instead of 80 (two more per pair and a wait state: 155
-// against 135 us at 300 rows; with one wavefront per SIMD what the vector unit does is time the matrix pipe waits).
+// gives one operand of the instruction: byte c of the eight dwords.  The source multiplies the widened weight b by its
+// column's scale s in fp16, one rounding.  Here that is v_perm and one v_pk_fma_f16 per two weights: the byte with its sign
+// flipped, b + 128, is the fp16 subnormal (b + 128) 2^-24; with s = m 2^e, 1 <= |m| < 2, that times m 2^14 minus m / 8 is b m
+// 2^-10 rounded once, and b s has the same rounding at every scale up to 511.75 (its smallest value other than zero is normal
+// where s is; where s is subnormal, products below 2^-13 are exact).  The fp32 sums are multiplied by 2^(e + 10), exactly.  40
+// vector instructions per step where the byte widened first and multiplied after takes 72.  A workgroup that has a larger
+// scale (whose products may overflow), an infinite one or a NaN among its columns takes those four: widen, times 512, times s.
 // The weights go in as the first source, so a lane's results are sixteen neighbouring columns of one row (columns 16 q + 4 v +
 // c for result v of instruction c, q = lane / 16): two 16-byte stores per row and lane.
 // What bounds it at 300 rows: the matrix instructions alone take 101 us, widening and LDS reads add 12, the loads 23.  Eight
@@ -83,6 +85,27 @@ __global__ __launch_bounds__(256, 1) void gemm_w8a16_tile_kernel(GemmW8A16Params
     const int chunk = min((lane & 15) ^ (((krow >> 3) & 3) << 2), (int)((p.N - n0) / 16 - 1));
     w_voff[i] = (uint32_t)(krow * p.ldw + 16 * chunk);
   });
+  // the scales of the columns a lane widens and of those it holds results of, and whether any of the workgroup's columns has
+  // one that needs the source's two steps (columns past N: some other column's)
+  uint16_t s_in[4], s_out[16], s_any[4];
+  const uint16_t *scales = (const uint16_t *)p.scale;
+  __builtin_memcpy(s_in, scales + min(n0 + 64 * (int)wave + 4 * l16, p.N - 4), 8);
+  __builtin_memcpy(s_any, scales + min(n0 + 4 * lane, p.N - 4), 8);
+  __builtin_memcpy(s_out, scales + min(n0 + 64 * (int)wave + 16 * q, p.N - 16), 32);
+  const bool literal = __builtin_amdgcn_ballot_w64(max(max(s_any[0] & 0x7fff, s_any[1] & 0x7fff), max(s_any[2] & 0x7fff, s_any[3] & 0x7fff)) > 0x5fff) != 0;
+  // s = m 2^e, 1 <= |m| < 2 (m = s, e = 0 for zeros; of no use for the scales above 0x5fff)
+  auto mantissa = [](uint16_t h) __attribute__((always_inline)) { return 2.f * __builtin_amdgcn_frexp_mantf((float)__builtin_bit_cast(_Float16, h)); };
+  auto power = [](uint16_t h) __attribute__((always_inline)) {  // 2^(e + 10)
+    return __builtin_amdgcn_ldexpf(1.f, __builtin_amdgcn_frexp_expf((float)__builtin_bit_cast(_Float16, h)) + 9);
+  };
+  uint32_t times[4], minus[4];  // per column, in both halves: what the subnormal is multiplied by and what is added; literal: the scale
+  static_for<0, 4>([&](auto cc) __attribute__((always_inline)) {
+    constexpr int c = decltype(cc)::value;
+    const float m = mantissa(s_in[c]);
+    const _Float16 t = literal ? __builtin_bit_cast(_Float16, s_in[c]) : (_Float16)(m * 16384.f), o = (_Float16)(m * -0.125f);
+    times[c] = (uint32_t)__builtin_bit_cast(uint16_t, t) * 0x10001u;
+    minus[c] = (uint32_t)__builtin_bit_cast(uint16_t, o) * 0x10001u;
+  });
   const char *a_base = (const char *)((const uint16_t *)p.a + m0 * p.lda);
   const char *w_base = (const char *)p.w + n0;
   const uint32_t lds0 = (uint32_t)(uintptr_t)TTS_LDS(smem);
@@ -113,11 +136,19 @@ __global__ __launch_bounds__(256, 1) void gemm_w8a16_tile_kernel(GemmW8A16Params
     raw[j] = *reinterpret_cast<const uint32_t *>(smem + stage * T::STAGE + w_off + (32 * s + j) * W8T_COLS);
   };
   auto bias_w = [&](int j) __attribute__((always_inline)) { raw[j] ^= 0x80808080u; };  // bytes b + 128
-  auto widen = [&](int c, int tp, uint32_t (&b)[4][4]) __attribute__((always_inline)) {  // k 2 tp and 2 tp + 1 of column c
+  auto widen = [&](auto lit, int c, int tp, uint32_t (&b)[4][4]) __attribute__((always_inline)) {  // k 2 tp and 2 tp + 1 of column c
     const uint32_t sel = 0x0c000c00u | (uint32_t)c | ((uint32_t)(4 + c) << 16);
     const f16x2 v = __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(raw[2 * tp + 1], raw[2 * tp], sel));
-    const f16x2 up = {(_Float16)32768.0f, (_Float16)32768.0f}, off = {(_Float16)-0.25f, (_Float16)-0.25f};
-    b[c][tp] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(v, up, off));
+    const f16x2 t = __builtin_bit_cast(f16x2, times[c]), o = __builtin_bit_cast(f16x2, minus[c]);
+    f16x2 w;
+    if constexpr (decltype(lit)::value) {
+      const f16x2 up = {(_Float16)32768.0f, (_Float16)32768.0f}, off = {(_Float16)-0.25f, (_Float16)-0.25f}, whole = {(_Float16)512.0f, (_Float16)512.0f};
+      w = __builtin_elementwise_fma(v, up, off) * whole;  // b, exactly
+      w = w * t;
+    } else {
+      w = __builtin_elementwise_fma(v, t, o);
+    }
+    b[c][tp] = __builtin_bit_cast(uint32_t, w);
   };
   // The matrix instruction from inline assembly, in place on the accumulation registers (see gemm_dma16_body).  The
   // compiler inserts no wait states in front of it: its operands are read from LDS or widened a phase earlier.
@@ -127,7 +158,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w8a16_tile_kernel(GemmW8A16Params
   };
   // One step: its 4 TM products, with the reads and the widening of the next step (step ns of the tile at stage `next`)
   // dealt out behind them; LOAD: and the loads of tile t into `free`.
-  auto step = [&](auto load, int next, auto nsc, int t, int free, uint4 (&Ac)[TM], uint4 (&An)[TM], uint32_t (&Bc)[4][4], uint32_t (&Bn)[4][4]) __attribute__((always_inline)) {
+  auto step = [&](auto lit, auto load, int next, auto nsc, int t, int free, uint4 (&Ac)[TM], uint4 (&An)[TM], uint32_t (&Bc)[4][4], uint32_t (&Bn)[4][4]) __attribute__((always_inline)) {
     constexpr int ns = decltype(nsc)::value;
     static_for<0, 4 * TM>([&](auto slot) __attribute__((always_inline)) {
       constexpr int n = decltype(slot)::value;
@@ -144,7 +175,7 @@ __global__ __launch_bounds__(256, 1) void gemm_w8a16_tile_kernel(GemmW8A16Params
       if constexpr (n >= W0 && n < W0 + WN)
         static_for<(n - W0) * 24 / WN, (n - W0 + 1) * 24 / WN>([&](auto g) __attribute__((always_inline)) {
           if constexpr (g.value < 8) bias_w(g.value);
-          else widen((g.value - 8) / 4, g.value % 4, Bn);
+          else widen(lit, (g.value - 8) / 4, g.value % 4, Bn);
         });
     });
     __builtin_amdgcn_sched_barrier(0);
@@ -157,18 +188,22 @@ __global__ __launch_bounds__(256, 1) void gemm_w8a16_tile_kernel(GemmW8A16Params
   static_for<0, 8>([&](auto j) __attribute__((always_inline)) { read_w(0, 0, j.value); });
   static_for<0, TM>([&](auto i) __attribute__((always_inline)) { read_a(0, 0, i.value, A[0]); });
   static_for<0, 8>([&](auto j) __attribute__((always_inline)) { bias_w(j.value); });
-  static_for<0, 16>([&](auto g) __attribute__((always_inline)) { widen(g.value / 4, g.value % 4, B[0]); });
-  __builtin_amdgcn_sched_barrier(0);
-  int stage = 0;
-  for (int t = 0; t < nk; t++) {
-    const int next = stage + 1 == STAGES ? 0 : stage + 1;
-    step(BoolConstant<false>(), stage, IntConstant<1>(), 0, 0, A[0], A[1], B[0], B[1]);
-    // own loads of tile t + 1 have landed, own reads of tile t are complete: behind the barrier its stage is free
-    __builtin_amdgcn_s_waitcnt(waitcnt_imm(T::DMA * (STAGES - 2), 0));
-    __syncthreads();
-    step(BoolConstant<true>(), next, IntConstant<0>(), t + STAGES, stage, A[1], A[0], B[1], B[0]);
-    stage = next;
-  }
+  auto sweep_k = [&](auto lit) __attribute__((always_inline)) {
+    static_for<0, 16>([&](auto g) __attribute__((always_inline)) { widen(lit, g.value / 4, g.value % 4, B[0]); });
+    __builtin_amdgcn_sched_barrier(0);
+    int stage = 0;
+    for (int t = 0; t < nk; t++) {
+      const int next = stage + 1 == STAGES ? 0 : stage + 1;
+      step(lit, BoolConstant<false>(), stage, IntConstant<1>(), 0, 0, A[0], A[1], B[0], B[1]);
+      // own loads of tile t + 1 have landed, own reads of tile t are complete: behind the barrier its stage is free
+      __builtin_amdgcn_s_waitcnt(waitcnt_imm(T::DMA * (STAGES - 2), 0));
+      __syncthreads();
+      step(lit, BoolConstant<true>(), next, IntConstant<0>(), t + STAGES, stage, A[1], A[0], B[1], B[0]);
+      stage = next;
+    }
+  };
+  if (literal) sweep_k(BoolConstant<true>());
+  else sweep_k(BoolConstant<false>());
   // wait states between the last matrix instructions and the first read of their results (see gemm_dma16_body)
   asm volatile("s_nop 15\n\ts_nop 15" : : : "memory");
   auto settle = [](f32x4 &x) __attribute__((always_inline)) { asm volatile("" : "+a"(x) : : "memory"); };
@@ -179,11 +214,10 @@ __global__ __launch_bounds__(256, 1) void gemm_w8a16_tile_kernel(GemmW8A16Params
   typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
   const int64_t col = n0 + 64 * (int)wave + 16 * q;
   const bool col_in = col < p.N;  // (N is a multiple of 16)
-  // The columns' scales, applied to the sums: the widened weights are b / 512, exactly.
   static_for<0, 4>([&](auto vc) __attribute__((always_inline)) {
     static_for<0, 4>([&](auto cc) __attribute__((always_inline)) {
       constexpr int v = decltype(vc)::value, c = decltype(cc)::value;
-      const float scale = 512.f * (float)((const _Float16 *)p.scale)[min(col, p.N - 16) + 4 * v + c];
+      const float scale = literal ? 1.f : power(s_out[4 * v + c]);
       static_for<0, TM>([&](auto i) __attribute__((always_inline)) { acc[i.value][c][v] *= scale; });
     });
   });
