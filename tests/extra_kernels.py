@@ -1395,3 +1395,55 @@ def column_moments(x_ptr, s_ptr, out_ptr, n_rows, n_cols, pitch, BR: tl.constexp
     tl.store(out_ptr + c, sa, mask=c < n_cols)
     tl.store(out_ptr + n_cols + c, sb, mask=c < n_cols)
     tl.store(out_ptr + 2 * n_cols + c, sa - 2.0 * sb, mask=c < n_cols)
+
+
+@triton.jit
+def attention_on_three_axes(Q, K, V, O, sm_scale, seq, blocks, heads, window, stride_b, stride_h, stride_s, BM: tl.constexpr, BN: tl.constexpr, D: tl.constexpr, FORM: tl.constexpr):
+    # attention on a grid with three axes whose key blocks depend on all of them.  FORM 0: a causal window, the loop's start
+    # depends on the query block; 1: causal in two stages, the blocks below the diagonal and those on it; 2: no mask, one flat
+    # program number over the whole grid
+    if FORM == 2:
+        flat = tl.program_id(0) + tl.num_programs(0) * (tl.program_id(1) + tl.num_programs(1) * tl.program_id(2))
+        pm = flat % blocks
+        ph = flat // blocks % heads
+        pb = flat // (blocks * heads)
+    else:
+        pm = tl.program_id(0)
+        ph = tl.program_id(1)
+        pb = tl.program_id(2)
+    base = pb * stride_b + ph * stride_h
+    rm = pm * BM + tl.arange(0, BM)
+    rd = tl.arange(0, D)
+    q = tl.load(Q + base + rm[:, None] * stride_s + rd[None, :], mask=rm[:, None] < seq, other=0.0)
+    m_i = tl.zeros([BM], dtype=tl.float32) - 1.0e30
+    l_i = tl.zeros([BM], dtype=tl.float32)
+    acc = tl.zeros([BM, D], dtype=tl.float32)
+    for stage in tl.static_range(2 if FORM == 1 else 1):
+        if FORM == 0:
+            lo = tl.maximum(pm * BM - window, 0) // BN * BN
+            hi = tl.minimum((pm + 1) * BM, seq)
+        elif FORM == 1:
+            lo = stage * (pm * BM // BN * BN)
+            hi = pm * BM // BN * BN if stage == 0 else tl.minimum((pm + 1) * BM, seq)
+        else:
+            lo = flat - flat
+            hi = seq
+        for start in range(lo, hi, BN):
+            rn = start + tl.arange(0, BN)
+            k = tl.load(K + base + rn[:, None] * stride_s + rd[None, :], mask=rn[:, None] < seq, other=0.0)
+            v = tl.load(V + base + rn[:, None] * stride_s + rd[None, :], mask=rn[:, None] < seq, other=0.0)
+            qk = tl.dot(q, tl.trans(k)) * sm_scale
+            ok = rn[None, :] < seq
+            if FORM == 0:
+                ok = ok & (rm[:, None] >= rn[None, :]) & (rm[:, None] - rn[None, :] < window)
+            if FORM == 1:
+                ok = ok & (rm[:, None] >= rn[None, :])
+            qk = tl.where(ok, qk, -1.0e30)
+            m_new = tl.maximum(m_i, tl.max(qk, axis=1))
+            p = tl.where(ok, tl.exp(qk - m_new[:, None]), 0.0)
+            alpha = tl.exp(m_i - m_new)
+            l_i = l_i * alpha + tl.sum(p, axis=1)
+            acc = acc * alpha[:, None] + tl.dot(p.to(V.dtype.element_ty), v)
+            m_i = m_new
+    acc = acc / l_i[:, None]
+    tl.store(O + base + rm[:, None] * stride_s + rd[None, :], acc.to(O.dtype.element_ty), mask=rm[:, None] < seq)

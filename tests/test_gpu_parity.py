@@ -888,6 +888,29 @@ def test_matrix_program_attention_scores_at_the_end_of_fp32(score):
     assert (o.cpu().double() - want).abs().max().item() <= 2.0 ** -10 * want.abs().max().item()  # every probability is exact: one rounding
 
 
+@pytest.mark.parametrize("form", [0, 1, 2])
+@pytest.mark.parametrize("BM,BN,D,seq", [(32, 32, 64, 150), (64, 64, 64, 200), (64, 32, 128, 65), (128, 64, 64, 300)])
+def test_matrix_program_attention_on_a_grid_with_no_free_axis(form, BM, BN, D, seq):
+    # (block, head, batch) grids whose key blocks depend on every axis: a workgroup holds one program, of 32, 64 or 128 rows
+    import extra_kernels as X
+    torch.manual_seed(seq + form)
+    batch, heads, window = 2, 3, 50
+    q, k, v = (torch.randn(batch, heads, seq, D, device=DEV).half() for _ in range(3))
+    o = torch.full((batch + 1, heads, seq, D), 3.0, device=DEV, dtype=torch.float16)
+    blocks = triton.cdiv(seq, BM)
+    kern = X.attention_on_three_axes[(blocks, heads, batch)](q, k, v, o, D ** -0.5, seq, blocks, heads, window, q.stride(0), q.stride(1), q.stride(2), BM=BM, BN=BN, D=D, FORM=form)
+    torch.cuda.synchronize()
+    assert kern.function.last_kernel == "tile_program (hipRTC, matrix layout)"
+    s = torch.matmul(q.cpu().double(), k.cpu().double().transpose(2, 3)) * D ** -0.5
+    i, j = torch.arange(seq)[:, None], torch.arange(seq)[None, :]
+    if form < 2:
+        s.masked_fill_((j > i) | (i - j >= (window if form == 0 else seq)), -float("inf"))
+    want = torch.matmul(torch.softmax(s, -1), v.cpu().double())
+    # probabilities and results are each rounded once to 16 bits: half an ulp of |v| and of |o| <= max |v|
+    assert (o[:batch].cpu().double() - want).abs().max().item() <= 2.0 ** -10 * v.abs().max().item()
+    assert (o[batch] == 3.0).all()
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("rows,BM,K,N,P,k_cols,turned", [(1, 32, 32, 32, 32, 32, False), (100, 64, 64, 128, 32, 50, True), (129, 128, 128, 64, 64, 128, False), (70, 32, 256, 32, 128, 200, True)])
 def test_matrix_program_chained_products(dtype, rows, BM, K, N, P, k_cols, turned):

@@ -627,3 +627,20 @@ def test_loops_end_with_a_barrier_behind_what_an_iteration_staged(native, tmp_pa
     assert "blk" in loop
     behind = loop[loop.rindex("blk"):]
     assert "__syncthreads();" in behind, behind
+
+
+@pytest.mark.parametrize("form", [0, 1, 2])
+@pytest.mark.parametrize("BM", [32, 64])
+def test_matrix_programs_walk_their_loops_with_every_wavefront(native, tmp_path, form, BM):
+    """All four wavefronts of a workgroup copy a share of every staged block and meet at its barrier.  On a grid whose staged
+    blocks depend on every axis, a program of fewer rows leaves some of them without rows: how far the loop goes must not
+    depend on having any."""
+    import extra_kernels as X
+    sig = {**{x: "*fp16" for x in "QKVO"}, "sm_scale": "fp32", **{x: "i32" for x in ("seq", "blocks", "heads", "window", "stride_b", "stride_h", "stride_s")},
+           **{x: "constexpr" for x in ("BM", "BN", "D", "FORM")}}
+    src = _generic_source(tmp_path, compile_ttir(X.attention_on_three_axes, sig, {"BM": BM, "BN": 32, "D": 64, "FORM": form}))
+    assert src.startswith("// tts: matrix 1 -1 256"), src[:40]
+    ends = re.findall(r"long long last(\d) = (.*);", src)
+    assert len(ends) == (2 if form == 1 else 1)
+    for loop, end in ends:
+        assert not re.search(r"\b(mine|ub%s|wave)\b" % loop, end), end

@@ -911,7 +911,8 @@ struct MmaGen : Gen {
       line("  (void)own;");
       line("}");
     } else {
-      line("const long long last" + L + " = ub" + L + ";");
+      // (every wavefront stages this program's blocks and meets its barriers, also one that has no rows of it)
+      line("const long long last" + L + " = " + ex(s.ub) + ";");
     }
     auto stage_all = [&](const std::string &buf) {
       for (auto &im : images)
