@@ -1447,3 +1447,22 @@ def attention_on_three_axes(Q, K, V, O, sm_scale, seq, blocks, heads, window, st
             m_i = m_new
     acc = acc / l_i[:, None]
     tl.store(O + base + rm[:, None] * stride_s + rd[None, :], acc.to(O.dtype.element_ty), mask=rm[:, None] < seq)
+
+
+@triton.jit
+def causal_product_sums(q_ptr, k_ptr, r_ptr, out_ptr, n, K: tl.constexpr, BM: tl.constexpr, BN: tl.constexpr):
+    # out[i, j] = the sum of q[i] . k[j + BN t] over the key blocks t up to the row block's end, plus r[trips, i]: a pointer moved
+    # once per block and read after the loop, whose length depends on the program
+    pm = tl.program_id(0)
+    rm = pm * BM + tl.arange(0, BM)
+    rk = tl.arange(0, K)
+    q = tl.load(q_ptr + rm[:, None] * K + rk[None, :], mask=rm[:, None] < n, other=0.0)
+    acc = tl.zeros([BM, BN], dtype=tl.float32)
+    pr = r_ptr + rm
+    for start in range(0, (pm + 1) * BM, BN):
+        rn = start + tl.arange(0, BN)
+        k = tl.load(k_ptr + rn[:, None] * K + rk[None, :], mask=rn[:, None] < n, other=0.0)
+        acc += tl.dot(q, tl.trans(k))
+        pr += n
+    r = tl.load(pr, mask=rm < n, other=0.0)
+    tl.store(out_ptr + rm[:, None] * BN + tl.arange(0, BN)[None, :], acc + r[:, None], mask=rm[:, None] < n)

@@ -911,6 +911,23 @@ def test_matrix_program_attention_on_a_grid_with_no_free_axis(form, BM, BN, D, s
     assert (o[batch] == 3.0).all()
 
 
+@pytest.mark.parametrize("BM,BN,n", [(32, 32, 300), (64, 32, 129), (64, 64, 64), (128, 32, 257)])
+def test_matrix_program_pointer_carried_out_of_a_loop(BM, BN, n):
+    # programs that share a workgroup have loops of different lengths; small integers: exact
+    import extra_kernels as X
+    g = torch.Generator().manual_seed(n)
+    q, k = (torch.randint(-2, 3, (n, 64), generator=g).half() for _ in range(2))
+    trips = [(i // BM + 1) * BM // BN for i in range(n)]
+    r = torch.randint(-1000, 1000, (max(trips) + 1, n), generator=g).float()
+    out = torch.full((n + 1, BN), 7.0, device=DEV)
+    kern = X.causal_product_sums[(triton.cdiv(n, BM),)](q.to(DEV), k.to(DEV), r.to(DEV), out, n, K=64, BM=BM, BN=BN)
+    torch.cuda.synchronize()
+    assert kern.function.last_kernel == "tile_program (hipRTC, matrix layout)"
+    padded = torch.nn.functional.pad(q.double() @ k.double().t(), (0, max(trips) * BN - n)).view(n, -1, BN)
+    want = torch.stack([padded[i, :trips[i]].sum(0) + r[trips[i], i].double() for i in range(n)])
+    assert torch.equal(out[:n].cpu().double(), want) and (out[n] == 7.0).all()
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("rows,BM,K,N,P,k_cols,turned", [(1, 32, 32, 32, 32, 32, False), (100, 64, 64, 128, 32, 50, True), (129, 128, 128, 64, 64, 128, False), (70, 32, 256, 32, 128, 200, True)])
 def test_matrix_program_chained_products(dtype, rows, BM, K, N, P, k_cols, turned):

@@ -644,3 +644,20 @@ def test_matrix_programs_walk_their_loops_with_every_wavefront(native, tmp_path,
     assert len(ends) == (2 if form == 1 else 1)
     for loop, end in ends:
         assert not re.search(r"\b(mine|ub%s|wave)\b" % loop, end), end
+
+
+def test_matrix_programs_that_share_a_workgroup_carry_their_own_integers_out_of_a_loop(native, tmp_path):
+    """Programs of one workgroup turn together as often as the one with the longest loop; a pointer that a shorter one moves in
+    the loop and reads after it has moved as often as its own loop is long."""
+    import extra_kernels as X
+    sig = {"q_ptr": "*fp16", "k_ptr": "*fp16", "r_ptr": "*fp32", "out_ptr": "*fp32", "n": "i32", "K": "constexpr", "BM": "constexpr", "BN": "constexpr"}
+    src = _generic_source(tmp_path, compile_ttir(X.causal_product_sums, sig, {"K": 64, "BM": 64, "BN": 32}))
+    assert src.startswith("// tts: matrix 2 0 256"), src[:40]
+    used = set(re.findall(r"\bres0_(\d)\b(?!; \(void)", src.split("const long long res0_0")[1]))
+    assert used
+    guard = src.index("if (iv0 < ub0) {")
+    for q in used:
+        held = re.search(r"const long long res0_%s = (\w+);" % q, src).group(1)
+        moved = [m.start() for m in re.finditer(r"(?<!long )\b%s = " % held, src)]
+        after = src.index("iv0 = next_iv0;", guard)      # the first statement behind what only the program's own iterations do
+        assert moved and all(guard < m < after for m in moved), (held, moved)

@@ -897,6 +897,10 @@ struct MmaGen : Gen {
       }
     }
     for (size_t q = 0; q < s.int_iters.size(); q++) line("long long it" + L + "_" + std::to_string(q) + " = " + ex(s.int_iters[q].init) + ";");
+    // Programs that share a workgroup turn together as often as the furthest of them: what one whose loop ends earlier carries
+    // out of it is what it had there.
+    const bool shared = G > 1;
+    if (shared) for (size_t q = 0; q < s.int_iters.size(); q++) line("long long own" + L + "_" + std::to_string(q) + " = it" + L + "_" + std::to_string(q) + ";");
     bool staged = false;
     for (auto &im : images) staged = staged || im.second.loop == s.loop;
     const std::string iv = "iv" + L;
@@ -977,6 +981,7 @@ struct MmaGen : Gen {
       if (r & TILE) tile_loop(a, tile_of[a] + "[rb][nb][i] = " + n + "[rb][nb][i];");
       if (r & ROW) row_loop(row_of[a] + "[rb] = " + n + "r[rb];");
     }
+    if (shared) for (size_t q = 0; q < s.int_iters.size(); q++) line("own" + L + "_" + std::to_string(q) + " = next" + L + "_" + std::to_string(q) + ";");
     tile_of = saved_t;
     row_of = saved_r;
     col_of = saved_c;
@@ -986,7 +991,7 @@ struct MmaGen : Gen {
     for (size_t q = 0; q < s.int_iters.size(); q++) line("it" + L + "_" + std::to_string(q) + " = next" + L + "_" + std::to_string(q) + ";");
     indent--;
     line("}");
-    for (size_t q = 0; q < s.int_iters.size(); q++) line("const long long res" + L + "_" + std::to_string(q) + " = it" + L + "_" + std::to_string(q) + "; (void)res" + L + "_" + std::to_string(q) + ";");
+    for (size_t q = 0; q < s.int_iters.size(); q++) line("const long long res" + L + "_" + std::to_string(q) + " = " + (shared ? "own" : "it") + L + "_" + std::to_string(q) + "; (void)res" + L + "_" + std::to_string(q) + ";");
     for (size_t q = 0; q < s.tile_args.size(); q++) {
       const int a = s.tile_args[q], res = s.results[q];
       if (res < 0) continue;
