@@ -1466,3 +1466,27 @@ def causal_product_sums(q_ptr, k_ptr, r_ptr, out_ptr, n, K: tl.constexpr, BM: tl
         pr += n
     r = tl.load(pr, mask=rm < n, other=0.0)
     tl.store(out_ptr + rm[:, None] * BN + tl.arange(0, BN)[None, :], acc + r[:, None], mask=rm[:, None] < n)
+
+
+@triton.jit
+def product_sums_in_two_loops(q_ptr, k_ptr, h_ptr, out_ptr, n, m, K: tl.constexpr, BM: tl.constexpr, BN: tl.constexpr, CAUSAL: tl.constexpr):
+    # the sums of q[i] . k[j + BN t] over the key blocks, and of q[i] . h[j + BN t] over as many blocks as the first loop counted
+    pm = tl.program_id(0)
+    rm = pm * BM + tl.arange(0, BM)
+    rk = tl.arange(0, K)
+    q = tl.load(q_ptr + rm[:, None] * K + rk[None, :], mask=rm[:, None] < n, other=0.0)
+    acc = tl.zeros([BM, BN], dtype=tl.float32)
+    done = pm - pm
+    last = n
+    if CAUSAL:
+        last = (pm + 1) * BM
+    for start in range(0, last, BN):
+        rn = start + tl.arange(0, BN)
+        k = tl.load(k_ptr + rn[:, None] * K + rk[None, :], mask=rn[:, None] < n, other=0.0)
+        acc += tl.dot(q, tl.trans(k))
+        done += BN
+    for start in range(0, done, BN):
+        rn = start + tl.arange(0, BN)
+        h = tl.load(h_ptr + rn[:, None] * K + rk[None, :], mask=rn[:, None] < m, other=0.0)
+        acc += tl.dot(q, tl.trans(h))
+    tl.store(out_ptr + rm[:, None] * BN + tl.arange(0, BN)[None, :], acc, mask=rm[:, None] < n)

@@ -928,6 +928,25 @@ def test_matrix_program_pointer_carried_out_of_a_loop(BM, BN, n):
     assert torch.equal(out[:n].cpu().double(), want) and (out[n] == 7.0).all()
 
 
+@pytest.mark.parametrize("BM,BN,n,m,causal", [(32, 32, 300, 290, True), (64, 32, 129, 500, True), (64, 64, 64, 10, False), (128, 32, 257, 128, True)])
+def test_matrix_program_loop_as_long_as_another_counted(BM, BN, n, m, causal):
+    import extra_kernels as X
+    g = torch.Generator().manual_seed(n)
+    q, k, h = (torch.randint(-2, 3, (rows, 64), generator=g).half() for rows in (n, n, m))
+    out = torch.full((n + 1, BN), 7.0, device=DEV)
+    kern = X.product_sums_in_two_loops[(triton.cdiv(n, BM),)](q.to(DEV), k.to(DEV), h.to(DEV), out, n, m, K=64, BM=BM, BN=BN, CAUSAL=causal)
+    torch.cuda.synchronize()
+    assert kern.function.last_kernel == "tile_program (hipRTC, matrix layout)"
+    want = torch.zeros(n, BN, dtype=torch.float64)
+    for i in range(n):
+        trips = triton.cdiv((i // BM + 1) * BM if causal else n, BN)
+        for keys in (k, h):
+            block = torch.zeros(trips * BN, 64, dtype=torch.float64)
+            block[:min(trips * BN, len(keys))] = keys[:trips * BN].double()
+            want[i] += block.view(trips, BN, 64).sum(0) @ q[i].double()
+    assert torch.equal(out[:n].cpu().double(), want) and (out[n] == 7.0).all()
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("rows,BM,K,N,P,k_cols,turned", [(1, 32, 32, 32, 32, 32, False), (100, 64, 64, 128, 32, 50, True), (129, 128, 128, 64, 64, 128, False), (70, 32, 256, 32, 128, 200, True)])
 def test_matrix_program_chained_products(dtype, rows, BM, K, N, P, k_cols, turned):

@@ -661,3 +661,18 @@ def test_matrix_programs_that_share_a_workgroup_carry_their_own_integers_out_of_
         moved = [m.start() for m in re.finditer(r"(?<!long )\b%s = " % held, src)]
         after = src.index("iv0 = next_iv0;", guard)      # the first statement behind what only the program's own iterations do
         assert moved and all(guard < m < after for m in moved), (held, moved)
+
+
+@pytest.mark.parametrize("BM", [32, 64, 128])
+@pytest.mark.parametrize("causal", [False, True])
+def test_matrix_programs_name_what_a_loop_leaves_behind_only_after_it(native, tmp_path, BM, causal):
+    """The second loop is as long as the first one counted: nothing above the first loop can name that, and no program of the
+    workgroup knows it for another."""
+    import extra_kernels as X
+    sig = {"q_ptr": "*fp16", "k_ptr": "*fp16", "h_ptr": "*fp16", "out_ptr": "*fp32", "n": "i32", "m": "i32", **{x: "constexpr" for x in ("K", "BM", "BN", "CAUSAL")}}
+    src = _generic_source(tmp_path, compile_ttir(X.product_sums_in_two_loops, sig, {"K": 64, "BM": BM, "BN": 32, "CAUSAL": causal}))
+    assert src.startswith("// tts: matrix 1 -1 256"), src[:40]
+    for q in set(re.findall(r"\bres0_(\d)\b", src)):
+        declared = src.index("const long long res0_%s = " % q)
+        assert not re.search(r"\bres0_%s\b" % q, src[:declared])
+    assert re.search(r"long long last1 = .*\bres0_\d\b", src)

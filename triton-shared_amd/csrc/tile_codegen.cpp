@@ -2475,7 +2475,7 @@ std::string matrix_program_source(const Program &p) {
       << "  else { other = blockIdx.x % others; group = blockIdx.x / others; }\n"
       << "  const long long " << PD[b1] << " = other % (unsigned)" << NP[b1] << ", " << PD[b2] << " = other / (unsigned)" << NP[b1] << ";\n";
   for (const SOp &s : p.body)
-    if (s.kind == SK::For && g.expr_uses_pid(s.ub, ax)) {
+    if (s.kind == SK::For && g.expr_uses_pid(s.ub, ax) && !p.pool.depends_on(s.ub, EK::Result)) {  // (nothing of the program has run here)
       all << "  {\n    auto end = [&](long long " << PD[ax] << ") { (void)" << PD[ax] << "; return " << g.ex(s.ub) << "; };\n"
           << "    if (end(" << NP[ax] << " - 1) > end(0)) group = groups - 1 - group;\n  }\n";
       break;

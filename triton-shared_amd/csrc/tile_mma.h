@@ -285,7 +285,15 @@ struct MmaGen : Gen {
     wpp = (int)(BM / (32 * R));
     G = 1;
     axis = -1;
-    for (int ax = 0; ax < 3 && wpp < WAVES && axis < 0; ax++) {
+    // (a loop whose bounds another loop leaves behind: one program's value says nothing about another's, so none is shared)
+    bool known = true;
+    for (const SOp &s : P.body)
+      if (s.kind == SK::For)
+        for (int e : {s.lb, s.ub, s.step}) {
+          if (mentions(P.pool, e, EK::Data)) decline("a loop bound that is data");
+          known = known && !mentions(P.pool, e, EK::Result);
+        }
+    for (int ax = 0; ax < 3 && wpp < WAVES && axis < 0 && known; ax++) {
       bool free = true;
       for (auto &im : images) {
         const Access &a = def_of(im.first)->acc;
