@@ -1490,3 +1490,21 @@ def product_sums_in_two_loops(q_ptr, k_ptr, h_ptr, out_ptr, n, m, K: tl.constexp
         h = tl.load(h_ptr + rn[:, None] * K + rk[None, :], mask=rn[:, None] < m, other=0.0)
         acc += tl.dot(q, tl.trans(h))
     tl.store(out_ptr + rm[:, None] * BN + tl.arange(0, BN)[None, :], acc, mask=rm[:, None] < n)
+
+
+@triton.jit
+def product_with_one_element_vectors(a_ptr, b_ptr, s_ptr, out_ptr, n, n_s, K: tl.constexpr, BM: tl.constexpr, N: tl.constexpr):
+    # out = (a @ b) * s[0] + 3 * s[1], the two scalars loaded as vectors of one element, along the rows and along both; an index
+    # vector of one element masks a column
+    rm = tl.program_id(0) * BM + tl.arange(0, BM)
+    rk = tl.arange(0, K)
+    rn = tl.arange(0, N)
+    one = tl.arange(0, 1)
+    s = tl.load(s_ptr + one, mask=one < n_s, other=0.0)
+    t = tl.load(s_ptr + 1 + one[:, None] + one[None, :])
+    a = tl.load(a_ptr + rm[:, None] * K + rk[None, :], mask=rm[:, None] < n, other=0.0)
+    b = tl.load(b_ptr + rk[:, None] * N + rn[None, :])
+    acc = tl.dot(a, b) * s[:, None] + t * 3.0
+    acc = tl.where((one[:, None] + 5) == rn[None, :], 0.0, acc)
+    acc = tl.where(rn[None, :] < (one + 40)[:, None], acc, 1.0)
+    tl.store(out_ptr + rm[:, None] * N + rn[None, :], acc, mask=rm[:, None] < n)

@@ -947,6 +947,22 @@ def test_matrix_program_loop_as_long_as_another_counted(BM, BN, n, m, causal):
     assert torch.equal(out[:n].cpu().double(), want) and (out[n] == 7.0).all()
 
 
+@pytest.mark.parametrize("BM,n,n_s", [(32, 33, 1), (64, 130, 1), (128, 100, 0)])
+def test_matrix_program_with_vectors_of_one_element(BM, n, n_s):
+    import extra_kernels as X
+    g = torch.Generator().manual_seed(n)
+    a, b = torch.randint(-2, 3, (n, 32), generator=g).half(), torch.randint(-2, 3, (32, 64), generator=g).half()
+    s = torch.tensor([2.0, 5.0])
+    out = torch.full((n + 1, 64), 7.0, device=DEV)
+    kern = X.product_with_one_element_vectors[(triton.cdiv(n, BM),)](a.to(DEV), b.to(DEV), s.to(DEV), out, n, n_s, K=32, BM=BM, N=64)
+    torch.cuda.synchronize()
+    assert kern.function.last_kernel == "tile_program (hipRTC, matrix layout)"
+    want = a.double() @ b.double() * (2.0 if n_s else 0.0) + 15.0
+    want[:, 5] = 0.0
+    want[:, 40:] = 1.0
+    assert torch.equal(out[:n].cpu().double(), want) and (out[n] == 7.0).all()
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("rows,BM,K,N,P,k_cols,turned", [(1, 32, 32, 32, 32, 32, False), (100, 64, 64, 128, 32, 50, True), (129, 128, 128, 64, 64, 128, False), (70, 32, 256, 32, 128, 200, True)])
 def test_matrix_program_chained_products(dtype, rows, BM, K, N, P, k_cols, turned):

@@ -676,3 +676,16 @@ def test_matrix_programs_name_what_a_loop_leaves_behind_only_after_it(native, tm
         declared = src.index("const long long res0_%s = " % q)
         assert not re.search(r"\bres0_%s\b" % q, src[:declared])
     assert re.search(r"long long last1 = .*\bres0_\d\b", src)
+
+
+def test_matrix_programs_read_vectors_of_one_element_at_their_element(native, tmp_path):
+    """A vector of one element next to a block has the same value in every row: its load does not move with the row (and so does
+    not leave its argument), nor does an index vector of one element."""
+    import extra_kernels as X
+    sig = {"a_ptr": "*fp16", "b_ptr": "*fp16", "s_ptr": "*fp32", "out_ptr": "*fp32", "n": "i32", "n_s": "i32", **{x: "constexpr" for x in ("K", "BM", "N")}}
+    src = _generic_source(tmp_path, compile_ttir(X.product_with_one_element_vectors, sig, {"K": 32, "BM": 64, "N": 64}))
+    assert src.startswith("// tts: matrix "), src[:40]
+    loads = [l for l in src.splitlines() if "(const float *)p.ptr[2]" in l]
+    assert len(loads) == 2 and not any("wrow" in l or "l32" in l for l in loads), loads
+    for picked in [l for l in src.splitlines() if "?" in l and ("(int)(0 + " in l)]:
+        assert not re.search(r"\(int\)\(0 \+ \(wrow", picked), picked

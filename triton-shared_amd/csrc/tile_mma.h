@@ -346,7 +346,7 @@ struct MmaGen : Gen {
     switch (d->kind) {
       case SK::Const: case SK::FromIndex: case SK::ScalarArg: return at(v, "0", "0");
       case SK::Splat: return at(d->operands[0], "0", "0");
-      case SK::Iota: return "(int)(" + std::to_string(d->ival) + " + " + (role == ROW ? ROWX : COLX) + ")";
+      case SK::Iota: return "(int)(" + std::to_string(d->ival) + " + " + (V.shape[0] == 1 ? "0" : role == ROW ? ROWX : COLX) + ")";  // (one element: the same for every row)
       case SK::ExpandDims: return el(d->operands[0], d->axis == 1 ? ROW : COL);
       case SK::Broadcast: {
         const Value &O = val(d->operands[0]);
@@ -408,7 +408,7 @@ struct MmaGen : Gen {
       case SK::Splat: return bounds(d->operands[0], role, lo, hi, given);
       case SK::Iota: {
         const std::string b = std::to_string(d->ival);
-        if (role == ROW) {
+        if (role == ROW && V.shape[0] > 1) {
           *lo = "(" + b + "LL + wrow)";
           *hi = "(" + b + "LL + wrow + " + std::to_string(32 * R - 1) + ")";
         } else {
@@ -687,7 +687,7 @@ struct MmaGen : Gen {
     if (r & ROW) {
       const std::string n = id("r", v), T = ctype(val(v).dtype);
       line(T + " " + n + "[" + std::to_string(R) + "];");
-      row_loop(n + "[rb] = " + elementwise(a.sizes.size() == 2 && a.sizes[0] == 1 ? "0" : ROWX, "0") + ";");
+      row_loop(n + "[rb] = " + elementwise(a.sizes[0] == 1 ? "0" : ROWX, "0") + ";");
       row_of[v] = n;
     }
     if (r & COL) {
