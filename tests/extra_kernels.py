@@ -1508,3 +1508,15 @@ def product_with_one_element_vectors(a_ptr, b_ptr, s_ptr, out_ptr, n, n_s, K: tl
     acc = tl.where((one[:, None] + 5) == rn[None, :], 0.0, acc)
     acc = tl.where(rn[None, :] < (one + 40)[:, None], acc, 1.0)
     tl.store(out_ptr + rm[:, None] * N + rn[None, :], acc, mask=rm[:, None] < n)
+
+
+@triton.jit
+def copy_under_a_scalar_condition(x_ptr, out_ptr, load_from, store_from, n, BR: tl.constexpr, BC: tl.constexpr):
+    # a block of rows per program; loads are masked by one scalar condition for the whole block, stores by another
+    pid = tl.program_id(0)
+    if BR == 1:
+        at = pid * BC + tl.arange(0, BC)
+    else:
+        at = (pid * BR + tl.arange(0, BR))[:, None] * BC + tl.arange(0, BC)[None, :]
+    x = tl.load(x_ptr + at, mask=pid >= load_from, other=-1.0)
+    tl.store(out_ptr + at, x + 1.0, mask=pid >= store_from)

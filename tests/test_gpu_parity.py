@@ -947,6 +947,19 @@ def test_matrix_program_loop_as_long_as_another_counted(BM, BN, n, m, causal):
     assert torch.equal(out[:n].cpu().double(), want) and (out[n] == 7.0).all()
 
 
+@pytest.mark.parametrize("BR", [1, 4])
+@pytest.mark.parametrize("load_from,store_from", [(0, 0), (2, 1), (0, 5), (7, 7)])
+def test_blocks_masked_by_one_scalar_condition(load_from, store_from, BR):
+    import extra_kernels as X
+    x = torch.arange(7 * BR * 64, device=DEV).float().view(7 * BR, 64)
+    out = torch.full((7 * BR, 64), 7.0, device=DEV)
+    X.copy_under_a_scalar_condition[(7,)](x, out, load_from, store_from, 0, BR=BR, BC=64)
+    torch.cuda.synchronize()
+    pid = torch.arange(7 * BR)[:, None] // BR
+    want = torch.where(pid >= store_from, torch.where(pid >= load_from, x.cpu() + 1.0, 0.0), 7.0)
+    assert torch.equal(out.cpu(), want)
+
+
 @pytest.mark.parametrize("BM,n,n_s", [(32, 33, 1), (64, 130, 1), (128, 100, 0)])
 def test_matrix_program_with_vectors_of_one_element(BM, n, n_s):
     import extra_kernels as X

@@ -689,3 +689,18 @@ def test_matrix_programs_read_vectors_of_one_element_at_their_element(native, tm
     assert len(loads) == 2 and not any("wrow" in l or "l32" in l for l in loads), loads
     for picked in [l for l in src.splitlines() if "?" in l and ("(int)(0 + " in l)]:
         assert not re.search(r"\(int\)\(0 \+ \(wrow", picked), picked
+
+
+@pytest.mark.parametrize("BR", [1, 4])
+def test_a_scalar_condition_is_a_mask_of_its_own(native, BR):
+    """`mask=flag` splats the flag over the block: all of the block or nothing of it."""
+    import extra_kernels as X
+    sig = {"x_ptr": "*fp32", "out_ptr": "*fp32", "load_from": "i32", "store_from": "i32", "n": "i32", "BR": "constexpr", "BC": "constexpr"}
+    s = native.ttir_to_structured(compile_ttir(X.copy_under_a_scalar_condition, sig, {"BR": BR, "BC": 64}))
+    acc = accesses(s)
+    assert [k for k, _ in acc] == ["load", "store"]
+    for (kind, text), arg in zip(acc, ("arg2", "arg3")):
+        dims = text[text.index("dims=["):]
+        assert arg in dims and "64" in dims, text
+    plan = native.PlanHandle(native.structured_to_plan(s)[0])
+    assert plan.family == "tile_program"   # (the kernels for maps know masks of the form index < bound)

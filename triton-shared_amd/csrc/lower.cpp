@@ -510,6 +510,15 @@ class Lowerer {
     throw Unsupported("MaskAnalysis: mask computed by " + op.name + " (line " + std::to_string(op.line) + ")");
   }
 
+  // The extents of an access under a whole mask.  A scalar condition splatted over the block leaves them whole when it holds
+  // and empties them otherwise, as in a conjunction.
+  std::vector<int> mask_extents(const std::string &name) {
+    MaskState m = mask_parse(name);
+    if (m.scalar >= 0)
+      for (int &d : m.dims) d = P.pool.cmpsel(5, m.scalar, c64(0), d, c64(0));
+    return m.dims;
+  }
+
   MaskState mask_cmp(const Op &op) {  // MaskAnalysis.cpp:461-603
     const std::string &pred = op.words.at(0);
     if (pred != "slt" && pred != "ult" && pred != "sge") throw Unsupported("MaskAnalysis: cmpi " + pred);
@@ -839,9 +848,8 @@ class Lowerer {
         PtrState st = visit(op.operands[0]);
         s.acc = make_access(st, rt);
         if (op.operands.size() >= 2) {
-          MaskState m = mask_parse(op.operands[1]);
-          if (m.rank() != st.rank()) throw Unsupported("mask rank differs from pointer rank");
-          s.acc.dims = m.dims;
+          s.acc.dims = mask_extents(op.operands[1]);
+          if (s.acc.dims.size() != st.rank()) throw Unsupported("mask rank differs from pointer rank");
         }
       } catch (const Unsupported &) {
         structured = false;
@@ -869,9 +877,8 @@ class Lowerer {
     } else {
       s.kind = SK::Load;
       if (op.operands.size() >= 2) {
-        MaskState m = mask_parse(op.operands[1]);
-        if (m.rank() != st.rank()) throw Unsupported("mask rank differs from pointer rank");
-        s.acc.dims = m.dims;
+        s.acc.dims = mask_extents(op.operands[1]);
+        if (s.acc.dims.size() != st.rank()) throw Unsupported("mask rank differs from pointer rank");
       }
       if (op.operands.size() >= 3) scalar_other(op.operands[2], s);
     }
@@ -913,9 +920,8 @@ class Lowerer {
     } else {
       s.kind = SK::Store;
       if (op.operands.size() >= 3) {
-        MaskState m = mask_parse(op.operands[2]);
-        if (m.rank() != st.rank()) throw Unsupported("mask rank differs from pointer rank");
-        s.acc.dims = m.dims;
+        s.acc.dims = mask_extents(op.operands[2]);
+        if (s.acc.dims.size() != st.rank()) throw Unsupported("mask rank differs from pointer rank");
       }
     }
     cur_->push_back(s);
