@@ -1520,3 +1520,16 @@ def copy_under_a_scalar_condition(x_ptr, out_ptr, load_from, store_from, n, BR: 
         at = (pid * BR + tl.arange(0, BR))[:, None] * BC + tl.arange(0, BC)[None, :]
     x = tl.load(x_ptr + at, mask=pid >= load_from, other=-1.0)
     tl.store(out_ptr + at, x + 1.0, mask=pid >= store_from)
+
+
+@triton.jit
+def product_with_double_rows(a_ptr, b_ptr, out_ptr, n, big, K: tl.constexpr, BM: tl.constexpr, N: tl.constexpr):
+    # out = a @ b plus each row's sum, which goes through a difference of large numbers in fp64
+    rm = tl.program_id(0) * BM + tl.arange(0, BM)
+    rk = tl.arange(0, K)
+    rn = tl.arange(0, N)
+    a = tl.load(a_ptr + rm[:, None] * K + rk[None, :], mask=rm[:, None] < n, other=0.0)
+    b = tl.load(b_ptr + rk[:, None] * N + rn[None, :])
+    acc = tl.dot(a, b)
+    r = (tl.sum(acc, axis=1).to(tl.float64) + big) - big
+    tl.store(out_ptr + rm[:, None] * N + rn[None, :], acc + r.to(tl.float32)[:, None], mask=rm[:, None] < n)

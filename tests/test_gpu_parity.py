@@ -960,6 +960,18 @@ def test_blocks_masked_by_one_scalar_condition(load_from, store_from, BR):
     assert torch.equal(out.cpu(), want)
 
 
+def test_product_with_rows_in_double_precision():
+    import extra_kernels as X
+    g = torch.Generator().manual_seed(1)
+    n = 70
+    a, b = torch.randint(-2, 3, (n, 32), generator=g).half(), torch.randint(-2, 3, (32, 64), generator=g).half()
+    out = torch.full((n + 1, 64), 7.0, device=DEV)
+    X.product_with_double_rows[(triton.cdiv(n, 64),)](a.to(DEV), b.to(DEV), out, n, 1.0e12, K=32, BM=64, N=64)
+    torch.cuda.synchronize()
+    want = a.double() @ b.double()
+    assert torch.equal(out[:n].cpu().double(), want + want.sum(1, keepdim=True)) and (out[n] == 7.0).all()
+
+
 @pytest.mark.parametrize("BM,n,n_s", [(32, 33, 1), (64, 130, 1), (128, 100, 0)])
 def test_matrix_program_with_vectors_of_one_element(BM, n, n_s):
     import extra_kernels as X

@@ -704,3 +704,11 @@ def test_a_scalar_condition_is_a_mask_of_its_own(native, BR):
         assert arg in dims and "64" in dims, text
     plan = native.PlanHandle(native.structured_to_plan(s)[0])
     assert plan.family == "tile_program"   # (the kernels for maps know masks of the form index < bound)
+
+
+def test_matrix_programs_leave_double_precision_rows_to_the_ordinary_form(native, tmp_path):
+    """The matrix layout holds rows in fp32 registers: a program that computes one in fp64 is not written in it."""
+    import extra_kernels as X
+    sig = {"a_ptr": "*fp16", "b_ptr": "*fp16", "out_ptr": "*fp32", "n": "i32", "big": "fp64", **{x: "constexpr" for x in ("K", "BM", "N")}}
+    src = _generic_source(tmp_path, compile_ttir(X.product_with_double_rows, sig, {"K": 32, "BM": 64, "N": 64}))
+    assert not src.startswith("// tts: matrix") and "double" in src

@@ -106,6 +106,7 @@ struct MmaGen : Gen {
     if (!d) decline("a value without a definition");
     const Value &V = val(v);
     if (role == TILE && !is_tile(V)) decline("a block of another number of rows");
+    if (V.dtype == "f64" || (role == TILE && !scalar_ok(V.dtype))) decline("blocks of " + V.dtype);  // (rows are held in fp32 registers too)
     auto role_of = [&](int o) -> int {  // of an operand with its own shape, inside a rank-2 result
       const Value &O = val(o);
       if (O.shape.size() != 2) decline("an operand of rank " + std::to_string(O.shape.size()));
@@ -280,8 +281,6 @@ struct MmaGen : Gen {
       if (roles.count(im.first) && roles[im.first]) decline("a right operand that is also read element by element");
     for (auto &rv : roles)
       if ((rv.second & FRAG) && (rv.second & ~FRAG)) decline("a left operand that is also read element by element");
-    for (auto &rv : roles)
-      if ((rv.second & TILE) && !scalar_ok(val(rv.first).dtype)) decline("blocks of " + val(rv.first).dtype);
     wpp = (int)(BM / (32 * R));
     G = 1;
     axis = -1;
