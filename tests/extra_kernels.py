@@ -1533,3 +1533,17 @@ def product_with_double_rows(a_ptr, b_ptr, out_ptr, n, big, K: tl.constexpr, BM:
     acc = tl.dot(a, b)
     r = (tl.sum(acc, axis=1).to(tl.float64) + big) - big
     tl.store(out_ptr + rm[:, None] * N + rn[None, :], acc + r.to(tl.float32)[:, None], mask=rm[:, None] < n)
+
+
+@triton.jit
+def product_beside_a_narrow_block(a_ptr, b_ptr, x_ptr, out_ptr, y_ptr, n, K: tl.constexpr, BM: tl.constexpr, N: tl.constexpr, C: tl.constexpr):
+    # out = a @ b plus each row's sum of x, a block of few columns beside the product; y = 2 x
+    rm = tl.program_id(0) * BM + tl.arange(0, BM)
+    rk = tl.arange(0, K)
+    rn = tl.arange(0, N)
+    rc = tl.arange(0, C)
+    a = tl.load(a_ptr + rm[:, None] * K + rk[None, :], mask=rm[:, None] < n, other=0.0)
+    b = tl.load(b_ptr + rk[:, None] * N + rn[None, :])
+    x = tl.load(x_ptr + rm[:, None] * C + rc[None, :], mask=rm[:, None] < n, other=0.0)
+    tl.store(out_ptr + rm[:, None] * N + rn[None, :], tl.dot(a, b) + tl.sum(x, axis=1)[:, None], mask=rm[:, None] < n)
+    tl.store(y_ptr + rm[:, None] * C + rc[None, :], x * 2.0, mask=rm[:, None] < n)

@@ -972,6 +972,21 @@ def test_product_with_rows_in_double_precision():
     assert torch.equal(out[:n].cpu().double(), want + want.sum(1, keepdim=True)) and (out[n] == 7.0).all()
 
 
+@pytest.mark.parametrize("C", [2, 16, 32])
+def test_product_beside_a_narrow_block(C):
+    import extra_kernels as X
+    g = torch.Generator().manual_seed(C)
+    n = 70
+    a, b = torch.randint(-2, 3, (n, 32), generator=g).half(), torch.randint(-2, 3, (32, 64), generator=g).half()
+    x = torch.randint(-9, 10, (n, C), generator=g).float()
+    out, y = torch.full((n + 1, 64), 7.0, device=DEV), torch.full((n + 1, C), 7.0, device=DEV)
+    kern = X.product_beside_a_narrow_block[(triton.cdiv(n, 64),)](a.to(DEV), b.to(DEV), x.to(DEV), out, y, n, K=32, BM=64, N=64, C=C)
+    torch.cuda.synchronize()
+    assert kern.function.last_kernel == ("tile_program (hipRTC, matrix layout)" if C == 32 else "tile_program (hipRTC)")
+    assert torch.equal(out[:n].cpu().double(), a.double() @ b.double() + x.double().sum(1, keepdim=True)) and (out[n] == 7.0).all()
+    assert torch.equal(y[:n].cpu(), x * 2.0) and (y[n] == 7.0).all()
+
+
 @pytest.mark.parametrize("BM,n,n_s", [(32, 33, 1), (64, 130, 1), (128, 100, 0)])
 def test_matrix_program_with_vectors_of_one_element(BM, n, n_s):
     import extra_kernels as X

@@ -712,3 +712,12 @@ def test_matrix_programs_leave_double_precision_rows_to_the_ordinary_form(native
     sig = {"a_ptr": "*fp16", "b_ptr": "*fp16", "out_ptr": "*fp32", "n": "i32", "big": "fp64", **{x: "constexpr" for x in ("K", "BM", "N")}}
     src = _generic_source(tmp_path, compile_ttir(X.product_with_double_rows, sig, {"K": 32, "BM": 64, "N": 64}))
     assert not src.startswith("// tts: matrix") and "double" in src
+
+
+@pytest.mark.parametrize("C", [2, 16, 32])
+def test_matrix_programs_hold_blocks_of_whole_column_groups_only(native, tmp_path, C):
+    """A lane's registers stand for groups of 32 columns: a program with a narrower block is written in the ordinary form."""
+    import extra_kernels as X
+    sig = {"a_ptr": "*fp16", "b_ptr": "*fp16", "x_ptr": "*fp32", "out_ptr": "*fp32", "y_ptr": "*fp32", "n": "i32", **{x: "constexpr" for x in ("K", "BM", "N", "C")}}
+    src = _generic_source(tmp_path, compile_ttir(X.product_beside_a_narrow_block, sig, {"K": 32, "BM": 64, "N": 64, "C": C}))
+    assert src.startswith("// tts: matrix") == (C == 32) and "[0]; " not in src

@@ -106,6 +106,7 @@ struct MmaGen : Gen {
     if (!d) decline("a value without a definition");
     const Value &V = val(v);
     if (role == TILE && !is_tile(V)) decline("a block of another number of rows");
+    if (role == TILE && V.shape[1] % 32) decline("a block of " + std::to_string(V.shape[1]) + " columns");  // (lanes hold columns in groups of 32)
     if (V.dtype == "f64" || (role == TILE && !scalar_ok(V.dtype))) decline("blocks of " + V.dtype);  // (rows are held in fp32 registers too)
     auto role_of = [&](int o) -> int {  // of an operand with its own shape, inside a rank-2 result
       const Value &O = val(o);
