@@ -721,3 +721,28 @@ def test_matrix_programs_hold_blocks_of_whole_column_groups_only(native, tmp_pat
     sig = {"a_ptr": "*fp16", "b_ptr": "*fp16", "x_ptr": "*fp32", "out_ptr": "*fp32", "y_ptr": "*fp32", "n": "i32", **{x: "constexpr" for x in ("K", "BM", "N", "C")}}
     src = _generic_source(tmp_path, compile_ttir(X.product_beside_a_narrow_block, sig, {"K": 32, "BM": 64, "N": 64, "C": C}))
     assert src.startswith("// tts: matrix") == (C == 32) and "[0]; " not in src
+
+
+def test_direct_loads_to_lds_stand_behind_their_operands(native, tmp_path):
+    """A direct-to-LDS load reads m0 one instruction behind its write at the earliest, and a scalar base address that a vector
+    instruction wrote five behind it.  Inside inline assembly nobody counts: there, something stands between the write of m0 and
+    the load, and a base address is a copy made by a scalar instruction (or there is none)."""
+    import glob
+    import os
+    from conftest import ROOT
+    import extra_kernels as X
+    sig = {**{x: "*fp16" for x in "QKVO"}, "sm_scale": "fp32", **{x: "i32" for x in ("seq", "stride_h", "stride_s")}, **{x: "constexpr" for x in ("BM", "BN", "D")}}
+    texts = {"generated": _generic_source(tmp_path, compile_ttir(X.attention_fwd, sig, {"BM": 64, "BN": 64, "D": 64}))}
+    for f in glob.glob(os.path.join(ROOT, "triton-shared_amd", "csrc", "*.h")) + glob.glob(os.path.join(ROOT, "triton-shared_amd", "csrc", "*.hip")):
+        texts[os.path.basename(f)] = open(f).read()
+    seen = 0
+    for name, text in texts.items():
+        for asm in re.findall(r'asm volatile\("([^"]*_load_lds_[^"]*)"', text):
+            lines = asm.replace("\\n", "\n").replace("\\t", "").split("\n")
+            at = next(i for i, l in enumerate(lines) if "_load_lds_" in l)
+            assert "m0" in lines[0] and at >= 2, (name, asm)
+            base = lines[at].split(",")[-1].strip()
+            # (beside a matrix instruction: a form the library alone compiles, where the base is a scalar register throughout)
+            assert base == "off" or any(l.startswith(("s_mov_b64 %s," % base, "v_mfma")) for l in lines[:at]), (name, asm)
+            seen += 1
+    assert seen >= 5

@@ -425,6 +425,15 @@ constexpr int F_A_BYTES = DmaTile<4, 4>::A_BYTES, F_STAGE_BYTES = DmaTile<4, 4>:
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 #define TTS_LDS(p) ((__attribute__((address_space(3))) void *)(p))
 
+// 64 lanes' 16-byte chunks, each `voff` bytes behind a base address that all lanes share, to 1 KB of LDS at `lds`.  The load
+// has to stand one instruction behind the write of m0, and five behind a vector instruction that wrote the base address (a
+// v_readfirstlane); the compiler does not look inside and counts neither.  Copying the base with a scalar instruction, which
+// itself waits for the vector one, is both.
+__device__ __forceinline__ void load_to_lds(const char *sbase, uint32_t voff, uint32_t lds) {
+  uint64_t base;
+  asm volatile("s_mov_b32 m0, %1\n\ts_mov_b64 %0, %3\n\tglobal_load_lds_dwordx4 %2, %0" : "=&s"(base) : "s"(lds), "v"(voff), "s"(sbase) : "memory", "m0");
+}
+
 // s_waitcnt immediate: vmcnt in bits 3:0 and 15:14, expcnt (not waited for) in 6:4, lgkmcnt in 11:8
 constexpr int waitcnt_imm(int vm, int lgkm) { return (vm & 15) | ((vm >> 4) << 14) | (7 << 4) | (lgkm << 8); }
 
@@ -546,7 +555,7 @@ __device__ __forceinline__ void gemm_dma_body(const GemmParams &p, int tiles_m, 
 #pragma unroll
       for (int h = 0; h < 2; h++)
         if (on[h])
-          asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, off" : : "s"(sink), "v"(line_at[h] + (int64_t)t * F_BK * p.ldb * 2) : "memory", "m0");
+          asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" : : "s"(sink), "v"(line_at[h] + (int64_t)t * F_BK * p.ldb * 2) : "memory", "m0");
     };
     for (int t = STAGES - 1; t < F_PF_AHEAD; t++) touch(t);
     __syncthreads();  // the others' barrier after the prologue ...
@@ -606,10 +615,10 @@ __device__ __forceinline__ void gemm_dma_body(const GemmParams &p, int tiles_m, 
     const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)b);
     sbase = (const char *)(uintptr_t)(((uint64_t)hi << 32) | (uint64_t)lo);
 #endif
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(lds), "v"(voff), "s"(sbase) : "memory", "m0");
+    load_to_lds(sbase, voff, lds);
   };
   auto dma_lane = [&](const char *addr, uint32_t lds) {  // every lane its own 64-bit address
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(lds), "v"(addr) : "memory", "m0");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(lds), "v"(addr) : "memory", "m0");
   };
   auto dma_one = [&](int t, int n) {  // n < A_DMA: A part, else B part of tile t, into stage t % STAGES
     int tc = min(t, nk - 1) + k_first;
@@ -872,17 +881,18 @@ __device__ __forceinline__ void gemm_dma16_body(const GemmParams &p, int tiles_m
     const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)b);
     sbase = (const char *)(uintptr_t)(((uint64_t)hi << 32) | (uint64_t)lo);
 #endif
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(lds), "v"(voff), "s"(sbase) : "memory", "m0");
+    load_to_lds(sbase, voff, lds);
   };
   // n < A_DMA: A part, else B part of tile t, into stage t % STAGES.  Loads past the last tile fetch the last tile again, so
   // that the wait count is the same in every iteration (a scalar branch around every load and between two waits instead
   // cost 5 us of 110: sixteen branches per tile in between the matrix instructions).
-  auto dma_one = [&](int t, int n) __attribute__((always_inline)) {
+  auto dma_at = [&](int t, int n, auto issue) __attribute__((always_inline)) {
     const int tc = min(t, nk - 1) + k_begin;
     const uint32_t st = lds0 + (t % STAGES) * STAGE_BYTES;
-    if (n < A_DMA) dma(a_base + (int64_t)tc * F_BK * 2, a_voff[n], st + (A_DMA * wave_u + n) * 1024);
-    else dma(b_base + (int64_t)tc * F_BK * p.ldb * 2, b_voff[n - A_DMA], st + A_BYTES + (B_DMA * wave_u + n - A_DMA) * 1024);
+    if (n < A_DMA) issue(a_base + (int64_t)tc * F_BK * 2, a_voff[n], st + (A_DMA * wave_u + n) * 1024);
+    else issue(b_base + (int64_t)tc * F_BK * p.ldb * 2, b_voff[n - A_DMA], st + A_BYTES + (B_DMA * wave_u + n - A_DMA) * 1024);
   };
+  auto dma_one = [&](int t, int n) __attribute__((always_inline)) { dma_at(t, n, dma); };
 
   const int l16 = lane & 15, q = lane >> 4;
   const int a_off = (wm * 128 + l16) * 64 + ((q ^ a_swizzle((l16 >> 2) & 3)) << 4);
@@ -909,13 +919,30 @@ __device__ __forceinline__ void gemm_dma16_body(const GemmParams &p, int tiles_m
     else
       asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(__builtin_bit_cast(u32x4_r, b)), "v"(__builtin_bit_cast(u32x4_r, a)));
   };
+  // A product and a load behind it.  The matrix instruction is what stands between the write of m0 and the load (4096^3: 99.2 us,
+  // with a scalar instruction there 100.1); a base address that had to be read from a vector register is left to load_to_lds.
+  auto mfma16_and_load = [&](int i, int j, const uint4 &a, const uint4 &b, int t, int n) __attribute__((always_inline)) {
+#ifdef TTS_GEMM_RTC
+    mfma16(i, j, a, b);
+    dma_one(t, n);
+#else
+    dma_at(t, n, [&](const char *sbase, uint32_t voff, uint32_t lds) __attribute__((always_inline)) {
+      if constexpr (BF16)
+        asm volatile("s_mov_b32 m0, %3\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, %0\n\tglobal_load_lds_dwordx4 %4, %5"
+                     : "+a"(acc[i][j]) : "v"(__builtin_bit_cast(u32x4_r, b)), "v"(__builtin_bit_cast(u32x4_r, a)), "s"(lds), "v"(voff), "s"(sbase) : "memory", "m0");
+      else
+        asm volatile("s_mov_b32 m0, %3\n\tv_mfma_f32_16x16x32_f16 %0, %1, %2, %0\n\tglobal_load_lds_dwordx4 %4, %5"
+                     : "+a"(acc[i][j]) : "v"(__builtin_bit_cast(u32x4_r, b)), "v"(__builtin_bit_cast(u32x4_r, a)), "s"(lds), "v"(voff), "s"(sbase) : "memory", "m0");
+    });
+#endif
+  };
   auto tile = [&](int t, uint4 (&Ac)[8], uint4 (&An)[8]) __attribute__((always_inline)) {
     static_for<0, 32>([&](auto slot) __attribute__((always_inline)) {
       constexpr int n = decltype(slot)::value;
       __builtin_amdgcn_sched_barrier(0);
-      mfma16(n >> 2, n & 3, Ac[n >> 2], B0[n & 3]);
+      if constexpr (n % 8 == 7) mfma16_and_load(n >> 2, n & 3, Ac[n >> 2], B0[n & 3], t + STAGES - 1, n / 8);
+      else mfma16(n >> 2, n & 3, Ac[n >> 2], B0[n & 3]);
       if constexpr (n < 8) read_b(t, 4 + (n >> 1), n & 1, B1[n >> 1]);
-      if constexpr (n % 8 == 7) dma_one(t + STAGES - 1, n / 8);
     });
     __builtin_amdgcn_sched_barrier(0);
     // own loads of tile t + 1 have landed (later ones may be in flight); own reads of tile t are complete
@@ -924,10 +951,10 @@ __device__ __forceinline__ void gemm_dma16_body(const GemmParams &p, int tiles_m
     static_for<0, 32>([&](auto slot) __attribute__((always_inline)) {
       constexpr int n = decltype(slot)::value;
       __builtin_amdgcn_sched_barrier(0);
-      mfma16(n >> 2, 4 + (n & 3), Ac[n >> 2], B1[n & 3]);
+      if constexpr (n % 8 == 7) mfma16_and_load(n >> 2, 4 + (n & 3), Ac[n >> 2], B1[n & 3], t + STAGES - 1, 4 + n / 8);
+      else mfma16(n >> 2, 4 + (n & 3), Ac[n >> 2], B1[n & 3]);
       if constexpr (n < 8) read_a(t + 1, n, An);
       else if constexpr (n < 16) read_b(t + 1, (n - 8) >> 1, n & 1, B0[(n - 8) >> 1]);
-      if constexpr (n % 8 == 7) dma_one(t + STAGES - 1, 4 + n / 8);
     });
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_waitcnt(waitcnt_imm(63, 0));

@@ -109,16 +109,13 @@ __global__ __launch_bounds__(256, 1) void gemm_w8a16_tile_kernel(GemmW8A16Params
   const char *a_base = (const char *)((const uint16_t *)p.a + m0 * p.lda);
   const char *w_base = (const char *)p.w + n0;
   const uint32_t lds0 = (uint32_t)(uintptr_t)TTS_LDS(smem);
-  auto dma = [&](const char *base, uint32_t voff, uint32_t lds) __attribute__((always_inline)) {
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(lds), "v"(voff), "s"(base) : "memory", "m0");
-  };
   // loads past the last tile fetch the last tile again: the wait count is the same in every iteration
   auto fetch = [&](int t, int stage, auto nc) __attribute__((always_inline)) {
     constexpr int n = decltype(nc)::value;
     const int tc = min(t, nk - 1) + k_begin;
     const uint32_t st = lds0 + stage * T::STAGE;
-    if constexpr (n < T::A_DMA) dma(a_base + (int64_t)tc * 128, a_voff[n], st + min(T::A_DMA * wave + n, (uint32_t)(2 * TM - 1)) * 1024);
-    else dma(w_base + (int64_t)tc * 64 * p.ldw, w_voff[n - T::A_DMA], st + T::A_BYTES + (4 * wave + n - T::A_DMA) * 1024);
+    if constexpr (n < T::A_DMA) load_to_lds(a_base + (int64_t)tc * 128, a_voff[n], st + min(T::A_DMA * wave + n, (uint32_t)(2 * TM - 1)) * 1024);
+    else load_to_lds(w_base + (int64_t)tc * 64 * p.ldw, w_voff[n - T::A_DMA], st + T::A_BYTES + (4 * wave + n - T::A_DMA) * 1024);
   };
 
   // step s of a tile: k 32 s + 8 q .. +7

@@ -1066,7 +1066,10 @@ __device__ __forceinline__ void copy_to_lds(const void *base, unsigned off, unsi
   const unsigned long long b = (unsigned long long)base;
   const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(b >> 32)), lo = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)b);
   const void *s = (const void *)(((unsigned long long)hi << 32) | (unsigned long long)lo);
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(__builtin_amdgcn_readfirstlane((int)to)), "v"(off), "s"(s) : "memory", "m0");
+  // (the copy of the base keeps the load one instruction behind the write of m0, and off registers that v_readfirstlane has
+  // just written, for which it would need five: the compiler counts neither)
+  unsigned long long own;
+  asm volatile("s_mov_b32 m0, %1\n\ts_mov_b64 %0, %3\n\tglobal_load_lds_dwordx4 %2, %0" : "=&s"(own) : "s"(__builtin_amdgcn_readfirstlane((int)to)), "v"(off), "s"(s) : "memory", "m0");
 }
 // this wavefront's copies have arrived, and after the barrier everybody's
 __device__ __forceinline__ void landed() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); __syncthreads(); }
