@@ -1547,3 +1547,20 @@ def product_beside_a_narrow_block(a_ptr, b_ptr, x_ptr, out_ptr, y_ptr, n, K: tl.
     x = tl.load(x_ptr + rm[:, None] * C + rc[None, :], mask=rm[:, None] < n, other=0.0)
     tl.store(out_ptr + rm[:, None] * N + rn[None, :], tl.dot(a, b) + tl.sum(x, axis=1)[:, None], mask=rm[:, None] < n)
     tl.store(y_ptr + rm[:, None] * C + rc[None, :], x * 2.0, mask=rm[:, None] < n)
+
+
+@triton.jit
+def product_exponentials(a_ptr, b_ptr, r_ptr, out_ptr, n, big, K: tl.constexpr, BM: tl.constexpr, N: tl.constexpr, BASE2: tl.constexpr):
+    # out = exp(a @ b - r) * big, r loaded: a weight recomputed from a saved log-sum, rescaled; 16-bit results
+    rm = tl.program_id(0) * BM + tl.arange(0, BM)
+    rk = tl.arange(0, K)
+    rn = tl.arange(0, N)
+    a = tl.load(a_ptr + rm[:, None] * K + rk[None, :], mask=rm[:, None] < n, other=0.0)
+    b = tl.load(b_ptr + rk[:, None] * N + rn[None, :])
+    r = tl.load(r_ptr + rm, mask=rm < n, other=0.0)
+    d = tl.dot(a, b) - r[:, None]
+    if BASE2:
+        e = tl.exp2(d)
+    else:
+        e = tl.exp(d)
+    tl.store(out_ptr + rm[:, None] * N + rn[None, :], (e * big).to(out_ptr.dtype.element_ty), mask=rm[:, None] < n)

@@ -987,6 +987,25 @@ def test_product_beside_a_narrow_block(C):
     assert torch.equal(y[:n].cpu(), x * 2.0) and (y[n] == 7.0).all()
 
 
+@pytest.mark.parametrize("base2,low,big", [(False, -95, 2.0 ** 125), (True, -140, 2.0 ** 127), (False, 60, 2.0 ** -100)])
+def test_product_exponentials_over_the_whole_range(base2, low, big):
+    # exponentials that are subnormal, and large ones, brought back into range before they are stored in 16 bits
+    import extra_kernels as X
+    g = torch.Generator().manual_seed(5)
+    n = 70
+    a, b = torch.randint(-1, 2, (n, 32), generator=g).half(), torch.randint(-1, 2, (32, 64), generator=g).half()
+    r = -(torch.randint(0, 9, (n,), generator=g).float() + low)
+    out = torch.full((n + 1, 64), 7.0, device=DEV, dtype=torch.bfloat16)
+    kern = X.product_exponentials[(triton.cdiv(n, 64),)](a.to(DEV), b.to(DEV), r.to(DEV), out, n, big, K=32, BM=64, N=64, BASE2=base2)
+    torch.cuda.synchronize()
+    assert kern.function.last_kernel == "tile_program (hipRTC, matrix layout)"
+    d = a.double() @ b.double() - r.double()[:, None]
+    e = torch.exp2(d) if base2 else torch.exp(d)
+    # half an ulp of the result, and of the exponential where it is subnormal
+    bound = e * big * (2.0 ** -8 + 2.0 ** -20) + 2.0 ** -149 * big
+    assert ((out[:n].cpu().double() - e * big).abs() <= bound).all() and (out[n] == 7.0).all()
+
+
 @pytest.mark.parametrize("BM,n,n_s", [(32, 33, 1), (64, 130, 1), (128, 100, 0)])
 def test_matrix_program_with_vectors_of_one_element(BM, n, n_s):
     import extra_kernels as X

@@ -746,3 +746,18 @@ def test_direct_loads_to_lds_stand_behind_their_operands(native, tmp_path):
             assert base == "off" or any(l.startswith(("s_mov_b64 %s," % base, "v_mfma")) for l in lines[:at]), (name, asm)
             seen += 1
     assert seen >= 5
+
+
+def test_matrix_programs_keep_the_hardware_exponential_to_differences_against_a_maximum(native, tmp_path):
+    """v_exp_f32 of a product with log2 e is as good as the library's function only where the result is at most 1 and stands next
+    to a 1: a softmax's scores against their maximum.  Any other exponential is the library's, also where 16 bits are stored."""
+    import extra_kernels as X
+    sig = {**{x: "*fp16" for x in "QKVO"}, "sm_scale": "fp32", **{x: "i32" for x in ("seq", "stride_h", "stride_s")}, **{x: "constexpr" for x in ("BM", "BN", "D")}}
+    src = _generic_source(tmp_path, compile_ttir(X.attention_fwd, sig, {"BM": 64, "BN": 64, "D": 64}))
+    body = src[src.index("void tile_program"):]
+    assert body.count("__builtin_amdgcn_exp2f(") == 2 and "expf(" not in body
+    sig = {"a_ptr": "*fp16", "b_ptr": "*fp16", "r_ptr": "*fp32", "out_ptr": "*bf16", "n": "i32", "big": "fp32", **{x: "constexpr" for x in ("K", "BM", "N", "BASE2")}}
+    for base2 in (False, True):
+        src = _generic_source(tmp_path, compile_ttir(X.product_exponentials, sig, {"K": 32, "BM": 64, "N": 64, "BASE2": base2}))
+        body = src[src.index("void tile_program"):]
+        assert src.startswith("// tts: matrix") and "__builtin_amdgcn_exp2f(" not in body and ("exp2f(" if base2 else "expf(") in body

@@ -361,34 +361,45 @@ struct MmaGen : Gen {
       default: decline("a value without an element form");
     }
   }
+  // The exponential of a difference against a maximum that its own minuend is one of (a softmax's scores against their row's
+  // maximum, the old maximum against the new one) is at most 1, and what counts is its error next to the largest of the row,
+  // which is 1: v_exp_f32 of the difference times log2 e is off by |d| 2^-24 of e^d at most, 0.4 2^-24 where that is largest, and
+  // flushes what is below 2^-126.  That is how programs that only store 16-bit values compute those; every other exponential is
+  // the library's, to an ulp over the whole range.
+  bool is_maximum_over(int m, int x, int depth = 0) const {
+    const SOp *d = def_of(m);
+    if (!d || depth > 16) return m == x;
+    if (m == x) return true;
+    const bool max = d->name == "arith.maxnumf" || d->name == "arith.maximumf";
+    if (d->kind == SK::Reduce) return max && d->operands.at(0) == x;
+    if (d->kind == SK::Broadcast || d->kind == SK::ExpandDims) return is_maximum_over(d->operands.at(0), x, depth + 1);
+    return d->kind == SK::Map && max && (is_maximum_over(d->operands.at(0), x, depth + 1) || is_maximum_over(d->operands.at(1), x, depth + 1));
+  }
+  const SOp *difference_against_maximum(const SOp &s) const {  // the subtraction behind such an exponential
+    if (!fast_exp || s.kind != SK::Map || (s.name != "math.exp" && s.name != "math.exp2") || val(s.result).dtype != "f32") return nullptr;
+    const SOp *d = def_of(s.operands[0]);
+    return d && d->kind == SK::Map && d->name == "arith.subf" && is_maximum_over(d->operands[1], d->operands[0]) ? d : nullptr;
+  }
   std::string map_text(const SOp &s, const std::vector<std::string> &a) {
-    if (fast_exp && val(s.result).dtype == "f32") {
-      if (s.name == "math.exp") return "__builtin_amdgcn_exp2f(" + a.at(0) + " * TTS_LOG2E)";
-      if (s.name == "math.exp2") return "__builtin_amdgcn_exp2f(" + a.at(0) + ")";
-    }
+    if (difference_against_maximum(s)) return std::string("__builtin_amdgcn_exp2f(") + a.at(0) + (s.name == "math.exp" ? " * TTS_LOG2E)" : ")");
     return map_expr(s, a);
   }
-  // exp(x - m) with m the same along a row, the difference written where it is read.  It is taken before the factor log2 e:
-  // with fma(x, log2e, -m log2e) a row of the type's lowest values (all keys masked with a finite number) is infinity minus
-  // infinity, and m log2e rounds by up to |m| 2^-24 of the exponent.
+  // The same with the difference written where it is read.  It is taken before the factor log2 e: with fma(x, log2e, -m log2e) a
+  // row of the type's lowest values (all keys masked with a finite number) is infinity minus infinity, and m log2e rounds by up
+  // to |m| 2^-24 of the exponent.
   bool exp_of_difference(const SOp &s, int role, std::string *text) {
-    if (!fast_exp || role != TILE || val(s.result).dtype != "f32" || (s.name != "math.exp" && s.name != "math.exp2")) return false;
-    const SOp *d = def_of(s.operands[0]);
-    if (!d || d->kind != SK::Map || d->name != "arith.subf" || val(d->result).dtype != "f32") return false;
-    const SOp *b = def_of(d->operands[1]);
-    if (!b || b->kind != SK::Broadcast || val(b->operands[0]).shape.size() != 2 || val(b->operands[0]).shape[1] != 1) return false;
-    const bool e2 = s.name == "math.exp2";
+    const SOp *d = difference_against_maximum(s);
+    if (!d || role != TILE) return false;
     const std::string x = el(d->operands[0], role), m = el(d->operands[1], role);
-    if (e2) *text = "__builtin_amdgcn_exp2f(" + x + " - " + m + ")";
-    else *text = "__builtin_amdgcn_exp2f((" + x + " - " + m + ") * TTS_LOG2E)";
+    *text = map_text(s, {"(" + x + " - " + m + ")"});
     return true;
   }
-  bool folded_into_exp(const SOp &s) const {  // a difference that only an exponential reads is written there
-    if (!fast_exp || s.name != "arith.subf" || val(s.result).dtype != "f32") return false;
+  bool folded_into_exp(const SOp &s) const {  // a difference that only such exponentials read is written there
+    if (s.name != "arith.subf") return false;
     auto u = users.find(s.result);
     if (u == users.end()) return false;
     for (const SOp *o : u->second)
-      if (o->kind != SK::Map || (o->name != "math.exp" && o->name != "math.exp2")) return false;
+      if (!difference_against_maximum(*o)) return false;
     return true;
   }
 
