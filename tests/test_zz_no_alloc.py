@@ -166,3 +166,43 @@ def test_noalloc_refusal_leaves_a_matmul_with_epilogue_on_its_kernel(native):
     torch.cuda.synchronize()
     assert fresh.last_kernel.startswith("gemm_dma_kernel + epilogue"), fresh.last_kernel
     assert torch.equal(c2.float(), torch.nn.functional.leaky_relu(a2.float() @ b2.float(), 0.5))
+
+
+def test_noalloc_launch_of_the_tiled_int8_product_asks_for_no_scratch_it_does_not_use(native):
+    # 64 rows run on the tiled kernel.  The decode kernels' partial tiles of this width would not fit the static array (9.4 MB in
+    # two slices), but nobody reads them; the tiled kernel's own slices do not fit either, and it runs without
+    plan, _ = plan_for(native, "w8a16_matmul")
+    stream = torch.cuda.current_stream().cuda_stream
+    M, N, Kd = 64, 36864, 512
+    a, w, s = _inputs(M, N, Kd, 1)
+    want, got = (torch.full((M, N), v, dtype=torch.float16, device=DEV) for v in (5.0, 7.0))
+    grid = (4, (N + 127) // 128, 1)
+    plan.launch(grid, stream, _values(a, w, s, want, M, N, Kd))
+    plan.launch_noalloc(grid, stream, _values(a, w, s, got, M, N, Kd))
+    torch.cuda.synchronize()
+    assert plan.last_kernel == "gemm_w8a16_tile_kernel"
+    ref = a.double() @ (w.half() * s[None, :]).double()
+    for c in (want, got):   # fp32 sums in two orders, rounded once to fp16
+        assert ((c.double() - ref).norm() / ref.norm()).item() <= 2.0 ** -11
+
+
+def test_recorded_launches_of_the_tiled_int8_product_allocate_nothing(native):
+    # the first launch on a stream, while it records a graph: nothing to allocate, clear or wait for
+    plan, _ = plan_for(native, "w8a16_matmul")
+    M, N, Kd = 64, 2048, 4096
+    a, w, s = _inputs(M, N, Kd, 2)
+    want, got = (torch.zeros(M, N, dtype=torch.float16, device=DEV) for _ in range(2))
+    grid = (4, N // 128, 1)
+    plan.launch(grid, torch.cuda.current_stream().cuda_stream, _values(a, w, s, want, M, N, Kd))
+    torch.cuda.synchronize()
+    graph, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    with torch.cuda.graph(graph, stream=side):
+        plan.launch(grid, torch.cuda.current_stream().cuda_stream, _values(a, w, s, got, M, N, Kd))
+    for seed in range(3):
+        a.copy_(_inputs(M, N, Kd, 10 + seed)[0])
+        got.zero_()
+        plan.launch(grid, torch.cuda.current_stream().cuda_stream, _values(a, w, s, want, M, N, Kd))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert ((got.double() - want.double()).norm() / want.double().norm()).item() <= 2.0 ** -11   # (the eager launch runs in K slices)

@@ -136,6 +136,7 @@ int gemm_w8a16_split(const GemmW8A16Params &p);  // how many K slices the kernel
 size_t gemm_w8a16_workspace_bytes(const GemmW8A16Params &p);
 size_t gemm_w8a16_counters(const GemmW8A16Params &p);
 size_t gemm_w8a16_widened_bytes(const GemmW8A16Params &p);  // 0: this shape runs on the decode kernels
+bool gemm_w8a16_is_tiled(const GemmW8A16Params &p);         // the tiled kernel runs this product: no workspace, counters or widened weights
 size_t gemm_w8a16_tile_bytes(const GemmW8A16Params &p);  // partial sums of the tiled kernel's K slices (0: none, or another kernel runs)
 // the tiled kernel (kernels_w8_tile.hip), and what it shares with kernels_gemm.hip
 bool w8_tile_ok(const GemmW8A16Params &p);

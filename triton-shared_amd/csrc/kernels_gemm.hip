@@ -1116,6 +1116,7 @@ static bool w8_widens(const GemmW8A16Params &p) {
 static bool w8_tiles(const GemmW8A16Params &p) {
   return (p.M >= 33 || (p.M >= 17 && p.K * p.N >= (int64_t)8 << 20)) && p.N >= 2048 && w8_tile_ok(p);
 }
+bool gemm_w8a16_is_tiled(const GemmW8A16Params &p) { return w8_tiles(p); }
 size_t gemm_w8a16_tile_bytes(const GemmW8A16Params &p) { return w8_tiles(p) ? w8_tile_partial_bytes(p) : 0; }
 hipError_t launch_splitk_reduce(const GemmParams &p, hipStream_t s) {
   hipLaunchKernelGGL(gemm_splitk_reduce_kernel<false>, dim3((unsigned)((p.M * (p.N / 4) + 255) / 256), std::max(1, p.batches)), dim3(256), 0, s, p);

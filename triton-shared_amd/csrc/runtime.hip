@@ -986,7 +986,8 @@ tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, con
         p.w = ptr_arg<const int8_t>(args, pl, "b_arg");
         p.scale = ptr_arg<const void>(args, pl, "s_arg");
         p.c = ptr_arg<void>(args, pl, "c_arg");
-        if (p.split > 1 && no_alloc) {
+        const bool tiled = gemm_w8a16_is_tiled(p);  // (p.split is the decode kernels')
+        if (p.split > 1 && no_alloc && !tiled) {
           const size_t need = gemm_w8a16_workspace_bytes(p), ncount = gemm_w8a16_counters(p);
           if (need > NOALLOC_WORKSPACE_BYTES || ncount > NOALLOC_COUNTERS)
             throw Unsupported("tts_launch_noalloc: the split-K partial tiles of this shape need " + std::to_string(need) + " bytes and " +
@@ -1002,7 +1003,7 @@ tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, con
             hipError_t e = hipGetLastError();
             if (e != hipSuccess) return fail(TTS_HIP_ERROR, std::string("clearing the split-K counters: ") + hipGetErrorString(e));
           }
-        } else if (p.split > 1) {
+        } else if (p.split > 1 && !tiled) {
           const size_t need = gemm_w8a16_workspace_bytes(p), ncount = gemm_w8a16_counters(p);
           std::lock_guard<std::mutex> lock(plan->mu);
           tts_plan::SplitK &sk = plan->split_k[stream];
