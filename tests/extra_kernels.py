@@ -1564,3 +1564,15 @@ def product_exponentials(a_ptr, b_ptr, r_ptr, out_ptr, n, big, K: tl.constexpr, 
     else:
         e = tl.exp(d)
     tl.store(out_ptr + rm[:, None] * N + rn[None, :], (e * big).to(out_ptr.dtype.element_ty), mask=rm[:, None] < n)
+
+
+@triton.jit
+def block_column_sums(x_ptr, out_ptr, rows, n_cols, BR: tl.constexpr, BC: tl.constexpr):
+    # sums of `rows` rows per block of rows (program_id(0)), a block of columns each (program_id(1))
+    b = tl.program_id(0)
+    c = tl.program_id(1) * BC + tl.arange(0, BC)
+    acc = tl.zeros((BR, BC), dtype=tl.float32)
+    for r0 in range(0, rows, BR):
+        r = r0 + tl.arange(0, BR)
+        acc += tl.load(x_ptr + (b * rows + r[:, None]) * n_cols + c[None, :], mask=(r[:, None] < rows) & (c[None, :] < n_cols), other=0.0)
+    tl.store(out_ptr + (b + tl.arange(0, 1))[:, None] * n_cols + c[None, :], tl.sum(acc, axis=0)[None, :], mask=c[None, :] < n_cols)

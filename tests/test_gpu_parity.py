@@ -1006,6 +1006,27 @@ def test_product_exponentials_over_the_whole_range(base2, low, big):
     assert ((out[:n].cpu().double() - e * big).abs() <= bound).all() and (out[n] == 7.0).all()
 
 
+@pytest.mark.parametrize("gy,gz", [(4096, 4097), (65535, 257), (70000, 2)])
+def test_matrix_programs_and_add_only_loops_on_grids_of_more_than_2_to_the_24_programs(gy, gz):
+    # every program of a column of the grid writes the same block; the last one also counts as a program
+    import extra_kernels as X
+    g = torch.Generator().manual_seed(9)
+    ints = lambda *shape: torch.randint(-1, 2, shape, generator=g).half()
+    rows, (a, b, c, r) = 40, (ints(40, 32), ints(32, 32), ints(32, 32), ints(40, 32))
+    out = torch.full((rows + 1, 32), 7.0, device=DEV)
+    kern = X.chained_products[(2, gy // 2, gz)](a.to(DEV), b.to(DEV), c.to(DEV), r.to(DEV), out, rows, 32, 32, 32, BM=32, K=32, N=32, P=32, TURNED=False)
+    torch.cuda.synchronize()
+    assert kern.function.last_kernel == "tile_program (hipRTC, matrix layout)"
+    want = torch.relu(a.double() @ b.double() + r.double()) @ c.double().t()
+    assert torch.equal(out[:rows].cpu().double(), want) and (out[rows] == 7.0).all()
+    x, s = torch.randint(-3, 4, (10, 40), generator=g).float().to(DEV), torch.randint(-2, 3, (10,), generator=g).float().to(DEV)
+    out = torch.full((4, 40), 9.0, device=DEV)
+    X.column_moments[(1, gy, gz)](x, s, out, 10, 40, 40, BR=16, BC=64)
+    torch.cuda.synchronize()
+    p, q = (x.double() * s[:, None].double()).sum(0) + 1, (x.double() ** 2).sum(0)
+    assert torch.equal(out[:3].double(), torch.stack([p, q, p - 2 * q])) and (out[3] == 9.0).all()
+
+
 @pytest.mark.parametrize("BM,n,n_s", [(32, 33, 1), (64, 130, 1), (128, 100, 0)])
 def test_matrix_program_with_vectors_of_one_element(BM, n, n_s):
     import extra_kernels as X
@@ -1064,6 +1085,19 @@ def test_loops_that_only_add_run_in_slices(dtype, rows, cols, pitch):
     assert k.function.family == "tile_program"
     for out in outs:
         assert torch.equal(out[:3].double(), want) and (out[3] == 9.0).all()
+
+
+@pytest.mark.parametrize("blocks,rows,cols", [(3, 700, 100), (5, 10, 70), (600, 20, 333), (1, 64, 64)])
+def test_loops_that_only_add_with_columns_on_program_id_1(blocks, rows, cols):
+    # neighbouring column blocks on neighbouring workgroups: in slices (few programs) and whole, with the grid exchanged (many)
+    import extra_kernels as X
+    g = torch.Generator().manual_seed(rows)
+    x = torch.randint(-3, 4, (blocks * rows, cols), generator=g).float()
+    out = torch.full((blocks + 1, cols), 9.0, device=DEV)
+    kern = X.block_column_sums[(blocks, triton.cdiv(cols, 64))](x.to(DEV), out, rows, cols, BR=16, BC=64)
+    torch.cuda.synchronize()
+    assert kern.function.family == "tile_program"
+    assert torch.equal(out[:blocks].cpu(), x.view(blocks, rows, cols).sum(1)) and (out[blocks] == 9.0).all()
 
 
 def test_loops_that_only_add_can_be_recorded_in_a_graph():

@@ -761,3 +761,12 @@ def test_matrix_programs_keep_the_hardware_exponential_to_differences_against_a_
         src = _generic_source(tmp_path, compile_ttir(X.product_exponentials, sig, {"K": 32, "BM": 64, "N": 64, "BASE2": base2}))
         body = src[src.index("void tile_program"):]
         assert src.startswith("// tts: matrix") and "__builtin_amdgcn_exp2f(" not in body and ("exp2f(" if base2 else "expf(") in body
+
+
+def test_add_only_loops_keep_the_order_of_their_grid(native, tmp_path):
+    """A loop that may run in slices is also launched whole, and then the mark for programs whose stores walk the columns with
+    program_id(1) holds for it as for any other."""
+    import extra_kernels as X
+    sig = {"x_ptr": "*fp32", "out_ptr": "*fp32", "rows": "i32", "n_cols": "i32", "BR": "constexpr", "BC": "constexpr"}
+    lines = _generic_source(tmp_path, compile_ttir(X.block_column_sums, sig, {"BR": 16, "BC": 64})).splitlines()
+    assert lines[0].startswith("// tts: sliced 64 ") and lines[1] == "// tts: swap_xy"

@@ -801,7 +801,9 @@ tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, con
         int64_t &shared = e[group_axis < 0 ? 0 : group_axis];
         shared = (shared + per_group - 1) / per_group;
         a.lgx = gx; a.lgy = gy; a.lgz = gz;
-        err = rtc_launch(*slot, (int)(e[0] * e[1] * e[2]), 1, 1, group_threads, &a, sizeof a, s);
+        // (a grid holds 2^32 - 1 threads along x: larger launches continue along y, where surplus workgroups find no program)
+        const int64_t workgroups = e[0] * e[1] * e[2], along_x = std::min<int64_t>(workgroups, 1 << 23);
+        err = rtc_launch(*slot, (int)along_x, (int)((workgroups + along_x - 1) / along_x), 1, group_threads, &a, sizeof a, s);
         return TTS_OK;
       }
       int slice_floats = 0, slice_loop = 0;
@@ -812,8 +814,6 @@ tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, con
         // is recorded into a graph: the graph may be replayed beside launches that use the same stream's workspace.
         const int64_t programs = (int64_t)gx * gy * gz;
         struct { TileArgs t; int slices; float *partial; int *counters; } sa{};
-        a.lgx = gx; a.lgy = gy; a.lgz = gz;
-        sa.t = a;
         sa.slices = (int)std::max<int64_t>(1, std::min({(int64_t)rtc_resident_workgroups(*slot) * compute_units() / programs, b->slice_trips / 2, (int64_t)1024}));
         if (sa.slices > 1 && (no_alloc || is_capturing(s))) sa.slices = 1;
         if (sa.slices > 1) {
@@ -825,6 +825,16 @@ tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, con
           sa.partial = sk.workspace;
           sa.counters = sk.counters;
         }
+        // one slice: the grid as it is, a workgroup per program, its x and y exchanged where the program asks for that (see below)
+        const bool whole = sa.slices == 1, swap = whole && tile_program_swaps_grid(source) && gy > 1 && gx <= 65535;
+        if (whole && (swap ? gx : gy) <= 65535 && gz <= 65535) {
+          a.swap_xy = swap ? 1 : 0;
+          sa.t = a;
+          err = swap ? rtc_launch(*slot, gy, gx, gz, 256, &sa, sizeof sa, s) : rtc_launch(*slot, gx, gy, gz, 256, &sa, sizeof sa, s);
+          return TTS_OK;
+        }
+        a.lgx = gx; a.lgy = gy; a.lgz = gz;
+        sa.t = a;
         err = rtc_launch(*slot, (int)(programs * sa.slices), 1, 1, 256, &sa, sizeof sa, s);
         return TTS_OK;
       }

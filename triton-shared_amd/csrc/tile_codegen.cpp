@@ -2372,7 +2372,10 @@ std::string per_program_thread_index(std::string body) {
 }
 }  // namespace
 
-bool tile_program_swaps_grid(const std::string &source) { return source.compare(0, strlen(SWAP_MARK), SWAP_MARK) == 0; }
+bool tile_program_swaps_grid(const std::string &source) {
+  const size_t at = source.compare(0, strlen(SLICED_MARK), SLICED_MARK) == 0 ? source.find('\n') + 1 : 0;
+  return source.compare(at, strlen(SWAP_MARK), SWAP_MARK) == 0;
+}
 bool tile_program_is_persistent(const std::string &source) { return source.compare(0, strlen(PERSISTENT_MARK), PERSISTENT_MARK) == 0; }
 
 std::string tile_program_source(const Program &p, bool allow_persistent) {
@@ -2398,8 +2401,10 @@ std::string tile_program_source(const Program &p, bool allow_persistent) {
     throw Unsupported("tile_program: the reductions of this program need " + std::to_string(g.pool_bytes + g.out_bytes) + " bytes of LDS (limit 131072)");
   std::ostringstream all;
   if (g.persistent) all << PERSISTENT_MARK;
-  else if (g.sliced) all << SLICED_MARK << g.slice_floats() << " " << g.sliced->loop << "\n";
-  else if (stores_walk_columns_with_pid1(p)) all << SWAP_MARK;
+  else {
+    if (g.sliced) all << SLICED_MARK << g.slice_floats() << " " << g.sliced->loop << "\n";
+    if (stores_walk_columns_with_pid1(p)) all << SWAP_MARK;  // (for launches of one slice)
+  }
   all << pre << g.fns.str();
   if (g.uses_dummy) all << "__device__ __attribute__((aligned(16))) unsigned tts_dummy[8];\n";
   // swap_xy: the launcher has exchanged the grid's x and y (see SWAP_MARK)
@@ -2470,9 +2475,11 @@ std::string matrix_program_source(const Program &p) {
   const int ax = g.axis < 0 ? 0 : g.axis, b1 = ax == 0 ? 1 : 0, b2 = ax == 2 ? 1 : 2;
   const std::string NP[3] = {"npx", "npy", "npz"}, PD[3] = {"pidx", "pidy", "pidz"};
   all << "  const unsigned others = (unsigned)(" << NP[b1] << " * " << NP[b2] << "), groups = (unsigned)((" << NP[ax] << " + " << g.G - 1 << ") / " << g.G << ");\n"
+      << "  const unsigned wg = blockIdx.x + gridDim.x * blockIdx.y;  // (along y from 2^23 workgroups on)\n"
+      << "  if (wg >= others * groups) return;\n"
       << "  unsigned other, group;\n"
-      << "  if (others % 8 == 0) { const unsigned j = blockIdx.x / 8, per = others / 8; other = blockIdx.x % 8 + 8 * (j % per); group = j / per; }\n"
-      << "  else { other = blockIdx.x % others; group = blockIdx.x / others; }\n"
+      << "  if (others % 8 == 0) { const unsigned j = wg / 8, per = others / 8; other = wg % 8 + 8 * (j % per); group = j / per; }\n"
+      << "  else { other = wg % others; group = wg / others; }\n"
       << "  const long long " << PD[b1] << " = other % (unsigned)" << NP[b1] << ", " << PD[b2] << " = other / (unsigned)" << NP[b1] << ";\n";
   for (const SOp &s : p.body)
     if (s.kind == SK::For && g.expr_uses_pid(s.ub, ax) && !p.pool.depends_on(s.ub, EK::Result)) {  // (nothing of the program has run here)
