@@ -770,3 +770,19 @@ def test_add_only_loops_keep_the_order_of_their_grid(native, tmp_path):
     sig = {"x_ptr": "*fp32", "out_ptr": "*fp32", "rows": "i32", "n_cols": "i32", "BR": "constexpr", "BC": "constexpr"}
     lines = _generic_source(tmp_path, compile_ttir(X.block_column_sums, sig, {"BR": 16, "BC": 64})).splitlines()
     assert lines[0].startswith("// tts: sliced 64 ") and lines[1] == "// tts: swap_xy"
+
+
+def test_loops_that_leave_nothing_in_lds_end_without_a_barrier(native, tmp_path):
+    """Sums of a block of columns: an iteration has the barrier between its loads and its arithmetic and no other.  One whose
+    carried vectors have LDS copies ends with theirs."""
+    import extra_kernels as X
+    sig = {"x_ptr": "*fp32", "out_ptr": "*fp32", "rows": "i32", "n_cols": "i32", "BR": "constexpr", "BC": "constexpr"}
+    src = _generic_source(tmp_path, compile_ttir(X.block_column_sums, sig, {"BR": 16, "BC": 64}))
+    loop = src[src.index("for (long long k0"):src.index("float *const st")]
+    loop = loop[:loop.index("\n  }\n")]
+    assert loop.count("__syncthreads();") == 1, loop
+    sig = {**{x: "*fp16" for x in "QKVO"}, "sm_scale": "fp32", **{x: "i32" for x in ("seq", "stride_h", "stride_s")}, **{x: "constexpr" for x in ("BM", "BN", "D")}}
+    src = _generic_source(tmp_path, compile_ttir(X.attention_fwd, sig, {"BM": 16, "BN": 16, "D": 16}))
+    assert "carm0_" in src
+    end = src[:src.index("\n  }\n", src.rindex("carm0_1[t]"))].rsplit("carm0_", 1)[1]
+    assert end.count("__syncthreads();") == 1, end

@@ -111,6 +111,7 @@ struct Gen {
   std::ostringstream fns;                           // combiner functions of reductions and scans (before the kernel)
   std::ostringstream decl;                          // LDS arrays holding their results (top of the kernel)
   size_t pool_bytes = 0, out_bytes = 0;             // staging pool shared by all reductions; result arrays
+  int lds_writes = 0;                               // ops written so far that leave something in LDS
   bool uses_mfma = false;
   bool uses_dummy = false;  // wide loads of invalid groups read this instead
 
@@ -635,6 +636,7 @@ struct Gen {
     };
     for (int r : roots) walk(r, false, 0);
     if (found.empty()) return;
+    lds_writes++;
     os << pad() << "__syncthreads();\n";
     for (int v : found) {
       const Value &V = val(v);
@@ -1128,6 +1130,7 @@ struct Gen {
         decl << "  __shared__ " << ctype(val(o.result).dtype) << " " << name << "[" << elems << "];\n";
         out_bytes += (bytes + 15) / 16 * 16;
         staged[o.result] = {name, pitch};
+        lds_writes++;
         // Inside a loop of the program: two loops, as for the run's own loads, so that every load is issued before the
         // first loaded value is looked at.  (In one loop, `lds[i] = valid ? *p : other` waits for each load before the
         // next goes out: the K block of a flash-attention step, 16 loads per thread, cost a fifth of the step.)  16-bit
@@ -1599,10 +1602,10 @@ struct Gen {
     indent++;
     std::vector<int> body_held;
     loop_depth++;
-    const size_t body_at = os.str().size();
+    const int lds_before = lds_writes;
     body(s.body, &body_held);
     loop_depth--;
-    const bool staged = os.str().find("__syncthreads", body_at) != std::string::npos;
+    const bool in_lds = lds_writes != lds_before;
     // the scalars' new values first, their assignment last: the blocks' new values may be written in terms of the old scalars
     for (size_t q = 0; q < s.tile_args.size(); q++)
       if (scalar(q)) os << pad() << "const " << ctype(val(s.tile_args[q]).dtype) << " nys" << L << "_" << q << " = " << at(s.tile_yields[q], "0", "0") << ";\n";
@@ -1646,9 +1649,12 @@ struct Gen {
     for (size_t q = 0; q < s.int_iters.size(); q++)
       os << pad() << "const long long nx" << L << "_" << q << " = " << ex(s.int_iters[q].next) << ";\n";
     for (size_t q = 0; q < s.int_iters.size(); q++) os << pad() << "it" << L << "_" << q << " = nx" << L << "_" << q << ";\n";
-    // what an iteration staged in LDS is still being read above (a row's scale next to a carried block, say) while the
-    // fastest wavefront could begin the next iteration and stage over it
-    if (staged) os << pad() << "__syncthreads();\n";
+    // what an iteration left in LDS is still being read above (a row's scale next to a carried block, say) while the
+    // fastest wavefront could begin the next iteration and write over it (behind the barriers of LDS copies only an index that
+    // is data still reads)
+    bool data_index = false;
+    for (const IntIter &it : s.int_iters) data_index = data_index || P.pool.depends_on(it.next, EK::Data);
+    if (in_lds && (!any_mirror || data_index)) os << pad() << "__syncthreads();\n";
     indent--;
     os << pad() << "}\n";
     for (size_t q = 0; q < s.int_iters.size(); q++)
@@ -1674,6 +1680,7 @@ struct Gen {
   // shaped like the tiled kernels of the GEMM families: a and b are staged in LDS as fp32, every thread folds k in
   // index order for the outputs it owns (the reference's loop order) and keeps them in registers.
   void dot(const SOp &s, std::vector<int> &mine) {
+    lds_writes++;
     const Value &A = val(s.operands.at(0)), &B = val(s.operands.at(1)), &R = val(s.result);
     if (A.shape.size() != 2 || B.shape.size() != 2 || R.shape.size() != 2 || A.shape[1] != B.shape[0] || R.shape[0] != A.shape[0] ||
         R.shape[1] != B.shape[1])
@@ -1895,6 +1902,7 @@ struct Gen {
   // The operand blocks are staged in LDS; each output line is cut into SEG pieces combined by SEG threads and then in
   // piece order by one (lines of >= 256 outputs: one thread per line, in element order, as the reference's loop does).
   void reduce(const SOp &s, const std::vector<int64_t> &shape) {
+    lds_writes++;
     const std::string i0 = idx0(shape), i1 = idx1(shape);
     const size_t k = s.operands.size();
     const bool scan = s.kind == SK::Scan;
