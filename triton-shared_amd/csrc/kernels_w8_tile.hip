@@ -254,13 +254,18 @@ W8TileChoice w8_tile_choice(const GemmW8A16Params &p) {
   W8TileChoice best{};
   double best_t = 0;
   const int64_t nk = p.K / 64;
+  static const int cus = [] {
+    int dev = 0, n = 0;
+    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
+    return n;
+  }();
   for (int tm = 1; tm <= W8T_MAX_TM; tm++) {
     W8TileChoice c;
     c.tm = tm;
     c.tiles_m = (int)((p.M + 16 * tm - 1) / (16 * tm));
     c.tiles_n = (int)((p.N + W8T_COLS - 1) / W8T_COLS);
     for (c.split = 1; c.split <= 16 && (c.split == 1 || nk / c.split >= 4); c.split++) {
-      const int64_t wgs = (int64_t)c.tiles_m * c.tiles_n * c.split, rounds = (wgs + 255) / 256;
+      const int64_t wgs = (int64_t)c.tiles_m * c.tiles_n * c.split, rounds = (wgs + cus - 1) / cus;
       double t = std::max((double)(rounds * ((nk + c.split - 1) / c.split)) * std::max(0.5e-6, 0.2e-6 + 0.077e-6 * tm), (double)p.K * (double)p.N / 5.5e12) + 7e-6;
       if (c.split > 1) t += 3e-6 + 8.0 * c.split * (double)p.M * (double)p.N / 4.5e12;
       if (best.tm == 0 || t < best_t) { best = c; best_t = t; }
