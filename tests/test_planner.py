@@ -742,7 +742,7 @@ def test_direct_loads_to_lds_stand_behind_their_operands(native, tmp_path):
             at = next(i for i, l in enumerate(lines) if "_load_lds_" in l)
             assert "m0" in lines[0] and at >= 2, (name, asm)
             base = lines[at].split(",")[-1].strip()
-            # (beside a matrix instruction: a form the library alone compiles, where the base is a scalar register throughout)
+            # (beside a matrix instruction: the base is made at the start of the phase, eight of those earlier)
             assert base == "off" or any(l.startswith(("s_mov_b64 %s," % base, "v_mfma")) for l in lines[:at]), (name, asm)
             seen += 1
     assert seen >= 5

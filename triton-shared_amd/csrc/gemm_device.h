@@ -873,26 +873,25 @@ __device__ __forceinline__ void gemm_dma16_body(const GemmParams &p, int tiles_m
   }
   const uint32_t lds0 = (uint32_t)(uintptr_t)TTS_LDS(smem);
   const uint32_t wave_u = __builtin_amdgcn_readfirstlane(wave);
-  auto dma = [&](const char *sbase, uint32_t voff, uint32_t lds) __attribute__((always_inline)) {
-#ifdef TTS_GEMM_RTC
-    // (an older run-time compiler does not see that the tile's base address is the same in every lane: say so)
-    const uint64_t b = (uint64_t)(uintptr_t)sbase;
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(b >> 32));
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)b);
-    sbase = (const char *)(uintptr_t)(((uint64_t)hi << 32) | (uint64_t)lo);
-#endif
-    load_to_lds(sbase, voff, lds);
-  };
   // n < A_DMA: A part, else B part of tile t, into stage t % STAGES.  Loads past the last tile fetch the last tile again, so
   // that the wait count is the same in every iteration (a scalar branch around every load and between two waits instead
   // cost 5 us of 110: sixteen branches per tile in between the matrix instructions).
-  auto dma_at = [&](int t, int n, auto issue) __attribute__((always_inline)) {
+  auto base_of = [&](int t, bool of_b) __attribute__((always_inline)) {
     const int tc = min(t, nk - 1) + k_begin;
-    const uint32_t st = lds0 + (t % STAGES) * STAGE_BYTES;
-    if (n < A_DMA) issue(a_base + (int64_t)tc * F_BK * 2, a_voff[n], st + (A_DMA * wave_u + n) * 1024);
-    else issue(b_base + (int64_t)tc * F_BK * p.ldb * 2, b_voff[n - A_DMA], st + A_BYTES + (B_DMA * wave_u + n - A_DMA) * 1024);
+    const char *base = of_b ? b_base + (int64_t)tc * F_BK * p.ldb * 2 : a_base + (int64_t)tc * F_BK * 2;
+#ifdef TTS_GEMM_RTC
+    // (an older run-time compiler does not see that the tile's base address is the same in every lane: say so, here)
+    const uint64_t b = (uint64_t)(uintptr_t)base;
+    uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(b >> 32)), lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)b);
+    asm volatile("" : "+s"(hi), "+s"(lo));
+    base = (const char *)(uintptr_t)(((uint64_t)hi << 32) | (uint64_t)lo);
+#endif
+    return base;
   };
-  auto dma_one = [&](int t, int n) __attribute__((always_inline)) { dma_at(t, n, dma); };
+  auto lds_of = [&](int t, int n) __attribute__((always_inline)) {
+    return lds0 + (t % STAGES) * STAGE_BYTES + (n < A_DMA ? (A_DMA * wave_u + n) * 1024 : A_BYTES + (B_DMA * wave_u + n - A_DMA) * 1024);
+  };
+  auto dma_one = [&](int t, int n) __attribute__((always_inline)) { load_to_lds(base_of(t, n >= A_DMA), n < A_DMA ? a_voff[n] : b_voff[n - A_DMA], lds_of(t, n)); };
 
   const int l16 = lane & 15, q = lane >> 4;
   const int a_off = (wm * 128 + l16) * 64 + ((q ^ a_swizzle((l16 >> 2) & 3)) << 4);
@@ -919,28 +918,23 @@ __device__ __forceinline__ void gemm_dma16_body(const GemmParams &p, int tiles_m
     else
       asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(__builtin_bit_cast(u32x4_r, b)), "v"(__builtin_bit_cast(u32x4_r, a)));
   };
-  // A product and a load behind it.  The matrix instruction is what stands between the write of m0 and the load (4096^3: 99.2 us,
-  // with a scalar instruction there 100.1); a base address that had to be read from a vector register is left to load_to_lds.
-  auto mfma16_and_load = [&](int i, int j, const uint4 &a, const uint4 &b, int t, int n) __attribute__((always_inline)) {
-#ifdef TTS_GEMM_RTC
-    mfma16(i, j, a, b);
-    dma_one(t, n);
-#else
-    dma_at(t, n, [&](const char *sbase, uint32_t voff, uint32_t lds) __attribute__((always_inline)) {
-      if constexpr (BF16)
-        asm volatile("s_mov_b32 m0, %3\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, %0\n\tglobal_load_lds_dwordx4 %4, %5"
-                     : "+a"(acc[i][j]) : "v"(__builtin_bit_cast(u32x4_r, b)), "v"(__builtin_bit_cast(u32x4_r, a)), "s"(lds), "v"(voff), "s"(sbase) : "memory", "m0");
-      else
-        asm volatile("s_mov_b32 m0, %3\n\tv_mfma_f32_16x16x32_f16 %0, %1, %2, %0\n\tglobal_load_lds_dwordx4 %4, %5"
-                     : "+a"(acc[i][j]) : "v"(__builtin_bit_cast(u32x4_r, b)), "v"(__builtin_bit_cast(u32x4_r, a)), "s"(lds), "v"(voff), "s"(sbase) : "memory", "m0");
-    });
-#endif
+  // A product and a load behind it.  The matrix instruction is what stands between the write of m0 and the load; a base address that
+  // had to be read from a vector register is further behind, at the start of the phase.  (4096^3 bf16 against loads without either
+  // wait: 95.3 / 96.4 us, with a compiled epilogue 96.4 / 99.3; through load_to_lds 100.1 / 98.6, 114.7 / 113.6.)
+  auto mfma16_and_load = [&](int i, int j, const uint4 &a, const uint4 &b, const char *base, uint32_t voff, uint32_t lds) __attribute__((always_inline)) {
+    if constexpr (BF16)
+      asm volatile("s_mov_b32 m0, %3\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, %0\n\tglobal_load_lds_dwordx4 %4, %5"
+                   : "+a"(acc[i][j]) : "v"(__builtin_bit_cast(u32x4_r, b)), "v"(__builtin_bit_cast(u32x4_r, a)), "s"(lds), "v"(voff), "s"(base) : "memory", "m0");
+    else
+      asm volatile("s_mov_b32 m0, %3\n\tv_mfma_f32_16x16x32_f16 %0, %1, %2, %0\n\tglobal_load_lds_dwordx4 %4, %5"
+                   : "+a"(acc[i][j]) : "v"(__builtin_bit_cast(u32x4_r, b)), "v"(__builtin_bit_cast(u32x4_r, a)), "s"(lds), "v"(voff), "s"(base) : "memory", "m0");
   };
   auto tile = [&](int t, uint4 (&Ac)[8], uint4 (&An)[8]) __attribute__((always_inline)) {
+    const char *base = base_of(t + STAGES - 1, false);
     static_for<0, 32>([&](auto slot) __attribute__((always_inline)) {
       constexpr int n = decltype(slot)::value;
       __builtin_amdgcn_sched_barrier(0);
-      if constexpr (n % 8 == 7) mfma16_and_load(n >> 2, n & 3, Ac[n >> 2], B0[n & 3], t + STAGES - 1, n / 8);
+      if constexpr (n % 8 == 7) mfma16_and_load(n >> 2, n & 3, Ac[n >> 2], B0[n & 3], base, a_voff[n / 8], lds_of(t + STAGES - 1, n / 8));
       else mfma16(n >> 2, n & 3, Ac[n >> 2], B0[n & 3]);
       if constexpr (n < 8) read_b(t, 4 + (n >> 1), n & 1, B1[n >> 1]);
     });
@@ -948,10 +942,11 @@ __device__ __forceinline__ void gemm_dma16_body(const GemmParams &p, int tiles_m
     // own loads of tile t + 1 have landed (later ones may be in flight); own reads of tile t are complete
     __builtin_amdgcn_s_waitcnt(waitcnt_imm(DMA * (STAGES - 3) + DMA / 2, 0));
     __syncthreads();
+    base = base_of(t + STAGES - 1, true);
     static_for<0, 32>([&](auto slot) __attribute__((always_inline)) {
       constexpr int n = decltype(slot)::value;
       __builtin_amdgcn_sched_barrier(0);
-      if constexpr (n % 8 == 7) mfma16_and_load(n >> 2, 4 + (n & 3), Ac[n >> 2], B1[n & 3], t + STAGES - 1, 4 + n / 8);
+      if constexpr (n % 8 == 7) mfma16_and_load(n >> 2, 4 + (n & 3), Ac[n >> 2], B1[n & 3], base, b_voff[n / 8], lds_of(t + STAGES - 1, A_DMA + n / 8));
       else mfma16(n >> 2, 4 + (n & 3), Ac[n >> 2], B1[n & 3]);
       if constexpr (n < 8) read_a(t + 1, n, An);
       else if constexpr (n < 16) read_b(t + 1, (n - 8) >> 1, n & 1, B0[(n - 8) >> 1]);
