@@ -156,7 +156,7 @@ bool gemm_fast_path_ok(const GemmParams &p) { return !p.a_trans && !p.b_trans &&
 // G: groups of W x W wavefronts that split the K tiles among them and add their sums through LDS at the end, in group order:
 // the chain of loads, LDS stores and matrix instructions of a group is 1 / G as long, and the SIMDs have several to run.
 // All K tiles but the last load 16 bytes a chunk, at any alignment and without a test, two tiles ahead (as gemm_mfma_body).
-// 768^3: 39.3 -> 19.0 us; 16 x 1000 x 1000: 11.7 (27 with 64 x 64 tiles).  (Eight groups at 768^3: 25.3.)
+// 768^3: 39.3 -> 17.6 us; 16 x 1000 x 1000: 11.7 (27 with 64 x 64 tiles).  (Eight groups at 768^3: 25.3.)
 constexpr int F32_BK = 16;
 
 template <int T, int W, int G>
@@ -368,7 +368,7 @@ hipError_t launch_gemm_f32(const GemmParams &p, hipStream_t s) {
     return hipGetLastError();
   };
   // Where the lines lie, us with 64 x 64 tiles / those in two groups / 32 x 32 tiles in four: 400 x 600 x 800 23.1 / 21.7 / 11.9;
-  // 768^3 (576 small tiles) 22.3 / 20.7 / 19.0; 1000^3 (1024) 30.1 / 27.3 / 36.8; 1024 x 2048 x 1024 (512 tiles of 64) 49.0 /
+  // 768^3 (576 small tiles) 22.3 / 20.7 / 17.6; 1000^3 (1024) 30.1 / 27.3 / 36.8; 1024 x 2048 x 1024 (512 tiles of 64) 49.0 /
   // 48.6 / 62.9; 1500 x 1500 x 1000 (576) 65.5 / 67.1 / 75.0.
   if (tiles(128) >= 2 * cus) return launch(gemm_f32_kernel<2, 2, 1>, 128, 256);
   if (2 * tiles(32) <= 5 * cus) return launch(gemm_f32_kernel<1, 1, 4>, 32, 256);

@@ -3,8 +3,8 @@
 //
 // What it replaces: a decode launch per 32 rows (every one reads all of W), and, from 193 rows, a pass that wrote the weights
 // to memory as fp16 (twice their bytes) before an ordinary product.  Here W crosses the memory once per launch.  At
-// [8192, 28672], before -> now: 32 rows 56.7 -> 52.2 us, 48 rows 101 -> 59, 100 rows 202 -> 87, 300 rows 368 -> 136 (1.04
-// PFLOP/s), 1024 rows 524 -> 409; 64 x 4096 x 4096 65 -> 20.
+// [8192, 28672], before -> now, in one run: 32 rows 51.1 -> 43.8 us, 48 rows 92 -> 47, 100 rows 192 -> 68, 300 rows 371 -> 126 (1.12
+// PFLOP/s; 136 on another device), 512 rows 451 -> 209, 1024 rows 523 -> 414; 64 x 4096 x 4096 63 -> 20.
 //
 // Workgroup: 4 wavefronts side by side, each 16 TM rows x 64 columns of C; all four share the A tile.  K advances by 64, two
 // steps of one v_mfma_f32_16x16x32_f16 each.  Both operands go to LDS by `global_load_lds_dwordx4` into a ring of K tiles:
@@ -24,7 +24,8 @@
 // scale (whose products may overflow), an infinite one or a NaN among its columns takes those four: widen, times 512, times s.
 // The weights go in as the first source, so a lane's results are sixteen neighbouring columns of one row (columns 16 q + 4 v +
 // c for result v of instruction c, q = lane / 16): two 16-byte stores per row and lane.
-// What bounds it at 300 rows: the matrix instructions alone take 101 us, widening and LDS reads add 12, the loads 23.  Eight
+// What bounds it at 300 rows: the matrix instructions alone take 101 us, widening and LDS reads add 12, the loads 23 (136 in all on that
+// device; with weights of few significant bits instead of the rounded products 4 us less, which is the power the multipliers draw).  Eight
 // wavefronts that share the rows two ways (the widening done twice) were slower at every size: 177 us.
 #include <algorithm>
 #include <cstdlib>
@@ -248,8 +249,8 @@ __global__ __launch_bounds__(256, 1) void gemm_w8a16_tile_kernel(GemmW8A16Params
 struct W8TileChoice { int tm, tiles_m, tiles_n, split; };
 // Row blocks per tile and K slices: the least modelled time.  A K tile of 64 takes a workgroup 0.2 us and 0.077 us per row
 // block (the matrix pipe), 0.5 us at least (its loads); the weights cross the memory at 5.5 TB/s whatever the tiles; slices
-// cost a second launch and their sums' way through memory.  (Measured at [8192, 28672], model in brackets: 48 rows 59 us (58),
-// 300 rows 136 (131), 400 rows 197 (197), 512 rows 215 (216), 1024 rows 409 (425).)
+// cost a second launch and their sums' way through memory.  (Measured at [8192, 28672], model in brackets: 48 rows 47 to 49 us (58),
+// 300 rows 126 to 136 (131), 400 rows 191 to 204 (197), 512 rows 209 to 224 (216), 1024 rows 414 to 446 (425).)
 W8TileChoice w8_tile_choice(const GemmW8A16Params &p) {
   W8TileChoice best{};
   double best_t = 0;

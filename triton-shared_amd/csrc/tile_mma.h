@@ -2,7 +2,7 @@
 // forward, its backward passes, a product with a chain of products behind it).  Included by tile_codegen.cpp, whose Gen
 // prints index expressions, scalars and elementwise ops.
 //
-// Layout.  Every block of the program has BM rows, and a wavefront owns whole rows: 32 R of them, row 32 rb + lane % 32
+// Layout.  Every block of the program has BM rows, and a wavefront owns whole rows: 32 R of them (R = 1 throughout), row 32 rb + lane % 32
 // in row block rb, both half wavefronts holding half of the row's columns each.  Products are computed transposed --
 // result^T = b^T a^T on v_mfma_f32_32x32x16, so that the instruction's columns (lane % 32) are the block's rows -- and a
 // lane then holds, of every 32 columns, columns 8 g + 4 (lane / 32) + {0..3}, g = 0..3.
@@ -18,7 +18,7 @@
 //     Blocks that stick out of their tensor or are not 16-byte aligned are staged through registers instead.
 // What the ordinary form of the family spends its time on -- operands, products and every reduced row going through LDS
 // element by element between some twenty barriers per iteration -- does not exist here: causal attention of 32 heads x
-// 4096 x 128 in bf16 (64 x 64 blocks) 12.4 ms -> 171 us, 805 TFLOP/s; 32 x 4096 x 64 in fp16, no mask, 2.7 ms -> 217 us.
+// 4096 x 128 in bf16 (64 x 64 blocks) 12.4 ms -> 174 us, 790 TFLOP/s; 32 x 4096 x 64 in fp16, no mask, 2.7 ms -> 217 us.
 // What bounds it: exponentials and the other elementwise work of the softmax, some nine vector instructions per score
 // (the exponential counts four), against 8 matrix-pipe cycles per score of a wavefront at D = 128; two workgroups per CU
 // (256 registers a lane) run their phases against each other, so that one's products hide the other's exponentials.
