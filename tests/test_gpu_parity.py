@@ -763,7 +763,8 @@ def test_w8a16_tiled_kernel_rounds_weights_as_the_program_does(K, M, N, Kd):
     s[:4] = torch.tensor([0.0, -0.0, 511.75, 2.0 ** -24])
     s[-8:] = torch.tensor([512.0, -600.0, 65504.0, float("inf"), -float("inf"), float("nan"), 0.001, 2.0 ** -15])
     cd = torch.full((M + 1, N), 5.0, dtype=torch.float16, device=DEV)
-    k = K.w8a16_matmul[(triton.cdiv(M, 64), triton.cdiv(N, 128))](a.to(DEV), w.to(DEV), s.to(DEV), cd, M, N, Kd, Kd, 1, N, 1, N, 1, BM=64, BN=128, BK=64)
+    sd = torch.cat([torch.full((1,), float("nan"), dtype=torch.float16), s]).to(DEV)[1:]   # (from an odd element on)
+    k = K.w8a16_matmul[(triton.cdiv(M, 64), triton.cdiv(N, 128))](a.to(DEV), w.to(DEV), sd, cd, M, N, Kd, Kd, 1, N, 1, N, 1, BM=64, BN=128, BK=64)
     torch.cuda.synchronize()
     assert k.function.last_kernel == "gemm_w8a16_tile_kernel"
     want = (a.double() @ (w.half() * s).double()).half()   # (0 x infinity is a NaN on both sides)
