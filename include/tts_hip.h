@@ -85,7 +85,8 @@ tts_status tts_launch(tts_plan *plan, int grid_x, int grid_y, int grid_z, void *
  * the call never allocates or frees device memory and never compiles: the split-K partial tiles and arrival counters
  * of the int8-weight product, and the partial sums of a matrix product that runs in K slices, live in a static device
  * array (8 MiB + 4096 counters per GPU, held until the process ends; its address is looked up with
- * hipGetSymbolAddress at the first call on each device).  An int8-weight launch whose partial tiles exceed that, or
+ * hipGetSymbolAddress at the first call on each device).  A launch of the int8-weight product's decode kernels whose
+ * partial tiles exceed that (the tiled kernel for more rows runs without slices instead), or
  * a launch that would need a run-time compiled kernel or a device-side table that no earlier tts_launch of the plan
  * has created yet, returns TTS_UNSUPPORTED with the reason; a matrix product runs in as many slices as fit there, or
  * without slices.  All calls on one GPU share the array:
