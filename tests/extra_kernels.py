@@ -1576,3 +1576,46 @@ def block_column_sums(x_ptr, out_ptr, rows, n_cols, BR: tl.constexpr, BC: tl.con
         r = r0 + tl.arange(0, BR)
         acc += tl.load(x_ptr + (b * rows + r[:, None]) * n_cols + c[None, :], mask=(r[:, None] < rows) & (c[None, :] < n_cols), other=0.0)
     tl.store(out_ptr + (b + tl.arange(0, 1))[:, None] * n_cols + c[None, :], tl.sum(acc, axis=0)[None, :], mask=c[None, :] < n_cols)
+
+
+@triton.jit
+def attention_scaled_maximum(Q, K, V, O, sm_scale, seq, stride_h, stride_s, BM: tl.constexpr, BN: tl.constexpr, D: tl.constexpr, CAUSAL: tl.constexpr, BASE2: tl.constexpr):
+    # flash-attention forward whose scores are scaled after their maximum was taken (the scale on the maximum alone), exponentials to
+    # base 2 or e; l starts at 1 beside a maximum of -inf
+    pm = tl.program_id(0)
+    ph = tl.program_id(1)
+    rm = pm * BM + tl.arange(0, BM)
+    rd = tl.arange(0, D)
+    q = tl.load(Q + ph * stride_h + rm[:, None] * stride_s + rd[None, :], mask=rm[:, None] < seq, other=0.0)
+    m_i = tl.zeros([BM], dtype=tl.float32) - float("inf")
+    l_i = tl.zeros([BM], dtype=tl.float32) + 1.0
+    acc = tl.zeros([BM, D], dtype=tl.float32)
+    qk_scale = sm_scale
+    if BASE2:
+        qk_scale *= 1.44269504
+    last = seq
+    if CAUSAL:
+        last = tl.minimum(seq, (pm + 1) * BM)
+    for start in range(0, last, BN):
+        rn = start + tl.arange(0, BN)
+        k = tl.load(K + ph * stride_h + rn[:, None] * stride_s + rd[None, :], mask=rn[:, None] < seq, other=0.0)
+        v = tl.load(V + ph * stride_h + rn[:, None] * stride_s + rd[None, :], mask=rn[:, None] < seq, other=0.0)
+        qk = tl.dot(q, tl.trans(k))
+        if CAUSAL:
+            qk = tl.where((rn[None, :] < seq) & (rm[:, None] >= rn[None, :]), qk, -1.0e6)
+        else:
+            qk = tl.where(rn[None, :] < seq, qk, -1.0e6)
+        m_ij = tl.maximum(m_i, tl.max(qk, 1) * qk_scale)
+        qk = qk * qk_scale - m_ij[:, None]
+        if BASE2:
+            p = tl.exp2(qk)
+            alpha = tl.exp2(m_i - m_ij)
+        else:
+            p = tl.exp(qk)
+            alpha = tl.exp(m_i - m_ij)
+        l_i = l_i * alpha + tl.sum(p, 1)
+        acc = acc * alpha[:, None]
+        acc = tl.dot(p.to(V.dtype.element_ty), v, acc)
+        m_i = m_ij
+    acc = acc / l_i[:, None]
+    tl.store(O + ph * stride_h + rm[:, None] * stride_s + rd[None, :], acc.to(O.dtype.element_ty), mask=rm[:, None] < seq)

@@ -1028,6 +1028,28 @@ def test_matrix_programs_and_add_only_loops_on_grids_of_more_than_2_to_the_24_pr
     assert torch.equal(out[:3].double(), torch.stack([p, q, p - 2 * q])) and (out[3] == 9.0).all()
 
 
+@pytest.mark.parametrize("base2", [False, True])
+@pytest.mark.parametrize("scale,D,BM,seq,causal", [(0.125, 64, 64, 200, True), (-0.1, 64, 64, 128, False), (0.0, 64, 32, 64, False), (3.0, 128, 128, 257, True)])
+def test_matrix_program_attention_scaled_after_its_maximum(base2, scale, D, BM, seq, causal):
+    # (with a negative scale the program's maximum is its scores' minimum: exponentials above 1, and still a softmax.  Masked
+    # scores of -1e6 times such a scale, or zero, would count: no masks there)
+    import extra_kernels as X
+    torch.manual_seed(seq)
+    H = 2
+    q, k, v = (torch.randn(H, seq, D, device=DEV).half() for _ in range(3))
+    o = torch.full((H + 1, seq, D), 3.0, device=DEV, dtype=torch.float16)
+    kern = X.attention_scaled_maximum[(triton.cdiv(seq, BM), H)](q, k, v, o, scale, seq, q.stride(0), q.stride(1), BM=BM, BN=32, D=D, CAUSAL=causal, BASE2=base2)
+    torch.cuda.synchronize()
+    assert kern.function.last_kernel == "tile_program (hipRTC, matrix layout)"
+    s = torch.matmul(q.cpu().double(), k.cpu().double().transpose(1, 2))
+    if causal:
+        s.masked_fill_(torch.triu(torch.ones(seq, seq, dtype=torch.bool), 1), -1.0e6)
+    want = torch.matmul(torch.softmax(s * scale, -1), v.cpu().double())
+    # probabilities and results are each rounded once to 16 bits: half an ulp of |v| and of |o| <= max |v|
+    assert (o[:H].cpu().double() - want).abs().max().item() <= 2.0 ** -10 * v.abs().max().item()
+    assert (o[H] == 3.0).all()
+
+
 @pytest.mark.parametrize("BM,n,n_s", [(32, 33, 1), (64, 130, 1), (128, 100, 0)])
 def test_matrix_program_with_vectors_of_one_element(BM, n, n_s):
     import extra_kernels as X

@@ -786,3 +786,18 @@ def test_loops_that_leave_nothing_in_lds_end_without_a_barrier(native, tmp_path)
     assert "carm0_" in src
     end = src[:src.index("\n  }\n", src.rindex("carm0_1[t]"))].rsplit("carm0_", 1)[1]
     assert end.count("__syncthreads();") == 1, end
+
+
+@pytest.mark.parametrize("base2", [False, True])
+def test_matrix_programs_ask_for_the_sign_of_a_scale_between_a_maximum_and_its_scores(native, tmp_path, base2):
+    """max(scores) * scale is the maximum of scores * scale if the scale is not negative: the kernel looks, and computes the
+    library's exponential otherwise."""
+    import extra_kernels as X
+    sig = {**{x: "*fp16" for x in "QKVO"}, "sm_scale": "fp32", **{x: "i32" for x in ("seq", "stride_h", "stride_s")}, **{x: "constexpr" for x in ("BM", "BN", "D", "CAUSAL", "BASE2")}}
+    src = _generic_source(tmp_path, compile_ttir(X.attention_scaled_maximum, sig, {"BM": 64, "BN": 64, "D": 64, "CAUSAL": True, "BASE2": base2}))
+    body = src[src.index("void tile_program"):]
+    at = body.index(">= 0.f) {")
+    assert "p.fval[4]" in body[body.rindex("if (", 0, at):at]
+    chosen = body[at:body.index("}\n", body.index("} else {", at))]
+    fast, otherwise = chosen.split("} else {")
+    assert "__builtin_amdgcn_exp2f(" in fast and "__builtin_amdgcn_exp2f(" not in otherwise and (" exp2f(" if base2 else " expf(") in otherwise

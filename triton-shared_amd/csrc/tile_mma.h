@@ -375,31 +375,78 @@ struct MmaGen : Gen {
     if (d->kind == SK::Broadcast || d->kind == SK::ExpandDims) return is_maximum_over(d->operands.at(0), x, depth + 1);
     return d->kind == SK::Map && max && (is_maximum_over(d->operands.at(0), x, depth + 1) || is_maximum_over(d->operands.at(1), x, depth + 1));
   }
-  const SOp *difference_against_maximum(const SOp &s) const {  // the subtraction behind such an exponential
+  // a product of a block (or row) with a scalar that is the same everywhere: the other factor and the scalar's value id
+  bool scaled(int v, int *factor, int *scalar) const {
+    const SOp *d = def_of(v);
+    if (!d || d->kind != SK::Map || d->name != "arith.mulf" || val(v).dtype != "f32") return false;
+    for (int q = 0; q < 2; q++) {
+      const SOp *o = def_of(d->operands[q]);
+      if (!o || o->kind != SK::Splat) continue;
+      *scalar = o->operands.at(0);
+      *factor = d->operands[1 - q];
+      return true;
+    }
+    return false;
+  }
+  // is m a maximum of values one of which is `scalar` times a maximum over x?  (With scalar >= 0 that is one over scalar * x.)
+  bool is_scaled_maximum_over(int m, int x, int scalar, int depth = 0) const {
+    const SOp *d = def_of(m);
+    if (!d || depth > 16) return false;
+    int f = -1, s = -1;
+    if (scaled(m, &f, &s) && s == scalar) return is_maximum_over(f, x);
+    if (d->kind == SK::Broadcast || d->kind == SK::ExpandDims) return is_scaled_maximum_over(d->operands.at(0), x, scalar, depth + 1);
+    const bool max = d->kind == SK::Map && (d->name == "arith.maxnumf" || d->name == "arith.maximumf");
+    return max && (is_scaled_maximum_over(d->operands.at(0), x, scalar, depth + 1) || is_scaled_maximum_over(d->operands.at(1), x, scalar, depth + 1));
+  }
+  // The subtraction behind such an exponential; `*scalar`: it is one if this scalar is not negative (scores scaled after their
+  // maximum was taken), which the kernel asks -- or -1.
+  const SOp *difference_against_maximum(const SOp &s, int *scalar) const {
+    *scalar = -1;
     if (!fast_exp || s.kind != SK::Map || (s.name != "math.exp" && s.name != "math.exp2") || val(s.result).dtype != "f32") return nullptr;
     const SOp *d = def_of(s.operands[0]);
-    return d && d->kind == SK::Map && d->name == "arith.subf" && is_maximum_over(d->operands[1], d->operands[0]) ? d : nullptr;
+    if (!d || d->kind != SK::Map || d->name != "arith.subf") return nullptr;
+    if (is_maximum_over(d->operands[1], d->operands[0])) return d;
+    int f = -1, by = -1;
+    if (!scaled(d->operands[0], &f, &by) || !is_scaled_maximum_over(d->operands[1], f, by)) return nullptr;
+    *scalar = by;
+    return d;
   }
+  std::string hardware_exp(const SOp &s, const std::string &x) const { return "__builtin_amdgcn_exp2f(" + x + (s.name == "math.exp" ? " * TTS_LOG2E)" : ")"); }
   std::string map_text(const SOp &s, const std::vector<std::string> &a) {
-    if (difference_against_maximum(s)) return std::string("__builtin_amdgcn_exp2f(") + a.at(0) + (s.name == "math.exp" ? " * TTS_LOG2E)" : ")");
-    return map_expr(s, a);
+    int scalar = -1;
+    return difference_against_maximum(s, &scalar) && scalar < 0 ? hardware_exp(s, a.at(0)) : map_expr(s, a);
   }
   // The same with the difference written where it is read.  It is taken before the factor log2 e: with fma(x, log2e, -m log2e) a
   // row of the type's lowest values (all keys masked with a finite number) is infinity minus infinity, and m log2e rounds by up
   // to |m| 2^-24 of the exponent.
-  bool exp_of_difference(const SOp &s, int role, std::string *text) {
-    const SOp *d = difference_against_maximum(s);
-    if (!d || role != TILE) return false;
-    const std::string x = el(d->operands[0], role), m = el(d->operands[1], role);
-    *text = map_text(s, {"(" + x + " - " + m + ")"});
+  bool emit_exp_of_difference(const SOp &s) {
+    int scalar = -1;
+    const SOp *d = difference_against_maximum(s, &scalar);
+    if (!d) return false;
+    const std::string n = declare_tile(s.result), x = "(" + el(d->operands[0], TILE) + " - " + el(d->operands[1], TILE) + ")";
+    if (scalar >= 0) {
+      line("if (" + at(scalar, "0", "0") + " >= 0.f) {");
+      indent++;
+    }
+    tile_loop(s.result, n + "[rb][nb][i] = " + hardware_exp(s, x) + ";");
+    if (scalar >= 0) {
+      indent--;
+      line("} else {");
+      indent++;
+      tile_loop(s.result, n + "[rb][nb][i] = " + map_expr(s, {x}) + ";");
+      indent--;
+      line("}");
+    }
+    tile_of[s.result] = n;
     return true;
   }
   bool folded_into_exp(const SOp &s) const {  // a difference that only such exponentials read is written there
     if (s.name != "arith.subf") return false;
     auto u = users.find(s.result);
     if (u == users.end()) return false;
+    int scalar = -1;
     for (const SOp *o : u->second)
-      if (!difference_against_maximum(*o)) return false;
+      if (!difference_against_maximum(*o, &scalar)) return false;
     return true;
   }
 
@@ -572,11 +619,10 @@ struct MmaGen : Gen {
           tile_of[v] = n;
           return;
         }
-      if (!exp_of_difference(s, TILE, &text)) {
-        std::vector<std::string> a;
-        for (int o : s.operands) a.push_back(el(o, TILE));
-        text = map_text(s, a);
-      }
+      if (emit_exp_of_difference(s)) return;
+      std::vector<std::string> a;
+      for (int o : s.operands) a.push_back(el(o, TILE));
+      text = map_text(s, a);
       const std::string n = declare_tile(v);
       tile_loop(v, n + "[rb][nb][i] = " + text + ";");
       tile_of[v] = n;
