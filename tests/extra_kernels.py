@@ -1619,3 +1619,19 @@ def attention_scaled_maximum(Q, K, V, O, sm_scale, seq, stride_h, stride_s, BM: 
         m_i = m_ij
     acc = acc / l_i[:, None]
     tl.store(O + ph * stride_h + rm[:, None] * stride_s + rd[None, :], acc.to(O.dtype.element_ty), mask=rm[:, None] < seq)
+
+
+@triton.jit
+def mixed_rows_less_their_maximum(x_ptr, r_ptr, k_ptr, b_ptr, y_ptr, z_ptr, n_cols, pitch, BLOCK: tl.constexpr):
+    """16-bit, fp32, 32-bit and 8-bit integer blocks of one shape in one program: each row's sum of them less its largest element, as 16 bits and as fp32."""
+    row = tl.program_id(0)
+    cols = tl.arange(0, BLOCK)
+    live = cols < n_cols
+    x = tl.load(x_ptr + row * pitch + cols, mask=live, other=-1000.0).to(tl.float32)
+    r = tl.load(r_ptr + row * pitch + cols, mask=live, other=0.0)
+    k = tl.load(k_ptr + row * pitch + cols, mask=live, other=0).to(tl.float32)
+    b = tl.load(b_ptr + row * pitch + cols, mask=live, other=0).to(tl.float32)
+    v = ((x + r) + k) + b
+    v = v - tl.max(v, axis=0)
+    tl.store(y_ptr + row * pitch + cols, v.to(y_ptr.dtype.element_ty), mask=live)
+    tl.store(z_ptr + row * pitch + cols, v, mask=live)

@@ -2305,6 +2305,37 @@ def test_tile_program_wide_rows_of_random_extent_and_alignment():
         assert (yb[:lead] == 5.0).all() and (yb[lead + total:] == 5.0).all(), (trial, batches, rows, n, lead)
 
 
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("n_cols", [1, 7, 8, 9, 15, 16, 2041, 2047, 2048, 2049, 3999, 4089, 4095, 4096])
+def test_tile_program_wide_groups_that_the_extent_cuts_off(dtype, n_cols):
+    """The last group of eight of a row is read from the row's last eight elements and moved into place (16-bit, 4-byte and
+    1-byte elements), rows of fewer than eight element by element; rows start at every offset from a 16-byte boundary.
+    Sums of at most four terms and a maximum: exact against torch, nothing written outside the rows."""
+    import extra_kernels as X
+    torch.manual_seed(n_cols)
+    dt = getattr(torch, dtype)
+    rows = 9
+    pitch = n_cols + (3 if n_cols % 2 else 1)  # (odd or even with the extent: rows drift over all offsets)
+    def rows_of(t):
+        buf = torch.zeros(5 + rows * pitch, device=DEV, dtype=t.dtype)
+        view = buf[5:].view(rows, pitch)
+        view[:, n_cols:] = 55                   # what a load past the extent would bring in
+        view[:, :n_cols] = t
+        return view
+    x = rows_of(torch.randn(rows, n_cols, device=DEV).to(dt))
+    r = rows_of(torch.randn(rows, n_cols, device=DEV))
+    k = rows_of(torch.randint(-4, 5, (rows, n_cols), device=DEV, dtype=torch.int32))
+    b = rows_of(torch.randint(-9, 9, (rows, n_cols), device=DEV, dtype=torch.int8))
+    y, z = rows_of(torch.zeros(rows, n_cols, device=DEV, dtype=dt)), rows_of(torch.zeros(rows, n_cols, device=DEV))
+    h = X.mixed_rows_less_their_maximum[(rows,)](x, r, k, b, y, z, n_cols, pitch, BLOCK=4096)
+    torch.cuda.synchronize()
+    assert h.function.family == "tile_program"
+    v = ((x.float() + r) + k.float()) + b.float()
+    v = v[:, :n_cols] - v[:, :n_cols].amax(1, keepdim=True)
+    assert torch.equal(z[:, :n_cols], v) and torch.equal(y[:, :n_cols], v.to(dt))
+    assert (z[:, n_cols:] == 55).all() and (y[:, n_cols:] == 55).all()
+
+
 @pytest.mark.parametrize("n_cols,pitch,lead", [(4096, 4096, 0), (4000, 4000, 0), (4093, 4099, 0), (2048, 2048, 5)])
 def test_tile_program_wide_rows_with_int8_neighbours(n_cols, pitch, lead):
     """Row-wise int8 quantisation and its inverse: 1-byte blocks next to 16-bit ones take the wide element order too

@@ -546,6 +546,10 @@ struct Gen {
     return sum;
   }
 
+  // How many of the eight elements from index i on (along the contiguous dimension) the extent cuts off.
+  std::string cut_off(const Access &a, const std::string &i) {
+    return "(int)smax(0LL, " + i + " + 8 - (" + ex(a.dims.back()) + "))";
+  }
   std::string mem_read(const Access &a, const std::string &addr) {
     const std::string ptr = "((const " + memtype(a.elem) + " *)p.ptr[" + std::to_string(a.base_arg) + "])[" + addr + "]";
     if (a.elem == "f16") return "up_f16(" + ptr + ")";
@@ -673,7 +677,9 @@ struct Gen {
   // contiguous, one element per lane.  For 16-bit data that is 2 bytes per lane and access; a program whose blocks of
   // 16-bit elements have whole groups of 2048 along the contiguous dimension is written "wide" instead: a thread owns
   // eight neighbouring elements, t = 8 threadIdx.x + (n & 7) + 2048 (n >> 3), and a group of eight that is valid as a
-  // whole and 16-byte aligned moves in one access (two for 4-byte elements).  Only blocks of the one shape `wide_shape`
+  // whole moves in one access (two for 4-byte elements), at any alignment: gfx950 reads and writes 16 bytes at any address
+  // (LayerNorm's input gradient on fp16 [8192, 5003], whose rows start anywhere: 146 us element by element, 64 this way;
+  // [4096, 8192], all aligned: 35 either way).  Only blocks of the one shape `wide_shape`
   // are laid out that way; every other shape of the program keeps the ordinary order.  Programs with scans, matrix
   // products or index shuffles (whose code relies on the ordinary order) are never wide.
   bool wide_mode = false;
@@ -1228,12 +1234,12 @@ struct Gen {
             close_loop();
             fill.clear();
           };
-          // Wide blocks: when every group of eight of these loads starts on a 16-byte boundary (the same answer in every
-          // thread of the program: the block's first element is aligned and, for blocks of rows, so is the row pitch), a
-          // group moves in one 16-byte access (two for 4-byte elements), unconditionally: a group whose first element is
-          // valid is read whole (what lies past the valid extent inside an aligned 16 bytes is on the same page), any
-          // other from a dummy; a second loop unpacks, widens and fills in `other`.  No branch sits between the loads, so
-          // none waits for another.  Otherwise the loads go element by element, as they would in the ordinary order.
+          // Wide blocks: a group of eight elements moves in one 16-byte access (two for 4-byte elements, one of 8 bytes for
+          // 1-byte ones) at whatever alignment it has, unconditionally: a group that is valid as a whole is read where it
+          // stands, the one that the extent cuts off is read from the last eight valid elements of its row and moved down
+          // afterwards (drop_front), any other from a dummy; a second loop unpacks, widens and fills in `other`.  No branch
+          // sits between the loads, so none waits for another.  Only a program whose extent is one to seven elements loads
+          // element by element, as it would in the ordinary order.
           auto wide_load_any = [&](const SOp &o) { return wide(ls) && mine_here(o) && vector_access(o.acc); };
           for (int pass = 0; pass < 2; pass++) {  // pass 0: the loads hoisted out of the program loop, into hoist_os
             auto wide_load = [&](const SOp &o) { return wide_load_any(o) && (hoisted.count(o.result) != 0) == (pass == 0); };
@@ -1248,18 +1254,13 @@ struct Gen {
             if (any_wide) {
               const int64_t G = count(ls) / 2048;
               uses_dummy = true;
-              std::string aligned;
+              std::string roomy;  // the extents of the masked ones leave eight elements to read, or none (the same in every thread)
               for (size_t q = k; q < end; q++)
-                if (wide_load(ops[q])) {
-                  const SOp &o = ops[q];
-                  std::string unused;
-                  const int esz = mem_bytes(o.acc.elem);
-                  const std::string mask = esz == 1 ? "7" : "15";  // a group of eight 1-byte elements is one 8-byte access
-                  aligned += std::string(aligned.empty() ? "" : " && ") + "((unsigned long long)((const " + memtype(o.acc.elem) + " *)p.ptr[" + std::to_string(o.acc.base_arg) +
-                             "] + (" + address(o.acc, "0", "0", unused) + ")) & " + mask + ") == 0";
-                  if (ls.size() == 2) aligned += " && (((unsigned long long)(" + ex(o.acc.strides[0]) + ") * " + std::to_string(esz) + ") & " + mask + ") == 0";
+                if (wide_load(ops[q]) && !ops[q].acc.dims.empty()) {
+                  const std::string ext = "(" + ex(ops[q].acc.dims.back()) + ")";
+                  if (roomy.find(ext) == std::string::npos) roomy += std::string(roomy.empty() ? "" : " && ") + "(" + ext + " <= 0 || " + ext + " >= 8)";
                 }
-              os << pad() << "if (" << aligned << ") {\n";
+              os << pad() << "if (" << (roomy.empty() ? "true" : roomy) << ") {\n";
               indent++;
               for (size_t q = k; q < end; q++)
                 if (wide_load(ops[q]) && !packed(ops[q]))
@@ -1274,21 +1275,38 @@ struct Gen {
                   std::string pred, addr = address(o.acc, l0, l1, pred);
                   os << pad() << "{\n";
                   indent++;
-                  const std::string vt = mem_bytes(o.acc.elem) == 1 ? "u32x2_t" : "u32x4_t";
-                  os << pad() << "const " << vt << " *const src = " << (pred.empty() ? "" : "!(" + pred + ") ? (const " + vt + " *)tts_dummy : ") << "(const " << vt << " *)((const " << mt
-                     << " *)p.ptr[" << o.acc.base_arg << "] + (" << addr << "));\n";
+                  const std::string vt = mem_bytes(o.acc.elem) == 1 ? "u32x2_any" : "u32x4_any";
+                  if (pred.empty())
+                    os << pad() << "const " << vt << " *const src = (const " << vt << " *)((const " << mt << " *)p.ptr[" << o.acc.base_arg << "] + (" << addr << "));\n";
+                  else
+                    os << pad() << "const " << vt << " *const src = !(" << pred << ") ? (const " << vt << " *)tts_dummy : (const " << vt << " *)((const " << mt << " *)p.ptr["
+                       << o.acc.base_arg << "] + (" << addr << ") - " << cut_off(o.acc, ls.size() < 2 ? l0 : l1) << ");\n";
                   if (mem_bytes(o.acc.elem) <= 2) os << pad() << "rw" << id << "[g] = src[0];\n";
-                  else {  // the second 16 bytes may lie on another page than the first: read only if their first element is valid
-                    std::string pred4;
-                    address(o.acc, along(ls, l0, " + 4").first, along(ls, l1, " + 4").second, pred4);
-                    os << pad() << "rw" << id << "[2 * g] = src[0];\n" << pad() << "rw" << id << "[2 * g + 1] = "
-                       << (pred4.empty() ? "src[1]" : "*(!(" + pred4 + ") ? (const u32x4_t *)tts_dummy : src + 1)") << ";\n";
-                  }
+                  else os << pad() << "rw" << id << "[2 * g] = src[0];\n" << pad() << "rw" << id << "[2 * g + 1] = src[1];\n";
                   indent--;
                   os << pad() << "}\n";
                 }
               indent--;
               os << pad() << "}\n";
+              for (size_t q = k; q < end; q++)
+                if (wide_load(ops[q]) && !ops[q].acc.dims.empty()) {
+                  const SOp &o = ops[q];
+                  const std::string id = std::to_string(o.result);
+                  const int esz = mem_bytes(o.acc.elem);
+                  std::string pred;
+                  address(o.acc, l0, l1, pred);
+                  os << pad() << "if (" << ex(o.acc.dims.back()) << " & 7) {\n";
+                  indent++;
+                  os << pad() << "#pragma unroll\n" << pad() << "for (int g = 0; g < " << G << "; g++) {\n";
+                  indent++;
+                  os << pad() << "const int n = 8 * g;\n" << pad() << "const int t = " << element_of_slot(ls) << ";\n" << pad() << "(void)t;\n";
+                  os << pad() << "const int cut = (" << pred << ") ? " << cut_off(o.acc, ls.size() < 2 ? l0 : l1) << " : 0;\n";
+                  os << pad() << "if (cut) " << (esz == 4 ? "drop_front_32(rw" + id + "[2 * g], rw" + id + "[2 * g + 1], cut)" : (esz == 2 ? "drop_front_16(rw" : "drop_front_8(rw") + id + "[g], cut)") << ";\n";
+                  indent--;
+                  os << pad() << "}\n";
+                  indent--;
+                  os << pad() << "}\n";
+                }
               bool any_packed = false, any_unpacked = false;
               for (size_t q = k; q < end; q++) {
                 any_packed = any_packed || (wide_load(ops[q]) && packed(ops[q]));
@@ -1465,8 +1483,8 @@ struct Gen {
             const Value &sv = val(o.operands.at(0));
             if (sv.shape != shape) no("a stored value whose shape is not the block's");
             if (two_phase && wide(shape) && vector_access(o.acc)) {
-              // the eighth element of a group writes the group: one 16-byte access (two for 4-byte elements) when all
-              // eight are valid and the first is 16-byte aligned, element by element otherwise
+              // the eighth element of a group writes the group: one 16-byte access (two for 4-byte elements) at any
+              // alignment when all eight are valid, element by element otherwise
               const bool half = is16(o.acc.elem), byte = mem_bytes(o.acc.elem) == 1;
               const std::string sv = "sv" + std::to_string(q), mt = memtype(o.acc.elem), value = at(o.operands[0], i0, i1);
               const std::string bits = o.acc.elem == "f16" ? "(unsigned)down_f16_exact(" + value + ")" : o.acc.elem == "bf16" ? "(unsigned)down_bf16(" + value + ")"
@@ -1478,16 +1496,16 @@ struct Gen {
               os << pad() << "if ((n & 7) == 7) {\n";
               indent++;
               os << pad() << mt << " *const dst = (" << mt << " *)p.ptr[" << o.acc.base_arg << "] + (" << addr0 << ");\n";
-              os << pad() << "if (" << (pred_last.empty() ? "" : "(" + pred_last + ") && ") << "((unsigned long long)dst & " << (byte ? 7 : 15) << ") == 0) {\n";
+              os << pad() << "if (" << (pred_last.empty() ? "true" : pred_last) << ") {\n";
               if (byte)
                 os << pad() << "  __builtin_nontemporal_store(u32x2_t{" << sv << "[0] | " << sv << "[1] << 8 | " << sv << "[2] << 16 | " << sv << "[3] << 24, " << sv << "[4] | " << sv
-                   << "[5] << 8 | " << sv << "[6] << 16 | " << sv << "[7] << 24}, (u32x2_t *)dst);\n";
+                   << "[5] << 8 | " << sv << "[6] << 16 | " << sv << "[7] << 24}, (u32x2_any *)dst);\n";
               else if (half)
                 os << pad() << "  __builtin_nontemporal_store(u32x4_t{" << sv << "[0] | " << sv << "[1] << 16, " << sv << "[2] | " << sv << "[3] << 16, " << sv << "[4] | " << sv
-                   << "[5] << 16, " << sv << "[6] | " << sv << "[7] << 16}, (u32x4_t *)dst);\n";
+                   << "[5] << 16, " << sv << "[6] | " << sv << "[7] << 16}, (u32x4_any *)dst);\n";
               else
-                os << pad() << "  __builtin_nontemporal_store(u32x4_t{" << sv << "[0], " << sv << "[1], " << sv << "[2], " << sv << "[3]}, (u32x4_t *)dst);\n"
-                   << pad() << "  __builtin_nontemporal_store(u32x4_t{" << sv << "[4], " << sv << "[5], " << sv << "[6], " << sv << "[7]}, (u32x4_t *)dst + 1);\n";
+                os << pad() << "  __builtin_nontemporal_store(u32x4_t{" << sv << "[0], " << sv << "[1], " << sv << "[2], " << sv << "[3]}, (u32x4_any *)dst);\n"
+                   << pad() << "  __builtin_nontemporal_store(u32x4_t{" << sv << "[4], " << sv << "[5], " << sv << "[6], " << sv << "[7]}, (u32x4_any *)dst + 1);\n";
               os << pad() << "} else {\n";
               os << pad() << "  #pragma unroll\n" << pad() << "  for (int e = 0; e < 8; e++)\n";
               os << pad() << "    if (" << (pred_e.empty() ? "true" : pred_e) << ") " << (byte ? "dst[e] = (signed char)" + sv + "[e]" : half ? "dst[e] = (unsigned short)" + sv + "[e]" : "((unsigned *)dst)[e] = " + sv + "[e]") << ";\n";
@@ -2312,6 +2330,23 @@ __device__ inline long long wrap(long long x, long long m) { return m > 0 ? ((x 
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef unsigned u32x4_t __attribute__((ext_vector_type(4)));
 typedef unsigned u32x2_t __attribute__((ext_vector_type(2)));
+typedef u32x4_t __attribute__((aligned(1))) u32x4_any;  // in memory at any address
+typedef u32x2_t __attribute__((aligned(1))) u32x2_any;
+// eight elements without their first k (1 .. 7), moved to the front
+__device__ inline void drop_front_16(u32x4_t &v, int k) {
+  if (k & 4) v = u32x4_t{v[2], v[3], 0, 0};
+  if (k & 2) v = u32x4_t{v[1], v[2], v[3], 0};
+  if (k & 1) v = u32x4_t{v[0] >> 16 | v[1] << 16, v[1] >> 16 | v[2] << 16, v[2] >> 16 | v[3] << 16, v[3] >> 16};
+}
+__device__ inline void drop_front_32(u32x4_t &a, u32x4_t &b, int k) {
+  if (k & 4) a = b;
+  if (k & 2) { a = u32x4_t{a[2], a[3], b[0], b[1]}; b = u32x4_t{b[2], b[3], 0, 0}; }
+  if (k & 1) { a = u32x4_t{a[1], a[2], a[3], b[0]}; b = u32x4_t{b[1], b[2], b[3], 0}; }
+}
+__device__ inline void drop_front_8(u32x2_t &v, int k) {
+  if (k & 4) v = u32x2_t{v[1], 0};
+  if (k & 3) v = u32x2_t{v[0] >> (8 * (k & 3)) | v[1] << (32 - 8 * (k & 3)), v[1] >> (8 * (k & 3))};
+}
 typedef unsigned short u16x8_t __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
