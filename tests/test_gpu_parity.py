@@ -156,6 +156,59 @@ def test_layernorm_shapes(K, oracle_cpu, M, N, dtype):
     assert (mean - mr).abs().max().item() <= 1e-5 and ((rstd - rr) / rr).abs().max().item() <= 1e-5
 
 
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16", "float32"])
+@pytest.mark.parametrize("M,N", [(5, 3), (9, 8), (9, 9), (4200, 257), (5, 511), (4200, 513), (1030, 1023), (70, 1025), (1030, 2047), (9, 2049),
+                                 (4100, 4095), (4200, 4097), (4100, 6145), (4200, 8190), (6, 9001), (5, 16383)])
+def test_layernorm_rows_at_any_alignment(K, dtype, M, N):
+    """Rows that start and end anywhere: a wavefront or a workgroup per row, and workgroups that walk the rows.  A sum of N
+    terms over T lanes rounds N / T + log2 T times at most; 32 ulp of fp32 for the statistics, one more rounding for y."""
+    torch.manual_seed(M + N)
+    dt = getattr(torch, dtype)
+    pitch = N + (2 if N % 2 else 1)
+    buf = torch.full((3 + M * pitch,), 9.0, device=DEV, dtype=dt)
+    x = buf[3:].view(M, pitch)[:, :N]
+    x.copy_(torch.randn(M, N, device=DEV) + 0.3)
+    w, b = (torch.zeros(N + 1, device=DEV, dtype=dt)[1:].copy_(torch.randn(N, device=DEV)) for _ in range(2))
+    yb = torch.full((1 + M * pitch + 8,), 5.0, device=DEV, dtype=dt)
+    y = yb[1:1 + M * pitch].view(M, pitch)[:, :N]
+    mean, rstd = torch.zeros(M, device=DEV), torch.zeros(M, device=DEV)
+    k = K.layer_norm_fwd[(M,)](x, y, w, b, mean, rstd, pitch, N, 1e-5, BLOCK=1024)
+    torch.cuda.synchronize()
+    assert k.function.family == "layernorm_fwd"
+    xd = x.double()
+    mu = xd.mean(1)
+    rs = 1 / torch.sqrt(((xd - mu[:, None]) ** 2).mean(1) + 1e-5)
+    want = (xd - mu[:, None]) * rs[:, None] * w.double() + b.double()
+    eps = 2.0 ** -19
+    assert ((mean - mu).abs() <= eps * xd.abs().mean(1)).all() and ((rstd - rs).abs() <= eps * rs * (1 + rs * mu.abs())).all()
+    ulp = {"float16": 2.0 ** -11, "bfloat16": 2.0 ** -8, "float32": 0.0}[dtype]
+    size = (xd - mu[:, None]).abs() * rs[:, None] * w.double().abs() + b.double().abs() + 1
+    assert ((y.double() - want).abs() <= ulp * want.abs() + eps * (rs[:, None] + 1) * size + 2.0 ** -24).all()
+    keep = torch.ones_like(yb, dtype=torch.bool)
+    keep[1:1 + M * pitch].view(M, pitch)[:, :N] = False
+    assert (yb[keep] == 5.0).all()
+
+
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("n,block", [(5, 512), (8, 512), (257, 512), (505, 512), (781, 1024), (1025, 2048), (2047, 2048), (3001, 4096), (8185, 8192), (16001, 16384), (20001, 32768)])
+def test_softmax_16_bit_rows_at_any_alignment(K, dtype, n, block):
+    """16-bit rows that start and end anywhere; probabilities round once to the 16-bit type (half an ulp, and as much again
+    where fp32 arithmetic lands on the other side of a tie)."""
+    torch.manual_seed(n)
+    dt = getattr(torch, dtype)
+    rows, pitch = 9, n + (2 if n % 2 else 1)
+    x = torch.full((3 + rows * pitch,), 99.0, device=DEV, dtype=dt)[3:].view(rows, pitch)
+    x[:, :n] = 3 * torch.randn(rows, n, device=DEV)
+    o = torch.full((1 + rows * pitch,), 5.0, device=DEV, dtype=dt)[1:].view(rows, pitch)
+    k = K.row_softmax[(rows,)](o, x, pitch, pitch, n, BLOCK=block)
+    torch.cuda.synchronize()
+    assert k.function.family == "row_softmax"
+    want = torch.softmax(x[:, :n].double(), 1)
+    ulp, tiny = (2.0 ** -10, 2.0 ** -24) if dtype == "float16" else (2.0 ** -7, 2.0 ** -133)
+    assert ((o[:, :n].double() - want).abs() <= ulp * want + tiny).all()
+    assert (o[:, n:] == 5.0).all()
+
+
 @pytest.mark.parametrize("M,N,kernel", [(4100, 8192, "layernorm_fwd_persistent_kernel"), (8200, 2048, "layernorm_fwd_persistent_kernel"), (300, 4096, "layernorm_fwd_kernel<4>"),
                                        (7, 1001, "layernorm_fwd_kernel<1>"), (5, 8191, "layernorm_fwd_kernel<8>"), (3, 20000, "layernorm_fwd_long_kernel")])
 def test_layernorm_on_fp32_tensors(K, M, N, kernel):

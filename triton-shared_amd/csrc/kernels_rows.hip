@@ -14,6 +14,7 @@
 // FMA contraction and no fast-math (backend/compiler.py:127-129,172-173).
 #include "kernels.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace tts {
@@ -102,6 +103,11 @@ __device__ __forceinline__ void ntstore(uint4 *p, uint4 v) {
   u32x4_t w = {v.x, v.y, v.z, v.w};
   __builtin_nontemporal_store(w, reinterpret_cast<u32x4_t *>(p));
 }
+template <class V>  // (a vector type of any alignment)
+__device__ __forceinline__ void ntstore(V *p, uint4 v) {
+  u32x4_t w = {v.x, v.y, v.z, v.w};
+  __builtin_nontemporal_store(w, p);
+}
 __device__ __forceinline__ void ntstore(float4 *p, float4 v) {
   f32x4_t w = {v.x, v.y, v.z, v.w};
   __builtin_nontemporal_store(w, reinterpret_cast<f32x4_t *>(p));
@@ -181,6 +187,22 @@ __device__ __forceinline__ float block_sum_256(float v, float *red) {
   return (red[0] + red[1]) + (red[2] + red[3]);
 }
 
+// The last chunk of a row of at least EPC elements is read from the row's last EPC elements when the row ends inside it (16
+// bytes at any address are one access on gfx950): its first `cut` elements, which the chunk before holds, are dropped and
+// what lies past the row is zero.
+typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(2)));  // in memory at any element's address
+template <int EPC, class V>
+__device__ __forceinline__ void drop_front(V &v, int cut) {
+  if constexpr (EPC == 8) {
+    if (cut & 4) v = V{v[2], v[3], 0, 0};
+    if (cut & 2) v = V{v[1], v[2], v[3], 0};
+    if (cut & 1) v = V{v[0] >> 16 | v[1] << 16, v[1] >> 16 | v[2] << 16, v[2] >> 16 | v[3] << 16, v[3] >> 16};
+  } else {
+    if (cut & 2) v = V{v[2], v[3], 0, 0};
+    if (cut & 1) v = V{v[1], v[2], v[3], 0};
+  }
+}
+
 // ---------------------------------------------------------------- softmax
 // T threads share one row; thread t holds elements t, t+T, ... (NPL of them).
 // VEC (block == NPL * T, NPL % 4 == 0, d_in >= 4): thread t holds the four-element chunks t, t+T, ...
@@ -189,9 +211,9 @@ __device__ __forceinline__ float block_sum_256(float v, float *red) {
 typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 
 // IO: the element type of the rows in memory (0 fp16, 1 bf16, 2 fp32); a 16-bit row is widened after the load and narrowed
-// before the store, as its Triton source does, and its VEC path moves whole 16-byte chunks of eight elements (the
-// launcher picks it for rows that are multiples of 8 elements long and start 16-byte aligned).
-template <int NPL, int WAVES, bool NAN_PROP, bool VEC, int WG = 256, int IO = 2>
+// before the store, as its Triton source does, and its VEC path moves 16-byte chunks of eight elements: whole ones of
+// aligned rows (VEC = 1) or, wherever a row starts and ends, any (2; fp16 [20000, 3001]: 106 us element by element, 40 this way).
+template <int NPL, int WAVES, bool NAN_PROP, int VEC, int WG = 256, int IO = 2>
 __global__ __launch_bounds__(WG) void softmax_f32_kernel(SoftmaxParams p, int gx, int gy, int64_t programs) {
   using E = typename std::conditional<IO == 2, float, uint16_t>::type;
   auto up = [](E e) -> float {
@@ -222,7 +244,7 @@ __global__ __launch_bounds__(WG) void softmax_f32_kernel(SoftmaxParams p, int gx
   // lanes beyond d_in hold `other` and take part in the reductions, as a filled
   // tile does; lanes beyond the block do not exist
   float v[NPL];
-  if constexpr (VEC && IO != 2) {
+  if constexpr (VEC == 1 && IO != 2) {
     // thread t holds the eight-element chunks t, t+T, ...; a chunk is whole or absent (an absent one reads the row's start)
 #pragma unroll
     for (int j = 0; j < NPL / 8; j++) {
@@ -235,6 +257,29 @@ __global__ __launch_bounds__(WG) void softmax_f32_kernel(SoftmaxParams p, int gx
         v[8 * j + 2 * k] = present ? up((uint16_t)(q[k] & 0xffff)) : p.other;
         v[8 * j + 2 * k + 1] = present ? up((uint16_t)(q[k] >> 16)) : p.other;
       }
+    }
+  } else if constexpr (VEC == 2) {
+    // the same chunks, each read with one access wherever the row starts; the row may end inside one
+    u32x4_t raw[NPL / 8];
+#pragma unroll
+    for (int j = 0; j < NPL / 8; j++) {
+      const int i0 = 8 * (t + j * T);
+      raw[j] = *reinterpret_cast<const u32x4_any *>(in + (i0 < d_in ? min(i0, d_in - 8) : 0));
+    }
+#pragma unroll
+    for (int j = 0; j < NPL / 8; j++) {
+      const int i0 = 8 * (t + j * T);
+      const bool present = i0 < d_in, cut = present && i0 + 8 > d_in;
+      if (cut) drop_front<8>(raw[j], i0 + 8 - d_in);
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        v[8 * j + 2 * k] = present ? up((uint16_t)(raw[j][k] & 0xffff)) : p.other;
+        v[8 * j + 2 * k + 1] = present ? up((uint16_t)(raw[j][k] >> 16)) : p.other;
+      }
+      if (cut)
+#pragma unroll
+        for (int k = 1; k < 8; k++)
+          if (i0 + k >= d_in) v[8 * j + k] = p.other;
     }
   } else if constexpr (VEC) {
     // The chunk grid lies on 16-byte boundaries of memory: it starts `lead` elements before the row (rows of 781 floats are
@@ -302,7 +347,15 @@ __global__ __launch_bounds__(WG) void softmax_f32_kernel(SoftmaxParams p, int gx
 #pragma unroll
       for (int k = 0; k < 4; k++)
         o[k] = (uint32_t)down(v[8 * j + 2 * k] * rsum) | ((uint32_t)down(v[8 * j + 2 * k + 1] * rsum) << 16);
-      if (i0 < d_out) ntstore(reinterpret_cast<uint4 *>(out + i0), make_uint4(o[0], o[1], o[2], o[3]));
+      if (VEC == 1) {
+        if (i0 < d_out) ntstore(reinterpret_cast<uint4 *>(out + i0), make_uint4(o[0], o[1], o[2], o[3]));
+      } else if (i0 + 8 <= d_out) {
+        ntstore(reinterpret_cast<u32x4_any *>(out + i0), make_uint4(o[0], o[1], o[2], o[3]));
+      } else if (i0 < d_out) {
+#pragma unroll
+        for (int k = 0; k < 8; k++)
+          if (i0 + k < d_out) out[i0 + k] = (uint16_t)(o[k / 2] >> (16 * (k % 2)));
+      }
     }
   } else if constexpr (VEC) {
     // slot s of the grid is element s - lead of the row; the output row's chunks are aligned stores when it sits at the
@@ -342,19 +395,22 @@ hipError_t launch_softmax_io(const SoftmaxParams &p, int gx, int gy, int gz, hip
   auto rows_on_boundaries = [&](const Affine &a, const void *base) {
     return (a.c0 | a.c[0] | a.c[1] | a.c[2]) % 4 == 0 && ((uintptr_t)base & 15) == 0;
   };
-  bool vec = CAN_VEC && p.block == NPL * WAVES * WAVE && p.d_in >= 4 &&
-             (IO != 2 || p.d_in + 3 <= p.block || rows_on_boundaries(p.in_off, p.in));
-  if (IO != 2) {  // whole chunks of aligned rows only
+  int vec = CAN_VEC && p.block == NPL * WAVES * WAVE && (IO != 2 ? p.d_in >= 8 : p.d_in >= 4 && (p.d_in + 3 <= p.block || rows_on_boundaries(p.in_off, p.in)));
+  if (IO != 2 && vec) {  // whole chunks of aligned rows (which the kernel for any rows takes 12 % longer for: fp16 [20000, 3000], 34.5 us against 38.6), or any rows
     auto aligned = [](const Affine &a) { return (a.c0 | a.c[0] | a.c[1] | a.c[2]) % 8 == 0; };
-    vec = vec && p.d_in % 8 == 0 && p.d_out % 8 == 0 && aligned(p.in_off) && aligned(p.out_off) && (((uintptr_t)p.in | (uintptr_t)p.out) & 15) == 0;
+    if (!(p.d_in % 8 == 0 && p.d_out % 8 == 0 && aligned(p.in_off) && aligned(p.out_off) && (((uintptr_t)p.in | (uintptr_t)p.out) & 15) == 0)) vec = 2;
   }
-  if (vec) {
-    if (p.propagate_nan) hipLaunchKernelGGL((softmax_f32_kernel<NPL, WAVES, true, CAN_VEC, WG, IO>), grid, dim3(WG), 0, s, p, gx, gy, programs);
-    else hipLaunchKernelGGL((softmax_f32_kernel<NPL, WAVES, false, CAN_VEC, WG, IO>), grid, dim3(WG), 0, s, p, gx, gy, programs);
-    return hipGetLastError();
+  constexpr int WHOLE = CAN_VEC ? 1 : 0, ANY = CAN_VEC && IO != 2 ? 2 : WHOLE;
+  if (vec == 2) {
+    if (p.propagate_nan) hipLaunchKernelGGL((softmax_f32_kernel<NPL, WAVES, true, ANY, WG, IO>), grid, dim3(WG), 0, s, p, gx, gy, programs);
+    else hipLaunchKernelGGL((softmax_f32_kernel<NPL, WAVES, false, ANY, WG, IO>), grid, dim3(WG), 0, s, p, gx, gy, programs);
+  } else if (vec) {
+    if (p.propagate_nan) hipLaunchKernelGGL((softmax_f32_kernel<NPL, WAVES, true, WHOLE, WG, IO>), grid, dim3(WG), 0, s, p, gx, gy, programs);
+    else hipLaunchKernelGGL((softmax_f32_kernel<NPL, WAVES, false, WHOLE, WG, IO>), grid, dim3(WG), 0, s, p, gx, gy, programs);
+  } else {
+    if (p.propagate_nan) hipLaunchKernelGGL((softmax_f32_kernel<NPL, WAVES, true, 0, WG, IO>), grid, dim3(WG), 0, s, p, gx, gy, programs);
+    else hipLaunchKernelGGL((softmax_f32_kernel<NPL, WAVES, false, 0, WG, IO>), grid, dim3(WG), 0, s, p, gx, gy, programs);
   }
-  if (p.propagate_nan) hipLaunchKernelGGL((softmax_f32_kernel<NPL, WAVES, true, false, WG, IO>), grid, dim3(WG), 0, s, p, gx, gy, programs);
-  else hipLaunchKernelGGL((softmax_f32_kernel<NPL, WAVES, false, false, WG, IO>), grid, dim3(WG), 0, s, p, gx, gy, programs);
   return hipGetLastError();
 }
 
@@ -402,82 +458,88 @@ struct LnType<2> {
   }
 };
 
-// One workgroup per row.  The row is read from HBM once and kept in registers
-// as fp32 (CPT chunks of EPC elements per thread); the Triton source's three
-// passes over the row all read these registers.
-// FAST: N is a multiple of EPC and every row of x, y, w, b starts 16-byte aligned, so a chunk is
-// either whole or absent and all loads are unconditional (an absent chunk re-reads chunk 0 and is
-// zeroed), which lets the compiler keep the CPT loads of a thread in flight together.
-template <int KIND, int CPT, bool FAST>
-__global__ __launch_bounds__(256, CPT <= 4 ? 8 : 4) void layernorm_fwd_kernel(LayerNormParams p) {
+template <int FROM, int COUNT, int N>
+__device__ __forceinline__ float pairwise(const float (&s)[N]) {
+  if constexpr (COUNT == 1) return s[FROM];
+  else return pairwise<FROM, (COUNT + 1) / 2>(s) + pairwise<FROM + (COUNT + 1) / 2, COUNT / 2>(s);
+}
+
+// One row per workgroup (WPR = 4 wavefronts) or per wavefront (WPR = 1), N >= EPC.  The row is read from HBM once and kept
+// in registers as fp32 (CPT chunks of EPC elements per thread); the Triton source's three passes over the row all read these
+// registers.  All loads are unconditional (an absent chunk reads the row's start and is zeroed), which lets the compiler
+// keep the CPT loads of a thread in flight together.
+// Loads and stores take 16 bytes wherever the row starts.  (Element by element, as rows off the 16-byte grid were read
+// before: fp16 [8192, 5003] 135 us, now 37.)  Short rows take a wavefront each: no barrier, four rows per workgroup
+// (fp32 [8000, 512]: 14.4 us with a workgroup per row, 8.0 with a wavefront).
+template <int KIND, int CPT, int WPR>
+__global__ __launch_bounds__(256, CPT <= 2 || (KIND == 2 && CPT <= 4) ? 8 : CPT <= 4 ? 6 : KIND == 2 ? 4 : 3) void layernorm_fwd_kernel(LayerNormParams p, int gx, int gy, int64_t programs) {
   using T = LnType<KIND>;
   using E = typename T::elem;
-  constexpr int EPC = T::EPC;
+  constexpr int EPC = T::EPC, THREADS = WPR * WAVE;
   __shared__ float red[4];
-  const ProgramId id = program_id(p.lin_gx, p.lin_gy);
-  const int px = id.x, py = id.y, pz = id.z;
+  const int64_t prog = ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * (4 / WPR) + (WPR == 1 ? threadIdx.x / WAVE : 0);  // (along y from 2^23 workgroups on)
+  if (prog >= programs) return;  // (whole wavefronts, or a whole workgroup where a row has one to itself)
+  const int t = threadIdx.x % THREADS;
+  int px = (int)prog, py = 0, pz = 0;
+  if (programs != gx) { px = (int)(prog % gx); py = (int)((prog / gx) % gy); pz = (int)(prog / ((int64_t)gx * gy)); }
+  auto sum_of_row = [&](float v) { return WPR == 1 ? wave_sum(v) : block_sum_256(v, red); };
   const E *__restrict__ x = (const E *)p.x + affine(p.x_off, px, py, pz);
   const E *__restrict__ w = (const E *)p.w + affine(p.w_off, px, py, pz);
   const E *__restrict__ b = (const E *)p.b + affine(p.b_off, px, py, pz);
   E *__restrict__ y = (E *)p.y + affine(p.y_off, px, py, pz);
   const int N = (int)p.N;
-  const bool vec = (((uintptr_t)x | (uintptr_t)w | (uintptr_t)b | (uintptr_t)y) & 15) == 0;
+  u32x4_t raw[CPT];
+#pragma unroll
+  for (int c = 0; c < CPT; c++) {
+    const int i0 = (t + c * THREADS) * EPC;
+    raw[c] = *reinterpret_cast<const u32x4_any *>(x + (i0 < N ? min(i0, N - EPC) : 0));
+  }
   float v[CPT][EPC];
 #pragma unroll
   for (int c = 0; c < CPT; c++) {
-    int i0 = (threadIdx.x + c * 256) * EPC;
-    if (FAST) {
-      const bool present = i0 < N;
-      uint4 raw = *reinterpret_cast<const uint4 *>(x + (present ? i0 : 0));
-      const uint32_t q[4] = {raw.x, raw.y, raw.z, raw.w};
-      T::unpack(q, v[c]);
-#pragma unroll
-      for (int k = 0; k < EPC; k++) v[c][k] = present ? v[c][k] : 0.f;
-    } else if (vec && i0 + EPC <= N) {
-      uint4 raw = *reinterpret_cast<const uint4 *>(x + i0);
-      const uint32_t q[4] = {raw.x, raw.y, raw.z, raw.w};
-      T::unpack(q, v[c]);
-    } else {
-#pragma unroll
-      for (int k = 0; k < EPC; k++) v[c][k] = i0 + k < N ? T::up(x[i0 + k]) : 0.f;  // other = 0
-    }
+    const int i0 = (t + c * THREADS) * EPC;
+    if (i0 >= N) raw[c] = u32x4_t{0, 0, 0, 0};  // other = 0
+    else if (i0 + EPC > N) drop_front<EPC>(raw[c], i0 + EPC - N);
+    const uint32_t q[4] = {raw[c][0], raw[c][1], raw[c][2], raw[c][3]};
+    T::unpack(q, v[c]);
   }
   const float n_f = (float)N;  // arith.sitofp
-  float s = 0.f;
-#pragma unroll
-  for (int c = 0; c < CPT; c++)
-#pragma unroll
-    for (int k = 0; k < EPC; k++) s += v[c][k];
-  const float mean = block_sum_256(s, red) / n_f;
-  float s2 = 0.f;
+  float s[CPT];  // a sum per chunk, added in pairs: no longer a chain of roundings for a thread with many chunks
 #pragma unroll
   for (int c = 0; c < CPT; c++) {
-    int i0 = (threadIdx.x + c * 256) * EPC;
+    s[c] = 0.f;
+#pragma unroll
+    for (int k = 0; k < EPC; k++) s[c] += v[c][k];
+  }
+  const float mean = sum_of_row(pairwise<0, CPT>(s)) / n_f;
+#pragma unroll
+  for (int c = 0; c < CPT; c++) {
+    const int i0 = (t + c * THREADS) * EPC;
+    s[c] = 0.f;
 #pragma unroll
     for (int k = 0; k < EPC; k++) {
       float d = i0 + k < N ? v[c][k] - mean : 0.f;  // tl.where(cols < N, x - mean, 0)
-      s2 += d * d;
+      s[c] += d * d;
     }
   }
-  const float var = block_sum_256(s2, red) / n_f;
+  const float var = sum_of_row(pairwise<0, CPT>(s)) / n_f;
   const float rstd = 1.0f / sqrtf(var + p.eps);
-  if (threadIdx.x == 0) {
+  if (t == 0) {
     p.mean[affine(p.mean_off, px, py, pz)] = mean;
     p.rstd[affine(p.rstd_off, px, py, pz)] = rstd;
   }
 #pragma unroll
   for (int c = 0; c < CPT; c++) {
-    int i0 = (threadIdx.x + c * 256) * EPC;
-    if (FAST ? i0 < N : (vec && i0 + EPC <= N)) {
-      uint4 wr = *reinterpret_cast<const uint4 *>(w + i0);
-      uint4 br = *reinterpret_cast<const uint4 *>(b + i0);
-      const uint32_t wq[4] = {wr.x, wr.y, wr.z, wr.w}, bq[4] = {br.x, br.y, br.z, br.w};
+    const int i0 = (t + c * THREADS) * EPC;
+    if (i0 + EPC <= N) {
+      const u32x4_t wr = *reinterpret_cast<const u32x4_any *>(w + i0), br = *reinterpret_cast<const u32x4_any *>(b + i0);
+      const uint32_t wq[4] = {wr[0], wr[1], wr[2], wr[3]}, bq[4] = {br[0], br[1], br[2], br[3]};
       float wv[EPC], bv[EPC], o[EPC];
       T::unpack(wq, wv);
       T::unpack(bq, bv);
 #pragma unroll
       for (int k = 0; k < EPC; k++) o[k] = (v[c][k] - mean) * rstd * wv[k] + bv[k];
-      ntstore(reinterpret_cast<uint4 *>(y + i0), T::pack(o));
+      ntstore(reinterpret_cast<u32x4_any *>(y + i0), T::pack(o));
     } else {
 #pragma unroll
       for (int k = 0; k < EPC; k++)
@@ -494,8 +556,9 @@ __global__ __launch_bounds__(256, CPT <= 4 ? 8 : 4) void layernorm_fwd_kernel(La
 // kernel loses is the 32 KB of w and b that every row fetches again through L2: taking those loads out of it, and
 // nothing else, gives 23.8 us.  512 or 1024 threads per workgroup, a third row in flight and nontemporal row loads
 // gain nothing or lose.  [8192, 8192]: 51.7 -> 44.8 us (6.0 TB/s).
-// For one-dimensional grids, rows of exactly CPT * 256 chunks starting 16-byte aligned, w and b the same for every row.
-template <int KIND, int CPT>
+// For one-dimensional grids, w and b the same for every row, N >= EPC.  WHOLE: rows of exactly CPT * 256 chunks; otherwise a
+// thread's last chunks may be absent or cut off (see above), which costs a select and a branch per chunk.
+template <int KIND, int CPT, bool WHOLE>
 __global__ __launch_bounds__(256) void layernorm_fwd_persistent_kernel(LayerNormParams p, int rows) {
   using T = LnType<KIND>;
   using E = typename T::elem;
@@ -507,12 +570,24 @@ __global__ __launch_bounds__(256) void layernorm_fwd_persistent_kernel(LayerNorm
   E *__restrict__ yb = (E *)p.y + p.y_off.c0;
   const E *__restrict__ w = (const E *)p.w + p.w_off.c0;
   const E *__restrict__ b = (const E *)p.b + p.b_off.c0;
-  uint4 wq[CPT], bq[CPT];
+  auto first = [&](int c) { return (tid + c * 256) * EPC; };  // the first element of a thread's chunk
+  auto from = [&](int c) { return WHOLE ? first(c) : first(c) < N ? min(first(c), N - EPC) : 0; };  // where it is read
+  auto settle = [&](u32x4_t &q, int c) {  // what was read there -> the chunk
+    if (WHOLE) return;
+    if (first(c) >= N) q = u32x4_t{0, 0, 0, 0};
+    else if (first(c) + EPC > N) drop_front<EPC>(q, first(c) + EPC - N);
+  };
+  u32x4_t wq[CPT], bq[CPT];
 #pragma unroll
   for (int c = 0; c < CPT; c++) {
-    wq[c] = *reinterpret_cast<const uint4 *>(w + (tid + c * 256) * EPC);
-    bq[c] = *reinterpret_cast<const uint4 *>(b + (tid + c * 256) * EPC);
+    wq[c] = *reinterpret_cast<const u32x4_any *>(w + from(c));
+    bq[c] = *reinterpret_cast<const u32x4_any *>(b + from(c));
+    settle(wq[c], c);
+    settle(bq[c], c);
   }
+  int stores = 0;  // of whole chunks by this wavefront, per row
+#pragma unroll
+  for (int c = 0; c < CPT; c++) stores += WHOLE || (__builtin_amdgcn_readfirstlane(wave) * WAVE + c * 256 + 1) * EPC <= N;
   // A row's loads are issued from inline assembly and waited for by hand (row_landed): left to the compiler, the wait
   // for a row also waits for the next row's loads, issued just before (it does not count memory operations across the
   // loop's back edge), and the rows do not overlap.
@@ -520,21 +595,16 @@ __global__ __launch_bounds__(256) void layernorm_fwd_persistent_kernel(LayerNorm
     const E *x = xb + (int64_t)r * p.x_off.c[0];
 #pragma unroll
     for (int c = 0; c < CPT; c++) {
-      const E *src = x + (tid + c * 256) * EPC;
+      const E *src = x + from(c);
       asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(q[c]) : "v"(src) : "memory");
     }
   };
-  // Waits until at most `newer` vector memory operations issued after the row's loads are outstanding (they complete in
-  // order, so the row has landed), and ties the row's registers to the wait so that no use moves above it.
-  auto row_landed = [&](u32x4_t (&q)[CPT], int newer) {
-    switch (newer) {  // a constant after inlining; the instruction takes an immediate
-      case 1: asm volatile("s_waitcnt vmcnt(1)" ::: "memory"); break;
-      case 2: asm volatile("s_waitcnt vmcnt(2)" ::: "memory"); break;
-      case 4: asm volatile("s_waitcnt vmcnt(4)" ::: "memory"); break;
-      case 8: asm volatile("s_waitcnt vmcnt(8)" ::: "memory"); break;
-      case 16: asm volatile("s_waitcnt vmcnt(16)" ::: "memory"); break;
-      default: asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); break;
-    }
+  // Waits until at most CPT + `earlier` vector memory operations issued after the row's loads are outstanding (they complete
+  // in order, so the row has landed), and ties the row's registers to the wait so that no use moves above it.
+  auto row_landed = [&](u32x4_t (&q)[CPT], int earlier) {
+#pragma unroll
+    for (int e = CPT; e >= 0; e--)  // (the instruction takes an immediate; one comparison is left where `earlier` is known)
+      if (earlier == e) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(CPT + e) : "memory");
 #pragma unroll
     for (int c = 0; c < CPT; c++) asm volatile("" : "+v"(q[c]) : : "memory");
   };
@@ -545,10 +615,11 @@ __global__ __launch_bounds__(256) void layernorm_fwd_persistent_kernel(LayerNorm
     return (red[which][parity][0] + red[which][parity][1]) + (red[which][parity][2] + red[which][parity][3]);
   };
   const float n_f = (float)N;  // arith.sitofp
-  auto process = [&](const u32x4_t (&raw)[CPT], int r, int parity) {
+  auto process = [&](u32x4_t (&raw)[CPT], int r, int parity) {
     float v[CPT][EPC];
 #pragma unroll
     for (int c = 0; c < CPT; c++) {
+      settle(raw[c], c);
       const uint32_t q[4] = {raw[c][0], raw[c][1], raw[c][2], raw[c][3]};
       T::unpack(q, v[c]);
     }
@@ -563,7 +634,7 @@ __global__ __launch_bounds__(256) void layernorm_fwd_persistent_kernel(LayerNorm
     for (int c = 0; c < CPT; c++)
 #pragma unroll
       for (int k = 0; k < EPC; k++) {
-        const float d = v[c][k] - mean;
+        const float d = WHOLE || first(c) + k < N ? v[c][k] - mean : 0.f;
         s2 += d * d;
       }
     const float var = block_sum(s2, 1, parity) / n_f;
@@ -573,13 +644,17 @@ __global__ __launch_bounds__(256) void layernorm_fwd_persistent_kernel(LayerNorm
     for (int c = 0; c < CPT; c++) {
       // (the optimiser widens w and b to fp32 once, outside the row loop: 16 registers per chunk, which a workgroup
       // that has a CU's register file nearly to itself can afford, and four operations per element and row saved)
-      const uint32_t wr[4] = {wq[c].x, wq[c].y, wq[c].z, wq[c].w}, br[4] = {bq[c].x, bq[c].y, bq[c].z, bq[c].w};
+      const uint32_t wr[4] = {wq[c][0], wq[c][1], wq[c][2], wq[c][3]}, br[4] = {bq[c][0], bq[c][1], bq[c][2], bq[c][3]};
       float wv[EPC], bv[EPC], o[EPC];
       T::unpack(wr, wv);
       T::unpack(br, bv);
 #pragma unroll
       for (int k = 0; k < EPC; k++) o[k] = (v[c][k] - mean) * rstd * wv[k] + bv[k];
-      ntstore(reinterpret_cast<uint4 *>(y + (tid + c * 256) * EPC), T::pack(o));
+      if (WHOLE || first(c) + EPC <= N) ntstore(reinterpret_cast<u32x4_any *>(y + first(c)), T::pack(o));
+      else
+#pragma unroll
+        for (int k = 0; k < EPC; k++)
+          if (first(c) + k < N) y[first(c) + k] = T::down(o[k]);
     }
     if (tid == 0) {
       p.mean[p.mean_off.c0 + (int64_t)r * p.mean_off.c[0]] = mean;
@@ -588,26 +663,26 @@ __global__ __launch_bounds__(256) void layernorm_fwd_persistent_kernel(LayerNorm
   };
   // Two register sets take turns, so that no row is copied from one to the other (a copy would wait for the loads).
   // Past the last row a workgroup loads the last row again: the loads are unconditional, hence countable.  Between a
-  // row's loads and its use lie the next row's CPT loads and, from the second row on, the previous row's CPT stores
-  // (every wavefront issues all of them: the rows are whole) -- plus the two statistics stores of the first wavefront,
-  // which only make its wait stricter than necessary.
+  // row's loads and its use lie the next row's CPT loads and, from the second row on, the previous row's stores: one for
+  // every chunk that is whole in any lane of the wavefront -- plus what it stores of a chunk that is cut off and the two
+  // statistics stores of the first wavefront, which only make the wait stricter than necessary.
   int r = blockIdx.x;
   if (r >= rows) return;
   const int step = gridDim.x, last = rows - 1;
   u32x4_t even[CPT], odd[CPT];
   load_row(even, r);
   load_row(odd, min(r + step, last));
-  row_landed(even, CPT);
+  row_landed(even, 0);
   process(even, r, 0);
   r += step;
   while (r < rows) {
     load_row(even, min(r + step, last));
-    row_landed(odd, 2 * CPT);
+    row_landed(odd, stores);
     process(odd, r, 1);
     r += step;
     if (r >= rows) break;
     load_row(odd, min(r + step, last));
-    row_landed(even, 2 * CPT);
+    row_landed(even, stores);
     process(even, r, 0);
     r += step;
   }
@@ -650,51 +725,72 @@ __global__ __launch_bounds__(256) void layernorm_fwd_long_kernel(LayerNormParams
 template <int KIND>
 hipError_t launch_layernorm_t(const LayerNormParams &p, dim3 grid, hipStream_t s, const char **name) {
   constexpr int EPC = LnType<KIND>::EPC;
-  int64_t chunks = (p.N + EPC - 1) / EPC;
-  auto aligned = [](const Affine &a) { return (a.c0 | a.c[0] | a.c[1] | a.c[2]) % EPC == 0; };
-  const bool fast = p.N % EPC == 0 && aligned(p.x_off) && aligned(p.y_off) && aligned(p.w_off) && aligned(p.b_off) &&
-                    (((uintptr_t)p.x | (uintptr_t)p.y | (uintptr_t)p.w | (uintptr_t)p.b) & 15) == 0;
-  // Rows walked by persistent workgroups (see layernorm_fwd_persistent_kernel): whole rows of 256, 512, 1024 or (fp32)
-  // 2048 chunks in one-dimensional grids with enough rows to amortise the walk (fewer, and the workgroup-per-row kernel
-  // measured faster), w and b the same for every row.  About 32 KB of row loads in flight per CU: one workgroup per CU
-  // for rows of 16 KB and more, four for 8 KB, eight for 4 KB (measured best of 1, 2, 4 and 8 per CU on fp16 [8192, 4096]
-  // and [16384, 2048]: 25.5 us against 26.3 and 26.5 us against 31.1 for a workgroup per row).
+  const int64_t chunks = (p.N + EPC - 1) / EPC, programs = (int64_t)grid.x * grid.y * grid.z;
+  if (p.N < EPC || chunks > 2048) {
+    hipLaunchKernelGGL((layernorm_fwd_long_kernel<KIND>), grid, dim3(256), 0, s, p);
+    *name = "layernorm_fwd_long_kernel";
+    return hipGetLastError();
+  }
+  // Rows walked by persistent workgroups (see layernorm_fwd_persistent_kernel): one-dimensional grids with enough rows to
+  // amortise the walk (fewer, and the workgroup-per-row kernel measured faster), w and b the same for every row.  About 32 KB
+  // of row loads in flight per CU: one workgroup per CU for rows of 16 KB and more, four for 8 KB, eight for 4 KB (measured
+  // best of 1, 2, 4 and 8 per CU on fp16 [8192, 4096] and [16384, 2048]: 25.5 us against 26.3 and 26.5 us against 31.1 for a
+  // workgroup per row).
   static const char *ln_env = getenv("TTS_LN");  // tuning aid: "0" = always one workgroup per row; "G" = G persistent workgroups
   static const int cus = [] {
     int dev = 0, n = 0;
     if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
     return n;
   }();
-  const int cpt = chunks == 256 ? 1 : chunks == 512 ? 2 : chunks == 1024 ? 4 : (chunks == 2048 && KIND == 2) ? 8 : 0;
-  int persistent_grid = cus * (cpt == 1 ? 8 : cpt == 2 ? 4 : 1);
+  const int cpt = chunks <= 256 ? 1 : chunks <= 512 ? 2 : chunks <= 768 ? 3 : chunks <= 1024 ? 4 : KIND == 2 && chunks <= 1536 ? 6 : KIND == 2 ? 8 : 0;
+  int persistent_grid = cus * (cpt == 1 ? 8 : cpt == 2 ? 4 : cpt == 3 ? 2 : 1);
   int64_t min_rows = (int64_t)persistent_grid * (cpt >= 4 ? 16 : 8);
   if (ln_env) {
     persistent_grid = atoi(ln_env);
     min_rows = 2 * (int64_t)persistent_grid;
   }
   auto row_invariant = [](const Affine &a) { return (a.c[0] | a.c[1] | a.c[2]) == 0; };
-  if (fast && cpt && persistent_grid > 0 && !p.lin_gx && grid.y == 1 && grid.z == 1 && (int64_t)grid.x >= min_rows && row_invariant(p.w_off) &&
-      row_invariant(p.b_off)) {
+  if (cpt && chunks > 128 && persistent_grid > 0 && !p.lin_gx && grid.y == 1 && grid.z == 1 && (int64_t)grid.x >= min_rows && row_invariant(p.w_off) && row_invariant(p.b_off)) {
     const int rows = (int)grid.x;
     const dim3 pg((unsigned)persistent_grid);
-    if (cpt == 1) hipLaunchKernelGGL((layernorm_fwd_persistent_kernel<KIND, 1>), pg, dim3(256), 0, s, p, rows);
-    else if (cpt == 2) hipLaunchKernelGGL((layernorm_fwd_persistent_kernel<KIND, 2>), pg, dim3(256), 0, s, p, rows);
-    else if (cpt == 4) hipLaunchKernelGGL((layernorm_fwd_persistent_kernel<KIND, 4>), pg, dim3(256), 0, s, p, rows);
-    else if constexpr (KIND == 2) hipLaunchKernelGGL((layernorm_fwd_persistent_kernel<KIND, 8>), pg, dim3(256), 0, s, p, rows);
+    const bool whole = p.N == (int64_t)cpt * 256 * EPC;
     *name = "layernorm_fwd_persistent_kernel";
-    return hipGetLastError();
-  }
-#define TTS_LN(CPT)                                                                                          \
-  do {                                                                                                       \
-    if (fast) hipLaunchKernelGGL((layernorm_fwd_kernel<KIND, CPT, true>), grid, dim3(256), 0, s, p);        \
-    else hipLaunchKernelGGL((layernorm_fwd_kernel<KIND, CPT, false>), grid, dim3(256), 0, s, p);            \
-    *name = "layernorm_fwd_kernel<" #CPT ">";                                                                \
+#define TTS_LN(CPT)                                                                                                                   \
+  do {                                                                                                                                \
+    if (whole) hipLaunchKernelGGL((layernorm_fwd_persistent_kernel<KIND, CPT, true>), pg, dim3(256), 0, s, p, rows);                 \
+    else hipLaunchKernelGGL((layernorm_fwd_persistent_kernel<KIND, CPT, false>), pg, dim3(256), 0, s, p, rows);                      \
+    return hipGetLastError();                                                                                                         \
   } while (0)
-  if (chunks <= 256) TTS_LN(1);
-  else if (chunks <= 512) TTS_LN(2);
-  else if (chunks <= 1024) TTS_LN(4);
-  else if (chunks <= 2048) TTS_LN(8);
-  else { hipLaunchKernelGGL((layernorm_fwd_long_kernel<KIND>), grid, dim3(256), 0, s, p); *name = "layernorm_fwd_long_kernel"; }
+    if (cpt == 1) TTS_LN(1);
+    if (cpt == 2) TTS_LN(2);
+    if (cpt == 3) TTS_LN(3);
+    if (cpt == 4) TTS_LN(4);
+    if constexpr (KIND == 2) {
+      if (cpt == 6) TTS_LN(6);
+      TTS_LN(8);
+    }
+#undef TTS_LN
+  }
+  const int gx = p.lin_gx ? p.lin_gx : (int)grid.x, gy = p.lin_gx ? p.lin_gy : (int)grid.y;
+  *name = chunks <= 256 ? "layernorm_fwd_kernel<1>" : chunks <= 512 ? "layernorm_fwd_kernel<2>" : chunks <= 1024 ? "layernorm_fwd_kernel<4>" : "layernorm_fwd_kernel<8>";
+#define TTS_LN(CPT, WPR)                                                                                                              \
+  do {                                                                                                                                \
+    const int64_t wgs = (programs + 4 / WPR - 1) / (4 / WPR), along_x = std::min<int64_t>(wgs, 1 << 23);                              \
+    hipLaunchKernelGGL((layernorm_fwd_kernel<KIND, CPT, WPR>), dim3((unsigned)along_x, (unsigned)((wgs + along_x - 1) / along_x)), dim3(256), 0, s, p, gx, gy, programs); \
+  } while (0)
+  // A wavefront per row up to 256 chunks, given four rows per CU or rows of a single chunk per lane (fp16 [4000, 2000]: 10.2
+  // us against 11.0 with a workgroup per row, fp32 [8000, 1000] 13.1 against 16.6; fp16 [300, 2000] 5.2 against 4.2); at 512
+  // chunks the workgroup wins again (fp16 [2000, 4096]: 9.6 against 10.9).
+  const bool short_rows = chunks <= 64 || (chunks <= 256 && programs >= 4 * cus);
+  if (short_rows && chunks <= 64) TTS_LN(1, 1);
+  else if (short_rows && chunks <= 128) TTS_LN(2, 1);
+  else if (short_rows) TTS_LN(4, 1);
+  else if (chunks <= 256) TTS_LN(1, 4);
+  else if (chunks <= 512) TTS_LN(2, 4);
+  else if (chunks <= 768) TTS_LN(3, 4);
+  else if (chunks <= 1024) TTS_LN(4, 4);
+  else if (chunks <= 1536) TTS_LN(6, 4);
+  else TTS_LN(8, 4);
 #undef TTS_LN
   return hipGetLastError();
 }
