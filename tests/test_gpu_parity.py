@@ -1163,6 +1163,30 @@ def test_loops_that_only_add_run_in_slices(dtype, rows, cols, pitch):
         assert torch.equal(out[:3].double(), want) and (out[3] == 9.0).all()
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("BR,BC,rows,cols,pitch", [(32, 64, 1, 1, 1), (32, 64, 33, 7, 9), (32, 128, 4000, 129, 129), (32, 128, 700, 1000, 1003), (128, 16, 1000, 23, 24),
+                                                   (256, 8, 3000, 20, 21), (2, 1024, 77, 1030, 1031), (16, 512, 500, 515, 520)])
+def test_column_sums_in_the_wide_order(dtype, BR, BC, rows, cols, pitch):
+    # sliced loops whose blocks move 16 bytes per access: column blocks that end inside a group of eight or hold fewer than
+    # eight, rows that start anywhere, row blocks that end inside a block; small integers keep every sum exact
+    import extra_kernels as X
+    g = torch.Generator().manual_seed(rows + cols)
+    x = torch.zeros(3 + rows * pitch, dtype=dtype)[3:].view(rows, pitch)
+    x[:, :] = 77
+    x[:, :cols] = torch.randint(-3, 4, (rows, cols), generator=g).to(dtype)
+    xd = torch.empty(3 + rows * pitch, dtype=dtype, device=DEV)[3:].view(rows, pitch).copy_(x)
+    s = torch.randint(-2, 3, (rows,), generator=g).float()
+    xc = x[:, :cols].double()
+    a, b = (xc * s[:, None].double()).sum(0) + 1, (xc * xc).sum(0)
+    want = torch.stack([a, b, a - 2 * b])
+    for _ in range(2):
+        out = torch.full((4, cols), 9.0, device=DEV)
+        k = X.column_moments[(triton.cdiv(cols, BC),)](xd, s.to(DEV), out, rows, cols, pitch, BR=BR, BC=BC)
+        torch.cuda.synchronize()
+        assert k.function.family == "tile_program"
+        assert torch.equal(out[:3].cpu().double(), want) and (out[3] == 9.0).all()
+
+
 @pytest.mark.parametrize("blocks,rows,cols", [(3, 700, 100), (5, 10, 70), (600, 20, 333), (1, 64, 64)])
 def test_loops_that_only_add_with_columns_on_program_id_1(blocks, rows, cols):
     # neighbouring column blocks on neighbouring workgroups: in slices (few programs) and whole, with the grid exchanged (many)

@@ -11,6 +11,7 @@
 
 #include <algorithm>
 #include <array>
+#include <cmath>
 #include <cstring>
 #include <list>
 #include <map>
@@ -810,17 +811,20 @@ tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, con
       if (tile_program_is_sliced(source, &slice_floats, &slice_loop)) {
         // As many workgroups as the device holds at once, each program's loop dealt to an equal number of them, two
         // iterations each at least (dw and db of LayerNorm on fp16 [4096, 8192], 64 programs of 128 iterations: 341 us with
-        // one workgroup per program, 43 us in 12 slices).  A launch that may not allocate keeps to one, and so does one that
-        // is recorded into a graph: the graph may be replayed beside launches that use the same stream's workspace.
+        // one workgroup per program, 31 us in 16 slices), and no more than 3 sqrt(iterations): an iteration takes some 0.75 us
+        // of a slice and a slice some 0.08 us of the workgroup that adds them all (16 programs of 94 iterations: 47 / 23 / 11
+        // slices 15.0 / 13.3 / 16.8 us; of 32 iterations: 16 / 8 / 4 slices 8.2 / 11.4 / 14.7 us).  A launch that may not
+        // allocate keeps to one slice, and so does one that is recorded into a graph: the graph may be replayed beside
+        // launches that use the same stream's workspace.
         const int64_t programs = (int64_t)gx * gy * gz;
         struct { TileArgs t; int slices; float *partial; int *counters; } sa{};
-        sa.slices = (int)std::max<int64_t>(1, std::min({(int64_t)rtc_resident_workgroups(*slot) * compute_units() / programs, b->slice_trips / 2, (int64_t)1024}));
+        sa.slices = (int)std::max<int64_t>(1, std::min({(int64_t)rtc_resident_workgroups(*slot) * compute_units() / programs, b->slice_trips / 2, 3 * (int64_t)std::sqrt((double)b->slice_trips), (int64_t)1024}));
         if (sa.slices > 1 && (no_alloc || is_capturing(s))) sa.slices = 1;
         if (sa.slices > 1) {
           std::lock_guard<std::mutex> lock(plan->mu);
           tts_plan::SplitK &sk = plan->split_k[stream];
           hipError_t e = plan->grow((void **)&sk.workspace, &sk.workspace_bytes, (size_t)programs * sa.slices * slice_floats * sizeof(float));
-          if (e == hipSuccess) e = plan->grow_counters(sk, (size_t)programs);
+          if (e == hipSuccess) e = plan->grow_counters(sk, (size_t)programs * 32);  // (128 bytes apart)
           if (e != hipSuccess) return fail(TTS_HIP_ERROR, std::string("hipMalloc(partial sums): ") + hipGetErrorString(e));
           sa.partial = sk.workspace;
           sa.counters = sk.counters;

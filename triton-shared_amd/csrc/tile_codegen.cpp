@@ -314,6 +314,7 @@ struct Gen {
         // a load that is not of the run's block shape (an index vector, a row of scales): from its copy in LDS when the
         // run staged one, else read where it is used (the program is then refused if anything stores to its base)
         if (staged.count(v)) return staged_at(v, i0, i1);
+        if (row_vectors.count(v) && i0 == idx0(wide_shape)) return row_vectors.at(v) + "[n >> 3]";
         all_inline_bases.insert(s.acc.base_arg);
         std::string pred, addr = address(s.acc, i0, i1, pred);
         const std::string rd = mem_read(s.acc, addr);
@@ -548,7 +549,7 @@ struct Gen {
 
   // How many of the eight elements from index i on (along the contiguous dimension) the extent cuts off.
   std::string cut_off(const Access &a, const std::string &i) {
-    return "(int)smax(0LL, " + i + " + 8 - (" + ex(a.dims.back()) + "))";
+    return "max(0, " + i + " + 8 - (int)smin(smax(" + ex(a.dims.back()) + ", 0LL), " + std::to_string(a.sizes.back()) + "LL))";
   }
   std::string mem_read(const Access &a, const std::string &addr) {
     const std::string ptr = "((const " + memtype(a.elem) + " *)p.ptr[" + std::to_string(a.base_arg) + "])[" + addr + "]";
@@ -847,10 +848,47 @@ struct Gen {
     for (const SOp &s : slice_head)
       if (s.kind == SK::For) sliced = &s;
   }
+  // Column sums: a sliced loop over blocks [R, C] of which every result is summed along the rows' axis.  Its blocks take the
+  // wide order whatever their elements' type (2048 / C rows per 16-byte group of every thread), a vector of R elements --
+  // the rows' statistics -- is read by the threads that own the rows, into registers, and as nothing is stored inside the
+  // loop and nothing shared, an iteration has no barrier.  (dw and db of LayerNorm with one element per access and the
+  // statistics staged in LDS behind two barriers: fp16 [4096, 8192] 47 us from HBM, 31 this way; [8192, 5003] 60 and 45.)
+  bool column_sums = false;
+  void choose_column_sums() {
+    if (!sliced || wide_mode) return;
+    if (const char *e = getenv("TTS_TILE_WIDE"))
+      if (e[0] == '0') return;
+    const std::vector<int64_t> &sh = val(sliced->tile_args[0]).shape;
+    if (sh.size() != 2 || sh[1] % 8 != 0 || 2048 % sh[1] != 0 || count(sh) % 2048 != 0 || count(sh) > TWO_PHASE_MAX || sh[0] == sh[1]) return;
+    for (int v : sliced->tile_args)
+      if (val(v).shape != sh) return;
+    bool any = false;
+    for (const SOp &s : sliced->body) {
+      if (s.kind == SK::Load && s.acc.sizes == sh) {
+        if (!vector_access(s.acc)) return;
+        any = true;
+      } else if (s.kind == SK::Load && s.acc.sizes.size() > 1) {
+        return;
+      }
+      if (s.kind == SK::Map && (s.name.rfind("tt.", 0) == 0 && s.name.rfind("tt.clampf", 0) != 0 && s.name.rfind("tt.precise", 0) != 0)) return;
+    }
+    for (const auto *ops : {&slice_head, &slice_tail})
+      for (const SOp &s : *ops) {
+        if (s.kind == SK::Map && s.name.rfind("tt.", 0) == 0) return;
+        if (s.kind == SK::Reduce && (s.axis != 0 || val(s.operands[0]).shape != sh)) return;
+        if ((s.kind == SK::Load || s.kind == SK::Store) && s.acc.sizes == sh) return;
+      }
+    if (!any) return;
+    column_sums = wide_mode = true;
+    wide_shape = sh;
+  }
+  std::vector<const SOp *> row_loads;      // of those, the ones of the run being written
+  std::map<int, std::string> row_vectors;  // value id of a load of R elements -> the registers of the rows' owners
   // The sums of a sliced program's workgroups: each leaves its own in `partial` (written through, complete before its
   // arrival is counted), and the one that arrives last adds all of them in slice order -- the result does not depend on
-  // who that is -- and goes on with the program.  Nobody waits for anybody.  (The slices' sums are large next to what a
-  // thread of one workgroup adds up: added in fp32, db of LayerNorm on fp32 [3000, 1000] was 1.05e-7 off, 7.1e-8 in one slice.)
+  // who that is -- and goes on with the program.  Nobody waits for anybody.  (The arrival
+  // counters lie 128 bytes apart: in one line, the arrivals of 752 workgroups took 7 us, each waiting for the others'.  The
+  // slices' sums are large next to what a thread of one workgroup adds up: added in fp32, db of LayerNorm on fp32 [3000, 1000] was 1.05e-7 off, 7.1e-8 in one slice.)
   void slices_meet() {
     int64_t total = 0;
     for (const SOp &s : slice_head)
@@ -868,20 +906,33 @@ struct Gen {
       }
     os << pad() << "asm volatile(\"s_waitcnt vmcnt(0)\" ::: \"memory\");\n" << pad() << "__syncthreads();\n"
        << pad() << "if (threadIdx.x == 0) {\n"
-       << pad() << "  arrived = __hip_atomic_fetch_add(&counters[lin], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);\n"
-       << pad() << "  if (arrived == slices - 1) __hip_atomic_store(&counters[lin], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next launch\n"
+       << pad() << "  arrived = __hip_atomic_fetch_add(&counters[32 * lin], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);\n"
+       << pad() << "  if (arrived == slices - 1) __hip_atomic_store(&counters[32 * lin], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next launch\n"
        << pad() << "}\n" << pad() << "__syncthreads();\n" << pad() << "if (arrived != slices - 1) return;\n";
-    off = 0;
-    for (const SOp &s : slice_head)
-      if (s.kind == SK::Reduce) {
-        const int64_t n = val(s.result).shape[0];
-        os << pad() << "for (int c = threadIdx.x; c < " << n << "; c += 256) {\n"
-           << pad() << "  double sum = 0;\n" << pad() << "#pragma unroll 8\n"
-           << pad() << "  for (int s = 0; s < slices; s++) sum += __hip_atomic_load(&partial[((long long)s * programs + lin) * " << total << " + " << off
-           << " + c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);\n"
-           << pad() << "  " << at(s.result, "c", "0") << " = (float)sum;\n" << pad() << "}\n";
-        off += n;
-      }
+    // The sums of all results side by side, every thread with sixteen loads in flight; up to 128 of them leave threads over,
+    // which take every PARTS-th slice each (a slice's sum comes from memory: its writer may sit on another XCD).
+    const int64_t parts = total >= 256 ? 1 : 256 / total;
+    if (parts > 1) os << pad() << "__shared__ double part[" << parts * total << "];\n";
+    os << pad() << "for (int q = threadIdx.x; q < " << parts * total << "; q += 256) {\n"
+       << pad() << "  const int c = q % " << total << ";\n" << pad() << "  double sum = 0;\n" << pad() << "  #pragma unroll 16\n"
+       << pad() << "  for (int s = q / " << total << "; s < slices; s += " << parts << ") sum += __hip_atomic_load(&partial[((long long)s * programs + lin) * " << total
+       << " + c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);\n";
+    auto put = [&](const std::string &sum) {
+      int64_t at0 = 0;
+      for (const SOp &s : slice_head)
+        if (s.kind == SK::Reduce) {
+          const int64_t n = val(s.result).shape[0];
+          os << pad() << "  if (c >= " << at0 << " && c < " << at0 + n << ") " << at(s.result, "(c - " + std::to_string(at0) + ")", "0") << " = (float)" << sum << ";\n";
+          at0 += n;
+        }
+    };
+    if (parts > 1) {
+      os << pad() << "  part[q] = sum;\n" << pad() << "}\n" << pad() << "__syncthreads();\n"
+         << pad() << "for (int c = threadIdx.x; c < " << total << "; c += 256) {\n" << pad() << "  double sum = part[c];\n"
+         << pad() << "  for (int h = 1; h < " << parts << "; h++) sum += part[c + h * " << total << "];\n";
+    }
+    put("sum");
+    os << pad() << "}\n";
     os << pad() << "__syncthreads();\n";
     indent--;
     os << pad() << "}\n";
@@ -902,12 +953,14 @@ struct Gen {
   std::string idx0(const std::vector<int64_t> &shape) const {
     if (shape.size() < 2) return "t";
     const int64_t C = shape.back();
+    if (wide(shape) && C % 2048) return "((int)threadIdx.x / " + std::to_string(C / 8) + " + " + std::to_string(2048 / C) + " * (n >> 3))";
     if (C % 256 == 0) return C == 256 ? "n" : "(n / " + std::to_string(C / 256) + ")";
     return "(t / " + std::to_string(C) + ")";
   }
   std::string idx1(const std::vector<int64_t> &shape) const {
     if (shape.size() < 2) return "0";
     const int64_t C = shape.back();
+    if (wide(shape) && C % 2048) return "(8 * ((int)threadIdx.x % " + std::to_string(C / 8) + ") + (n & 7))";
     if (wide(shape)) return "(8 * (int)threadIdx.x + (n & 7) + 2048 * ((n >> 3) % " + std::to_string(C / 2048) + "))";
     if (C % 256 == 0) return C == 256 ? "(int)threadIdx.x" : "((int)threadIdx.x + 256 * (n % " + std::to_string(C / 256) + "))";
     return "(t % " + std::to_string(C) + ")";
@@ -1128,6 +1181,21 @@ struct Gen {
         const SOp &o = ops[q];
         const bool behind_transpose = transposed.count(o.result) && o.acc.sizes.size() == 2;
         if (o.kind != SK::Load || ((own(o) || big_other(o)) && !behind_transpose) || staged.count(o.result)) continue;
+        if (column_sums && loop_depth && o.acc.sizes.size() == 1 && o.acc.sizes[0] == wide_shape[0]) {
+          const std::string name = "row" + std::to_string(o.result), ct = ctype(val(o.result).dtype), mt = memtype(o.acc.elem), g = std::to_string(count(wide_shape) / 2048);
+          const bool r16 = is16(o.acc.elem);
+          os << pad() << mt << " raw_" << name << "[" << g << "];\n" << pad() << "#pragma unroll\n" << pad() << "for (int g = 0; g < " << g << "; g++) {\n";
+          indent++;
+          os << pad() << "const int n = 8 * g;\n";
+          std::string pred, addr = address(o.acc, idx0(wide_shape), "0", pred);
+          const std::string at_mem = "((const " + mt + " *)p.ptr[" + std::to_string(o.acc.base_arg) + "] + (" + addr + "))";
+          os << pad() << "raw_" << name << "[g] = *(" << (pred.empty() ? at_mem : "(" + pred + ") ? " + at_mem + " : (const " + mt + " *)tts_dummy") << ");\n";
+          indent--;
+          os << pad() << "}\n";
+          uses_dummy = true;
+          row_loads.push_back(&o);
+          continue;
+        }
         const int64_t pitch = behind_transpose ? o.acc.sizes.back() + 1 : (o.acc.sizes.empty() ? 1 : o.acc.sizes.back());
         const int64_t elems = behind_transpose ? o.acc.sizes[0] * pitch : count(o.acc.sizes);
         const size_t bytes = (size_t)elems * held_bytes(val(o.result).dtype);
@@ -1438,7 +1506,18 @@ struct Gen {
           close_loop();
           fill_others();
         }
-        if (any_load) os << pad() << "__syncthreads();\n";
+        for (const SOp *o : row_loads) {
+          const std::string name = "row" + std::to_string(o->result), g = std::to_string(count(wide_shape) / 2048);
+          const std::string got = o->acc.elem == "f16" ? "up_f16(raw_" + name + "[g])" : o->acc.elem == "bf16" ? "up_bf16(raw_" + name + "[g])" : "raw_" + name + "[g]";
+          os << pad() << ctype(val(o->result).dtype) << " " << name << "[" << g << "];\n" << pad() << "#pragma unroll\n" << pad() << "for (int g = 0; g < " << g << "; g++) {\n";
+          os << pad() << "  const int n = 8 * g;\n" << pad() << "  (void)n;\n";
+          std::string pred;
+          address(o->acc, idx0(wide_shape), "0", pred);
+          os << pad() << "  " << name << "[g] = " << (pred.empty() ? got : "(" + pred + ") ? " + got + " : " + other_of(o->acc, idx0(wide_shape), "0")) << ";\n" << pad() << "}\n";
+          row_vectors[o->result] = name;
+        }
+        row_loads.clear();
+        if (any_load && !(column_sums && loop_depth)) os << pad() << "__syncthreads();\n";
         if (stores && wide(shape))  // wide stores collect a group's eight values (see the Store case below)
           for (size_t q = k; q < end; q++)
             if (ops[q].kind == SK::Store && vector_access(ops[q].acc)) os << pad() << "unsigned sv" << q << "[8];\n";
@@ -2431,6 +2510,7 @@ std::string tile_program_source(const Program &p, bool allow_persistent) {
   g.choose_wide_shape();
   if (allow_persistent) g.choose_persistent();
   if (!g.persistent) g.choose_slices();
+  g.choose_column_sums();
   if (g.persistent) g.indent = 2;
   if (g.sliced) {
     g.body(g.slice_head);
