@@ -47,6 +47,42 @@ def test_cfg1_vec_add_bit_exact(K, oracle_cpu):
     assert torch.equal(zd[n:].cpu(), torch.full((64,), -7.0))  # the masked tail is not written
 
 
+@pytest.mark.parametrize("form", ["tensors", "parameters", "addresses", "numpy", "object", "hooks", "no hooks", "wrong"])
+def test_launcher_takes_every_form_of_argument(form):
+    """The launcher's native part and its general one, each over the arguments that belong to it: the same launch."""
+    import test_boundary
+    import triton_shared_amd as tsa
+    plan, _ = plan_for(tsa._native, "vec_add")
+    launcher = tsa.HIPLauncher(test_boundary._Src, None)
+    n = 5000
+    x, y, z = torch.rand(n, device=DEV), torch.rand(n, device=DEV), torch.zeros(n, device=DEV)
+    class Holder:
+        def __init__(self, t): self.t = t
+        def data_ptr(self): return self.t.data_ptr()
+    events = []
+    enter, leave = (lambda md: events.append(("enter", md))), (lambda md: events.append(("exit", md)))
+    chain = triton.knobs.HookChain() if form == "no hooks" else None
+    ptrs, count, hooks = [x, y, z], n, (chain, chain)
+    if form == "parameters": ptrs = [torch.nn.Parameter(x), torch.nn.Parameter(y), z]
+    if form == "addresses": ptrs = [t.data_ptr() for t in ptrs]
+    if form == "numpy": count = np.int64(n)
+    if form == "object": ptrs = [Holder(t) for t in ptrs]
+    if form == "hooks": hooks = (enter, leave)
+    torch.cuda.synchronize()
+    stream = torch.cuda.current_stream().cuda_stream
+    if form == "wrong":
+        with pytest.raises(TypeError, match="lives on device"):
+            launcher(5, 1, 1, stream, plan, None, None, None, None, x, torch.zeros(n), z, n, 1024)
+        with pytest.raises(RuntimeError, match="expects"):
+            other, _ = plan_for(tsa._native, "row_softmax")
+            launcher(5, 1, 1, stream, other, None, None, None, None, x, y, z, n, 1024)
+        return
+    launcher(5, 1, 1, stream, plan, None, "md", *hooks, *ptrs, count, 1024)
+    torch.cuda.synchronize()
+    assert torch.equal(z, x + y)
+    assert events == ([("enter", "md"), ("exit", "md")] if form == "hooks" else [])
+
+
 @pytest.mark.parametrize("n", [1, 3, 1023, 1024, 1025, 5000, (1 << 22) + 5])
 def test_vec_add_sizes_and_unaligned_views(K, oracle_cpu, n):
     torch.manual_seed(n)

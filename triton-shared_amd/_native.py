@@ -1,10 +1,13 @@
 """ctypes binding of libtts_hip.so (C ABI declared in include/tts_hip.h)."""
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 import subprocess
 
 _CSRC = os.path.join(os.path.dirname(os.path.abspath(__file__)), "csrc")
 LIB_PATH = os.path.join(_CSRC, "libtts_hip.so")
+LAUNCH_PATH = os.path.join(_CSRC, "tts_launch.so")  # the launcher's base class (csrc/launch_module.cpp)
 
 TTS_OK, TTS_UNSUPPORTED, TTS_INVALID, TTS_HIP_ERROR = 0, 1, 2, 3
 ARG_PTR, ARG_INT, ARG_FLOAT = 0, 1, 2
@@ -60,8 +63,42 @@ def lib():
     L.tts_launch.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_void_p,
                              ctypes.POINTER(TtsArg), ctypes.c_int]
     L.tts_launch_noalloc.argtypes = L.tts_launch.argtypes
+    import torch
+    import triton
+    chain = getattr(getattr(triton, "knobs", None), "HookChain", None)
+    launch_module().setup(ctypes.cast(L.tts_launch, ctypes.c_void_p).value, PlanHandle, _raise, torch.Tensor, torch.nn.Parameter, chain)
     _lib = L
     return L
+
+
+_launch = None
+
+
+def launch_module():
+    """The extension module behind HIPLauncher; fails loudly if it has not been built."""
+    global _launch
+    if _launch is None:
+        if not os.path.exists(LAUNCH_PATH):
+            raise RuntimeError(f"{LAUNCH_PATH} is missing: the launch extension has not been built (run `make -C triton-shared_amd/csrc`)")
+        loader = importlib.machinery.ExtensionFileLoader("tts_launch", LAUNCH_PATH)
+        spec = importlib.util.spec_from_file_location("tts_launch", LAUNCH_PATH, loader=loader)
+        _launch = importlib.util.module_from_spec(spec)
+        loader.exec_module(_launch)
+    return _launch
+
+
+class _Unbuilt:
+    """Stands in for the native base in a process that imports the package before it is built: every call is `_generic`."""
+
+    def _bind(self, slots):
+        pass
+
+    def __call__(self, *args):
+        return self._generic(*args)
+
+
+def launcher_base():
+    return launch_module().Launcher if os.path.exists(LAUNCH_PATH) else _Unbuilt
 
 
 def _raise(status):
@@ -108,11 +145,13 @@ class PlanHandle:
         if st != TTS_OK:
             _raise(st)
         self._h = h
+        self._address = h.value  # for csrc/launch_module.cpp, with _kinds
         L = lib()
         self.kernel_name = L.tts_plan_kernel_name(h).decode()
         self.family = L.tts_plan_family(h).decode()
         self.signature = L.tts_plan_signature(h).decode()
         self.arg_kinds = [L.tts_plan_arg_kind(h, i) for i in range(L.tts_plan_num_args(h))]
+        self._kinds = bytes(self.arg_kinds)
 
     def __del__(self):
         try:

@@ -56,9 +56,12 @@ def _device_pointer(obj, index):
     return p
 
 
-class HIPLauncher(object):
+class HIPLauncher(_native.launcher_base()):
     """launch(gridX, gridY, gridZ, stream, function, kernel_metadata, launch_metadata,
-    launch_enter_hook, launch_exit_hook, *args) -- the call Triton's JIT makes."""
+    launch_enter_hook, launch_exit_hook, *args) -- the call Triton's JIT makes.
+
+    The base class (csrc/launch_module.cpp) takes the ordinary calls -- ints, floats and torch tensors on the GPU, no
+    hooks -- straight to tts_launch; `_generic` is every other call, and what both mean."""
 
     def __init__(self, src, metadata):
         constants = src.constants if hasattr(src, "constants") else dict()
@@ -73,8 +76,9 @@ class HIPLauncher(object):
                 continue
             _ty_to_cpp(ty)
             self.slots.append((i, ty[0] == "*"))
+        self._bind(self.slots)
 
-    def __call__(self, gridX, gridY, gridZ, stream, function, kernel_metadata, launch_metadata,
+    def _generic(self, gridX, gridY, gridZ, stream, function, kernel_metadata, launch_metadata,
                  launch_enter_hook, launch_exit_hook, *args):
         plan = function
         if not isinstance(plan, _native.PlanHandle):
@@ -146,11 +150,14 @@ class HIPDriver(DriverBase):
 
     def get_current_stream(self, device):
         import torch
-        return torch.cuda.current_stream(device).cuda_stream
+        # the current stream's handle without the Stream object around it (0.1 us of a launch instead of 1.2)
+        return torch._C._cuda_getCurrentRawStream(device)
 
     def get_current_device(self):
         import torch
-        return torch.cuda.current_device()
+        device = torch.cuda.current_device()  # (initialises the GPU if nothing has)
+        self.get_current_device = torch._C._cuda_getDevice
+        return device
 
     def set_current_device(self, device):
         import torch
