@@ -506,6 +506,29 @@ def test_gemm_any_shape_kernel_reads_and_writes_only_its_problem(K, M, N, Kd, pa
     assert (cd[M] == 7.0).all() and (cd[:, N] == 7.0).all()
 
 
+@pytest.mark.parametrize("at,bt", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("M,N,Kd", [(8, 8, 8), (64, 9, 9), (65, 127, 63), (63, 129, 65), (129, 200, 129), (9, 333, 320), (1000, 8, 193), (3001, 1031, 71), (7, 300, 100), (300, 7, 100), (300, 100, 7)])
+def test_gemm_any_shape_kernel_at_the_ends_of_its_tiles(K, M, N, Kd, at, bt):
+    # tiles of 64 and of 128 rows; a last K tile whose chunks are read from the last eight k (or the last row's last eight
+    # elements) and put right, operands of exactly eight and of fewer; NaN beside the operands reaches no result.  Small
+    # integers: exact in any order
+    g = torch.Generator().manual_seed(M + N + Kd)
+    def operand(rows, cols, turned):
+        x = torch.randint(-2, 3, (rows, cols), generator=g).to(torch.bfloat16)
+        full = torch.full((cols, rows + 1) if turned else (rows, cols + 1), float("nan"), dtype=torch.bfloat16)
+        full[:, :rows if turned else cols] = x.t() if turned else x
+        d = full.to(DEV)
+        return x, (d.t()[:rows] if turned else d[:, :cols])
+    (a, ad), (b, bd) = operand(M, Kd, at), operand(Kd, N, bt)
+    cd = torch.full((M + 1, N + 1), 7.0, dtype=torch.bfloat16, device=DEV)
+    k = K.matmul_tiles[(triton.cdiv(M, 128) * triton.cdiv(N, 128),)](ad, bd, cd, M, N, Kd, ad.stride(0), ad.stride(1), bd.stride(0), bd.stride(1), N + 1, 1, BM=128, BN=128, BK=64, GROUP_M=8)
+    torch.cuda.synchronize()
+    assert k.function.last_kernel.startswith("gemm_mfma_kernel")
+    want = (a.double() @ b.double()).bfloat16()
+    assert torch.equal(cd[:M, :N].cpu(), want)
+    assert (cd[M] == 7.0).all() and (cd[:, N] == 7.0).all()
+
+
 @pytest.mark.parametrize("M,N,Kd,bt,dtype", [(17, 129, 4095, True, torch.bfloat16), (100, 700, 2000, False, torch.float16), (200, 15, 1984, False, torch.bfloat16), (130, 257, 1153, True, torch.float16)])
 def test_gemm_any_shape_kernel_in_k_slices(K, M, N, Kd, bt, dtype):
     # few tiles and a long K: slices whose sums a second kernel adds, narrow and wide rows; with and without a functor that

@@ -2,7 +2,7 @@
 // time into the library (kernels_gemm.hip, results stored as they are), and at run time with hipRTC when the Triton
 // kernel applies elementwise ops to the accumulator before the store (a fused activation): the generated source
 // defines TTS_GEMM_RTC (which kernel: 0 whole 256 x 256 x 32 tiles, 1 any shape in 128 x 128 x 64 tiles, 2 the sum of the K
-// slices), TTS_GEMM_BF16 and the functor TtsEp (a plain struct, passed as the kernel's last argument) that maps an accumulator value and its position to the value stored, then this file's text.  Nothing here may need a host header.
+// slices, 3 as 1 in 64 x 128 x 64 tiles), TTS_GEMM_BF16 and the functor TtsEp (a plain struct, passed as the kernel's last argument) that maps an accumulator value and its position to the value stored, then this file's text.  Nothing here may need a host header.
 #pragma once
 #ifdef __HIPCC_RTC__
 typedef __INT64_TYPE__ int64_t;
@@ -90,10 +90,18 @@ __device__ __forceinline__ uint4 load8(const uint16_t *p, int valid, bool vec) {
   return make_uint4(w[0], w[1], w[2], w[3]);
 }
 
+// eight elements without their first k (1 .. 7), moved to the front
+__device__ __forceinline__ uint4 without_first(uint4 v, int k) {
+  if (k & 4) v = make_uint4(v.z, v.w, 0, 0);
+  if (k & 2) v = make_uint4(v.y, v.z, v.w, 0);
+  if (k & 1) v = make_uint4(v.x >> 16 | v.y << 16, v.y >> 16 | v.z << 16, v.z >> 16 | v.w << 16, v.w >> 16);
+  return v;
+}
+
 // ------------------------------------------------------------- 16-bit GEMM
 // The kernel for any shape, any alignment, and operands that are row- or column-major.
 // Workgroup: 256 threads = 2 x 2 wavefronts; each wavefront owns TM x TN MFMA tiles of 32 x 32.  An operand tile is
-// R = BM = BN rows (rows of A, columns of B) by BK values of k and is staged through LDS (two buffers) in the form it
+// R = BM or BN rows (rows of A, columns of B) by BK values of k and is staged through LDS (two buffers) in the form it
 // has in memory, with 16-byte loads and stores:
 //   k contiguous (A row-major, B column-major): LDS [r][k], pitch BK + 8 elements; a lane's MFMA operand (8 consecutive
 //     k of row lane % 32) is one 16-byte read, and 32 consecutive rows hit distinct banks;
@@ -101,10 +109,11 @@ __device__ __forceinline__ uint4 load8(const uint16_t *p, int valid, bool vec) {
 //     the way out -- within 16 lanes, lane i receives element i % 4 of the 8-byte rows addressed by lanes i / 4,
 //     i / 4 + 4, i / 4 + 8, i / 4 + 12, so lane j of a group addresses k row j / 4, elements 4 (j % 4) .. +3 of the
 //     group's 16, and two reads (k 0-3, k 4-7) make one operand.
-// What bounds it on ragged sizes is the way of the operands from memory, a chain of one load per K tile where a shape
-// gives the chip less than one workgroup per CU.  Chunks are therefore 16-byte loads at any alignment (global memory takes
-// them at element addresses), untested in all K tiles but the last, and two tiles are in flight.  1000 x 3001 x 1003 fp16 with
-// a fused activation: 27.8 us; with eight two-byte loads for every chunk that is not 16-byte aligned, each behind a test, 163.
+// What bounds it on ragged sizes is the way of the operands from memory: a chain of one load per K tile where a shape gives the
+// chip less than one workgroup per CU, else the rate at which a CU takes 16-byte loads that are not 16-byte aligned.  Chunks are
+// 16-byte loads at any alignment (global memory takes them at element addresses), untested, and two tiles are in flight.
+// 1000 x 3001 x 1003 fp16 with a fused activation: 25 us (163 with two-byte loads, each behind a test, and 30 while only the last
+// K tiles were loaded that way); TM, TN: 128 x 128 tiles or, for few of them, 64 x 128 (kernels_gemm.hip: any_rows).
 // Rows of A may be taken through an index vector (p.a_rows) and the base of B may depend on the block of rows
 // (p.b_block): a mixture-of-experts product is this kernel with both set.
 // `ep(acc, row, col)` maps an accumulator value to the value that is stored at (row, col) of C (the identity for a plain
@@ -112,6 +121,11 @@ __device__ __forceinline__ uint4 load8(const uint16_t *p, int valid, bool vec) {
 template <bool V>
 struct BoolConstant {
   static constexpr bool value = V;
+};
+
+template <int ROWS, int CHUNKS>  // an operand's tile: its rows, and how many 16-byte chunks of it a thread moves
+struct TileOf {
+  static constexpr int R = ROWS, N = CHUNKS;
 };
 
 template <int BM, int BN, int BK>
@@ -128,10 +142,8 @@ struct GemmStageLds {
 template <bool BF16, int TM, int TN, int BK, class Ep, bool SK = false>
 __device__ __forceinline__ void gemm_mfma_body(const GemmParams &p, int tiles_m, int tiles_n, const Ep &ep) {
   constexpr int BM = 2 * TM * 32, BN = 2 * TN * 32;
-  constexpr int PK = BK + 8;   // pitch of a k-contiguous tile
-  constexpr int PR = BM + 16;  // pitch of an r-contiguous tile
-  constexpr int CA = BM * BK / 8 / 256;  // 16-byte chunks of an operand tile per thread
-  static_assert(BM == BN, "both operands are staged by the same routines");
+  constexpr int PK = BK + 8;  // pitch of a k-contiguous tile (an r-contiguous one of R rows: R + 16)
+  constexpr int CA = BM * BK / 8 / 256, CB = BN * BK / 8 / 256;  // 16-byte chunks of an operand tile per thread
   using Lds = GemmStageLds<BM, BN, BK>;
 #ifdef TTS_GEMM_RTC
   __shared__ __align__(16) uint16_t smem[2 * Lds::BUFFER_ELEMS];
@@ -167,7 +179,7 @@ __device__ __forceinline__ void gemm_mfma_body(const GemmParams &p, int tiles_m,
 
   // where this thread's chunks of the tiles are: (row, k chunk) of a k-contiguous tile, (k, row chunk) of an
   // r-contiguous one; element offsets of the chunks' rows in memory (-1: outside the problem)
-  int64_t a_at[CA], b_at[CA];
+  int64_t a_at[CA], b_at[CB];
 #pragma unroll
   for (int j = 0; j < CA; j++) {
     const int c = tid + 256 * j;
@@ -179,6 +191,10 @@ __device__ __forceinline__ void gemm_mfma_body(const GemmParams &p, int tiles_m,
       else if (!p.a_rows) a_at[j] = gr * p.lda;
       else a_at[j] = (p.gather_mul32 & 1) ? (int64_t)(int)((uint32_t)p.a_rows[gr] * (uint32_t)p.lda) : (int64_t)p.a_rows[gr] * p.lda;
     }
+  }
+#pragma unroll
+  for (int j = 0; j < CB; j++) {
+    const int c = tid + 256 * j;
     if (p.b_trans) {
       const int64_t gn = n0 + c / (BK / 8);
       b_at[j] = gn < p.N ? gn * p.ldb : -1;
@@ -186,12 +202,13 @@ __device__ __forceinline__ void gemm_mfma_body(const GemmParams &p, int tiles_m,
       b_at[j] = n0 + (c % (BN / 8)) * 8;
     }
   }
-  auto load_operand = [&](uint4 (&reg)[CA], const uint16_t *P, bool r_contiguous, const int64_t (&at)[CA], int64_t ld, int64_t rows, bool vec, int k0) {
+  auto load_operand = [&](auto of, auto &reg, const uint16_t *P, bool r_contiguous, const auto &at, int64_t ld, int64_t rows, bool vec, int k0) {
+    constexpr int R = decltype(of)::R, N = decltype(of)::N;
 #pragma unroll
-    for (int j = 0; j < CA; j++) {
+    for (int j = 0; j < N; j++) {
       const int c = tid + 256 * j;
       if (r_contiguous) {
-        const int gk = k0 + c / (BM / 8);
+        const int gk = k0 + c / (R / 8);
         const int valid = (int)min((int64_t)8, rows - at[j]);
         reg[j] = (gk < K && valid > 0) ? load8(P + (int64_t)gk * ld + at[j], valid, vec) : make_uint4(0, 0, 0, 0);
       } else {
@@ -200,16 +217,19 @@ __device__ __forceinline__ void gemm_mfma_body(const GemmParams &p, int tiles_m,
       }
     }
   };
-  auto store_operand = [&](const uint4 (&reg)[CA], uint16_t *S, bool r_contiguous) {
+  auto store_operand = [&](auto of, const auto &reg, uint16_t *S, bool r_contiguous) {
+    constexpr int R = decltype(of)::R, N = decltype(of)::N;
 #pragma unroll
-    for (int j = 0; j < CA; j++) {
+    for (int j = 0; j < N; j++) {
       const int c = tid + 256 * j;
-      if (r_contiguous) *reinterpret_cast<uint4 *>(S + (c / (BM / 8)) * PR + (c % (BM / 8)) * 8) = reg[j];
+      if (r_contiguous) *reinterpret_cast<uint4 *>(S + (c / (R / 8)) * (R + 16) + (c % (R / 8)) * 8) = reg[j];
       else *reinterpret_cast<uint4 *>(S + (c / (BK / 8)) * PK + (c % (BK / 8)) * 8) = reg[j];
     }
   };
   // a lane's MFMA operand for the 32 rows starting at `row0` of a staged tile, k = ks * 16 + 8 (lane / 32) .. +7
-  auto fragment = [&](const uint16_t *S, bool r_contiguous, int row0, int ks) -> uint4 {
+  auto fragment = [&](auto of, const uint16_t *S, bool r_contiguous, int row0, int ks) -> uint4 {
+    constexpr int R = decltype(of)::R;
+    constexpr int PR = R + 16;
     if (!r_contiguous) return *reinterpret_cast<const uint4 *>(S + (row0 + (lane & 31)) * PK + ks * 16 + 8 * (lane >> 5));
     const int g = lane >> 4, j = lane & 15;
     const uint16_t *at = S + (ks * 16 + 8 * (g >> 1) + (j >> 2)) * PR + row0 + 16 * (g & 1) + 4 * (j & 3);
@@ -219,6 +239,8 @@ __device__ __forceinline__ void gemm_mfma_body(const GemmParams &p, int tiles_m,
     const uint2 l2 = __builtin_bit_cast(uint2, lo), h2 = __builtin_bit_cast(uint2, hi);
     return make_uint4(l2.x, l2.y, h2.x, h2.y);
   };
+  const TileOf<BM, CA> of_a;
+  const TileOf<BN, CB> of_b;
 
   f32x16 acc[TM][TN];
 #pragma unroll
@@ -235,46 +257,80 @@ __device__ __forceinline__ void gemm_mfma_body(const GemmParams &p, int tiles_m,
   const int nk = SK ? (int)((int64_t)(slice + 1) * nk_all / p.split) : nk_all;  // K tiles [k_begin, nk) are this workgroup's
   auto sweep_k = [&](auto a_form, auto b_form) {
     constexpr bool a_r = decltype(a_form)::value, b_r = decltype(b_form)::value;  // r-contiguous in memory and in LDS
-    // K tiles [0, nwide) load 16 bytes a chunk without a test, at any alignment: rows (columns) beyond the problem are
-    // replaced by others, they only reach results nobody stores; a chunk that starts inside a row of an r-contiguous
-    // operand and ends behind it reads into the next row, which the last k row does not have.
+    // Chunks are loaded without a test, at any alignment.  Rows (columns) beyond the problem are replaced by others, they only
+    // reach results nobody stores; a chunk that starts inside a row of an r-contiguous operand and ends behind it reads into
+    // the next row.  K tiles [0, nwide) have no chunk that reads past the operand that way.
     int nwide = K / BK;
-    if ((a_r && p.lda < 8) || (b_r && p.ldb < 8)) nwide = 0;
-    else if (K % BK == 0 && ((a_r && m0 + BM > p.M) || (b_r && n0 + BN > p.N))) nwide = nk_all - 1;
+    if (K % BK == 0 && ((a_r && m0 + BM > p.M) || (b_r && n0 + BN > p.N))) nwide = nk_all - 1;
     nwide = min(nwide, nk);
-    const uint16_t *a_ptr[CA], *b_ptr[CA];
-    auto first_chunk = [&](const uint16_t *P, bool r_contiguous, const int64_t at, int64_t other, int64_t ld, int64_t rows, int c) {
-      return r_contiguous ? P + (c / (BM / 8)) * ld + (at < rows ? at : 0) : P + (at >= 0 ? at : other) + (c % (BK / 8)) * 8;
-    };
     // a row beyond the problem: the tile's first, or where rows are gathered the operand's first (store_tiles clears them)
-    const int64_t a_first = a_r || p.a_rows ? 0 : m0 * p.lda;
+    const int64_t a_first = a_r || p.a_rows ? 0 : m0 * p.lda, b_first = n0 * p.ldb;
+    auto first_chunk = [&](auto of, auto &ptr, const uint16_t *P, bool r_contiguous, const auto &at, int64_t other, int64_t ld, int64_t rows) {
+      constexpr int R = decltype(of)::R, N = decltype(of)::N;
 #pragma unroll
-    for (int j = 0; j < CA; j++) {
-      a_ptr[j] = first_chunk(A, a_r, a_at[j], a_first, p.lda, p.M, tid + 256 * j);
-      b_ptr[j] = first_chunk(B, b_r, b_at[j], n0 * p.ldb, p.ldb, p.N, tid + 256 * j);
-    }
-    struct Tiles { uint4 a[CA], b[CA]; };
+      for (int j = 0; j < N; j++) {
+        const int c = tid + 256 * j;
+        ptr[j] = r_contiguous ? P + (c / (R / 8)) * ld + (at[j] < rows ? at[j] : 0) : P + (at[j] >= 0 ? at[j] : other) + (c % (BK / 8)) * 8;
+      }
+    };
+    const uint16_t *a_ptr[CA], *b_ptr[CB];
+    first_chunk(of_a, a_ptr, A, a_r, a_at, a_first, p.lda, p.M);
+    first_chunk(of_b, b_ptr, B, b_r, b_at, b_first, p.ldb, p.N);
+    struct Tiles { uint4 a[CA], b[CB]; };
     auto load_wide = [&](Tiles &t, int kt) {
       const int64_t a_k = a_r ? (int64_t)kt * BK * p.lda : (int64_t)kt * BK, b_k = b_r ? (int64_t)kt * BK * p.ldb : (int64_t)kt * BK;
 #pragma unroll
       for (int j = 0; j < CA; j++) __builtin_memcpy(&t.a[j], a_ptr[j] + a_k, 16);
 #pragma unroll
-      for (int j = 0; j < CA; j++) __builtin_memcpy(&t.b[j], b_ptr[j] + b_k, 16);
+      for (int j = 0; j < CB; j++) __builtin_memcpy(&t.b[j], b_ptr[j] + b_k, 16);
     };
-    auto load_any = [&](Tiles &t, int kt) {
-      if (kt < nwide) load_wide(t, kt);
-      else if (kt < nk) {
-        load_operand(t.a, A, a_r, a_at, p.lda, p.M, a_vec, kt * BK);
-        load_operand(t.b, B, b_r, b_at, p.ldb, p.N, b_vec, kt * BK);
+    // Any K tile, the one that ends the K loop included: there a chunk that sticks out of its row (k contiguous) or of the last k
+    // row (r contiguous) is read from the last eight elements and put right when it is stored to LDS, chunks past K become
+    // zeros.  Tiles past the last load it again, so that the loop's tail has no branch around a load either: at one, the
+    // compiler waits for every load in flight.  (Element by element behind tests, and with branches, the last tiles took a
+    // third of 1000 x 3001 x 1003 and of the slices of 600 x 601 x 3001.)
+    auto load_tail = [&](auto of, auto &reg, const uint16_t *P, bool r_contiguous, const auto &at, int64_t other, int64_t ld, int64_t rows, int kt) {
+      constexpr int R = decltype(of)::R, N = decltype(of)::N;
+#pragma unroll
+      for (int j = 0; j < N; j++) {
+        const int c = tid + 256 * j;
+        const uint16_t *src;
+        if (r_contiguous) {
+          const int row = min(kt * BK + c / (R / 8), K - 1);
+          src = P + (int64_t)row * ld + (row == K - 1 ? min(at[j], rows - 8) : at[j] < rows ? at[j] : 0);
+        } else {
+          src = P + (at[j] >= 0 ? at[j] : other) + min(kt * BK + (c % (BK / 8)) * 8, K - 8);
+        }
+        __builtin_memcpy(&reg[j], src, 16);
       }
     };
-    auto store_tiles = [&](const Tiles &t, int buf) {
+    auto settle_tail = [&](auto of, auto &reg, bool r_contiguous, const auto &at, int64_t rows, int kt) {
+      constexpr int R = decltype(of)::R, N = decltype(of)::N;
+#pragma unroll
+      for (int j = 0; j < N; j++) {
+        const int c = tid + 256 * j;
+        const int gk = kt * BK + (r_contiguous ? c / (R / 8) : (c % (BK / 8)) * 8);
+        const int cut = !r_contiguous ? max(0, gk + 8 - K) : gk == K - 1 ? (int)max((int64_t)0, at[j] + 8 - rows) : 0;
+        if (gk >= K) reg[j] = make_uint4(0, 0, 0, 0);
+        else if (cut > 0 && cut < 8) reg[j] = without_first(reg[j], cut);
+      }
+    };
+    auto load_any = [&](Tiles &t, int kt) {
+      kt = min(kt, nk - 1);
+      load_tail(of_a, t.a, A, a_r, a_at, a_first, p.lda, p.M, kt);
+      load_tail(of_b, t.b, B, b_r, b_at, b_first, p.ldb, p.N, kt);
+    };
+    auto store_tiles = [&](Tiles &t, int buf, bool last) {
+      if (last) {
+        settle_tail(of_a, t.a, a_r, a_at, p.M, nk_all - 1);
+        settle_tail(of_b, t.b, b_r, b_at, p.N, nk_all - 1);
+      }
       uint16_t *As = smem + buf * Lds::BUFFER_ELEMS, *Bs = As + Lds::A_ELEMS;
       uint4 a[CA];
 #pragma unroll
       for (int j = 0; j < CA; j++) a[j] = a_r || a_at[j] >= 0 ? t.a[j] : make_uint4(0, 0, 0, 0);
-      store_operand(a, As, a_r);
-      store_operand(t.b, Bs, b_r);
+      store_operand(of_a, a, As, a_r);
+      store_operand(of_b, t.b, Bs, b_r);
     };
     auto multiply = [&](int buf) {
       const uint16_t *As = smem + buf * Lds::BUFFER_ELEMS, *Bs = As + Lds::A_ELEMS;
@@ -282,41 +338,55 @@ __device__ __forceinline__ void gemm_mfma_body(const GemmParams &p, int tiles_m,
       for (int ks = 0; ks < BK / 16; ks++) {
         uint4 af[TM], bf[TN];
 #pragma unroll
-        for (int i = 0; i < TM; i++) af[i] = fragment(As, a_r, wm * TM * 32 + i * 32, ks);
+        for (int i = 0; i < TM; i++) af[i] = fragment(of_a, As, a_r, wm * TM * 32 + i * 32, ks);
 #pragma unroll
-        for (int j = 0; j < TN; j++) bf[j] = fragment(Bs, b_r, wn * TN * 32 + j * 32, ks);
+        for (int j = 0; j < TN; j++) bf[j] = fragment(of_b, Bs, b_r, wn * TN * 32 + j * 32, ks);
 #pragma unroll
         for (int i = 0; i < TM; i++)
 #pragma unroll
           for (int j = 0; j < TN; j++) acc[i][j] = mfma32<BF16>(af[i], bf[j], acc[i][j]);
       }
     };
-    // Two K tiles are in flight in registers beside the two in LDS: a tile's loads are issued two products before they are stored.
     Tiles even, odd;
+    // Products of fewer than eight rows, columns or k have no eight elements to read: a tile at a time, chunks element by element.
+    if (K < 8 || (a_r && (p.M < 8 || p.lda < 8)) || (b_r && (p.N < 8 || p.ldb < 8))) {
+      for (int kt = k_begin; kt < nk; kt++) {
+        load_operand(of_a, even.a, A, a_r, a_at, p.lda, p.M, a_vec, kt * BK);
+        load_operand(of_b, even.b, B, b_r, b_at, p.ldb, p.N, b_vec, kt * BK);
+        store_tiles(even, 0, false);
+        __syncthreads();
+        multiply(0);
+        __syncthreads();
+      }
+      return;
+    }
+    if (nk <= k_begin) return;
+    // Two K tiles are in flight in registers beside the two in LDS: a tile's loads are issued two products before they are stored.
     load_any(even, k_begin);
     load_any(odd, k_begin + 1);
-    if (nk > k_begin) store_tiles(even, 0);
+    store_tiles(even, 0, k_begin == nk_all - 1);
     load_any(even, k_begin + 2);
     __syncthreads();
     int kt = k_begin;
     for (; kt + 4 < nwide; kt += 2) {  // loads tiles kt + 3 and kt + 4
       multiply(0);
-      store_tiles(odd, 1);
+      store_tiles(odd, 1, false);
       load_wide(odd, kt + 3);
       __syncthreads();
       multiply(1);
-      store_tiles(even, 0);
+      store_tiles(even, 0, false);
       load_wide(even, kt + 4);
       __syncthreads();
     }
     for (; kt < nk; kt += 2) {
       multiply(0);
       if (kt + 1 >= nk) break;
-      store_tiles(odd, 1);
+      store_tiles(odd, 1, kt + 1 == nk_all - 1);
       load_any(odd, kt + 3);
       __syncthreads();
       multiply(1);
-      if (kt + 2 < nk) store_tiles(even, 0);
+      if (kt + 2 >= nk) break;
+      store_tiles(even, 0, kt + 2 == nk_all - 1);
       load_any(even, kt + 4);
       __syncthreads();
     }
@@ -1089,7 +1159,7 @@ extern "C" __global__ __launch_bounds__(256) void gemm_rtc(TtsGemmParams p, int 
 #elif TTS_GEMM_RTC == 2
   tts_gemm_device::gemm_splitk_reduce_body<TTS_GEMM_BF16 != 0>(p, tiles_m, tiles_n, ep);  // (across, col_blocks)
 #else
-  tts_gemm_device::gemm_mfma_body<TTS_GEMM_BF16 != 0, 2, 2, 64>(p, tiles_m, tiles_n, ep);
+  tts_gemm_device::gemm_mfma_body<TTS_GEMM_BF16 != 0, TTS_GEMM_RTC == 3 ? 1 : 2, 2, 64>(p, tiles_m, tiles_n, ep);
 #endif
 }
 #endif

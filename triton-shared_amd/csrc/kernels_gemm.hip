@@ -45,16 +45,40 @@ struct ReduceGrid {
   }
 };
 
+int device_cus() {  // of the current device (256 when the query fails)
+  static const int cus = [] {
+    int dev = 0, n = 0;
+    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
+    return n;
+  }();
+  return cus;
+}
+// The height of the any-shape kernel's tiles, 64 or 128 rows (their width is 128).  What bounds the kernel on a full chip is the
+// rate at which a CU takes 16-byte loads off the 16-byte grid, and the larger tile loads a third less for the same product
+// (4001 x 4003 x 4005 bf16: 208 us against 298; 3001 x 3003 x 1001 52.8 / 56.4).  Up to one and a half of the larger tiles per CU
+// the smaller ones spread better, or pad fewer rows (us with 128 / 64 rows: 33 x 4001 x 4001 21.2 / 13.5, 3001 x 401 x 2003 29.9 /
+// 23.5, 64 x 1003 x 517 17.6 / 11.8, 2000 x 1000 x 520 16.8 / 11.9, 1000 x 3001 x 1003 26.4 / 25.2, 2001 x 2003 x 2005 43.3 / 44.2).
+int any_rows(const GemmParams &p, int split) {
+  static const char *env = getenv("TTS_GEMM_ROWS");  // tuning aid: "64" or "128"
+  if (env) return atoi(env) == 64 ? 64 : 128;
+  const int64_t tiles = ((p.M + 127) / 128) * ((p.N + 127) / 128) * std::max(1, p.batches) * split;
+  return p.M <= 64 || 2 * tiles <= 3 * device_cus() ? 64 : 128;
+}
+
 // p.split > 1: the slices alone; whoever launches it adds them
-template <bool BF16, bool SK>
-hipError_t launch_gemm_any(const GemmParams &p, hipStream_t s) {
-  constexpr size_t lds = GemmStageLds<128, 128, 64>::BYTES;
-  auto kern = gemm_mfma_kernel<BF16, 2, 2, 64, SK>;
+template <bool BF16, bool SK, int TM>
+hipError_t launch_gemm_any_t(const GemmParams &p, hipStream_t s) {
+  constexpr size_t lds = GemmStageLds<64 * TM, 128, 64>::BYTES;
+  auto kern = gemm_mfma_kernel<BF16, TM, 2, 64, SK>;
   static const hipError_t attr = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (attr != hipSuccess) return attr;
-  const int tiles_m = (int)((p.M + 127) / 128), tiles_n = (int)((p.N + 127) / 128);
+  const int tiles_m = (int)((p.M + 64 * TM - 1) / (64 * TM)), tiles_n = (int)((p.N + 127) / 128);
   hipLaunchKernelGGL(kern, dim3(tiles_m * tiles_n * (SK ? p.split : 1), std::max(1, p.batches)), dim3(256), lds, s, p, tiles_m, tiles_n);
   return hipGetLastError();
+}
+template <bool BF16, bool SK>
+hipError_t launch_gemm_any(const GemmParams &p, hipStream_t s) {
+  return any_rows(p, SK ? p.split : 1) == 64 ? launch_gemm_any_t<BF16, SK, 1>(p, s) : launch_gemm_any_t<BF16, SK, 2>(p, s);
 }
 hipError_t launch_gemm_any_slices(const GemmParams &p, hipStream_t s) { return p.is_bf16 ? launch_gemm_any<true, true>(p, s) : launch_gemm_any<false, true>(p, s); }
 
@@ -884,23 +908,20 @@ DmaChoice choose_dma(const GemmParams &p, int max_split) {
 
 namespace {
 // K slices of the any-shape kernel (1: none), at most max_split: where its tiles leave CUs without work, every workgroup
-// would walk all of K alone.  Modelled like choose_dma's: the K tiles of 64 a workgroup walks (two share a CU), the slices'
-// sums through memory and the second launch.  Measured in bf16 with 1 / 2 / 4 / 8 / 16 slices, us: 33 x 4001 x 4001 62 / 40 /
-// 28 / 23 / 23; 600 x 601 x 3001 56 / 40 / 30 / 27 / 33; 100 x 700 x 2000 32 / 22 / 21 / 21 / 21 (19 to 20 is what the calls of
-// that loop took on the host); 1000 x 3001 x 1003 31 / 40 / 48; 64 x 1003 x 517 18.6 / 20.5 / 20.2: the model takes 1 where two lose.
+// would walk all of K alone.  Modelled like choose_dma's: the K tiles of 64 a workgroup walks -- 0.58 us each on 64 x 128 tiles
+// with a CU to itself, 1.4 of that per workgroup beyond one, 1.19 us and 1.1 on 128 x 128 -- the slices' sums through memory and
+// the second launch.  Measured in us per call with 1 / 2 / 4 / 8 / 16 slices: 33 x 4001 x 4001 40 / 25 / 17.7 / 15.0 / 17.3;
+// 600 x 601 x 3001 33.8 / 24.3 / 18.9 / 20.8 / 30.8; 504 x 2000 x 3000 28.9 / 24.8 / 27 / 35 / 50; 100 x 700 x 2000 20.3 / 15.1 / 13.6 /
+// 14.3 / 13.7; 1501^3 27 / 36; 500 x 600 x 700 11.9 / 14.4; 64 x 1003 x 517 11.9 / 14.0: the model takes 1 where two lose.
 int any_split(const GemmParams &p, int max_split) {
   if (p.a_rows || p.b_block) return 1;
-  static const int cus = [] {
-    int dev = 0, n = 0;
-    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-    return n;
-  }();
-  const int64_t tiles = ((p.M + 127) / 128) * ((p.N + 127) / 128) * std::max(1, p.batches), nk = (p.K + 63) / 64;
+  const int64_t nk = (p.K + 63) / 64;
   const double sums = (double)p.M * (double)p.N * std::max(1, p.batches) * 4;
   auto model = [&](int split) {
-    const double wgs = (double)tiles * split;
-    double t = std::max(1.0, wgs / (1.5 * cus)) * (double)((nk + split - 1) / split) * 1.0e-6 + 5e-6;
-    if (split > 1) t += 2 * split * sums / 4e12 + 6e-6;
+    const int64_t rows = any_rows(p, split);
+    const double w = (double)(((p.M + rows - 1) / rows) * ((p.N + 127) / 128) * std::max(1, p.batches) * split) / device_cus();
+    double t = (w <= 1 ? 1.0 : (rows == 64 ? 1.4 : 1.1) * w) * (double)((nk + split - 1) / split) * (rows == 64 ? 0.58e-6 : 1.19e-6) + 5e-6;
+    if (split > 1) t += 2 * split * sums / 6e12 + 4.5e-6;
     return t;
   };
   static const char *split_env = getenv("TTS_GEMM_SPLIT");  // tuning aid (see choose_dma)
@@ -973,16 +994,17 @@ int gemm_epilogue_kernel_index(const GemmParams &p) { return gemm_fast_path_ok(p
 // A launch in K slices only where the any-shape kernel (kernel 1 below) would run it whole.
 int gemm_epilogue_split(const GemmParams &p) { return gemm_epilogue_kernel_index(p) == 1 ? any_split(p, 16) : 1; }
 
-// Kernel 0: whole 256 x 256 x 32 tiles; 1: any shape in 128 x 128 x 64 tiles; 2: the sum of the K slices that the any-shape
+// Kernel 0: whole 256 x 256 x 32 tiles; 1: any shape in 128 x 128 x 64 tiles; 3 (if `small_tiles` allows it): 64 x 128 x 64
+// tiles (any_rows); 2: the sum of the K slices that the any-shape
 // kernel without a functor leaves (p.split > 1) -- compiled from gemm_device.h plus the epilogue functor at the first launch
-// that needs it.  A launch in slices also compiles the kernel it would be without, so that a later one of the same plan that
+// that needs it.  A launch in slices or small tiles also compiles the kernel it would be without, so that a later one of the same plan that
 // may not use a workspace finds it.
-hipError_t launch_gemm_epilogue(const GemmParams &p, const std::string &epilogue, RtcModule **modules, const GemmEpilogueArgs &ep,
+hipError_t launch_gemm_epilogue(const GemmParams &p, const std::string &epilogue, RtcModule **modules, bool small_tiles, const GemmEpilogueArgs &ep,
                                 hipStream_t s, const char **name, std::string *err) {
   static const char *names[3] = {"gemm_dma_kernel + epilogue (hipRTC)", "gemm_mfma_kernel<128x128x64> + epilogue (hipRTC)",
                                  "gemm_mfma_kernel<128x128x64> + epilogue (hipRTC), K slices"};
-  const int whole = gemm_epilogue_kernel_index(p), which = p.split > 1 ? 2 : whole;
-  *name = names[which];
+  const int whole = gemm_epilogue_kernel_index(p), which = p.split > 1 ? 2 : small_tiles && whole == 1 && any_rows(p, 1) == 64 ? 3 : whole;
+  *name = names[which == 3 ? 1 : which];
   for (int m : {whole, which}) {
     if (modules[m]) continue;
     const std::string source = epilogue + "#define TTS_GEMM_RTC " + std::to_string(m) + "\n#define TTS_GEMM_BF16 " + std::to_string(p.is_bf16 ? 1 : 0) +
@@ -1008,8 +1030,8 @@ hipError_t launch_gemm_epilogue(const GemmParams &p, const std::string &epilogue
     a.tiles_n = g.col_blocks;
     return rtc_launch(modules[2], g.workgroups, 1, 1, 256, &a, sizeof a, s);
   }
-  const int64_t tile = which == 1 ? 128 : 256;
-  a.tiles_m = (int)((p.M + tile - 1) / tile);
+  const int64_t tile = which ? 128 : 256, rows = which == 3 ? 64 : tile;
+  a.tiles_m = (int)((p.M + rows - 1) / rows);
   a.tiles_n = (int)((p.N + tile - 1) / tile);
   return rtc_launch(modules[which], a.tiles_m * a.tiles_n, 1, 1, 256, &a, sizeof a, s);
 }

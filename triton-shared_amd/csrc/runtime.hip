@@ -148,7 +148,7 @@ struct tts_plan {
   }
   RtcModule *fused = nullptr;  // the kernel compiled for this plan at its first launch (fused maps, tile programs)
   bool fused_is_plain = false; // a tile program whose source is persistent but whose kernel with a workgroup per program was kept
-  RtcModule *gemm_rtc[3] = {nullptr, nullptr, nullptr};  // matrix products with a fused epilogue: launch_gemm_epilogue's kernels
+  RtcModule *gemm_rtc[4] = {nullptr, nullptr, nullptr, nullptr};  // matrix products with a fused epilogue: launch_gemm_epilogue's kernels
   RtcModule *fallback = nullptr;  // the generic family's kernel for a matrix-product plan (launches the product kernels decline)
   ~tts_plan() {
     for (auto &kv : split_k) {
@@ -989,7 +989,8 @@ tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, con
             if (e != hipSuccess) return fail(TTS_HIP_ERROR, std::string("hipMalloc(split-K workspace): ") + hipGetErrorString(e));
             p.partial = sk.workspace;
           }
-          err = launch_gemm_epilogue(p, pl.source, plan->gemm_rtc, a, s, &kname, &why);
+          // (a call that may not compile keeps to the kernel every launch of this shape has compiled)
+          err = launch_gemm_epilogue(p, pl.source, plan->gemm_rtc, !no_alloc || plan->gemm_rtc[3], a, s, &kname, &why);
         }
         if (err != hipSuccess && !why.empty()) return fail(TTS_HIP_ERROR, "gemm epilogue: " + why);
         break;
