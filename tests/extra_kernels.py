@@ -1635,3 +1635,16 @@ def mixed_rows_less_their_maximum(x_ptr, r_ptr, k_ptr, b_ptr, y_ptr, z_ptr, n_co
     v = v - tl.max(v, axis=0)
     tl.store(y_ptr + row * pitch + cols, v.to(y_ptr.dtype.element_ty), mask=live)
     tl.store(z_ptr + row * pitch + cols, v, mask=live)
+
+
+@triton.jit
+def take_rows_scaled(src_ptr, rows_ptr, s_ptr, add_ptr, dst_ptr, n_rows, n_cols, pitch, BR: tl.constexpr, BC: tl.constexpr):
+    """dst[r, c] = src[rows[r], c] * s[r] + add[r, c]; masked elements of the gathered block read as 3."""
+    r = tl.program_id(0) * BR + tl.arange(0, BR)
+    c = tl.program_id(1) * BC + tl.arange(0, BC)
+    which = tl.load(rows_ptr + r, mask=r < n_rows, other=0)
+    s = tl.load(s_ptr + r, mask=r < n_rows, other=0.0)
+    m = (r[:, None] < n_rows) & (c[None, :] < n_cols)
+    x = tl.load(src_ptr + which[:, None] * pitch + c[None, :], mask=m, other=3.0).to(tl.float32)
+    a = tl.load(add_ptr + r[:, None] * pitch + c[None, :], mask=m, other=0.0)
+    tl.store(dst_ptr + r[:, None] * pitch + c[None, :], (x * s[:, None] + a).to(dst_ptr.dtype.element_ty), mask=m)

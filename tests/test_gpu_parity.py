@@ -2472,6 +2472,38 @@ def test_tile_program_wide_groups_that_the_extent_cuts_off(dtype, n_cols):
     assert (z[:, n_cols:] == 55).all() and (y[:, n_cols:] == 55).all()
 
 
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("n_rows,n_cols,pitch,BR,BC", [(1, 1, 1, 8, 256), (9, 255, 255, 8, 256), (37, 511, 513, 16, 512), (100, 1000, 1000, 4, 1024), (33, 1017, 1021, 2, 1024),
+                                                       (10, 2047, 2047, 1, 2048), (21, 4096, 4096, 4, 4096), (21, 4001, 4003, 4, 4096), (7, 7296, 7296, 4, 8192), (18, 8185, 8187, 16, 8192)])
+def test_rows_gathered_eight_elements_at_a_time(dtype, n_rows, n_cols, pitch, BR, BC):
+    """16-bit rows taken through an index vector: blocks of one piece and of several, rows that start anywhere and end inside a
+    group of eight; copied bit by bit, and scaled beside a block that is not gathered (each result rounds once to 16 bits)."""
+    import extra_kernels as X
+    torch.manual_seed(n_cols)
+    dt = getattr(torch, dtype)
+    src = torch.full((3 + 50 * pitch,), 9.0, device=DEV, dtype=dt)[3:].view(50, pitch)
+    src[:, :n_cols] = torch.randn(50, n_cols, device=DEV)
+    which = torch.randint(0, 50, (n_rows,), device=DEV, dtype=torch.int32)
+    dst = torch.full((1 + n_rows * pitch + 9,), 5.0, device=DEV, dtype=dt)[1:]
+    out = dst[:n_rows * pitch].view(n_rows, pitch)
+    k = K_mod().take_rows[(triton.cdiv(n_rows, BR),)](src, which, out, n_rows, n_cols, pitch, pitch, BR=BR, BC=BC)
+    torch.cuda.synchronize()
+    assert k.function.family == "tile_program"
+    want = src[which.long(), :n_cols]
+    assert torch.equal(out[:, :n_cols], want) and (out[:, n_cols:] == 5.0).all() and (dst[n_rows * pitch:] == 5.0).all()
+    s = torch.randn(n_rows, device=DEV)
+    add = torch.randn(n_rows, pitch, device=DEV)
+    if BC <= 2048:
+        out.fill_(5.0)
+        X.take_rows_scaled[(triton.cdiv(n_rows, BR), triton.cdiv(n_cols, BC))](src, which, s, add, out, n_rows, n_cols, pitch, BR=BR, BC=BC)
+        torch.cuda.synchronize()
+        exact = want.double() * s.double()[:, None] + add[:, :n_cols].double()
+        ulp = 2.0 ** -11 if dt == torch.float16 else 2.0 ** -8
+        size = (want.double() * s.double()[:, None]).abs() + add[:, :n_cols].double().abs()
+        assert ((out[:, :n_cols].double() - exact).abs() <= ulp * exact.abs() + 2.0 ** -22 * size + 2.0 ** -24).all()
+        assert (out[:, n_cols:] == 5.0).all()
+
+
 @pytest.mark.parametrize("n_cols,pitch,lead", [(4096, 4096, 0), (4000, 4000, 0), (4093, 4099, 0), (2048, 2048, 5)])
 def test_tile_program_wide_rows_with_int8_neighbours(n_cols, pitch, lead):
     """Row-wise int8 quantisation and its inverse: 1-byte blocks next to 16-bit ones take the wide element order too

@@ -30,6 +30,7 @@
 // whose address waits for another load's result, or a select between a loaded value and `other` right
 // after the load, serialises the whole run (see the notes at the two places).
 #include <algorithm>
+#include <cmath>
 #include <cstdlib>
 #include <cstring>
 #include <functional>
@@ -694,9 +695,82 @@ struct Gen {
     int64_t st = 0;
     return P.pool.is_const(a.strides.back(), &st) && st == 1;
   }
+  // Rows gathered through an index vector: a load of 16-bit elements whose offsets are data but go up by one along the last
+  // dimension (rows[:, None] * pitch + cols[None, :]).  A group of eight whose elements are all valid and whose last address
+  // is seven past its first moves in one access like any other wide group.
+  enum Along { UNIFORM, UNIT, OTHER };  // how a value changes along its last dimension
+  Along along_last(int v, int depth = 0) const {
+    const Value &V = val(v);
+    if (V.shape.empty() || V.shape.back() == 1) return UNIFORM;
+    auto d = def.find(v);
+    if (d == def.end() || depth > 32) return OTHER;
+    const SOp &o = *d->second;
+    switch (o.kind) {
+      case SK::Const: case SK::Splat: case SK::FromIndex: case SK::ScalarArg: return UNIFORM;
+      case SK::Iota: return UNIT;
+      case SK::ExpandDims: return along_last(o.operands.at(0), depth + 1);  // (an added last dimension has size 1)
+      case SK::Broadcast: return along_last(o.operands.at(0), depth + 1);
+      case SK::Map: {
+        bool uniform = true;
+        for (int x : o.operands) uniform = uniform && val(x).shape.size() <= V.shape.size() && along_last(x, depth + 1) == UNIFORM;
+        if (o.name.rfind("tt.", 0) == 0) return OTHER;  // (transposes, reshapes and the like)
+        if (uniform) return UNIFORM;
+        if (o.name == "arith.extsi") return along_last(o.operands.at(0), depth + 1);
+        if (o.name == "arith.addi" || o.name == "arith.subi") {
+          const Along a = along_last(o.operands.at(0), depth + 1), b = along_last(o.operands.at(1), depth + 1);
+          if (a == UNIT && b == UNIFORM) return UNIT;
+          if (a == UNIFORM && b == UNIT && o.name == "arith.addi") return UNIT;
+        }
+        return OTHER;
+      }
+      default: return OTHER;
+    }
+  }
+  bool gathers_rows = false;  // a program of one run of loads, elementwise ops and stores with such loads, all of one shape
+  bool row_gather(const Access &a) const { return gathers_rows && a.gather >= 0 && is16(a.elem) && a.sizes == wide_shape && along_last(a.gather) == UNIT; }
+  // Such a run goes through its block in pieces of 8192 elements (`piece` in the generated source): nothing needs the whole
+  // of it at once, and the loads of a piece are enough in flight.  (Rows of fp16 [4000, 4096], four per program, element by
+  // element: 20.1 us, this way 12.4; rows of 7296, whose blocks of 32768 went one element at a time: 35.2 us for 275 of them, now 8.2.)
+  static constexpr int64_t PIECE = 8192, GATHER_MAX = 1 << 20;
+  bool in_pieces(const std::vector<int64_t> &shape) const { return gathers_rows && wide(shape) && count(shape) > PIECE; }
+  int64_t held_count(const std::vector<int64_t> &shape) const { return in_pieces(shape) ? PIECE : count(shape); }
+  void choose_row_gathers() {
+    std::vector<int64_t> sh;
+    std::set<int> loaded, written;
+    std::map<int, const SOp *> saved = def;
+    for (const SOp &s : P.body)
+      if (s.result >= 0) def[s.result] = &s;
+    bool ok = true, any = false;
+    for (const SOp &s : P.body) {
+      if (s.kind == SK::Load || s.kind == SK::Store) {
+        (s.kind == SK::Load ? loaded : written).insert(s.acc.base_arg);
+        if (s.kind == SK::Load && s.acc.sizes.size() == 1) continue;  // an index vector
+        if (s.acc.sizes.size() != 2 || (!sh.empty() && s.acc.sizes != sh)) ok = false;
+        sh = s.acc.sizes;
+        const bool rows = s.acc.gather >= 0 && s.kind == SK::Load && is16(s.acc.elem) && along_last(s.acc.gather) == UNIT;
+        any = any || rows;
+        ok = ok && (rows || vector_access(s.acc));
+      } else if (s.kind == SK::Map) {
+        ok = ok && s.name.rfind("tt.", 0) != 0;
+      } else if (s.kind != SK::Const && s.kind != SK::Splat && s.kind != SK::Iota && s.kind != SK::FromIndex && s.kind != SK::ScalarArg && s.kind != SK::ExpandDims && s.kind != SK::Broadcast) {
+        ok = false;
+      }
+    }
+    for (int b : written) ok = ok && !loaded.count(b);
+    if (ok && any) {
+      const int64_t C = sh[1], T = count(sh);
+      ok = C >= 256 && PIECE % C == 0 && T % 2048 == 0 && T <= GATHER_MAX && (T <= PIECE || T % PIECE == 0);
+    }
+    def = saved;
+    if (!ok || !any) return;
+    gathers_rows = wide_mode = true;
+    wide_shape = sh;
+  }
   void choose_wide_shape() {
     if (const char *e = getenv("TTS_TILE_WIDE"))
       if (e[0] == '0') return;
+    choose_row_gathers();
+    if (gathers_rows) return;
     bool refuse = false;
     std::vector<int64_t> best;
     std::function<void(const std::vector<SOp> &)> scan = [&](const std::vector<SOp> &ops) {
@@ -737,7 +811,7 @@ struct Gen {
   std::ostringstream hoist_os;
   std::ostringstream loop_top;  // first statements of the program loop
   void choose_persistent() {
-    if (!wide_mode) return;
+    if (!wide_mode || gathers_rows) return;
     if (const char *e = getenv("TTS_TILE_PERSISTENT"))
       if (e[0] == '0') return;
     std::set<int> stored;
@@ -944,7 +1018,7 @@ struct Gen {
     return total;
   }
   std::string element_of_slot(const std::vector<int64_t> &shape) const {
-    return wide(shape) ? "8 * (int)threadIdx.x + (n & 7) + 2048 * (n >> 3)" : "threadIdx.x + 256 * n";
+    return wide(shape) ? std::string("8 * (int)threadIdx.x + (n & 7) + 2048 * (n >> 3)") + (in_pieces(shape) ? " + " + std::to_string(PIECE) + " * piece" : "") : "threadIdx.x + 256 * n";
   }
   // Row and column of element t of a block.  Every loop that names t names n as well (element_of_slot); with rows of a
   // multiple of 256 elements the row depends on n alone, which is a constant once the loop is unrolled (or the same in
@@ -953,7 +1027,9 @@ struct Gen {
   std::string idx0(const std::vector<int64_t> &shape) const {
     if (shape.size() < 2) return "t";
     const int64_t C = shape.back();
-    if (wide(shape) && C % 2048) return "((int)threadIdx.x / " + std::to_string(C / 8) + " + " + std::to_string(2048 / C) + " * (n >> 3))";
+    const std::string rows_before = in_pieces(shape) ? " + " + std::to_string(PIECE / C) + " * piece" : "";
+    if (wide(shape) && C % 2048) return "((int)threadIdx.x / " + std::to_string(C / 8) + " + " + std::to_string(2048 / C) + " * (n >> 3)" + rows_before + ")";
+    if (!rows_before.empty()) return "(n / " + std::to_string(C / 256) + rows_before + ")";
     if (C % 256 == 0) return C == 256 ? "n" : "(n / " + std::to_string(C / 256) + ")";
     return "(t / " + std::to_string(C) + ")";
   }
@@ -967,7 +1043,7 @@ struct Gen {
   }
   std::string cur_i0, cur_i1;  // the index expressions of the element loop being written
   void open_element_loop(const std::vector<int64_t> &shape) {
-    const int64_t T = count(shape);
+    const int64_t T = held_count(shape);
     cur_i0 = idx0(shape);
     cur_i1 = idx1(shape);
     os << pad() << "#pragma unroll\n" << pad() << "for (int n = 0; n < " << (T + 255) / 256 << "; n++) {\n";
@@ -1158,7 +1234,7 @@ struct Gen {
           if (ops[q].kind == SK::Load) load_bases.insert(ops[q].acc.base_arg);
         for (size_t q = k; q < end; q++) hazard = hazard || (ops[q].kind == SK::Store && load_bases.count(ops[q].acc.base_arg));
       }
-      const bool two_phase_run = count(shape) <= (hazard ? HAZARD_MAX : TWO_PHASE_MAX);
+      const bool two_phase_run = count(shape) <= (hazard ? HAZARD_MAX : gathers_rows && wide(shape) ? GATHER_MAX : TWO_PHASE_MAX);
       auto big_other = [&](const SOp &o) {
         return two_phase_run && o.kind == SK::Load && o.acc.sizes != shape && count(o.acc.sizes) >= 2048 && count(o.acc.sizes) <= TWO_PHASE_MAX;
       };
@@ -1247,6 +1323,11 @@ struct Gen {
         }
         os << pad() << "__syncthreads();\n";
       }
+      const bool pieces = stores && in_pieces(shape);
+      if (pieces) {
+        os << pad() << "#pragma unroll 1\n" << pad() << "for (int piece = 0; piece < " << T / PIECE << "; piece++) {\n";
+        indent++;
+      }
       if (two_phase) {
         // Registers for the run's own loads, and for large blocks of another shape (a [K, N] operand next to an [M, K]
         // one): those are held by the threads that own their elements and can be named in loops over their own shape.
@@ -1272,8 +1353,8 @@ struct Gen {
                 }
                 else hoist_os << "  " << ctype(val(ops[q].result).dtype) << " ld" << ops[q].result << "[" << (count(ls) + 255) / 256 << "];\n";
               }
-              else  // (inside a program loop a slot that a masked load leaves unwritten would otherwise hold, and carry, the last program's)
-                os << pad() << ctype(val(ops[q].result).dtype) << " ld" << ops[q].result << "[" << (count(ls) + 255) / 256 << "]" << (persistent ? " = {}" : "") << ";\n";
+              else if (!row_gather(ops[q].acc))  // (inside a program loop a slot that a masked load leaves unwritten would otherwise hold, and carry, the last program's)
+                os << pad() << ctype(val(ops[q].result).dtype) << " ld" << ops[q].result << "[" << (held_count(ls) + 255) / 256 << "]" << (persistent ? " = {}" : "") << ";\n";
               any = true;
             }
           if (!any) continue;
@@ -1320,7 +1401,7 @@ struct Gen {
             bool any_wide = false;
             for (size_t q = k; q < end; q++) any_wide = any_wide || wide_load(ops[q]);
             if (any_wide) {
-              const int64_t G = count(ls) / 2048;
+              const int64_t G = held_count(ls) / 2048;
               uses_dummy = true;
               std::string roomy;  // the extents of the masked ones leave eight elements to read, or none (the same in every thread)
               for (size_t q = k; q < end; q++)
@@ -1473,7 +1554,50 @@ struct Gen {
               indent = saved_indent;
             }
           }
-          auto wide_load = wide_load_any;
+          for (size_t q = k; q < end; q++)
+            if (mine_here(ops[q]) && row_gather(ops[q].acc)) {
+              const SOp &o = ops[q];
+              const std::string id = std::to_string(o.result), G = std::to_string(held_count(ls) / 2048);
+              const std::string base = "(const unsigned short *)p.ptr[" + std::to_string(o.acc.base_arg) + "]";
+              uses_dummy = true;
+              map_vars({-1});
+              cur_i0.clear();
+              cur_i1.clear();
+              std::string pred, all, first = address(o.acc, l0, l1, pred), unused;
+              for (int e = 0; e < 8 && !pred.empty(); e++) {
+                std::string one;
+                address(o.acc, l0, "(" + l1 + " + " + std::to_string(e) + ")", one);
+                all += "(" + one + ") && ";
+              }
+              const std::string last = address(o.acc, l0, "(" + l1 + " + 7)", unused), at_e = address(o.acc, l0, "(" + l1 + " + e)", unused);
+              std::string pred_e;
+              address(o.acc, l0, "(" + l1 + " + e)", pred_e);
+              os << pad() << "u32x4_t rw" << id << "[" << G << "];\n" << pad() << "unsigned whole" << id << " = 0;\n"
+                 << pad() << "#pragma unroll\n" << pad() << "for (int g = 0; g < " << G << "; g++) {\n";
+              indent++;
+              os << pad() << "const int n = 8 * g, t = " << element_of_slot(ls) << ";\n" << pad() << "(void)t;\n"
+                 << pad() << "const long long first = " << first << ";\n"
+                 << pad() << "const bool whole = " << all << "(" << last << ") - first == 7;\n"
+                 << pad() << "rw" << id << "[g] = *(whole ? (const u32x4_any *)(" << base << " + first) : (const u32x4_any *)tts_dummy);\n"
+                 << pad() << "whole" << id << " |= (unsigned)whole << g;\n";
+              indent--;
+              os << pad() << "}\n" << pad() << "#pragma unroll\n" << pad() << "for (int g = 0; g < " << G << "; g++) {\n";
+              indent++;
+              os << pad() << "if (whole" << id << " >> g & 1) continue;\n"
+                 << pad() << "const int n = 8 * g, t = " << element_of_slot(ls) << ";\n" << pad() << "(void)t;\n"
+                 << pad() << "unsigned one[8] = {};\n" << pad() << "#pragma unroll\n" << pad() << "for (int e = 0; e < 8; e++)\n"
+                 << pad() << "  " << (pred_e.empty() ? "" : "if (" + pred_e + ") ") << "one[e] = (" << base << ")[" << at_e << "];\n"
+                 << pad() << "rw" << id << "[g] = u32x4_t{one[0] | one[1] << 16, one[2] | one[3] << 16, one[4] | one[5] << 16, one[6] | one[7] << 16};\n";
+              indent--;
+              os << pad() << "}\n";
+              const std::string word = "rw" + id + "[n >> 3][(n & 7) >> 1]";
+              const std::string got = std::string(o.acc.elem == "f16" ? "up_f16(" : "up_bf16(") + "(unsigned short)((n & 1) ? " + word + " >> 16 : " + word + "))";
+              const bool zero = pred.empty() || (o.acc.other_value < 0 && (!o.acc.has_other || (o.acc.other_f == 0.0 && !std::signbit(o.acc.other_f))));
+              held[o.result] = {"rw" + id, ls, "(" + (zero ? got : "(" + pred + ") ? " + got + " : " + other_of(o.acc, l0, l1)) + ")"};
+              mine.push_back(o.result);
+              any_load = true;
+            }
+          auto wide_load = [&](const SOp &o) { return wide_load_any(o) || row_gather(o.acc); };
           bool any_classic = false;
           for (size_t q = k; q < end; q++) any_classic = any_classic || (mine_here(ops[q]) && !wide_load(ops[q]));
           if (!any_classic) continue;
@@ -1517,7 +1641,7 @@ struct Gen {
           row_vectors[o->result] = name;
         }
         row_loads.clear();
-        if (any_load && !(column_sums && loop_depth)) os << pad() << "__syncthreads();\n";
+        if (any_load && !(column_sums && loop_depth) && !gathers_rows) os << pad() << "__syncthreads();\n";
         if (stores && wide(shape))  // wide stores collect a group's eight values (see the Store case below)
           for (size_t q = k; q < end; q++)
             if (ops[q].kind == SK::Store && vector_access(ops[q].acc)) os << pad() << "unsigned sv" << q << "[8];\n";
@@ -1598,8 +1722,9 @@ struct Gen {
           }
         }
         close_loop();
-        os << pad() << "__syncthreads();\n";
+        if (!gathers_rows) os << pad() << "__syncthreads();\n";
       }
+      if (pieces) close_loop();
       // values named inside the loop end with it (a load of a two-phase run stays in its registers)
       for (size_t q = k; q < end; q++)
         if (ops[q].result >= 0 && (ops[q].kind == SK::Map || (ops[q].kind == SK::Load && !held.count(ops[q].result)))) var.erase(ops[q].result);
