@@ -2,7 +2,7 @@
 // time into the library (kernels_gemm.hip, results stored as they are), and at run time with hipRTC when the Triton
 // kernel applies elementwise ops to the accumulator before the store (a fused activation): the generated source
 // defines TTS_GEMM_RTC (which kernel: 0 whole 256 x 256 x 32 tiles, 1 any shape in 128 x 128 x 64 tiles, 2 the sum of the K
-// slices, 3 as 1 in 64 x 128 x 64 tiles), TTS_GEMM_BF16 and the functor TtsEp (a plain struct, passed as the kernel's last argument) that maps an accumulator value and its position to the value stored, then this file's text.  Nothing here may need a host header.
+// slices, 3 as 1 in 64 x 128 x 64 tiles, 4 and up the other direct-to-LDS tiles), TTS_GEMM_BF16 and the functor TtsEp (a plain struct, passed as the kernel's last argument) that maps an accumulator value and its position to the value stored, then this file's text.  Nothing here may need a host header.
 #pragma once
 #ifdef __HIPCC_RTC__
 typedef __INT64_TYPE__ int64_t;
@@ -1158,6 +1158,9 @@ extern "C" __global__ __launch_bounds__(256) void gemm_rtc(TtsGemmParams p, int 
   tts_gemm_device::gemm_dma16_body<TTS_GEMM_BF16 != 0>(p, tiles_m, tiles_n, ep);
 #elif TTS_GEMM_RTC == 2
   tts_gemm_device::gemm_splitk_reduce_body<TTS_GEMM_BF16 != 0>(p, tiles_m, tiles_n, ep);  // (across, col_blocks)
+#elif TTS_GEMM_RTC >= 4
+  constexpr int TM = TTS_GEMM_RTC == 5 ? 4 : 2, TN = TTS_GEMM_RTC == 4 ? 4 : 2;  // 128 x 256, 256 x 128, 128 x 128
+  tts_gemm_device::gemm_dma_body<TTS_GEMM_BF16 != 0, TM, TN>(p, tiles_m, tiles_n, ep);
 #else
   tts_gemm_device::gemm_mfma_body<TTS_GEMM_BF16 != 0, TTS_GEMM_RTC == 3 ? 1 : 2, 2, 64>(p, tiles_m, tiles_n, ep);
 #endif

@@ -99,8 +99,9 @@ int gemm_split(const GemmParams &p);
 size_t gemm_workspace_bytes(const GemmParams &p);
 hipError_t launch_gemm(const GemmParams &p, hipStream_t s, const char **kernel_name);
 // The same product with elementwise ops fused into the epilogue: `epilogue` is the source of the functor (match.h:
-// gemm_epilogue_source), `modules` the plan's four slots for the kernels compiled from it (one per tiling, the sum of K slices, the smaller tiles
-// if `small_tiles` allows them; filled at the first launch that needs it), `args` / `args_size` the generic families' argument block.
+// gemm_epilogue_source), `modules` the plan's slots for the kernels compiled from it (one per tiling and the sum of K slices,
+// filled at the first launch that needs it and may compile), `args` / `args_size` the generic families' argument block.
+constexpr int GEMM_EPILOGUE_KERNELS = 7;
 struct RtcModule;
 // The epilogue functor as the kernel receives it (the generated `struct TtsEp` has this layout): every kernel argument
 // by index, then what it takes to find the Triton program that owns an element -- tile_pid[(row / BM) * tiles_n +
@@ -114,8 +115,8 @@ struct GemmEpilogueArgs {
 };
 int gemm_epilogue_split(const GemmParams &p);  // K slices (1: none), as gemm_split(p) for a product with a functor
 bool gemm_any_shape(const GemmParams &p);      // the any-shape kernel runs this product
-int gemm_epilogue_kernel_index(const GemmParams &p);  // which of `modules` a launch of this shape uses
-hipError_t launch_gemm_epilogue(const GemmParams &p, const std::string &epilogue, RtcModule **modules, bool small_tiles, const GemmEpilogueArgs &ep,
+bool gemm_epilogue_compiled(const GemmParams &p, RtcModule *const *modules);  // a whole launch of this shape finds its kernel there
+hipError_t launch_gemm_epilogue(const GemmParams &p, const std::string &epilogue, RtcModule **modules, bool may_compile, const GemmEpilogueArgs &ep,
                                 hipStream_t s, const char **kernel_name, std::string *err);
 
 // C[M,N] = A[M,K] * (f16(W[K,N]) * scale[N]), A/scale/C fp16, W int8, fp32 accumulate, M <= 16

@@ -114,18 +114,26 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(GemmParams batc
   reinterpret_cast<uint32_t *>(dst)[1] = w.y;
 }
 
+// p.split K slices of a product; whoever launches them adds them
+template <bool BF16, int TM, int TN, bool BT, bool AT>
+hipError_t launch_gemm_dma_slices(const GemmParams &p, hipStream_t s) {
+  using T = DmaTile<TM, TN>;
+  constexpr size_t lds = T::LDS_BYTES;
+  auto kern = gemm_dma_kernel<BF16, TM, TN, BT, AT, false, true>;
+  static const hipError_t attr = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  if (attr != hipSuccess) return attr;
+  int tiles_m = (int)((p.M + T::BM - 1) / T::BM), tiles_n = (int)((p.N + T::BN - 1) / T::BN);
+  hipLaunchKernelGGL(kern, dim3(tiles_m * tiles_n * p.split, std::max(1, p.batches)), dim3(256), lds, s, p, tiles_m, tiles_n);
+  return hipGetLastError();
+}
+
 template <bool BF16, int TM, int TN, bool BT, bool AT, bool PF = false>
 hipError_t launch_gemm_dma_t(const GemmParams &p, hipStream_t s) {
   using T = DmaTile<TM, TN>;
   constexpr size_t lds = T::LDS_BYTES;
   if constexpr (!PF) {
     if (p.split > 1) {
-      auto kern = gemm_dma_kernel<BF16, TM, TN, BT, AT, false, true>;
-      static const hipError_t attr = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-      if (attr != hipSuccess) return attr;
-      int tiles_m = (int)((p.M + T::BM - 1) / T::BM), tiles_n = (int)((p.N + T::BN - 1) / T::BN);
-      hipLaunchKernelGGL(kern, dim3(tiles_m * tiles_n * p.split, std::max(1, p.batches)), dim3(256), lds, s, p, tiles_m, tiles_n);
-      hipError_t e = hipGetLastError();
+      hipError_t e = launch_gemm_dma_slices<BF16, TM, TN, BT, AT>(p, s);
       if (e != hipSuccess) return e;
       hipLaunchKernelGGL(gemm_splitk_reduce_kernel<BF16>, dim3((unsigned)((p.M * (p.N / 4) + 255) / 256), std::max(1, p.batches)), dim3(256), 0, s, p);
       return hipGetLastError();
@@ -989,22 +997,52 @@ hipError_t launch_gemm(const GemmParams &p, hipStream_t s, const char **name) {
   return hipGetLastError();
 }
 
-int gemm_epilogue_kernel_index(const GemmParams &p) { return gemm_fast_path_ok(p) ? 0 : 1; }
+namespace {
+// The kernels compiled with a functor: 0 whole 256 x 256 x 32 tiles on the 16 x 16 x 32 instruction; 1 any shape in 128 x 128 x 64
+// tiles; 2 the sum of K slices; 3 any shape in 64 x 128 x 64 tiles; 4 ... the other direct-to-LDS tiles, in the order of DMA_CANDS.
+int epilogue_dma_index(const DmaCand *tile) { return tile == &DMA_CANDS[0] ? 0 : 3 + (int)(tile - DMA_CANDS); }
 
-// A launch in K slices only where the any-shape kernel (kernel 1 below) would run it whole.
-int gemm_epilogue_split(const GemmParams &p) { return gemm_epilogue_kernel_index(p) == 1 ? any_split(p, 16) : 1; }
+template <int TM, int TN>
+hipError_t launch_dma_slices(const GemmParams &p, hipStream_t s) {
+  return p.is_bf16 ? launch_gemm_dma_slices<true, TM, TN, false, false>(p, s) : launch_gemm_dma_slices<false, TM, TN, false, false>(p, s);
+}
 
-// Kernel 0: whole 256 x 256 x 32 tiles; 1: any shape in 128 x 128 x 64 tiles; 3 (if `small_tiles` allows it): 64 x 128 x 64
-// tiles (any_rows); 2: the sum of the K slices that the any-shape
-// kernel without a functor leaves (p.split > 1) -- compiled from gemm_device.h plus the epilogue functor at the first launch
-// that needs it.  A launch in slices or small tiles also compiles the kernel it would be without, so that a later one of the same plan that
-// may not use a workspace finds it.
-hipError_t launch_gemm_epilogue(const GemmParams &p, const std::string &epilogue, RtcModule **modules, bool small_tiles, const GemmEpilogueArgs &ep,
+// What a product with a functor runs on, in at most max_split K slices.  Row-major operands of whole K tiles take the
+// direct-to-LDS tile and the slices that the plain product takes (choose_dma): one 256 x 256 tile for each size, as these
+// launches once had, leaves most of the chip idle where there are few.
+struct EpilogueChoice { int whole, split; const DmaCand *tile; };  // the kernel without slices; the tile the slices run on (null: any shape)
+EpilogueChoice choose_epilogue(const GemmParams &p, int max_split) {
+  if (!gemm_fast_path_ok(p)) return {any_rows(p, 1) == 64 ? 3 : 1, any_split(p, max_split), nullptr};
+  const DmaChoice choice = choose_dma(p, max_split);
+  if (!choice.tile) return {0, 1, &DMA_CANDS[0]};  // (only where a tuning variable names a tile that does not apply)
+  return {epilogue_dma_index(choice.split > 1 ? choose_dma(p, 1).tile : choice.tile), choice.split, choice.tile};
+}
+// A kernel that is compiled already and computes what `whole` does: any direct-to-LDS tile for another of them, the any-shape
+// kernel's 128 rows for its 64 (-1: none).
+int compiled_epilogue(int whole, RtcModule *const *modules) {
+  if (modules[whole]) return whole;
+  if (whole == 1 || whole == 3) return modules[4 - whole] ? 4 - whole : -1;
+  for (int m : {0, 4, 5, 6})
+    if (modules[m]) return m;
+  return -1;
+}
+}  // namespace
+
+bool gemm_epilogue_compiled(const GemmParams &p, RtcModule *const *modules) { return compiled_epilogue(choose_epilogue(p, 1).whole, modules) >= 0; }
+int gemm_epilogue_split(const GemmParams &p) { return choose_epilogue(p, 16).split; }
+
+// Kernels are compiled from gemm_device.h plus the epilogue functor at the first launch that needs them.  A launch in slices
+// (p.split > 1) also compiles the kernel it would be without, so that a later one of the same plan that may not use a workspace
+// finds it; one that may not compile takes the kernel that is there.
+hipError_t launch_gemm_epilogue(const GemmParams &p, const std::string &epilogue, RtcModule **modules, bool may_compile, const GemmEpilogueArgs &ep,
                                 hipStream_t s, const char **name, std::string *err) {
-  static const char *names[3] = {"gemm_dma_kernel + epilogue (hipRTC)", "gemm_mfma_kernel<128x128x64> + epilogue (hipRTC)",
-                                 "gemm_mfma_kernel<128x128x64> + epilogue (hipRTC), K slices"};
-  const int whole = gemm_epilogue_kernel_index(p), which = p.split > 1 ? 2 : small_tiles && whole == 1 && any_rows(p, 1) == 64 ? 3 : whole;
-  *name = names[which == 3 ? 1 : which];
+  const EpilogueChoice choice = choose_epilogue(p, std::max(1, p.split));
+  const bool sliced = choice.split > 1;
+  const int whole = may_compile ? choice.whole : compiled_epilogue(choice.whole, modules), which = sliced ? 2 : whole;
+  if (which < 0) return hipErrorInvalidValue;  // (gemm_epilogue_compiled said so)
+  const bool any_shape = sliced ? !choice.tile : which == 1 || which == 3;
+  *name = any_shape ? (sliced ? "gemm_mfma_kernel<128x128x64> + epilogue (hipRTC), K slices" : "gemm_mfma_kernel<128x128x64> + epilogue (hipRTC)")
+                    : (sliced ? "gemm_dma_kernel + epilogue (hipRTC), K slices" : "gemm_dma_kernel + epilogue (hipRTC)");
   for (int m : {whole, which}) {
     if (modules[m]) continue;
     const std::string source = epilogue + "#define TTS_GEMM_RTC " + std::to_string(m) + "\n#define TTS_GEMM_BF16 " + std::to_string(p.is_bf16 ? 1 : 0) +
@@ -1021,18 +1059,21 @@ hipError_t launch_gemm_epilogue(const GemmParams &p, const std::string &epilogue
     GemmEpilogueArgs ep;   // the functor: same layout as the generated struct TtsEp
   } a;
   a.p = p;
+  a.p.split = choice.split;
   a.ep = ep;
-  if (which == 2) {
-    hipError_t e = launch_gemm_any_slices(p, s);
+  if (sliced) {
+    const int t = choice.tile ? epilogue_dma_index(choice.tile) : 1;
+    hipError_t e = t == 0 ? launch_dma_slices<4, 4>(a.p, s) : t == 4 ? launch_dma_slices<2, 4>(a.p, s) : t == 5 ? launch_dma_slices<4, 2>(a.p, s)
+                 : t == 6 ? launch_dma_slices<2, 2>(a.p, s) : launch_gemm_any_slices(a.p, s);
     if (e != hipSuccess) return e;
     const ReduceGrid g(p);
     a.tiles_m = g.across;
     a.tiles_n = g.col_blocks;
     return rtc_launch(modules[2], g.workgroups, 1, 1, 256, &a, sizeof a, s);
   }
-  const int64_t tile = which ? 128 : 256, rows = which == 3 ? 64 : tile;
+  const int64_t rows = which == 3 ? 64 : which == 0 || which == 5 ? 256 : 128, cols = which == 0 || which == 4 ? 256 : 128;
   a.tiles_m = (int)((p.M + rows - 1) / rows);
-  a.tiles_n = (int)((p.N + tile - 1) / tile);
+  a.tiles_n = (int)((p.N + cols - 1) / cols);
   return rtc_launch(modules[which], a.tiles_m * a.tiles_n, 1, 1, 256, &a, sizeof a, s);
 }
 

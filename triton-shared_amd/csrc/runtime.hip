@@ -148,7 +148,7 @@ struct tts_plan {
   }
   RtcModule *fused = nullptr;  // the kernel compiled for this plan at its first launch (fused maps, tile programs)
   bool fused_is_plain = false; // a tile program whose source is persistent but whose kernel with a workgroup per program was kept
-  RtcModule *gemm_rtc[4] = {nullptr, nullptr, nullptr, nullptr};  // matrix products with a fused epilogue: launch_gemm_epilogue's kernels
+  RtcModule *gemm_rtc[GEMM_EPILOGUE_KERNELS] = {};  // matrix products with a fused epilogue: launch_gemm_epilogue's kernels
   RtcModule *fallback = nullptr;  // the generic family's kernel for a matrix-product plan (launches the product kernels decline)
   ~tts_plan() {
     for (auto &kv : split_k) {
@@ -974,10 +974,8 @@ tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, con
         a.gz = gz;
         std::string why;
         if (no_alloc) {
-          const GemmParams &gp = p;
-          const int which = gemm_epilogue_kernel_index(gp);
           std::lock_guard<std::mutex> lock(plan->mu);
-          if (!plan->gemm_rtc[which]) may_allocate("to compile the matrix product with its fused epilogue");
+          if (!gemm_epilogue_compiled(p, plan->gemm_rtc)) may_allocate("to compile the matrix product with its fused epilogue");
         }
         {
           std::lock_guard<std::mutex> lock(plan->mu);
@@ -989,8 +987,7 @@ tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, con
             if (e != hipSuccess) return fail(TTS_HIP_ERROR, std::string("hipMalloc(split-K workspace): ") + hipGetErrorString(e));
             p.partial = sk.workspace;
           }
-          // (a call that may not compile keeps to the kernel every launch of this shape has compiled)
-          err = launch_gemm_epilogue(p, pl.source, plan->gemm_rtc, !no_alloc || plan->gemm_rtc[3], a, s, &kname, &why);
+          err = launch_gemm_epilogue(p, pl.source, plan->gemm_rtc, !no_alloc, a, s, &kname, &why);
         }
         if (err != hipSuccess && !why.empty()) return fail(TTS_HIP_ERROR, "gemm epilogue: " + why);
         break;
