@@ -2783,6 +2783,43 @@ def test_gemm_with_fused_epilogue(M, N, K, kernel, dtype):
     assert ((c.double() - want).norm() / want.norm()) <= 1e-2
 
 
+@pytest.mark.parametrize("M,N,Kd,sliced", [(2, 8, 4096, True), (100, 264, 4096, True), (300, 2056, 2048, True), (500, 4096, 4096, True), (130, 264, 96, False),
+                                           (4090, 2056, 64, False), (4000, 2040, 512, False), (3500, 4096, 512, False), (2041, 2048, 512, False)])
+def test_fused_epilogue_on_every_direct_to_lds_tile(M, N, Kd, sliced):
+    """A product with a functor takes the tile and the K slices of the plain product: ragged edges of each tile, alone and in
+    slices on two streams, against exact results; then the launch that may not allocate, which runs whole on what is compiled."""
+    import extra_kernels as X
+    dtype = torch.bfloat16 if M % 4 else torch.float16
+    g = torch.Generator().manual_seed(M + N)
+    a = torch.zeros(M, Kd, dtype=dtype)
+    a.scatter_(1, torch.randint(0, Kd, (M, 40), generator=g), 1.0)
+    b = torch.randint(-2, 3, (Kd, N), generator=g).to(dtype)
+    bias, held = torch.randint(-4, 5, (N,), generator=g).float(), torch.randint(-8, 9, (M, N), generator=g).to(dtype)
+    product = (a.to(DEV).float() @ b.to(DEV).float()).double().cpu()   # sums of at most 40 small integers: exact
+    want = torch.nn.functional.leaky_relu(product + bias.double(), 0.5)
+    ad, bd, biasd = a.to(DEV), b.to(DEV), bias.to(DEV)
+    grid = (triton.cdiv(M, 128), triton.cdiv(N, 128))
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    for i in range(3):
+        with torch.cuda.stream(streams[i % 2]):
+            c = torch.full((M + 1, N + 2), 7.0, dtype=dtype, device=DEV)
+            k = X.matmul_leaky[grid](ad, bd, c, M, N, Kd, Kd, N, N + 2, 0.5, BM=128, BN=128, BK=64, ACT=2, bias_ptr=biasd)
+        torch.cuda.synchronize()
+        assert k.function.last_kernel == "gemm_dma_kernel + epilogue (hipRTC)" + (", K slices" if sliced else "")
+        assert torch.equal(c[:M, :N].cpu().double(), want) and (c[M] == 7.0).all() and (c[:, N:] == 7.0).all()
+    c.fill_(7.0)
+    values = [ad.data_ptr(), bd.data_ptr(), c.data_ptr(), M, N, Kd, Kd, N, N + 2, 0.5, biasd.data_ptr()]
+    assert len(values) == len(k.function.arg_kinds)
+    k.function.launch_noalloc((*grid, 1), torch.cuda.current_stream().cuda_stream, values)
+    torch.cuda.synchronize()
+    assert k.function.last_kernel == "gemm_dma_kernel + epilogue (hipRTC)" and torch.equal(c[:M, :N].cpu().double(), want)
+    c = held.to(DEV)
+    X.matmul_leaky[grid](ad, bd, c, M, N, Kd, Kd, N, N, 0.5, BM=128, BN=128, BK=64, ACT=3)
+    torch.cuda.synchronize()
+    assert torch.equal(c.cpu().double(), product * 0.5 + held.double())
+
+
 # ------------------------------------------------------------------ grids beyond the device's extents
 def test_grid_extents_beyond_the_device_limit():
     """The reference's launcher loops over any grid (backend/driver.py:116-133); the device's grid holds 65535 along y and

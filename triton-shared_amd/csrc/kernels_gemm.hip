@@ -11,6 +11,7 @@
 // dense C = A*B, so these kernels choose their own tiling.
 #include "kernels.h"
 
+#include <cmath>
 #include <cstring>
 
 namespace tts {
@@ -847,23 +848,19 @@ constexpr int W8_WAVES = 16;
 
 namespace {
 // Which direct-to-LDS tile a product runs on (null: none applies), and in how many K slices.
-struct DmaCand { const char *tag; int64_t bm, bn; double eff; };
-const DmaCand DMA_CANDS[4] = {{"256x256", 256, 256, 1.0}, {"128x256", 128, 256, 0.77}, {"256x128", 256, 128, 0.73}, {"128x128", 128, 128, 0.59}};
+// first, more, fixed: us per K tile of a round of workgroups that is all but empty, what a full round adds to it, and per launch,
+// fitted to the table at unsliced_time.
+struct DmaCand { const char *tag; int64_t bm, bn; double eff, first, more, fixed; };
+const DmaCand DMA_CANDS[4] = {{"256x256", 256, 256, 1.0, 0.53, 0.25, 8}, {"128x256", 128, 256, 0.77, 0.33, 0.15, 9},
+                              {"256x128", 256, 128, 0.73, 0.36, 0.16, 9}, {"128x128", 128, 128, 0.59, 0.22, 0.07, 8}};
 struct DmaChoice { const DmaCand *tile = nullptr; int split = 1; };
 
 DmaChoice choose_dma(const GemmParams &p, int max_split) {
   static const char *dma_env = getenv("TTS_GEMM_DMA");      // tuning aid: "256x256", "128x256", "256x128", "128x128" or unset
   static const char *split_env = getenv("TTS_GEMM_SPLIT");  // tuning aid: the number of K slices (1 = never split)
-  static const int cus = [] {
-    int dev = 0, n = 0;
-    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-    return n;
-  }();
+  const int cus = device_cus();
   // (tiles of all the batch's products: they share the launch)
   auto tiles = [&](const DmaCand &c) { return ((p.M + c.bm - 1) / c.bm) * ((p.N + c.bn - 1) / c.bn) * std::max(1, p.batches); };
-  // Among the tiles that give every CU a workgroup (128 x 128: always), the one with the least padded work per unit
-  // of the tile's measured efficiency at 4096^3 (105 / 136 / 144 / 179 us): a ragged edge counts against a tile that
-  // overshoots it by more.
   // Rows with a weight matrix per block stream their weights from HBM, and the 128 x 256 tile's prefetching wavefront is ahead
   // from half a workgroup per CU on (us with 128 x 128 / 128 x 256 tiles: 144 of the latter 65 / 58, 160 42.4 / 40.1, 192 57.8 /
   // 50.8; below, 72 29.0 / 43.9, 28 16.4 / 19.6), but not where they make a second round that is mostly empty (288 73.3 / 79.1, 320
@@ -871,12 +868,26 @@ DmaChoice choose_dma(const GemmParams &p, int max_split) {
   // 800 210 / 210).  A few tiles over one round count as one: blocks of rows that pad the last matrix have nothing to do.
   const bool grouped = p.b_block != nullptr && !p.b_trans;
   auto grouped_wide = [&](int64_t t) { return 2 * t >= cus && !(10 * t > 11 * cus && 10 * t < 16 * cus); };
+  // The other products: the least modelled time without slices.  What decides is whole rounds of workgroups over the chip (the
+  // 128 x 128 tile's two workgroups per CU blur them), and that a round runs faster the emptier it is.  Measured, us with 256 x 256
+  // / 128 x 256 / 128 x 128 tiles: 3500 x 4096 x 4096 101 / 132 / 147; 3000 x 4096 x 2048 50.5 / 67.6 / 65.9; 3000 x 2048 x 4096 80.8 / 61.1 /
+  // 68.2; 4096 x 2048 x 2048 48 / 39 / 45; 2500 x 2048 x 1024 25.7 / 18.3 / 20.8; 2048^3 42.3 / 28.2 / 21.7; 1024 x 1024 x 4096 74 / 49 / 33.
+  // (By the rule of short K below, the first two ran at 131 and 68 us.)  Below K = 512 the fixed costs decide and the tiles measure
+  // alike: among the tiles that give every CU a workgroup (128 x 128: always) the one with the least padded work per unit of
+  // the tile's measured efficiency at 4096^3 (105 / 136 / 144 / 179 us).
+  const bool by_rounds = !grouped && p.K >= 512;
+  auto unsliced_time = [&](const DmaCand &c) {
+    const double f = (double)tiles(c) / cus, whole = std::floor(f), rest = f - whole;
+    double rounds = whole * (c.first + c.more) + (rest > 0 ? c.first + c.more * rest : 0);
+    if (c.bm + c.bn == 256 && f > 1) rounds = (c.first + c.more) * 0.5 * (f + std::ceil(f));
+    return (rounds * (double)(p.K / F_BK) + c.fixed) * 1e-6;
+  };
   DmaChoice best;
   double best_cost = 0;
   for (const DmaCand &c : DMA_CANDS) {
     if (!gemm_dma_ok(p, c.bm, c.bn)) continue;
-    if (dma_env ? std::string(dma_env) != c.tag : (c.bm + c.bn != 256 && (grouped ? !grouped_wide(tiles(c)) : tiles(c) < cus))) continue;
-    const double cost = (double)(tiles(c) * c.bm * c.bn) / c.eff;
+    if (dma_env ? std::string(dma_env) != c.tag : !by_rounds && c.bm + c.bn != 256 && (grouped ? !grouped_wide(tiles(c)) : tiles(c) < cus)) continue;
+    const double cost = by_rounds ? unsliced_time(c) : (double)(tiles(c) * c.bm * c.bn) / c.eff;
     if (!best.tile || cost < best_cost) { best.tile = &c; best_cost = cost; }
   }
   if (!best.tile || max_split < 2 || p.a_rows || p.b_block) return best;
@@ -898,7 +909,8 @@ DmaChoice choose_dma(const GemmParams &p, int max_split) {
     return t;
   };
   DmaChoice pick = best;
-  double pick_t = model(*best.tile, 1);
+  // (the times without slices were measured on operands that partly sat in the Infinity Cache)
+  double pick_t = by_rounds ? std::min(model(*best.tile, 1), 1.15 * unsliced_time(*best.tile)) : model(*best.tile, 1);
   if (!(split_env && atoi(split_env) == 1))
     for (const DmaCand &c : DMA_CANDS) {
       if (!gemm_dma_ok(p, c.bm, c.bn) || (dma_env && std::string(dma_env) != c.tag)) continue;
@@ -1008,8 +1020,9 @@ hipError_t launch_dma_slices(const GemmParams &p, hipStream_t s) {
 }
 
 // What a product with a functor runs on, in at most max_split K slices.  Row-major operands of whole K tiles take the
-// direct-to-LDS tile and the slices that the plain product takes (choose_dma): one 256 x 256 tile for each size, as these
-// launches once had, leaves most of the chip idle where there are few.
+// direct-to-LDS tile and the slices that the plain product takes (choose_dma).  With leaky_relu in bf16, us, against 256 x 256
+// tiles at every size: 128 x 4096 x 4096 22.5 / 80.6; 16 x 4096 x 4096 19 / 79; 512^3 12 / 17; 1024^3 13 / 25.5; 2048^3 24 / 44;
+// 1000 x 4096 x 4096 53 / 88; 4096 x 2048 x 2048 40 / 48.6.  (A column-major operand goes to the any-shape kernel.)
 struct EpilogueChoice { int whole, split; const DmaCand *tile; };  // the kernel without slices; the tile the slices run on (null: any shape)
 EpilogueChoice choose_epilogue(const GemmParams &p, int max_split) {
   if (!gemm_fast_path_ok(p)) return {any_rows(p, 1) == 64 ? 3 : 1, any_split(p, max_split), nullptr};
