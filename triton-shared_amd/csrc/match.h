@@ -42,8 +42,7 @@ struct Plan {
 // (tile_codegen.cpp).  Throws Unsupported for anything else.  The kernel's argument block holds
 // every kernel argument by index: { void *ptr[N]; long long ival[N]; double fval[N]; }, N = TILE_MAX_ARGS.
 constexpr int TILE_MAX_ARGS = 32;
-std::string tile_program_source(const Program &p, bool allow_persistent = true);  // (persistent: see tile_program_is_persistent)
-bool tile_program_is_persistent(const std::string &source);  // the kernel walks the programs itself: any one-dimensional launch, lgx/lgy/lgz = the grid
+std::string tile_program_source(const Program &p);
 // The same program in the form for programs built around 16-bit matrix products (tile_mma.h); empty if it is not one.
 std::string matrix_program_source(const Program &p);
 bool tile_program_is_matrix(const std::string &source, int *programs, int *axis, int *threads);  // programs per workgroup along which axis (-1: x), threads

@@ -795,46 +795,6 @@ struct Gen {
   static std::pair<std::string, std::string> along(const std::vector<int64_t> &shape, const std::string &i, const std::string &delta) {
     return {shape.size() < 2 ? "(" + i + delta + ")" : i, shape.size() < 2 ? i : "(" + i + delta + ")"};
   }
-  // A wide program whose body loads a block that is the same for every program (a row of weights next to the row it
-  // scales: its address and extent name no program id, loop variable or loaded value, and nothing stores to its argument)
-  // is written "persistent": the launch has a few workgroups per CU, each walks the programs lin = blockIdx.x,
-  // blockIdx.x + gridDim.x, ... and the shared blocks are loaded once per workgroup, before that loop (hoisted: their
-  // code goes to hoist_os).  Read again by every program they stay in L2, but the L2 -> CU traffic is that of a second
-  // row (RMSNorm fp16 [4096, 8192]: 27.5 -> 25.5 us).
-  bool persistent = false;
-  // In a persistent kernel every wide 16-bit load stays packed (two elements per register, widened where used): RMSNorm
-  // on rows of 8192 then takes 75 registers instead of 111.  (With a workgroup per program the compiler keeps packed and
-  // widened values side by side and takes more registers than without: 121 against 108; the launcher compiles that form,
-  // unpacked, when the persistent one holds too few workgroups per CU.)
-  bool pack_wide = false;
-  std::set<int> hoisted;  // value ids of the loads emitted before the program loop
-  std::ostringstream hoist_os;
-  std::ostringstream loop_top;  // first statements of the program loop
-  void choose_persistent() {
-    if (!wide_mode || gathers_rows) return;
-    if (const char *e = getenv("TTS_TILE_PERSISTENT"))
-      if (e[0] == '0') return;
-    std::set<int> stored;
-    std::function<void(const std::vector<SOp> &)> scan = [&](const std::vector<SOp> &ops) {
-      for (const SOp &s : ops) {
-        if (s.kind == SK::Store || s.kind == SK::ScalarStore) stored.insert(s.acc.base_arg);
-        if (s.kind == SK::For || s.kind == SK::If) scan(s.body);
-      }
-    };
-    scan(P.body);
-    for (const SOp &s : P.body) {
-      if (s.kind != SK::Load || !wide(s.acc.sizes) || !vector_access(s.acc) || stored.count(s.acc.base_arg) || s.acc.other_value >= 0) continue;
-      std::vector<int> es = s.acc.offsets;
-      es.insert(es.end(), s.acc.strides.begin(), s.acc.strides.end());
-      es.insert(es.end(), s.acc.dims.begin(), s.acc.dims.end());
-      bool fixed = true;
-      for (int e : es)
-        for (EK k : {EK::Pid, EK::NProg, EK::IV, EK::Iter, EK::Result, EK::Data}) fixed = fixed && (e < 0 || !P.pool.depends_on(e, k));  // (what the code before the program loop can name: arguments and constants)
-      if (fixed) hoisted.insert(s.result);
-    }
-    persistent = !hoisted.empty();
-    pack_wide = persistent;
-  }
   // A loop that only adds -- every carried block is `arg + x` with x free of carried values, nothing in the body stores, and
   // after the loop the blocks are only summed along an axis -- may run in slices: a program's iterations are dealt to
   // several workgroups, whose sums meet before anything after the loop (see slices_meet).  The column sums of a
@@ -1340,21 +1300,8 @@ struct Gen {
           bool any = false;
           for (size_t q = k; q < end; q++)
             if (mine_here(ops[q])) {
-              if (pack_wide && !hoisted.count(ops[q].result) && wide(ls) && vector_access(ops[q].acc) && is16(ops[q].acc.elem))
-                os << pad() << "u32x4_t rw" << ops[q].result << "[" << count(ls) / 2048 << "];\n";
-              else if (hoisted.count(ops[q].result)) {
-                // (16-bit blocks that stay in registers for the whole launch stay packed, two elements per register, and
-                // are widened where they are used)
-                if (is16(ops[q].acc.elem)) {
-                  hoist_os << "  u32x4_t rw" << ops[q].result << "[" << count(ls) / 2048 << "];\n";
-                  // (the empty asm says the words may have changed: the compiler would otherwise widen them once, before
-                  // the loop, and keep twice the registers for the whole launch)
-                  for (int64_t g = 0; g < count(ls) / 2048; g++) loop_top << "    asm volatile(\"\" : \"+v\"(rw" << ops[q].result << "[" << g << "]));\n";
-                }
-                else hoist_os << "  " << ctype(val(ops[q].result).dtype) << " ld" << ops[q].result << "[" << (count(ls) + 255) / 256 << "];\n";
-              }
-              else if (!row_gather(ops[q].acc))  // (inside a program loop a slot that a masked load leaves unwritten would otherwise hold, and carry, the last program's)
-                os << pad() << ctype(val(ops[q].result).dtype) << " ld" << ops[q].result << "[" << (held_count(ls) + 255) / 256 << "]" << (persistent ? " = {}" : "") << ";\n";
+              if (!row_gather(ops[q].acc))
+                os << pad() << ctype(val(ops[q].result).dtype) << " ld" << ops[q].result << "[" << (held_count(ls) + 255) / 256 << "];\n";
               any = true;
             }
           if (!any) continue;
@@ -1389,170 +1336,127 @@ struct Gen {
           // afterwards (drop_front), any other from a dummy; a second loop unpacks, widens and fills in `other`.  No branch
           // sits between the loads, so none waits for another.  Only a program whose extent is one to seven elements loads
           // element by element, as it would in the ordinary order.
-          auto wide_load_any = [&](const SOp &o) { return wide(ls) && mine_here(o) && vector_access(o.acc); };
-          for (int pass = 0; pass < 2; pass++) {  // pass 0: the loads hoisted out of the program loop, into hoist_os
-            auto wide_load = [&](const SOp &o) { return wide_load_any(o) && (hoisted.count(o.result) != 0) == (pass == 0); };
-            const int saved_indent = indent;
-            if (pass == 0) {
-              os.swap(hoist_os);
-              indent = 1;
-            }
-            auto packed = [&](const SOp &o) { return (pass == 0 || pack_wide) && is16(o.acc.elem); };
-            bool any_wide = false;
-            for (size_t q = k; q < end; q++) any_wide = any_wide || wide_load(ops[q]);
-            if (any_wide) {
-              const int64_t G = held_count(ls) / 2048;
-              uses_dummy = true;
-              std::string roomy;  // the extents of the masked ones leave eight elements to read, or none (the same in every thread)
-              for (size_t q = k; q < end; q++)
-                if (wide_load(ops[q]) && !ops[q].acc.dims.empty()) {
-                  const std::string ext = "(" + ex(ops[q].acc.dims.back()) + ")";
-                  if (roomy.find(ext) == std::string::npos) roomy += std::string(roomy.empty() ? "" : " && ") + "(" + ext + " <= 0 || " + ext + " >= 8)";
-                }
-              os << pad() << "if (" << (roomy.empty() ? "true" : roomy) << ") {\n";
-              indent++;
-              for (size_t q = k; q < end; q++)
-                if (wide_load(ops[q]) && !packed(ops[q]))
-                  os << pad() << (mem_bytes(ops[q].acc.elem) == 1 ? "u32x2_t rw" : "u32x4_t rw") << ops[q].result << "[" << G * (mem_bytes(ops[q].acc.elem) == 4 ? 2 : 1) << "];\n";
-              os << pad() << "#pragma unroll\n" << pad() << "for (int g = 0; g < " << G << "; g++) {\n";
-              indent++;
-              os << pad() << "const int n = 8 * g;\n" << pad() << "const int t = " << element_of_slot(ls) << ";\n";
-              for (size_t q = k; q < end; q++)
-                if (wide_load(ops[q])) {
-                  const SOp &o = ops[q];
-                  const std::string id = std::to_string(o.result), mt = memtype(o.acc.elem);
-                  std::string pred, addr = address(o.acc, l0, l1, pred);
-                  os << pad() << "{\n";
-                  indent++;
-                  const std::string vt = mem_bytes(o.acc.elem) == 1 ? "u32x2_any" : "u32x4_any";
-                  if (pred.empty())
-                    os << pad() << "const " << vt << " *const src = (const " << vt << " *)((const " << mt << " *)p.ptr[" << o.acc.base_arg << "] + (" << addr << "));\n";
-                  else
-                    os << pad() << "const " << vt << " *const src = !(" << pred << ") ? (const " << vt << " *)tts_dummy : (const " << vt << " *)((const " << mt << " *)p.ptr["
-                       << o.acc.base_arg << "] + (" << addr << ") - " << cut_off(o.acc, ls.size() < 2 ? l0 : l1) << ");\n";
-                  if (mem_bytes(o.acc.elem) <= 2) os << pad() << "rw" << id << "[g] = src[0];\n";
-                  else os << pad() << "rw" << id << "[2 * g] = src[0];\n" << pad() << "rw" << id << "[2 * g + 1] = src[1];\n";
-                  indent--;
-                  os << pad() << "}\n";
-                }
-              indent--;
-              os << pad() << "}\n";
-              for (size_t q = k; q < end; q++)
-                if (wide_load(ops[q]) && !ops[q].acc.dims.empty()) {
-                  const SOp &o = ops[q];
-                  const std::string id = std::to_string(o.result);
-                  const int esz = mem_bytes(o.acc.elem);
-                  std::string pred;
-                  address(o.acc, l0, l1, pred);
-                  os << pad() << "if (" << ex(o.acc.dims.back()) << " & 7) {\n";
-                  indent++;
-                  os << pad() << "#pragma unroll\n" << pad() << "for (int g = 0; g < " << G << "; g++) {\n";
-                  indent++;
-                  os << pad() << "const int n = 8 * g;\n" << pad() << "const int t = " << element_of_slot(ls) << ";\n" << pad() << "(void)t;\n";
-                  os << pad() << "const int cut = (" << pred << ") ? " << cut_off(o.acc, ls.size() < 2 ? l0 : l1) << " : 0;\n";
-                  os << pad() << "if (cut) " << (esz == 4 ? "drop_front_32(rw" + id + "[2 * g], rw" + id + "[2 * g + 1], cut)" : (esz == 2 ? "drop_front_16(rw" : "drop_front_8(rw") + id + "[g], cut)") << ";\n";
-                  indent--;
-                  os << pad() << "}\n";
-                  indent--;
-                  os << pad() << "}\n";
-                }
-              bool any_packed = false, any_unpacked = false;
-              for (size_t q = k; q < end; q++) {
-                any_packed = any_packed || (wide_load(ops[q]) && packed(ops[q]));
-                any_unpacked = any_unpacked || (wide_load(ops[q]) && !packed(ops[q]));
+          auto wide_load = [&](const SOp &o) { return wide(ls) && mine_here(o) && vector_access(o.acc); };
+          bool any_wide = false;
+          for (size_t q = k; q < end; q++) any_wide = any_wide || wide_load(ops[q]);
+          if (any_wide) {
+            const int64_t G = held_count(ls) / 2048;
+            uses_dummy = true;
+            std::string roomy;  // the extents of the masked ones leave eight elements to read, or none (the same in every thread)
+            for (size_t q = k; q < end; q++)
+              if (wide_load(ops[q]) && !ops[q].acc.dims.empty()) {
+                const std::string ext = "(" + ex(ops[q].acc.dims.back()) + ")";
+                if (roomy.find(ext) == std::string::npos) roomy += std::string(roomy.empty() ? "" : " && ") + "(" + ext + " <= 0 || " + ext + " >= 8)";
               }
-              if (any_unpacked) open_element_loop(ls);
-              for (size_t q = k; q < end; q++)
-                if (wide_load(ops[q]) && !packed(ops[q])) {
-                  const SOp &o = ops[q];
-                  const std::string id = std::to_string(o.result);
-                  std::string pred, addr = address(o.acc, l0, l1, pred);
-                  std::string got;
-                  if (is16(o.acc.elem)) {
-                    const std::string word = "rw" + id + "[n >> 3][(n & 7) >> 1]";
-                    got = std::string(o.acc.elem == "f16" ? "up_f16(" : "up_bf16(") + "(unsigned short)((n & 1) ? " + word + " >> 16 : " + word + "))";
-                  } else if (mem_bytes(o.acc.elem) == 1) {
-                    got = "(signed char)(rw" + id + "[n >> 3][(n & 7) >> 2] >> (8 * (n & 3)))";
-                  } else {
-                    const std::string word = "rw" + id + "[n >> 2][n & 3]";
-                    got = o.acc.elem == "f32" ? "__uint_as_float(" + word + ")" : "(int)" + word;
-                  }
-                  os << pad() << "ld" << id << "[n] = " << (pred.empty() ? got : "(" + pred + ") ? " + got + " : " + other_of(o.acc, l0, l1)) << ";\n";
+            os << pad() << "if (" << (roomy.empty() ? "true" : roomy) << ") {\n";
+            indent++;
+            for (size_t q = k; q < end; q++)
+              if (wide_load(ops[q]))
+                os << pad() << (mem_bytes(ops[q].acc.elem) == 1 ? "u32x2_t rw" : "u32x4_t rw") << ops[q].result << "[" << G * (mem_bytes(ops[q].acc.elem) == 4 ? 2 : 1) << "];\n";
+            os << pad() << "#pragma unroll\n" << pad() << "for (int g = 0; g < " << G << "; g++) {\n";
+            indent++;
+            os << pad() << "const int n = 8 * g;\n" << pad() << "const int t = " << element_of_slot(ls) << ";\n";
+            for (size_t q = k; q < end; q++)
+              if (wide_load(ops[q])) {
+                const SOp &o = ops[q];
+                const std::string id = std::to_string(o.result), mt = memtype(o.acc.elem);
+                std::string pred, addr = address(o.acc, l0, l1, pred);
+                os << pad() << "{\n";
+                indent++;
+                const std::string vt = mem_bytes(o.acc.elem) == 1 ? "u32x2_any" : "u32x4_any";
+                if (pred.empty())
+                  os << pad() << "const " << vt << " *const src = (const " << vt << " *)((const " << mt << " *)p.ptr[" << o.acc.base_arg << "] + (" << addr << "));\n";
+                else
+                  os << pad() << "const " << vt << " *const src = !(" << pred << ") ? (const " << vt << " *)tts_dummy : (const " << vt << " *)((const " << mt << " *)p.ptr["
+                     << o.acc.base_arg << "] + (" << addr << ") - " << cut_off(o.acc, ls.size() < 2 ? l0 : l1) << ");\n";
+                if (mem_bytes(o.acc.elem) <= 2) os << pad() << "rw" << id << "[g] = src[0];\n";
+                else os << pad() << "rw" << id << "[2 * g] = src[0];\n" << pad() << "rw" << id << "[2 * g + 1] = src[1];\n";
+                indent--;
+                os << pad() << "}\n";
+              }
+            indent--;
+            os << pad() << "}\n";
+            for (size_t q = k; q < end; q++)
+              if (wide_load(ops[q]) && !ops[q].acc.dims.empty()) {
+                const SOp &o = ops[q];
+                const std::string id = std::to_string(o.result);
+                const int esz = mem_bytes(o.acc.elem);
+                std::string pred;
+                address(o.acc, l0, l1, pred);
+                os << pad() << "if (" << ex(o.acc.dims.back()) << " & 7) {\n";
+                indent++;
+                os << pad() << "#pragma unroll\n" << pad() << "for (int g = 0; g < " << G << "; g++) {\n";
+                indent++;
+                os << pad() << "const int n = 8 * g;\n" << pad() << "const int t = " << element_of_slot(ls) << ";\n" << pad() << "(void)t;\n";
+                os << pad() << "const int cut = (" << pred << ") ? " << cut_off(o.acc, ls.size() < 2 ? l0 : l1) << " : 0;\n";
+                os << pad() << "if (cut) " << (esz == 4 ? "drop_front_32(rw" + id + "[2 * g], rw" + id + "[2 * g + 1], cut)" : (esz == 2 ? "drop_front_16(rw" : "drop_front_8(rw") + id + "[g], cut)") << ";\n";
+                indent--;
+                os << pad() << "}\n";
+                indent--;
+                os << pad() << "}\n";
+              }
+            open_element_loop(ls);
+            for (size_t q = k; q < end; q++)
+              if (wide_load(ops[q])) {
+                const SOp &o = ops[q];
+                const std::string id = std::to_string(o.result);
+                std::string pred, addr = address(o.acc, l0, l1, pred);
+                std::string got;
+                if (is16(o.acc.elem)) {
+                  const std::string word = "rw" + id + "[n >> 3][(n & 7) >> 1]";
+                  got = std::string(o.acc.elem == "f16" ? "up_f16(" : "up_bf16(") + "(unsigned short)((n & 1) ? " + word + " >> 16 : " + word + "))";
+                } else if (mem_bytes(o.acc.elem) == 1) {
+                  got = "(signed char)(rw" + id + "[n >> 3][(n & 7) >> 2] >> (8 * (n & 3)))";
+                } else {
+                  const std::string word = "rw" + id + "[n >> 2][n & 3]";
+                  got = o.acc.elem == "f32" ? "__uint_as_float(" + word + ")" : "(int)" + word;
                 }
-              if (any_unpacked) close_loop();
-              indent--;
-              os << pad() << "} else {\n";
-              indent++;
+                os << pad() << "ld" << id << "[n] = " << (pred.empty() ? got : "(" + pred + ") ? " + got + " : " + other_of(o.acc, l0, l1)) << ";\n";
+              }
+            close_loop();
+            indent--;
+            os << pad() << "} else {\n";
+            indent++;
+            open_element_loop(ls);
+            for (size_t q = k; q < end; q++)
+              if (wide_load(ops[q])) {
+                const SOp &o = ops[q];
+                const std::string name = "ld" + std::to_string(o.result);
+                std::string pred, addr = address(o.acc, l0, l1, pred);
+                if (pred.empty()) os << pad() << name << "[n] = " << mem_read(o.acc, addr) << ";\n";
+                else if (is16(o.acc.elem))
+                  os << pad() << "if (" << pred << ") " << name << "[n] = __uint_as_float(((const unsigned short *)p.ptr[" << o.acc.base_arg << "])[" << addr << "]);\n";
+                else os << pad() << "if (" << pred << ") " << name << "[n] = " << mem_read(o.acc, addr) << ";\n";
+              }
+            close_loop();
+            bool any_masked = false;
+            for (size_t q = k; q < end; q++) any_masked = any_masked || (wide_load(ops[q]) && !ops[q].acc.dims.empty());
+            if (any_masked) {
+              open_element_loop(ls);
               for (size_t q = k; q < end; q++)
-                if (wide_load(ops[q]) && packed(ops[q])) os << pad() << "unsigned tm" << ops[q].result << "[" << count(ls) / 256 << "] = {};\n";
-              if (any_packed) open_element_loop(ls);
-              for (size_t q = k; q < end; q++)
-                if (wide_load(ops[q]) && packed(ops[q])) {
-                  std::string pred, addr = address(ops[q].acc, l0, l1, pred);
-                  os << pad() << (pred.empty() ? "" : "if (" + pred + ") ") << "tm" << ops[q].result << "[n] = ((const unsigned short *)p.ptr[" << ops[q].acc.base_arg << "])[" << addr << "];\n";
-                }
-              if (any_packed) close_loop();
-              for (size_t q = k; q < end; q++)
-                if (wide_load(ops[q]) && packed(ops[q])) {
-                  os << pad() << "#pragma unroll\n" << pad() << "for (int g = 0; g < " << G << "; g++)\n";
-                  os << pad() << "  rw" << ops[q].result << "[g] = u32x4_t{";
-                  for (int c = 0; c < 4; c++)
-                    os << (c ? ", " : "") << "tm" << ops[q].result << "[8 * g + " << 2 * c << "] | tm" << ops[q].result << "[8 * g + " << 2 * c + 1 << "] << 16";
-                  os << "};\n";
-                }
-              if (any_unpacked) open_element_loop(ls);
-              for (size_t q = k; q < end; q++)
-                if (wide_load(ops[q]) && !packed(ops[q])) {
+                if (wide_load(ops[q]) && !ops[q].acc.dims.empty()) {
                   const SOp &o = ops[q];
                   const std::string name = "ld" + std::to_string(o.result);
                   std::string pred, addr = address(o.acc, l0, l1, pred);
-                  if (pred.empty()) os << pad() << name << "[n] = " << mem_read(o.acc, addr) << ";\n";
-                  else if (is16(o.acc.elem))
-                    os << pad() << "if (" << pred << ") " << name << "[n] = __uint_as_float(((const unsigned short *)p.ptr[" << o.acc.base_arg << "])[" << addr << "]);\n";
-                  else os << pad() << "if (" << pred << ") " << name << "[n] = " << mem_read(o.acc, addr) << ";\n";
+                  if (is16(o.acc.elem)) {
+                    os << pad() << "asm volatile(\"\" : \"+v\"(" << name << "[n]));\n";
+                    os << pad() << name << "[n] = (" << pred << ") ? " << (o.acc.elem == "f16" ? "up_f16(" : "up_bf16(") << "(unsigned short)__float_as_uint(" << name
+                       << "[n])) : " << other_of(o.acc, l0, l1) << ";\n";
+                  } else
+                    os << pad() << "if (!(" << pred << ")) " << name << "[n] = " << other_of(o.acc, l0, l1) << ";\n";
                 }
-              if (any_unpacked) close_loop();
-              bool any_masked = false;
-              for (size_t q = k; q < end; q++) any_masked = any_masked || (wide_load(ops[q]) && !packed(ops[q]) && !ops[q].acc.dims.empty());
-              if (any_masked) {
-                open_element_loop(ls);
-                for (size_t q = k; q < end; q++)
-                  if (wide_load(ops[q]) && !packed(ops[q]) && !ops[q].acc.dims.empty()) {
-                    const SOp &o = ops[q];
-                    const std::string name = "ld" + std::to_string(o.result);
-                    std::string pred, addr = address(o.acc, l0, l1, pred);
-                    if (is16(o.acc.elem)) {
-                      os << pad() << "asm volatile(\"\" : \"+v\"(" << name << "[n]));\n";
-                      os << pad() << name << "[n] = (" << pred << ") ? " << (o.acc.elem == "f16" ? "up_f16(" : "up_bf16(") << "(unsigned short)__float_as_uint(" << name
-                         << "[n])) : " << other_of(o.acc, l0, l1) << ";\n";
-                    } else
-                      os << pad() << "if (!(" << pred << ")) " << name << "[n] = " << other_of(o.acc, l0, l1) << ";\n";
-                  }
-                close_loop();
+              close_loop();
+            }
+            indent--;
+            os << pad() << "}\n";
+            for (size_t q = k; q < end; q++)
+              if (wide_load(ops[q])) {
+                const SOp &o = ops[q];
+                const std::string name = "ld" + std::to_string(o.result);
+                held[o.result] = {name, ls};
+                var[o.result] = name + "[n]";
+                mine.push_back(o.result);
               }
-              indent--;
-              os << pad() << "}\n";
-              for (size_t q = k; q < end; q++)
-                if (wide_load(ops[q])) {
-                  const SOp &o = ops[q];
-                  if (packed(o)) {
-                    const std::string word = "rw" + std::to_string(o.result) + "[n >> 3][(n & 7) >> 1]";
-                    std::string pred, addr = address(o.acc, l0, l1, pred);
-                    const std::string got = std::string(o.acc.elem == "f16" ? "up_f16(" : "up_bf16(") + "(unsigned short)((n & 1) ? " + word + " >> 16 : " + word + "))";
-                    held[o.result] = {"rw" + std::to_string(o.result), ls, "(" + (pred.empty() ? got : "(" + pred + ") ? " + got + " : " + other_of(o.acc, l0, l1)) + ")"};
-                    var[o.result] = held[o.result].expr;
-                  } else {
-                    const std::string name = "ld" + std::to_string(o.result);
-                    held[o.result] = {name, ls};
-                    var[o.result] = name + "[n]";
-                  }
-                  mine.push_back(o.result);
-                }
-            }
-            if (pass == 0) {
-              os.swap(hoist_os);
-              indent = saved_indent;
-            }
           }
           for (size_t q = k; q < end; q++)
             if (mine_here(ops[q]) && row_gather(ops[q].acc)) {
@@ -1597,13 +1501,13 @@ struct Gen {
               mine.push_back(o.result);
               any_load = true;
             }
-          auto wide_load = [&](const SOp &o) { return wide_load_any(o) || row_gather(o.acc); };
+          auto loaded = [&](const SOp &o) { return wide_load(o) || row_gather(o.acc); };
           bool any_classic = false;
-          for (size_t q = k; q < end; q++) any_classic = any_classic || (mine_here(ops[q]) && !wide_load(ops[q]));
+          for (size_t q = k; q < end; q++) any_classic = any_classic || (mine_here(ops[q]) && !loaded(ops[q]));
           if (!any_classic) continue;
           open_element_loop(ls);
           for (size_t q = k; q < end; q++)
-            if (mine_here(ops[q]) && !wide_load(ops[q])) {
+            if (mine_here(ops[q]) && !loaded(ops[q])) {
               const std::string name = "ld" + std::to_string(ops[q].result);
               std::string pred, addr = address(ops[q].acc, l0, l1, pred);
               bool needs_filled = false;  // indexed or masked by a load that still lacks its `other`
@@ -2569,7 +2473,6 @@ namespace {
 const char *const SWAP_MARK = "// tts: swap_xy\n";
 const char *const MATRIX_MARK = "// tts: matrix ";  // followed by: programs per workgroup, the axis they lie on, threads per workgroup
 const char *const SLICED_MARK = "// tts: sliced ";  // followed by: floats of partial sums per program and slice, the loop's id
-const char *const PERSISTENT_MARK = "// tts: persistent\n";  // the launcher starts a few workgroups per CU, which walk the programs
 bool stores_walk_columns_with_pid1(const Program &p) {
   int votes_for = 0, votes_against = 0;
   std::function<void(const std::vector<SOp> &)> scan = [&](const std::vector<SOp> &ops) {
@@ -2609,23 +2512,14 @@ std::string without_double_barriers(std::string src) {
   }
   return src;
 }
-// The body of a persistent kernel's program loop with the thread's index read from a variable that an empty asm renews in
-// every iteration: what depends on it alone -- 32 element masks, 32 64-bit element offsets -- is otherwise computed once,
-// before the loop, and held in registers for the whole launch (LayerNorm's input gradient: 211 registers instead of 149).
-std::string per_program_thread_index(std::string body) {
-  const std::string from = "threadIdx.x", to = "tidx";
-  for (size_t pos = 0; (pos = body.find(from, pos)) != std::string::npos; pos += to.size()) body.replace(pos, from.size(), to);
-  return "    unsigned tidx = threadIdx.x;\n    asm volatile(\"\" : \"+v\"(tidx));\n" + body;
-}
 }  // namespace
 
 bool tile_program_swaps_grid(const std::string &source) {
   const size_t at = source.compare(0, strlen(SLICED_MARK), SLICED_MARK) == 0 ? source.find('\n') + 1 : 0;
   return source.compare(at, strlen(SWAP_MARK), SWAP_MARK) == 0;
 }
-bool tile_program_is_persistent(const std::string &source) { return source.compare(0, strlen(PERSISTENT_MARK), PERSISTENT_MARK) == 0; }
 
-std::string tile_program_source(const Program &p, bool allow_persistent) {
+std::string tile_program_source(const Program &p) {
   if ((int)p.arg_names.size() > TILE_MAX_ARGS) throw Unsupported("tile_program: more than " + std::to_string(TILE_MAX_ARGS) + " kernel arguments");
   Gen g(p);
   std::string pre = TILE_PRELUDE;
@@ -2633,10 +2527,8 @@ std::string tile_program_source(const Program &p, bool allow_persistent) {
   for (size_t pos = 0; (pos = pre.find("%N%", pos)) != std::string::npos;) pre.replace(pos, 3, n);
   g.collect_bases(p.body);
   g.choose_wide_shape();
-  if (allow_persistent) g.choose_persistent();
-  if (!g.persistent) g.choose_slices();
+  g.choose_slices();
   g.choose_column_sums();
-  if (g.persistent) g.indent = 2;
   if (g.sliced) {
     g.body(g.slice_head);
     g.slices_meet();
@@ -2648,11 +2540,8 @@ std::string tile_program_source(const Program &p, bool allow_persistent) {
   if (g.pool_bytes + g.out_bytes > 128 * 1024)
     throw Unsupported("tile_program: the reductions of this program need " + std::to_string(g.pool_bytes + g.out_bytes) + " bytes of LDS (limit 131072)");
   std::ostringstream all;
-  if (g.persistent) all << PERSISTENT_MARK;
-  else {
-    if (g.sliced) all << SLICED_MARK << g.slice_floats() << " " << g.sliced->loop << "\n";
-    if (stores_walk_columns_with_pid1(p)) all << SWAP_MARK;  // (for launches of one slice)
-  }
+  if (g.sliced) all << SLICED_MARK << g.slice_floats() << " " << g.sliced->loop << "\n";
+  if (stores_walk_columns_with_pid1(p)) all << SWAP_MARK;  // (for launches of one slice)
   all << pre << g.fns.str();
   if (g.uses_dummy) all << "__device__ __attribute__((aligned(16))) unsigned tts_dummy[8];\n";
   // swap_xy: the launcher has exchanged the grid's x and y (see SWAP_MARK)
@@ -2662,26 +2551,15 @@ std::string tile_program_source(const Program &p, bool allow_persistent) {
       << (g.sliced ? ", const int slices, float *partial, int *counters" : "") << ") {\n";
   if (g.pool_bytes) all << "  __shared__ __attribute__((aligned(16))) unsigned char pool[" << g.pool_bytes << "];\n";
   all << g.decl.str();
-  if (g.persistent) {
-    // a one-dimensional launch of any number of workgroups (lgx, lgy, lgz always hold the grid); what the programs share
-    // is loaded first; the barrier at the end keeps a program's LDS arrays from the next program's writes
-    all << g.hoist_os.str()
-        << "  for (unsigned lin = blockIdx.x; lin < (unsigned)lgx * (unsigned)lgy * (unsigned)lgz; lin += gridDim.x) {  // (fewer than 2^31 programs: the launcher sees to it)\n"
-        << "    const long long pidx = lin % (unsigned)lgx, pidy = (lin / (unsigned)lgx) % (unsigned)lgy, pidz = lin / ((unsigned)lgx * (unsigned)lgy);\n"
-        << "    const long long npx = lgx, npy = lgy, npz = lgz;\n"
-        << "    (void)pidx; (void)pidy; (void)pidz; (void)npx; (void)npy; (void)npz; (void)swap_xy;\n"
-        << g.loop_top.str() << per_program_thread_index(g.os.str()) << "    __syncthreads();\n  }\n}\n";
-  } else {
-    // sliced: the launch is one-dimensional, the slices of a program lie gridDim.x / slices workgroups apart, so that
-    // workgroups that run at the same time read neighbouring blocks
-    if (g.sliced) all << "  const int programs = (int)gridDim.x / slices, slice = (int)blockIdx.x / programs;\n  const long long lin = blockIdx.x - slice * programs;\n";
-    else all << "  const long long lin = blockIdx.x;\n";
-    all << "  const long long pidx = lgx ? lin % lgx : swap_xy ? blockIdx.y : blockIdx.x, pidy = lgx ? (lin / lgx) % lgy : swap_xy ? blockIdx.x : blockIdx.y,\n"
-        << "                  pidz = lgx ? lin / ((long long)lgx * lgy) : blockIdx.z;\n"
-        << "  const long long npx = lgx ? lgx : swap_xy ? gridDim.y : gridDim.x, npy = lgx ? lgy : swap_xy ? gridDim.x : gridDim.y, npz = lgx ? lgz : gridDim.z;\n"
-        << "  (void)pidx; (void)pidy; (void)pidz; (void)npx; (void)npy; (void)npz;\n"
-        << g.os.str() << "}\n";
-  }
+  // sliced: the launch is one-dimensional, the slices of a program lie gridDim.x / slices workgroups apart, so that
+  // workgroups that run at the same time read neighbouring blocks
+  if (g.sliced) all << "  const int programs = (int)gridDim.x / slices, slice = (int)blockIdx.x / programs;\n  const long long lin = blockIdx.x - slice * programs;\n";
+  else all << "  const long long lin = blockIdx.x;\n";
+  all << "  const long long pidx = lgx ? lin % lgx : swap_xy ? blockIdx.y : blockIdx.x, pidy = lgx ? (lin / lgx) % lgy : swap_xy ? blockIdx.x : blockIdx.y,\n"
+      << "                  pidz = lgx ? lin / ((long long)lgx * lgy) : blockIdx.z;\n"
+      << "  const long long npx = lgx ? lgx : swap_xy ? gridDim.y : gridDim.x, npy = lgx ? lgy : swap_xy ? gridDim.x : gridDim.y, npz = lgx ? lgz : gridDim.z;\n"
+      << "  (void)pidx; (void)pidy; (void)pidz; (void)npx; (void)npy; (void)npz;\n"
+      << g.os.str() << "}\n";
   for (int b : g.all_inline_bases)
     if (g.all_store_bases.count(b))
       throw Unsupported("tile_program: an argument is both stored to and read by a load that is not of its body's block shape");
