@@ -2472,6 +2472,20 @@ def test_tile_program_wide_groups_that_the_extent_cuts_off(dtype, n_cols):
     assert (z[:, n_cols:] == 55).all() and (y[:, n_cols:] == 55).all()
 
 
+@pytest.mark.parametrize("BR,BC", [(4, 4096), (8, 1024), (16, 512), (2, 8192)])
+def test_gathered_rows_are_all_read_before_one_is_written(BR, BC):
+    """Blocks of up to 16384 elements run in two phases, also where source and destination are one buffer under two names: a
+    program that permutes its own rows through an index vector is exact."""
+    g = torch.Generator().manual_seed(BC)
+    programs = 40
+    x = torch.randn(programs * BR, BC, generator=g).half().to(DEV)
+    which = torch.cat([BR * p + torch.randperm(BR, generator=g) for p in range(programs)]).int().to(DEV)
+    want = x[which.long()]
+    k = K_mod().take_rows[(programs,)](x, which, x, programs * BR, BC, BC, BC, BR=BR, BC=BC)
+    torch.cuda.synchronize()
+    assert k.function.family == "tile_program" and torch.equal(x, want)
+
+
 @pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
 @pytest.mark.parametrize("n_rows,n_cols,pitch,BR,BC", [(1, 1, 1, 8, 256), (9, 255, 255, 8, 256), (37, 511, 513, 16, 512), (100, 1000, 1000, 4, 1024), (33, 1017, 1021, 2, 1024),
                                                        (10, 2047, 2047, 1, 2048), (21, 4096, 4096, 4, 4096), (21, 4001, 4003, 4, 4096), (7, 7296, 7296, 4, 8192), (18, 8185, 8187, 16, 8192)])

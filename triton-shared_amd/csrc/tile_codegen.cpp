@@ -728,11 +728,11 @@ struct Gen {
   }
   bool gathers_rows = false;  // a program of one run of loads, elementwise ops and stores with such loads, all of one shape
   bool row_gather(const Access &a) const { return gathers_rows && a.gather >= 0 && is16(a.elem) && a.sizes == wide_shape && along_last(a.gather) == UNIT; }
-  // Such a run goes through its block in pieces of 8192 elements (`piece` in the generated source): nothing needs the whole
-  // of it at once, and the loads of a piece are enough in flight.  (Rows of fp16 [4000, 4096], four per program, element by
+  // Blocks that are larger than what runs in two phases go piece by piece, 8192 elements each (`piece` in the generated source):
+  // the loads of a piece are enough in flight.  (Rows of fp16 [4000, 4096], four per program, element by
   // element: 20.1 us, this way 12.4; rows of 7296, whose blocks of 32768 went one element at a time: 35.2 us for 275 of them, now 8.2.)
   static constexpr int64_t PIECE = 8192, GATHER_MAX = 1 << 20;
-  bool in_pieces(const std::vector<int64_t> &shape) const { return gathers_rows && wide(shape) && count(shape) > PIECE; }
+  bool in_pieces(const std::vector<int64_t> &shape) const { return gathers_rows && wide(shape) && count(shape) > TWO_PHASE_MAX; }
   int64_t held_count(const std::vector<int64_t> &shape) const { return in_pieces(shape) ? PIECE : count(shape); }
   void choose_row_gathers() {
     std::vector<int64_t> sh;
@@ -1545,7 +1545,7 @@ struct Gen {
           row_vectors[o->result] = name;
         }
         row_loads.clear();
-        if (any_load && !(column_sums && loop_depth) && !gathers_rows) os << pad() << "__syncthreads();\n";
+        if (any_load && !(column_sums && loop_depth) && !in_pieces(shape)) os << pad() << "__syncthreads();\n";
         if (stores && wide(shape))  // wide stores collect a group's eight values (see the Store case below)
           for (size_t q = k; q < end; q++)
             if (ops[q].kind == SK::Store && vector_access(ops[q].acc)) os << pad() << "unsigned sv" << q << "[8];\n";
@@ -1626,7 +1626,7 @@ struct Gen {
           }
         }
         close_loop();
-        if (!gathers_rows) os << pad() << "__syncthreads();\n";
+        if (!in_pieces(shape)) os << pad() << "__syncthreads();\n";
       }
       if (pieces) close_loop();
       // values named inside the loop end with it (a load of a two-phase run stays in its registers)
