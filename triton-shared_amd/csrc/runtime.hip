@@ -829,7 +829,8 @@ tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, con
       a.swap_xy = tile_program_swaps_grid(source) && gy > 1 && gx <= 65535 ? 1 : 0;
       // A workgroup per program.  (A few workgroups per CU that walk the programs with the weights they share held in
       // registers lose since every row moves in 16-byte accesses, us walking / a workgroup each: LayerNorm's dx bf16 [8192, 4096]
-      // 54.3 / 42.8, [8192, 2048] 32.4 / 24.4, [8192, 3001] 57.8 / 45.3; RMSNorm fp16 [4000, 8192] 23.9 / 22.7, [8000, 5120] 40.5 / 35.0.)
+      // 54.3 / 42.8, [8192, 2048] 32.4 / 24.4, [8192, 3001] 57.8 / 45.3; RMSNorm fp16 [8000, 5120] 40.5 / 35.0, [8000, 4096]
+      // from HBM 29.0 / 26.4; ahead only on few whole rows of 8192 from HBM, RMSNorm [4096, 8192] 26.6 / 27.8.)
       if ((a.swap_xy ? gx : gy) > 65535 || gz > 65535) {  // the kernel numbers the programs itself (x fastest)
         a.swap_xy = 0;
         a.lgx = gx; a.lgy = gy; a.lgz = gz;
