@@ -358,6 +358,22 @@ def test_gemm_whole_tile_kernel(K, M, N, Kd, dtype, pad):
     assert torch.equal(c.cpu(), -a.cpu()[:, perm])
 
 
+@pytest.mark.parametrize("M,N,Kd,at,bt", [(976, 1984, 2816, False, False), (752, 2368, 2560, False, True), (1504, 3072, 4096, True, True), (888, 1920, 3136, True, False)])
+def test_gemm_that_fills_half_a_round_runs_in_k_slices(K, M, N, Kd, at, bt):
+    """Products whose tiles fill about half of a round of workgroups are ahead in K slices, whichever way the operands lie.  Small
+    integers: exact in any order."""
+    g = torch.Generator().manual_seed(M)
+    A = torch.randint(-1, 2, (Kd, M) if at else (M, Kd), generator=g).half().to(DEV)
+    B = torch.randint(-1, 2, (N, Kd) if bt else (Kd, N), generator=g).half().to(DEV)
+    a, b = (A.t() if at else A), (B.t() if bt else B)
+    c = torch.full((M + 1, N), 7.0, dtype=torch.float16, device=DEV)
+    k = K.matmul_tiles[(triton.cdiv(M, 128) * triton.cdiv(N, 128),)](a, b, c, M, N, Kd, a.stride(0), a.stride(1), b.stride(0), b.stride(1), N, 1, BM=128, BN=128, BK=64, GROUP_M=8)
+    torch.cuda.synchronize()
+    assert k.function.last_kernel.endswith("K slices"), k.function.last_kernel
+    want = a.float() @ b.float()  # |sums| < 2048
+    assert torch.equal(c[:M].float(), want) and (c[M] == 7).all()
+
+
 @pytest.mark.parametrize("M,N,Kd,dtype,bt", [(128, 4096, 4096, torch.bfloat16, False), (300, 1032, 2048, torch.float16, False), (512, 2048, 8192, torch.bfloat16, True),
                                             (1000, 2048, 4096, torch.bfloat16, False), (64, 8192, 8192, torch.float16, False), (1, 256, 4096, torch.bfloat16, False),
                                             (512, 8192, 8192, torch.bfloat16, False), (500, 4104, 8192, torch.float16, False), (768, 2048, 16384, torch.bfloat16, False)])

@@ -849,10 +849,10 @@ constexpr int W8_WAVES = 16;
 namespace {
 // Which direct-to-LDS tile a product runs on (null: none applies), and in how many K slices.
 // first, more, fixed: us per K tile of a round of workgroups that is all but empty, what a full round adds to it, and per launch,
-// fitted to the table at unsliced_time.
+// fitted at `time` below.
 struct DmaCand { const char *tag; int64_t bm, bn; double eff, first, more, fixed; };
-const DmaCand DMA_CANDS[4] = {{"256x256", 256, 256, 1.0, 0.53, 0.25, 8}, {"128x256", 128, 256, 0.77, 0.33, 0.15, 9},
-                              {"256x128", 256, 128, 0.73, 0.36, 0.16, 9}, {"128x128", 128, 128, 0.59, 0.22, 0.07, 8}};
+const DmaCand DMA_CANDS[4] = {{"256x256", 256, 256, 1.0, 0.57, 0.16, 8}, {"128x256", 128, 256, 0.77, 0.41, 0.15, 5},
+                              {"256x128", 256, 128, 0.73, 0.42, 0.15, 5}, {"128x128", 128, 128, 0.59, 0.29, 0.07, 3}};
 struct DmaChoice { const DmaCand *tile = nullptr; int split = 1; };
 
 DmaChoice choose_dma(const GemmParams &p, int max_split) {
@@ -868,57 +868,45 @@ DmaChoice choose_dma(const GemmParams &p, int max_split) {
   // 800 210 / 210).  A few tiles over one round count as one: blocks of rows that pad the last matrix have nothing to do.
   const bool grouped = p.b_block != nullptr && !p.b_trans;
   auto grouped_wide = [&](int64_t t) { return 2 * t >= cus && !(10 * t > 11 * cus && 10 * t < 16 * cus); };
-  // The other products: the least modelled time without slices.  What decides is whole rounds of workgroups over the chip (the
-  // 128 x 128 tile's two workgroups per CU blur them), and that a round runs faster the emptier it is.  Measured, us with 256 x 256
-  // / 128 x 256 / 128 x 128 tiles: 3500 x 4096 x 4096 101 / 132 / 147; 3000 x 4096 x 2048 50.5 / 67.6 / 65.9; 3000 x 2048 x 4096 80.8 / 61.1 /
-  // 68.2; 4096 x 2048 x 2048 48 / 39 / 45; 2500 x 2048 x 1024 25.7 / 18.3 / 20.8; 2048^3 42.3 / 28.2 / 21.7; 1024 x 1024 x 4096 74 / 49 / 33.
-  // (By the rule of short K below, the first two ran at 131 and 68 us.)  Below K = 512 the fixed costs decide and the tiles measure
-  // alike: among the tiles that give every CU a workgroup (128 x 128: always) the one with the least padded work per unit of
-  // the tile's measured efficiency at 4096^3 (105 / 136 / 144 / 179 us).
+  // The other products: the least modelled time.  What decides is whole rounds of workgroups over the chip (the 128 x 128 tile's two
+  // workgroups per CU blur them), and that a round runs faster the emptier it is.  Few tiles (a skinny product, M = 128 ... 1024
+  // against N, K in the thousands) leave CUs idle while every workgroup walks all of K alone: K is then cut into slices, whose fp32
+  // sums a second kernel adds, and whose workgroups count in rounds like any others.
+  // Fitted to 130 products from HBM (M 128 ... 4200, N to 4200, K 512 ... 8300, each operand row- or column-major, batches of 2 to 12)
+  // on every tile in 1 to 16 slices: a scatter of 7 % with slices, 8 to 11 % without, and the choice is 2.4 % behind the best of
+  // each.  us on 256 x 256 / 128 x 256 / 128 x 128 tiles: 3000 x 4096 x 2048 50.5 / 67.6 / 65.9; 3000 x 2048 x 4096 80.8 / 61.1 / 68.2;
+  // 2048^3 42.3 / 28.2 / 21.7; in 1 / 2 / 3 / 4 slices: 1504 x 3072 x 4096 on 256 x 256 84 / 64 / 56 / 79 (the fourth begins a second
+  // round), 976 x 1984 x 2816 on 128 x 128 33.7 / 27.0 / 33.3 / 31.0, 464 x 4160 x 6016 on 128 x 256 87 / 57 / 48 / 68.
+  // Below K = 512 the fixed costs decide and the tiles measure alike: among the tiles that give every CU a workgroup (128 x 128:
+  // always) the one with the least padded work per unit of the tile's measured efficiency at 4096^3 (105 / 136 / 144 / 179 us).
   const bool by_rounds = !grouped && p.K >= 512;
-  auto unsliced_time = [&](const DmaCand &c) {
-    const double f = (double)tiles(c) / cus, whole = std::floor(f), rest = f - whole;
+  const int64_t nk = p.K / F_BK;
+  const double sums = (double)p.M * (double)p.N * std::max(1, p.batches) * 4;  // bytes of one slice's
+  auto time = [&](const DmaCand &c, int split) {
+    const double f = (double)tiles(c) * split / cus, whole = std::floor(f), rest = f - whole;
     double rounds = whole * (c.first + c.more) + (rest > 0 ? c.first + c.more * rest : 0);
     if (c.bm + c.bn == 256 && f > 1) rounds = (c.first + c.more) * 0.5 * (f + std::ceil(f));
-    return (rounds * (double)(p.K / F_BK) + c.fixed) * 1e-6;
+    return rounds * (double)((nk + split - 1) / split) + c.fixed + (split > 1 ? 4.4 + split * sums / 2.9e6 : 0);
   };
   DmaChoice best;
   double best_cost = 0;
   for (const DmaCand &c : DMA_CANDS) {
     if (!gemm_dma_ok(p, c.bm, c.bn)) continue;
     if (dma_env ? std::string(dma_env) != c.tag : !by_rounds && c.bm + c.bn != 256 && (grouped ? !grouped_wide(tiles(c)) : tiles(c) < cus)) continue;
-    const double cost = by_rounds ? unsliced_time(c) : (double)(tiles(c) * c.bm * c.bn) / c.eff;
+    const double cost = by_rounds ? time(c, 1) : (double)(tiles(c) * c.bm * c.bn) / c.eff;
     if (!best.tile || cost < best_cost) { best.tile = &c; best_cost = cost; }
   }
-  if (!best.tile || max_split < 2 || p.a_rows || p.b_block) return best;
-  // Too few tiles for the chip (a skinny product: M = 128 ... 1024 against N, K in the thousands): every workgroup then walks
-  // all of K alone, at the pace one workgroup streams its operands, and the launch takes as long as with a fraction of
-  // its rows -- 4096 x 4096 weights took 50 us at M = 128, 256, 512 and 1024 alike.  K is cut into slices so that about
-  // every CU has a workgroup; each slice leaves fp32 sums that a second kernel adds.  Modelled time: the K tiles a
-  // workgroup walks at the tile's measured time per K tile (times the rounds of workgroups the chip needs), the launch's
-  // fixed cost, and the partial sums' way through memory (measured: 512 x 8192 x 8192 in four slices of 256 x 256 tiles
-  // 79 us for a model of 82; 512 x 4096 x 4096 in four of 128 x 256 34.5 for 34.5; 128 x 4096 x 4096 in eight of
-  // 128 x 128 20.9 for 22.3).
-  const int64_t nk = p.K / F_BK;
-  auto model = [&](const DmaCand &c, int split) {
-    // per K tile and workgroup with operands from HBM (the 128 x 256 tile: 0.42 us from cache)
-    const double step = c.bm + c.bn == 512 ? 0.80e-6 : c.bm + c.bn == 256 ? 0.39e-6 : c.bm == 128 ? 0.60e-6 : 0.62e-6;
-    const double wgs = (double)tiles(c) * split;
-    double t = std::max(1.0, wgs / cus) * (double)((nk + split - 1) / split) * step + 8e-6;
-    if (split > 1) t += 1.2 * split * (double)p.M * (double)p.N * std::max(1, p.batches) * 4 / 4e12 + 3e-6;
-    return t;
-  };
+  if (!best.tile || max_split < 2 || !by_rounds || p.a_rows || p.b_block) return best;
   DmaChoice pick = best;
-  // (the times without slices were measured on operands that partly sat in the Infinity Cache)
-  double pick_t = by_rounds ? std::min(model(*best.tile, 1), 1.15 * unsliced_time(*best.tile)) : model(*best.tile, 1);
+  double pick_t = 0.95 * best_cost;  // (a second launch has to be worth it by more than the model errs for it)
   if (!(split_env && atoi(split_env) == 1))
     for (const DmaCand &c : DMA_CANDS) {
       if (!gemm_dma_ok(p, c.bm, c.bn) || (dma_env && std::string(dma_env) != c.tag)) continue;
       const int64_t most = std::min<int64_t>(std::min<int64_t>(std::min<int64_t>(16, max_split), nk / 8), (2 * cus + tiles(c) - 1) / tiles(c));
       for (int64_t sp = split_env ? atoi(split_env) : 2; sp <= most; sp++) {
-        if ((size_t)sp * p.M * p.N * std::max(1, p.batches) * 4 > ((size_t)256 << 20)) break;
-        const double t = model(c, (int)sp);
-        if (t < 0.9 * pick_t || (pick.split > 1 && t < pick_t)) { pick.tile = &c; pick.split = (int)sp; pick_t = t; }
+        if (sp * sums > (double)((size_t)256 << 20)) break;
+        const double t = time(c, (int)sp);
+        if (t < pick_t || (split_env && pick.split == 1)) { pick.tile = &c; pick.split = (int)sp; pick_t = t; }
         if (split_env) break;
       }
     }
