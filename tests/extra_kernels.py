@@ -1648,3 +1648,16 @@ def take_rows_scaled(src_ptr, rows_ptr, s_ptr, add_ptr, dst_ptr, n_rows, n_cols,
     x = tl.load(src_ptr + which[:, None] * pitch + c[None, :], mask=m, other=3.0).to(tl.float32)
     a = tl.load(add_ptr + r[:, None] * pitch + c[None, :], mask=m, other=0.0)
     tl.store(dst_ptr + r[:, None] * pitch + c[None, :], (x * s[:, None] + a).to(dst_ptr.dtype.element_ty), mask=m)
+
+
+@triton.jit
+def rms_norm_weight_bias_rows(x_ptr, w_ptr, b_ptr, y_ptr, pitch, n_cols, n_bias, eps, BLOCK: tl.constexpr):
+    """y = x / sqrt(mean(x^2) + eps) * w + b, a row per program; w and b are loaded after the mean, b has an extent of its own."""
+    row = tl.program_id(0)
+    c = tl.arange(0, BLOCK)
+    m = c < n_cols
+    x = tl.load(x_ptr + row * pitch + c, mask=m, other=0.0).to(tl.float32)
+    ms = tl.sum(x * x, axis=0) / n_cols
+    w = tl.load(w_ptr + c, mask=m, other=0.0).to(tl.float32)
+    b = tl.load(b_ptr + c, mask=c < n_bias, other=0.5).to(tl.float32)
+    tl.store(y_ptr + row * pitch + c, (x * tl.rsqrt(ms + eps) * w + b).to(y_ptr.dtype.element_ty), mask=m)

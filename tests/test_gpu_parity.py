@@ -2374,6 +2374,35 @@ def test_tile_program_wide_blocks_of_rows_loops_and_mixed_widths():
             assert torch.equal(ki[lead:lead + n], torch.where(xs.float() > 0, o, -o)) and (ki[lead + n:] == 5).all()
 
 
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("n_cols,n_bias,block", [(1, 1, 2048), (7, 7, 2048), (8, 3, 2048), (9, 2048, 2048), (2047, 2047, 2048), (4001, 4001, 4096), (4096, 5, 4096), (8191, 8191, 8192),
+                                                 (8192, 8192, 8192), (8192, 0, 8192), (16384, 16384, 16384), (12001, 12001, 16384)])
+def test_rows_of_weights_loaded_behind_the_row(dtype, n_cols, n_bias, block):
+    """Rows of weights that a program loads after a row's reduction are read beside the row where their extents allow the same
+    accesses (8192-wide blocks: two of them; 16384-wide ones: after the reduction): every mix of extents, off the 16-byte grid."""
+    import extra_kernels as X
+    torch.manual_seed(n_cols + n_bias)
+    dt, rows, pitch = getattr(torch, dtype), 5, n_cols + 3
+    buf = torch.full((1 + rows * pitch,), 7.0, device=DEV, dtype=dt)
+    x = buf[1:].view(rows, pitch)[:, :n_cols]
+    x.copy_(torch.randn(rows, n_cols, device=DEV))
+    w = (1 + 0.1 * torch.randn(n_cols + 1, device=DEV)).to(dt)[1:]
+    b = torch.randn(max(n_bias, 1), device=DEV).to(dt)
+    yb = torch.full((rows * pitch,), 55.0, device=DEV, dtype=dt)
+    k = X.rms_norm_weight_bias_rows[(rows,)](x, w, b, yb, pitch, n_cols, n_bias, 1e-6, BLOCK=block)
+    torch.cuda.synchronize()
+    assert k.function.family == "tile_program"
+    xd, bd = x.double(), torch.full((n_cols,), 0.5, device=DEV, dtype=torch.float64)
+    bd[:min(n_bias, n_cols)] = b[:min(n_bias, n_cols)].double()
+    xw = xd / torch.sqrt((xd * xd).mean(1, keepdim=True) + 1e-6) * w.double()
+    # fp32: the sum of squares rounds at most 64 + 8 times, the rest six times, of terms of at most |x w| + |b|; then the store's rounding
+    half_ulp = 2.0 ** (-8 if dtype == "bfloat16" else -11)  # 7 and 10 fraction bits: an ulp is at most 2^-7 and 2^-10 of the value
+    bound = half_ulp * (xw + bd).abs() + 80 * 2.0 ** -24 * (xw.abs() + bd.abs()) + 2.0 ** -25
+    y = yb.view(rows, pitch)
+    assert ((y[:, :n_cols].double() - (xw + bd)).abs() <= bound).all()
+    assert (y[:, n_cols:] == 55).all()
+
+
 def test_tile_program_persistent_programs_walk_the_whole_grid():
     """A program whose block of weights is the same for every program runs as a loop over programs in a launch of a few
     workgroups per CU: more programs than such a launch has workgroups, on one- and two-dimensional grids."""

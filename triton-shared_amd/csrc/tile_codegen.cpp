@@ -791,6 +791,45 @@ struct Gen {
     wide_mode = true;
     wide_shape = best;
   }
+  // Whether the extents of these wide loads all leave eight elements to read, or none: the condition as source, the same in
+  // every thread (empty: none of them is masked).
+  std::string leaves_eight(const std::vector<const SOp *> &loads) {
+    std::string text;
+    std::set<std::string> seen;
+    for (const SOp *o : loads)
+      if (!o->acc.dims.empty()) {
+        const std::string ext = "(" + ex(o->acc.dims.back()) + ")";
+        if (seen.insert(ext).second) text += std::string(text.empty() ? "" : " && ") + "(" + ext + " <= 0 || " + ext + " >= 8)";
+      }
+    return text;
+  }
+  // Loads that the run after the next reduction makes of a block laid out like this run's -- the row of weights of a
+  // normalisation -- are issued behind this run's and wait, packed, in `ahead` registers (32 of them at most): made where they
+  // stand, after the reduction, their way from L2 is added to the row's from memory.  RMSNorm fp16 from HBM, us after / behind:
+  // [4096, 8192] 28.5 / 26.0, [2000, 8192] 15.5 / 14.9, [8000, 5120] 35.9 / 34.5, [8000, 4096] 26.5 / 25.3, [16000, 2048] 31.0 / 28.1.
+  std::set<int> loaded_ahead;
+  std::vector<const SOp *> loads_of_next_run(const std::vector<SOp> &ops, size_t from, const std::vector<int64_t> &shape, const std::string &roomy) {
+    std::vector<const SOp *> loads, none;
+    bool reduced = false;
+    size_t q = from;
+    for (; q < ops.size(); q++) {
+      const SK k = ops[q].kind;
+      if (k == SK::Reduce && !loads.empty()) break;
+      reduced = reduced || k == SK::Reduce;
+      if (k == SK::Store || k == SK::ScalarStore || k == SK::For || k == SK::If || k == SK::Scan || k == SK::Dot || k == SK::ScalarLoad) break;
+      if (k == SK::Load && reduced && wide(ops[q].acc.sizes) && ops[q].acc.sizes == shape && vector_access(ops[q].acc)) loads.push_back(&ops[q]);
+    }
+    if (loads.empty() || held_count(shape) / 2048 * (int64_t)loads.size() > 8 || leaves_eight(loads) != roomy) return none;
+    for (const SOp *o : loads) {
+      std::vector<int> es = o->acc.offsets;
+      es.insert(es.end(), o->acc.strides.begin(), o->acc.strides.end());
+      es.insert(es.end(), o->acc.dims.begin(), o->acc.dims.end());
+      for (int e : es)
+        if (e >= 0 && P.pool.depends_on(e, EK::Data)) return none;
+      if (!is16(o->acc.elem) || scalar_store_bases_anywhere.count(o->acc.base_arg)) return none;
+    }
+    return loads;
+  }
   // (i0, i1) moved by `delta` along the contiguous dimension: called once with i0 (use .first) and once with i1 (.second)
   static std::pair<std::string, std::string> along(const std::vector<int64_t> &shape, const std::string &i, const std::string &delta) {
     return {shape.size() < 2 ? "(" + i + delta + ")" : i, shape.size() < 2 ? i : "(" + i + delta + ")"};
@@ -1337,17 +1376,15 @@ struct Gen {
           // sits between the loads, so none waits for another.  Only a program whose extent is one to seven elements loads
           // element by element, as it would in the ordinary order.
           auto wide_load = [&](const SOp &o) { return wide(ls) && mine_here(o) && vector_access(o.acc); };
-          bool any_wide = false;
-          for (size_t q = k; q < end; q++) any_wide = any_wide || wide_load(ops[q]);
-          if (any_wide) {
+          std::vector<const SOp *> wide_loads;
+          for (size_t q = k; q < end; q++)
+            if (wide_load(ops[q])) wide_loads.push_back(&ops[q]);
+          if (!wide_loads.empty()) {
             const int64_t G = held_count(ls) / 2048;
             uses_dummy = true;
-            std::string roomy;  // the extents of the masked ones leave eight elements to read, or none (the same in every thread)
-            for (size_t q = k; q < end; q++)
-              if (wide_load(ops[q]) && !ops[q].acc.dims.empty()) {
-                const std::string ext = "(" + ex(ops[q].acc.dims.back()) + ")";
-                if (roomy.find(ext) == std::string::npos) roomy += std::string(roomy.empty() ? "" : " && ") + "(" + ext + " <= 0 || " + ext + " >= 8)";
-              }
+            const std::string roomy = leaves_eight(wide_loads);
+            const std::vector<const SOp *> ahead = stores || loop_depth ? std::vector<const SOp *>() : loads_of_next_run(ops, end, ls, roomy);
+            for (const SOp *o : ahead) os << pad() << "u32x4_t ahead" << o->result << "[" << G << "];\n";
             os << pad() << "if (" << (roomy.empty() ? "true" : roomy) << ") {\n";
             indent++;
             for (size_t q = k; q < end; q++)
@@ -1356,26 +1393,40 @@ struct Gen {
             os << pad() << "#pragma unroll\n" << pad() << "for (int g = 0; g < " << G << "; g++) {\n";
             indent++;
             os << pad() << "const int n = 8 * g;\n" << pad() << "const int t = " << element_of_slot(ls) << ";\n";
-            for (size_t q = k; q < end; q++)
-              if (wide_load(ops[q])) {
-                const SOp &o = ops[q];
-                const std::string id = std::to_string(o.result), mt = memtype(o.acc.elem);
-                std::string pred, addr = address(o.acc, l0, l1, pred);
-                os << pad() << "{\n";
-                indent++;
-                const std::string vt = mem_bytes(o.acc.elem) == 1 ? "u32x2_any" : "u32x4_any";
-                if (pred.empty())
-                  os << pad() << "const " << vt << " *const src = (const " << vt << " *)((const " << mt << " *)p.ptr[" << o.acc.base_arg << "] + (" << addr << "));\n";
-                else
-                  os << pad() << "const " << vt << " *const src = !(" << pred << ") ? (const " << vt << " *)tts_dummy : (const " << vt << " *)((const " << mt << " *)p.ptr["
-                     << o.acc.base_arg << "] + (" << addr << ") - " << cut_off(o.acc, ls.size() < 2 ? l0 : l1) << ");\n";
-                if (mem_bytes(o.acc.elem) <= 2) os << pad() << "rw" << id << "[g] = src[0];\n";
-                else os << pad() << "rw" << id << "[2 * g] = src[0];\n" << pad() << "rw" << id << "[2 * g + 1] = src[1];\n";
-                indent--;
-                os << pad() << "}\n";
-              }
+            auto read_group = [&](const SOp &o, const std::string &into) {
+              const std::string mt = memtype(o.acc.elem);
+              std::string pred, addr = address(o.acc, l0, l1, pred);
+              os << pad() << "{\n";
+              indent++;
+              const std::string vt = mem_bytes(o.acc.elem) == 1 ? "u32x2_any" : "u32x4_any";
+              if (pred.empty())
+                os << pad() << "const " << vt << " *const src = (const " << vt << " *)((const " << mt << " *)p.ptr[" << o.acc.base_arg << "] + (" << addr << "));\n";
+              else
+                os << pad() << "const " << vt << " *const src = !(" << pred << ") ? (const " << vt << " *)tts_dummy : (const " << vt << " *)((const " << mt << " *)p.ptr["
+                   << o.acc.base_arg << "] + (" << addr << ") - " << cut_off(o.acc, ls.size() < 2 ? l0 : l1) << ");\n";
+              if (mem_bytes(o.acc.elem) <= 2) os << pad() << into << "[g] = src[0];\n";
+              else os << pad() << into << "[2 * g] = src[0];\n" << pad() << into << "[2 * g + 1] = src[1];\n";
+              indent--;
+              os << pad() << "}\n";
+            };
+            for (const SOp *o : wide_loads) {
+              const std::string id = std::to_string(o->result);
+              if (loaded_ahead.count(o->result)) os << pad() << "rw" << id << "[g] = ahead" << id << "[g];\n";
+              else read_group(*o, "rw" + id);
+            }
             indent--;
             os << pad() << "}\n";
+            if (!ahead.empty()) {
+              os << pad() << "#pragma unroll\n" << pad() << "for (int g = 0; g < " << G << "; g++) {\n";
+              indent++;
+              os << pad() << "const int n = 8 * g;\n" << pad() << "const int t = " << element_of_slot(ls) << ";\n";
+              for (const SOp *o : ahead) {
+                read_group(*o, "ahead" + std::to_string(o->result));
+                loaded_ahead.insert(o->result);
+              }
+              indent--;
+              os << pad() << "}\n";
+            }
             for (size_t q = k; q < end; q++)
               if (wide_load(ops[q]) && !ops[q].acc.dims.empty()) {
                 const SOp &o = ops[q];
