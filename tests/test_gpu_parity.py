@@ -2403,6 +2403,22 @@ def test_rows_of_weights_loaded_behind_the_row(dtype, n_cols, n_bias, block):
     assert (y[:, n_cols:] == 55).all()
 
 
+@pytest.mark.parametrize("grid", [((1 << 23) + 3, 1, 1), ((1 << 24) + 5, 1, 1), (3, 70000, 40), (1, (1 << 23) + 1, 1)])
+def test_tile_program_on_more_programs_than_a_grid_holds_along_x(grid):
+    """A grid holds 2^32 - 1 threads along x, a workgroup has 256: launches of 2^24 programs and more continue along y."""
+    import extra_kernels as X
+    programs, n = grid[0] * grid[1] * grid[2], 8
+    x = torch.randn(programs, n, device=DEV).half()
+    w = torch.randn(n, device=DEV).half()
+    y = torch.zeros_like(x)
+    k = X.scale_rows_of_a_3d_grid[grid](x, w, y, n, BLOCK=2048)
+    torch.cuda.synchronize()
+    assert k.function.family == "tile_program"
+    for part in range(0, programs, 1 << 22):
+        at = slice(part, part + (1 << 22))
+        assert torch.equal(y[at], (x[at].float() * w.float()).half())
+
+
 def test_tile_program_persistent_programs_walk_the_whole_grid():
     """A program whose block of weights is the same for every program runs as a loop over programs in a launch of a few
     workgroups per CU: more programs than such a launch has workgroups, on one- and two-dimensional grids."""

@@ -778,6 +778,14 @@ tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, con
         }
       }
       kname = "tile_program (hipRTC)";
+      // A grid holds 2^32 - 1 threads along x and 65535 workgroups along y and z.  Launches beyond that are one-dimensional and the
+      // kernel numbers the programs itself (x fastest), along y from 2^23 workgroups on, where surplus ones find no program.
+      constexpr int64_t MOST_ALONG_X = 1 << 23;
+      auto grid_fits = [&](bool swapped) { return (swapped ? gy : gx) <= MOST_ALONG_X && (swapped ? gx : gy) <= 65535 && gz <= 65535; };
+      auto launch_numbered = [&](int64_t workgroups, void *arguments, size_t size) {
+        const int64_t along_x = std::min(workgroups, MOST_ALONG_X);
+        return rtc_launch(*slot, (int)along_x, (int)((workgroups + along_x - 1) / along_x), 1, 256, arguments, size, s);
+      };
       int per_group = 1, group_axis = -1, group_threads = 256;
       if (tile_program_is_matrix(source, &per_group, &group_axis, &group_threads)) {  // a one-dimensional launch that numbers the programs itself
         kname = "tile_program (hipRTC, matrix layout)";
@@ -814,7 +822,7 @@ tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, con
         }
         // one slice: the grid as it is, a workgroup per program, its x and y exchanged where the program asks for that (see below)
         const bool whole = sa.slices == 1, swap = whole && tile_program_swaps_grid(source) && gy > 1 && gx <= 65535;
-        if (whole && (swap ? gx : gy) <= 65535 && gz <= 65535) {
+        if (whole && grid_fits(swap)) {
           a.swap_xy = swap ? 1 : 0;
           sa.t = a;
           err = swap ? rtc_launch(*slot, gy, gx, gz, 256, &sa, sizeof sa, s) : rtc_launch(*slot, gx, gy, gz, 256, &sa, sizeof sa, s);
@@ -822,7 +830,7 @@ tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, con
         }
         a.lgx = gx; a.lgy = gy; a.lgz = gz;
         sa.t = a;
-        err = rtc_launch(*slot, (int)(programs * sa.slices), 1, 1, 256, &sa, sizeof sa, s);
+        err = launch_numbered(programs * sa.slices, &sa, sizeof sa);
         return TTS_OK;
       }
       // the program asks for neighbouring workgroups along program_id(1) (tile_codegen.cpp); grid.y holds 65535 at most
@@ -831,10 +839,10 @@ tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, con
       // registers lose since every row moves in 16-byte accesses, us walking / a workgroup each: LayerNorm's dx bf16 [8192, 4096]
       // 54.3 / 42.8, [8192, 2048] 32.4 / 24.4, [8192, 3001] 57.8 / 45.3; RMSNorm fp16 [8000, 5120] 40.5 / 35.0, [8000, 4096]
       // from HBM 29.0 / 26.4; ahead only on few whole rows of 8192 from HBM, RMSNorm [4096, 8192] 26.6 / 27.8.)
-      if ((a.swap_xy ? gx : gy) > 65535 || gz > 65535) {  // the kernel numbers the programs itself (x fastest)
+      if (!grid_fits(a.swap_xy)) {
         a.swap_xy = 0;
         a.lgx = gx; a.lgy = gy; a.lgz = gz;
-        err = rtc_launch(*slot, (int)((int64_t)gx * gy * gz), 1, 1, 256, &a, sizeof a, s);
+        err = launch_numbered((int64_t)gx * gy * gz, &a, sizeof a);
       } else {
         err = a.swap_xy ? rtc_launch(*slot, gy, gx, gz, 256, &a, sizeof a, s) : rtc_launch(*slot, gx, gy, gz, 256, &a, sizeof a, s);
       }

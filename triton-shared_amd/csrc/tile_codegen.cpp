@@ -2604,8 +2604,11 @@ std::string tile_program_source(const Program &p) {
   all << g.decl.str();
   // sliced: the launch is one-dimensional, the slices of a program lie gridDim.x / slices workgroups apart, so that
   // workgroups that run at the same time read neighbouring blocks
-  if (g.sliced) all << "  const int programs = (int)gridDim.x / slices, slice = (int)blockIdx.x / programs;\n  const long long lin = blockIdx.x - slice * programs;\n";
-  else all << "  const long long lin = blockIdx.x;\n";
+  // numbered launches continue along y (one slice only: others have as many workgroups as the device holds)
+  const std::string rows_before = " + (lgx ? (long long)gridDim.x * blockIdx.y : 0)";
+  if (g.sliced) all << "  const int programs = (int)gridDim.x / slices, slice = (int)blockIdx.x / programs;\n  const long long lin = blockIdx.x - slice * programs" << rows_before << ";\n";
+  else all << "  const long long lin = blockIdx.x" << rows_before << ";\n";
+  all << "  if (lgx && lin >= (long long)lgx * lgy * lgz) return;\n";
   all << "  const long long pidx = lgx ? lin % lgx : swap_xy ? blockIdx.y : blockIdx.x, pidy = lgx ? (lin / lgx) % lgy : swap_xy ? blockIdx.x : blockIdx.y,\n"
       << "                  pidz = lgx ? lin / ((long long)lgx * lgy) : blockIdx.z;\n"
       << "  const long long npx = lgx ? lgx : swap_xy ? gridDim.y : gridDim.x, npy = lgx ? lgy : swap_xy ? gridDim.x : gridDim.y, npz = lgx ? lgz : gridDim.z;\n"
