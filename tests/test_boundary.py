@@ -6,6 +6,8 @@ reference launcher does (driver.py:140-223).  Nothing here launches a kernel."""
 import ctypes
 import os
 import re
+import subprocess
+import sys
 
 import pytest
 
@@ -131,6 +133,26 @@ def test_missing_extension_fails_loudly(monkeypatch):
     monkeypatch.setattr(tsa._native, "LIB_PATH", "/nonexistent/libtts_hip.so")
     with pytest.raises(RuntimeError, match="has not been built"):
         tsa.HIPDriver()
+
+
+def test_planning_needs_neither_torch_nor_triton_nor_the_launch_extension():
+    # the binding alone, in a process where those three cannot be imported
+    code = f"""
+import importlib.util, os, sys
+for name in ("torch", "triton"):
+    sys.modules[name] = None
+spec = importlib.util.spec_from_file_location("binding", {os.path.join(ROOT, "triton-shared_amd", "_native.py")!r})
+n = importlib.util.module_from_spec(spec)
+spec.loader.exec_module(n)
+n.LAUNCH_PATH = "/nonexistent"
+structured = n.ttir_to_structured(open({os.path.join(ROOT, "tests", "golden", "vec_add.ttir")!r}).read())
+plan, name = n.structured_to_plan(structured)
+assert name == "vec_add" and n.PlanHandle(plan).family == "map1d"
+n.connect_launches()
+assert n.launcher_base() is n._GeneralLauncher
+"""
+    res = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True)
+    assert res.returncode == 0, res.stderr
 
 
 def test_product_does_not_import_the_oracle():

@@ -4,6 +4,7 @@ import importlib.machinery
 import importlib.util
 import os
 import subprocess
+import sys
 
 _CSRC = os.path.join(os.path.dirname(os.path.abspath(__file__)), "csrc")
 LIB_PATH = os.path.join(_CSRC, "libtts_hip.so")
@@ -63,10 +64,6 @@ def lib():
     L.tts_launch.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_void_p,
                              ctypes.POINTER(TtsArg), ctypes.c_int]
     L.tts_launch_noalloc.argtypes = L.tts_launch.argtypes
-    import torch
-    import triton
-    chain = getattr(getattr(triton, "knobs", None), "HookChain", None)
-    launch_module().setup(ctypes.cast(L.tts_launch, ctypes.c_void_p).value, PlanHandle, _raise, torch.Tensor, torch.nn.Parameter, chain)
     _lib = L
     return L
 
@@ -75,11 +72,9 @@ _launch = None
 
 
 def launch_module():
-    """The extension module behind HIPLauncher; fails loudly if it has not been built."""
+    """The extension module behind HIPLauncher, or None where it has not been built."""
     global _launch
-    if _launch is None:
-        if not os.path.exists(LAUNCH_PATH):
-            raise RuntimeError(f"{LAUNCH_PATH} is missing: the launch extension has not been built (run `make -C triton-shared_amd/csrc`)")
+    if _launch is None and os.path.exists(LAUNCH_PATH):
         loader = importlib.machinery.ExtensionFileLoader("tts_launch", LAUNCH_PATH)
         spec = importlib.util.spec_from_file_location("tts_launch", LAUNCH_PATH, loader=loader)
         _launch = importlib.util.module_from_spec(spec)
@@ -87,8 +82,20 @@ def launch_module():
     return _launch
 
 
-class _Unbuilt:
-    """Stands in for the native base in a process that imports the package before it is built: every call is `_generic`."""
+def connect_launches():
+    """Hands the launch extension what it calls and the types that it recognises.  Types of torch and Triton are those of a
+    process that has imported them; until then their objects take the general way, so that planning needs neither."""
+    if launch_module() is None:
+        return
+    torch, triton = sys.modules.get("torch"), sys.modules.get("triton")
+    chain = getattr(getattr(triton, "knobs", None), "HookChain", None)
+    tensor = getattr(torch, "Tensor", None)
+    parameter = getattr(getattr(torch, "nn", None), "Parameter", None)
+    _launch.setup(ctypes.cast(lib().tts_launch, ctypes.c_void_p).value, PlanHandle, _raise, tensor, parameter, chain)
+
+
+class _GeneralLauncher:
+    """Stands in for the native base where that is not built: every call is `_generic`."""
 
     def _bind(self, slots):
         pass
@@ -98,7 +105,8 @@ class _Unbuilt:
 
 
 def launcher_base():
-    return launch_module().Launcher if os.path.exists(LAUNCH_PATH) else _Unbuilt
+    module = launch_module()
+    return module.Launcher if module else _GeneralLauncher
 
 
 def _raise(status):

@@ -76,6 +76,7 @@ class HIPLauncher(_native.launcher_base()):
                 continue
             _ty_to_cpp(ty)
             self.slots.append((i, ty[0] == "*"))
+        _native.connect_launches()
         self._bind(self.slots)
 
     def _generic(self, gridX, gridY, gridZ, stream, function, kernel_metadata, launch_metadata,
