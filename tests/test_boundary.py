@@ -8,6 +8,7 @@ import os
 import re
 import subprocess
 import sys
+import sysconfig
 
 import pytest
 
@@ -153,6 +154,12 @@ assert n.launcher_base() is n._GeneralLauncher
 """
     res = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True)
     assert res.returncode == 0, res.stderr
+
+
+def test_launch_extension_belongs_to_the_python_it_was_built_for():
+    import triton_shared_amd as tsa
+    assert tsa._native.LAUNCH_PATH.endswith("tts_launch" + sysconfig.get_config_var("EXT_SUFFIX"))
+    assert issubclass(tsa.HIPLauncher, tsa._native.launch_module().Launcher)
 
 
 def test_product_does_not_import_the_oracle():

@@ -8,7 +8,8 @@ import sys
 
 _CSRC = os.path.join(os.path.dirname(os.path.abspath(__file__)), "csrc")
 LIB_PATH = os.path.join(_CSRC, "libtts_hip.so")
-LAUNCH_PATH = os.path.join(_CSRC, "tts_launch.so")  # the launcher's base class (csrc/launch_module.cpp)
+# the launcher's base class (csrc/launch_module.cpp), named for the Python that it was built for: another one does not see it
+LAUNCH_PATH = os.path.join(_CSRC, "tts_launch" + importlib.machinery.EXTENSION_SUFFIXES[0])
 
 TTS_OK, TTS_UNSUPPORTED, TTS_INVALID, TTS_HIP_ERROR = 0, 1, 2, 3
 ARG_PTR, ARG_INT, ARG_FLOAT = 0, 1, 2
@@ -24,7 +25,7 @@ class TtsArg(ctypes.Structure):
 
 def build(verbose=False):
     """Compiles the library in-tree with hipcc for gfx950 (cross-compiles without a GPU)."""
-    cmd = ["make", "-C", _CSRC, "-j8", "all"]
+    cmd = ["make", "-C", _CSRC, "-j8", f"PYTHON={sys.executable}", "all"]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError("building libtts_hip.so failed:\n" + res.stdout[-4000:] + res.stderr[-4000:])
@@ -72,7 +73,7 @@ _launch = None
 
 
 def launch_module():
-    """The extension module behind HIPLauncher, or None where it has not been built."""
+    """The extension module behind HIPLauncher, or None where it has not been built for this Python."""
     global _launch
     if _launch is None and os.path.exists(LAUNCH_PATH):
         loader = importlib.machinery.ExtensionFileLoader("tts_launch", LAUNCH_PATH)
@@ -95,7 +96,7 @@ def connect_launches():
 
 
 class _GeneralLauncher:
-    """Stands in for the native base where that is not built: every call is `_generic`."""
+    """Stands in for the native base where that is not built (for this Python): every call is `_generic`."""
 
     def _bind(self, slots):
         pass
