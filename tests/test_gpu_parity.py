@@ -196,6 +196,24 @@ def test_layernorm_shapes(K, oracle_cpu, M, N, dtype):
 @pytest.mark.parametrize("M,N", [(5, 3), (9, 8), (9, 9), (4200, 257), (5, 511), (4200, 513), (1030, 1023), (70, 1025), (1030, 2047), (9, 2049),
                                  (4100, 4095), (4200, 4097), (4100, 6145), (4200, 8190), (6, 9001), (5, 16383)])
 def test_layernorm_rows_at_any_alignment(K, dtype, M, N):
+    check_layernorm_rows(K, dtype, M, N)
+
+
+@pytest.mark.parametrize("dtype,M,N,kernel", [
+    ("float16", 16500, 2047, "layernorm_fwd_persistent_kernel"), ("bfloat16", 16400, 1033, "layernorm_fwd_persistent_kernel"), ("bfloat16", 8200, 4095, "layernorm_fwd_persistent_kernel"),
+    ("float16", 4200, 5001, "layernorm_fwd_persistent_kernel"), ("float32", 16500, 1023, "layernorm_fwd_persistent_kernel"), ("float32", 8200, 2047, "layernorm_fwd_persistent_kernel"),
+    ("float32", 8200, 1030, "layernorm_fwd_persistent_kernel"), ("float32", 4200, 3001, "layernorm_fwd_persistent_kernel"),
+    ("float16", 4200, 257, "layernorm_fwd_kernel<1>, a wavefront per row"), ("bfloat16", 4200, 513, "layernorm_fwd_kernel<2>, a wavefront per row"),
+    ("float32", 1030, 1023, "layernorm_fwd_kernel<4>, a wavefront per row"), ("float16", 70, 1025, "layernorm_fwd_kernel<1>"), ("float32", 9, 2047, "layernorm_fwd_kernel<2>"),
+    ("float32", 9, 2500, "layernorm_fwd_kernel<3>"), ("bfloat16", 9, 8191, "layernorm_fwd_kernel<4>"), ("float32", 9, 6001, "layernorm_fwd_kernel<6>"), ("bfloat16", 9, 9001, "layernorm_fwd_kernel<6>"),
+    ("float16", 5, 16383, "layernorm_fwd_kernel<8>")])
+def test_layernorm_kernel_that_each_size_of_row_reaches(K, dtype, M, N, kernel):
+    """Every number of chunks per thread, on rows that end inside one: workgroups that walk the rows (each wavefront counts the
+    stores that it waits behind), a wavefront per row, a workgroup per row."""
+    assert check_layernorm_rows(K, dtype, M, N) == kernel
+
+
+def check_layernorm_rows(K, dtype, M, N):
     """Rows that start and end anywhere: a wavefront or a workgroup per row, and workgroups that walk the rows.  A sum of N
     terms over T lanes rounds N / T + log2 T times at most; 32 ulp of fp32 for the statistics, one more rounding for y."""
     torch.manual_seed(M + N)
@@ -223,6 +241,7 @@ def test_layernorm_rows_at_any_alignment(K, dtype, M, N):
     keep = torch.ones_like(yb, dtype=torch.bool)
     keep[1:1 + M * pitch].view(M, pitch)[:, :N] = False
     assert (yb[keep] == 5.0).all()
+    return k.function.last_kernel
 
 
 @pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
@@ -523,9 +542,10 @@ def test_gemm_any_shape_kernel_reads_and_writes_only_its_problem(K, M, N, Kd, pa
 
 
 @pytest.mark.parametrize("at,bt", [(False, False), (False, True), (True, False), (True, True)])
-@pytest.mark.parametrize("M,N,Kd", [(8, 8, 8), (64, 9, 9), (65, 127, 63), (63, 129, 65), (129, 200, 129), (9, 333, 320), (1000, 8, 193), (3001, 1031, 71), (7, 300, 100), (300, 7, 100), (300, 100, 7)])
+@pytest.mark.parametrize("M,N,Kd", [(8, 8, 8), (64, 9, 9), (65, 127, 63), (63, 129, 65), (129, 200, 129), (9, 333, 320), (1000, 8, 193), (3001, 1031, 71), (7, 300, 100), (300, 7, 100), (300, 100, 7),
+                                    (2900, 2999, 71), (2900, 2999, 64), (2900, 2999, 7), (2900, 2999, 321)])
 def test_gemm_any_shape_kernel_at_the_ends_of_its_tiles(K, M, N, Kd, at, bt):
-    # tiles of 64 and of 128 rows; a last K tile whose chunks are read from the last eight k (or the last row's last eight
+    # tiles of 64 rows and, for more than one and a half of them per CU, of 128; a last K tile whose chunks are read from the last eight k (or the last row's last eight
     # elements) and put right, operands of exactly eight and of fewer; NaN beside the operands reaches no result.  Small
     # integers: exact in any order
     g = torch.Generator().manual_seed(M + N + Kd)
@@ -539,7 +559,7 @@ def test_gemm_any_shape_kernel_at_the_ends_of_its_tiles(K, M, N, Kd, at, bt):
     cd = torch.full((M + 1, N + 1), 7.0, dtype=torch.bfloat16, device=DEV)
     k = K.matmul_tiles[(triton.cdiv(M, 128) * triton.cdiv(N, 128),)](ad, bd, cd, M, N, Kd, ad.stride(0), ad.stride(1), bd.stride(0), bd.stride(1), N + 1, 1, BM=128, BN=128, BK=64, GROUP_M=8)
     torch.cuda.synchronize()
-    assert k.function.last_kernel.startswith("gemm_mfma_kernel")
+    assert k.function.last_kernel.startswith("gemm_mfma_kernel<128x128x64>" if M == 2900 else "gemm_mfma_kernel<64x128x64>"), k.function.last_kernel
     want = (a.double() @ b.double()).bfloat16()
     assert torch.equal(cd[:M, :N].cpu(), want)
     assert (cd[M] == 7.0).all() and (cd[:, N] == 7.0).all()
@@ -563,7 +583,7 @@ def test_gemm_any_shape_kernel_in_k_slices(K, M, N, Kd, bt, dtype):
             cd = torch.full((M + 1, N + 3), 7.0, dtype=dtype, device=DEV)
             k = K.matmul_tiles[(triton.cdiv(M, 128) * triton.cdiv(N, 128),)](ad, bd, cd, M, N, Kd, Kd, 1, bd.stride(0), bd.stride(1), N + 3, 1, BM=128, BN=128, BK=64, GROUP_M=8)
         torch.cuda.synchronize()
-        assert k.function.last_kernel == "gemm_mfma_kernel<128x128x64>, K slices"
+        assert k.function.last_kernel == "gemm_mfma_kernel<64x128x64>, K slices"
         assert torch.equal(cd[:M, :N].cpu().double(), want) and (cd[M] == 7.0).all() and (cd[:, N:] == 7.0).all()
     bias = torch.randint(-4, 5, (N,), generator=g).float()
     held = torch.randint(-8, 9, (M, N), generator=g).to(dtype)
@@ -571,7 +591,7 @@ def test_gemm_any_shape_kernel_in_k_slices(K, M, N, Kd, bt, dtype):
     c = held.to(DEV)
     k = run(c, ACT=2, bias_ptr=bias.to(DEV))
     torch.cuda.synchronize()
-    assert k.function.last_kernel == "gemm_mfma_kernel<128x128x64> + epilogue (hipRTC), K slices"
+    assert k.function.last_kernel == "gemm_mfma_kernel<64x128x64> + epilogue (hipRTC), K slices"
     assert torch.equal(c.cpu().double(), torch.nn.functional.leaky_relu(want + bias.double(), 0.5))
     c = held.to(DEV)
     run(c, ACT=3)
@@ -2817,14 +2837,15 @@ def test_matmul_with_gathered_rows_on_whole_tiles(case):
     assert torch.equal(c, want)
 
 
-@pytest.mark.parametrize("M,N,K,kernel", [(512, 768, 96, "gemm_dma_kernel + epilogue"), (200, 300, 150, "gemm_mfma_kernel<128x128x64> + epilogue"),
+@pytest.mark.parametrize("M,N,K,kernel", [(512, 768, 96, "gemm_dma_kernel + epilogue"), (200, 300, 150, "gemm_mfma_kernel<64x128x64> + epilogue"),
                                           (521, 776, 96, "gemm_dma_kernel + epilogue"),
-                                          (2100, 2060, 72, "gemm_mfma_kernel<128x128x64> + epilogue")])
+                                          (2100, 2060, 72, "gemm_mfma_kernel<64x128x64> + epilogue"),
+                                          (2900, 2999, 71, "gemm_mfma_kernel<128x128x64> + epilogue")])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_gemm_with_fused_epilogue(M, N, K, kernel, dtype):
     """The tutorial matmul's fused activation (test_matmul.py:98-99, 112-117): ops on the accumulator alone are compiled into
     the epilogue of the matmul kernels.  Operands of -1 / 0 / 1 and a slope of 1/2 make every value exact in 16 bits, so
-    the result must equal leaky_relu(A @ B) bit for bit, on each of the three kernels the launcher chooses from."""
+    the result must equal leaky_relu(A @ B) bit for bit, on each kernel the launcher chooses from."""
     import extra_kernels as X
     g = torch.Generator(device="cpu").manual_seed(M + K)
     a = torch.randint(-1, 2, (M, K), generator=g).to(dtype).to(DEV)

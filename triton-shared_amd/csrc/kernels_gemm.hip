@@ -81,6 +81,13 @@ template <bool BF16, bool SK>
 hipError_t launch_gemm_any(const GemmParams &p, hipStream_t s) {
   return any_rows(p, SK ? p.split : 1) == 64 ? launch_gemm_any_t<BF16, SK, 1>(p, s) : launch_gemm_any_t<BF16, SK, 2>(p, s);
 }
+const char *any_name(int64_t rows, bool functor, bool sliced) {  // of the any-shape kernel in tiles of that height
+  static const char *names[2][2][2] = {{{"gemm_mfma_kernel<128x128x64>", "gemm_mfma_kernel<128x128x64>, K slices"},
+                                        {"gemm_mfma_kernel<128x128x64> + epilogue (hipRTC)", "gemm_mfma_kernel<128x128x64> + epilogue (hipRTC), K slices"}},
+                                       {{"gemm_mfma_kernel<64x128x64>", "gemm_mfma_kernel<64x128x64>, K slices"},
+                                        {"gemm_mfma_kernel<64x128x64> + epilogue (hipRTC)", "gemm_mfma_kernel<64x128x64> + epilogue (hipRTC), K slices"}}};
+  return names[rows == 64][functor][sliced];
+}
 hipError_t launch_gemm_any_slices(const GemmParams &p, hipStream_t s) { return p.is_bf16 ? launch_gemm_any<true, true>(p, s) : launch_gemm_any<false, true>(p, s); }
 
 // PF: a fifth wavefront that touches B's lines ahead of the four that work (gemm_device.h); the accumulators then sit in
@@ -980,15 +987,12 @@ hipError_t launch_gemm(const GemmParams &p, hipStream_t s, const char **name) {
     if (best) TTS_DMA(2, 2, q.split > 1 ? "gemm_dma_kernel<128x128>, K slices" : "gemm_dma_kernel<128x128>");
 #undef TTS_DMA
   }
-  // anything else: 128 x 128 x 64 tiles, two workgroups per CU (a 256 x 256 x 32 form of the same kernel measured behind it
+  // anything else: 128 x 128 x 64 tiles, two workgroups per CU, or half as high (a 256 x 256 x 32 form of the same kernel measured behind it
   // at every size tried: 4096^3: 202 against 197 us; 4096 x 2048 x 2048: 112 against 56 us)
   GemmParams q = p;
   q.split = tile_env || !p.partial ? 1 : any_split(p, std::max(1, p.split));
-  if (q.split == 1) {
-    *name = "gemm_mfma_kernel<128x128x64>";
-    return p.is_bf16 ? launch_gemm_any<true, false>(q, s) : launch_gemm_any<false, false>(q, s);
-  }
-  *name = "gemm_mfma_kernel<128x128x64>, K slices";
+  *name = any_name(any_rows(q, q.split), false, q.split > 1);
+  if (q.split == 1) return p.is_bf16 ? launch_gemm_any<true, false>(q, s) : launch_gemm_any<false, false>(q, s);
   hipError_t e = launch_gemm_any_slices(q, s);
   if (e != hipSuccess) return e;
   const ReduceGrid g(q);
@@ -1042,7 +1046,7 @@ hipError_t launch_gemm_epilogue(const GemmParams &p, const std::string &epilogue
   const int whole = may_compile ? choice.whole : compiled_epilogue(choice.whole, modules), which = sliced ? 2 : whole;
   if (which < 0) return hipErrorInvalidValue;  // (gemm_epilogue_compiled said so)
   const bool any_shape = sliced ? !choice.tile : which == 1 || which == 3;
-  *name = any_shape ? (sliced ? "gemm_mfma_kernel<128x128x64> + epilogue (hipRTC), K slices" : "gemm_mfma_kernel<128x128x64> + epilogue (hipRTC)")
+  *name = any_shape ? any_name(sliced ? any_rows(p, choice.split) : which == 3 ? 64 : 128, true, sliced)
                     : (sliced ? "gemm_dma_kernel + epilogue (hipRTC), K slices" : "gemm_dma_kernel + epilogue (hipRTC)");
   for (int m : {whole, which}) {
     if (modules[m]) continue;

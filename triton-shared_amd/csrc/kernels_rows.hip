@@ -772,9 +772,9 @@ hipError_t launch_layernorm_t(const LayerNormParams &p, dim3 grid, hipStream_t s
 #undef TTS_LN
   }
   const int gx = p.lin_gx ? p.lin_gx : (int)grid.x, gy = p.lin_gx ? p.lin_gy : (int)grid.y;
-  *name = chunks <= 256 ? "layernorm_fwd_kernel<1>" : chunks <= 512 ? "layernorm_fwd_kernel<2>" : chunks <= 1024 ? "layernorm_fwd_kernel<4>" : "layernorm_fwd_kernel<8>";
 #define TTS_LN(CPT, WPR)                                                                                                              \
   do {                                                                                                                                \
+    *name = WPR == 1 ? "layernorm_fwd_kernel<" #CPT ">, a wavefront per row" : "layernorm_fwd_kernel<" #CPT ">";                      \
     const int64_t wgs = (programs + 4 / WPR - 1) / (4 / WPR), along_x = std::min<int64_t>(wgs, 1 << 23);                              \
     hipLaunchKernelGGL((layernorm_fwd_kernel<KIND, CPT, WPR>), dim3((unsigned)along_x, (unsigned)((wgs + along_x - 1) / along_x)), dim3(256), 0, s, p, gx, gy, programs); \
   } while (0)
