@@ -186,6 +186,49 @@ def test_noalloc_launch_of_the_tiled_int8_product_asks_for_no_scratch_it_does_no
         assert ((c.double() - ref).norm() / ref.norm()).item() <= 2.0 ** -11
 
 
+def test_recorded_matmul_with_epilogue_runs_on_a_kernel_that_is_compiled(native):
+    # a plan that has compiled the any-shape product in 128-row tiles records one that would take 64-row tiles: the recording
+    # compiles nothing; outside of it the launch compiles its own
+    import triton
+    import triton_shared_amd as tsa
+    import extra_kernels as X
+    tsa.activate()
+    g = torch.Generator(device="cpu").manual_seed(4)
+
+    def problem(M, N, K):
+        a = torch.randint(-1, 2, (M, K), generator=g).to(torch.bfloat16).to(DEV)
+        b = torch.randint(-1, 2, (K, N), generator=g).to(torch.bfloat16).to(DEV)
+        c = torch.full((M, N), 7, device=DEV, dtype=torch.bfloat16)
+        return a, b, c, (triton.cdiv(M, 128), triton.cdiv(N, 128), 1), [a.data_ptr(), b.data_ptr(), c.data_ptr(), M, N, K, K, N, N, 0.5]
+
+    want = lambda a, b: torch.nn.functional.leaky_relu(a.float() @ b.float(), 0.5).bfloat16()
+    a, b, c, grid, values = problem(2900, 2999, 71)
+    k = X.matmul_leaky[grid[:2]](a, b, c, *values[3:], BM=128, BN=128, BK=64)
+    torch.cuda.synchronize()
+    large, small = "gemm_mfma_kernel<128x128x64> + epilogue (hipRTC)", "gemm_mfma_kernel<64x128x64> + epilogue (hipRTC)"
+    assert k.function.last_kernel == large and torch.equal(c, want(a, b))
+    plan = native.PlanHandle(k.kernel)
+    plan.launch(grid, torch.cuda.current_stream().cuda_stream, values)
+    a, b, c, grid, values = problem(200, 300, 150)
+    assert plan.describe_launch(grid, values)["kernel"] == "gemm_mfma"   # (the table of this shape's tile owners is there then)
+    torch.cuda.synchronize()
+    graph, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    with torch.cuda.graph(graph, stream=side):
+        plan.launch(grid, torch.cuda.current_stream().cuda_stream, values)
+    assert plan.last_kernel == large
+    for _ in range(3):
+        a.copy_(torch.randint(-1, 2, a.shape, generator=g))
+        c.fill_(7)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(c, want(a, b))
+    c.fill_(7)
+    plan.launch(grid, torch.cuda.current_stream().cuda_stream, values)
+    torch.cuda.synchronize()
+    assert plan.last_kernel == small and torch.equal(c, want(a, b))
+
+
 def test_recorded_launches_of_the_tiled_int8_product_allocate_nothing(native):
     # the first launch on a stream, while it records a graph: nothing to allocate, clear or wait for
     plan, _ = plan_for(native, "w8a16_matmul")

@@ -967,14 +967,18 @@ tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, con
         {
           std::lock_guard<std::mutex> lock(plan->mu);
           const int want = gemm_epilogue_split(p);
-          if (want > 1 && !no_alloc && !is_capturing(s)) {
+          const bool recorded = is_capturing(s);
+          // (a launch that a graph records takes an equivalent kernel that is there, as one that may not allocate does: compiling
+          // would load a module in the middle of the recording)
+          const bool may_compile = !no_alloc && !(recorded && gemm_epilogue_compiled(p, plan->gemm_rtc));
+          if (want > 1 && !no_alloc && !recorded) {
             p.split = want;
             tts_plan::SplitK &sk = plan->split_k[stream];
             hipError_t e = plan->grow((void **)&sk.workspace, &sk.workspace_bytes, gemm_workspace_bytes(p));
             if (e != hipSuccess) return fail(TTS_HIP_ERROR, std::string("hipMalloc(split-K workspace): ") + hipGetErrorString(e));
             p.partial = sk.workspace;
           }
-          err = launch_gemm_epilogue(p, pl.source, plan->gemm_rtc, !no_alloc, a, s, &kname, &why);
+          err = launch_gemm_epilogue(p, pl.source, plan->gemm_rtc, may_compile, a, s, &kname, &why);
         }
         if (err != hipSuccess && !why.empty()) return fail(TTS_HIP_ERROR, "gemm epilogue: " + why);
         break;
