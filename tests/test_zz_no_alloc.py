@@ -229,6 +229,40 @@ def test_recorded_matmul_with_epilogue_runs_on_a_kernel_that_is_compiled(native)
     assert plan.last_kernel == small and torch.equal(c, want(a, b))
 
 
+@pytest.mark.parametrize("M,N,Kd", [(976, 1984, 2816), (128, 2048, 4096), (1504, 3072, 4096)])
+def test_recorded_matmul_in_k_slices_allocates_nothing(native, M, N, Kd):
+    # a product that runs in K slices, first launched on a stream while that stream records a graph: there is no workspace and
+    # none is allocated, the product is recorded whole; once an eager launch has left one there, the slices are recorded
+    plan, _ = plan_for(native, "matmul_tiles")
+    g = torch.Generator().manual_seed(M)
+    a = torch.zeros(M, Kd)
+    a = a.scatter_(1, torch.randint(0, Kd, (M, 40), generator=g), 1.0).bfloat16().to(DEV)
+    b, c = torch.zeros(Kd, N, dtype=torch.bfloat16, device=DEV), torch.zeros(M, N, dtype=torch.bfloat16, device=DEV)
+    grid = (((M + 127) // 128) * ((N + 127) // 128), 1, 1)
+    launch = lambda: plan.launch(grid, torch.cuda.current_stream().cuda_stream, [a.data_ptr(), b.data_ptr(), c.data_ptr(), M, N, Kd, Kd, N, N])
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    for sliced in (False, True):
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            launch()
+        assert plan.last_kernel.endswith("K slices") == sliced, plan.last_kernel
+        for _ in range(3):
+            b.copy_(torch.randint(-2, 3, (Kd, N), generator=g))
+            want = (a.float() @ b.float()).bfloat16()   # sums of at most 40 small integers: exact
+            c.fill_(7)
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(c, want)
+            c.fill_(7)
+            torch.cuda.synchronize()
+            with torch.cuda.stream(side):
+                launch()
+            torch.cuda.synchronize()
+            assert plan.last_kernel.endswith("K slices") and torch.equal(c, want)
+
+
 def test_recorded_launches_of_the_tiled_int8_product_allocate_nothing(native):
     # the first launch on a stream, while it records a graph: nothing to allocate, clear or wait for
     plan, _ = plan_for(native, "w8a16_matmul")

@@ -939,9 +939,13 @@ tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, con
             } else {
               std::lock_guard<std::mutex> lock(plan->mu);
               tts_plan::SplitK &sk = plan->split_k[stream];
-              hipError_t e = plan->grow((void **)&sk.workspace, &sk.workspace_bytes, need);
-              if (e != hipSuccess) return fail(TTS_HIP_ERROR, std::string("hipMalloc(split-K workspace): ") + hipGetErrorString(e));
-              p.partial = sk.workspace;
+              if (sk.workspace_bytes < need && is_capturing(s)) {  // nothing is allocated while a graph is recorded: the whole product
+                p.split = 1;
+              } else {
+                hipError_t e = plan->grow((void **)&sk.workspace, &sk.workspace_bytes, need);
+                if (e != hipSuccess) return fail(TTS_HIP_ERROR, std::string("hipMalloc(split-K workspace): ") + hipGetErrorString(e));
+                p.partial = sk.workspace;
+              }
             }
           }
           err = launch_gemm(p, s, &kname);
