@@ -151,16 +151,11 @@ class HIPDriver(DriverBase):
 
     def get_current_stream(self, device):
         import torch
-        raw = torch._C._cuda_getCurrentRawStream
-
-        # the current stream's handle without the Stream object around it (0.1 us of a launch instead of 1.2); that call knows
-        # only device numbers, and the first call initialises the GPU if nothing has
-        def current_stream(device):
-            return raw(device) if type(device) is int else torch.cuda.current_stream(device).cuda_stream
-
-        stream = torch.cuda.current_stream(device).cuda_stream
-        self.get_current_stream = current_stream
-        return stream
+        # the current stream's handle without the Stream object around it (0.1 us of a launch instead of 1.2), by a call that
+        # knows device numbers only
+        if type(device) is int:
+            return torch._C._cuda_getCurrentRawStream(device)
+        return torch.cuda.current_stream(device).cuda_stream
 
     def get_current_device(self):
         import torch
