@@ -749,7 +749,7 @@ def test_gemm_with_column_major_b(K, M, N, Kd, dtype, kernel):
 
 @pytest.mark.parametrize("M,N,Kd,dtype,b_too,kernel", [(1024, 512, 96, torch.bfloat16, False, "gemm_dma_kernel<128x128>"), (4096, 4096, 64, torch.bfloat16, False, "gemm_dma_kernel"),
                                                       (1000, 264, 64, torch.float16, True, "gemm_dma_kernel<128x128>"), (4096, 2048, 32, torch.float16, True, "gemm_dma_kernel<128x256>"),
-                                                      (4088, 2176, 96, torch.bfloat16, False, "gemm_dma_kernel<256x128>"), (1004, 256, 64, torch.bfloat16, False, "gemm_mfma_kernel<128x128x64>")])
+                                                      (4088, 2176, 96, torch.bfloat16, False, "gemm_dma_kernel<256x128>"), (1004, 256, 64, torch.bfloat16, False, "gemm_mfma_kernel<64x128x64>")])
 def test_gemm_with_column_major_a_on_whole_k_tiles(K, M, N, Kd, dtype, b_too, kernel):
     # A stored [K, M] (the product A^T B of a weight gradient), alone or with a column-major B: whole K tiles of 32 and M a
     # multiple of 8 run on the direct-to-LDS kernels (A's stage laid out like a row-major B's); exact on a selection
