@@ -377,10 +377,11 @@ def test_gemm_whole_tile_kernel(K, M, N, Kd, dtype, pad):
     assert torch.equal(c.cpu(), -a.cpu()[:, perm])
 
 
-@pytest.mark.parametrize("M,N,Kd,at,bt", [(976, 1984, 2816, False, False), (752, 2368, 2560, False, True), (1504, 3072, 4096, True, True), (888, 1920, 3136, True, False)])
+@pytest.mark.parametrize("M,N,Kd,at,bt", [(976, 1984, 2816, False, False), (752, 2368, 2560, False, True), (1504, 3072, 4096, True, True), (888, 1920, 3136, True, False),
+                                            (2048, 1536, 5120, False, False), (512, 14336, 4096, False, False), (1024, 2560, 3584, False, True)])
 def test_gemm_that_fills_half_a_round_runs_in_k_slices(K, M, N, Kd, at, bt):
-    """Products whose tiles fill about half of a round of workgroups are ahead in K slices, whichever way the operands lie.  Small
-    integers: exact in any order."""
+    """Products whose tiles fill about half of a round of workgroups are ahead in K slices, whichever way the operands lie, and so are
+    some that fill one with small tiles, in slices of larger ones.  Small integers: exact in any order."""
     g = torch.Generator().manual_seed(M)
     A = torch.randint(-1, 2, (Kd, M) if at else (M, Kd), generator=g).half().to(DEV)
     B = torch.randint(-1, 2, (N, Kd) if bt else (Kd, N), generator=g).half().to(DEV)

@@ -195,7 +195,8 @@ bool gemm_fast_path_ok(const GemmParams &p) { return !p.a_trans && !p.b_trans &&
 // a tile's matrix instructions all run on one CU, 13 us of them for a 64 x 64 tile at K = 1000).
 // G: groups of W x W wavefronts that split the K tiles among them and add their sums through LDS at the end, in group order:
 // the chain of loads, LDS stores and matrix instructions of a group is 1 / G as long, and the SIMDs have several to run.
-// All K tiles but the last load 16 bytes a chunk, at any alignment and without a test, two tiles ahead (as gemm_mfma_body).
+// All K tiles but the last load 16 bytes a chunk, at any alignment and without a test, two tiles ahead; the last goes element by
+// element where a chunk sticks out (gemm_mfma_body reads that one in 16 bytes, too).
 // 768^3: 39.3 -> 17.6 us; 16 x 1000 x 1000: 11.7 (27 with 64 x 64 tiles).  (Eight groups at 768^3: 25.3.)
 constexpr int F32_BK = 16;
 
@@ -855,11 +856,11 @@ constexpr int W8_WAVES = 16;
 
 namespace {
 // Which direct-to-LDS tile a product runs on (null: none applies), and in how many K slices.
-// first, more, fixed: us per K tile of a round of workgroups that is all but empty, what a full round adds to it, and per launch,
-// fitted at `time` below.
-struct DmaCand { const char *tag; int64_t bm, bn; double eff, first, more, fixed; };
-const DmaCand DMA_CANDS[4] = {{"256x256", 256, 256, 1.0, 0.57, 0.16, 8}, {"128x256", 128, 256, 0.77, 0.41, 0.15, 5},
-                              {"256x128", 256, 128, 0.73, 0.42, 0.15, 5}, {"128x128", 128, 128, 0.59, 0.29, 0.07, 3}};
+// round, turned, fill, fixed: us per K tile and round of workgroups, what a column-major B adds to it, us per K tile and workgroup
+// per CU, and per launch; fitted at `time` below.
+struct DmaCand { const char *tag; int64_t bm, bn; double eff, round, turned, fill, fixed; };
+const DmaCand DMA_CANDS[4] = {{"256x256", 256, 256, 1.0, 0.59, 0.07, 0.04, 9}, {"128x256", 128, 256, 0.77, 0.48, 0.07, 0.05, 6},
+                              {"256x128", 256, 128, 0.73, 0.51, 0.03, 0.04, 6.3}, {"128x128", 128, 128, 0.59, 0.34, 0, 0.03, 3.8}};
 struct DmaChoice { const DmaCand *tile = nullptr; int split = 1; };
 
 DmaChoice choose_dma(const GemmParams &p, int max_split) {
@@ -875,25 +876,25 @@ DmaChoice choose_dma(const GemmParams &p, int max_split) {
   // 800 210 / 210).  A few tiles over one round count as one: blocks of rows that pad the last matrix have nothing to do.
   const bool grouped = p.b_block != nullptr && !p.b_trans;
   auto grouped_wide = [&](int64_t t) { return 2 * t >= cus && !(10 * t > 11 * cus && 10 * t < 16 * cus); };
-  // The other products: the least modelled time.  What decides is whole rounds of workgroups over the chip (the 128 x 128 tile's two
-  // workgroups per CU blur them), and that a round runs faster the emptier it is.  Few tiles (a skinny product, M = 128 ... 1024
-  // against N, K in the thousands) leave CUs idle while every workgroup walks all of K alone: K is then cut into slices, whose fp32
-  // sums a second kernel adds, and whose workgroups count in rounds like any others.
-  // Fitted to 130 products from HBM (M 128 ... 4200, N to 4200, K 512 ... 8300, each operand row- or column-major, batches of 2 to 12)
-  // on every tile in 1 to 16 slices: a scatter of 7 % with slices, 8 to 11 % without, and the choice is 2.4 % behind the best of
-  // each.  us on 256 x 256 / 128 x 256 / 128 x 128 tiles: 3000 x 4096 x 2048 50.5 / 67.6 / 65.9; 3000 x 2048 x 4096 80.8 / 61.1 / 68.2;
-  // 2048^3 42.3 / 28.2 / 21.7; in 1 / 2 / 3 / 4 slices: 1504 x 3072 x 4096 on 256 x 256 84 / 64 / 56 / 79 (the fourth begins a second
-  // round), 976 x 1984 x 2816 on 128 x 128 33.7 / 27.0 / 33.3 / 31.0, 464 x 4160 x 6016 on 128 x 256 87 / 57 / 48 / 68.
+  // The other products: the least modelled time.  What decides is the number of rounds of workgroups over the chip, begun ones
+  // included: a K tile of a round takes about the same however many of the CUs work (128 x 128 tiles, two of which share a CU,
+  // up to 1 / 2 / 3 / 4 per CU: 0.38 / 0.69 / 1.0 / 1.4 us).  Few tiles (a skinny product, M = 16 ... 1024 against N, K in the thousands)
+  // leave CUs idle while every workgroup walks all of K alone: K is then cut into slices, whose fp32 sums a second kernel adds, and
+  // whose workgroups count in rounds like any others.
+  // Fitted to 1820 products from HBM (M 16 ... 4200, N to 14336, K 512 ... 14336, powers of two and their like, model widths and sizes
+  // nothing divides, either operand column-major) on every tile in 1 to 16 slices, for the choice rather than the times: it is
+  // 1.9 % behind the best of each; the tile by the rule below and slices as if they filled the chip evenly are 9 % behind.
+  // us: 3000 x 4096 x 2048 on 256 x 256 / 128 x 256 / 128 x 128 tiles 50.5 / 67.6 / 65.9; 3000 x 2048 x 4096 80.8 / 61.1 / 68.2; 2048 x 1536 x
+  // 5120 on 128 x 128 tiles 64, in five slices of 256 x 256 50; 512 x 14336 x 4096 on 128 x 256 81, in two slices of 256 x 256 71; in 1 / 2 /
+  // 3 / 4 slices 1504 x 3072 x 4096 on 256 x 256 84 / 64 / 56 / 79 (the fourth begins a second round).
   // Below K = 512 the fixed costs decide and the tiles measure alike: among the tiles that give every CU a workgroup (128 x 128:
   // always) the one with the least padded work per unit of the tile's measured efficiency at 4096^3 (105 / 136 / 144 / 179 us).
   const bool by_rounds = !grouped && p.K >= 512;
   const int64_t nk = p.K / F_BK;
   const double sums = (double)p.M * (double)p.N * std::max(1, p.batches) * 4;  // bytes of one slice's
   auto time = [&](const DmaCand &c, int split) {
-    const double f = (double)tiles(c) * split / cus, whole = std::floor(f), rest = f - whole;
-    double rounds = whole * (c.first + c.more) + (rest > 0 ? c.first + c.more * rest : 0);
-    if (c.bm + c.bn == 256 && f > 1) rounds = (c.first + c.more) * 0.5 * (f + std::ceil(f));
-    return rounds * (double)((nk + split - 1) / split) + c.fixed + (split > 1 ? 4.4 + split * sums / 2.9e6 : 0);
+    const double f = (double)tiles(c) * split / cus;
+    return (double)((nk + split - 1) / split) * (std::ceil(f) * (c.round + (p.b_trans ? c.turned : 0)) + f * c.fill) + c.fixed + (split > 1 ? 5.5 + 0.28e-6 * split * sums : 0);
   };
   DmaChoice best;
   double best_cost = 0;
@@ -905,7 +906,7 @@ DmaChoice choose_dma(const GemmParams &p, int max_split) {
   }
   if (!best.tile || max_split < 2 || !by_rounds || p.a_rows || p.b_block) return best;
   DmaChoice pick = best;
-  double pick_t = 0.95 * best_cost;  // (a second launch has to be worth it by more than the model errs for it)
+  double pick_t = best_cost;
   if (!(split_env && atoi(split_env) == 1))
     for (const DmaCand &c : DMA_CANDS) {
       if (!gemm_dma_ok(p, c.bm, c.bn) || (dma_env && std::string(dma_env) != c.tag)) continue;
