@@ -112,7 +112,7 @@ __device__ __forceinline__ uint4 without_first(uint4 v, int k) {
 // What bounds it on ragged sizes is the way of the operands from memory: a chain of one load per K tile where a shape gives the
 // chip less than one workgroup per CU, else the rate at which a CU takes 16-byte loads that are not 16-byte aligned.  Chunks are
 // 16-byte loads at any alignment (global memory takes them at element addresses), untested, and two tiles are in flight.
-// 1000 x 3001 x 1003 fp16 with a fused activation: 25 us (163 with two-byte loads, each behind a test, and 30 while only the last
+// 1000 x 3001 x 1003 fp16 with a fused activation: 22 us, 26 from HBM (163 with two-byte loads, each behind a test, and 30 while only the last
 // K tiles were loaded that way); TM, TN: 128 x 128 tiles or, for few of them, 64 x 128 (kernels_gemm.hip: any_rows).
 // Rows of A may be taken through an index vector (p.a_rows) and the base of B may depend on the block of rows
 // (p.b_block): a mixture-of-experts product is this kernel with both set.
