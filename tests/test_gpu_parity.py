@@ -200,9 +200,12 @@ def test_layernorm_rows_at_any_alignment(K, dtype, M, N):
 
 
 @pytest.mark.parametrize("dtype,M,N,kernel", [
-    ("float16", 16500, 2047, "layernorm_fwd_persistent_kernel"), ("bfloat16", 16400, 1033, "layernorm_fwd_persistent_kernel"), ("bfloat16", 8200, 4095, "layernorm_fwd_persistent_kernel"),
-    ("float16", 4200, 5001, "layernorm_fwd_persistent_kernel"), ("float32", 16500, 1023, "layernorm_fwd_persistent_kernel"), ("float32", 8200, 2047, "layernorm_fwd_persistent_kernel"),
-    ("float32", 8200, 1030, "layernorm_fwd_persistent_kernel"), ("float32", 4200, 3001, "layernorm_fwd_persistent_kernel"),
+    ("bfloat16", 8200, 4095, "layernorm_fwd_persistent_kernel"), ("float16", 8300, 2100, "layernorm_fwd_persistent_kernel"), ("float32", 16500, 1023, "layernorm_fwd_persistent_kernel"),
+    ("float32", 8200, 2047, "layernorm_fwd_persistent_kernel"), ("float32", 8200, 1032, "layernorm_fwd_persistent_kernel"), ("float32", 4200, 3001, "layernorm_fwd_persistent_kernel"),
+    ("float32", 4200, 3999, "layernorm_fwd_persistent_kernel"), ("float32", 4200, 5760, "layernorm_fwd_persistent_kernel"), ("float32", 4200, 7998, "layernorm_fwd_persistent_kernel"),
+    ("bfloat16", 16400, 2048, "layernorm_fwd_persistent_kernel"), ("bfloat16", 4200, 6144, "layernorm_fwd_persistent_kernel"), ("float16", 4200, 8192, "layernorm_fwd_persistent_kernel"),
+    ("float16", 16500, 2047, "layernorm_fwd_kernel<4>, a wavefront per row"), ("bfloat16", 8300, 2304, "layernorm_fwd_kernel<2>"), ("float16", 4200, 5001, "layernorm_fwd_kernel<3>"),
+    ("bfloat16", 4200, 7040, "layernorm_fwd_kernel<4>"), ("float32", 4200, 4288, "layernorm_fwd_kernel<6>"), ("float32", 4200, 6272, "layernorm_fwd_kernel<8>"),
     ("float16", 4200, 257, "layernorm_fwd_kernel<1>, a wavefront per row"), ("bfloat16", 4200, 513, "layernorm_fwd_kernel<2>, a wavefront per row"),
     ("float32", 1030, 1023, "layernorm_fwd_kernel<4>, a wavefront per row"), ("float16", 70, 1025, "layernorm_fwd_kernel<1>"), ("float32", 9, 2047, "layernorm_fwd_kernel<2>"),
     ("float32", 9, 2500, "layernorm_fwd_kernel<3>"), ("bfloat16", 9, 8191, "layernorm_fwd_kernel<4>"), ("float32", 9, 6001, "layernorm_fwd_kernel<6>"), ("bfloat16", 9, 9001, "layernorm_fwd_kernel<6>"),

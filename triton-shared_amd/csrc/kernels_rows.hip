@@ -471,14 +471,16 @@ __device__ __forceinline__ float pairwise(const float (&s)[N]) {
 // Loads and stores take 16 bytes wherever the row starts.  (Element by element, as rows off the 16-byte grid were read
 // before: fp16 [8192, 5003] 135 us, now 37.)  Short rows take a wavefront each: no barrier, four rows per workgroup
 // (fp32 [8000, 512]: 14.4 us with a workgroup per row, 8.0 with a wavefront).
-template <int KIND, int CPT, int WPR>
-__global__ __launch_bounds__(256, CPT <= 2 || (KIND == 2 && CPT <= 4) ? 8 : CPT <= 4 ? 6 : KIND == 2 ? 4 : 3) void layernorm_fwd_kernel(LayerNormParams p, int gx, int gy, int64_t programs) {
+// CUT: rows may end inside a chunk.  Without, eight workgroups of up to four chunks per thread fit a CU, where the code for that end
+// leaves six (fp16 [2040, 8192]: 17.4 us in two rounds of them, 13.2 in one), and short launches have half as much code to
+// fetch (bf16 [419, 928]: 4.4 us / 3.8).
+template <int KIND, int CPT, int WPR, bool CUT>
+__global__ __launch_bounds__(256, CPT <= 2 || (CPT <= 4 && (KIND == 2 || !CUT)) ? 8 : CPT <= 4 ? 6 : KIND == 2 || !CUT ? 4 : 3) void layernorm_fwd_kernel(LayerNormParams p, int gx, int gy, int64_t programs) {
   using T = LnType<KIND>;
   using E = typename T::elem;
   constexpr int EPC = T::EPC, THREADS = WPR * WAVE;
   __shared__ float red[4];
   const int64_t prog = ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * (4 / WPR) + (WPR == 1 ? threadIdx.x / WAVE : 0);  // (along y from 2^23 workgroups on)
-  if (prog >= programs) return;  // (whole wavefronts, or a whole workgroup where a row has one to itself)
   const int t = threadIdx.x % THREADS;
   int px = (int)prog, py = 0, pz = 0;
   if (programs != gx) { px = (int)(prog % gx); py = (int)((prog / gx) % gy); pz = (int)(prog / ((int64_t)gx * gy)); }
@@ -488,18 +490,20 @@ __global__ __launch_bounds__(256, CPT <= 2 || (KIND == 2 && CPT <= 4) ? 8 : CPT 
   const E *__restrict__ b = (const E *)p.b + affine(p.b_off, px, py, pz);
   E *__restrict__ y = (E *)p.y + affine(p.y_off, px, py, pz);
   const int N = (int)p.N;
+  if (prog >= programs) return;  // (whole wavefronts, or a whole workgroup where a row has one to itself)
   u32x4_t raw[CPT];
 #pragma unroll
   for (int c = 0; c < CPT; c++) {
     const int i0 = (t + c * THREADS) * EPC;
-    raw[c] = *reinterpret_cast<const u32x4_any *>(x + (i0 < N ? min(i0, N - EPC) : 0));
+    raw[c] = *reinterpret_cast<const u32x4_any *>(x + (i0 < N ? (CUT ? min(i0, N - EPC) : i0) : 0));
   }
+  __builtin_amdgcn_sched_barrier(0);  // (the scheduler would otherwise put a chunk's first use, and the wait for it, before the next chunk's load)
   float v[CPT][EPC];
 #pragma unroll
   for (int c = 0; c < CPT; c++) {
     const int i0 = (t + c * THREADS) * EPC;
     if (i0 >= N) raw[c] = u32x4_t{0, 0, 0, 0};  // other = 0
-    else if (i0 + EPC > N) drop_front<EPC>(raw[c], i0 + EPC - N);
+    else if (CUT && i0 + EPC > N) drop_front<EPC>(raw[c], i0 + EPC - N);
     const uint32_t q[4] = {raw[c][0], raw[c][1], raw[c][2], raw[c][3]};
     T::unpack(q, v[c]);
   }
@@ -518,7 +522,7 @@ __global__ __launch_bounds__(256, CPT <= 2 || (KIND == 2 && CPT <= 4) ? 8 : CPT 
     s[c] = 0.f;
 #pragma unroll
     for (int k = 0; k < EPC; k++) {
-      float d = i0 + k < N ? v[c][k] - mean : 0.f;  // tl.where(cols < N, x - mean, 0)
+      float d = i0 + (CUT ? k : 0) < N ? v[c][k] - mean : 0.f;  // tl.where(cols < N, x - mean, 0)
       s[c] += d * d;
     }
   }
@@ -531,7 +535,7 @@ __global__ __launch_bounds__(256, CPT <= 2 || (KIND == 2 && CPT <= 4) ? 8 : CPT 
 #pragma unroll
   for (int c = 0; c < CPT; c++) {
     const int i0 = (t + c * THREADS) * EPC;
-    if (i0 + EPC <= N) {
+    if (CUT ? i0 + EPC <= N : i0 < N) {
       const u32x4_t wr = *reinterpret_cast<const u32x4_any *>(w + i0), br = *reinterpret_cast<const u32x4_any *>(b + i0);
       const uint32_t wq[4] = {wr[0], wr[1], wr[2], wr[3]}, bq[4] = {br[0], br[1], br[2], br[3]};
       float wv[EPC], bv[EPC], o[EPC];
@@ -540,7 +544,7 @@ __global__ __launch_bounds__(256, CPT <= 2 || (KIND == 2 && CPT <= 4) ? 8 : CPT 
 #pragma unroll
       for (int k = 0; k < EPC; k++) o[k] = (v[c][k] - mean) * rstd * wv[k] + bv[k];
       ntstore(reinterpret_cast<u32x4_any *>(y + i0), T::pack(o));
-    } else {
+    } else if (CUT) {
 #pragma unroll
       for (int k = 0; k < EPC; k++)
         if (i0 + k < N) y[i0 + k] = T::down((v[c][k] - mean) * rstd * T::up(w[i0 + k]) + T::up(b[i0 + k]));
@@ -557,7 +561,8 @@ __global__ __launch_bounds__(256, CPT <= 2 || (KIND == 2 && CPT <= 4) ? 8 : CPT 
 // nothing else, gives 23.8 us.  512 or 1024 threads per workgroup, a third row in flight and nontemporal row loads
 // gain nothing or lose.  [8192, 8192]: 51.7 -> 44.8 us (6.0 TB/s).
 // For one-dimensional grids, w and b the same for every row, N >= EPC.  WHOLE: rows of exactly CPT * 256 chunks; otherwise a
-// thread's last chunks may be absent or cut off (see above), which costs a select and a branch per chunk.
+// thread's last chunks may be absent or cut off (see above), which costs registers, a select and a branch per chunk: 16-bit rows
+// of 513 chunks and more then take up to twice as long as with a workgroup each (see the launcher).
 template <int KIND, int CPT, bool WHOLE>
 __global__ __launch_bounds__(256) void layernorm_fwd_persistent_kernel(LayerNormParams p, int rows) {
   using T = LnType<KIND>;
@@ -749,16 +754,22 @@ hipError_t launch_layernorm_t(const LayerNormParams &p, dim3 grid, hipStream_t s
     persistent_grid = atoi(ln_env);
     min_rows = 2 * (int64_t)persistent_grid;
   }
+  // Rows of fewer chunks than CPT * 256 are walked where that was measured ahead (us walked / a workgroup or wavefront per row):
+  // 16-bit rows of 257 to 511 chunks that end inside one (fp16 [18067, 2901] 52 / 60, [17314, 3537] 56.3 / 57.9; ending on a chunk
+  // [22810, 2192] 52.8 / 49.8, bf16 [15881, 2304] 44.8 / 40.2; of other lengths fp16 [19115, 1088] 26.8 / 21.7, bf16 [13346, 4480] 73.5 /
+  // 49.8, [19065, 7040] 200 / 101), fp32 rows of 257 to 768 chunks ([25369, 1152] 44.2 / 56.3, [4274, 2556] 18.9 / 20.0) and those that
+  // fill nine tenths of the threads' chunks ([12213, 5760] 100 / 107, [13291, 7680] 143 / 157; [8605, 4288] 75.6 / 56.8, [4669, 3200] 29.8 / 25.7).
+  const bool whole = p.N == (int64_t)cpt * 256 * EPC;
+  const bool walked = whole || (KIND == 2 ? cpt == 2 || cpt == 3 || 10 * chunks >= 9 * 256 * cpt : cpt == 2 && p.N % EPC != 0);
   auto row_invariant = [](const Affine &a) { return (a.c[0] | a.c[1] | a.c[2]) == 0; };
-  if (cpt && chunks > 128 && persistent_grid > 0 && !p.lin_gx && grid.y == 1 && grid.z == 1 && (int64_t)grid.x >= min_rows && row_invariant(p.w_off) && row_invariant(p.b_off)) {
+  if (cpt && walked && chunks > 128 && persistent_grid > 0 && !p.lin_gx && grid.y == 1 && grid.z == 1 && (int64_t)grid.x >= min_rows && row_invariant(p.w_off) && row_invariant(p.b_off)) {
     const int rows = (int)grid.x;
     const dim3 pg((unsigned)persistent_grid);
-    const bool whole = p.N == (int64_t)cpt * 256 * EPC;
     *name = "layernorm_fwd_persistent_kernel";
 #define TTS_LN(CPT)                                                                                                                   \
   do {                                                                                                                                \
     if (whole) hipLaunchKernelGGL((layernorm_fwd_persistent_kernel<KIND, CPT, true>), pg, dim3(256), 0, s, p, rows);                 \
-    else hipLaunchKernelGGL((layernorm_fwd_persistent_kernel<KIND, CPT, false>), pg, dim3(256), 0, s, p, rows);                      \
+    else if constexpr (KIND == 2 || CPT == 2) hipLaunchKernelGGL((layernorm_fwd_persistent_kernel<KIND, CPT, false>), pg, dim3(256), 0, s, p, rows); \
     return hipGetLastError();                                                                                                         \
   } while (0)
     if (cpt == 1) TTS_LN(1);
@@ -776,12 +787,15 @@ hipError_t launch_layernorm_t(const LayerNormParams &p, dim3 grid, hipStream_t s
   do {                                                                                                                                \
     *name = WPR == 1 ? "layernorm_fwd_kernel<" #CPT ">, a wavefront per row" : "layernorm_fwd_kernel<" #CPT ">";                      \
     const int64_t wgs = (programs + 4 / WPR - 1) / (4 / WPR), along_x = std::min<int64_t>(wgs, 1 << 23);                              \
-    hipLaunchKernelGGL((layernorm_fwd_kernel<KIND, CPT, WPR>), dim3((unsigned)along_x, (unsigned)((wgs + along_x - 1) / along_x)), dim3(256), 0, s, p, gx, gy, programs); \
+    const dim3 wg_grid((unsigned)along_x, (unsigned)((wgs + along_x - 1) / along_x));                                                 \
+    if (p.N % EPC) hipLaunchKernelGGL((layernorm_fwd_kernel<KIND, CPT, WPR, true>), wg_grid, dim3(256), 0, s, p, gx, gy, programs);   \
+    else hipLaunchKernelGGL((layernorm_fwd_kernel<KIND, CPT, WPR, false>), wg_grid, dim3(256), 0, s, p, gx, gy, programs);            \
   } while (0)
-  // A wavefront per row up to 256 chunks, given four rows per CU or rows of a single chunk per lane (fp16 [4000, 2000]: 10.2
-  // us against 11.0 with a workgroup per row, fp32 [8000, 1000] 13.1 against 16.6; fp16 [300, 2000] 5.2 against 4.2); at 512
-  // chunks the workgroup wins again (fp16 [2000, 4096]: 9.6 against 10.9).
-  const bool short_rows = chunks <= 64 || (chunks <= 256 && programs >= 4 * cus);
+  // A wavefront per row of a single chunk per lane, of up to 128 chunks given four rows per CU and of up to 256 given four in fp32
+  // and ten in 16 bits (us with a wavefront / a workgroup per row: fp16 [1042, 968] 4.2 / 4.9, bf16 [6595, 1008] 8.7 / 13.5; fp32 [1040,
+  // 580] 4.3 / 4.7, [8352, 604] 11.1 / 16.0; bf16 [1203, 2035] 8.1 / 6.7, [2098, 1773] 8.2 / 8.1, [2823, 1456] 7.1 / 8.2, [8264, 1600] 16.2 /
+  // 19.7; fp16 [300, 2000] 5.2 / 4.2); at 512 chunks the workgroup wins again (fp16 [2000, 4096]: 9.6 against 10.9).
+  const bool short_rows = chunks <= 64 || (programs >= 4 * cus && (chunks <= 128 || (chunks <= 256 && (KIND == 2 || programs >= 10 * cus))));
   if (short_rows && chunks <= 64) TTS_LN(1, 1);
   else if (short_rows && chunks <= 128) TTS_LN(2, 1);
   else if (short_rows) TTS_LN(4, 1);
