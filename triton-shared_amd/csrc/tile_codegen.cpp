@@ -803,11 +803,33 @@ struct Gen {
       }
     return text;
   }
+  // Element n of a wide 16-bit block that is kept packed, two elements per register, with zeros where it is not valid.
+  std::string from_packed(const SOp &o, const std::string &words, const std::string &pred, const std::string &i0, const std::string &i1) {
+    const std::string word = words + "[n >> 3][(n & 7) >> 1]";
+    const std::string got = std::string(o.acc.elem == "f16" ? "up_f16(" : "up_bf16(") + "(unsigned short)((n & 1) ? " + word + " >> 16 : " + word + "))";
+    const bool zero = pred.empty() || (o.acc.other_value < 0 && (!o.acc.has_other || (o.acc.other_f == 0.0 && !std::signbit(o.acc.other_f))));
+    return "(" + (zero ? got : "(" + pred + ") ? " + got + " : " + other_of(o.acc, i0, i1)) + ")";
+  }
+  // Where `when` holds, the group of a wide block that the extent cuts off -- read from the last eight valid elements -- is moved down.
+  void put_in_place(const SOp &o, const std::string &words, const std::string &pred, const std::string &when, int64_t groups, const std::vector<int64_t> &ls) {
+    const int esz = mem_bytes(o.acc.elem);
+    os << pad() << "if (" << when << ") {\n";
+    indent++;
+    os << pad() << "#pragma unroll\n" << pad() << "for (int g = 0; g < " << groups << "; g++) {\n";
+    indent++;
+    os << pad() << "const int n = 8 * g;\n" << pad() << "const int t = " << element_of_slot(ls) << ";\n" << pad() << "(void)t;\n";
+    os << pad() << "const int cut = (" << pred << ") ? " << cut_off(o.acc, ls.size() < 2 ? idx0(ls) : idx1(ls)) << " : 0;\n";
+    os << pad() << "if (cut) " << (esz == 4 ? "drop_front_32(" + words + "[2 * g], " + words + "[2 * g + 1], cut)" : (esz == 2 ? "drop_front_16(" : "drop_front_8(") + words + "[g], cut)") << ";\n";
+    indent--;
+    os << pad() << "}\n";
+    indent--;
+    os << pad() << "}\n";
+  }
   // Loads that the run after the next reduction makes of a block laid out like this run's -- the row of weights of a
   // normalisation -- are issued behind this run's and wait, packed, in `ahead` registers (32 of them at most): made where they
-  // stand, after the reduction, their way from L2 is added to the row's from memory.  RMSNorm fp16 from HBM, us after / behind:
+  // stand, after the reduction, their way from L2 is added to the row's from memory.  They stay packed until each element's use.  RMSNorm fp16 from HBM, us after / behind:
   // [4096, 8192] 28.5 / 26.0, [2000, 8192] 15.5 / 14.9, [8000, 5120] 35.9 / 34.5, [8000, 4096] 26.5 / 25.3, [16000, 2048] 31.0 / 28.1.
-  std::set<int> loaded_ahead;
+  std::map<int, std::string> loaded_ahead;  // value id -> the condition under which the loads went in groups (leaves_eight)
   std::vector<const SOp *> loads_of_next_run(const std::vector<SOp> &ops, size_t from, const std::vector<int64_t> &shape, const std::string &roomy) {
     std::vector<const SOp *> loads, none;
     bool reduced = false;
@@ -1339,7 +1361,7 @@ struct Gen {
           bool any = false;
           for (size_t q = k; q < end; q++)
             if (mine_here(ops[q])) {
-              if (!row_gather(ops[q].acc))
+              if (!row_gather(ops[q].acc) && !loaded_ahead.count(ops[q].result))
                 os << pad() << ctype(val(ops[q].result).dtype) << " ld" << ops[q].result << "[" << (held_count(ls) + 255) / 256 << "];\n";
               any = true;
             }
@@ -1376,9 +1398,23 @@ struct Gen {
           // sits between the loads, so none waits for another.  Only a program whose extent is one to seven elements loads
           // element by element, as it would in the ordinary order.
           auto wide_load = [&](const SOp &o) { return wide(ls) && mine_here(o) && vector_access(o.acc); };
+          auto packed = [&](const SOp &o) { return loaded_ahead.count(o.result) != 0; };  // loaded by the run before, stays packed
           std::vector<const SOp *> wide_loads;
-          for (size_t q = k; q < end; q++)
-            if (wide_load(ops[q])) wide_loads.push_back(&ops[q]);
+          for (size_t q = k; q < end; q++) {
+            if (!wide_load(ops[q])) continue;
+            const SOp &o = ops[q];
+            if (!packed(o)) {
+              wide_loads.push_back(&o);
+              continue;
+            }
+            const std::string words = "ahead" + std::to_string(o.result), &in_groups = loaded_ahead.at(o.result);
+            std::string pred;
+            address(o.acc, l0, l1, pred);
+            if (!o.acc.dims.empty()) put_in_place(o, words, pred, (in_groups.empty() ? "" : "(" + in_groups + ") && ") + "(" + ex(o.acc.dims.back()) + " & 7)", held_count(ls) / 2048, ls);
+            held[o.result] = {words, ls, from_packed(o, words, pred, l0, l1)};
+            var[o.result] = held[o.result].expr;
+            mine.push_back(o.result);
+          }
           if (!wide_loads.empty()) {
             const int64_t G = held_count(ls) / 2048;
             uses_dummy = true;
@@ -1388,7 +1424,7 @@ struct Gen {
             os << pad() << "if (" << (roomy.empty() ? "true" : roomy) << ") {\n";
             indent++;
             for (size_t q = k; q < end; q++)
-              if (wide_load(ops[q]))
+              if (wide_load(ops[q]) && !packed(ops[q]))
                 os << pad() << (mem_bytes(ops[q].acc.elem) == 1 ? "u32x2_t rw" : "u32x4_t rw") << ops[q].result << "[" << G * (mem_bytes(ops[q].acc.elem) == 4 ? 2 : 1) << "];\n";
             os << pad() << "#pragma unroll\n" << pad() << "for (int g = 0; g < " << G << "; g++) {\n";
             indent++;
@@ -1409,46 +1445,26 @@ struct Gen {
               indent--;
               os << pad() << "}\n";
             };
-            for (const SOp *o : wide_loads) {
-              const std::string id = std::to_string(o->result);
-              if (loaded_ahead.count(o->result)) os << pad() << "rw" << id << "[g] = ahead" << id << "[g];\n";
-              else read_group(*o, "rw" + id);
-            }
+            for (const SOp *o : wide_loads) read_group(*o, "rw" + std::to_string(o->result));
             indent--;
             os << pad() << "}\n";
             if (!ahead.empty()) {
               os << pad() << "#pragma unroll\n" << pad() << "for (int g = 0; g < " << G << "; g++) {\n";
               indent++;
               os << pad() << "const int n = 8 * g;\n" << pad() << "const int t = " << element_of_slot(ls) << ";\n";
-              for (const SOp *o : ahead) {
-                read_group(*o, "ahead" + std::to_string(o->result));
-                loaded_ahead.insert(o->result);
-              }
+              for (const SOp *o : ahead) read_group(*o, "ahead" + std::to_string(o->result));
               indent--;
               os << pad() << "}\n";
             }
-            for (size_t q = k; q < end; q++)
-              if (wide_load(ops[q]) && !ops[q].acc.dims.empty()) {
-                const SOp &o = ops[q];
-                const std::string id = std::to_string(o.result);
-                const int esz = mem_bytes(o.acc.elem);
+            for (const SOp *o : wide_loads)
+              if (!o->acc.dims.empty()) {
                 std::string pred;
-                address(o.acc, l0, l1, pred);
-                os << pad() << "if (" << ex(o.acc.dims.back()) << " & 7) {\n";
-                indent++;
-                os << pad() << "#pragma unroll\n" << pad() << "for (int g = 0; g < " << G << "; g++) {\n";
-                indent++;
-                os << pad() << "const int n = 8 * g;\n" << pad() << "const int t = " << element_of_slot(ls) << ";\n" << pad() << "(void)t;\n";
-                os << pad() << "const int cut = (" << pred << ") ? " << cut_off(o.acc, ls.size() < 2 ? l0 : l1) << " : 0;\n";
-                os << pad() << "if (cut) " << (esz == 4 ? "drop_front_32(rw" + id + "[2 * g], rw" + id + "[2 * g + 1], cut)" : (esz == 2 ? "drop_front_16(rw" : "drop_front_8(rw") + id + "[g], cut)") << ";\n";
-                indent--;
-                os << pad() << "}\n";
-                indent--;
-                os << pad() << "}\n";
+                address(o->acc, l0, l1, pred);
+                put_in_place(*o, "rw" + std::to_string(o->result), pred, ex(o->acc.dims.back()) + " & 7", G, ls);
               }
             open_element_loop(ls);
             for (size_t q = k; q < end; q++)
-              if (wide_load(ops[q])) {
+              if (wide_load(ops[q]) && !packed(ops[q])) {
                 const SOp &o = ops[q];
                 const std::string id = std::to_string(o.result);
                 std::string pred, addr = address(o.acc, l0, l1, pred);
@@ -1470,7 +1486,7 @@ struct Gen {
             indent++;
             open_element_loop(ls);
             for (size_t q = k; q < end; q++)
-              if (wide_load(ops[q])) {
+              if (wide_load(ops[q]) && !packed(ops[q])) {
                 const SOp &o = ops[q];
                 const std::string name = "ld" + std::to_string(o.result);
                 std::string pred, addr = address(o.acc, l0, l1, pred);
@@ -1481,11 +1497,11 @@ struct Gen {
               }
             close_loop();
             bool any_masked = false;
-            for (size_t q = k; q < end; q++) any_masked = any_masked || (wide_load(ops[q]) && !ops[q].acc.dims.empty());
+            for (size_t q = k; q < end; q++) any_masked = any_masked || (wide_load(ops[q]) && !packed(ops[q]) && !ops[q].acc.dims.empty());
             if (any_masked) {
               open_element_loop(ls);
               for (size_t q = k; q < end; q++)
-                if (wide_load(ops[q]) && !ops[q].acc.dims.empty()) {
+                if (wide_load(ops[q]) && !packed(ops[q]) && !ops[q].acc.dims.empty()) {
                   const SOp &o = ops[q];
                   const std::string name = "ld" + std::to_string(o.result);
                   std::string pred, addr = address(o.acc, l0, l1, pred);
@@ -1498,16 +1514,28 @@ struct Gen {
                 }
               close_loop();
             }
+            for (const SOp *load : ahead) {
+              const SOp &o = *load;
+              std::string pred, addr = address(o.acc, along(ls, l0, " + e").first, along(ls, l1, " + e").second, pred);
+              os << pad() << "#pragma unroll\n" << pad() << "for (int g = 0; g < " << G << "; g++) {\n";
+              indent++;
+              os << pad() << "const int n = 8 * g, t = " << element_of_slot(ls) << ";\n" << pad() << "(void)t;\n"
+                 << pad() << "unsigned one[8] = {};\n" << pad() << "#pragma unroll\n" << pad() << "for (int e = 0; e < 8; e++)\n"
+                 << pad() << "  " << (pred.empty() ? "" : "if (" + pred + ") ") << "one[e] = ((const unsigned short *)p.ptr[" << o.acc.base_arg << "])[" << addr << "];\n"
+                 << pad() << "ahead" << o.result << "[g] = u32x4_t{one[0] | one[1] << 16, one[2] | one[3] << 16, one[4] | one[5] << 16, one[6] | one[7] << 16};\n"
+                 << pad() << "__builtin_amdgcn_sched_barrier(0);  // (a group at a time: these few loads are not worth registers)\n";
+              indent--;
+              os << pad() << "}\n";
+            }
             indent--;
             os << pad() << "}\n";
-            for (size_t q = k; q < end; q++)
-              if (wide_load(ops[q])) {
-                const SOp &o = ops[q];
-                const std::string name = "ld" + std::to_string(o.result);
-                held[o.result] = {name, ls};
-                var[o.result] = name + "[n]";
-                mine.push_back(o.result);
-              }
+            for (const SOp *o : wide_loads) {
+              const std::string name = "ld" + std::to_string(o->result);
+              held[o->result] = {name, ls};
+              var[o->result] = name + "[n]";
+              mine.push_back(o->result);
+            }
+            for (const SOp *o : ahead) loaded_ahead[o->result] = roomy;
           }
           for (size_t q = k; q < end; q++)
             if (mine_here(ops[q]) && row_gather(ops[q].acc)) {
@@ -1545,10 +1573,7 @@ struct Gen {
                  << pad() << "rw" << id << "[g] = u32x4_t{one[0] | one[1] << 16, one[2] | one[3] << 16, one[4] | one[5] << 16, one[6] | one[7] << 16};\n";
               indent--;
               os << pad() << "}\n";
-              const std::string word = "rw" + id + "[n >> 3][(n & 7) >> 1]";
-              const std::string got = std::string(o.acc.elem == "f16" ? "up_f16(" : "up_bf16(") + "(unsigned short)((n & 1) ? " + word + " >> 16 : " + word + "))";
-              const bool zero = pred.empty() || (o.acc.other_value < 0 && (!o.acc.has_other || (o.acc.other_f == 0.0 && !std::signbit(o.acc.other_f))));
-              held[o.result] = {"rw" + id, ls, "(" + (zero ? got : "(" + pred + ") ? " + got + " : " + other_of(o.acc, l0, l1)) + ")"};
+              held[o.result] = {"rw" + id, ls, from_packed(o, "rw" + id, pred, l0, l1)};
               mine.push_back(o.result);
               any_load = true;
             }
