@@ -1005,13 +1005,20 @@ struct Gen {
        << pad() << "  if (arrived == slices - 1) __hip_atomic_store(&counters[32 * lin], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next launch\n"
        << pad() << "}\n" << pad() << "__syncthreads();\n" << pad() << "if (arrived != slices - 1) return;\n";
     // The sums of all results side by side, every thread with sixteen loads in flight; up to 128 of them leave threads over,
-    // which take every PARTS-th slice each (a slice's sum comes from memory: its writer may sit on another XCD).
+    // which take every PARTS-th slice each (a slice's sum comes from memory: its writer may sit on another XCD).  Slices that
+    // do not fill a sixteen are loaded eight, four, two and one at a time: one after the other they took a microsecond each.
     const int64_t parts = total >= 256 ? 1 : 256 / total;
     if (parts > 1) os << pad() << "__shared__ double part[" << parts * total << "];\n";
     os << pad() << "for (int q = threadIdx.x; q < " << parts * total << "; q += 256) {\n"
-       << pad() << "  const int c = q % " << total << ";\n" << pad() << "  double sum = 0;\n" << pad() << "  #pragma unroll 16\n"
-       << pad() << "  for (int s = q / " << total << "; s < slices; s += " << parts << ") sum += __hip_atomic_load(&partial[((long long)s * programs + lin) * " << total
-       << " + c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);\n";
+       << pad() << "  const int c = q % " << total << ";\n" << pad() << "  double sum = 0;\n"
+       << pad() << "  int s = q / " << total << ";\n";
+    for (int width = 16; width; width /= 2) {
+      const std::string w = std::to_string(width), last = std::to_string((width - 1) * parts), step = std::to_string(width * parts);
+      os << pad() << (width == 16 ? "  for (; s + " + last + " < slices; s += " + step + ") {\n" : "  if (s + " + last + " < slices) {\n") << pad() << "    float got[" << w << "];\n"
+         << pad() << "    #pragma unroll\n" << pad() << "    for (int u = 0; u < " << w << "; u++) got[u] = __hip_atomic_load(&partial[((long long)(s + " << parts
+         << " * u) * programs + lin) * " << total << " + c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);\n" << pad() << "    #pragma unroll\n" << pad() << "    for (int u = 0; u < " << w
+         << "; u++) sum += got[u];\n" << (width == 16 ? "" : pad() + "    s += " + step + ";\n") << pad() << "  }\n";
+    }
     auto put = [&](const std::string &sum) {
       int64_t at0 = 0;
       for (const SOp &s : slice_head)
