@@ -802,7 +802,7 @@ tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, con
       if (tile_program_is_sliced(source, &slice_floats, &slice_loop)) {
         // As many workgroups as the device holds at once, each program's loop dealt to an equal number of them, two
         // iterations each at least (dw and db of LayerNorm on fp16 [4096, 8192], 64 programs of 128 iterations: 341 us with
-        // one workgroup per program, 30 us in 12 slices), and no more than 3 sqrt(iterations): an iteration takes some 0.75 us
+        // one workgroup per program, 27 us in 12 slices), and no more than 3 sqrt(iterations): an iteration takes some 0.75 us
         // of a slice and a slice some 0.08 us of the workgroup that adds them all (16 programs of 94 iterations: 47 / 23 / 11
         // slices 15.0 / 13.3 / 16.8 us; of 32 iterations: 16 / 8 / 4 slices 8.2 / 11.4 / 14.7 us).  A launch that may not
         // allocate keeps to one slice, and so does one that is recorded into a graph: the graph may be replayed beside
@@ -837,8 +837,8 @@ tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, con
       a.swap_xy = tile_program_swaps_grid(source) && gy > 1 && gx <= 65535 ? 1 : 0;
       // A workgroup per program.  (A few workgroups per CU that walk the programs with the weights they share held in
       // registers lose since every row moves in 16-byte accesses, us walking / a workgroup each: LayerNorm's dx bf16 [8192, 4096]
-      // 54.3 / 42.8, [8192, 2048] 32.4 / 24.4, [8192, 3001] 57.8 / 45.3; RMSNorm fp16 [8000, 5120] 38.1 / 34.5, [8000, 4096]
-      // 28.7 / 25.2, [4096, 8192] 26.7 / 26.2; ahead only on few whole rows of 8192, [2000, 8192] 14.8 / 15.0.)
+      // 54.3 / 42.8, [8192, 2048] 32.4 / 24.4, [8192, 3001] 57.8 / 45.3; RMSNorm fp16 [8000, 5120] 38.1 / 33.1, [8000, 4096]
+      // 28.7 / 25.3; ahead only on some numbers of whole rows of 8192, [2000, 8192] 14.7 / 16.2, [2760, 8192] 18.6 / 20.0.)
       if (!grid_fits(a.swap_xy)) {
         a.swap_xy = 0;
         a.lgx = gx; a.lgy = gy; a.lgz = gz;

@@ -827,8 +827,10 @@ struct Gen {
   }
   // Loads that the run after the next reduction makes of a block laid out like this run's -- the row of weights of a
   // normalisation -- are issued behind this run's and wait, packed, in `ahead` registers (32 of them at most): made where they
-  // stand, after the reduction, their way from L2 is added to the row's from memory.  They stay packed until each element's use.  RMSNorm fp16 from HBM, us after / behind:
-  // [4096, 8192] 28.5 / 26.0, [2000, 8192] 15.5 / 14.9, [8000, 5120] 35.9 / 34.5, [8000, 4096] 26.5 / 25.3, [16000, 2048] 31.0 / 28.1.
+  // stand, after the reduction, their way from L2 is added to the row's from memory.  RMSNorm fp16 from
+  // HBM, us after / behind: [8000, 5120] 35.9 / 33.1, [8000, 4096] 26.5 / 25.3, [16000, 2048] 31.0 / 29.3, [4096, 8192] 28.5 / 27.8, [2000, 8192]
+  // 15.5 / 16.2.  They stay packed until each element's use: widened at once, rows of 16384 hold two workgroups per CU instead of three
+  // (bf16 [630, 14336] 15.6 / 12.5); some whole rows of 8192 are ahead widened (25.5 and 15.1), others behind (125 sizes: 2 % in the mean).
   std::map<int, std::string> loaded_ahead;  // value id -> the condition under which the loads went in groups (leaves_eight)
   std::vector<const SOp *> loads_of_next_run(const std::vector<SOp> &ops, size_t from, const std::vector<int64_t> &shape, const std::string &roomy) {
     std::vector<const SOp *> loads, none;
