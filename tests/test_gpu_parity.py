@@ -2881,6 +2881,32 @@ def test_gemm_with_fused_epilogue(M, N, K, kernel, dtype):
     assert ((c.double() - want).norm() / want.norm()) <= 1e-2
 
 
+@pytest.mark.parametrize("M,N,K", [(2, 3, 5), (33, 31, 17), (128, 64, 448), (1000, 1021, 33), (1500, 1537, 16), (2900, 2999, 40)])  # every fp32 tiling
+def test_fp32_gemm_with_fused_epilogue(M, N, K):
+    import extra_kernels as X
+    g = torch.Generator(device="cpu").manual_seed(M + K)
+    a, b = (torch.randint(-4, 5, s, generator=g).float().to(DEV) for s in ((M, K), (K, N)))
+    c = torch.full((M, N), 7.0, device=DEV)
+    launch = lambda **kw: X.matmul_leaky[(triton.cdiv(M, 32), triton.cdiv(N, 64))](a, b, c, M, N, K, K, N, N, 0.5, BM=32, BN=64, BK=16, **kw)
+    k = launch()
+    torch.cuda.synchronize()
+    assert k.function.family == "gemm" and k.function.last_kernel == "gemm_f32_kernel + epilogue (hipRTC)"
+    assert torch.equal(c, torch.nn.functional.leaky_relu(a @ b, 0.5))   # (small integers: exact)
+    a, b = torch.randn(M, K, device=DEV), torch.randn(K, N, device=DEV)
+    launch(ACT=1)
+    z = a.double() @ b.double()
+    want = z * torch.sigmoid(z * 0.5)
+    # fp32 sums of K products in any order, then an activation of slope at most 1.1: well within (K + 8) roundings
+    assert ((c.double() - want).norm() / want.norm()).item() <= (K + 8) * 2.0 ** -24 * 2
+    # what depends on the element's position stays on the generic kernel
+    held = torch.randint(-8, 9, (M, N), generator=g).float().to(DEV)
+    c.copy_(held)
+    a, b = (torch.randint(-4, 5, s, generator=g).float().to(DEV) for s in ((M, K), (K, N)))
+    k = launch(ACT=3)
+    torch.cuda.synchronize()
+    assert k.function.last_kernel.startswith("tile_program") and torch.equal(c, (a @ b) * 0.5 + held)
+
+
 @pytest.mark.parametrize("M,N,Kd,sliced", [(2, 8, 4096, True), (100, 264, 4096, True), (300, 2056, 2048, True), (500, 4096, 4096, True), (130, 264, 96, False),
                                            (4090, 2056, 64, False), (4000, 2040, 512, False), (3500, 4096, 512, False), (2041, 2048, 512, False)])
 def test_fused_epilogue_on_every_direct_to_lds_tile(M, N, Kd, sliced):

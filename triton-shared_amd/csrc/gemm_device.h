@@ -1,8 +1,8 @@
-// Device code of the 16-bit matrix-product kernels, in a header of its own because it is compiled twice: ahead of
+// Device code of the 16-bit and fp32 matrix-product kernels, in a header of its own because it is compiled twice: ahead of
 // time into the library (kernels_gemm.hip, results stored as they are), and at run time with hipRTC when the Triton
 // kernel applies elementwise ops to the accumulator before the store (a fused activation): the generated source
 // defines TTS_GEMM_RTC (which kernel: 0 whole 256 x 256 x 32 tiles, 1 any shape in 128 x 128 x 64 tiles, 2 the sum of the K
-// slices, 3 as 1 in 64 x 128 x 64 tiles, 4 and up the other direct-to-LDS tiles), TTS_GEMM_BF16 and the functor TtsEp (a plain struct, passed as the kernel's last argument) that maps an accumulator value and its position to the value stored, then this file's text.  Nothing here may need a host header.
+// slices, 3 as 1 in 64 x 128 x 64 tiles, 4 ... 6 the other direct-to-LDS tiles, 7 ... 10 fp32 operands in four tilings), TTS_GEMM_BF16 and the functor TtsEp (a plain struct, passed as the kernel's last argument) that maps an accumulator value and its position to the value stored, then this file's text.  Nothing here may need a host header.
 #pragma once
 #ifdef __HIPCC_RTC__
 typedef __INT64_TYPE__ int64_t;
@@ -1150,14 +1150,230 @@ __device__ __forceinline__ void gemm_dma16_body(const GemmParams &p, int tiles_m
   __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 15));  // the surplus loads land before the LDS goes away
 }
 
+// ------------------------------------------------------------- fp32 GEMM
+// tl.dot on fp32 blocks: the reference multiplies in fp32 (linalg.matmul on f32, ConversionPatterns.hpp:1128-1201; it
+// ignores the dot's inputPrecision), so this kernel uses the fp32 matrix instruction (v_mfma_f32_32x32x2_f32), not a
+// reduced-precision one.  Any shape and alignment, A and B row- or column-major.
+// Largest workgroup: 128 x 128 of C, 2 x 2 wavefronts of 64 x 64 (2 x 2 MFMA tiles of 32 x 32, 64 accumulator registers), K in
+// steps of 16.  Both operand tiles sit in LDS as [k][r] (r = row of A / column of B, pitch = tile + 4 floats): a lane's MFMA
+// operand is element (k0 + lane / 32, r0 + lane % 32), so a wavefront reads two runs of 32 consecutive floats.
+// Tiles go global -> registers -> LDS with the next tile's loads in flight during the current tile's arithmetic (two
+// LDS buffers, one barrier per tile); 16-byte global loads along whichever dimension is contiguous in memory.
+// T: MFMA tiles per wavefront and dimension, W: wavefronts per dimension: 2, 2 = 128 x 128 per workgroup; 1, 2 = 64 x 64 (for
+// problems that give fewer than two of the large tiles per CU); 1, 1 = 32 x 32 (for those that do not fill the chip with 64 x 64:
+// a tile's matrix instructions all run on one CU, 13 us of them for a 64 x 64 tile at K = 1000).
+// G: groups of W x W wavefronts that split the K tiles among them and add their sums through LDS at the end, in group order:
+// the chain of loads, LDS stores and matrix instructions of a group is 1 / G as long, and the SIMDs have several to run.
+// All K tiles but the last load 16 bytes a chunk, at any alignment and without a test, two tiles ahead; the last goes element by
+// element where a chunk sticks out (gemm_mfma_body reads that one in 16 bytes, too).
+// 768^3: 39.3 -> 17.6 us; 16 x 1000 x 1000: 11.7 (27 with 64 x 64 tiles).  (Eight groups at 768^3: 25.3.)
+constexpr int F32_BK = 16;
+
+template <int T, int W, int G, class Ep>
+__device__ __forceinline__ void gemm_f32_body(const GemmParams &p, int tiles_m, int tiles_n, const Ep &ep) {
+  constexpr int BT = 32 * T * W;      // rows of A / columns of B per workgroup
+  constexpr int PITCH = BT + 4;       // floats between k rows in LDS
+  constexpr int NT = 64 * W * W;      // threads per group
+  constexpr int CH = 4 * BT / NT;     // chunks of 4 floats per thread and operand tile (BT x 16 floats = 4 BT chunks)
+  __shared__ __align__(16) float stage[G][2][2][F32_BK * PITCH];  // [group][buffer][A, B][k][r]
+  static_assert(sizeof(stage) >= (size_t)(G - 1) * BT * BT * sizeof(float), "the groups' sums fit where the tiles were");
+  const int tid = threadIdx.x % NT, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int group = G > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / NT) : 0;
+  float(&smem)[2][2][F32_BK * PITCH] = stage[group];
+  const int wm = wave / W, wn = wave % W;
+  int bid = blockIdx.x;
+  const int nwg = tiles_m * tiles_n;
+  if (nwg % 8 == 0) bid = (bid % 8) * (nwg / 8) + bid / 8;  // consecutive ids on one XCD
+  const int tall = 8 * tiles_n;
+  const int g0 = (bid / tall) * 8;
+  const int gh = min(tiles_m - g0, 8);
+  const int tile_m = g0 + (bid % tall) % gh, tile_n = (bid % tall) / gh;
+  const int64_t m0 = (int64_t)tile_m * BT, n0 = (int64_t)tile_n * BT;
+  const float *__restrict__ A = (const float *)p.a;
+  const float *__restrict__ B = (const float *)p.b;
+  const int64_t K = p.K;
+  const bool a_r = p.a_trans != 0, b_r = p.b_trans == 0;  // r contiguous in memory
+
+  const int64_t nk_all = (K + F32_BK - 1) / F32_BK;
+  const int64_t k_begin = nk_all * group / G, nk = nk_all * (group + 1) / G;  // this group's K tiles
+  const int64_t steps = W > 1 ? (nk_all + G - 1) / G : nk - k_begin;          // the most any group has, where they meet at barriers
+  // K tiles below nwide load whole chunks: rows (columns) beyond the problem are replaced by others whose results nobody
+  // stores, and a chunk that ends behind its row reads into the next, which the last k row does not have
+  int64_t nwide = K / F32_BK;
+  if ((a_r && p.lda < 4) || (b_r && p.ldb < 4)) nwide = 0;
+  else if (K % F32_BK == 0 && ((a_r && m0 + BT > p.M) || (b_r && n0 + BT > p.N))) nwide = nk_all - 1;
+  nwide = min(nwide, nk);
+
+  // An operand tile is BT r x 16 k = 4 BT chunks of 4 floats, CH per thread.  k contiguous in memory (A row-major, B
+  // column-major): chunk c = (r = c / 4, k = 4 (c % 4)); r contiguous (A column-major, B row-major): (k = c / (BT / 4), r = 4 (c % (BT / 4))).
+  struct Tiles { float4 a[CH], b[CH]; };
+  const float *a_ptr[CH], *b_ptr[CH];
+  auto chunk_ptr = [&](const float *P, bool r_contig, int64_t ld, int64_t r_base, int64_t rows, int c) {
+    if (r_contig) {
+      const int64_t r = r_base + 4 * (c % (BT / 4));
+      return P + (int64_t)(c / (BT / 4)) * ld + (r < rows ? r : 0);
+    }
+    return P + min(r_base + c / 4, rows - 1) * ld + 4 * (c % 4);
+  };
+#pragma unroll
+  for (int j = 0; j < CH; j++) {
+    a_ptr[j] = chunk_ptr(A, a_r, p.lda, m0, p.M, tid + NT * j);
+    b_ptr[j] = chunk_ptr(B, b_r, p.ldb, n0, p.N, tid + NT * j);
+  }
+  const int64_t a_step = F32_BK * (a_r ? p.lda : 1), b_step = F32_BK * (b_r ? p.ldb : 1);
+  auto load_wide = [&](Tiles &t, int64_t kt) {
+#pragma unroll
+    for (int j = 0; j < CH; j++) __builtin_memcpy(&t.a[j], a_ptr[j] + kt * a_step, 16);
+#pragma unroll
+    for (int j = 0; j < CH; j++) __builtin_memcpy(&t.b[j], b_ptr[j] + kt * b_step, 16);
+  };
+  auto load_edge = [&](float4 (&reg)[CH], const float *P, bool r_contig, int64_t ld, int64_t r_base, int64_t rows, int64_t k0) {
+#pragma unroll
+    for (int j = 0; j < CH; j++) {
+      const int c = tid + NT * j;
+      float v[4] = {0.f, 0.f, 0.f, 0.f};
+      if (r_contig) {
+        const int64_t k = k0 + c / (BT / 4), r = r_base + 4 * (c % (BT / 4));
+        if (k < K)
+          for (int i = 0; i < 4; i++) if (r + i < rows) v[i] = P[k * ld + r + i];
+      } else {
+        const int64_t r = r_base + c / 4, k = k0 + 4 * (c % 4);
+        if (r < rows)
+          for (int i = 0; i < 4; i++) if (k + i < K) v[i] = P[r * ld + k + i];
+      }
+      reg[j] = make_float4(v[0], v[1], v[2], v[3]);
+    }
+  };
+  auto load_any = [&](Tiles &t, int64_t kt) {
+    if (kt < nwide) load_wide(t, kt);
+    else if (kt < nk) {
+      load_edge(t.a, A, a_r, p.lda, m0, p.M, kt * F32_BK);
+      load_edge(t.b, B, b_r, p.ldb, n0, p.N, kt * F32_BK);
+    }
+  };
+  auto store_tile = [&](const float4 (&reg)[CH], float *S, bool r_contig) {
+#pragma unroll
+    for (int j = 0; j < CH; j++) {
+      const int c = tid + NT * j;
+      if (r_contig) {
+        *reinterpret_cast<float4 *>(S + (c / (BT / 4)) * PITCH + 4 * (c % (BT / 4))) = reg[j];
+      } else {  // four k of one r: one float into each of four k rows
+        float *dst = S + (4 * (c % 4)) * PITCH + c / 4;
+        dst[0] = reg[j].x; dst[PITCH] = reg[j].y; dst[2 * PITCH] = reg[j].z; dst[3 * PITCH] = reg[j].w;
+      }
+    }
+  };
+  auto store_tiles = [&](const Tiles &t, int buf) {
+    store_tile(t.a, smem[buf][0], a_r);
+    store_tile(t.b, smem[buf][1], b_r);
+  };
+  f32x16 acc[T][T];
+#pragma unroll
+  for (int i = 0; i < T; i++)
+#pragma unroll
+    for (int j = 0; j < T; j++)
+#pragma unroll
+      for (int v = 0; v < 16; v++) acc[i][j][v] = 0.f;
+  auto multiply = [&](int buf) {
+    const float *As = smem[buf][0] + (lane >> 5) * PITCH + wm * (32 * T) + (lane & 31);
+    const float *Bs = smem[buf][1] + (lane >> 5) * PITCH + wn * (32 * T) + (lane & 31);
+#pragma unroll
+    for (int ks = 0; ks < F32_BK; ks += 2) {
+      float af[T], bf[T];
+#pragma unroll
+      for (int i = 0; i < T; i++) af[i] = As[ks * PITCH + 32 * i];
+#pragma unroll
+      for (int j = 0; j < T; j++) bf[j] = Bs[ks * PITCH + 32 * j];
+#pragma unroll
+      for (int i = 0; i < T; i++)
+#pragma unroll
+        for (int j = 0; j < T; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(af[i], bf[j], acc[i][j], 0, 0, 0);
+    }
+  };
+  // Groups of one wavefront share nothing until the end: a wavefront's LDS accesses complete in order.  Others meet at
+  // barriers (a turn of either loop has two: every group meets the same number, also when it has a tile fewer).
+  auto sync = [&]() {
+    if constexpr (W > 1) __syncthreads();
+    else {
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    }
+  };
+  Tiles even, odd;
+  load_any(even, k_begin);
+  load_any(odd, k_begin + 1);
+  if (k_begin < nk) store_tiles(even, 0);
+  load_any(even, k_begin + 2);
+  sync();
+  int64_t kt = k_begin, step = 0;
+  for (; kt + 4 < nwide; step += 2, kt += 2) {  // loads tiles kt + 3 and kt + 4
+    multiply(0);
+    store_tiles(odd, 1);
+    load_wide(odd, kt + 3);
+    sync();
+    multiply(1);
+    store_tiles(even, 0);
+    load_wide(even, kt + 4);
+    sync();
+  }
+  for (; step < steps; step += 2, kt += 2) {
+    if (kt < nk) multiply(0);
+    if (kt + 1 < nk) store_tiles(odd, 1);
+    load_any(odd, kt + 3);
+    sync();
+    if (kt + 1 < nk) multiply(1);
+    if (kt + 2 < nk) store_tiles(even, 0);
+    load_any(even, kt + 4);
+    sync();
+  }
+  if constexpr (G > 1) {
+    if (W == 1) __syncthreads();  // (the last barrier of the loop otherwise) the tiles are free
+    float *sums = reinterpret_cast<float *>(stage);
+    auto place = [&](int g, int i, int j, int v) { return (((g * W * W + wave) * T + i) * T + j) * 1024 + v * 64 + lane; };
+#pragma unroll
+    for (int i = 0; i < T; i++)
+#pragma unroll
+      for (int j = 0; j < T; j++)
+#pragma unroll
+        for (int v = 0; v < 16; v++)
+          if (group > 0) sums[place(group - 1, i, j, v)] = acc[i][j][v];
+    __syncthreads();
+    if (group > 0) return;
+#pragma unroll
+    for (int g = 0; g < G - 1; g++)
+#pragma unroll
+      for (int i = 0; i < T; i++)
+#pragma unroll
+        for (int j = 0; j < T; j++)
+#pragma unroll
+          for (int v = 0; v < 16; v++) acc[i][j][v] += sums[place(g, i, j, v)];
+  }
+  // lane holds column (lane % 32), rows 8 (v / 4) + 4 (lane / 32) + v % 4 of each 32 x 32 tile
+  float *__restrict__ C = (float *)p.c;
+#pragma unroll
+  for (int i = 0; i < T; i++)
+#pragma unroll
+    for (int j = 0; j < T; j++) {
+      const int64_t col = n0 + wn * (32 * T) + j * 32 + (lane & 31);
+#pragma unroll
+      for (int v = 0; v < 16; v++) {
+        const int64_t row = m0 + wm * (32 * T) + i * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
+        if (row < p.M && col < p.N) C[row * p.ldc + col] = ep(acc[i][j][v], row, col);
+      }
+    }
+}
+
 }  // namespace tts_gemm_device
 
 #ifdef TTS_GEMM_RTC
-extern "C" __global__ __launch_bounds__(256) void gemm_rtc(TtsGemmParams p, int tiles_m, int tiles_n, TtsEp ep) {
+extern "C" __global__ __launch_bounds__(TTS_GEMM_RTC == 9 ? 512 : 256) void gemm_rtc(TtsGemmParams p, int tiles_m, int tiles_n, TtsEp ep) {
 #if TTS_GEMM_RTC == 0
   tts_gemm_device::gemm_dma16_body<TTS_GEMM_BF16 != 0>(p, tiles_m, tiles_n, ep);
 #elif TTS_GEMM_RTC == 2
   tts_gemm_device::gemm_splitk_reduce_body<TTS_GEMM_BF16 != 0>(p, tiles_m, tiles_n, ep);  // (across, col_blocks)
+#elif TTS_GEMM_RTC >= 7
+  constexpr int T = TTS_GEMM_RTC == 7 ? 2 : 1, W = TTS_GEMM_RTC == 8 ? 1 : 2, G = TTS_GEMM_RTC == 8 ? 4 : TTS_GEMM_RTC == 9 ? 2 : 1;
+  tts_gemm_device::gemm_f32_body<T, W, G>(p, tiles_m, tiles_n, ep);
 #elif TTS_GEMM_RTC >= 4
   constexpr int TM = TTS_GEMM_RTC == 5 ? 4 : 2, TN = TTS_GEMM_RTC == 4 ? 4 : 2;  // 128 x 256, 256 x 128, 128 x 128
   tts_gemm_device::gemm_dma_body<TTS_GEMM_BF16 != 0, TM, TN>(p, tiles_m, tiles_n, ep);

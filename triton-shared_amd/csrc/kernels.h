@@ -101,7 +101,7 @@ hipError_t launch_gemm(const GemmParams &p, hipStream_t s, const char **kernel_n
 // The same product with elementwise ops fused into the epilogue: `epilogue` is the source of the functor (match.h:
 // gemm_epilogue_source), `modules` the plan's slots for the kernels compiled from it (one per tiling and the sum of K slices,
 // filled at the first launch that needs it and may compile), `args` / `args_size` the generic families' argument block.
-constexpr int GEMM_EPILOGUE_KERNELS = 7;
+constexpr int GEMM_EPILOGUE_KERNELS = 11;
 struct RtcModule;
 // The epilogue functor as the kernel receives it (the generated `struct TtsEp` has this layout): every kernel argument
 // by index, then what it takes to find the Triton program that owns an element -- tile_pid[(row / BM) * tiles_n +

@@ -181,240 +181,31 @@ bool gemm_dma_ok(const GemmParams &p, int64_t bm, int64_t bn) {
 }
 bool gemm_fast_path_ok(const GemmParams &p) { return !p.a_trans && !p.b_trans && gemm_dma_ok(p, F_BM, F_BN); }  // (the kernel compiled with an epilogue)
 
-// ------------------------------------------------------------- fp32 GEMM
-// tl.dot on fp32 blocks: the reference multiplies in fp32 (linalg.matmul on f32, ConversionPatterns.hpp:1128-1201; it
-// ignores the dot's inputPrecision), so this kernel uses the fp32 matrix instruction (v_mfma_f32_32x32x2_f32), not a
-// reduced-precision one.  Any shape and alignment, A and B row- or column-major.
-// Largest workgroup: 128 x 128 of C, 2 x 2 wavefronts of 64 x 64 (2 x 2 MFMA tiles of 32 x 32, 64 accumulator registers), K in
-// steps of 16.  Both operand tiles sit in LDS as [k][r] (r = row of A / column of B, pitch = tile + 4 floats): a lane's MFMA
-// operand is element (k0 + lane / 32, r0 + lane % 32), so a wavefront reads two runs of 32 consecutive floats.
-// Tiles go global -> registers -> LDS with the next tile's loads in flight during the current tile's arithmetic (two
-// LDS buffers, one barrier per tile); 16-byte global loads along whichever dimension is contiguous in memory.
-// T: MFMA tiles per wavefront and dimension, W: wavefronts per dimension: 2, 2 = 128 x 128 per workgroup; 1, 2 = 64 x 64 (for
-// problems that give fewer than two of the large tiles per CU); 1, 1 = 32 x 32 (for those that do not fill the chip with 64 x 64:
-// a tile's matrix instructions all run on one CU, 13 us of them for a 64 x 64 tile at K = 1000).
-// G: groups of W x W wavefronts that split the K tiles among them and add their sums through LDS at the end, in group order:
-// the chain of loads, LDS stores and matrix instructions of a group is 1 / G as long, and the SIMDs have several to run.
-// All K tiles but the last load 16 bytes a chunk, at any alignment and without a test, two tiles ahead; the last goes element by
-// element where a chunk sticks out (gemm_mfma_body reads that one in 16 bytes, too).
-// 768^3: 39.3 -> 17.6 us; 16 x 1000 x 1000: 11.7 (27 with 64 x 64 tiles).  (Eight groups at 768^3: 25.3.)
-constexpr int F32_BK = 16;
-
+// ------------------------------------------------------------- fp32 GEMM (gemm_device.h: gemm_f32_body)
 template <int T, int W, int G>
 __global__ __launch_bounds__(64 * W * W * G) void gemm_f32_kernel(GemmParams batch, int tiles_m, int tiles_n) {
-  const GemmParams p = of_batch(batch, 4);
-  constexpr int BT = 32 * T * W;      // rows of A / columns of B per workgroup
-  constexpr int PITCH = BT + 4;       // floats between k rows in LDS
-  constexpr int NT = 64 * W * W;      // threads per group
-  constexpr int CH = 4 * BT / NT;     // chunks of 4 floats per thread and operand tile (BT x 16 floats = 4 BT chunks)
-  __shared__ __align__(16) float stage[G][2][2][F32_BK * PITCH];  // [group][buffer][A, B][k][r]
-  static_assert(sizeof(stage) >= (size_t)(G - 1) * BT * BT * sizeof(float), "the groups' sums fit where the tiles were");
-  const int tid = threadIdx.x % NT, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int group = G > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / NT) : 0;
-  float(&smem)[2][2][F32_BK * PITCH] = stage[group];
-  const int wm = wave / W, wn = wave % W;
-  int bid = blockIdx.x;
-  const int nwg = tiles_m * tiles_n;
-  if (nwg % 8 == 0) bid = (bid % 8) * (nwg / 8) + bid / 8;  // consecutive ids on one XCD
-  const int tall = 8 * tiles_n;
-  const int g0 = (bid / tall) * 8;
-  const int gh = min(tiles_m - g0, 8);
-  const int tile_m = g0 + (bid % tall) % gh, tile_n = (bid % tall) / gh;
-  const int64_t m0 = (int64_t)tile_m * BT, n0 = (int64_t)tile_n * BT;
-  const float *__restrict__ A = (const float *)p.a;
-  const float *__restrict__ B = (const float *)p.b;
-  const int64_t K = p.K;
-  const bool a_r = p.a_trans != 0, b_r = p.b_trans == 0;  // r contiguous in memory
-
-  const int64_t nk_all = (K + F32_BK - 1) / F32_BK;
-  const int64_t k_begin = nk_all * group / G, nk = nk_all * (group + 1) / G;  // this group's K tiles
-  const int64_t steps = W > 1 ? (nk_all + G - 1) / G : nk - k_begin;          // the most any group has, where they meet at barriers
-  // K tiles below nwide load whole chunks: rows (columns) beyond the problem are replaced by others whose results nobody
-  // stores, and a chunk that ends behind its row reads into the next, which the last k row does not have
-  int64_t nwide = K / F32_BK;
-  if ((a_r && p.lda < 4) || (b_r && p.ldb < 4)) nwide = 0;
-  else if (K % F32_BK == 0 && ((a_r && m0 + BT > p.M) || (b_r && n0 + BT > p.N))) nwide = nk_all - 1;
-  nwide = min(nwide, nk);
-
-  // An operand tile is BT r x 16 k = 4 BT chunks of 4 floats, CH per thread.  k contiguous in memory (A row-major, B
-  // column-major): chunk c = (r = c / 4, k = 4 (c % 4)); r contiguous (A column-major, B row-major): (k = c / (BT / 4), r = 4 (c % (BT / 4))).
-  struct Tiles { float4 a[CH], b[CH]; };
-  const float *a_ptr[CH], *b_ptr[CH];
-  auto chunk_ptr = [&](const float *P, bool r_contig, int64_t ld, int64_t r_base, int64_t rows, int c) {
-    if (r_contig) {
-      const int64_t r = r_base + 4 * (c % (BT / 4));
-      return P + (int64_t)(c / (BT / 4)) * ld + (r < rows ? r : 0);
-    }
-    return P + min(r_base + c / 4, rows - 1) * ld + 4 * (c % 4);
-  };
-#pragma unroll
-  for (int j = 0; j < CH; j++) {
-    a_ptr[j] = chunk_ptr(A, a_r, p.lda, m0, p.M, tid + NT * j);
-    b_ptr[j] = chunk_ptr(B, b_r, p.ldb, n0, p.N, tid + NT * j);
-  }
-  const int64_t a_step = F32_BK * (a_r ? p.lda : 1), b_step = F32_BK * (b_r ? p.ldb : 1);
-  auto load_wide = [&](Tiles &t, int64_t kt) {
-#pragma unroll
-    for (int j = 0; j < CH; j++) __builtin_memcpy(&t.a[j], a_ptr[j] + kt * a_step, 16);
-#pragma unroll
-    for (int j = 0; j < CH; j++) __builtin_memcpy(&t.b[j], b_ptr[j] + kt * b_step, 16);
-  };
-  auto load_edge = [&](float4 (&reg)[CH], const float *P, bool r_contig, int64_t ld, int64_t r_base, int64_t rows, int64_t k0) {
-#pragma unroll
-    for (int j = 0; j < CH; j++) {
-      const int c = tid + NT * j;
-      float v[4] = {0.f, 0.f, 0.f, 0.f};
-      if (r_contig) {
-        const int64_t k = k0 + c / (BT / 4), r = r_base + 4 * (c % (BT / 4));
-        if (k < K)
-          for (int i = 0; i < 4; i++) if (r + i < rows) v[i] = P[k * ld + r + i];
-      } else {
-        const int64_t r = r_base + c / 4, k = k0 + 4 * (c % 4);
-        if (r < rows)
-          for (int i = 0; i < 4; i++) if (k + i < K) v[i] = P[r * ld + k + i];
-      }
-      reg[j] = make_float4(v[0], v[1], v[2], v[3]);
-    }
-  };
-  auto load_any = [&](Tiles &t, int64_t kt) {
-    if (kt < nwide) load_wide(t, kt);
-    else if (kt < nk) {
-      load_edge(t.a, A, a_r, p.lda, m0, p.M, kt * F32_BK);
-      load_edge(t.b, B, b_r, p.ldb, n0, p.N, kt * F32_BK);
-    }
-  };
-  auto store_tile = [&](const float4 (&reg)[CH], float *S, bool r_contig) {
-#pragma unroll
-    for (int j = 0; j < CH; j++) {
-      const int c = tid + NT * j;
-      if (r_contig) {
-        *reinterpret_cast<float4 *>(S + (c / (BT / 4)) * PITCH + 4 * (c % (BT / 4))) = reg[j];
-      } else {  // four k of one r: one float into each of four k rows
-        float *dst = S + (4 * (c % 4)) * PITCH + c / 4;
-        dst[0] = reg[j].x; dst[PITCH] = reg[j].y; dst[2 * PITCH] = reg[j].z; dst[3 * PITCH] = reg[j].w;
-      }
-    }
-  };
-  auto store_tiles = [&](const Tiles &t, int buf) {
-    store_tile(t.a, smem[buf][0], a_r);
-    store_tile(t.b, smem[buf][1], b_r);
-  };
-  f32x16 acc[T][T];
-#pragma unroll
-  for (int i = 0; i < T; i++)
-#pragma unroll
-    for (int j = 0; j < T; j++)
-#pragma unroll
-      for (int v = 0; v < 16; v++) acc[i][j][v] = 0.f;
-  auto multiply = [&](int buf) {
-    const float *As = smem[buf][0] + (lane >> 5) * PITCH + wm * (32 * T) + (lane & 31);
-    const float *Bs = smem[buf][1] + (lane >> 5) * PITCH + wn * (32 * T) + (lane & 31);
-#pragma unroll
-    for (int ks = 0; ks < F32_BK; ks += 2) {
-      float af[T], bf[T];
-#pragma unroll
-      for (int i = 0; i < T; i++) af[i] = As[ks * PITCH + 32 * i];
-#pragma unroll
-      for (int j = 0; j < T; j++) bf[j] = Bs[ks * PITCH + 32 * j];
-#pragma unroll
-      for (int i = 0; i < T; i++)
-#pragma unroll
-        for (int j = 0; j < T; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(af[i], bf[j], acc[i][j], 0, 0, 0);
-    }
-  };
-  // Groups of one wavefront share nothing until the end: a wavefront's LDS accesses complete in order.  Others meet at
-  // barriers (a turn of either loop has two: every group meets the same number, also when it has a tile fewer).
-  auto sync = [&]() {
-    if constexpr (W > 1) __syncthreads();
-    else {
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-    }
-  };
-  Tiles even, odd;
-  load_any(even, k_begin);
-  load_any(odd, k_begin + 1);
-  if (k_begin < nk) store_tiles(even, 0);
-  load_any(even, k_begin + 2);
-  sync();
-  int64_t kt = k_begin, step = 0;
-  for (; kt + 4 < nwide; step += 2, kt += 2) {  // loads tiles kt + 3 and kt + 4
-    multiply(0);
-    store_tiles(odd, 1);
-    load_wide(odd, kt + 3);
-    sync();
-    multiply(1);
-    store_tiles(even, 0);
-    load_wide(even, kt + 4);
-    sync();
-  }
-  for (; step < steps; step += 2, kt += 2) {
-    if (kt < nk) multiply(0);
-    if (kt + 1 < nk) store_tiles(odd, 1);
-    load_any(odd, kt + 3);
-    sync();
-    if (kt + 1 < nk) multiply(1);
-    if (kt + 2 < nk) store_tiles(even, 0);
-    load_any(even, kt + 4);
-    sync();
-  }
-  if constexpr (G > 1) {
-    if (W == 1) __syncthreads();  // (the last barrier of the loop otherwise) the tiles are free
-    float *sums = reinterpret_cast<float *>(stage);
-    auto place = [&](int g, int i, int j, int v) { return (((g * W * W + wave) * T + i) * T + j) * 1024 + v * 64 + lane; };
-#pragma unroll
-    for (int i = 0; i < T; i++)
-#pragma unroll
-      for (int j = 0; j < T; j++)
-#pragma unroll
-        for (int v = 0; v < 16; v++)
-          if (group > 0) sums[place(group - 1, i, j, v)] = acc[i][j][v];
-    __syncthreads();
-    if (group > 0) return;
-#pragma unroll
-    for (int g = 0; g < G - 1; g++)
-#pragma unroll
-      for (int i = 0; i < T; i++)
-#pragma unroll
-        for (int j = 0; j < T; j++)
-#pragma unroll
-          for (int v = 0; v < 16; v++) acc[i][j][v] += sums[place(g, i, j, v)];
-  }
-  // lane holds column (lane % 32), rows 8 (v / 4) + 4 (lane / 32) + v % 4 of each 32 x 32 tile
-  float *__restrict__ C = (float *)p.c;
-#pragma unroll
-  for (int i = 0; i < T; i++)
-#pragma unroll
-    for (int j = 0; j < T; j++) {
-      const int64_t col = n0 + wn * (32 * T) + j * 32 + (lane & 31);
-#pragma unroll
-      for (int v = 0; v < 16; v++) {
-        const int64_t row = m0 + wm * (32 * T) + i * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
-        if (row < p.M && col < p.N) C[row * p.ldc + col] = acc[i][j][v];
-      }
-    }
+  gemm_f32_body<T, W, G>(of_batch(batch, 4), tiles_m, tiles_n, IdentityEp());
 }
 
-hipError_t launch_gemm_f32(const GemmParams &p, hipStream_t s) {
-  static const int cus = [] {
-    int dev = 0, n = 0;
-    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-    return n;
-  }();
-  const int batches = std::max(1, p.batches);
-  auto tiles = [&](int64_t t) { return ((p.M + t - 1) / t) * ((p.N + t - 1) / t) * batches; };
-  auto launch = [&](auto kern, int t, int threads) {
-    const int tiles_m = (int)((p.M + t - 1) / t), tiles_n = (int)((p.N + t - 1) / t);
-    hipLaunchKernelGGL(kern, dim3(tiles_m * tiles_n, batches), dim3(threads), 0, s, p, tiles_m, tiles_n);
-    return hipGetLastError();
-  };
+// The tilings gemm_f32_body is built for: edge of a workgroup's tile, threads.
+struct F32Tiling { int edge, threads; };
+constexpr F32Tiling F32_TILINGS[4] = {{128, 256}, {32, 256}, {64, 512}, {64, 256}};
+int f32_tiling(const GemmParams &p) {
+  const int cus = device_cus();
+  auto tiles = [&](int64_t t) { return ((p.M + t - 1) / t) * ((p.N + t - 1) / t) * std::max(1, p.batches); };
   // Where the lines lie, us with 64 x 64 tiles / those in two groups / 32 x 32 tiles in four: 400 x 600 x 800 23.1 / 21.7 / 11.9;
   // 768^3 (576 small tiles) 22.3 / 20.7 / 17.6; 1000^3 (1024) 30.1 / 27.3 / 36.8; 1024 x 2048 x 1024 (512 tiles of 64) 49.0 /
   // 48.6 / 62.9; 1500 x 1500 x 1000 (576) 65.5 / 67.1 / 75.0.
-  if (tiles(128) >= 2 * cus) return launch(gemm_f32_kernel<2, 2, 1>, 128, 256);
-  if (2 * tiles(32) <= 5 * cus) return launch(gemm_f32_kernel<1, 1, 4>, 32, 256);
-  if (tiles(64) <= 2 * cus) return launch(gemm_f32_kernel<1, 2, 2>, 64, 512);
-  return launch(gemm_f32_kernel<1, 2, 1>, 64, 256);
+  if (tiles(128) >= 2 * cus) return 0;
+  if (2 * tiles(32) <= 5 * cus) return 1;
+  return tiles(64) <= 2 * cus ? 2 : 3;
+}
+hipError_t launch_gemm_f32(const GemmParams &p, hipStream_t s) {
+  const int which = f32_tiling(p), t = F32_TILINGS[which].edge;
+  const int tiles_m = (int)((p.M + t - 1) / t), tiles_n = (int)((p.N + t - 1) / t);
+  const auto kern = which == 0 ? gemm_f32_kernel<2, 2, 1> : which == 1 ? gemm_f32_kernel<1, 1, 4> : which == 2 ? gemm_f32_kernel<1, 2, 2> : gemm_f32_kernel<1, 2, 1>;
+  hipLaunchKernelGGL(kern, dim3(tiles_m * tiles_n, std::max(1, p.batches)), dim3(F32_TILINGS[which].threads), 0, s, p, tiles_m, tiles_n);
+  return hipGetLastError();
 }
 
 // ------------------------------------------------------ int8-weight GEMM
@@ -1004,7 +795,8 @@ hipError_t launch_gemm(const GemmParams &p, hipStream_t s, const char **name) {
 
 namespace {
 // The kernels compiled with a functor: 0 whole 256 x 256 x 32 tiles on the 16 x 16 x 32 instruction; 1 any shape in 128 x 128 x 64
-// tiles; 2 the sum of K slices; 3 any shape in 64 x 128 x 64 tiles; 4 ... the other direct-to-LDS tiles, in the order of DMA_CANDS.
+// tiles; 2 the sum of K slices; 3 any shape in 64 x 128 x 64 tiles; 4 ... the other direct-to-LDS tiles, in the order of DMA_CANDS;
+// 7 ... fp32 operands, in the order of F32_TILINGS (768^3 leaky_relu 68 us on the generic kernel, 18 here: the plain product's).
 int epilogue_dma_index(const DmaCand *tile) { return tile == &DMA_CANDS[0] ? 0 : 3 + (int)(tile - DMA_CANDS); }
 
 template <int TM, int TN>
@@ -1018,15 +810,21 @@ hipError_t launch_dma_slices(const GemmParams &p, hipStream_t s) {
 // 1000 x 4096 x 4096 53 / 88; 4096 x 2048 x 2048 40 / 48.6.  (A column-major operand goes to the any-shape kernel.)
 struct EpilogueChoice { int whole, split; const DmaCand *tile; };  // the kernel without slices; the tile the slices run on (null: any shape)
 EpilogueChoice choose_epilogue(const GemmParams &p, int max_split) {
+  if (p.is_f32) return {7 + f32_tiling(p), 1, nullptr};
   if (!gemm_fast_path_ok(p)) return {any_rows(p, 1) == 64 ? 3 : 1, any_split(p, max_split), nullptr};
   const DmaChoice choice = choose_dma(p, max_split);
   if (!choice.tile) return {0, 1, &DMA_CANDS[0]};  // (only where a tuning variable names a tile that does not apply)
   return {epilogue_dma_index(choice.split > 1 ? choose_dma(p, 1).tile : choice.tile), choice.split, choice.tile};
 }
 // A kernel that is compiled already and computes what `whole` does: any direct-to-LDS tile for another of them, the any-shape
-// kernel's 128 rows for its 64 (-1: none).
+// kernel's 128 rows for its 64, any fp32 tiling (-1: none).
 int compiled_epilogue(int whole, RtcModule *const *modules) {
   if (modules[whole]) return whole;
+  if (whole >= 7) {
+    for (int m = 7; m < GEMM_EPILOGUE_KERNELS; m++)
+      if (modules[m]) return m;
+    return -1;
+  }
   if (whole == 1 || whole == 3) return modules[4 - whole] ? 4 - whole : -1;
   for (int m : {0, 4, 5, 6})
     if (modules[m]) return m;
@@ -1047,7 +845,7 @@ hipError_t launch_gemm_epilogue(const GemmParams &p, const std::string &epilogue
   const int whole = may_compile ? choice.whole : compiled_epilogue(choice.whole, modules), which = sliced ? 2 : whole;
   if (which < 0) return hipErrorInvalidValue;  // (gemm_epilogue_compiled said so)
   const bool any_shape = sliced ? !choice.tile : which == 1 || which == 3;
-  *name = any_shape ? any_name(sliced ? any_rows(p, choice.split) : which == 3 ? 64 : 128, true, sliced)
+  *name = p.is_f32 ? "gemm_f32_kernel + epilogue (hipRTC)" : any_shape ? any_name(sliced ? any_rows(p, choice.split) : which == 3 ? 64 : 128, true, sliced)
                     : (sliced ? "gemm_dma_kernel + epilogue (hipRTC), K slices" : "gemm_dma_kernel + epilogue (hipRTC)");
   for (int m : {whole, which}) {
     if (modules[m]) continue;
@@ -1076,6 +874,12 @@ hipError_t launch_gemm_epilogue(const GemmParams &p, const std::string &epilogue
     a.tiles_m = g.across;
     a.tiles_n = g.col_blocks;
     return rtc_launch(modules[2], g.workgroups, 1, 1, 256, &a, sizeof a, s);
+  }
+  if (p.is_f32) {
+    const F32Tiling &t = F32_TILINGS[which - 7];
+    a.tiles_m = (int)((p.M + t.edge - 1) / t.edge);
+    a.tiles_n = (int)((p.N + t.edge - 1) / t.edge);
+    return rtc_launch(modules[which], a.tiles_m * a.tiles_n, 1, 1, t.threads, &a, sizeof a, s);
   }
   const int64_t rows = which == 3 ? 64 : which == 0 || which == 5 ? 256 : 128, cols = which == 0 || which == 4 ? 256 : 128;
   a.tiles_m = (int)((p.M + rows - 1) / rows);

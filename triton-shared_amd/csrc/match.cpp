@@ -1022,22 +1022,28 @@ static bool try_gemm_with_epilogue(Plan &pl) {
   if (loop.results.size() != 1 || loop.results[0] < 0 || st.operands.empty()) return false;
   const int acc = loop.results[0], out = st.operands[0];
   const std::string T = st.acc.elem;
-  if ((T != "bf16" && T != "f16") || P.values[acc].dtype != "f32" || P.values[out].shape != P.values[acc].shape) return false;
+  // (fp32 results: functors of the accumulator alone.  Others stay on the generic kernel, which needs no table of tile owners and so
+  // takes every launch that may not allocate once it is compiled)
+  const bool f32 = T == "f32";
+  if ((!f32 && T != "bf16" && T != "f16") || P.values[acc].dtype != "f32" || P.values[out].shape != P.values[acc].shape) return false;
+  if (f32 && (out == acc || P.values[out].dtype != "f32")) return false;
   if (store_at == loop_at + 2 && P.body[loop_at + 1].kind == SK::Map && P.body[loop_at + 1].name == "arith.truncf" &&
       P.body[loop_at + 1].operands.at(0) == acc)
     return false;  // the plain product: nothing to take out
   // the product without the epilogue
   Program Q = P;
-  Value narrowed = P.values[acc];
-  narrowed.dtype = T;
-  Q.values.push_back(narrowed);
-  SOp cast;
-  cast.kind = SK::Map;
-  cast.name = "arith.truncf";
-  cast.operands = {acc};
-  cast.result = (int)Q.values.size() - 1;
-  SOp store = st;
-  store.operands[0] = cast.result;
+  SOp cast, store = st;
+  store.operands[0] = acc;
+  if (!f32) {
+    Value narrowed = P.values[acc];
+    narrowed.dtype = T;
+    Q.values.push_back(narrowed);
+    cast.kind = SK::Map;
+    cast.name = "arith.truncf";
+    cast.operands = {acc};
+    cast.result = (int)Q.values.size() - 1;
+    store.operands[0] = cast.result;
+  }
   // values the loop reads keep their definitions; what only the epilogue read goes
   std::set<int> used;
   std::function<void(const SOp &)> reads = [&](const SOp &s) {
@@ -1057,7 +1063,7 @@ static bool try_gemm_with_epilogue(Plan &pl) {
   }
   Q.body = kept;
   Q.body.push_back(loop);
-  Q.body.push_back(cast);
+  if (!f32) Q.body.push_back(cast);
   Q.body.push_back(store);
   Plan q;
   q.prog = std::move(Q);
@@ -1067,7 +1073,7 @@ static bool try_gemm_with_epilogue(Plan &pl) {
     std::vector<const SOp *> ops;
     for (auto &s : P.body)
       if (s.kind != SK::For && s.kind != SK::Store) ops.push_back(&s);
-    q.source = gemm_epilogue_source(P, ops, acc, out, q.k.at("BM"), q.k.at("BN"));
+    q.source = gemm_epilogue_source(P, ops, acc, out, q.k.at("BM"), q.k.at("BN"), !f32);
   } catch (const Unsupported &) {
     return false;  // not this shape of program: the other families get their turn
   }

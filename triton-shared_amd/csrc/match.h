@@ -51,7 +51,7 @@ bool tile_program_is_sliced(const std::string &source, int *floats, int *loop);
 bool tile_program_swaps_grid(const std::string &source);  // the launcher exchanges the grid's x and y for this source (when y fits)
 // Matmul family with ops between the K loop and the store: the source of the functor that applies them to one
 // accumulator value (tile_codegen.cpp), compiled at run time together with the kernels of gemm_device.h.
-std::string gemm_epilogue_source(const Program &p, const std::vector<const SOp *> &ops, int acc, int out, int64_t BM, int64_t BN);
+std::string gemm_epilogue_source(const Program &p, const std::vector<const SOp *> &ops, int acc, int out, int64_t BM, int64_t BN, bool owned);
 
 // Normalised listing of a program's ops (no shapes, no expression ids).
 std::string signature(const Program &p);

@@ -490,9 +490,8 @@ void bind_gemm(const Resolver &r, Bound &b) {
   p.is_bf16 = (int)r.pl.k.at("is_bf16");
   p.is_f32 = r.pl.k.count("is_f32") ? (int)r.pl.k.at("is_f32") : 0;
   p.batches = (int)d.batches; p.batch_a = d.batch_a; p.batch_b = d.batch_b; p.batch_c = d.batch_c;
-  if (p.is_f32 && !r.pl.source.empty()) throw Unsupported("gemm: a fused epilogue on fp32 operands");
   if (p.batches > 1 && !r.pl.source.empty()) throw Unsupported("gemm: a fused epilogue on a batch of products");
-  if (!r.pl.source.empty()) {  // a fused epilogue looks up the program that owns an element
+  if (!r.pl.source.empty() && !p.is_f32) {  // a fused epilogue on 16-bit results looks up the program that owns an element
     may_allocate("a table of tile owners on the device");
     hipError_t e = hipMalloc((void **)&b.tile_pid, d.tile_pid.size() * sizeof(int));
     if (e == hipSuccess) e = hipMemcpy(b.tile_pid, d.tile_pid.data(), d.tile_pid.size() * sizeof(int), hipMemcpyHostToDevice);

@@ -2719,8 +2719,10 @@ bool tile_program_is_matrix(const std::string &source, int *programs, int *axis,
 // Triton kernel's block.  Those kernels use a tiling of their own, so the functor finds the program that owns the element
 // (its ids through a table the launcher fills) and the element's indices inside that program's block, and evaluates the
 // stored value for that one element: whatever can be written out per element goes (loads of a bias row or a residual
-// block included); anything that needs other elements of the accumulator throws Unsupported.
-std::string gemm_epilogue_source(const Program &p, const std::vector<const SOp *> &ops, int acc, int out, int64_t BM, int64_t BN) {
+// block included); anything that needs other elements of the accumulator throws Unsupported.  Not `owned`: a functor of the
+// accumulator and scalar arguments alone, which looks nothing up; one that depends on the element's position or reads memory
+// throws Unsupported.
+std::string gemm_epilogue_source(const Program &p, const std::vector<const SOp *> &ops, int acc, int out, int64_t BM, int64_t BN, bool owned) {
   if ((int)p.arg_names.size() > TILE_MAX_ARGS) throw Unsupported("more than " + std::to_string(TILE_MAX_ARGS) + " kernel arguments");
   Gen g(p);
   for (const SOp *s : ops) {
@@ -2754,6 +2756,22 @@ std::string gemm_epilogue_source(const Program &p, const std::vector<const SOp *
   const std::string n = std::to_string(TILE_MAX_ARGS);
   for (size_t pos = 0; (pos = pre.find("%N%", pos)) != std::string::npos;) pre.replace(pos, 3, n);
   std::ostringstream all;
+  if (!owned) {
+    const std::string text = g.index_locals.str() + expr;
+    for (size_t i = 0; i < text.size();) {
+      size_t j = i;
+      while (j < text.size() && (isalnum((unsigned char)text[j]) || text[j] == '_')) j++;
+      const std::string word = text.substr(i, j - i);
+      for (const char *w : {"i0", "i1", "pidx", "pidy", "pidz", "npx", "npy", "npz", "ptr"})
+        if (word == w) throw Unsupported("an epilogue that depends on the element's position or on memory");
+      i = j + (j == i);
+    }
+    all << pre << "struct TtsEp {\n  Args p;\n  const int *tile_pid;\n  int tiles_n, gx, gy, gz;\n"
+        << "  static constexpr int BM = 0, BN = 0;\n"
+        << "  __device__ __forceinline__ float operator()(float acc, long long, long long) const {\n"
+        << g.index_locals.str() << "    return " << expr << ";\n  }\n};\n";
+    return all.str();
+  }
   // `at`: the stored value of element (i0, i1) of the block of program q (its linear id); the call operator looks the owner
   // of (row, col) up.  A kernel that knows which of its elements share an owner (BM, BN say how far one owner reaches)
   // looks it up once for all of them and calls `at`, so that what depends on the program alone is computed once.
