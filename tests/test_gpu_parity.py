@@ -1041,6 +1041,25 @@ def test_matrix_program_attention_scores_at_the_end_of_fp32(score):
     assert (o.cpu().double() - want).abs().max().item() <= 2.0 ** -10 * want.abs().max().item()  # every probability is exact: one rounding
 
 
+@pytest.mark.parametrize("scale", [0.0, -0.1, 0.1, 6.0, 2.0 ** -70, 2.0 ** 70])
+def test_matrix_program_attention_scaled_before_its_maximum(scale):
+    # scores held without their scale, and every way out of that: scales that are not positive or out of range, rows whose
+    # maximum is too large for the exponential in one fma (scale 6), a row of equal scores
+    import extra_kernels as X
+    torch.manual_seed(11)
+    H, seq, D = 2, 200, 64
+    q, k, v = (torch.randint(-2, 3, (H, seq, D), device=DEV).half() for _ in range(3))
+    q[1, 70] = 0.0
+    o = torch.zeros_like(v)
+    kern = X.attention_fwd[(triton.cdiv(seq, 64), H)](q, k, v, o, scale, seq, seq * D, D, BM=64, BN=64, D=D)
+    torch.cuda.synchronize()
+    assert kern.function.last_kernel == "tile_program (hipRTC, matrix layout)"
+    s = torch.matmul(q.cpu().double(), k.cpu().double().transpose(1, 2)) * float(torch.tensor(scale))   # (whole numbers times the scale)
+    want = torch.matmul(torch.softmax(s, -1), v.cpu().double())
+    # probabilities and results are each rounded once to 16 bits; scores of up to 2^9 in fp32 are off by 2^-15 at scale 6
+    assert (o.cpu().double() - want).abs().max().item() <= (2.0 ** -10 + 2.0 ** -13) * v.abs().max().item()
+
+
 @pytest.mark.parametrize("form", [0, 1, 2])
 @pytest.mark.parametrize("BM,BN,D,seq", [(32, 32, 64, 150), (64, 64, 64, 200), (64, 32, 128, 65), (128, 64, 64, 300)])
 def test_matrix_program_attention_on_a_grid_with_no_free_axis(form, BM, BN, D, seq):

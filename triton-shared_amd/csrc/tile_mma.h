@@ -18,10 +18,11 @@
 //     Blocks that stick out of their tensor or are not 16-byte aligned are staged through registers instead.
 // What the ordinary form of the family spends its time on -- operands, products and every reduced row going through LDS
 // element by element between some twenty barriers per iteration -- does not exist here: causal attention of 32 heads x
-// 4096 x 128 in bf16 (64 x 64 blocks) 12.4 ms -> 174 us, 790 TFLOP/s; 32 x 4096 x 64 in fp16, no mask, 2.7 ms -> 217 us.
-// What bounds it: exponentials and the other elementwise work of the softmax, some nine vector instructions per score
-// (the exponential counts four), against 8 matrix-pipe cycles per score of a wavefront at D = 128; two workgroups per CU
-// (256 registers a lane) run their phases against each other, so that one's products hide the other's exponentials.
+// 4096 x 128 in bf16 (64 x 64 blocks) 12.4 ms -> 165 us, 830 TFLOP/s; 32 x 4096 x 64 in fp16, no mask, 2.7 ms -> 200 us.
+// What bounds it is the chain of an iteration, of which a SIMD holds two at most: the copies' way to LDS (a quarter of it while every
+// wavefront sent its copies at once: with the next blocks' copies among the first product's instructions, fragments read four
+// instructions ahead, the loop's tests in 32 bits and the row sums among the second product's instructions, 8 heads x 4096 x 128
+// causal, a workgroup per CU, 120.7 -> 88.9 us, 3763 -> 3100 cycles an iteration), then the softmax between the two products.
 //
 // Programs of a grid axis on which no staged block depends (the query blocks of one head) share a workgroup, and with it
 // the staged blocks: four wavefronts, each program taking BM / (32 R) of them.
@@ -33,6 +34,7 @@ struct MmaGen : Gen {
   bool fast_exp = false;
   std::map<int, int> roles;             // value id -> roles it is needed in
   std::map<int, std::string> tile_of, row_of, col_of;  // materialised values
+  std::map<int, std::string> factor_of;  // tiles held without a factor (a positive scalar) that their value has: see emit_scaled
   struct Image {
     int load = -1;
     int outer = 0, inner = 0;           // dimensions of the load: rows of the LDS image, and the dimension contiguous in memory
@@ -337,7 +339,8 @@ struct MmaGen : Gen {
     if (V.shape.empty()) return at(v, "0", "0");
     if (role == TILE && tile_of.count(v)) {
       if (is16(V.dtype)) return std::string(V.dtype == "f16" ? "up_f16" : "up_bf16") + "((unsigned short)(" + tile_of[v] + "[rb][nb][i >> 1] >> (16 * (i & 1))))";
-      return tile_of[v] + "[rb][nb][i]";
+      const std::string x = tile_of[v] + "[rb][nb][i]";
+      return factor_of.count(v) ? "(" + x + " * " + factor_of[v] + ")" : x;
     }
     if (role == ROW && row_of.count(v)) return row_of[v] + "[rb]";
     if (role == COL && col_of.count(v)) return col_of[v] + "[nb][i]";
@@ -416,14 +419,80 @@ struct MmaGen : Gen {
     int scalar = -1;
     return difference_against_maximum(s, &scalar) && scalar < 0 ? hardware_exp(s, a.at(0)) : map_expr(s, a);
   }
-  // The same with the difference written where it is read.  It is taken before the factor log2 e: with fma(x, log2e, -m log2e) a
-  // row of the type's lowest values (all keys masked with a finite number) is infinity minus infinity, and m log2e rounds by up
-  // to |m| 2^-24 of the exponent.
+  // Scores that a positive scalar scales before such an exponential are held as the product left them (factor_of), and so are
+  // they behind a select that puts -infinity in the place of some: the factor meets log2 e in the exponential's fma, and a maximum
+  // over them is scaled once it is taken (rounding keeps the order, so it is the same maximum).  A scalar outside of [2^-60,
+  // 2^60] -- nothing that scales scores -- is multiplied in at once, and the factor is one.
+  bool minus_infinity(int v) const {
+    const SOp *d = def_of(v);
+    while (d && (d->kind == SK::Splat || d->kind == SK::Broadcast)) d = def_of(d->operands.at(0));
+    return d && d->kind == SK::Const && val(d->result).dtype == "f32" && d->fval == -__builtin_inf();
+  }
+  bool read_by_such_an_exponential(int v) const {
+    auto u = users.find(v);
+    if (u == users.end()) return false;
+    int scalar = -1;
+    for (const SOp *o : u->second) {
+      if (o->name == "arith.subf" && o->operands.at(0) == v && folded_into_exp(*o)) {
+        bool all = true;
+        for (const SOp *e : users.at(o->result)) all = all && difference_against_maximum(*e, &scalar) && scalar < 0;
+        if (all) return true;
+      }
+      if (o->name == "arith.select" && o->operands.at(1) == v && minus_infinity(o->operands.at(2)) && read_by_such_an_exponential(o->result)) return true;
+    }
+    return false;
+  }
+  bool emit_scaled(const SOp &s) {
+    int x = -1, by = -1;
+    if (!scaled(s.result, &x, &by) || !tile_of.count(x) || factor_of.count(x) || !read_by_such_an_exponential(s.result)) return false;
+    const std::string n = declare_tile(s.result), f = "f" + std::to_string(s.result);
+    line("const float s" + f + " = " + at(by, "0", "0") + ";");
+    line("const bool fits_" + f + " = s" + f + " >= 0x1p-60f && s" + f + " <= 0x1p60f;");
+    line("const float " + f + " = fits_" + f + " ? s" + f + " : 1.0f;");
+    tile_loop(s.result, n + "[rb][nb][i] = " + el(x, TILE) + ";");
+    line("if (!fits_" + f + ") {");
+    indent++;
+    tile_loop(s.result, n + "[rb][nb][i] *= s" + f + ";");
+    indent--;
+    line("}");
+    tile_of[s.result] = n;
+    factor_of[s.result] = f;
+    return true;
+  }
+  // The same with the difference written where it is read: exp2((x - m) log2 e) as one fma, fma(x, log2 e, -(m log2 e)), with a factor
+  // that x is held without in place of log2 e times that factor.  What m log2 e rounds by is the same for all of a row, and no more
+  // than 2^-19 of them where |m log2 e| <= 64, which a wavefront asks of all its rows (values that are narrowed to 16 bits, or divided by their
+  // sum); other rows -- of infinities and NaN, or of a type's lowest values, which the fma would turn into infinity minus infinity
+  // -- take the difference first.  Causal attention bf16, a workgroup per CU (8 heads x 4096 x 128) 100.8 -> 96.1 us, two (32 heads)
+  // 168 -> 163.
   bool emit_exp_of_difference(const SOp &s) {
     int scalar = -1;
     const SOp *d = difference_against_maximum(s, &scalar);
     if (!d) return false;
     const std::string n = declare_tile(s.result), x = "(" + el(d->operands[0], TILE) + " - " + el(d->operands[1], TILE) + ")";
+    const SOp *b = def_of(d->operands[1]);
+    if (scalar < 0 && tile_of.count(d->operands[0]) && b && b->kind == SK::Broadcast && val(b->operands[0]).shape.size() == 2 && val(b->operands[0]).shape[1] == 1) {
+      const std::string m = "m" + std::to_string(s.result), c = "c" + std::to_string(s.result), log2e = s.name == "math.exp" ? "TTS_LOG2E" : "1.0f";
+      line("float " + m + "[" + std::to_string(R) + "];");
+      line("bool near_" + m + " = true;");
+      row_loop("{");
+      line("  " + m + "[rb] = " + el(d->operands[1], TILE) + " * " + log2e + ";");
+      line("  near_" + m + " = near_" + m + " && fabsf(" + m + "[rb]) <= 64.f;");
+      line("}");
+      const std::string held = tile_of[d->operands[0]] + "[rb][nb][i]";
+      line("const float " + c + " = " + (factor_of.count(d->operands[0]) ? factor_of[d->operands[0]] + " * " : std::string()) + log2e + ";");
+      line("if (!__builtin_amdgcn_ballot_w64(!near_" + m + ")) {");
+      indent++;
+      tile_loop(s.result, n + "[rb][nb][i] = __builtin_amdgcn_exp2f(__builtin_fmaf(" + held + ", " + c + ", -" + m + "[rb]));");
+      indent--;
+      line("} else {");
+      indent++;
+      tile_loop(s.result, n + "[rb][nb][i] = " + hardware_exp(s, x) + ";");
+      indent--;
+      line("}");
+      tile_of[s.result] = n;
+      return true;
+    }
     if (scalar >= 0) {
       line("if (" + at(scalar, "0", "0") + " >= 0.f) {");
       indent++;
@@ -450,31 +519,50 @@ struct MmaGen : Gen {
     return true;
   }
 
-  // Lower and upper bound of an integer value over the rows of this wavefront and the columns of the block, as scalar
-  // expressions; conditions under which they hold (no 32-bit wrap) are added to `given`.
-  bool bounds(int v, int role, std::string *lo, std::string *hi, std::string *given) {
+  // Lower and upper bound of an integer value over the rows of this wavefront and the columns of the block, as a scalar
+  // expression and a constant beside it; conditions under which they hold (no 32-bit wrap) are added to `given`.
+  struct Bound {
+    std::string v;      // "": nothing but the constant
+    int64_t c = 0;
+    bool turns = false;  // v is one 32-bit value that changes from iteration to iteration
+    bool mixed = false;  // v is a sum that holds such a value
+    std::string text() const { return v.empty() ? std::to_string(c) + "LL" : "(" + v + " + " + std::to_string(c) + "LL)"; }
+  };
+  // a < b + slack, or something narrower.  A value that changes in the loop is compared in 32 bits with a bound that does not: one
+  // scalar instruction and nothing else inside the loop.
+  static std::string below(const Bound &a, const Bound &b, int64_t slack) {
+    if (a.turns && !b.turns && !b.mixed) return "(int)" + a.v + " < sat32(" + (b.v.empty() ? "0LL" : b.v) + " + " + std::to_string(b.c + slack - a.c) + "LL)";
+    if (b.turns && !a.turns && !a.mixed) return "(int)" + b.v + " > sat32(" + (a.v.empty() ? "0LL" : a.v) + " + " + std::to_string(a.c - slack - b.c) + "LL)";
+    return a.text() + " < " + b.text() + " + " + std::to_string(slack) + "LL";
+  }
+  bool bounds(int v, int role, Bound *lo, Bound *hi, std::string *given) {
     const Value &V = val(v);
     if (V.dtype != "i32" && V.dtype != "i64") return false;
-    if (V.shape.empty()) {
-      *lo = *hi = "(long long)" + at(v, "0", "0");
+    auto scalar = [&](int x) {
+      *lo = Bound();
+      lo->v = "(long long)" + at(x, "0", "0");
+      const bool varies = lo->v.find("iv") != std::string::npos || lo->v.find("it") != std::string::npos;
+      lo->turns = varies && V.dtype == "i32";
+      lo->mixed = varies && !lo->turns;
+      *hi = *lo;
       return true;
-    }
+    };
+    if (V.shape.empty()) return scalar(v);
     const SOp *d = def_of(v);
     if (!d) return false;
     switch (d->kind) {
-      case SK::Const: case SK::FromIndex: *lo = *hi = "(long long)" + at(v, "0", "0"); return true;
+      case SK::Const: case SK::FromIndex: return scalar(v);
       case SK::Splat: return bounds(d->operands[0], role, lo, hi, given);
-      case SK::Iota: {
-        const std::string b = std::to_string(d->ival);
+      case SK::Iota:
+        *lo = *hi = Bound();
+        lo->c = hi->c = d->ival;
         if (role == ROW && V.shape[0] > 1) {
-          *lo = "(" + b + "LL + wrow)";
-          *hi = "(" + b + "LL + wrow + " + std::to_string(32 * R - 1) + ")";
+          lo->v = hi->v = "wrow";
+          hi->c += 32 * R - 1;
         } else {
-          *lo = b + "LL";
-          *hi = std::to_string(d->ival + V.shape[0] - 1) + "LL";
+          hi->c += V.shape[0] - 1;
         }
         return true;
-      }
       case SK::ExpandDims: return bounds(d->operands[0], d->axis == 1 ? ROW : COL, lo, hi, given);
       case SK::Broadcast: {
         const Value &O = val(d->operands[0]);
@@ -483,11 +571,25 @@ struct MmaGen : Gen {
       }
       case SK::Map: {
         if (d->name != "arith.addi" && d->name != "arith.subi") return false;
-        std::string a0, a1, b0, b1;
+        Bound a0, a1, b0, b1;
         if (!bounds(d->operands[0], role, &a0, &a1, given) || !bounds(d->operands[1], role, &b0, &b1, given)) return false;
-        if (d->name == "arith.addi") { *lo = "(" + a0 + " + " + b0 + ")"; *hi = "(" + a1 + " + " + b1 + ")"; }
-        else { *lo = "(" + a0 + " - " + b1 + ")"; *hi = "(" + a1 + " - " + b0 + ")"; }
-        if (V.dtype == "i32") *given += " && " + *lo + " >= -2147483648LL && " + *hi + " <= 2147483647LL";
+        const bool minus = d->name == "arith.subi";
+        auto sum = [&](const Bound &a, const Bound &b) {
+          Bound r;
+          r.c = minus ? a.c - b.c : a.c + b.c;
+          r.v = b.v.empty() ? a.v : a.v.empty() ? (minus ? "-" + b.v : b.v) : "(" + a.v + (minus ? " - " : " + ") + b.v + ")";
+          r.turns = (a.turns && b.v.empty()) || (b.turns && a.v.empty() && !minus);
+          r.mixed = !r.turns && (a.turns || a.mixed || b.turns || b.mixed);
+          return r;
+        };
+        *lo = sum(a0, minus ? b1 : b0);
+        *hi = sum(a1, minus ? b0 : b1);
+        if (V.dtype == "i32") {
+          Bound least, most;
+          least.c = INT32_MIN;
+          most.c = INT32_MAX;
+          *given += " && " + below(least, *lo, 1) + " && " + below(*hi, most, 1);
+        }
         return true;
       }
       default: return false;
@@ -520,15 +622,15 @@ struct MmaGen : Gen {
         }
         if (d->name.rfind("arith.cmpi.", 0) != 0) return false;
         const std::string p = d->name.substr(11);
-        std::string a0, a1, b0, b1, given;
+        Bound a0, a1, b0, b1;
+        std::string given;
         if (!bounds(d->operands[0], role, &a0, &a1, &given) || !bounds(d->operands[1], role, &b0, &b1, &given)) return false;
-        std::string c;
-        if (p == "slt") c = a1 + " < " + b0;
-        else if (p == "sle") c = a1 + " <= " + b0;
-        else if (p == "sgt") c = a0 + " > " + b1;
-        else if (p == "sge") c = a0 + " >= " + b1;
+        if (p == "slt") *text = below(a1, b0, 0);
+        else if (p == "sle") *text = below(a1, b0, 1);
+        else if (p == "sgt") *text = below(b1, a0, 0);
+        else if (p == "sge") *text = below(b1, a0, 1);
         else return false;
-        *text = "(" + c + given + ")";
+        *text = "(" + *text + given + ")";
         return true;
       }
       default: return false;
@@ -590,7 +692,9 @@ struct MmaGen : Gen {
       // a select that keeps the computed value wherever a mask holds: most blocks lie inside the mask as a whole
       if (s.name == "arith.select" && tile_of.count(s.operands[1]) && all_true(s.operands[0], TILE, &text)) {
         const std::string n = declare_tile(v);
-        tile_loop(v, n + "[rb][nb][i] = " + el(s.operands[1], TILE) + ";");
+        const bool held = factor_of.count(s.operands[1]) && minus_infinity(s.operands[2]);
+        tile_loop(v, n + "[rb][nb][i] = " + (held ? tile_of[s.operands[1]] + "[rb][nb][i]" : el(s.operands[1], TILE)) + ";");
+        if (held) factor_of[v] = factor_of[s.operands[1]];
         line("if (!" + text + ") {");
         indent++;
         tile_loop(v, "if (!" + el(s.operands[0], TILE) + ") " + n + "[rb][nb][i] = " + el(s.operands[2], TILE) + ";");
@@ -619,7 +723,7 @@ struct MmaGen : Gen {
           tile_of[v] = n;
           return;
         }
-      if (emit_exp_of_difference(s)) return;
+      if (emit_exp_of_difference(s) || emit_scaled(s)) return;
       std::vector<std::string> a;
       for (int o : s.operands) a.push_back(el(o, TILE));
       text = map_text(s, a);
@@ -650,8 +754,9 @@ struct MmaGen : Gen {
     const int nb = (int)(val(x).shape[1] / 32);
     // four chains, folded together at the end
     line("float f[4];");
+    const bool held = factor_of.count(x) && (s.name == "arith.maxnumf" || s.name == "arith.maximumf");
     auto elem = [&](int b, int i) {
-      std::string e = el(x, TILE), out;
+      std::string e = held ? tile_of[x] + "[rb][nb][i]" : el(x, TILE), out;
       for (size_t q = 0; q < e.size(); q++) {
         auto word = [&](const char *w) {
           const size_t l = strlen(w);
@@ -671,7 +776,7 @@ struct MmaGen : Gen {
     line("const float g0 = " + combine("f[0]", "f[1]") + ", g1 = " + combine("f[2]", "f[3]") + ", g = " + combine("g0", "g1") + ";");
     line("unsigned lo = __float_as_uint(g), hi = lo;");
     line("swap_halves(lo, hi);");
-    line(n + "[rb] = " + combine("__uint_as_float(lo)", "__uint_as_float(hi)") + ";");
+    line(n + "[rb] = " + combine("__uint_as_float(lo)", "__uint_as_float(hi)") + (held ? " * " + factor_of[x] : "") + ";");
     indent--;
     line("}");
     row_of[s.result] = n;
@@ -760,38 +865,75 @@ struct MmaGen : Gen {
     }
   }
   std::map<int, std::string> frag_of;
+  bool copies_due = false;  // the next product of the loop takes the copies of the next iteration's blocks
 
+  // a scalar condition that is true only if every row (column) of dimension d is inside the access: for the usual extent
+  // max(start, min(start + size, n)) - start with start the loop's own variable, start < n - size + 1 in 32 bits
+  std::string whole(const Access &a, size_t d) {
+    if (full(a, d)) return "true";
+    const std::string size = std::to_string(a.sizes[d]);
+    const Expr &e = P.pool.at(a.dims[d]);
+    if (e.k == EK::Sub && P.pool.at(e.a).k == EK::MaxS) {
+      const int start = e.b;
+      const Expr &mx = P.pool.at(e.a);
+      const int inner = mx.a == start ? mx.b : mx.b == start ? mx.a : -1;
+      const Expr &st = P.pool.at(P.pool.at(start).k == EK::Sext ? P.pool.at(start).a : start);
+      if (inner >= 0 && P.pool.at(inner).k == EK::MinS && st.k == EK::IV && P.pool.at(loop_by_id(st.a)->lb).bits == 32)
+        for (int q = 0; q < 2; q++) {
+          const Expr &mn = P.pool.at(inner);
+          const int end = q ? mn.b : mn.a, n = q ? mn.a : mn.b;
+          const Expr &en = P.pool.at(end);
+          int64_t c = 0;
+          if (en.k != EK::Add || !((en.a == start && P.pool.is_const(en.b, &c)) || (en.b == start && P.pool.is_const(en.a, &c))) || c < a.sizes[d]) continue;
+          if (mentions(P.pool, n, EK::IV) || mentions(P.pool, n, EK::Iter)) continue;
+          return "((int)" + ex(start) + " < sat32(" + ex(n) + " - " + std::to_string(a.sizes[d] - 1) + "LL))";
+        }
+    }
+    return "(" + extent(a, d) + " >= " + size + ")";
+  }
+  // What a copy of a right operand's block into its LDS image needs, as locals: the block's address, its pitch, and whether it
+  // can go by direct-to-LDS loads as a whole (the same answer in every wavefront of the workgroup).
+  std::string stage_base(const Image &im) {
+    const Access &a = def_of(im.load)->acc;
+    return "(const unsigned short *)p.ptr[" + std::to_string(a.base_arg) + "] + (" + ex(a.offsets[0]) + " + " + ex(a.offsets[1]) + ")";
+  }
+  std::string stage_direct(const Image &im, const std::string &base, const std::string &pitch) {
+    const Access &a = def_of(im.load)->acc;
+    return whole(a, im.outer) + " && " + whole(a, im.inner) + " && (((unsigned long long)" + base + ") & 15) == 0 && (" + pitch + " & 7) == 0 && " + pitch + " >= 0 && " + pitch + " < " +
+           std::to_string((int64_t)(1u << 30) / im.rows);
+  }
+  int stage_turns(const Image &im) const { return (int)((im.bytes() / 1024 + WAVES - 1) / WAVES); }  // direct-to-LDS loads per wavefront (1 KB each)
+  std::string stage_copy(const Image &im, int turn, const std::string &base, const std::string &pitch, const std::string &at_bytes) {
+    const int NI = (int)(im.bytes() / 1024), RPI = 1024 / im.row_bytes;  // instructions of 1 KB, image rows per instruction
+    const std::string ins = "(wave + " + std::to_string(WAVES * turn) + ")", row = "(" + ins + " * " + std::to_string(RPI) + " + lane / " + std::to_string(im.chunks) + ")";
+    const std::string guard = WAVES * turn + WAVES > NI ? "if " + ins.substr(0, ins.size() - 1) + " < " + std::to_string(NI) + ") " : "";
+    return guard + "copy_to_lds(" + base + ", (unsigned)(" + row + " * (int)" + pitch + " + 8 * ((lane & " + std::to_string(im.chunks - 1) + ") ^ (" + swizzle(im, row) + "))) * 2u, lds0 + " + at_bytes +
+           " + " + ins + " * 1024);";
+  }
   // copies a right operand's block into its LDS image at byte offset `at` of the LDS array
   void emit_stage(const Image &im, const std::string &at_bytes) {
-    const Access &a = def_of(im.load)->acc;
-    const int NI = (int)(im.bytes() / 1024), RPI = 1024 / im.row_bytes;  // instructions of 1 KB, image rows per instruction
     line("{");
     indent++;
-    line("const unsigned short *base = (const unsigned short *)p.ptr[" + std::to_string(a.base_arg) + "] + (" + ex(a.offsets[0]) + " + " + ex(a.offsets[1]) + ");");
-    line("const long long pitch = " + ex(a.strides[im.outer]) + ";");
-    line("const int rows = " + extent(a, im.outer) + ", cols = " + extent(a, im.inner) + ";");
-    const std::string swz = swizzle(im, "row");
-    line("if (rows >= " + std::to_string(im.rows) + " && cols >= " + std::to_string(im.cols) + " && (((unsigned long long)base) & 15) == 0 && (pitch & 7) == 0 && pitch >= 0 && pitch < " +
-         std::to_string((int64_t)(1u << 30) / im.rows) + ") {");
-    indent++;
-    line("#pragma unroll");
-    line("for (int j = 0; j < " + std::to_string((NI + WAVES - 1) / WAVES) + "; j++) {");
-    line("  const int ins = wave + " + std::to_string(WAVES) + " * j;");
-    if (NI % WAVES) line("  if (ins >= " + std::to_string(NI) + ") break;");
-    line("  const int row0 = lane / " + std::to_string(im.chunks) + ", row = ins * " + std::to_string(RPI) + " + row0;");
-    line("  const unsigned off = (unsigned)(row * (int)pitch + 8 * ((lane & " + std::to_string(im.chunks - 1) + ") ^ (" + swz + "))) * 2u;");
-    line("  copy_to_lds(base, off, lds0 + " + at_bytes + " + ins * 1024);");
+    line("const unsigned short *base = " + stage_base(im) + ";");
+    line("const long long pitch = " + ex(def_of(im.load)->acc.strides[im.outer]) + ";");
+    emit_stage(im, at_bytes, "base", "pitch", stage_direct(im, "base", "pitch"));
+    indent--;
     line("}");
+  }
+  void emit_stage(const Image &im, const std::string &at_bytes, const std::string &base, const std::string &pitch, const std::string &direct) {
+    const Access &a = def_of(im.load)->acc;
+    line("if (" + direct + ") {");
+    indent++;
+    for (int j = 0; j < stage_turns(im); j++) line(stage_copy(im, j, base, pitch, at_bytes));
     indent--;
     line("} else {");
     indent++;
-    line("const bool vec = (((unsigned long long)base) & 15) == 0 && (pitch & 7) == 0;");
+    line("const int rows = " + extent(a, im.outer) + ", cols = " + extent(a, im.inner) + ";");
+    line("const bool vec = (((unsigned long long)" + base + ") & 15) == 0 && (" + pitch + " & 7) == 0;");
     line("for (int c = threadIdx.x; c < " + std::to_string(im.rows * im.chunks) + "; c += " + std::to_string(64 * WAVES) + ") {");
     line("  const int row = c / " + std::to_string(im.chunks) + ", chunk = c & " + std::to_string(im.chunks - 1) + ";");
-    line("  const u32x4_t w = frag8(base + row * pitch + 8 * chunk, row < rows ? cols - 8 * chunk : 0, vec);");
-    line("  *(u32x4_t *)(lds + " + at_bytes + " + row * " + std::to_string(im.row_bytes) + " + ((chunk ^ (" + swz + ")) << 4)) = w;");
-    line("}");
-    indent--;
+    line("  const u32x4_t w = frag8(" + base + " + row * " + pitch + " + 8 * chunk, row < rows ? cols - 8 * chunk : 0, vec);");
+    line("  *(u32x4_t *)(lds + " + at_bytes + " + row * " + std::to_string(im.row_bytes) + " + ((chunk ^ (" + swizzle(im, "row") + ")) << 4)) = w;");
     line("}");
     indent--;
     line("}");
@@ -820,41 +962,83 @@ struct MmaGen : Gen {
     line("{");
     indent++;
     line("const char *im = lds + " + at_bytes + ";");
-    line("#pragma unroll");
-    line("for (int ks = 0; ks < " + std::to_string(kss) + "; ks++)");
-    line("#pragma unroll");
-    line("for (int nb = 0; nb < " + std::to_string(nbs) + "; nb++) {");
-    indent++;
-    const std::string RB = std::to_string(im.row_bytes);
-    if (!im.transposing) {
-      line("const char *row = im + (32 * nb + l32) * " + RB + ";");
-      line("const int sw = " + swizzle(im, "l32") + ";");  // (32 nb does not reach the swizzle: 32 / (16 / chunks) is a multiple of chunks)
-      if (natural) {
-        line("const u32x4_t b = *(const u32x4_t *)(row + (((2 * ks + (h4 >> 2)) ^ sw) << 4));");
+    // The right operand's fragments are read DEPTH instructions ahead of the one that multiplies them (a read takes as long as
+    // four), and the copies of the next iteration's blocks are spread among the instructions of the iteration's first product:
+    // sent together, four wavefronts' copies of 32 KB hold the CU's memory pipe, and their senders, for some 640 cycles.
+    const int frags = kss * nbs, depth = std::min(4, frags);
+    std::vector<std::string> copies;
+    if (copies_due) {
+      for (auto &q : images)
+        if (q.second.loop == cur_loop)
+          for (int j = 0; j < stage_turns(q.second); j++)
+            copies.push_back(stage_copy(q.second, j, id("sb", q.first), id("sp", q.first), std::to_string(q.second.offset) + " + (buf ^ 1) * " + std::to_string(q.second.bytes())));
+      copies_due = false;
+    }
+    const std::string RB = std::to_string(im.row_bytes), F = std::to_string(frags), D = std::to_string(depth), NBS = std::to_string(nbs);
+    auto steps = [&](const std::vector<std::string> &between) {
+      line("u32x4_t q[" + F + "];");
+      line("#pragma unroll");
+      line("for (int t = 0; t < " + F + " + " + D + "; t++) {");
+      indent++;
+      line("if (t < " + F + ") {");
+      indent++;
+      line("const int ks = t / " + NBS + ", nb = t % " + NBS + ";");
+      if (!im.transposing) {
+        line("const char *row = im + (32 * nb + l32) * " + RB + ";");
+        line("const int sw = " + swizzle(im, "l32") + ";");  // (32 nb does not reach the swizzle: 32 / (16 / chunks) is a multiple of chunks)
+        if (natural) {
+          line("q[t] = *(const u32x4_t *)(row + (((2 * ks + (h4 >> 2)) ^ sw) << 4));");
+        } else {
+          line("const u32x2_t b0 = *(const u32x2_t *)(row + (((2 * ks) ^ sw) << 4) + 2 * h4), b1 = *(const u32x2_t *)(row + (((2 * ks + 1) ^ sw) << 4) + 2 * h4);");
+          line("q[t] = (u32x4_t){b0.x, b0.y, b1.x, b1.y};");
+        }
       } else {
-        line("const u32x2_t b0 = *(const u32x2_t *)(row + (((2 * ks) ^ sw) << 4) + 2 * h4), b1 = *(const u32x2_t *)(row + (((2 * ks + 1) ^ sw) << 4) + 2 * h4);");
-        line("const u32x4_t b = {b0.x, b0.y, b1.x, b1.y};");
+        const std::string r0 = natural ? "16 * ks + 2 * h4 + (r16 >> 2)" : "16 * ks + h4 + (r16 >> 2)";
+        const int second = natural ? 4 : 8;
+        line("const int sw = " + swizzle(im, "r16 >> 2") + ";");
+        line("const char *row = im + (" + r0 + ") * " + RB + " + 8 * (r16 & 1) + (((4 * nb + 2 * ((lane >> 4) & 1) + ((r16 & 3) >> 1)) ^ sw) << 4);");
+        line("const u32x2_t b0 = read_tr(row), b1 = read_tr(row + " + std::to_string(second * im.row_bytes) + ");");
+        line("q[t] = (u32x4_t){b0.x, b0.y, b1.x, b1.y};");
       }
-    } else {
-      const std::string r0 = natural ? "16 * ks + 2 * h4 + (r16 >> 2)" : "16 * ks + h4 + (r16 >> 2)";
-      const int second = natural ? 4 : 8;
-      line("const int sw = " + swizzle(im, "r16 >> 2") + ";");
-      line("const char *row = im + (" + r0 + ") * " + RB + " + 8 * (r16 & 1) + (((4 * nb + 2 * ((lane >> 4) & 1) + ((r16 & 3) >> 1)) ^ sw) << 4);");
-      line("const u32x2_t b0 = read_tr(row), b1 = read_tr(row + " + std::to_string(second * im.row_bytes) + ");");
-      line("const u32x4_t b = {b0.x, b0.y, b1.x, b1.y};");
+      indent--;
+      line("}");
+      line("if (t >= " + D + ") {");
+      indent++;
+      line("const int ks = (t - " + D + ") / " + NBS + ", nb = (t - " + D + ") % " + NBS + ";");
+      line("#pragma unroll");
+      line("for (int rb = 0; rb < " + std::to_string(R) + "; rb++) {");
+      if (natural) line("  const u32x4_t a = " + frag_of[s.operands[0]] + "[rb][ks];");
+      else {
+        const std::string t = tile_of.at(s.operands[0]);
+        line("  const u32x4_t a = {" + t + "[rb][ks >> 1][4 * (ks & 1)], " + t + "[rb][ks >> 1][4 * (ks & 1) + 1], " + t + "[rb][ks >> 1][4 * (ks & 1) + 2], " + t +
+             "[rb][ks >> 1][4 * (ks & 1) + 3]};");
+      }
+      line("  " + n + "[rb][nb] = mfma<" + (bf ? "true" : "false") + ">(q[t - " + D + "], a, " + n + "[rb][nb]);");
+      line("}");
+      indent--;
+      line("}");
+      for (size_t c = 0; c < between.size(); c++) line("if (t == " + std::to_string(depth + (int)(c * frags / between.size())) + ") " + (between[c].rfind("if", 0) == 0 ? "{ " + between[c] + " }" : between[c]));
+      indent--;
+      line("}");
+      if (between.empty()) {  // (the compiler would read each fragment where it is used)
+        const int reads = !im.transposing && natural ? 1 : 2;
+        line("__builtin_amdgcn_sched_group_barrier(0x100, " + std::to_string(depth * reads) + ", 0);");
+        for (int t = depth; t < frags; t++) line("__builtin_amdgcn_sched_group_barrier(0x008, " + std::to_string(R) + ", 0); __builtin_amdgcn_sched_group_barrier(0x100, " + std::to_string(reads) + ", 0);");
+      }
+    };
+    if (!copies.empty()) {
+      line("if (ahead) {");
+      indent++;
+      steps(copies);
+      indent--;
+      line("} else {");
+      indent++;
     }
-    line("#pragma unroll");
-    line("for (int rb = 0; rb < " + std::to_string(R) + "; rb++) {");
-    if (natural) line("  const u32x4_t a = " + frag_of[s.operands[0]] + "[rb][ks];");
-    else {
-      const std::string t = tile_of.at(s.operands[0]);
-      line("  const u32x4_t a = {" + t + "[rb][ks >> 1][4 * (ks & 1)], " + t + "[rb][ks >> 1][4 * (ks & 1) + 1], " + t + "[rb][ks >> 1][4 * (ks & 1) + 2], " + t +
-           "[rb][ks >> 1][4 * (ks & 1) + 3]};");
+    steps({});
+    if (!copies.empty()) {
+      indent--;
+      line("}");
     }
-    line("  " + n + "[rb][nb] = mfma<" + (bf ? "true" : "false") + ">(b, a, " + n + "[rb][nb]);");
-    line("}");
-    indent--;
-    line("}");
     indent--;
     line("}");
     tile_of[v] = n;
@@ -939,6 +1123,21 @@ struct MmaGen : Gen {
     }
   }
 
+  // The ops of a loop body with those that no product needs behind the last product: a softmax's row sums are then added up
+  // between the second product's matrix instructions.  (Stores read nothing that is stored to: analyse().)
+  std::vector<SOp> products_first(const std::vector<SOp> &ops) const {
+    std::set<int> wanted;
+    for (const SOp &o : ops)
+      if (o.kind == SK::Dot) wanted.insert(o.result);
+    for (size_t i = ops.size(); i-- > 0;)
+      if (ops[i].result >= 0 && wanted.count(ops[i].result)) wanted.insert(ops[i].operands.begin(), ops[i].operands.end());
+    std::vector<SOp> order;
+    for (bool w : {true, false})
+      for (const SOp &o : ops)
+        if ((o.result >= 0 && wanted.count(o.result)) == w) order.push_back(o);
+    return order;
+  }
+
   void emit_for(const SOp &s) {
     const std::string L = std::to_string(s.loop);
     const bool i32 = P.pool.at(s.lb).bits == 32;
@@ -995,36 +1194,61 @@ struct MmaGen : Gen {
       indent--;
       line("}");
     }
-    line("for (int buf = 0; " + iv + " < last" + L + "; buf ^= 1) {");
+    line("for (int buf = 0; " + (i32 ? "(int)" + iv + " < (int)last" : iv + " < last") + L + "; buf ^= 1) {");
     indent++;
     line("const long long next_iv" + L + " = " + std::string(i32 ? "(long long)(int)" : "") + "(" + iv + " + " + ex(s.step) + ");");
     for (size_t q = 0; q < s.int_iters.size(); q++)
       line("const long long next" + L + "_" + std::to_string(q) + " = " + ex(s.int_iters[q].next) + ";");
+    const std::string I = i32 ? "(int)" : "";  // (32-bit compares are one scalar instruction, 64-bit ones go through the vector unit)
     if (staged) {
       line("landed();");
-      line("if (next_iv" + L + " < last" + L + ") {");
+      // The next iteration's blocks: a wavefront that has a product to do in this one sends their copies between its instructions
+      // (emit_dot), any other, and every one whose blocks do not go by direct-to-LDS loads as a whole, sends them here.
+      line("bool ahead = false;");
+      for (auto &im : images)
+        if (im.second.loop == s.loop) line("const unsigned short *" + id("sb", im.first) + " = nullptr; long long " + id("sp", im.first) + " = 0;");
+      line("if (" + I + "next_iv" + L + " < " + I + "last" + L + ") {");
       indent++;
       // the names the index expressions use, at the next iteration's values
+      line("const bool turn = " + I + iv + " < " + I + "ub" + L + ";");
       line("const long long at_iv = next_iv" + L + ";");
       for (size_t q = 0; q < s.int_iters.size(); q++) line("const long long at_it" + std::to_string(q) + " = next" + L + "_" + std::to_string(q) + ";");
       line("{");
       indent++;
       line("const long long " + iv + " = at_iv; (void)" + iv + ";");
       for (size_t q = 0; q < s.int_iters.size(); q++) line("const long long it" + L + "_" + std::to_string(q) + " = at_it" + std::to_string(q) + "; (void)it" + L + "_" + std::to_string(q) + ";");
-      stage_all("buf ^ 1");
+      std::string all = "turn";
+      for (auto &im : images) {
+        if (im.second.loop != s.loop) continue;
+        const std::string sb = id("sb", im.first), sp = id("sp", im.first), sd = id("sd", im.first);
+        line(sb + " = " + stage_base(im.second) + ";");
+        line(sp + " = " + ex(def_of(im.first)->acc.strides[im.second.outer]) + ";");
+        line("const bool " + sd + " = " + stage_direct(im.second, sb, sp) + ";");
+        all += " && " + sd;
+      }
+      line("ahead = " + all + ";");
+      line("if (!ahead) {");
+      indent++;
+      for (auto &im : images)
+        if (im.second.loop == s.loop)
+          emit_stage(im.second, std::to_string(im.second.offset) + " + (buf ^ 1) * " + std::to_string(im.second.bytes()), id("sb", im.first), id("sp", im.first), id("sd", im.first));
       indent--;
       line("}");
       indent--;
       line("}");
+      indent--;
+      line("}");
+      copies_due = true;
     }
-    line("if (" + iv + " < ub" + L + ") {");
+    line("if (" + I + iv + " < " + I + "ub" + L + ") {");
     indent++;
     auto saved_t = tile_of;
     auto saved_r = row_of;
     auto saved_c = col_of;
     cur_loop = s.loop;
-    emit_ops(s.body);
+    emit_ops(products_first(s.body));
     cur_loop = -1;
+    copies_due = false;
     // every new value before the first assignment (a yield may name another carried value)
     for (size_t q = 0; q < s.tile_args.size(); q++) {
       const int a = s.tile_args[q], y = s.tile_yields[q];
@@ -1092,6 +1316,7 @@ typedef float f32x2_t __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
 #define TTS_LDS(q) ((__attribute__((address_space(3))) void *)(q))
+__device__ __forceinline__ int sat32(long long x) { return (int)smin(smax(x, -2147483648LL), 2147483647LL); }
 template <bool BF16>
 __device__ __forceinline__ f32x16_t mfma(u32x4_t a, u32x4_t b, f32x16_t c) {
   if (BF16) return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
