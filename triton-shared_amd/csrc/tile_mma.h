@@ -483,13 +483,14 @@ struct MmaGen : Gen {
       line("const float " + c + " = " + (factor_of.count(d->operands[0]) ? factor_of[d->operands[0]] + " * " : std::string()) + log2e + ";");
       line("if (!__builtin_amdgcn_ballot_w64(!near_" + m + ")) {");
       indent++;
-      tile_loop(s.result, n + "[rb][nb][i] = __builtin_amdgcn_exp2f(__builtin_fmaf(" + held + ", " + c + ", -" + m + "[rb]));");
+      tile_loop(s.result, n + "[rb][nb][i] = __builtin_fmaf(" + held + ", " + c + ", -" + m + "[rb]);");
       indent--;
       line("} else {");
       indent++;
-      tile_loop(s.result, n + "[rb][nb][i] = " + hardware_exp(s, x) + ";");
+      tile_loop(s.result, n + "[rb][nb][i] = " + x + " * " + log2e + ";");
       indent--;
       line("}");
+      tile_loop(s.result, n + "[rb][nb][i] = __builtin_amdgcn_exp2f(" + n + "[rb][nb][i]);");
       tile_of[s.result] = n;
       return true;
     }
@@ -1168,8 +1169,10 @@ struct MmaGen : Gen {
     bool staged = false;
     for (auto &im : images) staged = staged || im.second.loop == s.loop;
     const std::string iv = "iv" + L;
-    line("long long " + iv + " = " + ex(s.lb) + ";");
-    line("const long long ub" + L + " = mine ? " + ex(s.ub) + " : " + iv + ";");
+    // (32-bit loops count in 32 bits: a compare is one scalar instruction then, where a 64-bit one goes through the vector unit)
+    const std::string T = i32 ? "int " : "long long ", cast = i32 ? "(int)" : "";
+    line(T + iv + " = " + cast + ex(s.lb) + ";");
+    line("const " + T + "ub" + L + " = mine ? " + cast + ex(s.ub) + " : " + iv + ";");
     if (G > 1) {
       const std::string px = std::string("pid") + "xyz"[axis], np = std::string("np") + "xyz"[axis];
       line("long long last" + L + " = " + iv + ";  // the furthest of this workgroup's programs");
@@ -1182,24 +1185,24 @@ struct MmaGen : Gen {
       // (every wavefront stages this program's blocks and meets its barriers, also one that has no rows of it)
       line("const long long last" + L + " = " + ex(s.ub) + ";");
     }
+    line("const " + T + "end" + L + " = " + cast + "last" + L + ";");
     auto stage_all = [&](const std::string &buf) {
       for (auto &im : images)
         if (im.second.loop == s.loop) emit_stage(im.second, std::to_string(im.second.offset) + " + (" + buf + ") * " + std::to_string(im.second.bytes()));
     };
     if (staged) {
       line("__syncthreads();");
-      line("if (" + iv + " < last" + L + ") {");
+      line("if (" + iv + " < end" + L + ") {");
       indent++;
       stage_all("0");
       indent--;
       line("}");
     }
-    line("for (int buf = 0; " + (i32 ? "(int)" + iv + " < (int)last" : iv + " < last") + L + "; buf ^= 1) {");
+    line("for (int buf = 0; " + iv + " < end" + L + "; buf ^= 1) {");
     indent++;
-    line("const long long next_iv" + L + " = " + std::string(i32 ? "(long long)(int)" : "") + "(" + iv + " + " + ex(s.step) + ");");
+    line("const " + T + "next_iv" + L + " = " + cast + "(" + iv + " + " + ex(s.step) + ");");
     for (size_t q = 0; q < s.int_iters.size(); q++)
       line("const long long next" + L + "_" + std::to_string(q) + " = " + ex(s.int_iters[q].next) + ";");
-    const std::string I = i32 ? "(int)" : "";  // (32-bit compares are one scalar instruction, 64-bit ones go through the vector unit)
     if (staged) {
       line("landed();");
       // The next iteration's blocks: a wavefront that has a product to do in this one sends their copies between its instructions
@@ -1207,15 +1210,15 @@ struct MmaGen : Gen {
       line("bool ahead = false;");
       for (auto &im : images)
         if (im.second.loop == s.loop) line("const unsigned short *" + id("sb", im.first) + " = nullptr; long long " + id("sp", im.first) + " = 0;");
-      line("if (" + I + "next_iv" + L + " < " + I + "last" + L + ") {");
+      line("if (next_iv" + L + " < end" + L + ") {");
       indent++;
       // the names the index expressions use, at the next iteration's values
-      line("const bool turn = " + I + iv + " < " + I + "ub" + L + ";");
-      line("const long long at_iv = next_iv" + L + ";");
+      line("const bool turn = " + iv + " < ub" + L + ";");
+      line("const " + T + "at_iv = next_iv" + L + ";");
       for (size_t q = 0; q < s.int_iters.size(); q++) line("const long long at_it" + std::to_string(q) + " = next" + L + "_" + std::to_string(q) + ";");
       line("{");
       indent++;
-      line("const long long " + iv + " = at_iv; (void)" + iv + ";");
+      line("const " + T + iv + " = at_iv; (void)" + iv + ";");
       for (size_t q = 0; q < s.int_iters.size(); q++) line("const long long it" + L + "_" + std::to_string(q) + " = at_it" + std::to_string(q) + "; (void)it" + L + "_" + std::to_string(q) + ";");
       std::string all = "turn";
       for (auto &im : images) {
@@ -1240,7 +1243,7 @@ struct MmaGen : Gen {
       line("}");
       copies_due = true;
     }
-    line("if (" + I + iv + " < " + I + "ub" + L + ") {");
+    line("if (" + iv + " < ub" + L + ") {");
     indent++;
     auto saved_t = tile_of;
     auto saved_r = row_of;
