@@ -1025,6 +1025,62 @@ def test_matrix_program_attention(dtype, D, BM, BN, seq, pad, causal, k_columns)
     assert (lse[H] == 5.0).all() and (o[H] == 3.0).all() and (o[:, :, D:] == 3.0).all()
 
 
+@pytest.mark.parametrize("dtype,D,BM,BN,H,seq,causal,masked", [
+    (torch.float16, 64, 64, 32, 2, 1000, True, None), (torch.bfloat16, 128, 64, 64, 1, 2100, False, None), (torch.float16, 64, 128, 32, 2, 700, True, None),
+    (torch.float16, 32, 32, 32, 3, 1500, False, (400, 900)), (torch.float16, 64, 128, 64, 1, 1025, False, (0, 64)), (torch.bfloat16, 64, 128, 64, 1, 3000, True, (64, 128))])
+def test_matrix_program_attention_in_slices(dtype, D, BM, BN, H, seq, causal, masked):
+    # few programs with long loops: their iterations are dealt to several workgroups.  Rows masked as a whole at the start of a slice
+    # (BM > BN under a causal mask, and runs of masked keys) add nothing; in the loop's first block they are not a number, as in
+    # the program.  Every launch gives the same bits, on two streams side by side too, and one recorded into a graph runs whole.
+    import extra_kernels as X
+    torch.manual_seed(seq)
+    q, k, v = (torch.randn(H, seq, D, device=DEV).to(dtype) for _ in range(3))
+    b = torch.randn(seq, device=DEV)
+    if masked:
+        b[masked[0]:masked[1]] = -float("inf")
+    outs = lambda: (torch.full((H + 1, seq, D), 3.0, device=DEV, dtype=dtype), torch.full((H + 1, seq), 5.0, device=DEV))
+    launch = lambda o, lse: X.attention_biased[(triton.cdiv(seq, BM), H)](q, k, v, b, o, lse, D ** -0.5, seq, seq, seq * D, D, seq * D, 1, D, BM=BM, BN=BN, D=D, CAUSAL=causal)
+    o, lse = outs()
+    kern = launch(o, lse)
+    torch.cuda.synchronize()
+    assert kern.function.last_kernel == "tile_program (hipRTC, matrix layout)"
+
+    def check(o, lse):
+        s = torch.matmul(q.cpu().double(), k.cpu().double().transpose(1, 2)) * D ** -0.5 + b.cpu().double()
+        if causal:
+            s.masked_fill_(torch.triu(torch.ones(seq, seq, dtype=torch.bool), 1), -float("inf"))
+        want, sums = torch.matmul(torch.softmax(s, -1), v.cpu().double()), torch.logsumexp(s, -1)
+        lost = torch.isinf(s[:, :, :BN]).all(-1)   # rows without a key in the first block
+        assert torch.isnan(o[:H].cpu()[lost]).all() and torch.isnan(lse[:H].cpu()[lost]).all()
+        # as in test_matrix_program_attention: probabilities and results rounded once to 16 bits; fp32 sums
+        ulp = 2.0 ** -10 if dtype == torch.float16 else 2.0 ** -7
+        assert not (~lost).any() or (o[:H].cpu().double() - want)[~lost].abs().max().item() <= ulp * v.abs().max().item()
+        assert not (~lost).any() or (lse[:H].cpu().double() - sums)[~lost].abs().max().item() <= 2e-5
+        assert (lse[H] == 5.0).all() and (o[H] == 3.0).all()
+
+    check(o, lse)
+    same = lambda a, c: torch.equal(torch.nan_to_num(a.float(), 9.0), torch.nan_to_num(c.float(), 9.0))
+    streams, kept = [torch.cuda.Stream() for _ in range(2)], []
+    torch.cuda.synchronize()
+    for turn in range(6):
+        with torch.cuda.stream(streams[turn % 2]):
+            kept.append(outs())
+            launch(*kept[-1])
+    torch.cuda.synchronize()
+    assert all(same(a, o) and same(c, lse) for a, c in kept)
+    graph = torch.cuda.CUDAGraph()
+    o2, lse2 = outs()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=streams[0]):
+        launch(o2, lse2)
+    for turn in range(2):
+        v.copy_(torch.randn(H, seq, D, device=DEV).to(dtype))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        check(o2, lse2)
+
+
 @pytest.mark.parametrize("score", [torch.finfo(torch.float32).min, 2.6e38])
 def test_matrix_program_attention_scores_at_the_end_of_fp32(score):
     # every score of a row is the same number (a finite mask on all keys, for one): the result is the mean of the values

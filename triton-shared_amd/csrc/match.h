@@ -45,10 +45,15 @@ constexpr int TILE_MAX_ARGS = 32;
 std::string tile_program_source(const Program &p);
 // The same program in the form for programs built around 16-bit matrix products (tile_mma.h); empty if it is not one.
 std::string matrix_program_source(const Program &p);
-bool tile_program_is_matrix(const std::string &source, int *programs, int *axis, int *threads);  // programs per workgroup along which axis (-1: x), threads
-// The program's loop may be dealt to several workgroups per program: the floats of partial sums each needs, the loop's id.
-bool tile_program_is_sliced(const std::string &source, int *floats, int *loop);
-bool tile_program_swaps_grid(const std::string &source);  // the launcher exchanges the grid's x and y for this source (when y fits)
+// What the launcher has to know about a generated source: its first lines say so.
+struct TileTraits {
+  bool matrix = false;  // in matrix layout: `programs` per workgroup along `axis` (-1: x), `threads` per workgroup
+  int programs = 1, axis = -1, threads = 256;
+  bool sliced = false;  // loop `loop` may be dealt to several workgroups per program (in matrix layout: per workgroup), `floats` of state each
+  int loop = -1, floats = 0;
+  bool swaps_grid = false;  // the launcher exchanges the grid's x and y (when y fits)
+};
+TileTraits tile_traits(const std::string &source);
 // Matmul family with ops between the K loop and the store: the source of the functor that applies them to one
 // accumulator value (tile_codegen.cpp), compiled at run time together with the kernels of gemm_device.h.
 std::string gemm_epilogue_source(const Program &p, const std::vector<const SOp *> &ops, int acc, int out, int64_t BM, int64_t BN, bool owned);

@@ -71,6 +71,7 @@ struct Bound {
   bool empty = false;  // nothing to do (e.g. zero trip count with nothing stored)
   bool fallback = false;  // the family's kernels do not take this launch; the generic family's kernel for the same program runs it
   int64_t slice_trips = 0;  // a generic program whose loop may run in slices: iterations of it (at most, over the grid's corners)
+  double mean_trips = 0;    // and the mean of the corners'
   std::string describe;
   // matrix products with a fused epilogue: which program owns which BM x BN tile (device memory, owned by the binding)
   int *tile_pid = nullptr;
@@ -88,6 +89,7 @@ struct Bound {
 struct tts_plan {
   Plan plan;
   std::string family;
+  TileTraits traits, fallback_traits;  // of plan.source and plan.fallback_source
   std::vector<int> arg_kinds;
   // bindings per (grid, scalar arguments), least recently used last; the oldest goes when there are more than 256
   struct CacheEntry {
@@ -559,14 +561,15 @@ std::shared_ptr<Bound> resolve(tts_plan *h, int gx, int gy, int gz, const tts_ar
     case Family::FusedMap: bind_fused_map(r, *b); break;
     case Family::TileProgram: {
       b->describe = "kernel=tile_program\n";
-      int floats = 0, loop = 0;
-      if (tile_program_is_sliced(h->plan.source, &floats, &loop))
+      if (h->traits.sliced)
         for (const SOp &s : h->plan.prog.body)
-          if (s.kind == SK::For && s.loop == loop)
+          if (s.kind == SK::For && s.loop == h->traits.loop)
             for (int corner = 0; corner < 2; corner++) {
               const EvalEnv e = corner ? r.env(gx - 1, gy - 1, gz - 1) : r.env();
               const int64_t lb = r.X.eval(s.lb, e), ub = r.X.eval(s.ub, e), step = r.X.eval(s.step, e);
-              if (ub > lb && step > 0) b->slice_trips = std::max(b->slice_trips, (ub - lb + step - 1) / step);
+              const int64_t trips = ub > lb && step > 0 ? (ub - lb + step - 1) / step : 0;
+              b->slice_trips = std::max(b->slice_trips, trips);
+              b->mean_trips += 0.5 * (double)trips;
             }
       break;
     }
@@ -680,6 +683,8 @@ tts_status tts_plan_load(const char *plan_bytes, size_t len, tts_plan **out) {
     auto h = std::make_unique<tts_plan>();
     h->plan = make_plan(read_program(text.substr(nl + 1)));
     h->family = family_name(h->plan.family);
+    if (h->plan.family == Family::TileProgram) h->traits = tile_traits(h->plan.source);
+    h->fallback_traits = tile_traits(h->plan.fallback_source);
     if (header.find("family=" + h->family) == std::string::npos) throw Invalid("plan header and plan body disagree on the kernel family");
     for (auto &t : h->plan.prog.arg_types)
       h->arg_kinds.push_back(t.ptr ? TTS_ARG_PTR : t.is_float() ? TTS_ARG_FLOAT : TTS_ARG_INT);
@@ -733,6 +738,27 @@ bool is_capturing(hipStream_t s) {
   return false;
 }
 
+// Slices of an online softmax's loop (tile_mma.h): where its workgroups leave CUs idle each walks all of its blocks alone, and where
+// they fill them about once the longest loops are what the launch waits for.  The least modelled time, in iterations of a
+// workgroup alone on its CU (half as long again beside another): the longest slice, or the work of the chip and half of that
+// where workgroups wait for a place; a meeting of n slices takes 1.5 + 0.8 n.  Measured, us in 1 / 2 / 3 / 4 / 8 slices: 2 heads x 4096 x 128 causal (64
+// workgroups) 90 / 51 / 39 / 32 / 30.5; 8 x 1405 x 64 (88) 26.9 / 19.4 / 19.7 / 18.1 / 18.5; 15 x 638 x 128 causal (75 of at most ten iterations)
+// 23.4 / 20.8 / 20.3 / 21.8 / 26.2; 8 x 4096 x 128 causal (256) 91 / 72 / 60 / 61 / 77; 23 x 225 x 128 (46 of at most four) 14.3 / 16.0 / 16.8.
+int softmax_slices(int64_t workgroups, int64_t turns, double mean, int resident) {
+  const double cus = compute_units();
+  int pick = 1;
+  double pick_t = 0;
+  for (int64_t n = 1; n <= std::min<int64_t>(16, std::max<int64_t>(turns, 1)); n++) {
+    const double per_cu = (double)(workgroups * n) / cus;
+    if (n > 1 && per_cu > 3) break;
+    double t = (double)((turns + n - 1) / n) * (1 + 0.5 * std::max(0.0, std::min(1.0, per_cu - 1)));
+    if (per_cu > resident) t = std::max(t, (double)workgroups * mean / cus * 0.75 + 0.5 * t);
+    if (n > 1) t += 1.5 + 0.8 * (double)n;
+    if (n == 1 || t < pick_t) { pick = (int)n; pick_t = t; }
+  }
+  return pick;
+}
+
 // tts_launch and tts_launch_noalloc (no_alloc: nothing below may allocate device memory or compile)
 tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, const tts_arg *args, int n, bool no_alloc) {
   if (!plan || (n > 0 && !args)) return fail(TTS_INVALID, "null argument");
@@ -760,7 +786,7 @@ tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, con
     hipError_t err = hipSuccess;
     const char *kname = "";
     // one workgroup of 256 threads per Triton program, on the kernel generated for the program (compiled at its first use)
-    auto run_tile_program = [&](RtcModule **slot, const std::string &source) -> tts_status {
+    auto run_tile_program = [&](RtcModule **slot, const std::string &source, const TileTraits &traits) -> tts_status {
       struct TileArgs { void *ptr[TILE_MAX_ARGS]; long long ival[TILE_MAX_ARGS]; double fval[TILE_MAX_ARGS]; int swap_xy, lgx, lgy, lgz; } a{};
       for (int i = 0; i < n; i++) {
         if (args[i].kind == TTS_ARG_PTR) a.ptr[i] = args[i].v.ptr;
@@ -785,20 +811,36 @@ tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, con
         const int64_t along_x = std::min(workgroups, MOST_ALONG_X);
         return rtc_launch(*slot, (int)along_x, (int)((workgroups + along_x - 1) / along_x), 1, 256, arguments, size, s);
       };
-      int per_group = 1, group_axis = -1, group_threads = 256;
-      if (tile_program_is_matrix(source, &per_group, &group_axis, &group_threads)) {  // a one-dimensional launch that numbers the programs itself
+      if (traits.matrix) {  // a one-dimensional launch that numbers the programs itself
         kname = "tile_program (hipRTC, matrix layout)";
         int64_t e[3] = {gx, gy, gz};
-        int64_t &shared = e[group_axis < 0 ? 0 : group_axis];
-        shared = (shared + per_group - 1) / per_group;
+        int64_t &shared = e[traits.axis < 0 ? 0 : traits.axis];
+        shared = (shared + traits.programs - 1) / traits.programs;
         a.lgx = gx; a.lgy = gy; a.lgz = gz;
         // (a grid holds 2^32 - 1 threads along x: larger launches continue along y, where surplus workgroups find no program)
         const int64_t workgroups = e[0] * e[1] * e[2], along_x = std::min<int64_t>(workgroups, 1 << 23);
-        err = rtc_launch(*slot, (int)along_x, (int)((workgroups + along_x - 1) / along_x), 1, group_threads, &a, sizeof a, s);
+        if (traits.sliced) {
+          struct { TileArgs t; int slices; float *partial; int *counters; } sa{};
+          sa.t = a;
+          sa.slices = softmax_slices(workgroups, b->slice_trips, b->mean_trips, rtc_resident_workgroups(*slot));
+          if (sa.slices > 1 && (no_alloc || is_capturing(s))) sa.slices = 1;  // (as for the sums below)
+          if (sa.slices > 1) {
+            std::lock_guard<std::mutex> lock(plan->mu);
+            tts_plan::SplitK &sk = plan->split_k[stream];
+            hipError_t e = plan->grow((void **)&sk.workspace, &sk.workspace_bytes, (size_t)workgroups * sa.slices * traits.floats * sizeof(float));
+            if (e == hipSuccess) e = plan->grow_counters(sk, (size_t)workgroups * 32);  // (128 bytes apart)
+            if (e != hipSuccess) return fail(TTS_HIP_ERROR, std::string("hipMalloc(slices' states): ") + hipGetErrorString(e));
+            sa.partial = sk.workspace;
+            sa.counters = sk.counters;
+          }
+          const int64_t all = workgroups * sa.slices, x = std::min<int64_t>(all, 1 << 23);
+          err = rtc_launch(*slot, (int)x, (int)((all + x - 1) / x), 1, traits.threads, &sa, sizeof sa, s);
+          return TTS_OK;
+        }
+        err = rtc_launch(*slot, (int)along_x, (int)((workgroups + along_x - 1) / along_x), 1, traits.threads, &a, sizeof a, s);
         return TTS_OK;
       }
-      int slice_floats = 0, slice_loop = 0;
-      if (tile_program_is_sliced(source, &slice_floats, &slice_loop)) {
+      if (traits.sliced) {
         // As many workgroups as the device holds at once, each program's loop dealt to an equal number of them, two
         // iterations each at least (dw and db of LayerNorm on fp16 [4096, 8192], 64 programs of 128 iterations: 341 us with
         // one workgroup per program, 27 us in 12 slices), and no more than 3 sqrt(iterations): an iteration takes some 0.75 us
@@ -813,14 +855,14 @@ tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, con
         if (sa.slices > 1) {
           std::lock_guard<std::mutex> lock(plan->mu);
           tts_plan::SplitK &sk = plan->split_k[stream];
-          hipError_t e = plan->grow((void **)&sk.workspace, &sk.workspace_bytes, (size_t)programs * sa.slices * slice_floats * sizeof(float));
+          hipError_t e = plan->grow((void **)&sk.workspace, &sk.workspace_bytes, (size_t)programs * sa.slices * traits.floats * sizeof(float));
           if (e == hipSuccess) e = plan->grow_counters(sk, (size_t)programs * 32);  // (128 bytes apart)
           if (e != hipSuccess) return fail(TTS_HIP_ERROR, std::string("hipMalloc(partial sums): ") + hipGetErrorString(e));
           sa.partial = sk.workspace;
           sa.counters = sk.counters;
         }
         // one slice: the grid as it is, a workgroup per program, its x and y exchanged where the program asks for that (see below)
-        const bool whole = sa.slices == 1, swap = whole && tile_program_swaps_grid(source) && gy > 1 && gx <= 65535;
+        const bool whole = sa.slices == 1, swap = whole && traits.swaps_grid && gy > 1 && gx <= 65535;
         if (whole && grid_fits(swap)) {
           a.swap_xy = swap ? 1 : 0;
           sa.t = a;
@@ -833,7 +875,7 @@ tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, con
         return TTS_OK;
       }
       // the program asks for neighbouring workgroups along program_id(1) (tile_codegen.cpp); grid.y holds 65535 at most
-      a.swap_xy = tile_program_swaps_grid(source) && gy > 1 && gx <= 65535 ? 1 : 0;
+      a.swap_xy = traits.swaps_grid && gy > 1 && gx <= 65535 ? 1 : 0;
       // A workgroup per program.  (A few workgroups per CU that walk the programs with the weights they share held in
       // registers lose since every row moves in 16-byte accesses, us walking / a workgroup each: LayerNorm's dx bf16 [8192, 4096]
       // 54.3 / 42.8, [8192, 2048] 32.4 / 24.4, [8192, 3001] 57.8 / 45.3; RMSNorm fp16 [8000, 5120] 38.1 / 33.1, [8000, 4096]
@@ -848,7 +890,7 @@ tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, con
       return TTS_OK;
     };
     if (b->fallback) {
-      tts_status st = run_tile_program(&plan->fallback, pl.fallback_source);
+      tts_status st = run_tile_program(&plan->fallback, pl.fallback_source, plan->fallback_traits);
       if (st != TTS_OK) return st;
       plan->last_kernel = kname;
       if (err != hipSuccess) return fail(TTS_HIP_ERROR, std::string("kernel launch failed: ") + hipGetErrorString(err));
@@ -888,7 +930,7 @@ tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, con
         break;
       }
       case Family::TileProgram: {
-        tts_status st = run_tile_program(&plan->fused, pl.source);
+        tts_status st = run_tile_program(&plan->fused, pl.source, plan->traits);
         if (st != TTS_OK) return st;
         break;
       }

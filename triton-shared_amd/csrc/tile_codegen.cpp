@@ -2556,7 +2556,7 @@ namespace {
 // the line below, and the launcher swaps the grid's x and y (x + bias[None, :] on [32, 256] tiles of an 8192 x 8192 matrix,
 // row blocks on program_id(0): 119 us; with column blocks there: 100).
 const char *const SWAP_MARK = "// tts: swap_xy\n";
-const char *const MATRIX_MARK = "// tts: matrix ";  // followed by: programs per workgroup, the axis they lie on, threads per workgroup
+const char *const MATRIX_MARK = "// tts: matrix ";  // followed by: programs per workgroup, the axis they lie on, threads per workgroup, and "slices", a loop and floats of state if that loop may run in slices
 const char *const SLICED_MARK = "// tts: sliced ";  // followed by: floats of partial sums per program and slice, the loop's id
 bool stores_walk_columns_with_pid1(const Program &p) {
   int votes_for = 0, votes_against = 0;
@@ -2599,9 +2599,18 @@ std::string without_double_barriers(std::string src) {
 }
 }  // namespace
 
-bool tile_program_swaps_grid(const std::string &source) {
-  const size_t at = source.compare(0, strlen(SLICED_MARK), SLICED_MARK) == 0 ? source.find('\n') + 1 : 0;
-  return source.compare(at, strlen(SWAP_MARK), SWAP_MARK) == 0;
+TileTraits tile_traits(const std::string &source) {
+  TileTraits t;
+  const std::string head = source.substr(0, source.find('\n'));
+  if (head.compare(0, strlen(MATRIX_MARK), MATRIX_MARK) == 0) {
+    const int got = sscanf(head.c_str() + strlen(MATRIX_MARK), "%d %d %d slices %d %d", &t.programs, &t.axis, &t.threads, &t.loop, &t.floats);
+    t.matrix = got >= 3;
+    t.sliced = got == 5;
+    return t;
+  }
+  t.sliced = head.compare(0, strlen(SLICED_MARK), SLICED_MARK) == 0 && sscanf(head.c_str() + strlen(SLICED_MARK), "%d %d", &t.floats, &t.loop) == 2;
+  t.swaps_grid = source.compare(t.sliced ? head.size() + 1 : 0, strlen(SWAP_MARK), SWAP_MARK) == 0;
+  return t;
 }
 
 std::string tile_program_source(const Program &p) {
@@ -2654,11 +2663,6 @@ std::string tile_program_source(const Program &p) {
   return without_double_barriers(all.str());
 }
 
-bool tile_program_is_sliced(const std::string &source, int *floats, int *loop) {
-  if (source.compare(0, strlen(SLICED_MARK), SLICED_MARK) != 0) return false;
-  return sscanf(source.c_str() + strlen(SLICED_MARK), "%d %d", floats, loop) == 2;
-}
-
 std::string matrix_program_source(const Program &p) {
   if ((int)p.arg_names.size() > TILE_MAX_ARGS) return std::string();
   MmaGen g(p);
@@ -2674,10 +2678,13 @@ std::string matrix_program_source(const Program &p) {
   for (size_t pos = 0; (pos = pre.find("%N%", pos)) != std::string::npos;) pre.replace(pos, 3, n);
   const std::string G = std::to_string(g.G), wpp = std::to_string(g.wpp), waves = std::to_string(g.G * g.wpp);
   std::ostringstream all;
-  all << MATRIX_MARK << g.G << " " << g.axis << " " << MmaGen::WAVES * 64 << "\n" << pre << MMA_PRELUDE;
+  all << MATRIX_MARK << g.G << " " << g.axis << " " << MmaGen::WAVES * 64;
+  if (g.meeting) all << " slices " << g.meeting->loop << " " << MmaGen::WAVES * 64 * g.state_floats();
+  all << "\n" << pre << MMA_PRELUDE;
   // two workgroups per CU (256 registers a lane) unless the blocks need more
   all << "extern \"C\" __global__ __launch_bounds__(" << MmaGen::WAVES * 64 << ", " << (mma_registers(g) <= 208 ? 2 : 1)
-      << ") void tile_program(const Args p, const int swap_xy, const int lgx, const int lgy, const int lgz) {\n"
+      << ") void tile_program(const Args p, const int swap_xy, const int lgx, const int lgy, const int lgz"
+      << (g.meeting ? ", const int slices, float *partial, int *counters" : "") << ") {\n"
       << "  __shared__ __attribute__((aligned(1024))) char lds[" << std::max<int64_t>(g.lds_bytes, 16) << "];\n"
       << "  const unsigned lds0 = (unsigned)(unsigned long long)TTS_LDS(lds);\n"
       << "  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), l32 = lane & 31, h4 = 4 * (lane >> 5), r16 = lane & 15;\n"
@@ -2689,8 +2696,8 @@ std::string matrix_program_source(const Program &p) {
   const int ax = g.axis < 0 ? 0 : g.axis, b1 = ax == 0 ? 1 : 0, b2 = ax == 2 ? 1 : 2;
   const std::string NP[3] = {"npx", "npy", "npz"}, PD[3] = {"pidx", "pidy", "pidz"};
   all << "  const unsigned others = (unsigned)(" << NP[b1] << " * " << NP[b2] << "), groups = (unsigned)((" << NP[ax] << " + " << g.G - 1 << ") / " << g.G << ");\n"
-      << "  const unsigned wg = blockIdx.x + gridDim.x * blockIdx.y;  // (along y from 2^23 workgroups on)\n"
-      << "  if (wg >= others * groups) return;\n"
+      << "  " << (g.meeting ? "" : "const ") << "unsigned wg = blockIdx.x + gridDim.x * blockIdx.y;  // (along y from 2^23 workgroups on)\n"
+      << (g.meeting ? "  const int slice = (int)(wg / (others * groups));\n  if (slice >= slices) return;\n  wg -= slice * (others * groups);\n" : "  if (wg >= others * groups) return;\n")
       << "  unsigned other, group;\n"
       << "  if (others % 8 == 0) { const unsigned j = wg / 8, per = others / 8; other = wg % 8 + 8 * (j % per); group = j / per; }\n"
       << "  else { other = wg % others; group = wg / others; }\n"
@@ -2706,11 +2713,6 @@ std::string matrix_program_source(const Program &p) {
       << "  (void)pidx; (void)pidy; (void)pidz; (void)npx; (void)npy; (void)npz; (void)swap_xy; (void)lds0; (void)r16; (void)mine; (void)groups;\n"
       << g.os.str() << "}\n";
   return all.str();
-}
-
-bool tile_program_is_matrix(const std::string &source, int *programs, int *axis, int *threads) {
-  if (source.compare(0, strlen(MATRIX_MARK), MATRIX_MARK) != 0) return false;
-  return sscanf(source.c_str() + strlen(MATRIX_MARK), "%d %d %d", programs, axis, threads) == 3;
 }
 
 // What a matmul kernel does to its accumulator between the K loop and the store (an activation, a bias, a residual, the

@@ -46,6 +46,9 @@ struct MmaGen : Gen {
     int64_t bytes() const { return rows * row_bytes; }
   };
   std::map<int, Image> images;          // load value id -> its image
+  const SOp *meeting = nullptr;         // the loop that may run in slices: see softmax_loop
+  size_t maximum_slot = 0;              // its carried row maximum
+  std::string meeting_exp;              // and the exponential that rescales what it carries: math.exp or math.exp2
   int64_t lds_bytes = 0;
   int cur_loop = -1;
 
@@ -307,6 +310,14 @@ struct MmaGen : Gen {
       if (free) axis = ax;
     }
     if (axis >= 0) G = WAVES / wpp;
+    // (the only loop, with nothing stored before it: workgroups whose slice is empty leave)
+    size_t loops = 0;
+    bool stored = false;
+    for (const SOp &s : P.body) {
+      if (s.kind == SK::For && ++loops == 1 && !stored && softmax_loop(s)) meeting = &s;
+      stored = stored || s.kind == SK::Store;
+    }
+    if (loops > 1) meeting = nullptr;
     fast_exp = true;
     std::function<void(const std::vector<SOp> &)> outs = [&](const std::vector<SOp> &ops) {
       for (const SOp &s : ops) {
@@ -328,6 +339,219 @@ struct MmaGen : Gen {
     if (s.acc.sizes.size() == 2 && is_tile(V)) need(s.operands[0], TILE);
     else if (s.acc.sizes.size() == 1 && V.shape.size() == 1 && V.shape[0] == BM) need(s.operands[0], ROW);
     else decline("a store of this shape");
+  }
+
+  // ---- slices -------------------------------------------------------------------
+  // An online softmax: a loop that carries a row maximum m' = max(m, max over x) and rows and blocks v' = v * exp(m - m') + s
+  // where s is a row sum of, or a product with, p = exp(x - m') (narrowed or not) and x knows nothing of what is carried.
+  // What such a loop has over some of its iterations is a state (m, v ...) like that of the others, and two states are one after
+  // scaling both to the larger maximum: a program's iterations may be dealt to several workgroups (slices_meet).
+  const SOp *seen_through(int v) const {  // the op behind broadcasts and added dimensions
+    const SOp *d = def_of(v);
+    while (d && (d->kind == SK::Broadcast || d->kind == SK::ExpandDims)) d = def_of(d->operands.at(0));
+    return d;
+  }
+  int behind(int v) const {
+    const SOp *d = def_of(v);
+    while (d && (d->kind == SK::Broadcast || d->kind == SK::ExpandDims)) {
+      v = d->operands.at(0);
+      d = def_of(v);
+    }
+    return v;
+  }
+  bool reaches_carried(int v, const SOp &L, int depth = 0) const {
+    if (depth > 64) return true;
+    for (int a : L.tile_args)
+      if (a == v) return true;
+    const SOp *d = def_of(v);
+    if (!d) return true;
+    for (int o : d->operands)
+      if (reaches_carried(o, L, depth + 1)) return true;
+    return false;
+  }
+  bool softmax_loop(const SOp &L) {
+    int64_t step = 0;
+    if (!L.int_iters.empty() || !P.pool.is_const(L.step, &step) || step <= 0 || mentions(P.pool, L.lb, EK::Result) || mentions(P.pool, L.ub, EK::Result)) return false;
+    for (const SOp &o : L.body)
+      if (o.kind == SK::Store || o.kind == SK::For) return false;
+    auto is_max = [](const std::string &n) { return n == "arith.maxnumf" || n == "arith.maximumf"; };
+    for (size_t q = 0; q < L.tile_args.size(); q++) {
+      const int m = L.tile_args[q], next = L.tile_yields[q];
+      const SOp *y = def_of(next);
+      if (val(m).shape.size() != 1 || val(m).dtype != "f32" || !y || y->kind != SK::Map || !is_max(y->name)) continue;
+      const int other = y->operands.at(0) == m ? y->operands.at(1) : y->operands.at(1) == m ? y->operands.at(0) : -1;
+      const SOp *r = other >= 0 ? def_of(other) : nullptr;
+      if (!r || r->kind != SK::Reduce || r->name != y->name || reaches_carried(r->operands.at(0), L)) return false;
+      std::string fn;
+      auto exponential = [&](int v) -> const SOp * {  // exp(a - m'): the subtraction
+        const SOp *e = seen_through(v);
+        if (!e || e->kind != SK::Map || (e->name != "math.exp" && e->name != "math.exp2") || (!fn.empty() && e->name != fn)) return nullptr;
+        const SOp *d = def_of(e->operands.at(0));
+        if (!d || d->kind != SK::Map || d->name != "arith.subf" || behind(d->operands.at(1)) != next) return nullptr;
+        fn = e->name;
+        return d;
+      };
+      auto rescaled = [&](int v, int arg) {  // arg * exp(m - m')
+        const SOp *d = def_of(v);
+        if (!d || d->kind != SK::Map || d->name != "arith.mulf") return false;
+        const int by = d->operands.at(0) == arg ? d->operands.at(1) : d->operands.at(1) == arg ? d->operands.at(0) : -1;
+        const SOp *sub = by >= 0 ? exponential(by) : nullptr;
+        return sub && behind(sub->operands.at(0)) == m;
+      };
+      auto probabilities = [&](int v) {  // exp(x - m'), narrowed or not
+        const SOp *d = def_of(v);
+        while (d && d->kind == SK::Map && (d->name == "arith.truncf" || d->name == "arith.extf")) d = def_of(v = d->operands.at(0));
+        const SOp *sub = d && d->kind == SK::Map ? exponential(v) : nullptr;
+        return sub && !reaches_carried(sub->operands.at(0), L);
+      };
+      auto product = [&](int v, int *into) {  // p . b + into
+        const SOp *d = def_of(v);
+        if (!d || d->kind != SK::Dot || !probabilities(d->operands.at(0)) || reaches_carried(d->operands.at(1), L)) return false;
+        *into = d->operands.at(2);
+        return true;
+      };
+      auto summand = [&](int v) {
+        const SOp *d = def_of(v);
+        int into = -1;
+        if (d && d->kind == SK::Reduce) return d->name == "arith.addf" && probabilities(d->operands.at(0));
+        const SOp *c = product(v, &into) ? def_of(into) : nullptr;
+        return c && c->kind == SK::Const && c->fval == 0;
+      };
+      auto only_read_by = [&](int v, const std::set<const SOp *> &ops) {
+        auto u = users.find(v);
+        for (const SOp *o : u == users.end() ? std::vector<const SOp *>() : u->second)
+          if (!ops.count(o)) return false;
+        return true;
+      };
+      std::set<const SOp *> of_m = {y};
+      for (size_t k = 0; k < L.tile_args.size(); k++) {
+        if (k == q) continue;
+        const int v = L.tile_args[k], w = L.tile_yields[k];
+        const SOp *d = def_of(w);
+        if (val(v).dtype != "f32" || !d) return false;
+        int into = -1, kept = -1;
+        if (d->kind == SK::Map && d->name == "arith.addf") {
+          for (int t = 0; t < 2; t++)
+            if (rescaled(d->operands.at(t), v) && summand(d->operands.at(1 - t))) kept = d->operands.at(t);
+        } else if (product(w, &into) && rescaled(into, v)) {
+          kept = into;
+        }
+        if (kept < 0 || !only_read_by(v, {def_of(kept)})) return false;
+        const SOp *mul = def_of(kept);
+        of_m.insert(def_of(seen_through(mul->operands.at(0) == v ? mul->operands.at(1) : mul->operands.at(0))->operands.at(0)));
+      }
+      // the maximum is read by itself and by its factors alone, the new one by exponentials alone
+      if (of_m.size() < 2 || !only_read_by(m, of_m)) return false;
+      std::function<bool(int)> fine = [&](int v) {
+        auto u = users.find(v);
+        for (const SOp *o : u == users.end() ? std::vector<const SOp *>() : u->second) {
+          if (o == &L) continue;  // (the yield)
+          if ((o->kind == SK::Broadcast || o->kind == SK::ExpandDims) && fine(o->result)) continue;
+          if (o->kind != SK::Map || o->name != "arith.subf" || o->operands.at(1) != v) return false;
+          for (const SOp *e : users.count(o->result) ? users.at(o->result) : std::vector<const SOp *>())
+            if (e->kind != SK::Map || e->name != fn) return false;
+        }
+        return true;
+      };
+      if (!fine(next)) return false;
+      maximum_slot = q;
+      meeting_exp = fn;
+      return true;
+    }
+    return false;
+  }
+  // floats of a lane's state: the carried rows, then the carried blocks
+  int state_floats() const {
+    int n = 0;
+    for (int a : meeting->tile_args) n += R * (val(a).shape.size() == 1 ? 1 : NB(a) * 16);
+    return (n + 3) / 4 * 4;
+  }
+  // The slices' states become one: every workgroup leaves its own in `partial` as its lanes hold it (written through, complete
+  // before its arrival is counted), and the one that arrives last scales all of them to the largest maximum, adds them up in slice
+  // order -- the result does not depend on who that is -- and goes on with the program.  Nobody waits for anybody.
+  void slices_meet() {
+    std::vector<std::string> regs;  // the maximum first
+    auto add = [&](size_t q) {
+      const int a = meeting->tile_args[q];
+      for (int rb = 0; rb < R; rb++) {
+        if (val(a).shape.size() == 1) regs.push_back(row_of.at(a) + "[" + std::to_string(rb) + "]");
+        else
+          for (int nb = 0; nb < NB(a); nb++)
+            for (int i = 0; i < 16; i++) regs.push_back(tile_of.at(a) + "[" + std::to_string(rb) + "][" + std::to_string(nb) + "][" + std::to_string(i) + "]");
+      }
+    };
+    add(maximum_slot);
+    for (size_t q = 0; q < meeting->tile_args.size(); q++)
+      if (q != maximum_slot) add(q);
+    const int n = state_floats();
+    const std::string N = std::to_string(n), Q = std::to_string(n / 4);
+    line("if (parts > 1) {");
+    indent++;
+    line("__shared__ int arrived;");
+    // this wavefront's place in slice h: 16 bytes of every lane, Q times
+    line("const long long stride = (long long)(others * groups) * " + std::to_string(WAVES * 64 * n) + ";");
+    line("float *const slot = partial + ((long long)wg * " + std::to_string(WAVES) + " + wave) * " + std::to_string(64 * n) + ";");
+    line("{");
+    indent++;
+    line("const float st[" + N + "] = {");
+    indent++;
+    for (size_t r = 0; r < regs.size(); r += 8) {
+      std::string t;
+      for (size_t k = r; k < std::min(r + 8, regs.size()); k++) t += regs[k] + ", ";
+      line(t);
+    }
+    indent--;
+    line("};");
+    line("const shared_memory_t at = shared_memory(slot + slice * stride);");
+    line("#pragma unroll");
+    line("for (int r = 0; r < " + Q + "; r++) put_through(at, r * 1024 + lane * 16, (f32x4_t){st[4 * r], st[4 * r + 1], st[4 * r + 2], st[4 * r + 3]});");
+    indent--;
+    line("}");
+    line("asm volatile(\"s_waitcnt vmcnt(0)\" ::: \"memory\");");
+    line("__syncthreads();");
+    line("if (threadIdx.x == 0) {");
+    line("  arrived = __hip_atomic_fetch_add(&counters[32 * wg], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);");
+    line("  if (arrived == parts - 1) __hip_atomic_store(&counters[32 * wg], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next launch");
+    line("}");
+    line("__syncthreads();");
+    line("if (arrived != parts - 1) return;");
+    const std::string mx = row_of.at(meeting->tile_args[maximum_slot]) + "[0]";  // (R = 1)
+    SOp op = *def_of(meeting->tile_yields[maximum_slot]);
+    // (a load takes one or two microseconds, what the slices wrote sits behind other XCDs: all the maxima are loaded together, and
+    // each slice's state while the one before it is added)
+    line("float top = 0.f;");
+    line("{");
+    line("  float tops[16];");
+    line("  #pragma unroll");
+    line("  for (int h = 0; h < 16; h++) tops[h] = take_through(shared_memory(slot + (h < parts ? h : 0) * stride), lane * 16)[0];");
+    line("  top = tops[0];");
+    line("  #pragma unroll");
+    line("  for (int h = 1; h < 16; h++) top = " + map_text_f32(op, "top", "tops[h]") + ";");
+    line("}");
+    line("float sum[" + N + "];");
+    line("#pragma unroll");
+    line("for (int r = 0; r < " + N + "; r++) sum[r] = 0.f;");
+    line("f32x4_t got[" + Q + "], next[" + Q + "];");
+    line("#pragma unroll");
+    line("for (int r = 0; r < " + Q + "; r++) got[r] = take_through(shared_memory(slot), r * 1024 + lane * 16);");
+    line("for (int h = 0; h < parts; h++) {");
+    indent++;
+    line("const shared_memory_t at = shared_memory(slot + (h + 1 < parts ? h + 1 : h) * stride);");
+    line("#pragma unroll");
+    line("for (int r = 0; r < " + Q + "; r++) next[r] = take_through(at, r * 1024 + lane * 16);");
+    const std::string d = "(got[0][0] - top)";
+    // (equal maxima are scaled by one, also where both are infinite)
+    line("const float by = got[0][0] == top ? 1.0f : " + (fast_exp ? "hardware_exp2(" + d + (meeting_exp == "math.exp" ? " * TTS_LOG2E)" : ")") : (meeting_exp == "math.exp" ? "expf(" : "exp2f(") + d + ")") + ";");
+    line("#pragma unroll");
+    line("for (int r = 0; r < " + N + "; r++) sum[r] += got[r >> 2][r & 3] * by;");
+    line("#pragma unroll");
+    line("for (int r = 0; r < " + Q + "; r++) got[r] = next[r];");
+    indent--;
+    line("}");
+    line(mx + " = top;");
+    for (size_t r = 1; r < regs.size(); r++) line(regs[r] + " = sum[" + std::to_string(r) + "];");
+    indent--;
+    line("}");
   }
 
   // ---- elements ---------------------------------------------------------------
@@ -740,8 +964,17 @@ struct MmaGen : Gen {
       line("float " + n + "[" + std::to_string(R) + "];");
       row_loop(n + "[rb] = " + text + ";");
       row_of[v] = n;
+      if (meeting && v == meeting->tile_yields[maximum_slot]) {
+        // A slice other than the first may begin with blocks in which a row is masked as a whole: its maximum is -infinity until then,
+        // and what it adds to its sums is nothing.  (In the first slice that is as it is in the program: not a number.)
+        next_maximum = n;
+        line("float from" + n + "[" + std::to_string(R) + "];");
+        row_loop("from" + n + "[rb] = " + n + "[rb] == nothing ? 0.f : " + n + "[rb];");
+        row_of[v] = "from" + n;
+      }
     }
   }
+  std::string next_maximum;
 
   void emit_reduce(const SOp &s) {
     const int x = s.operands[0];
@@ -892,49 +1125,52 @@ struct MmaGen : Gen {
     }
     return "(" + extent(a, d) + " >= " + size + ")";
   }
-  // What a copy of a right operand's block into its LDS image needs, as locals: the block's address, its pitch, and whether it
-  // can go by direct-to-LDS loads as a whole (the same answer in every wavefront of the workgroup).
-  std::string stage_base(const Image &im) {
+  // A copy of a right operand's block into its LDS image, as locals: the block's address, its pitch, and whether all of it can go by
+  // direct-to-LDS loads (the same answer in every wavefront of the workgroup).
+  void declare_stage(const Image &im) { line("const unsigned short *" + id("sb", im.load) + " = nullptr; long long " + id("sp", im.load) + " = 0; bool " + id("st", im.load) + " = false, " + id("sd", im.load) + " = false;"); }
+  void locate_stage(const Image &im) {
     const Access &a = def_of(im.load)->acc;
-    return "(const unsigned short *)p.ptr[" + std::to_string(a.base_arg) + "] + (" + ex(a.offsets[0]) + " + " + ex(a.offsets[1]) + ")";
-  }
-  std::string stage_direct(const Image &im, const std::string &base, const std::string &pitch) {
-    const Access &a = def_of(im.load)->acc;
-    return whole(a, im.outer) + " && " + whole(a, im.inner) + " && (((unsigned long long)" + base + ") & 15) == 0 && (" + pitch + " & 7) == 0 && " + pitch + " >= 0 && " + pitch + " < " +
-           std::to_string((int64_t)(1u << 30) / im.rows);
+    const std::string sb = id("sb", im.load), sp = id("sp", im.load), st = id("st", im.load);
+    line(sb + " = (const unsigned short *)p.ptr[" + std::to_string(a.base_arg) + "] + (" + ex(a.offsets[0]) + " + " + ex(a.offsets[1]) + ");");
+    line(sp + " = " + ex(a.strides[im.outer]) + ";");
+    line(st + " = " + whole(a, im.inner) + " && (((unsigned long long)" + sb + ") & 15) == 0 && (" + sp + " & 7) == 0 && " + sp + " >= 0 && " + sp + " < " + std::to_string((int64_t)(1u << 29) / im.rows) + ";  // straight");
+    line(id("sd", im.load) + " = " + st + " && " + whole(a, im.outer) + ";");
   }
   int stage_turns(const Image &im) const { return (int)((im.bytes() / 1024 + WAVES - 1) / WAVES); }  // direct-to-LDS loads per wavefront (1 KB each)
-  std::string stage_copy(const Image &im, int turn, const std::string &base, const std::string &pitch, const std::string &at_bytes) {
+  std::string stage_copy(const Image &im, int turn, const std::string &from, const std::string &at_bytes) {
     const int NI = (int)(im.bytes() / 1024), RPI = 1024 / im.row_bytes;  // instructions of 1 KB, image rows per instruction
     const std::string ins = "(wave + " + std::to_string(WAVES * turn) + ")", row = "(" + ins + " * " + std::to_string(RPI) + " + lane / " + std::to_string(im.chunks) + ")";
-    const std::string guard = WAVES * turn + WAVES > NI ? "if " + ins.substr(0, ins.size() - 1) + " < " + std::to_string(NI) + ") " : "";
-    return guard + "copy_to_lds(" + base + ", (unsigned)(" + row + " * (int)" + pitch + " + 8 * ((lane & " + std::to_string(im.chunks - 1) + ") ^ (" + swizzle(im, row) + "))) * 2u, lds0 + " + at_bytes +
-           " + " + ins + " * 1024);";
+    const std::string guard = WAVES * turn + WAVES > NI ? "if (wave < " + std::to_string(NI - WAVES * turn) + ") " : "";
+    return guard + "copy_to_lds(" + from + ", (unsigned)(" + row + " * (int)" + id("sp", im.load) + " + 8 * ((lane & " + std::to_string(im.chunks - 1) + ") ^ (" + swizzle(im, row) + "))) * 2u, lds0 + " +
+           at_bytes + " + " + ins + " * 1024);";
   }
-  // copies a right operand's block into its LDS image at byte offset `at` of the LDS array
+  // Copies the block to byte offset `at` of the LDS array.  Whole blocks and last blocks of fewer rows go by direct-to-LDS loads, the
+  // latter through a buffer resource that ends with the last row (what lies behind it is zero in LDS; rows must not overlap for
+  // that); others through registers, which cost a loop 3 us where its last block is such a one (6 heads x 401 x 128: 16.8 -> 13.9 us).
   void emit_stage(const Image &im, const std::string &at_bytes) {
-    line("{");
-    indent++;
-    line("const unsigned short *base = " + stage_base(im) + ";");
-    line("const long long pitch = " + ex(def_of(im.load)->acc.strides[im.outer]) + ";");
-    emit_stage(im, at_bytes, "base", "pitch", stage_direct(im, "base", "pitch"));
-    indent--;
-    line("}");
-  }
-  void emit_stage(const Image &im, const std::string &at_bytes, const std::string &base, const std::string &pitch, const std::string &direct) {
     const Access &a = def_of(im.load)->acc;
-    line("if (" + direct + ") {");
+    const std::string sb = id("sb", im.load), sp = id("sp", im.load);
+    line("if (" + id("sd", im.load) + ") {");
     indent++;
-    for (int j = 0; j < stage_turns(im); j++) line(stage_copy(im, j, base, pitch, at_bytes));
+    for (int j = 0; j < stage_turns(im); j++) line(stage_copy(im, j, sb, at_bytes));
     indent--;
     line("} else {");
     indent++;
     line("const int rows = " + extent(a, im.outer) + ", cols = " + extent(a, im.inner) + ";");
-    line("const bool vec = (((unsigned long long)" + base + ") & 15) == 0 && (" + pitch + " & 7) == 0;");
+    line("if (" + id("st", im.load) + " && " + sp + " >= " + std::to_string(im.cols) + ") {");
+    indent++;
+    line("const u32x4_t block = block_of(" + sb + ", rows > 0 ? (unsigned)((rows - 1) * (int)" + sp + " + " + std::to_string(im.cols) + ") * 2u : 0u);");
+    for (int j = 0; j < stage_turns(im); j++) line(stage_copy(im, j, "block", at_bytes));
+    indent--;
+    line("} else {");
+    indent++;
+    line("const bool vec = (((unsigned long long)" + sb + ") & 15) == 0 && (" + sp + " & 7) == 0;");
     line("for (int c = threadIdx.x; c < " + std::to_string(im.rows * im.chunks) + "; c += " + std::to_string(64 * WAVES) + ") {");
     line("  const int row = c / " + std::to_string(im.chunks) + ", chunk = c & " + std::to_string(im.chunks - 1) + ";");
-    line("  const u32x4_t w = frag8(" + base + " + row * " + pitch + " + 8 * chunk, row < rows ? cols - 8 * chunk : 0, vec);");
+    line("  const u32x4_t w = frag8(" + sb + " + row * " + sp + " + 8 * chunk, row < rows ? cols - 8 * chunk : 0, vec);");
     line("  *(u32x4_t *)(lds + " + at_bytes + " + row * " + std::to_string(im.row_bytes) + " + ((chunk ^ (" + swizzle(im, "row") + ")) << 4)) = w;");
+    line("}");
+    indent--;
     line("}");
     indent--;
     line("}");
@@ -972,7 +1208,7 @@ struct MmaGen : Gen {
       for (auto &q : images)
         if (q.second.loop == cur_loop)
           for (int j = 0; j < stage_turns(q.second); j++)
-            copies.push_back(stage_copy(q.second, j, id("sb", q.first), id("sp", q.first), std::to_string(q.second.offset) + " + (buf ^ 1) * " + std::to_string(q.second.bytes())));
+            copies.push_back(stage_copy(q.second, j, id("sb", q.first), std::to_string(q.second.offset) + " + (buf ^ 1) * " + std::to_string(q.second.bytes())));
       copies_due = false;
     }
     const std::string RB = std::to_string(im.row_bytes), F = std::to_string(frags), D = std::to_string(depth), NBS = std::to_string(nbs);
@@ -1107,7 +1343,13 @@ struct MmaGen : Gen {
         case SK::Load:
           if (images.count(s.result)) {
             if (images.at(s.result).loop < 0) {
+              line("{");
+              indent++;
+              declare_stage(images.at(s.result));
+              locate_stage(images.at(s.result));
               emit_stage(images.at(s.result), std::to_string(images.at(s.result).offset));
+              indent--;
+              line("}");
               line("landed();");
             }
           } else emit_load(s);
@@ -1148,16 +1390,17 @@ struct MmaGen : Gen {
       if (V.shape.empty()) decline("a carried scalar");
       const int r = roles.count(a) ? roles[a] : 0;
       const std::string n = "car" + L + "_" + std::to_string(q);
+      const std::string later = meeting == &s && q != maximum_slot ? "slice ? 0.f : " : "";  // (what the sums start from counts once)
       if (r & TILE) {
         if (V.dtype != "f32") decline("a carried block of " + V.dtype);
         line("f32x16_t " + n + "[" + std::to_string(R) + "][" + std::to_string(NB(a)) + "];");
-        tile_loop(a, n + "[rb][nb][i] = " + el(s.tile_inits[q], TILE) + ";");
+        tile_loop(a, n + "[rb][nb][i] = " + later + el(s.tile_inits[q], TILE) + ";");
         tile_of[a] = n;
       }
       if (r & ROW) {
         if (V.dtype != "f32") decline("a carried vector of " + V.dtype);
         line("float " + n + "r[" + std::to_string(R) + "];");
-        row_loop(n + "r[rb] = " + el(s.tile_inits[q], ROW) + ";");
+        row_loop(n + "r[rb] = " + later + el(s.tile_inits[q], ROW) + ";");
         row_of[a] = n + "r";
       }
     }
@@ -1185,15 +1428,36 @@ struct MmaGen : Gen {
       // (every wavefront stages this program's blocks and meets its barriers, also one that has no rows of it)
       line("const long long last" + L + " = " + ex(s.ub) + ";");
     }
-    line("const " + T + "end" + L + " = " + cast + "last" + L + ";");
-    auto stage_all = [&](const std::string &buf) {
+    if (meeting == &s) {
+      int64_t step = 0;
+      P.pool.is_const(s.step, &step);
+      const std::string S = std::to_string(step) + "LL", whole = "whole" + L;
+      // this workgroup's share of the iterations; more slices than iterations leave some workgroups without any
+      line("const long long turns = last" + L + " > " + iv + " ? (last" + L + " - " + iv + " + " + std::to_string(step - 1) + "LL) / " + S + " : 0;");
+      line("const int parts = (int)smax(1, smin(slices, turns));");
+      line("if (slice >= parts) return;");
+      line("const float nothing = slice > 0 ? -__builtin_inff() : __builtin_nanf(\"\");  // (equal to no maximum in the first slice)");
+      line("const " + T + whole + " = " + cast + "last" + L + ";");
+      line("const " + T + "end" + L + " = slice + 1 < parts ? " + cast + "(" + iv + " + turns * (slice + 1) / parts * " + S + ") : " + whole + ";");
+      line(iv + " = " + cast + "(" + iv + " + turns * slice / parts * " + S + ");");
+      line("const " + T + "own_ub" + L + " = ub" + L + " < end" + L + " ? ub" + L + " : end" + L + ";");
+    } else {
+      line("const " + T + "end" + L + " = " + cast + "last" + L + ";");
+    }
+    const std::string ub = (meeting == &s ? "own_ub" : "ub") + L;
+    auto of_loop = [&](auto &&f) {
       for (auto &im : images)
-        if (im.second.loop == s.loop) emit_stage(im.second, std::to_string(im.second.offset) + " + (" + buf + ") * " + std::to_string(im.second.bytes()));
+        if (im.second.loop == s.loop) f(im.second);
+    };
+    auto stage_all = [&](const std::string &buf) {
+      of_loop([&](const Image &im) { emit_stage(im, std::to_string(im.offset) + " + (" + buf + ") * " + std::to_string(im.bytes())); });
     };
     if (staged) {
       line("__syncthreads();");
       line("if (" + iv + " < end" + L + ") {");
       indent++;
+      of_loop([&](const Image &im) { declare_stage(im); });
+      of_loop([&](const Image &im) { locate_stage(im); });
       stage_all("0");
       indent--;
       line("}");
@@ -1208,12 +1472,11 @@ struct MmaGen : Gen {
       // The next iteration's blocks: a wavefront that has a product to do in this one sends their copies between its instructions
       // (emit_dot), any other, and every one whose blocks do not go by direct-to-LDS loads as a whole, sends them here.
       line("bool ahead = false;");
-      for (auto &im : images)
-        if (im.second.loop == s.loop) line("const unsigned short *" + id("sb", im.first) + " = nullptr; long long " + id("sp", im.first) + " = 0;");
+      of_loop([&](const Image &im) { declare_stage(im); });
       line("if (next_iv" + L + " < end" + L + ") {");
       indent++;
       // the names the index expressions use, at the next iteration's values
-      line("const bool turn = " + iv + " < ub" + L + ";");
+      line("const bool turn = " + iv + " < " + ub + ";");
       line("const " + T + "at_iv = next_iv" + L + ";");
       for (size_t q = 0; q < s.int_iters.size(); q++) line("const long long at_it" + std::to_string(q) + " = next" + L + "_" + std::to_string(q) + ";");
       line("{");
@@ -1221,20 +1484,14 @@ struct MmaGen : Gen {
       line("const " + T + iv + " = at_iv; (void)" + iv + ";");
       for (size_t q = 0; q < s.int_iters.size(); q++) line("const long long it" + L + "_" + std::to_string(q) + " = at_it" + std::to_string(q) + "; (void)it" + L + "_" + std::to_string(q) + ";");
       std::string all = "turn";
-      for (auto &im : images) {
-        if (im.second.loop != s.loop) continue;
-        const std::string sb = id("sb", im.first), sp = id("sp", im.first), sd = id("sd", im.first);
-        line(sb + " = " + stage_base(im.second) + ";");
-        line(sp + " = " + ex(def_of(im.first)->acc.strides[im.second.outer]) + ";");
-        line("const bool " + sd + " = " + stage_direct(im.second, sb, sp) + ";");
-        all += " && " + sd;
-      }
+      of_loop([&](const Image &im) {
+        locate_stage(im);
+        all += " && " + id("sd", im.load);
+      });
       line("ahead = " + all + ";");
       line("if (!ahead) {");
       indent++;
-      for (auto &im : images)
-        if (im.second.loop == s.loop)
-          emit_stage(im.second, std::to_string(im.second.offset) + " + (buf ^ 1) * " + std::to_string(im.second.bytes()), id("sb", im.first), id("sp", im.first), id("sd", im.first));
+      stage_all("buf ^ 1");
       indent--;
       line("}");
       indent--;
@@ -1243,7 +1500,7 @@ struct MmaGen : Gen {
       line("}");
       copies_due = true;
     }
-    line("if (" + iv + " < ub" + L + ") {");
+    line("if (" + iv + " < " + ub + ") {");
     indent++;
     auto saved_t = tile_of;
     auto saved_r = row_of;
@@ -1263,7 +1520,7 @@ struct MmaGen : Gen {
       }
       if (r & ROW) {
         line("float " + n + "r[" + std::to_string(R) + "];");
-        row_loop(n + "r[rb] = " + el(y, ROW) + ";");
+        row_loop(n + "r[rb] = " + (meeting == &s && q == maximum_slot ? next_maximum + "[rb]" : el(y, ROW)) + ";");
       }
     }
     for (size_t q = 0; q < s.tile_args.size(); q++) {
@@ -1290,6 +1547,7 @@ struct MmaGen : Gen {
       if (tile_of.count(a)) tile_of[res] = tile_of[a];
       if (row_of.count(a)) row_of[res] = row_of[a];
     }
+    if (meeting == &s) slices_meet();
   }
 };
 
@@ -1316,9 +1574,11 @@ typedef unsigned u32x8_t __attribute__((ext_vector_type(8)));
 typedef int i32x16_t __attribute__((ext_vector_type(16)));
 typedef short s16x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x2_t __attribute__((ext_vector_type(2)));
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
 #define TTS_LDS(q) ((__attribute__((address_space(3))) void *)(q))
+__device__ __forceinline__ float hardware_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 __device__ __forceinline__ int sat32(long long x) { return (int)smin(smax(x, -2147483648LL), 2147483647LL); }
 template <bool BF16>
 __device__ __forceinline__ f32x16_t mfma(u32x4_t a, u32x4_t b, f32x16_t c) {
@@ -1356,6 +1616,20 @@ __device__ __forceinline__ void copy_to_lds(const void *base, unsigned off, unsi
   unsigned long long own;
   asm volatile("s_mov_b32 m0, %1\n\ts_mov_b64 %0, %3\n\tglobal_load_lds_dwordx4 %2, %0" : "=&s"(own) : "s"(__builtin_amdgcn_readfirstlane((int)to)), "v"(off), "s"(s) : "memory", "m0");
 }
+// a block of `bytes` bytes as a buffer resource: loads behind its end give zeros.  (The s_nop is the distance described above.)
+__device__ __forceinline__ u32x4_t block_of(const void *base, unsigned bytes) {
+  const unsigned long long b = (unsigned long long)base;
+  return (u32x4_t){(unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)b), (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(b >> 32)), (unsigned)__builtin_amdgcn_readfirstlane((int)bytes), 0x00027000u};
+}
+__device__ __forceinline__ void copy_to_lds(u32x4_t block, unsigned off, unsigned to) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" :: "s"(__builtin_amdgcn_readfirstlane((int)to)), "v"(off), "s"(block) : "memory", "m0");
+}
+// 16 bytes per lane behind a base address that a wavefront shares, written through to and read past the caches of an XCD (sc1): what
+// workgroups on different XCDs hand over
+typedef __amdgpu_buffer_rsrc_t shared_memory_t;
+__device__ __forceinline__ shared_memory_t shared_memory(float *base) { return __builtin_amdgcn_make_buffer_rsrc(base, 0, 0x7fffffff, 0x00027000); }
+__device__ __forceinline__ void put_through(shared_memory_t at, int offset, f32x4_t v) { __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, v), at, offset, 0, 16); }
+__device__ __forceinline__ f32x4_t take_through(shared_memory_t at, int offset) { return __builtin_bit_cast(f32x4_t, __builtin_amdgcn_raw_buffer_load_b128(at, offset, 0, 16)); }
 // this wavefront's copies have arrived, and after the barrier everybody's
 __device__ __forceinline__ void landed() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); __syncthreads(); }
 )SRC";
