@@ -880,6 +880,24 @@ def test_w8a16_beyond_the_decode_shape(K, oracle_cpu, M, N, Kd, BM, kernel):
     assert torch.equal(cd[M:].cpu(), torch.full((3, N), 5.0, dtype=torch.float16))
 
 
+@pytest.mark.parametrize("M,N,Kd", [(1, 1040, 512), (16, 1024 + 128, 2048), (5, 2048, 6400), (16, 2304, 3200), (20, 1040, 3968), (32, 1168, 1024), (3, 8832, 2048)])
+def test_w8a16_wide_kernel_slabs_and_slices(K, M, N, Kd):
+    # last slabs of 16 to 240 columns, one to two groups of rows, K in one slice and in many (the columns behind N belong to nobody)
+    g = torch.Generator().manual_seed(N + Kd)
+    a = torch.randint(-2, 3, (M, Kd), generator=g).half().to(DEV)
+    w = torch.randint(-3, 4, (Kd, N), generator=g).to(torch.int8).to(DEV)
+    s = (torch.randint(1, 3, (N,), generator=g) / 4).half().to(DEV)
+    c = torch.full((M + 1, N + 32), 7.0, device=DEV, dtype=torch.float16)
+    want = a.double() @ (w.double() * s.double())   # multiples of 1/4 below 2^10 in most places: fp32 sums are exact, one rounding to fp16
+    for _ in range(3):
+        c.fill_(7.0)
+        k = K.w8a16_matmul[(triton.cdiv(M, 16), triton.cdiv(N, 128))](a, w, s, c, M, N, Kd, Kd, 1, N, 1, N + 32, 1, BM=16, BN=128, BK=128)
+        torch.cuda.synchronize()
+        assert k.function.last_kernel == "gemm_w8a16_wide_kernel"
+        assert torch.equal(c[:M, :N].double(), want.half().double())
+        assert (c[M] == 7.0).all() and (c[:, N:] == 7.0).all()
+
+
 @pytest.mark.parametrize("M,N,Kd", [(33, 2048, 64), (40, 2064, 128), (100, 2304, 1088), (161, 4112, 320), (300, 2048, 2048), (513, 3088, 192), (17, 4096, 2048), (1000, 2560, 576)])
 def test_w8a16_tiled_kernel(K, M, N, Kd):
     # rows around the heights of its tiles, ragged column tiles, one K tile up to many K slices; weights over the whole int8

@@ -377,6 +377,9 @@ __global__ __launch_bounds__(NW * 64) void gemm_w8a16_kernel(GemmW8A16Params p, 
   }
 }
 
+// Ints from one slab's arrival counter to the next: the arrivals of many slices in one line would wait for each other.
+__host__ __device__ constexpr int w8_counter_pitch(int split) { return split > 4 ? 32 : 1; }
+
 // Partial tiles cross between workgroups (and so between the XCDs' L2 caches) through agent-scope
 // relaxed atomic accesses: the stores are written through to memory and the loads bypass stale
 // lines, without the whole-cache write-back and invalidate that a release/acquire pair costs
@@ -396,7 +399,7 @@ __device__ __forceinline__ float4 load_through(float4 *src) {
 }
 
 // The decode shape's kernel: 256-column slabs, 16-byte weight loads (a lane holds 16 columns of
-// 8 rows per step), one workgroup per (slab, K slice).  Requires K % 32 == 0, N % 256 == 0,
+// 8 rows per step), one workgroup per (slab, K slice).  Requires K % 32 == 0, N % 16 == 0 (the last slab may have fewer columns),
 // 16-byte-aligned rows of W and A.
 //
 // Tail: the NW wavefronts' partial tiles are summed through LDS in one round (float4 per lane,
@@ -408,7 +411,9 @@ __device__ __forceinline__ float4 load_through(float4 *src) {
 // that share a workspace must not overlap.
 // MT: groups of 16 rows of A a launch takes (1 or 2).  The weights are widened once per step and multiplied with every
 // group's rows; the tails below (the sum over the wavefronts, the hand-over between K slices, the stores) run once per group.
-template <int NW, int DEPTH, int MT>
+// ANY: more than four slices, or a last slab of fewer columns (in a kernel of its own: whole slabs in few slices run 0.4 us of 42.4
+// longer on it at the decode shape).
+template <int NW, int DEPTH, int MT, bool ANY>
 __global__ __launch_bounds__(NW * 64) void gemm_w8a16_wide_kernel(GemmW8A16Params p, int first_steps, int other_steps) {
   extern __shared__ float4 w8_lds[];  // [NW][16][64]
   __shared__ int is_last;
@@ -416,11 +421,12 @@ __global__ __launch_bounds__(NW * 64) void gemm_w8a16_wide_kernel(GemmW8A16Param
   const int j = lane & 15, g = lane >> 4;
   const int slab = blockIdx.x, slice = blockIdx.y;
   const int64_t n0 = (int64_t)slab * W8_COLS_WIDE;
+  const int col = ANY ? min(16 * j, (int)min(p.N - 16 - n0, (int64_t)W8_COLS_WIDE)) : 16 * j;  // this lane's sixteen of the slab (behind the last: others, which are not stored)
   const uint16_t *__restrict__ S = (const uint16_t *)p.scale;
 
   uint32_t scale2[16];
   {
-    const uint4 *sp = reinterpret_cast<const uint4 *>(S + n0 + 16 * j);
+    const uint4 *sp = reinterpret_cast<const uint4 *>(S + n0 + col);
     const bool s_vec = (((uintptr_t)S) & 15) == 0;
     uint16_t sv[16];
     if (s_vec) {
@@ -430,7 +436,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_w8a16_wide_kernel(GemmW8A16Param
       for (int c = 0; c < 16; c++) sv[c] = (uint16_t)(wds[c / 2] >> (16 * (c & 1)));
     } else {
 #pragma unroll
-      for (int c = 0; c < 16; c++) sv[c] = S[n0 + 16 * j + c];
+      for (int c = 0; c < 16; c++) sv[c] = S[n0 + col + c];
     }
 #pragma unroll
     for (int c = 0; c < 16; c++) scale2[c] = (uint32_t)sv[c] | ((uint32_t)sv[c] << 16);
@@ -444,7 +450,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_w8a16_wide_kernel(GemmW8A16Param
   // slice 0 takes first_steps steps of 32 rows, every other slice other_steps
   const int step_begin = slice == 0 ? 0 : first_steps + (slice - 1) * other_steps;
   const int step_end = min(step_begin + (slice == 0 ? first_steps : other_steps), (int)(p.K / 32));
-  const int8_t *w_lane = p.w + (int64_t)(8 * g) * p.ldw + n0 + 16 * j;
+  const int8_t *w_lane = p.w + (int64_t)(8 * g) * p.ldw + n0 + col;
   const uint16_t *a_lane[MT];
 #pragma unroll
   for (int m = 0; m < MT; m++) a_lane[m] = (const uint16_t *)p.a + (int64_t)min(16 * m + j, (int)p.M - 1) * p.lda + 8 * g;
@@ -522,50 +528,41 @@ __global__ __launch_bounds__(NW * 64) void gemm_w8a16_wide_kernel(GemmW8A16Param
   if (p.split > 1) {
     // a slab's slots: [slice][group][1024 float4]
     float4 *slots = reinterpret_cast<float4 *>(p.workspace) + (int64_t)slab * p.split * MT * 1024;
-    int *counter = p.counters + slab;
+    int *counter = p.counters + w8_counter_pitch(p.split) * slab;
     // tot = the slices' tiles added in slice order, whoever adds them (so the sum does not depend on who arrived when);
-    // `self` is this workgroup's slice, whose tile is tot.  Up to four slices, every load is issued before the first add
-    // (one round trip to memory instead of one per slice).
+    // `self` is this workgroup's slice, whose tile is tot.  Four or eight slices at a time, every load is issued before the first add: one round trip to memory instead of one per slice, of which 25 slices (15 x 2048 x 6400) made
+    // most of 22.7 us (now 13.7).
     auto add_slices = [&](int self) {
-      constexpr int EAGER = 4;
-      if (p.split <= EAGER) {
+      constexpr int EAGER = ANY && MT == 1 ? 8 : 4;
+      float4 sum[MT][PER] = {};
+      for (int s0 = 0; s0 < (ANY ? p.split : 1); s0 += EAGER) {
         float4 u[EAGER][MT][PER];
 #pragma unroll
-        for (int sl = 0; sl < EAGER; sl++)
-          if (sl < p.split && sl != self) {
+        for (int d = 0; d < EAGER; d++)
+          if (s0 + d < p.split && s0 + d != self) {
 #pragma unroll
             for (int m = 0; m < MT; m++)
 #pragma unroll
-              for (int e = 0; e < PER; e++) u[sl][m][e] = load_through(slots + (sl * MT + m) * 1024 + tid + e * NW * 64);
+              for (int e = 0; e < PER; e++) u[d][m][e] = load_through(slots + ((s0 + d) * MT + m) * 1024 + tid + e * NW * 64);
           }
 #pragma unroll
-        for (int m = 0; m < MT; m++)
+        for (int d = 0; d < EAGER; d++)
+          if (s0 + d < p.split) {
 #pragma unroll
-          for (int e = 0; e < PER; e++) {
-            float4 t = self == 0 ? tot[m][e] : u[0][m][e];
+            for (int m = 0; m < MT; m++)
 #pragma unroll
-            for (int sl = 1; sl < EAGER; sl++)
-              if (sl < p.split) {
-                const float4 v = sl == self ? tot[m][e] : u[sl][m][e];
-                t.x += v.x; t.y += v.y; t.z += v.z; t.w += v.w;
+              for (int e = 0; e < PER; e++) {
+                const float4 v = s0 + d == self ? tot[m][e] : u[d][m][e];
+                float4 &t = sum[m][e];
+                if (s0 + d == 0) t = v;
+                else { t.x += v.x; t.y += v.y; t.z += v.z; t.w += v.w; }
               }
-            tot[m][e] = t;
           }
-        return;
       }
 #pragma unroll
       for (int m = 0; m < MT; m++)
 #pragma unroll
-        for (int e = 0; e < PER; e++) {
-          const int idx = tid + e * NW * 64;
-          float4 t = make_float4(0.f, 0.f, 0.f, 0.f);
-          for (int sl = 0; sl < p.split; sl++) {
-            float4 u = sl == self ? tot[m][e] : load_through(slots + (sl * MT + m) * 1024 + idx);
-            if (sl == 0) t = u;
-            else { t.x += u.x; t.y += u.y; t.z += u.z; t.w += u.w; }
-          }
-          tot[m][e] = t;
-        }
+        for (int e = 0; e < PER; e++) tot[m][e] = sum[m][e];
     };
     bool others_done = false;
     if (slice == 0) {
@@ -615,7 +612,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_w8a16_wide_kernel(GemmW8A16Param
     __syncthreads();
     for (int item = tid; item < 16 * (W8_COLS_WIDE / 8); item += NW * 64) {
       const int m = item / (W8_COLS_WIDE / 8), n8 = (item % (W8_COLS_WIDE / 8)) * 8;
-      if (16 * grp + m >= p.M) continue;
+      if (16 * grp + m >= p.M || (ANY && n0 + n8 >= p.N)) continue;
       const float *src = tile + m * PITCH + n8;
       uint16_t h[8];
 #pragma unroll
@@ -890,14 +887,24 @@ hipError_t launch_gemm_epilogue(const GemmParams &p, const std::string &epilogue
 namespace {
 struct W8Config { int cw, nw, depth, split; };
 
+// Whether the 16-byte-load kernel takes a shape: N in whole slabs of 256, and from 1024 columns on in groups of 16 (below, a last slab that
+// is half empty is a good part of all).  The 8-byte kernel in 128-column slabs stays ahead where it fills the chip without slices and
+// K is short (us, 8-byte / 16-byte loads: 6 x 26752 x 2944 16.7 / 18.5, 8 x 25472 x 3456 18.7 / 19.8, but 8 x 27520 x 4096 23.9 / 22.8, 16 x 28544 x
+// 8192 45.6 / 39.3), and for few slabs of long K, whose many slices its second kernel adds (14 x 2432 x 5888 13.2 / 13.9, 8 x 1152 x 8192
+// 13.0 / 14.1, but 16 x 2176 x 4096 12.9 / 11.8).
+bool w8_wide_shape(const GemmW8A16Params &p) {
+  if (p.K % 32 != 0 || p.lda % 8 != 0 || p.ldw % 16 != 0) return false;
+  if (p.N % W8_COLS_WIDE == 0) return true;
+  return p.N % 16 == 0 && p.N >= 1024 && !(p.N >= 192 * W8_COLS && p.K < 4096) && !(p.N < 2560 && p.K > 4096);
+}
+
 // The shape decides the kernel: 256-column slabs with 16-byte weight loads when N and the
 // weight pitch allow, split over K so that about one workgroup lands on each CU.
 // TTS_W8=cw,nw,depth,split overrides the choice (tuning aid).
 W8Config w8_config(const GemmW8A16Params &p) {
   const int64_t steps = (p.K + 31) / 32;
   W8Config c{8, 16, 2, 1};
-  const bool fast = p.K % 32 == 0 && p.N % W8_COLS == 0 && p.lda % 8 == 0 && p.ldw % 8 == 0;
-  if (fast && p.N % W8_COLS_WIDE == 0 && p.ldw % 16 == 0) c = W8Config{16, 8, 1, 1};
+  if (w8_wide_shape(p)) c = W8Config{16, 8, 1, 1};
   static const char *env = getenv("TTS_W8");
   int want_split = 0;
   if (env) {
@@ -908,11 +915,20 @@ W8Config w8_config(const GemmW8A16Params &p) {
   }
   const int64_t slabs = (p.N + 16 * c.cw - 1) / (16 * c.cw);
   if (want_split > 0) c.split = want_split;
-  else if (slabs < 192) {
-    // about one workgroup per CU; the wide kernel's LDS tile admits only one, so never more than 256 of those
-    int64_t want = c.cw == 16 ? std::max<int64_t>(1, 256 / slabs) : (256 + slabs - 1) / slabs;
-    int64_t most = std::max<int64_t>(1, steps / c.nw);        // keep every wavefront busy
-    c.split = (int)std::max<int64_t>(1, std::min<int64_t>(std::min(want, most), 64));
+  else if (c.cw == 16) {
+    // At most one workgroup per CU (its LDS tile admits no more), and the least modelled time: a workgroup's round of eight steps takes
+    // 1.35 us where the chip is idle and 12 ns per workgroup where memory is the limit, a meeting 0.35 us per slice beyond five.
+    // Measured, us in 2 / 4 / 8 / 12 / 24 slices: 15 x 2048 x 6400 25.0 / 16.8 / 13.7 / 13.4 / 16.4; 9 x 6272 x 5376 22.3 / 16.1 / 14.5 / 19.9 / 26.9;
+    // 3 x 9856 x 2432 13.9 / 12.1 / 16.5 / 18.5 / 27.9; 8 x 20096 x 7296 in 2 / 3 / 4 30.4 / 27.6 / 36.9.  (As many as fill the chip, as before: 16.8, 15.7, 12.3.)
+    double best = 0;
+    for (int64_t n = 1; n <= std::min<int64_t>(64, std::max<int64_t>(1, steps / c.nw)) && (n == 1 || slabs * n <= 256); n++) {
+      const double rounds = std::max(1.0, (double)steps / (double)(c.nw * n)), memory = 0.0117 * (double)(slabs * n);
+      const double t = rounds * std::sqrt(1.35 * 1.35 + memory * memory) + 0.35 * (double)std::max<int64_t>(0, n - 5);
+      if (n == 1 || t < best) { c.split = (int)n; best = t; }
+    }
+  } else if (slabs < 192) {  // about one workgroup per CU, every wavefront busy
+    const int64_t most = std::max<int64_t>(1, steps / c.nw);
+    c.split = (int)std::max<int64_t>(1, std::min<int64_t>(std::min((256 + slabs - 1) / slabs, most), 64));
   }
   return c;
 }
@@ -923,14 +939,14 @@ void w8_launch(const GemmW8A16Params &p, int steps_per_slice, hipStream_t s) {
   hipLaunchKernelGGL((gemm_w8a16_kernel<NW, DEPTH, FAST, 8>), grid, dim3(NW * 64), 0, s, p, steps_per_slice);
 }
 
-template <int NW, int DEPTH, int MT = 1>
+template <int NW, int DEPTH, int MT, bool ANY>
 hipError_t w8_launch_wide(const GemmW8A16Params &p, int first_steps, int other_steps, hipStream_t s) {
   constexpr size_t lds = (size_t)NW * 16 * 64 * sizeof(float4);
-  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_w8a16_wide_kernel<NW, DEPTH, MT>),
+  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_w8a16_wide_kernel<NW, DEPTH, MT, ANY>),
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (attr != hipSuccess) return attr;
-  dim3 grid((unsigned)(p.N / W8_COLS_WIDE), p.split);
-  hipLaunchKernelGGL((gemm_w8a16_wide_kernel<NW, DEPTH, MT>), grid, dim3(NW * 64), lds, s, p, first_steps, other_steps);
+  dim3 grid((unsigned)((p.N + W8_COLS_WIDE - 1) / W8_COLS_WIDE), p.split);
+  hipLaunchKernelGGL((gemm_w8a16_wide_kernel<NW, DEPTH, MT, ANY>), grid, dim3(NW * 64), lds, s, p, first_steps, other_steps);
   return hipGetLastError();
 }
 }  // namespace
@@ -943,7 +959,7 @@ size_t gemm_w8a16_workspace_bytes(const GemmW8A16Params &p) {
   return (size_t)p.split * (p.M > 16 ? 32 : 16) * (size_t)((p.N + 255) / 256 * 256) * sizeof(float);
 }
 
-size_t gemm_w8a16_counters(const GemmW8A16Params &p) { return p.split <= 1 ? 0 : (size_t)((p.N + 255) / 256); }
+size_t gemm_w8a16_counters(const GemmW8A16Params &p) { return p.split <= 1 ? 0 : w8_counter_pitch(p.split) * (size_t)((p.N + 255) / 256); }
 
 static hipError_t launch_gemm_w8a16_rows(const GemmW8A16Params &p, hipStream_t s, const char **name);
 
@@ -1032,7 +1048,9 @@ hipError_t launch_gemm_w8a16(const GemmW8A16Params &p, hipStream_t s, const char
 static bool w8_fast(const GemmW8A16Params &p) {
   return p.K % 32 == 0 && p.N % W8_COLS == 0 && p.lda % 8 == 0 && p.ldw % 8 == 0 && ((uintptr_t)p.a & 15) == 0 && ((uintptr_t)p.w & 7) == 0;
 }
-static bool w8_wide(const GemmW8A16Params &p) { return w8_fast(p) && w8_config(p).cw == 16 && ((uintptr_t)p.w & 15) == 0; }
+static bool w8_wide(const GemmW8A16Params &p) {
+  return w8_wide_shape(p) && w8_config(p).cw == 16 && ((uintptr_t)p.a & 15) == 0 && ((uintptr_t)p.w & 15) == 0;
+}
 
 static hipError_t launch_gemm_w8a16_rows(const GemmW8A16Params &p, hipStream_t s, const char **name) {
   W8Config c = w8_config(p);
@@ -1051,9 +1069,9 @@ static hipError_t launch_gemm_w8a16_rows(const GemmW8A16Params &p, hipStream_t s
       if (sps - take >= 8 && sps * p.split == steps) { first = sps + take * (p.split - 1); other = sps - take; }
     }
     // one step in flight per wavefront; two measured 1.2 us slower at the decode shape
-    if (p.M > 16) return w8_launch_wide<8, 1, 2>(p, first, other, s);
-    if (c.depth == 2) return w8_launch_wide<8, 2>(p, first, other, s);
-    return w8_launch_wide<8, 1>(p, first, other, s);
+    const bool any = p.split > 4 || p.N % W8_COLS_WIDE != 0;
+    if (p.M > 16) return any ? w8_launch_wide<8, 1, 2, true>(p, first, other, s) : w8_launch_wide<8, 1, 2, false>(p, first, other, s);
+    return any ? w8_launch_wide<8, 1, 1, true>(p, first, other, s) : w8_launch_wide<8, 1, 1, false>(p, first, other, s);
   }
   *name = "gemm_w8a16_kernel";
   if (!fast) w8_launch<W8_WAVES, 2, false>(p, sps, s);
