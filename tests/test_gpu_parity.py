@@ -569,6 +569,45 @@ def test_gemm_any_shape_kernel_at_the_ends_of_its_tiles(K, M, N, Kd, at, bt):
     assert (cd[M] == 7.0).all() and (cd[:, N] == 7.0).all()
 
 
+@pytest.mark.parametrize("M,N,Kd,at,bt,dtype", [(256, 512, 1600, False, False, torch.bfloat16), (1000, 2048, 4096, False, True, torch.float16),
+                                                 (770, 776, 1536, False, False, torch.float16), (136, 648, 2048, True, False, torch.bfloat16), (520, 512, 1600, True, True, torch.float16)])
+def test_gemm_slices_that_meet_in_the_kernel(K, M, N, Kd, at, bt, dtype):
+    """128 x 128 tiles in two to five K slices, which the workgroup of a tile that arrives last adds: whole and ragged tiles, either
+    operand column-major, again and again over one workspace whose counters every launch leaves at zero, and recorded, where a second
+    kernel adds them.  Small integers with few of them at once: exact in any order, and results of at most 8 bits."""
+    g = torch.Generator().manual_seed(M + N)
+    A = torch.zeros(M, Kd, dtype=dtype)
+    A.scatter_(1, torch.randint(0, Kd, (M, 60), generator=g), 1.0)
+    B = torch.randint(-2, 3, (Kd, N), generator=g).to(dtype)
+    want = (A.double() @ B.double()).to(dtype)
+    a = A.t().contiguous().to(DEV).t() if at else A.to(DEV)
+    b = B.t().contiguous().to(DEV).t() if bt else B.to(DEV)
+    c = torch.empty((M + 1, N + 8), dtype=dtype, device=DEV)
+    run = lambda: K.matmul_tiles[(triton.cdiv(M, 128) * triton.cdiv(N, 128),)](a, b, c, M, N, Kd, a.stride(0), a.stride(1), b.stride(0), b.stride(1), N + 8, 1, BM=128, BN=128, BK=64, GROUP_M=8)
+    def check():
+        torch.cuda.synchronize()
+        assert torch.equal(c[:M, :N].cpu(), want) and (c[M] == 7).all() and (c[:, N:] == 7).all()
+        c.fill_(7.0)
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    c.fill_(7.0)
+    for i in range(6):
+        torch.cuda.synchronize()
+        with torch.cuda.stream(streams[i % 2]):
+            k = run()
+            assert k.function.last_kernel == "gemm_dma_kernel<128x128>, K slices", k.function.last_kernel
+        check()
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=streams[0]):
+        run()
+    for _ in range(3):
+        graph.replay()
+        check()
+        with torch.cuda.stream(streams[0]):
+            run()
+        check()
+
+
 @pytest.mark.parametrize("M,N,Kd,bt,dtype", [(17, 129, 4095, True, torch.bfloat16), (100, 700, 2000, False, torch.float16), (200, 15, 1984, False, torch.bfloat16), (130, 257, 1153, True, torch.float16)])
 def test_gemm_any_shape_kernel_in_k_slices(K, M, N, Kd, bt, dtype):
     # few tiles and a long K: slices whose sums a second kernel adds, narrow and wide rows; with and without a functor that

@@ -37,6 +37,8 @@ struct TtsGemmParams {
   // leaves its fp32 sums at partial[s * M * N + m * N + n], and a second kernel adds the slices and narrows (1 = none)
   int split;
   float *partial;
+  int meet;               // 1: slices may meet in the kernel (slices_meet), which counts their arrivals in
+  int *counters;          // ... counters, 32 ints apart, zero between launches
   // A batch of products of one shape (grid.y of the launch = batches): batch b reads a + b * batch_a and b + b * batch_b
   // and writes c + b * batch_c (in elements); 1 / 0 for a single product
   int batches;
@@ -507,6 +509,55 @@ __device__ __forceinline__ void load_to_lds(const char *sbase, uint32_t voff, ui
 // s_waitcnt immediate: vmcnt in bits 3:0 and 15:14, expcnt (not waited for) in 6:4, lgkmcnt in 11:8
 constexpr int waitcnt_imm(int vm, int lgkm) { return (vm & 15) | ((vm >> 4) << 14) | (7 << 4) | (lgkm << 8); }
 
+// The K slices of a tile become one without a second kernel: every workgroup leaves its sums in p.partial as its lanes hold them
+// (written through: sc1), and the one that arrives last adds all of them in slice order into `acc` -- as the kernel that adds
+// slices does, bit for bit -- and stores the tile.  false: this workgroup is done.  Nobody waits for anybody.  Bound by what one
+// CU reads of others' sums, about 2.4 us per slice of 64 KiB with the trip through memory, where the second kernel has a launch
+// and the whole chip: 1024 x 1024 x 1792 17.6 -> 14.7 us, 256 x 512 x 1600 14.6 -> 12.0.
+template <int TM, int TN>
+__device__ __forceinline__ bool slices_meet(const GemmParams &p, f32x16 (&acc)[TM][TN], int slice, int tile, int tiles, int wave, int lane) {
+  typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
+  constexpr int Q = TM * TN * 4;  // 16-byte pieces of a lane
+  __shared__ int arrived;
+  float *const slot = p.partial + ((int64_t)tile * 4 + wave) * (Q * 256);
+  auto place = [&](int s) { return __builtin_amdgcn_make_buffer_rsrc(slot + (int64_t)s * tiles * (4 * Q * 256), 0, 0x7fffffff, 0x00027000); };
+  {
+    const auto own = place(slice);
+#pragma unroll
+    for (int q = 0; q < Q; q++) {
+      const f32x16 &a = acc[q / 4 / TN][q / 4 % TN];
+      const f32x4 v = {a[4 * (q % 4)], a[4 * (q % 4) + 1], a[4 * (q % 4) + 2], a[4 * (q % 4) + 3]};
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, v), own, q * 1024 + lane * 16, 0, 16);
+    }
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // in memory, and behind the barrier everybody's
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    arrived = __hip_atomic_fetch_add(p.counters + 32 * tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (arrived == p.split - 1) __hip_atomic_store(p.counters + 32 * tile, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next launch
+  }
+  __syncthreads();
+  if (arrived != p.split - 1) return false;
+  f32x4 got[Q], next[Q];
+  auto take = [&](f32x4 (&to)[Q], int s) {
+    const auto from = place(s);
+#pragma unroll
+    for (int q = 0; q < Q; q++) to[q] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(from, q * 1024 + lane * 16, 0, 16));
+  };
+  take(got, 0);
+  for (int s = 0; s < p.split; s++) {  // (the next slice's while one is added)
+    take(next, s + 1 < p.split ? s + 1 : s);
+#pragma unroll
+    for (int q = 0; q < Q; q++) {
+      f32x16 &a = acc[q / 4 / TN][q / 4 % TN];
+#pragma unroll
+      for (int e = 0; e < 4; e++) a[4 * (q % 4) + e] = s ? a[4 * (q % 4) + e] + got[q][e] : got[q][e];
+      got[q] = next[q];
+    }
+  }
+  return true;
+}
+
 // TM x TN = 4 x 4: the 256 x 256 tile described above.  Smaller tiles (2 x 2: 128 x 128, 2 x 4: 128 x 256, 4 x 2:
 // 256 x 128) use the same stages, swizzles and phases with fewer rows and columns: an A instruction still covers 16
 // rows of 64 bytes, a B instruction 1024 / (2 BN) k rows of 2 BN bytes (position q of k row k holds chunk
@@ -523,7 +574,7 @@ template <bool E> struct EdgeTile { static constexpr bool value = E; };
 constexpr int F_PF_AHEAD = 8;
 // SK: the grid holds p.split workgroups per tile; workgroup (tile, s) walks the s-th share of the K tiles and leaves its sums
 // in p.partial.
-template <bool BF16, int TM, int TN, class Ep, bool BT = false, bool AT = false, bool PF = false, bool SK = false>
+template <bool BF16, int TM, int TN, class Ep, bool BT = false, bool AT = false, bool PF = false, bool SK = false, bool MEET = false>
 __device__ __forceinline__ void gemm_dma_body(const GemmParams &p, int tiles_m, int tiles_n, const Ep &ep) {
   using T = DmaTile<TM, TN>;
   constexpr int BM = T::BM, BN = T::BN, STAGES = T::STAGES, A_BYTES = T::A_BYTES, STAGE_BYTES = T::STAGE_BYTES, ROWB = T::B_ROW_BYTES;
@@ -794,7 +845,10 @@ __device__ __forceinline__ void gemm_dma_body(const GemmParams &p, int tiles_m, 
   // are narrowed at once (v_cvt_pk_bf16_f32 for bf16: round to nearest even, NaNs quieted), the pair is exchanged with
   // the neighbouring lane, and the even lane stores row r at columns (n, n+1), the odd lane row r+1 at (n-1, n):
   // half as many store instructions as one 2-byte store per element, and a handful of VALU ops per pair.
-  if constexpr (SK) {
+  if constexpr (MEET) {
+    if (!slices_meet<TM, TN>(p, acc, slice, tile_m * tiles_n + tile_n, nwg, wave, lane)) return;
+  }
+  if constexpr (SK && !MEET) {
     // the slice's sums as they are: a lane's 32 x 32 block column by column, two rows of 32 consecutive floats per store
     float *__restrict__ part = p.partial + (int64_t)slice * p.M * p.N;
 #pragma unroll

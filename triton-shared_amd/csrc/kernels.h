@@ -97,6 +97,7 @@ using GemmParams = ::TtsGemmParams;  // gemm_device.h
 // p.split = at most gemm_split(p) K slices (1: none) with p.partial = gemm_workspace_bytes(p) bytes of device memory for them
 int gemm_split(const GemmParams &p);
 size_t gemm_workspace_bytes(const GemmParams &p);
+size_t gemm_meeting(const GemmParams &p, size_t *bytes);  // p.split slices meet in the kernel: that many tiles, bytes of p.partial (0: they do not)
 hipError_t launch_gemm(const GemmParams &p, hipStream_t s, const char **kernel_name);
 // The same product with elementwise ops fused into the epilogue: `epilogue` is the source of the functor (match.h:
 // gemm_epilogue_source), `modules` the plan's slots for the kernels compiled from it (one per tiling and the sum of K slices,

@@ -135,10 +135,26 @@ hipError_t launch_gemm_dma_slices(const GemmParams &p, hipStream_t s) {
   return hipGetLastError();
 }
 
+// 128 x 128 tiles in K slices that meet in the kernel (slices_meet; chosen by slices_may_meet)
+template <bool BF16, bool BT, bool AT>
+__global__ __launch_bounds__(256) void gemm_dma_meeting_kernel(GemmParams p, int tiles_m, int tiles_n) {
+  gemm_dma_body<BF16, 2, 2, IdentityEp, BT, AT, false, true, true>(p, tiles_m, tiles_n, IdentityEp());
+}
+
 template <bool BF16, int TM, int TN, bool BT, bool AT, bool PF = false>
 hipError_t launch_gemm_dma_t(const GemmParams &p, hipStream_t s) {
   using T = DmaTile<TM, TN>;
   constexpr size_t lds = T::LDS_BYTES;
+  if constexpr (!PF && TM == 2 && TN == 2) {
+    if (p.split > 1 && p.counters) {
+      auto kern = gemm_dma_meeting_kernel<BF16, BT, AT>;
+      static const hipError_t attr = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+      if (attr != hipSuccess) return attr;
+      const int tiles_m = (int)((p.M + 127) / 128), tiles_n = (int)((p.N + 127) / 128);
+      hipLaunchKernelGGL(kern, dim3(tiles_m * tiles_n * p.split), dim3(256), lds, s, p, tiles_m, tiles_n);
+      return hipGetLastError();
+    }
+  }
   if constexpr (!PF) {
     if (p.split > 1) {
       hipError_t e = launch_gemm_dma_slices<BF16, TM, TN, BT, AT>(p, s);
@@ -651,6 +667,18 @@ const DmaCand DMA_CANDS[4] = {{"256x256", 256, 256, 1.0, 0.59, 0.07, 0.04, 9}, {
                               {"256x128", 256, 128, 0.73, 0.51, 0.03, 0.04, 6.3}, {"128x128", 128, 128, 0.59, 0.34, 0, 0.03, 3.8}};
 struct DmaChoice { const DmaCand *tile = nullptr; int split = 1; };
 
+// us that the slices of a product take to become one: through a second kernel that the whole chip runs, or, on 128 x 128 tiles,
+// in the workgroup of a tile that arrives last, which reads its 64 KiB per slice alone.  Modelled on 16 ... 64 tiles in 2 ... 8 slices.
+// us per call, second kernel / in the kernel, each in the slices it chooses: 256 x 512 x 1600 14.6 / 12.0; 256 x 4096 x 2048 17.5 / 14.9;
+// 576 x 960 x 1408 15.3 / 13.2; 768 x 768 x 1536 16.5 / 14.0; 1024 x 1024 x 1792 17.6 / 14.7; 1024 x 2048 x 3072 24.0 / 22.3; 512 x 1536 x 2560
+// 15.8 / 15.9; 1408 x 704 x 2496 17.0 / 17.5, the one of 17 that lost; in 8 slices and more, where the rule keeps the second kernel,
+// 16 x 4096 x 4096 16.0 / 22.3 and 128 x 4096 x 4096 19.7 / 22.7.
+double added_us(const GemmParams &p, int split) { return 5.5 + 0.28e-6 * split * 4 * (double)p.M * (double)p.N * std::max(1, p.batches); }
+double meeting_us(int split) { return 2.4 * split - 4; }
+bool slices_may_meet(const GemmParams &p, const DmaCand &c, int split) {
+  return p.meet && &c == &DMA_CANDS[3] && split > 1 && p.batches <= 1 && meeting_us(split) < added_us(p, split);
+}
+
 DmaChoice choose_dma(const GemmParams &p, int max_split) {
   static const char *dma_env = getenv("TTS_GEMM_DMA");      // tuning aid: "256x256", "128x256", "256x128", "128x128" or unset
   static const char *split_env = getenv("TTS_GEMM_SPLIT");  // tuning aid: the number of K slices (1 = never split)
@@ -680,32 +708,41 @@ DmaChoice choose_dma(const GemmParams &p, int max_split) {
   const bool by_rounds = !grouped && p.K >= 512;
   const int64_t nk = p.K / F_BK;
   const double sums = (double)p.M * (double)p.N * std::max(1, p.batches) * 4;  // bytes of one slice's
-  auto time = [&](const DmaCand &c, int split) {
+  auto time = [&](const DmaCand &c, int split, bool meet) {
     const double f = (double)tiles(c) * split / cus;
-    return (double)((nk + split - 1) / split) * (std::ceil(f) * (c.round + (p.b_trans ? c.turned : 0)) + f * c.fill) + c.fixed + (split > 1 ? 5.5 + 0.28e-6 * split * sums : 0);
+    return (double)((nk + split - 1) / split) * (std::ceil(f) * (c.round + (p.b_trans ? c.turned : 0)) + f * c.fill) + c.fixed +
+           (split == 1 ? 0 : meet && slices_may_meet(p, c, split) ? meeting_us(split) : added_us(p, split));
   };
   DmaChoice best;
   double best_cost = 0;
   for (const DmaCand &c : DMA_CANDS) {
     if (!gemm_dma_ok(p, c.bm, c.bn)) continue;
     if (dma_env ? std::string(dma_env) != c.tag : !by_rounds && c.bm + c.bn != 256 && (grouped ? !grouped_wide(tiles(c)) : tiles(c) < cus)) continue;
-    const double cost = by_rounds ? time(c, 1) : (double)(tiles(c) * c.bm * c.bn) / c.eff;
+    const double cost = by_rounds ? time(c, 1, false) : (double)(tiles(c) * c.bm * c.bn) / c.eff;
     if (!best.tile || cost < best_cost) { best.tile = &c; best_cost = cost; }
   }
   if (!best.tile || max_split < 2 || !by_rounds || p.a_rows || p.b_block) return best;
+  // (the model's times of short walks are too long: in 128 x 128 tiles K to 1024 is ahead whole, us whole / in slices that a second
+  // kernel adds / that meet: 256 x 1024 x 1024 11.0 / 13.6 / 11.9, 64 x 4096 x 1024 11.4 / 13.5 / 11.8; 512 x 1024 x 1216 11.9 / 14.3 / 11.8)
+  if (best.tile == &DMA_CANDS[3] && p.K <= 1024 && !split_env && p.batches <= 1) return best;
   DmaChoice pick = best;
   double pick_t = best_cost;
-  if (!(split_env && atoi(split_env) == 1))
+  // (what is ahead whole of slices that a second kernel adds stays whole, however little their meeting takes: 1152 x 1536 x 1024
+  // 11.5 us against 14.9 in two slices)
+  for (const bool meet : {false, true}) {
+    if (split_env && atoi(split_env) == 1) break;
+    if (meet && (!p.meet || pick.split == 1)) break;
     for (const DmaCand &c : DMA_CANDS) {
       if (!gemm_dma_ok(p, c.bm, c.bn) || (dma_env && std::string(dma_env) != c.tag)) continue;
       const int64_t most = std::min<int64_t>(std::min<int64_t>(std::min<int64_t>(16, max_split), nk / 8), (2 * cus + tiles(c) - 1) / tiles(c));
       for (int64_t sp = split_env ? atoi(split_env) : 2; sp <= most; sp++) {
         if (sp * sums > (double)((size_t)256 << 20)) break;
-        const double t = time(c, (int)sp);
+        const double t = time(c, (int)sp, meet);
         if (t < pick_t || (split_env && pick.split == 1)) { pick.tile = &c; pick.split = (int)sp; pick_t = t; }
         if (split_env) break;
       }
     }
+  }
   return pick;
 }
 }  // namespace
@@ -748,6 +785,14 @@ int gemm_split(const GemmParams &p) {
   return choice.tile ? choice.split : any_split(p, 16);
 }
 bool gemm_any_shape(const GemmParams &p) { return !p.is_f32 && !choose_dma(p, 1).tile; }
+// p.split slices that meet in the kernel: the tiles that count arrivals, and the bytes of p.partial (0: a second kernel adds them).
+size_t gemm_meeting(const GemmParams &p, size_t *bytes) {
+  const DmaChoice choice = choose_dma(p, 16);
+  if (!choice.tile || choice.split != p.split || !slices_may_meet(p, *choice.tile, p.split)) return 0;
+  const size_t tiles = (size_t)(((p.M + 127) / 128) * ((p.N + 127) / 128));
+  *bytes = (size_t)p.split * tiles * (128 * 128 * sizeof(float));
+  return tiles;
+}
 size_t gemm_workspace_bytes(const GemmParams &p) { return p.split > 1 ? (size_t)p.split * p.M * p.N * std::max(1, p.batches) * sizeof(float) : 0; }
 
 // p.split: the most K slices p.partial has room for (what gemm_split(p) said, or fewer; 1: none).
@@ -761,7 +806,7 @@ hipError_t launch_gemm(const GemmParams &p, hipStream_t s, const char **name) {
   if (!tile_env) {
     // Whole K tiles go to the direct-to-LDS kernels.
     // at most p.split slices: what gemm_split said, or fewer when the caller's workspace holds no more (1: none)
-    const DmaChoice choice = choose_dma(p, std::max(1, p.split));
+    const DmaChoice choice = p.counters ? DmaChoice{&DMA_CANDS[3], p.split} : choose_dma(p, std::max(1, p.split));
     GemmParams q = p;
     q.split = choice.split;
     const DmaCand *best = choice.tile;

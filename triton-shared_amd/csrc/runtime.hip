@@ -963,15 +963,26 @@ tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, con
         }
         p.split = 1;
         p.partial = nullptr;
+        p.meet = 0;
+        p.counters = nullptr;
         if (pl.source.empty()) {
           // a product with too few tiles for the chip runs in K slices, whose partial sums need memory: the stream's
           // workspace (as for the int8-weight product), or the static array of the call that may not allocate, when
           // they fit there (else that call runs the product without slices)
           // (the any-shape kernel keeps to whole products where the launch may not allocate or is recorded into a graph)
+          // slices that meet in the kernel count their arrivals: not where a graph could be replayed beside other launches
+          p.meet = !no_alloc && !is_capturing(s);
           const int want = gemm_split(p);
           if (want > 1 && !(gemm_any_shape(p) && (no_alloc || is_capturing(s)))) {
             p.split = want;
-            const size_t need = gemm_workspace_bytes(p);
+            size_t need = gemm_workspace_bytes(p), meeting_bytes = 0;
+            const size_t meeting = p.meet ? gemm_meeting(p, &meeting_bytes) : 0;
+            if (meeting) {  // (a later recording finds room for the sums that a second kernel adds)
+              GemmParams recorded = p;
+              recorded.meet = 0;
+              recorded.split = gemm_split(recorded);
+              need = std::max(meeting_bytes, gemm_workspace_bytes(recorded));
+            }
             if (no_alloc) {  // as many slices as the static array holds
               const size_t one = (size_t)p.M * p.N * std::max(1, p.batches) * sizeof(float);
               p.split = (int)std::min<size_t>((size_t)want, NOALLOC_WORKSPACE_BYTES / one);
@@ -984,8 +995,10 @@ tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, con
                 p.split = 1;
               } else {
                 hipError_t e = plan->grow((void **)&sk.workspace, &sk.workspace_bytes, need);
+                if (e == hipSuccess && meeting) e = plan->grow_counters(sk, 32 * meeting);
                 if (e != hipSuccess) return fail(TTS_HIP_ERROR, std::string("hipMalloc(split-K workspace): ") + hipGetErrorString(e));
                 p.partial = sk.workspace;
+                if (meeting) p.counters = sk.counters;
               }
             }
           }
