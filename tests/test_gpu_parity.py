@@ -608,6 +608,30 @@ def test_gemm_slices_that_meet_in_the_kernel(K, M, N, Kd, at, bt, dtype):
         check()
 
 
+@pytest.mark.parametrize("M,N,Kd", [(512, 512, 1536), (256, 256, 4096), (768, 768, 1024)])
+def test_gemm_is_chosen_by_the_alignment_of_each_launch(K, M, N, Kd):
+    # one binding (the same sizes and strides) launched on operands that are aligned and not, in turn: what it was chosen to run on
+    # for the one is not kept for the other
+    g = torch.Generator().manual_seed(M + Kd)
+    A = torch.zeros(M, Kd)
+    A.scatter_(1, torch.randint(0, Kd, (M, 60), generator=g), 1.0)
+    B = torch.randint(-2, 3, (Kd, N), generator=g).float()
+    want = (A.double() @ B.double()).bfloat16()
+    def at(x, off):
+        flat = torch.zeros(x.numel() + 8, dtype=torch.bfloat16, device=DEV)
+        flat[off:off + x.numel()] = x.flatten().bfloat16().to(DEV)
+        return flat[off:off + x.numel()].view(x.shape)
+    names = set()
+    for oa, ob, oc in [(0, 0, 0), (1, 0, 0), (0, 0, 0), (0, 1, 0), (0, 0, 1), (0, 0, 0)] * 2:
+        a, b, c = at(A, oa), at(B, ob), at(torch.zeros(M, N), oc)
+        k = K.matmul_tiles[(triton.cdiv(M, 128) * triton.cdiv(N, 128),)](a, b, c, M, N, Kd, Kd, 1, N, 1, N, 1, BM=128, BN=128, BK=64, GROUP_M=8)
+        torch.cuda.synchronize()
+        assert k.function.last_kernel.startswith("gemm_mfma_kernel" if oa or ob or oc else "gemm_dma_kernel"), (oa, ob, oc, k.function.last_kernel)
+        names.add(k.function.last_kernel)
+        assert torch.equal(c.cpu(), want), (oa, ob, oc)
+    assert len(names) >= 2
+
+
 @pytest.mark.parametrize("M,N,Kd,bt,dtype", [(17, 129, 4095, True, torch.bfloat16), (100, 700, 2000, False, torch.float16), (200, 15, 1984, False, torch.bfloat16), (130, 257, 1153, True, torch.float16)])
 def test_gemm_any_shape_kernel_in_k_slices(K, M, N, Kd, bt, dtype):
     # few tiles and a long K: slices whose sums a second kernel adds, narrow and wide rows; with and without a functor that

@@ -94,11 +94,19 @@ hipError_t launch_layernorm(const LayerNormParams &p, int gx, int gy, int gz, hi
 
 // C[M,N] = A[M,K] * B[K,N], 16-bit inputs, fp32 accumulate, 16-bit output (RTNE)
 using GemmParams = ::TtsGemmParams;  // gemm_device.h
-// p.split = at most gemm_split(p) K slices (1: none) with p.partial = gemm_workspace_bytes(p) bytes of device memory for them
-int gemm_split(const GemmParams &p);
-size_t gemm_workspace_bytes(const GemmParams &p);
-size_t gemm_meeting(const GemmParams &p, size_t *bytes);  // p.split slices meet in the kernel: that many tiles, bytes of p.partial (0: they do not)
-hipError_t launch_gemm(const GemmParams &p, hipStream_t s, const char **kernel_name);
+// What a product runs on: it depends on sizes, pitches, layouts, the operands' alignment and p.meet, and takes the host up to a
+// microsecond to find, so whoever launches the same product again keeps it (host us of a call, chosen up to four times in it / kept: 256 x
+// 256 x 4096 12.6 / 10.8, 64 x 2048 x 2048 11.4 / 10.4, 512 x 512 x 1536 8.4 / 7.7).
+struct GemmChoice {
+  int tile = -1;       // which direct-to-LDS tile (-1: the any-shape kernel, or fp32)
+  int split = 1;       // K slices (1: none)
+  size_t meeting = 0;  // tiles whose slices meet in the kernel (0: a second kernel adds them)
+  size_t bytes = 0;    // of p.partial that the slices need
+};
+GemmChoice gemm_choose(const GemmParams &p);
+// p.split = at most the choice's K slices (1: none), with p.partial the bytes it says; `choice`: what gemm_choose(p) said (null: it is asked).
+hipError_t launch_gemm(const GemmParams &p, hipStream_t s, const char **kernel_name, const GemmChoice *choice = nullptr);
+size_t gemm_workspace_bytes(const GemmParams &p);  // of p.partial for p.split slices that a second kernel adds
 // The same product with elementwise ops fused into the epilogue: `epilogue` is the source of the functor (match.h:
 // gemm_epilogue_source), `modules` the plan's slots for the kernels compiled from it (one per tiling and the sum of K slices,
 // filled at the first launch that needs it and may compile), `args` / `args_size` the generic families' argument block.
@@ -115,7 +123,6 @@ struct GemmEpilogueArgs {
   int tiles_n, gx, gy, gz;
 };
 int gemm_epilogue_split(const GemmParams &p);  // K slices (1: none), as gemm_split(p) for a product with a functor
-bool gemm_any_shape(const GemmParams &p);      // the any-shape kernel runs this product
 bool gemm_epilogue_compiled(const GemmParams &p, RtcModule *const *modules);  // a whole launch of this shape finds its kernel there
 hipError_t launch_gemm_epilogue(const GemmParams &p, const std::string &epilogue, RtcModule **modules, bool may_compile, const GemmEpilogueArgs &ep,
                                 hipStream_t s, const char **kernel_name, std::string *err);

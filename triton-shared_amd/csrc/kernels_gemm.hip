@@ -778,35 +778,36 @@ int any_split(const GemmParams &p, int max_split) {
 }
 }  // namespace
 
-int gemm_split(const GemmParams &p) {
-  static const char *tile_env = getenv("TTS_GEMM_TILE");
-  if (p.is_f32 || tile_env) return 1;
-  const DmaChoice choice = choose_dma(p, 16);
-  return choice.tile ? choice.split : any_split(p, 16);
-}
-bool gemm_any_shape(const GemmParams &p) { return !p.is_f32 && !choose_dma(p, 1).tile; }
-// p.split slices that meet in the kernel: the tiles that count arrivals, and the bytes of p.partial (0: a second kernel adds them).
-size_t gemm_meeting(const GemmParams &p, size_t *bytes) {
-  const DmaChoice choice = choose_dma(p, 16);
-  if (!choice.tile || choice.split != p.split || !slices_may_meet(p, *choice.tile, p.split)) return 0;
-  const size_t tiles = (size_t)(((p.M + 127) / 128) * ((p.N + 127) / 128));
-  *bytes = (size_t)p.split * tiles * (128 * 128 * sizeof(float));
-  return tiles;
+GemmChoice gemm_choose(const GemmParams &p) {
+  static const char *tile_env = getenv("TTS_GEMM_TILE");  // tuning aid: set = the any-shape kernel even for whole tiles
+  GemmChoice c;
+  if (p.is_f32 || tile_env) return c;
+  const DmaChoice dma = choose_dma(p, 16);
+  if (dma.tile) c.tile = (int)(dma.tile - DMA_CANDS);
+  GemmParams q = p;
+  q.split = c.split = dma.tile ? dma.split : any_split(p, 16);
+  c.bytes = gemm_workspace_bytes(q);
+  if (dma.tile && slices_may_meet(p, *dma.tile, c.split)) {
+    c.meeting = (size_t)(((p.M + 127) / 128) * ((p.N + 127) / 128));
+    c.bytes = (size_t)c.split * c.meeting * (128 * 128 * sizeof(float));
+  }
+  return c;
 }
 size_t gemm_workspace_bytes(const GemmParams &p) { return p.split > 1 ? (size_t)p.split * p.M * p.N * std::max(1, p.batches) * sizeof(float) : 0; }
 
-// p.split: the most K slices p.partial has room for (what gemm_split(p) said, or fewer; 1: none).
-hipError_t launch_gemm(const GemmParams &p, hipStream_t s, const char **name) {
+// p.split: the most K slices p.partial has room for (what gemm_choose(p) said, or fewer; 1: none).
+hipError_t launch_gemm(const GemmParams &p, hipStream_t s, const char **name, const GemmChoice *chosen) {
   if (p.is_f32) {
     if (p.a_rows || p.b_block) return hipErrorInvalidValue;  // (the matcher takes gathered rows on 16-bit operands only)
     *name = "gemm_f32_kernel";
     return launch_gemm_f32(p, s);
   }
-  static const char *tile_env = getenv("TTS_GEMM_TILE");  // tuning aid: set = the any-shape kernel even for whole tiles
+  static const char *tile_env = getenv("TTS_GEMM_TILE");  // (as in gemm_choose)
+  const bool kept = chosen && chosen->split == std::max(1, p.split);
   if (!tile_env) {
     // Whole K tiles go to the direct-to-LDS kernels.
-    // at most p.split slices: what gemm_split said, or fewer when the caller's workspace holds no more (1: none)
-    const DmaChoice choice = p.counters ? DmaChoice{&DMA_CANDS[3], p.split} : choose_dma(p, std::max(1, p.split));
+    // at most p.split slices: what was chosen, or fewer when the caller's workspace holds no more (1: none)
+    const DmaChoice choice = !kept ? choose_dma(p, std::max(1, p.split)) : chosen->tile < 0 ? DmaChoice{} : DmaChoice{&DMA_CANDS[chosen->tile], chosen->split};
     GemmParams q = p;
     q.split = choice.split;
     const DmaCand *best = choice.tile;
@@ -824,7 +825,7 @@ hipError_t launch_gemm(const GemmParams &p, hipStream_t s, const char **name) {
   // anything else: 128 x 128 x 64 tiles, two workgroups per CU, or half as high (a 256 x 256 x 32 form of the same kernel measured behind it
   // at every size tried: 4096^3: 202 against 197 us; 4096 x 2048 x 2048: 112 against 56 us)
   GemmParams q = p;
-  q.split = tile_env || !p.partial ? 1 : any_split(p, std::max(1, p.split));
+  q.split = tile_env || !p.partial ? 1 : kept ? chosen->split : any_split(p, std::max(1, p.split));
   *name = any_name(any_rows(q, q.split), false, q.split > 1);
   if (q.split == 1) return p.is_bf16 ? launch_gemm_any<true, false>(q, s) : launch_gemm_any<false, false>(q, s);
   hipError_t e = launch_gemm_any_slices(q, s);

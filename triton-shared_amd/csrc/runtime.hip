@@ -66,6 +66,10 @@ struct Bound {
   SoftmaxParams softmax{};
   LayerNormParams layernorm{};
   GemmParams gemm{};
+  // What the product runs on (gemm_choose) with its operands as aligned as in some launch before, and its slices meeting in the
+  // kernel or not: at the index the launcher makes of these; under the plan's mutex.
+  GemmChoice gemm_choice[16];
+  bool gemm_chosen[16] = {};
   GemmW8A16Params w8{};
   MapNParams mapn{};
   bool empty = false;  // nothing to do (e.g. zero trip count with nothing stored)
@@ -504,6 +508,12 @@ void bind_gemm(const Resolver &r, Bound &b) {
   os << "kernel=gemm_mfma\nM=" << p.M << "\nN=" << p.N << "\nK=" << p.K << "\nlda=" << p.lda << "\nldb=" << p.ldb
      << "\nldc=" << p.ldc << "\nbf16=" << p.is_bf16 << "\nf32=" << p.is_f32 << "\na_trans=" << p.a_trans << "\nb_trans=" << p.b_trans << "\n";
   if (p.batches > 1) os << "batches=" << p.batches << "\nbatch_a=" << p.batch_a << "\nbatch_b=" << p.batch_b << "\nbatch_c=" << p.batch_c << "\n";
+  if (r.pl.source.empty()) {  // what it runs on with operands that are aligned (as these null ones are) and memory to be had
+    p.meet = 1;
+    const GemmChoice &choice = b.gemm_choice[15] = gemm_choose(p);
+    b.gemm_chosen[15] = true;
+    os << "slices=" << choice.split << "\nmeet=" << (choice.meeting > 0) << "\n";
+  }
   b.describe = os.str();
 }
 
@@ -971,38 +981,42 @@ tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, con
           // they fit there (else that call runs the product without slices)
           // (the any-shape kernel keeps to whole products where the launch may not allocate or is recorded into a graph)
           // slices that meet in the kernel count their arrivals: not where a graph could be replayed beside other launches
-          p.meet = !no_alloc && !is_capturing(s);
-          const int want = gemm_split(p);
-          if (want > 1 && !(gemm_any_shape(p) && (no_alloc || is_capturing(s)))) {
-            p.split = want;
-            size_t need = gemm_workspace_bytes(p), meeting_bytes = 0;
-            const size_t meeting = p.meet ? gemm_meeting(p, &meeting_bytes) : 0;
-            if (meeting) {  // (a later recording finds room for the sums that a second kernel adds)
-              GemmParams recorded = p;
-              recorded.meet = 0;
-              recorded.split = gemm_split(recorded);
-              need = std::max(meeting_bytes, gemm_workspace_bytes(recorded));
+          const bool recorded = is_capturing(s);
+          auto choose = [&](bool meet) {
+            p.meet = meet;
+            const int at = (((uintptr_t)p.a & 15) == 0) | (((uintptr_t)p.b & 15) == 0) << 1 | (((uintptr_t)p.c & 3) == 0) << 2 | meet << 3;
+            std::lock_guard<std::mutex> lock(plan->mu);
+            if (!b->gemm_chosen[at]) {
+              b->gemm_choice[at] = gemm_choose(p);
+              b->gemm_chosen[at] = true;
             }
+            return b->gemm_choice[at];
+          };
+          const GemmChoice choice = choose(!no_alloc && !recorded);
+          if (choice.split > 1 && !(choice.tile < 0 && (no_alloc || recorded))) {
+            p.split = choice.split;
+            // (a later recording finds room for the sums that a second kernel adds)
+            const size_t need = choice.meeting ? std::max(choice.bytes, choose(false).bytes) : choice.bytes;
             if (no_alloc) {  // as many slices as the static array holds
               const size_t one = (size_t)p.M * p.N * std::max(1, p.batches) * sizeof(float);
-              p.split = (int)std::min<size_t>((size_t)want, NOALLOC_WORKSPACE_BYTES / one);
+              p.split = (int)std::min<size_t>((size_t)choice.split, NOALLOC_WORKSPACE_BYTES / one);
               if (p.split > 1) p.partial = reinterpret_cast<float *>(noalloc_scratch());
               else p.split = 1;
             } else {
               std::lock_guard<std::mutex> lock(plan->mu);
               tts_plan::SplitK &sk = plan->split_k[stream];
-              if (sk.workspace_bytes < need && is_capturing(s)) {  // nothing is allocated while a graph is recorded: the whole product
+              if (sk.workspace_bytes < need && recorded) {  // nothing is allocated while a graph is recorded: the whole product
                 p.split = 1;
               } else {
                 hipError_t e = plan->grow((void **)&sk.workspace, &sk.workspace_bytes, need);
-                if (e == hipSuccess && meeting) e = plan->grow_counters(sk, 32 * meeting);
+                if (e == hipSuccess && choice.meeting) e = plan->grow_counters(sk, 32 * choice.meeting);
                 if (e != hipSuccess) return fail(TTS_HIP_ERROR, std::string("hipMalloc(split-K workspace): ") + hipGetErrorString(e));
                 p.partial = sk.workspace;
-                if (meeting) p.counters = sk.counters;
+                if (choice.meeting) p.counters = sk.counters;
               }
             }
           }
-          err = launch_gemm(p, s, &kname);
+          err = launch_gemm(p, s, &kname, &choice);
           break;
         }
         static_assert(TILE_MAX_ARGS == 32, "GemmEpilogueArgs holds 32 arguments");
