@@ -570,11 +570,13 @@ def test_gemm_any_shape_kernel_at_the_ends_of_its_tiles(K, M, N, Kd, at, bt):
 
 
 @pytest.mark.parametrize("M,N,Kd,at,bt,dtype", [(256, 512, 1600, False, False, torch.bfloat16), (1000, 2048, 4096, False, True, torch.float16),
-                                                 (770, 776, 1536, False, False, torch.float16), (136, 648, 2048, True, False, torch.bfloat16), (520, 512, 1600, True, True, torch.float16)])
+                                                 (770, 776, 1536, False, False, torch.float16), (136, 648, 2048, True, False, torch.bfloat16), (520, 512, 1600, True, True, torch.float16),
+                                                 (512, 512, 1536, True, False, torch.bfloat16), (893, 1144, 1408, False, False, torch.float16), (1016, 1000, 1536, True, True, torch.bfloat16),
+                                                 (384, 384, 1088, False, True, torch.bfloat16)])
 def test_gemm_slices_that_meet_in_the_kernel(K, M, N, Kd, at, bt, dtype):
-    """128 x 128 tiles in two to five K slices, which the workgroup of a tile that arrives last adds: whole and ragged tiles, either
-    operand column-major, again and again over one workspace whose counters every launch leaves at zero, and recorded, where a second
-    kernel adds them.  Small integers with few of them at once: exact in any order, and results of at most 8 bits."""
+    """128 x 128 tiles in K slices, which the workgroup of a tile that arrives last adds or (three of the sizes) a second kernel: whole
+    and ragged tiles, either operand column-major, again and again over one workspace whose counters every launch leaves at zero, and
+    recorded, where a second kernel adds them.  Small integers with few of them at once: exact in any order, and results of at most 8 bits."""
     g = torch.Generator().manual_seed(M + N)
     A = torch.zeros(M, Kd, dtype=dtype)
     A.scatter_(1, torch.randint(0, Kd, (M, 60), generator=g), 1.0)
@@ -596,6 +598,8 @@ def test_gemm_slices_that_meet_in_the_kernel(K, M, N, Kd, at, bt, dtype):
             k = run()
             assert k.function.last_kernel == "gemm_dma_kernel<128x128>, K slices", k.function.last_kernel
         check()
+    said = k.function.describe_launch((triton.cdiv(M, 128) * triton.cdiv(N, 128), 1, 1), [0, 0, 0, M, N, Kd] + [x for x in (a.stride(0), a.stride(1), b.stride(0), b.stride(1), N + 8, 1) if x != 1])
+    assert said["meet"] == str(int(M not in (770, 136, 520))) and int(said["slices"]) > 1, said
     graph = torch.cuda.CUDAGraph()
     torch.cuda.synchronize()
     with torch.cuda.graph(graph, stream=streams[0]):

@@ -723,6 +723,17 @@ def test_matrix_programs_hold_blocks_of_whole_column_groups_only(native, tmp_pat
     assert src.startswith("// tts: matrix") == (C == 32) and "[0]; " not in src
 
 
+@pytest.mark.parametrize("M,N,K,meet", [(768, 768, 1536, 1), (1024, 1024, 1792, 1), (1024, 2048, 3072, 1), (512, 512, 1536, 1), (1024, 1536, 4096, 1),
+                                        (200, 1600, 1600, 0), (808, 1144, 2816, 0), (1024, 1024, 4096, 0), (183, 3384, 3968, 0), (245, 568, 1664, 0), (594, 144, 1312, 0),
+                                        (1715, 408, 7008, 0), (256, 256, 4096, 0)])
+def test_slices_meet_in_the_kernel_only_where_that_is_ahead(native, M, N, K, meet):
+    """Two or three slices of filled tiles are added by the workgroup that arrives last; in more slices, and where tiles stick out of C,
+    a second kernel was measured ahead (200 x 1600 x 1600 13.5 us against 14.5, 808 x 1144 x 2816 19.2 against 21.3)."""
+    plan, _ = plan_for(native, "matmul_tiles")
+    said = plan.describe_launch((-(-M // 128) * -(-N // 128), 1, 1), [0, 0, 0, M, N, K, K, N, N])
+    assert int(said["slices"]) > 1 and int(said["meet"]) == meet and (not meet or int(said["slices"]) <= 3), said
+
+
 def test_direct_loads_to_lds_stand_behind_their_operands(native, tmp_path):
     """A direct-to-LDS load reads m0 one instruction behind its write at the earliest, and a scalar base address that a vector
     instruction wrote five behind it.  Inside inline assembly nobody counts: there, something stands between the write of m0 and

@@ -135,7 +135,7 @@ hipError_t launch_gemm_dma_slices(const GemmParams &p, hipStream_t s) {
   return hipGetLastError();
 }
 
-// 128 x 128 tiles in K slices that meet in the kernel (slices_meet; chosen by slices_may_meet)
+// 128 x 128 tiles in K slices that meet in the kernel (slices_meet; chosen by choose_dma)
 template <bool BF16, bool BT, bool AT>
 __global__ __launch_bounds__(256) void gemm_dma_meeting_kernel(GemmParams p, int tiles_m, int tiles_n) {
   gemm_dma_body<BF16, 2, 2, IdentityEp, BT, AT, false, true, true>(p, tiles_m, tiles_n, IdentityEp());
@@ -665,18 +665,26 @@ namespace {
 struct DmaCand { const char *tag; int64_t bm, bn; double eff, round, turned, fill, fixed; };
 const DmaCand DMA_CANDS[4] = {{"256x256", 256, 256, 1.0, 0.59, 0.07, 0.04, 9}, {"128x256", 128, 256, 0.77, 0.48, 0.07, 0.05, 6},
                               {"256x128", 256, 128, 0.73, 0.51, 0.03, 0.04, 6.3}, {"128x128", 128, 128, 0.59, 0.34, 0, 0.03, 3.8}};
-struct DmaChoice { const DmaCand *tile = nullptr; int split = 1; };
+struct DmaChoice { const DmaCand *tile = nullptr; int split = 1; bool meet = false; };  // meet: the slices meet in the kernel
 
-// us that the slices of a product take to become one: through a second kernel that the whole chip runs, or, on 128 x 128 tiles,
-// in the workgroup of a tile that arrives last, which reads its 64 KiB per slice alone.  Modelled on 16 ... 64 tiles in 2 ... 8 slices.
-// us per call, second kernel / in the kernel, each in the slices it chooses: 256 x 512 x 1600 14.6 / 12.0; 256 x 4096 x 2048 17.5 / 14.9;
-// 576 x 960 x 1408 15.3 / 13.2; 768 x 768 x 1536 16.5 / 14.0; 1024 x 1024 x 1792 17.6 / 14.7; 1024 x 2048 x 3072 24.0 / 22.3; 512 x 1536 x 2560
-// 15.8 / 15.9; 1408 x 704 x 2496 17.0 / 17.5, the one of 17 that lost; in 8 slices and more, where the rule keeps the second kernel,
-// 16 x 4096 x 4096 16.0 / 22.3 and 128 x 4096 x 4096 19.7 / 22.7.
+// us that K slices take to become one through a second kernel that the whole chip runs.
 double added_us(const GemmParams &p, int split) { return 5.5 + 0.28e-6 * split * 4 * (double)p.M * (double)p.N * std::max(1, p.batches); }
-double meeting_us(int split) { return 2.4 * split - 4; }
-bool slices_may_meet(const GemmParams &p, const DmaCand &c, int split) {
-  return p.meet && &c == &DMA_CANDS[3] && split > 1 && p.batches <= 1 && meeting_us(split) < added_us(p, split);
+// On 128 x 128 tiles the workgroup of a tile that arrives last can add the slices instead (slices_meet), reading 64 KiB of each alone.
+// Two or three slices gain by it; more lose, every slice costing that workgroup a trip to memory, and so do tiles that stick out of C,
+// which are handed over and stored as a whole where the second kernel reads only what belongs to C.  us of a product whose operands
+// are in cache, by its second kernel in the slices that `time` says and by their meeting in two or three, both fitted (5 % rms) to 207
+// sizes of 6 ... 140 tiles, K 1056 ... 8192; the host takes some 13 us for two launches from Python and 10.5 for one, whatever the GPU does.
+// us, apart / together: 768 x 768 x 1536 16.4 / 14.1, 1024 x 1024 x 1792 17.7 / 14.6, 941 x 768 x 1376 15.9 / 13.1, 512 x 512 x 1536 13.8 / 12.1,
+// 1024 x 2048 x 3072 24.7 / 23.3; where the rule keeps the second kernel 200 x 1600 x 1600 13.5 / 14.5, 808 x 1144 x 2816 19.2 / 21.3, 1024 x 1024
+// x 4096 19.7 / 20.6, 183 x 3384 x 3968 21.6 / 23.0, 245 x 568 x 1664 13.0 / 13.8, 256 x 256 x 4096 in eight slices 12.8 / 17.4.
+constexpr double APART_HOST_US = 13.0, TOGETHER_HOST_US = 10.5;
+double apart_us(const GemmParams &p, int64_t tiles, int64_t nk, int split, int cus) {
+  const double mb = 4e-6 * (double)p.M * (double)p.N, f = std::min(1.0, (double)tiles * split / cus);
+  return std::max(APART_HOST_US, 5.6 + 0.38 * split + (0.4 + 0.33 * split) * mb + (0.237 - 0.026 * f) * (double)((nk + split - 1) / split) + (p.M % 128 ? 0.8 : 0) - (p.N % 128 ? 0.2 : 0));
+}
+double together_us(const GemmParams &p, int64_t tiles, int64_t nk, int split, int cus) {
+  const double t = (double)tiles / 64, f = (double)tiles * split / cus;
+  return std::max(TOGETHER_HOST_US, 4.8 + 1.03 * split + (0.81 * split - 0.09) * t + (0.2355 + 0.016 * f) * (double)((nk + split - 1) / split) + (p.M % 128 ? 0.5 : 0) + (p.N % 128 ? 0.9 : 0));
 }
 
 DmaChoice choose_dma(const GemmParams &p, int max_split) {
@@ -708,17 +716,17 @@ DmaChoice choose_dma(const GemmParams &p, int max_split) {
   const bool by_rounds = !grouped && p.K >= 512;
   const int64_t nk = p.K / F_BK;
   const double sums = (double)p.M * (double)p.N * std::max(1, p.batches) * 4;  // bytes of one slice's
-  auto time = [&](const DmaCand &c, int split, bool meet) {
+  auto time = [&](const DmaCand &c, int split) {
     const double f = (double)tiles(c) * split / cus;
     return (double)((nk + split - 1) / split) * (std::ceil(f) * (c.round + (p.b_trans ? c.turned : 0)) + f * c.fill) + c.fixed +
-           (split == 1 ? 0 : meet && slices_may_meet(p, c, split) ? meeting_us(split) : added_us(p, split));
+           (split == 1 ? 0 : added_us(p, split));
   };
   DmaChoice best;
   double best_cost = 0;
   for (const DmaCand &c : DMA_CANDS) {
     if (!gemm_dma_ok(p, c.bm, c.bn)) continue;
     if (dma_env ? std::string(dma_env) != c.tag : !by_rounds && c.bm + c.bn != 256 && (grouped ? !grouped_wide(tiles(c)) : tiles(c) < cus)) continue;
-    const double cost = by_rounds ? time(c, 1, false) : (double)(tiles(c) * c.bm * c.bn) / c.eff;
+    const double cost = by_rounds ? time(c, 1) : (double)(tiles(c) * c.bm * c.bn) / c.eff;
     if (!best.tile || cost < best_cost) { best.tile = &c; best_cost = cost; }
   }
   if (!best.tile || max_split < 2 || !by_rounds || p.a_rows || p.b_block) return best;
@@ -727,20 +735,33 @@ DmaChoice choose_dma(const GemmParams &p, int max_split) {
   if (best.tile == &DMA_CANDS[3] && p.K <= 1024 && !split_env && p.batches <= 1) return best;
   DmaChoice pick = best;
   double pick_t = best_cost;
-  // (what is ahead whole of slices that a second kernel adds stays whole, however little their meeting takes: 1152 x 1536 x 1024
-  // 11.5 us against 14.9 in two slices)
-  for (const bool meet : {false, true}) {
-    if (split_env && atoi(split_env) == 1) break;
-    if (meet && (!p.meet || pick.split == 1)) break;
+  if (!(split_env && atoi(split_env) == 1))
     for (const DmaCand &c : DMA_CANDS) {
       if (!gemm_dma_ok(p, c.bm, c.bn) || (dma_env && std::string(dma_env) != c.tag)) continue;
       const int64_t most = std::min<int64_t>(std::min<int64_t>(std::min<int64_t>(16, max_split), nk / 8), (2 * cus + tiles(c) - 1) / tiles(c));
       for (int64_t sp = split_env ? atoi(split_env) : 2; sp <= most; sp++) {
         if (sp * sums > (double)((size_t)256 << 20)) break;
-        const double t = time(c, (int)sp, meet);
+        const double t = time(c, (int)sp);
         if (t < pick_t || (split_env && pick.split == 1)) { pick.tile = &c; pick.split = (int)sp; pick_t = t; }
         if (split_env) break;
       }
+    }
+  // Slices that would meet in the kernel instead.  (What is ahead whole of slices that a second kernel adds stays whole: 1152 x 1536 x
+  // 1024 11.5 us against 14.9 in two slices.)  From larger tiles, for which `time` knows what 128 x 128 in few slices would take with
+  // their meeting in place of the second kernel: 1024 x 1536 x 4096 24.1 us against five slices of 128 x 256 at 26.9; only where the tiles are
+  // filled (1715 x 408 x 7008 28.0 / 26.1).
+  if (p.meet && pick.split > 1 && p.batches <= 1 && !split_env) {
+    const DmaCand &c = DMA_CANDS[3];
+    const int64_t t = tiles(c);
+    const bool same = pick.tile == &c, filled = (double)p.M * (double)p.N >= 0.85 * 128 * 128 * (double)t;
+    const double apart = same ? apart_us(p, t, nk, pick.split, cus) : 0;
+    // us to be gained at least: of 207 sizes 66 gain 1.085 in the geometric mean, three lose 1.8 % at most (at 1.0 five, 3.6 %)
+    double most = !same ? 0 : apart > APART_HOST_US ? 1.2 : 0.6;
+    for (int sp = 2; sp <= 3; sp++) {
+      if (!gemm_dma_ok(p, c.bm, c.bn) || (dma_env && std::string(dma_env) != c.tag) || sp > max_split || nk / 8 < sp || t * sp > cus || !(same || filled)) continue;
+      const double gain = same ? apart - together_us(p, t, nk, sp, cus)
+                               : pick_t - (time(c, sp) - added_us(p, sp) + 2.4 * sp - 4);
+      if (gain > most) { pick = {&c, sp, true}; most = gain; }
     }
   }
   return pick;
@@ -787,7 +808,7 @@ GemmChoice gemm_choose(const GemmParams &p) {
   GemmParams q = p;
   q.split = c.split = dma.tile ? dma.split : any_split(p, 16);
   c.bytes = gemm_workspace_bytes(q);
-  if (dma.tile && slices_may_meet(p, *dma.tile, c.split)) {
+  if (dma.meet) {
     c.meeting = (size_t)(((p.M + 127) / 128) * ((p.N + 127) / 128));
     c.bytes = (size_t)c.split * c.meeting * (128 * 128 * sizeof(float));
   }
