@@ -283,3 +283,92 @@ def test_recorded_launches_of_the_tiled_int8_product_allocate_nothing(native):
         graph.replay()
         torch.cuda.synchronize()
         assert ((got.double() - want.double()).norm() / want.double().norm()).item() <= 2.0 ** -11   # (the eager launch runs in K slices)
+
+
+@pytest.mark.parametrize("M,N,Kd", [(4, 24704, 4096), (15, 2048, 6400), (40, 1040, 4096)])
+def test_recorded_first_launches_of_the_int8_decode_kernels_allocate_nothing(native, M, N, Kd):
+    # products that run in K slices, first launched on a stream while it records a graph: recorded whole, without workspace and
+    # counters; an eager launch on the stream then runs in slices, and one recorded after it, too
+    plan, _ = plan_for(native, "w8a16_matmul")
+    a, w, s = _inputs(M, N, Kd, 3)
+    got = torch.zeros(M, N, dtype=torch.float16, device=DEV)
+    grid = ((M + 15) // 16, (N + 127) // 128, 1)
+    launch = lambda: plan.launch(grid, torch.cuda.current_stream().cuda_stream, _values(a, w, s, got, M, N, Kd))
+    assert int(plan.describe_launch(grid, _values(a, w, s, got, M, N, Kd))["split"]) > 1
+    launch()                                   # (on another stream)
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream()
+    for turn in range(2):
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            launch()
+        for seed in range(3):
+            a.copy_(_inputs(M, N, Kd, 10 + seed)[0])
+            ref = a.double() @ (w.half() * s[None, :]).double()
+            for run in (graph.replay, launch):
+                got.zero_()
+                torch.cuda.synchronize()
+                with torch.cuda.stream(side):
+                    run()
+                torch.cuda.synchronize()
+                # fp32 sums in two orders, rounded once to fp16
+                assert ((got.double() - ref).norm() / ref.norm()).item() <= 2.0 ** -11
+
+
+@pytest.mark.parametrize("kind", ["softmax loop in slices", "sums in slices", "slices that meet", "int8 weights"])
+def test_first_launches_beside_a_stream_that_records(native, kind):
+    # a launch that takes a workspace and counters, the first on its stream, while another stream records a graph: it neither fails
+    # nor ends the recording
+    import triton
+    import triton_shared_amd as tsa
+    import extra_kernels as X
+    from triton_shared_amd.examples import kernels as K
+    tsa.activate()
+    g = torch.Generator().manual_seed(8)
+    if kind == "softmax loop in slices":
+        H, seq, D = 2, 1500, 64
+        q, k, v = (torch.randn(H, seq, D, generator=g).half().to(DEV) for _ in range(3))
+        out = torch.zeros(H, seq, D, dtype=torch.float16, device=DEV)
+        launch = lambda: X.attention_fwd[(triton.cdiv(seq, 64), H)](q, k, v, out, D ** -0.5, seq, seq * D, D, BM=64, BN=64, D=D)
+        want = torch.nn.functional.scaled_dot_product_attention(q.float().cpu(), k.float().cpu(), v.float().cpu())
+    elif kind == "sums in slices":
+        rows, cols = 4096, 512
+        x = torch.randn(rows, cols, generator=g).to(DEV)
+        out = torch.zeros(cols, device=DEV)
+        launch = lambda: X.block_column_sums[(1, cols // 64)](x, out, rows, cols, BR=16, BC=64)
+        want = x.double().sum(0).cpu()
+    elif kind == "slices that meet":
+        M, N, Kd = 768, 768, 1536
+        a, b = torch.randn(M, Kd, generator=g).bfloat16().to(DEV), torch.randn(Kd, N, generator=g).bfloat16().to(DEV)
+        out = torch.zeros(M, N, dtype=torch.bfloat16, device=DEV)
+        launch = lambda: K.matmul_tiles[(36,)](a, b, out, M, N, Kd, Kd, 1, N, 1, N, 1, BM=128, BN=128, BK=64, GROUP_M=8)
+        want = (a.double() @ b.double()).cpu()
+    else:
+        M, N, Kd = 15, 2048, 6400
+        a, w, s = _inputs(M, N, Kd, 3)
+        out = torch.zeros(M, N, dtype=torch.float16, device=DEV)
+        launch = lambda: K.w8a16_matmul[(1, 16)](a, w, s, out, M, N, Kd, Kd, 1, N, 1, N, 1, BM=16, BN=128, BK=128)
+        want = (a.double() @ (w.half() * s[None, :]).double()).cpu()
+    launch()   # (compiles what it needs)
+    torch.cuda.synchronize()
+    count = torch.zeros(1, device=DEV)
+    one, other = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    out.zero_()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=one):
+        count.add_(1)
+        with torch.cuda.stream(other):
+            launch()
+        count.add_(1)
+    torch.cuda.synchronize()
+    assert ((out.double().cpu() - want.double()).norm() / want.double().norm()).item() <= 5e-3   # (16-bit results)
+    for turn in range(3):
+        out.zero_()
+        graph.replay()
+        with torch.cuda.stream(other):
+            launch()
+        torch.cuda.synchronize()
+        assert count.item() == 2 * (turn + 1)
+        assert ((out.double().cpu() - want.double()).norm() / want.double().norm()).item() <= 5e-3

@@ -59,6 +59,20 @@ void may_allocate(const char *what) {
     throw WouldAllocate(std::string("tts_launch_noalloc: this launch needs ") + what + ", which allocates; run it once through tts_launch first");
 }
 
+// Whether the stream records a graph: nothing may be allocated then, and a workspace of the stream's would be shared by
+// every replay.
+bool is_capturing(hipStream_t s) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &status) == hipSuccess) return status != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return false;
+}
+
+__global__ void clear_ints_kernel(int *p, int n) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) p[i] = 0;
+}
+
 // Everything a launch needs besides the pointers, resolved for one (scalars, grid).
 struct Bound {
   Family family;
@@ -137,20 +151,39 @@ struct tts_plan {
     *have = got;
     return hipSuccess;
   }
-  // At least `need` arrival counters for a stream; called with `mu` held.  (New counters start at zero; the old ones, which
-  // launches in flight may still be bumping, are retired.)
-  hipError_t grow_counters(SplitK &sk, size_t need) {
+  // At least `need` arrival counters for a stream; called with `mu` held.  New counters are cleared on the stream, in front of the
+  // launches on it that use them, so that nothing waits for the device; the old ones, which launches in flight may still be
+  // bumping, are retired.
+  hipError_t grow_counters(SplitK &sk, size_t need, hipStream_t s) {
     if (sk.counters_count >= need) return hipSuccess;
     int *fresh = nullptr;
     const size_t count = std::max(need, 2 * sk.counters_count);
     hipError_t e = hipMalloc((void **)&fresh, count * sizeof(int));
-    if (e == hipSuccess) e = hipMemset(fresh, 0, count * sizeof(int));
-    if (e == hipSuccess) e = hipDeviceSynchronize();  // the fill has landed before a launch on any stream reads the counters
     if (e != hipSuccess) return e;
-    if (sk.counters) retired.push_back(sk.counters);
+    hipLaunchKernelGGL(clear_ints_kernel, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, s, fresh, (int)count);
+    e = hipGetLastError();
+    retired.push_back(e == hipSuccess ? sk.counters : fresh);  // (freeing null is nothing)
+    if (e != hipSuccess) return e;
     sk.counters = fresh;
     sk.counters_count = count;
     return hipSuccess;
+  }
+  // The stream's scratch memory, with at least so many bytes of workspace, counters and widened weights: null where that cannot be had,
+  // because the stream records a graph and does not have it yet, or because there is no memory.  Called with `mu` held; every
+  // caller has a way to launch without.  (Another stream may be recording: allocating is allowed beside that in the relaxed mode alone.)
+  SplitK *room(hipStream_t s, size_t bytes, size_t counters, size_t widened = 0) {
+    SplitK &sk = split_k[s];
+    if (sk.workspace_bytes >= bytes && sk.counters_count >= counters && sk.widened_bytes >= widened) return &sk;
+    if (is_capturing(s)) return nullptr;
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    const bool changed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    hipError_t e = grow((void **)&sk.workspace, &sk.workspace_bytes, bytes);
+    if (e == hipSuccess) e = grow(&sk.widened, &sk.widened_bytes, widened);
+    if (e == hipSuccess) e = grow_counters(sk, counters, s);
+    if (changed) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (e == hipSuccess) return &sk;
+    (void)hipGetLastError();
+    return nullptr;
   }
   RtcModule *fused = nullptr;  // the kernel compiled for this plan at its first launch (fused maps, tile programs)
   RtcModule *gemm_rtc[GEMM_EPILOGUE_KERNELS] = {};  // matrix products with a fused epilogue: launch_gemm_epilogue's kernels
@@ -629,11 +662,6 @@ static __device__ __align__(256) unsigned char scratch[NOALLOC_WORKSPACE_BYTES +
 
 namespace {
 
-__global__ void clear_ints_kernel(int *p, int n) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = 0;
-}
-
 // the current device's copy of `scratch`
 unsigned char *noalloc_scratch() {
   static std::mutex mu;
@@ -739,15 +767,6 @@ int compute_units() {  // of the current device (256 when the query fails)
   return cus;
 }
 
-// Whether the stream records a graph: nothing may be allocated then, and a workspace of the stream's would be shared by
-// every replay.
-bool is_capturing(hipStream_t s) {
-  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(s, &status) == hipSuccess) return status != hipStreamCaptureStatusNone;
-  (void)hipGetLastError();
-  return false;
-}
-
 // Slices of an online softmax's loop (tile_mma.h): where its workgroups leave CUs idle each walks all of its blocks alone, and where
 // they fill them about once the longest loops are what the launch waits for.  The least modelled time, in iterations of a
 // workgroup alone on its CU (half as long again beside another): the longest slice, or the work of the chip and half of that
@@ -836,12 +855,12 @@ tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, con
           if (sa.slices > 1 && (no_alloc || is_capturing(s))) sa.slices = 1;  // (as for the sums below)
           if (sa.slices > 1) {
             std::lock_guard<std::mutex> lock(plan->mu);
-            tts_plan::SplitK &sk = plan->split_k[stream];
-            hipError_t e = plan->grow((void **)&sk.workspace, &sk.workspace_bytes, (size_t)workgroups * sa.slices * traits.floats * sizeof(float));
-            if (e == hipSuccess) e = plan->grow_counters(sk, (size_t)workgroups * 32);  // (128 bytes apart)
-            if (e != hipSuccess) return fail(TTS_HIP_ERROR, std::string("hipMalloc(slices' states): ") + hipGetErrorString(e));
-            sa.partial = sk.workspace;
-            sa.counters = sk.counters;
+            if (const tts_plan::SplitK *sk = plan->room(s, (size_t)workgroups * sa.slices * traits.floats * sizeof(float), (size_t)workgroups * 32)) {  // (128 bytes apart)
+              sa.partial = sk->workspace;
+              sa.counters = sk->counters;
+            } else {
+              sa.slices = 1;
+            }
           }
           const int64_t all = workgroups * sa.slices, x = std::min<int64_t>(all, 1 << 23);
           err = rtc_launch(*slot, (int)x, (int)((all + x - 1) / x), 1, traits.threads, &sa, sizeof sa, s);
@@ -864,12 +883,12 @@ tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, con
         if (sa.slices > 1 && (no_alloc || is_capturing(s))) sa.slices = 1;
         if (sa.slices > 1) {
           std::lock_guard<std::mutex> lock(plan->mu);
-          tts_plan::SplitK &sk = plan->split_k[stream];
-          hipError_t e = plan->grow((void **)&sk.workspace, &sk.workspace_bytes, (size_t)programs * sa.slices * traits.floats * sizeof(float));
-          if (e == hipSuccess) e = plan->grow_counters(sk, (size_t)programs * 32);  // (128 bytes apart)
-          if (e != hipSuccess) return fail(TTS_HIP_ERROR, std::string("hipMalloc(partial sums): ") + hipGetErrorString(e));
-          sa.partial = sk.workspace;
-          sa.counters = sk.counters;
+          if (const tts_plan::SplitK *sk = plan->room(s, (size_t)programs * sa.slices * traits.floats * sizeof(float), (size_t)programs * 32)) {  // (128 bytes apart)
+            sa.partial = sk->workspace;
+            sa.counters = sk->counters;
+          } else {
+            sa.slices = 1;
+          }
         }
         // one slice: the grid as it is, a workgroup per program, its x and y exchanged where the program asks for that (see below)
         const bool whole = sa.slices == 1, swap = whole && traits.swaps_grid && gy > 1 && gx <= 65535;
@@ -992,27 +1011,29 @@ tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, con
             }
             return b->gemm_choice[at];
           };
-          const GemmChoice choice = choose(!no_alloc && !recorded);
+          GemmChoice choice = choose(!no_alloc && !recorded);
           if (choice.split > 1 && !(choice.tile < 0 && (no_alloc || recorded))) {
             p.split = choice.split;
-            // (a later recording finds room for the sums that a second kernel adds)
-            const size_t need = choice.meeting ? std::max(choice.bytes, choose(false).bytes) : choice.bytes;
             if (no_alloc) {  // as many slices as the static array holds
               const size_t one = (size_t)p.M * p.N * std::max(1, p.batches) * sizeof(float);
               p.split = (int)std::min<size_t>((size_t)choice.split, NOALLOC_WORKSPACE_BYTES / one);
               if (p.split > 1) p.partial = reinterpret_cast<float *>(noalloc_scratch());
               else p.split = 1;
             } else {
-              std::lock_guard<std::mutex> lock(plan->mu);
-              tts_plan::SplitK &sk = plan->split_k[stream];
-              if (sk.workspace_bytes < need && recorded) {  // nothing is allocated while a graph is recorded: the whole product
-                p.split = 1;
-              } else {
-                hipError_t e = plan->grow((void **)&sk.workspace, &sk.workspace_bytes, need);
-                if (e == hipSuccess && choice.meeting) e = plan->grow_counters(sk, 32 * choice.meeting);
-                if (e != hipSuccess) return fail(TTS_HIP_ERROR, std::string("hipMalloc(split-K workspace): ") + hipGetErrorString(e));
-                p.partial = sk.workspace;
-                if (choice.meeting) p.counters = sk.counters;
+              auto room = [&](size_t bytes, size_t counters) {
+                std::lock_guard<std::mutex> lock(plan->mu);
+                const tts_plan::SplitK *sk = plan->room(s, bytes, counters);
+                if (!sk) return false;
+                p.partial = sk->workspace;
+                if (counters) p.counters = sk->counters;
+                return true;
+              };
+              // without memory the second kernel's sums may still fit what the stream has, and the whole product needs none
+              // (a later recording finds room for the sums that a second kernel adds)
+              if (!room(choice.meeting ? std::max(choice.bytes, choose(false).bytes) : choice.bytes, 32 * choice.meeting)) {
+                if (choice.meeting) choice = choose(false);
+                else choice.split = 1;
+                p.split = choice.split > 1 && room(choice.bytes, 0) ? choice.split : 1;
               }
             }
           }
@@ -1045,10 +1066,8 @@ tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, con
           const bool may_compile = !no_alloc && !(recorded && gemm_epilogue_compiled(p, plan->gemm_rtc));
           if (want > 1 && !no_alloc && !recorded) {
             p.split = want;
-            tts_plan::SplitK &sk = plan->split_k[stream];
-            hipError_t e = plan->grow((void **)&sk.workspace, &sk.workspace_bytes, gemm_workspace_bytes(p));
-            if (e != hipSuccess) return fail(TTS_HIP_ERROR, std::string("hipMalloc(split-K workspace): ") + hipGetErrorString(e));
-            p.partial = sk.workspace;
+            if (const tts_plan::SplitK *sk = plan->room(s, gemm_workspace_bytes(p), 0)) p.partial = sk->workspace;
+            else p.split = 1;
           }
           err = launch_gemm_epilogue(p, pl.source, plan->gemm_rtc, may_compile, a, s, &kname, &why);
         }
@@ -1079,35 +1098,27 @@ tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, con
             if (e != hipSuccess) return fail(TTS_HIP_ERROR, std::string("clearing the split-K counters: ") + hipGetErrorString(e));
           }
         } else if (p.split > 1 && !tiled) {
-          const size_t need = gemm_w8a16_workspace_bytes(p), ncount = gemm_w8a16_counters(p);
           std::lock_guard<std::mutex> lock(plan->mu);
-          tts_plan::SplitK &sk = plan->split_k[stream];
-          hipError_t e = plan->grow((void **)&sk.workspace, &sk.workspace_bytes, need);
-          if (e != hipSuccess) return fail(TTS_HIP_ERROR, std::string("hipMalloc(split-K workspace): ") + hipGetErrorString(e));
-          e = plan->grow_counters(sk, ncount);
-          if (e != hipSuccess) return fail(TTS_HIP_ERROR, std::string("hipMalloc(split-K counters): ") + hipGetErrorString(e));
-          p.workspace = sk.workspace;
-          p.counters = sk.counters;
+          if (const tts_plan::SplitK *sk = plan->room(s, gemm_w8a16_workspace_bytes(p), gemm_w8a16_counters(p))) {
+            p.workspace = sk->workspace;
+            p.counters = sk->counters;
+          } else {
+            p.split = 1;
+          }
         }
         p.widened = nullptr;
         if (!no_alloc) {  // (the call that may not allocate stays on the decode kernels, a launch per 32 rows)
           const size_t need = gemm_w8a16_widened_bytes(p);
           if (need) {
             std::lock_guard<std::mutex> lock(plan->mu);
-            tts_plan::SplitK &sk = plan->split_k[stream];
-            hipError_t e = plan->grow(&sk.widened, &sk.widened_bytes, need);
-            if (e != hipSuccess) return fail(TTS_HIP_ERROR, std::string("hipMalloc(widened weights): ") + hipGetErrorString(e));
-            p.widened = sk.widened;
+            if (const tts_plan::SplitK *sk = plan->room(s, 0, 0, need)) p.widened = sk->widened;
           }
         }
         p.partial = nullptr;
         if (const size_t need = gemm_w8a16_tile_bytes(p)) {
           if (!no_alloc && !is_capturing(s)) {
             std::lock_guard<std::mutex> lock(plan->mu);
-            tts_plan::SplitK &sk = plan->split_k[stream];
-            hipError_t e = plan->grow((void **)&sk.workspace, &sk.workspace_bytes, need);
-            if (e != hipSuccess) return fail(TTS_HIP_ERROR, std::string("hipMalloc(split-K workspace): ") + hipGetErrorString(e));
-            p.partial = sk.workspace;
+            if (const tts_plan::SplitK *sk = plan->room(s, need, 0)) p.partial = sk->workspace;
           } else if (no_alloc && need <= NOALLOC_WORKSPACE_BYTES) {
             p.partial = reinterpret_cast<float *>(noalloc_scratch());
           }
