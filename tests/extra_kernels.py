@@ -1096,6 +1096,32 @@ def attention_fwd(Q, K, V, O, sm_scale, seq, stride_h, stride_s, BM: tl.constexp
 
 
 @triton.jit
+def attention_denominators(Q, K, V, O, R, scale, seq, BM: tl.constexpr, BN: tl.constexpr, D: tl.constexpr):
+    # attention_fwd for one head, and how far the sum of every row's probabilities is from the number of keys, times 2^20, in 16 bits
+    rm = tl.program_id(0) * BM + tl.arange(0, BM)
+    rd = tl.arange(0, D)
+    q = tl.load(Q + rm[:, None] * D + rd[None, :], mask=rm[:, None] < seq, other=0.0)
+    m_i = tl.zeros([BM], dtype=tl.float32) - float("inf")
+    l_i = tl.zeros([BM], dtype=tl.float32)
+    acc = tl.zeros([BM, D], dtype=tl.float32)
+    for start in range(0, seq, BN):
+        rn = start + tl.arange(0, BN)
+        k = tl.load(K + rn[:, None] * D + rd[None, :], mask=rn[:, None] < seq, other=0.0)
+        v = tl.load(V + rn[:, None] * D + rd[None, :], mask=rn[:, None] < seq, other=0.0)
+        qk = tl.dot(q, tl.trans(k)) * scale
+        qk = tl.where(rn[None, :] < seq, qk, -float("inf"))
+        m_new = tl.maximum(m_i, tl.max(qk, axis=1))
+        p = tl.exp(qk - m_new[:, None])
+        alpha = tl.exp(m_i - m_new)
+        l_i = l_i * alpha + tl.sum(p, axis=1)
+        acc = acc * alpha[:, None] + tl.dot(p.to(tl.float16), v)
+        m_i = m_new
+    acc = acc / l_i[:, None]
+    tl.store(O + rm[:, None] * D + rd[None, :], acc.to(tl.float16), mask=rm[:, None] < seq)
+    tl.store(R + rm, ((l_i - seq) * 1048576.0).to(tl.float16), mask=rm < seq)
+
+
+@triton.jit
 def narrow_scaled(x_ptr, y_ptr, n, scale, BLOCK: tl.constexpr):
     # y = (x * scale) narrowed to y's element type: one elementwise pass
     o = tl.program_id(0) * BLOCK + tl.arange(0, BLOCK)

@@ -1166,6 +1166,24 @@ def test_matrix_program_attention_in_slices(dtype, D, BM, BN, H, seq, causal, ma
         check(o2, lse2)
 
 
+@pytest.mark.parametrize("seq", [64, 200, 1500])
+def test_matrix_program_probabilities_of_a_rows_largest_scores_are_one(seq):
+    # every score of a row is that row's number, scaled by a power of two, so that every probability is 1 and every sum the number of keys:
+    # the difference against the maximum comes before the factor log2 e (a sum in which m log2 e is rounded is off by up to 2^-19 of it)
+    import extra_kernels as X
+    D = 64
+    q = torch.zeros(seq, D, dtype=torch.float16, device=DEV)
+    q[:, 0] = 301.0 + 0.25 * torch.arange(seq, device=DEV).remainder(5).half()
+    k = torch.zeros(seq, D, dtype=torch.float16, device=DEV)
+    k[:, 0] = 1.0
+    v = torch.full((seq, D), 0.75, dtype=torch.float16, device=DEV)
+    o, r = torch.zeros(seq, D, dtype=torch.float16, device=DEV), torch.full((seq,), 5.0, dtype=torch.float16, device=DEV)
+    kern = X.attention_denominators[(triton.cdiv(seq, 64),)](q, k, v, o, r, 0.125, seq, BM=64, BN=64, D=D)
+    torch.cuda.synchronize()
+    assert kern.function.last_kernel == "tile_program (hipRTC, matrix layout)"
+    assert (r == 0).all() and (o == 0.75).all(), r.abs().max()
+
+
 @pytest.mark.parametrize("score", [torch.finfo(torch.float32).min, 2.6e38])
 def test_matrix_program_attention_scores_at_the_end_of_fp32(score):
     # every score of a row is the same number (a finite mask on all keys, for one): the result is the mean of the values

@@ -774,6 +774,19 @@ def test_matrix_programs_keep_the_hardware_exponential_to_differences_against_a_
         assert src.startswith("// tts: matrix") and "__builtin_amdgcn_exp2f(" not in body and ("exp2f(" if base2 else "expf(") in body
 
 
+def test_matrix_programs_take_the_difference_before_the_factor_of_their_exponential(native, tmp_path):
+    """Scores held without their scale meet it in an fma with the row's maximum itself; log2 e comes behind the difference."""
+    import extra_kernels as X
+    sig = {**{x: "*fp16" for x in "QKVO"}, "sm_scale": "fp32", **{x: "i32" for x in ("seq", "stride_h", "stride_s")}, **{x: "constexpr" for x in ("BM", "BN", "D")}}
+    src = _generic_source(tmp_path, compile_ttir(X.attention_fwd, sig, {"BM": 64, "BN": 64, "D": 64}))
+    body = src[src.index("void tile_program"):]
+    fma = re.findall(r"= __builtin_fmaf\(\w+\[rb\]\[nb\]\[i\], (f\d+), -(m\d+)\[rb\]\);", body)
+    assert len(fma) == 1 and body.count("__builtin_fmaf(") == 1
+    maximum = re.search(r"  %s\[rb\] = (.*);" % fma[0][1], body).group(1)
+    assert "TTS_LOG2E" not in maximum and re.fullmatch(r"\w+\[rb\]", maximum), maximum
+    assert len(re.findall(r"__builtin_amdgcn_exp2f\(\w+\[rb\]\[nb\]\[i\] \* TTS_LOG2E\)", body)) == 1
+
+
 def test_add_only_loops_keep_the_order_of_their_grid(native, tmp_path):
     """A loop that may run in slices is also launched whole, and then the mark for programs whose stores walk the columns with
     program_id(1) holds for it as for any other."""
