@@ -1122,6 +1122,40 @@ def attention_denominators(Q, K, V, O, R, scale, seq, BM: tl.constexpr, BN: tl.c
 
 
 @triton.jit
+def attention_16_bits(Q, K, V, O, sm_scale, seq, stride_h, stride_s, BM: tl.constexpr, BN: tl.constexpr, D: tl.constexpr, CAUSAL: tl.constexpr):
+    # attention that stores 16-bit results alone, with or without a causal mask: scores held without their scale, the hardware's
+    # exponentials; the grid's first axis holds the query blocks
+    pm = tl.program_id(0)
+    ph = tl.program_id(1)
+    rm = pm * BM + tl.arange(0, BM)
+    rd = tl.arange(0, D)
+    q = tl.load(Q + ph * stride_h + rm[:, None] * stride_s + rd[None, :], mask=rm[:, None] < seq, other=0.0)
+    m_i = tl.zeros([BM], dtype=tl.float32) - float("inf")
+    l_i = tl.zeros([BM], dtype=tl.float32)
+    acc = tl.zeros([BM, D], dtype=tl.float32)
+    last = seq
+    if CAUSAL:
+        last = tl.minimum(seq, (pm + 1) * BM)
+    for start in range(0, last, BN):
+        rn = start + tl.arange(0, BN)
+        k = tl.load(K + ph * stride_h + rn[:, None] * stride_s + rd[None, :], mask=rn[:, None] < seq, other=0.0)
+        v = tl.load(V + ph * stride_h + rn[:, None] * stride_s + rd[None, :], mask=rn[:, None] < seq, other=0.0)
+        qk = tl.dot(q, tl.trans(k)) * sm_scale
+        ok = rn[None, :] < seq
+        if CAUSAL:
+            ok = ok & (rm[:, None] >= rn[None, :])
+        qk = tl.where(ok, qk, -float("inf"))
+        m_new = tl.maximum(m_i, tl.max(qk, axis=1))
+        p = tl.exp(qk - m_new[:, None])
+        alpha = tl.exp(m_i - m_new)
+        l_i = l_i * alpha + tl.sum(p, axis=1)
+        acc = acc * alpha[:, None] + tl.dot(p.to(V.dtype.element_ty), v)
+        m_i = m_new
+    acc = acc / l_i[:, None]
+    tl.store(O + ph * stride_h + rm[:, None] * stride_s + rd[None, :], acc.to(O.dtype.element_ty), mask=rm[:, None] < seq)
+
+
+@triton.jit
 def narrow_scaled(x_ptr, y_ptr, n, scale, BLOCK: tl.constexpr):
     # y = (x * scale) narrowed to y's element type: one elementwise pass
     o = tl.program_id(0) * BLOCK + tl.arange(0, BLOCK)

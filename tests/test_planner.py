@@ -774,6 +774,20 @@ def test_matrix_programs_keep_the_hardware_exponential_to_differences_against_a_
         assert src.startswith("// tts: matrix") and "__builtin_amdgcn_exp2f(" not in body and ("exp2f(" if base2 else "expf(") in body
 
 
+def test_matrix_programs_compare_the_loops_variable_with_an_argument_in_32_bits(native, tmp_path):
+    """`rn < seq` over a block of keys, seq a kernel argument: whether the block lies inside as a whole is one 32-bit compare of the
+    loop's variable with a bound that the loop does not change."""
+    import extra_kernels as X
+    types = {**{x: "*fp16" for x in "QKVO"}, "sm_scale": "fp32", **{x: "i32" for x in ("seq", "stride_h", "stride_s")}, **{x: "constexpr" for x in ("BM", "BN", "D")}}
+    for fn, sig, const in [(X.attention_fwd, types, {"BM": 64, "BN": 64, "D": 64}), (X.attention_16_bits, {**types, "CAUSAL": "constexpr"}, {"BM": 64, "BN": 64, "D": 128, "CAUSAL": True})]:
+        src = _generic_source(tmp_path, compile_ttir(fn, sig, const))
+        body = src[src.index("void tile_program"):]
+        masks = re.findall(r"if \(!\((.*)\)\) \{", body)
+        mask = next(m for m in masks if "p.ival[5]" in m)
+        assert re.search(r"\(int\)\(long long\)\(int\)iv0 < sat32\([^;&]*p\.ival\[5\]\) \+ -63LL\)", mask), mask
+        assert "(long long)(int)iv0 +" not in mask, mask
+
+
 def test_matrix_programs_take_the_difference_before_the_factor_of_their_exponential(native, tmp_path):
     """Scores held without their scale meet it in an fma with the row's maximum itself; log2 e comes behind the difference."""
     import extra_kernels as X

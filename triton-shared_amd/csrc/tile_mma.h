@@ -18,7 +18,7 @@
 //     Blocks that stick out of their tensor or are not 16-byte aligned are staged through registers instead.
 // What the ordinary form of the family spends its time on -- operands, products and every reduced row going through LDS
 // element by element between some twenty barriers per iteration -- does not exist here: causal attention of 32 heads x
-// 4096 x 128 in bf16 (64 x 64 blocks) 12.4 ms -> 165 us, 830 TFLOP/s; 32 x 4096 x 64 in fp16, no mask, 2.7 ms -> 200 us.
+// 4096 x 128 in bf16 (64 x 64 blocks) 12.4 ms -> 170 us, 810 TFLOP/s; 32 x 4096 x 64 in fp16, no mask, 2.7 ms -> 200 us.
 // What bounds it is the chain of an iteration, of which a SIMD holds two at most: the copies' way to LDS (a quarter of it while every
 // wavefront sent its copies at once: with the next blocks' copies among the first product's instructions, fragments read four
 // instructions ahead, the loop's tests in 32 bits and the row sums among the second product's instructions, 8 heads x 4096 x 128
@@ -758,13 +758,26 @@ struct MmaGen : Gen {
     if (b.turns && !a.turns && !a.mixed) return "(int)" + b.v + " > sat32(" + (a.v.empty() ? "0LL" : a.v) + " + " + std::to_string(a.c - slack - b.c) + "LL)";
     return a.text() + " < " + b.text() + " + " + std::to_string(slack) + "LL";
   }
+  bool changes_in_a_loop(int v) const {  // may a scalar's value be another in the next iteration?
+    const SOp *d = def_of(v);
+    if (!d) return true;
+    switch (d->kind) {
+      case SK::Const: case SK::ScalarArg: return false;
+      case SK::FromIndex: return mentions(P.pool, d->expr, EK::IV) || mentions(P.pool, d->expr, EK::Iter) || mentions(P.pool, d->expr, EK::Data);
+      case SK::Map:
+        for (int o : d->operands)
+          if (changes_in_a_loop(o)) return true;
+        return false;
+      default: return true;
+    }
+  }
   bool bounds(int v, int role, Bound *lo, Bound *hi, std::string *given) {
     const Value &V = val(v);
     if (V.dtype != "i32" && V.dtype != "i64") return false;
     auto scalar = [&](int x) {
       *lo = Bound();
       lo->v = "(long long)" + at(x, "0", "0");
-      const bool varies = lo->v.find("iv") != std::string::npos || lo->v.find("it") != std::string::npos;
+      const bool varies = changes_in_a_loop(x);
       lo->turns = varies && V.dtype == "i32";
       lo->mixed = varies && !lo->turns;
       *hi = *lo;
