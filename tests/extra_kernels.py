@@ -775,6 +775,26 @@ def softmax_persistent(out_ptr, in_ptr, in_pitch, out_pitch, n_rows, n_cols, BLO
 
 
 @triton.jit
+def matmul_leaky_any_stride(a_ptr, b_ptr, c_ptr, M, N, K, s_am, s_ak, s_bk, s_cm, slope, BM: tl.constexpr, BN: tl.constexpr, BK: tl.constexpr):
+    # leaky_relu(a @ b) with both of a's strides as arguments
+    rm = tl.program_id(0) * BM + tl.arange(0, BM)
+    rn = tl.program_id(1) * BN + tl.arange(0, BN)
+    rk = tl.arange(0, BK)
+    pa = a_ptr + rm[:, None] * s_am + rk[None, :] * s_ak
+    pb = b_ptr + rk[:, None] * s_bk + rn[None, :]
+    acc = tl.zeros((BM, BN), dtype=tl.float32)
+    for k in range(0, tl.cdiv(K, BK)):
+        left = K - k * BK
+        a = tl.load(pa, mask=(rm[:, None] < M) & (rk[None, :] < left), other=0.0)
+        b = tl.load(pb, mask=(rk[:, None] < left) & (rn[None, :] < N), other=0.0)
+        acc = tl.dot(a, b, acc, input_precision="ieee")
+        pa += BK * s_ak
+        pb += BK * s_bk
+    acc = tl.where(acc >= 0, acc, acc * slope)
+    tl.store(c_ptr + rm[:, None] * s_cm + rn[None, :], acc, mask=(rm[:, None] < M) & (rn[None, :] < N))
+
+
+@triton.jit
 def matmul_leaky(a_ptr, b_ptr, c_ptr, M, N, K, s_am, s_bk, s_cm, slope, BM: tl.constexpr, BN: tl.constexpr, BK: tl.constexpr,
                  ACT: tl.constexpr = 0, bias_ptr=None):
     # a tiled matmul with elementwise ops fused before the narrowing store (the tutorial's ACTIVATION hook).  ACT 0: leaky

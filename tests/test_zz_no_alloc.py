@@ -7,6 +7,7 @@ import pytest
 import torch
 
 from conftest import plan_for
+from test_planner import compile_ttir
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -166,6 +167,43 @@ def test_noalloc_refusal_leaves_a_matmul_with_epilogue_on_its_kernel(native):
     torch.cuda.synchronize()
     assert fresh.last_kernel.startswith("gemm_dma_kernel + epilogue"), fresh.last_kernel
     assert torch.equal(c2.float(), torch.nn.functional.leaky_relu(a2.float() @ b2.float(), 0.5))
+
+
+@pytest.mark.parametrize("first", ["contiguous", "strided"])
+def test_noalloc_launch_of_an_fp32_product_with_an_activation_takes_every_stride(native, first):
+    """leaky_relu(A . B) on fp32 operands runs on the matrix kernel where A's rows are contiguous and on the generic one where they are
+    not: once either has been launched, the launch that may not allocate runs both, in a size of another tiling too."""
+    import triton_shared_amd as tsa
+    import extra_kernels as X
+    tsa.activate()
+    g = torch.Generator(device="cpu").manual_seed(5)
+    stream = torch.cuda.current_stream().cuda_stream
+
+    def case(M, N, K, strided):
+        a = torch.randint(-2, 3, (M, K), generator=g).float()
+        b = torch.randint(-2, 3, (K, N), generator=g).float()
+        held = torch.zeros(M, 3 * K, device=DEV)
+        at = held[:, ::3] if strided else torch.zeros(M, K, device=DEV)
+        at.copy_(a)
+        bd, c = b.to(DEV), torch.full((M, N), 7.0, device=DEV)
+        grid = (-(-M // 64), -(-N // 64), 1)
+        vals = [at.data_ptr(), bd.data_ptr(), c.data_ptr(), M, N, K, at.stride(0), at.stride(1), bd.stride(0), c.stride(0), 0.5]
+        return grid, vals, c, torch.nn.functional.leaky_relu(a @ b, 0.5), (held, at, bd)
+
+    ttir = compile_ttir(X.matmul_leaky_any_stride, {"a_ptr": "*fp32", "b_ptr": "*fp32", "c_ptr": "*fp32", **{x: "i32" for x in ("M", "N", "K", "s_am", "s_ak", "s_bk", "s_cm")}, "slope": "fp32",
+                                                    **{x: "constexpr" for x in ("BM", "BN", "BK")}}, {"BM": 64, "BN": 64, "BK": 32})
+    plan = native.PlanHandle(native.structured_to_plan(native.ttir_to_structured(ttir))[0])
+    grid, vals, c, want, keep = case(100, 130, 96, first == "strided")
+    plan.launch(grid, stream, vals)
+    torch.cuda.synchronize()
+    assert torch.equal(c.cpu(), want)
+    for M, N, K in [(100, 130, 96), (700, 900, 64)]:
+        for strided in (True, False):
+            grid, vals, c, want, keep = case(M, N, K, strided)
+            plan.launch_noalloc(grid, stream, vals)
+            torch.cuda.synchronize()
+            assert torch.equal(c.cpu(), want), (M, strided)
+            assert plan.last_kernel.startswith("tile_program") == (strided or first == "strided"), plan.last_kernel
 
 
 def test_noalloc_launch_of_the_tiled_int8_product_asks_for_no_scratch_it_does_not_use(native):

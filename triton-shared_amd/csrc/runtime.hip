@@ -1053,6 +1053,25 @@ tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, con
         a.gy = gy;
         a.gz = gz;
         std::string why;
+        if (p.is_f32 && !pl.fallback_source.empty()) {
+          // The generic kernel takes every launch of a product on fp32 operands, the matrix kernel most: the first launch compiles both, so
+          // that later ones that may not compile find a kernel whichever they need.
+          bool generic = false;
+          {
+            std::lock_guard<std::mutex> lock(plan->mu);
+            const bool compiled = gemm_epilogue_compiled(p, plan->gemm_rtc);
+            generic = plan->fallback && !compiled && (no_alloc || is_capturing(s));
+            if (!plan->fallback && !no_alloc && !compiled) {
+              const hipError_t ce = rtc_compile(pl.fallback_source, "tile_program", &plan->fallback, &why);
+              if (ce != hipSuccess) return fail(TTS_HIP_ERROR, "tile_program: " + why);
+            }
+          }
+          if (generic) {
+            tts_status st = run_tile_program(&plan->fallback, pl.fallback_source, plan->fallback_traits);
+            if (st != TTS_OK) return st;
+            break;
+          }
+        }
         if (no_alloc) {
           std::lock_guard<std::mutex> lock(plan->mu);
           if (!gemm_epilogue_compiled(p, plan->gemm_rtc)) may_allocate("to compile the matrix product with its fused epilogue");
