@@ -141,6 +141,16 @@ def test_plan_bytes_are_self_contained(native):
         native.PlanHandle(plan_bytes.replace(b"family=row_softmax", b"family=gemm", 1))
 
 
+def test_plans_written_before_their_program_had_a_family_still_load(native):
+    """A family is chosen from a plan's body when it is loaded; what the generic family ran once may have kernels of its own by then."""
+    import extra_kernels as X
+    sig = {"a_ptr": "*fp32", "b_ptr": "*fp32", "c_ptr": "*fp32", **{x: "i32" for x in ("M", "N", "K", "s_am", "s_bk", "s_cm")}, "slope": "fp32", **{x: "constexpr" for x in ("BM", "BN", "BK")}}
+    plan_bytes, _ = native.structured_to_plan(native.ttir_to_structured(compile_ttir(X.matmul_leaky, sig, {"BM": 64, "BN": 64, "BK": 32})))
+    head, body = plan_bytes.split(b"\n", 1)
+    assert head == b"tts.plan 1 family=gemm"
+    assert native.PlanHandle(b"tts.plan 1 family=tile_program\n" + body).family == "gemm"
+
+
 # ------------------------------------------------------------------ refusals
 def test_unsupported_kernels_are_refused(native):
     import extra_kernels as X

@@ -723,7 +723,9 @@ tts_status tts_plan_load(const char *plan_bytes, size_t len, tts_plan **out) {
     h->family = family_name(h->plan.family);
     if (h->plan.family == Family::TileProgram) h->traits = tile_traits(h->plan.source);
     h->fallback_traits = tile_traits(h->plan.fallback_source);
-    if (header.find("family=" + h->family) == std::string::npos) throw Invalid("plan header and plan body disagree on the kernel family");
+    // (a plan written before its program had a family of its own says tile_program, which runs any)
+    if (header.find("family=" + h->family) == std::string::npos && header.find("family=tile_program") == std::string::npos)
+      throw Invalid("plan header and plan body disagree on the kernel family");
     for (auto &t : h->plan.prog.arg_types)
       h->arg_kinds.push_back(t.ptr ? TTS_ARG_PTR : t.is_float() ? TTS_ARG_FLOAT : TTS_ARG_INT);
     *out = h.release();
