@@ -1184,6 +1184,23 @@ def test_matrix_program_probabilities_of_a_rows_largest_scores_are_one(seq):
     assert (r == 0).all() and (o == 0.75).all(), r.abs().max()
 
 
+@pytest.mark.parametrize("seq,pitch", [(64, (1 << 23) + 8), (65, (1 << 23) + 8), (96, (1 << 24) - 8), (64, 1 << 24)])
+def test_matrix_program_attention_on_rows_far_apart(seq, pitch):
+    # pitches around those from which a block no longer goes straight to LDS: a whole block alone, with one of fewer rows behind it
+    import extra_kernels as X
+    D = 64
+    torch.manual_seed(seq)
+    held = [torch.empty((seq - 1) * pitch + D, device=DEV, dtype=torch.float16) for _ in range(4)]
+    q, k, v, o = (h.as_strided((seq, D), (pitch, 1)) for h in held)
+    for x in (q, k, v):
+        x.copy_(torch.randn(seq, D).half())
+    X.attention_fwd[(triton.cdiv(seq, 64), 1)](q, k, v, o, D ** -0.5, seq, 0, pitch, BM=64, BN=64, D=D)
+    torch.cuda.synchronize()
+    q, k, v, o = (x.cpu().double() for x in (q, k, v, o))
+    want = torch.softmax(q @ k.T * D ** -0.5, -1) @ v
+    assert (o - want).abs().max().item() <= 2.0 ** -10 * v.abs().max().item()   # probabilities and results are each rounded once to 16 bits
+
+
 @pytest.mark.parametrize("score", [torch.finfo(torch.float32).min, 2.6e38])
 def test_matrix_program_attention_scores_at_the_end_of_fp32(score):
     # every score of a row is the same number (a finite mask on all keys, for one): the result is the mean of the values

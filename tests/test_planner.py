@@ -798,6 +798,16 @@ def test_matrix_programs_compare_the_loops_variable_with_an_argument_in_32_bits(
         assert "(long long)(int)iv0 +" not in mask, mask
 
 
+def test_matrix_programs_copy_blocks_of_wide_pitch_straight_to_lds(native, tmp_path):
+    """Whole blocks go by direct-to-LDS loads as long as a block's rows lie within 2^31 bytes, last blocks of fewer rows, whose loads go
+    through a buffer resource, within 2^30."""
+    import extra_kernels as X
+    sig = {**{x: "*fp16" for x in "QKVO"}, "sm_scale": "fp32", **{x: "i32" for x in ("seq", "stride_h", "stride_s")}, **{x: "constexpr" for x in ("BM", "BN", "D")}}
+    src = _generic_source(tmp_path, compile_ttir(X.attention_fwd, sig, {"BM": 64, "BN": 64, "D": 64}))
+    assert len(re.findall(r"sp\d+ >= 0 && sp\d+ < %d;  // straight" % (2 ** 30 // 64), src)) >= 2
+    assert len(re.findall(r"if \(st\d+ && sp\d+ >= 64 && sp\d+ < %d\) \{" % (2 ** 29 // 64), src)) >= 2
+
+
 def test_matrix_programs_take_the_difference_before_the_factor_of_their_exponential(native, tmp_path):
     """Scores held without their scale meet it in an fma with the row's maximum itself; log2 e comes behind the difference."""
     import extra_kernels as X

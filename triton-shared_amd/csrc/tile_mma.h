@@ -1144,7 +1144,7 @@ struct MmaGen : Gen {
     const std::string sb = id("sb", im.load), sp = id("sp", im.load), st = id("st", im.load);
     line(sb + " = (const unsigned short *)p.ptr[" + std::to_string(a.base_arg) + "] + (" + ex(a.offsets[0]) + " + " + ex(a.offsets[1]) + ");");
     line(sp + " = " + ex(a.strides[im.outer]) + ";");
-    line(st + " = " + whole(a, im.inner) + " && (((unsigned long long)" + sb + ") & 15) == 0 && (" + sp + " & 7) == 0 && " + sp + " >= 0 && " + sp + " < " + std::to_string((int64_t)(1u << 29) / im.rows) + ";  // straight");
+    line(st + " = " + whole(a, im.inner) + " && (((unsigned long long)" + sb + ") & 15) == 0 && (" + sp + " & 7) == 0 && " + sp + " >= 0 && " + sp + " < " + std::to_string((int64_t)(1u << 30) / im.rows) + ";  // straight");
     line(id("sd", im.load) + " = " + st + " && " + whole(a, im.outer) + ";");
   }
   int stage_turns(const Image &im) const { return (int)((im.bytes() / 1024 + WAVES - 1) / WAVES); }  // direct-to-LDS loads per wavefront (1 KB each)
@@ -1168,7 +1168,7 @@ struct MmaGen : Gen {
     line("} else {");
     indent++;
     line("const int rows = " + extent(a, im.outer) + ", cols = " + extent(a, im.inner) + ";");
-    line("if (" + id("st", im.load) + " && " + sp + " >= " + std::to_string(im.cols) + ") {");
+    line("if (" + id("st", im.load) + " && " + sp + " >= " + std::to_string(im.cols) + " && " + sp + " < " + std::to_string((int64_t)(1u << 29) / im.rows) + ") {");
     indent++;
     line("const u32x4_t block = block_of(" + sb + ", rows > 0 ? (unsigned)((rows - 1) * (int)" + sp + " + " + std::to_string(im.cols) + ") * 2u : 0u);");
     for (int j = 0; j < stage_turns(im); j++) line(stage_copy(im, j, "block", at_bytes));
