@@ -429,7 +429,7 @@ __device__ __forceinline__ float4 load_through(float4 *src) {
 // group's rows; the tails below (the sum over the wavefronts, the hand-over between K slices, the stores) run once per group.
 // ANY: more than four slices, or a last slab of fewer columns (in a kernel of its own: whole slabs in few slices run 0.4 us of 42.4
 // longer on it at the decode shape).
-template <int NW, int DEPTH, int MT, bool ANY>
+template <int NW, int MT, bool ANY>
 __global__ __launch_bounds__(NW * 64) void gemm_w8a16_wide_kernel(GemmW8A16Params p, int first_steps, int other_steps) {
   extern __shared__ float4 w8_lds[];  // [NW][16][64]
   __shared__ int is_last;
@@ -504,20 +504,14 @@ __global__ __launch_bounds__(NW * 64) void gemm_w8a16_wide_kernel(GemmW8A16Param
         acc[m][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, af[m]), __builtin_bit_cast(f16x8, bfrag), acc[m][c], 0, 0, 0);
     }
   };
-  uint4 q[DEPTH][8];
-  uint4 a[DEPTH][MT];
+  // one step in flight per wavefront; two measured 1.2 us slower at the decode shape
+  uint4 q[8];
+  uint4 a[MT];
   int step = step_begin + wave;
-#pragma unroll
-  for (int d = 0; d < DEPTH; d++)
-    if (step + d * NW < step_end) { load_w(step + d * NW, q[d]); load_a(step + d * NW, a[d]); }
-  for (; step < step_end; step += DEPTH * NW) {
-#pragma unroll
-    for (int d = 0; d < DEPTH; d++) {
-      if (step + d * NW < step_end) {
-        consume(q[d], a[d]);
-        if (step + (d + DEPTH) * NW < step_end) { load_w(step + (d + DEPTH) * NW, q[d]); load_a(step + (d + DEPTH) * NW, a[d]); }
-      }
-    }
+  if (step < step_end) { load_w(step, q); load_a(step, a); }
+  for (; step < step_end; step += NW) {
+    consume(q, a);
+    if (step + NW < step_end) { load_w(step + NW, q); load_a(step + NW, a); }
   }
 
   // sum the wavefronts' tiles: entry (c, lane) is rows 4g..4g+3 (of the group) of column n0 + 16j + c
@@ -952,7 +946,7 @@ hipError_t launch_gemm_epilogue(const GemmParams &p, const std::string &epilogue
 }
 
 namespace {
-struct W8Config { int cw, nw, depth, split; };
+struct W8Config { int cw, nw, split; };
 
 // Whether the 16-byte-load kernel takes a shape: N in whole slabs of 256, and from 1024 columns on in groups of 16 (below, a last slab that
 // is half empty is a good part of all).  The 8-byte kernel in 128-column slabs stays ahead where it fills the chip without slices and
@@ -967,17 +961,17 @@ bool w8_wide_shape(const GemmW8A16Params &p) {
 
 // The shape decides the kernel: 256-column slabs with 16-byte weight loads when N and the
 // weight pitch allow, split over K so that about one workgroup lands on each CU.
-// TTS_W8=cw,nw,depth,split overrides the choice (tuning aid).
+// TTS_W8=cw,nw,split overrides the choice (tuning aid).
 W8Config w8_config(const GemmW8A16Params &p) {
   const int64_t steps = (p.K + 31) / 32;
-  W8Config c{8, 16, 2, 1};
-  if (w8_wide_shape(p)) c = W8Config{16, 8, 1, 1};
+  W8Config c{8, 16, 1};
+  if (w8_wide_shape(p)) c = W8Config{16, 8, 1};
   static const char *env = getenv("TTS_W8");
   int want_split = 0;
   if (env) {
-    int cw = 0, nw = 0, depth = 0;
-    if (sscanf(env, "%d,%d,%d,%d", &cw, &nw, &depth, &want_split) >= 3 && (cw == 8 || (cw == 16 && c.cw == 16))) {
-      c.cw = cw; c.nw = nw; c.depth = depth;
+    int cw = 0, nw = 0;
+    if (sscanf(env, "%d,%d,%d", &cw, &nw, &want_split) >= 2 && (cw == 8 || (cw == 16 && c.cw == 16))) {
+      c.cw = cw; c.nw = nw;
     }
   }
   const int64_t slabs = (p.N + 16 * c.cw - 1) / (16 * c.cw);
@@ -1006,14 +1000,14 @@ void w8_launch(const GemmW8A16Params &p, int steps_per_slice, hipStream_t s) {
   hipLaunchKernelGGL((gemm_w8a16_kernel<NW, DEPTH, FAST, 8>), grid, dim3(NW * 64), 0, s, p, steps_per_slice);
 }
 
-template <int NW, int DEPTH, int MT, bool ANY>
+template <int NW, int MT, bool ANY>
 hipError_t w8_launch_wide(const GemmW8A16Params &p, int first_steps, int other_steps, hipStream_t s) {
   constexpr size_t lds = (size_t)NW * 16 * 64 * sizeof(float4);
-  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_w8a16_wide_kernel<NW, DEPTH, MT, ANY>),
+  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_w8a16_wide_kernel<NW, MT, ANY>),
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (attr != hipSuccess) return attr;
   dim3 grid((unsigned)((p.N + W8_COLS_WIDE - 1) / W8_COLS_WIDE), p.split);
-  hipLaunchKernelGGL((gemm_w8a16_wide_kernel<NW, DEPTH, MT, ANY>), grid, dim3(NW * 64), lds, s, p, first_steps, other_steps);
+  hipLaunchKernelGGL((gemm_w8a16_wide_kernel<NW, MT, ANY>), grid, dim3(NW * 64), lds, s, p, first_steps, other_steps);
   return hipGetLastError();
 }
 }  // namespace
@@ -1120,7 +1114,6 @@ static bool w8_wide(const GemmW8A16Params &p) {
 }
 
 static hipError_t launch_gemm_w8a16_rows(const GemmW8A16Params &p, hipStream_t s, const char **name) {
-  W8Config c = w8_config(p);
   const int steps = (int)((p.K + 31) / 32);
   const int sps = (steps + p.split - 1) / p.split;
   const bool fast = w8_fast(p);
@@ -1135,10 +1128,9 @@ static hipError_t launch_gemm_w8a16_rows(const GemmW8A16Params &p, hipStream_t s
       const int take = (bias + p.split - 2) / (p.split - 1);  // per other slice
       if (sps - take >= 8 && sps * p.split == steps) { first = sps + take * (p.split - 1); other = sps - take; }
     }
-    // one step in flight per wavefront; two measured 1.2 us slower at the decode shape
     const bool any = p.split > 4 || p.N % W8_COLS_WIDE != 0;
-    if (p.M > 16) return any ? w8_launch_wide<8, 1, 2, true>(p, first, other, s) : w8_launch_wide<8, 1, 2, false>(p, first, other, s);
-    return any ? w8_launch_wide<8, 1, 1, true>(p, first, other, s) : w8_launch_wide<8, 1, 1, false>(p, first, other, s);
+    if (p.M > 16) return any ? w8_launch_wide<8, 2, true>(p, first, other, s) : w8_launch_wide<8, 2, false>(p, first, other, s);
+    return any ? w8_launch_wide<8, 1, true>(p, first, other, s) : w8_launch_wide<8, 1, false>(p, first, other, s);
   }
   *name = "gemm_w8a16_kernel";
   if (!fast) w8_launch<W8_WAVES, 2, false>(p, sps, s);
