@@ -96,6 +96,10 @@ tts_status tts_launch_noalloc(tts_plan *plan, int grid_x, int grid_y, int grid_z
 
 /* Name of the device kernel the last tts_launch on this plan used (for profiles). */
 const char *tts_plan_last_kernel(const tts_plan *plan);
+/* Into how many slices (workgroups per program or tile) the last tts_launch on this plan dealt a program's loop, or the K of a
+ * product; 1: none.  *meet (may be NULL): 1 if the slices met in that kernel, 0 if a second kernel added them.  For tests.  (Of the
+ * int8-weight product tts_plan_describe_launch tells.) */
+int tts_plan_last_slices(const tts_plan *plan, int *meet);
 
 #ifdef __cplusplus
 }

@@ -597,6 +597,8 @@ def test_gemm_slices_that_meet_in_the_kernel(K, M, N, Kd, at, bt, dtype):
         with torch.cuda.stream(streams[i % 2]):
             k = run()
             assert k.function.last_kernel == "gemm_dma_kernel<128x128>, K slices", k.function.last_kernel
+            n, met = k.function.last_slices
+            assert n > 1 and met == (M not in (770, 136, 520)), (n, met)
         check()
     said = k.function.describe_launch((triton.cdiv(M, 128) * triton.cdiv(N, 128), 1, 1), [0, 0, 0, M, N, Kd] + [x for x in (a.stride(0), a.stride(1), b.stride(0), b.stride(1), N + 8, 1) if x != 1])
     assert said["meet"] == str(int(M not in (770, 136, 520))) and int(said["slices"]) > 1, said
@@ -604,6 +606,7 @@ def test_gemm_slices_that_meet_in_the_kernel(K, M, N, Kd, at, bt, dtype):
     torch.cuda.synchronize()
     with torch.cuda.graph(graph, stream=streams[0]):
         run()
+    assert k.function.last_slices[0] > 1 and not k.function.last_slices[1]
     for _ in range(3):
         graph.replay()
         check()
@@ -1129,6 +1132,7 @@ def test_matrix_program_attention_in_slices(dtype, D, BM, BN, H, seq, causal, ma
     kern = launch(o, lse)
     torch.cuda.synchronize()
     assert kern.function.last_kernel == "tile_program (hipRTC, matrix layout)"
+    assert kern.function.last_slices[0] > 1 and kern.function.last_slices[1]
 
     def check(o, lse):
         s = torch.matmul(q.cpu().double(), k.cpu().double().transpose(1, 2)) * D ** -0.5 + b.cpu().double()
@@ -1158,12 +1162,64 @@ def test_matrix_program_attention_in_slices(dtype, D, BM, BN, H, seq, causal, ma
     torch.cuda.synchronize()
     with torch.cuda.graph(graph, stream=streams[0]):
         launch(o2, lse2)
+    assert kern.function.last_slices == (1, False)
     for turn in range(2):
         v.copy_(torch.randn(H, seq, D, device=DEV).to(dtype))
         torch.cuda.synchronize()
         graph.replay()
         torch.cuda.synchronize()
         check(o2, lse2)
+
+
+@pytest.mark.parametrize("dtype,D,BM,BN,H,seq,causal", [
+    (torch.bfloat16, 128, 64, 64, 2, 2100, True), (torch.float16, 64, 128, 64, 1, 1500, True), (torch.bfloat16, 64, 64, 32, 3, 1000, True),
+    (torch.float16, 128, 32, 64, 1, 1025, True), (torch.float16, 32, 32, 32, 2, 900, False), (torch.bfloat16, 256, 64, 32, 1, 700, True)])
+def test_matrix_program_attention_of_16_bit_results_in_slices(dtype, D, BM, BN, H, seq, causal):
+    # the same where 16-bit results alone are stored: scores held without their scale, the hardware's exponentials in the loop and
+    # where the slices meet; two and four programs in a workgroup, rows masked as a whole in later slices (BM > BN), ragged last blocks
+    import extra_kernels as X
+    torch.manual_seed(seq + D)
+    q, k, v = (torch.randn(H, seq, D, device=DEV).to(dtype) for _ in range(3))
+    outs = lambda: torch.full((H + 1, seq, D), 3.0, device=DEV, dtype=dtype)
+    launch = lambda o: X.attention_16_bits[(triton.cdiv(seq, BM), H)](q, k, v, o, D ** -0.5, seq, seq * D, D, BM=BM, BN=BN, D=D, CAUSAL=causal)
+
+    def check(o):
+        s = torch.matmul(q.cpu().double(), k.cpu().double().transpose(1, 2)) * D ** -0.5
+        if causal:
+            s.masked_fill_(torch.triu(torch.ones(seq, seq, dtype=torch.bool), 1), -float("inf"))
+        want = torch.matmul(torch.softmax(s, -1), v.cpu().double())
+        # as in test_matrix_program_attention: probabilities and results rounded once to 16 bits
+        ulp = 2.0 ** -10 if dtype == torch.float16 else 2.0 ** -7
+        assert (o[:H].cpu().double() - want).abs().max().item() <= ulp * v.abs().max().item() and (o[H] == 3.0).all()
+
+    o = outs()
+    kern = launch(o)
+    torch.cuda.synchronize()
+    n, met = kern.function.last_slices
+    assert kern.function.last_kernel == "tile_program (hipRTC, matrix layout)" and n > 1 and met, n
+    check(o)
+    streams, kept = [torch.cuda.Stream() for _ in range(2)], []
+    torch.cuda.synchronize()
+    for turn in range(6):
+        with torch.cuda.stream(streams[turn % 2]):
+            kept.append(outs())
+            launch(kept[-1])
+    torch.cuda.synchronize()
+    assert all(torch.equal(a, o) for a in kept)
+    graph, o2 = torch.cuda.CUDAGraph(), outs()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=streams[0]):
+        launch(o2)
+    assert kern.function.last_slices == (1, False)
+    for turn in range(3):
+        v.copy_(torch.randn(H, seq, D, device=DEV).to(dtype))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        check(o2)
+        launch(o)   # (in slices, beside what was recorded)
+        torch.cuda.synchronize()
+        check(o)
 
 
 @pytest.mark.parametrize("seq", [64, 200, 1500])

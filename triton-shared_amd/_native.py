@@ -58,6 +58,7 @@ def lib():
     for name in ("tts_plan_kernel_name", "tts_plan_family", "tts_plan_signature", "tts_plan_last_kernel"):
         getattr(L, name).argtypes = [ctypes.c_void_p]
         getattr(L, name).restype = ctypes.c_char_p
+    L.tts_plan_last_slices.argtypes = [ctypes.c_void_p, ctypes.POINTER(ctypes.c_int)]
     L.tts_plan_num_args.argtypes = [ctypes.c_void_p]
     L.tts_plan_arg_kind.argtypes = [ctypes.c_void_p, ctypes.c_int]
     L.tts_plan_describe_launch.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_int,
@@ -214,3 +215,10 @@ class PlanHandle:
     @property
     def last_kernel(self):
         return lib().tts_plan_last_kernel(self._h).decode()
+
+    @property
+    def last_slices(self):
+        """(slices of the last launch, 1: none; whether they met in its kernel)"""
+        meet = ctypes.c_int(0)
+        n = lib().tts_plan_last_slices(self._h, ctypes.byref(meet))
+        return n, bool(meet.value)

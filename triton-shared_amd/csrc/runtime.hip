@@ -118,6 +118,7 @@ struct tts_plan {
   std::list<std::string> lru;
   std::mutex mu;
   const char *last_kernel = "";
+  int last_slices = 1, last_meet = 0;
   // Split-K partial sums and arrival counters (device memory, owned by the plan), one set per stream the plan has been
   // launched on: launches on one stream run one after the other, launches on different streams may overlap and must
   // not share them.  Counters are zero between launches.
@@ -742,6 +743,10 @@ int tts_plan_arg_kind(const tts_plan *plan, int i) {
   return i >= 0 && i < (int)plan->arg_kinds.size() ? plan->arg_kinds[i] : -1;
 }
 const char *tts_plan_last_kernel(const tts_plan *plan) { return plan->last_kernel; }
+int tts_plan_last_slices(const tts_plan *plan, int *meet) {
+  if (meet) *meet = plan->last_meet;
+  return plan->last_slices;
+}
 
 tts_status tts_plan_describe_launch(tts_plan *plan, int gx, int gy, int gz, const tts_arg *args, int n, char **out) {
   if (!plan || !out || (n > 0 && !args)) return fail(TTS_INVALID, "null argument");
@@ -816,6 +821,7 @@ tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, con
     hipStream_t s = (hipStream_t)stream;
     hipError_t err = hipSuccess;
     const char *kname = "";
+    int slices = 1, meet = 0;
     // one workgroup of 256 threads per Triton program, on the kernel generated for the program (compiled at its first use)
     auto run_tile_program = [&](RtcModule **slot, const std::string &source, const TileTraits &traits) -> tts_status {
       struct TileArgs { void *ptr[TILE_MAX_ARGS]; long long ival[TILE_MAX_ARGS]; double fval[TILE_MAX_ARGS]; int swap_xy, lgx, lgy, lgz; } a{};
@@ -864,6 +870,8 @@ tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, con
               sa.slices = 1;
             }
           }
+          slices = sa.slices;
+          meet = slices > 1;
           const int64_t all = workgroups * sa.slices, x = std::min<int64_t>(all, 1 << 23);
           err = rtc_launch(*slot, (int)x, (int)((all + x - 1) / x), 1, traits.threads, &sa, sizeof sa, s);
           return TTS_OK;
@@ -892,6 +900,8 @@ tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, con
             sa.slices = 1;
           }
         }
+        slices = sa.slices;
+        meet = slices > 1;
         // one slice: the grid as it is, a workgroup per program, its x and y exchanged where the program asks for that (see below)
         const bool whole = sa.slices == 1, swap = whole && traits.swaps_grid && gy > 1 && gx <= 65535;
         if (whole && grid_fits(swap)) {
@@ -924,6 +934,8 @@ tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, con
       tts_status st = run_tile_program(&plan->fallback, pl.fallback_source, plan->fallback_traits);
       if (st != TTS_OK) return st;
       plan->last_kernel = kname;
+      plan->last_slices = slices;
+      plan->last_meet = meet;
       if (err != hipSuccess) return fail(TTS_HIP_ERROR, std::string("kernel launch failed: ") + hipGetErrorString(err));
       return TTS_OK;
     }
@@ -1039,6 +1051,8 @@ tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, con
               }
             }
           }
+          slices = p.split;
+          meet = p.counters != nullptr;
           err = launch_gemm(p, s, &kname, &choice);
           break;
         }
@@ -1090,6 +1104,7 @@ tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, con
             if (const tts_plan::SplitK *sk = plan->room(s, gemm_workspace_bytes(p), 0)) p.partial = sk->workspace;
             else p.split = 1;
           }
+          slices = p.split;
           err = launch_gemm_epilogue(p, pl.source, plan->gemm_rtc, may_compile, a, s, &kname, &why);
         }
         if (err != hipSuccess && !why.empty()) return fail(TTS_HIP_ERROR, "gemm epilogue: " + why);
@@ -1149,6 +1164,8 @@ tts_status launch_impl(tts_plan *plan, int gx, int gy, int gz, void *stream, con
       }
     }
     plan->last_kernel = kname;
+    plan->last_slices = slices;
+    plan->last_meet = meet;
     if (err != hipSuccess) return fail(TTS_HIP_ERROR, std::string("kernel launch failed: ") + hipGetErrorString(err));
     return TTS_OK;
   });
