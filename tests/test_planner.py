@@ -756,7 +756,7 @@ def test_direct_loads_to_lds_stand_behind_their_operands(native, tmp_path):
     texts = {"generated": _generic_source(tmp_path, compile_ttir(X.attention_fwd, sig, {"BM": 64, "BN": 64, "D": 64}))}
     for f in glob.glob(os.path.join(ROOT, "triton-shared_amd", "csrc", "*.h")) + glob.glob(os.path.join(ROOT, "triton-shared_amd", "csrc", "*.hip")):
         texts[os.path.basename(f)] = open(f).read()
-    seen = 0
+    seen, buffered = 0, set()
     for name, text in texts.items():
         for asm in re.findall(r'asm volatile\("([^"]*_load_lds_[^"]*)"', text):
             lines = asm.replace("\\n", "\n").replace("\\t", "").split("\n")
@@ -766,7 +766,16 @@ def test_direct_loads_to_lds_stand_behind_their_operands(native, tmp_path):
             # (beside a matrix instruction: the base is made at the start of the phase, eight of those earlier)
             assert base == "off" or any(l.startswith(("s_mov_b64 %s," % base, "v_mfma")) for l in lines[:at]), (name, asm)
             seen += 1
-    assert seen >= 5
+        # a buffer resource is four scalars, made by vector instructions (v_readfirstlane) as the compiler pleases: the wait between the
+        # write of m0 and the load is theirs, too
+        for asm in re.findall(r'asm volatile\("([^"]*buffer_load_[^"]* lds[^"]*)"', text):
+            lines = asm.replace("\\n", "\n").replace("\\t", "").split("\n")
+            at = next(i for i, l in enumerate(lines) if l.startswith("buffer_load_") and " lds" in l)
+            assert lines[at].split()[-1] == "lds" and lines[0].startswith("s_mov_b32 m0,"), (name, asm)
+            nops = [int(l.split()[1]) + 1 for l in lines[1:at] if l.startswith("s_nop ")]
+            assert sum(nops) >= 5, (name, asm)
+            buffered.add(name)
+    assert seen >= 5 and buffered == {"generated", "tile_mma.h"}, buffered
 
 
 def test_matrix_programs_keep_the_hardware_exponential_to_differences_against_a_maximum(native, tmp_path):
