@@ -968,6 +968,26 @@ def test_w8a16_wide_kernel_slabs_and_slices(K, M, N, Kd):
         assert (c[M] == 7.0).all() and (c[:, N:] == 7.0).all()
 
 
+@pytest.mark.parametrize("M,N,Kd,wide", [(16, 24704, 736, True), (3, 24704, 768, False), (16, 32640, 3040, False), (2, 28800, 3072, True), (5, 32896, 1024, True), (16, 24592, 1024, True), (9, 24656, 2080, True),
+                                         (1, 1152, 4096, True), (16, 1152, 4128, False), (7, 1920, 8192, False), (4, 2176, 8192, True), (16, 1408, 12288, True), (16, 1040, 8192, True), (2, 2064, 4128, True)])
+def test_w8a16_kernels_of_widths_in_part_slabs(K, M, N, Kd, wide):
+    # around the lines between the 16-byte-load kernel and the 8-byte one: few and many slabs, short and long K, widths in
+    # whole slabs of 128 columns and in groups of 16
+    g = torch.Generator().manual_seed(N + Kd)
+    a = torch.zeros(M, Kd).scatter_(1, torch.randint(0, Kd, (M, 500), generator=g), 1.0).half().to(DEV)
+    w = torch.randint(-3, 4, (Kd, N), generator=g, dtype=torch.int8).to(DEV)
+    s = (torch.randint(1, 3, (N,), generator=g) / 4).half().to(DEV)
+    c = torch.full((M + 1, N + 32), 7.0, device=DEV, dtype=torch.float16)
+    want = a.cpu().double() @ (w.cpu().double() * s.cpu().double())   # multiples of 1/4 up to 750 in magnitude: fp32 sums are exact, one rounding to fp16
+    for _ in range(2):
+        c.fill_(7.0)
+        k = K.w8a16_matmul[(triton.cdiv(M, 16), triton.cdiv(N, 128))](a, w, s, c, M, N, Kd, Kd, 1, N, 1, N + 32, 1, BM=16, BN=128, BK=128)
+        torch.cuda.synchronize()
+        assert k.function.last_kernel == ("gemm_w8a16_wide_kernel" if wide else "gemm_w8a16_kernel")
+        assert torch.equal(c[:M, :N].cpu().double(), want.half().double())
+        assert (c[M] == 7.0).all() and (c[:, N:] == 7.0).all()
+
+
 @pytest.mark.parametrize("M,N,Kd", [(33, 2048, 64), (40, 2064, 128), (100, 2304, 1088), (161, 4112, 320), (300, 2048, 2048), (513, 3088, 192), (17, 4096, 2048), (1000, 2560, 576)])
 def test_w8a16_tiled_kernel(K, M, N, Kd):
     # rows around the heights of its tiles, ragged column tiles, one K tile up to many K slices; weights over the whole int8

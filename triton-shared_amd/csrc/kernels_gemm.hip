@@ -949,14 +949,23 @@ namespace {
 struct W8Config { int cw, nw, split; };
 
 // Whether the 16-byte-load kernel takes a shape: N in whole slabs of 256, and from 1024 columns on in groups of 16 (below, a last slab that
-// is half empty is a good part of all).  The 8-byte kernel in 128-column slabs stays ahead where it fills the chip without slices and
-// K is short (us, 8-byte / 16-byte loads: 6 x 26752 x 2944 16.7 / 18.5, 8 x 25472 x 3456 18.7 / 19.8, but 8 x 27520 x 4096 23.9 / 22.8, 16 x 28544 x
-// 8192 45.6 / 39.3), and for few slabs of long K, whose many slices its second kernel adds (14 x 2432 x 5888 13.2 / 13.9, 8 x 1152 x 8192
-// 13.0 / 14.1, but 16 x 2176 x 4096 12.9 / 11.8).
+// is half empty is a good part of all).  Whole slabs of 128 stay on the 8-byte kernel in two ranges where it is ahead, in 1 and in 16 rows, us 8-byte /
+// 16-byte loads with the weights from memory (from cache as far apart), of 378 and 126 sizes measured:
+//   * the 128-column slabs are a workgroup per CU at most and need no slices, K from 768 to below 3072: 28800 columns, K 512 10.3 / 10.2,
+//     768 10.3 / 11.4, 1024 10.6 / 12.9, 2048 15.0 / 16.7, 2560 17.1 / 18.6, 3072 19.8 / 20.5 (16 rows 20.9 / 20.5), 4096 24.4 / 23.8.  In more
+//     slabs than CUs it is behind: 32896 x 2048 25.1 / 17.7;
+//   * K beyond 4096 where a step of 32 rows for each wavefront that the chip's CUs hold, 16, is all there is: 1152 columns x 12288
+//     14.7 / 16.8, 2432 x 5888 12.4 / 14.0, 1920 x 8192 13.2 / 14.7, but two steps for some 1408 x 12288 20.9 / 17.2, 3200 x 5888 18.3 / 14.2, 2432 x 8192
+//     18.6 / 14.9; K = 4096 behind by 2 to 6 % throughout.
+// Other widths would take its form for any shape: 40016 x 2048 46.6 / 22.6, 2544 x 8192 25.8 / 16.2, 1040 x 8192 16.0 / 15.3.
 bool w8_wide_shape(const GemmW8A16Params &p) {
   if (p.K % 32 != 0 || p.lda % 8 != 0 || p.ldw % 16 != 0) return false;
   if (p.N % W8_COLS_WIDE == 0) return true;
-  return p.N % 16 == 0 && p.N >= 1024 && !(p.N >= 192 * W8_COLS && p.K < 4096) && !(p.N < 2560 && p.K > 4096);
+  if (p.N % 16 != 0 || p.N < 1024) return false;
+  if (p.N % W8_COLS != 0) return true;
+  const int64_t slabs = p.N / W8_COLS, steps = p.K / 32;
+  if (slabs >= 192) return slabs > 256 || p.K < 768 || p.K >= 3072;  // (from 192 slabs on it takes no slices: w8_config)
+  return p.K <= 4096 || slabs * steps > 16 * 256;
 }
 
 // The shape decides the kernel: 256-column slabs with 16-byte weight loads when N and the
