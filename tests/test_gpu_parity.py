@@ -1295,8 +1295,8 @@ def test_matrix_program_attention_scores_at_the_end_of_fp32(score):
 
 @pytest.mark.parametrize("scale", [0.0, -0.1, 0.1, 6.0, 2.0 ** -70, 2.0 ** 70])
 def test_matrix_program_attention_scaled_before_its_maximum(scale):
-    # scores held without their scale, and every way out of that: scales that are not positive or out of range, rows whose
-    # maximum is too large for the exponential in one fma (scale 6), a row of equal scores
+    # scores held without their scale, and every way out of that: scales that are not positive, above one (6) or out of
+    # range, whose scores are scaled at once, a row of equal scores
     import extra_kernels as X
     torch.manual_seed(11)
     H, seq, D = 2, 200, 64

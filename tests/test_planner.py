@@ -823,11 +823,9 @@ def test_matrix_programs_take_the_difference_before_the_factor_of_their_exponent
     sig = {**{x: "*fp16" for x in "QKVO"}, "sm_scale": "fp32", **{x: "i32" for x in ("seq", "stride_h", "stride_s")}, **{x: "constexpr" for x in ("BM", "BN", "D")}}
     src = _generic_source(tmp_path, compile_ttir(X.attention_fwd, sig, {"BM": 64, "BN": 64, "D": 64}))
     body = src[src.index("void tile_program"):]
-    fma = re.findall(r"= __builtin_fmaf\(\w+\[rb\]\[nb\]\[i\], (f\d+), -(m\d+)\[rb\]\);", body)
+    fma = re.findall(r"__builtin_amdgcn_exp2f\(__builtin_fmaf\(\w+\[rb\]\[nb\]\[i\], f\d+, -\((\w+)\[rb\]\)\) \* TTS_LOG2E\)", body)
     assert len(fma) == 1 and body.count("__builtin_fmaf(") == 1
-    maximum = re.search(r"  %s\[rb\] = (.*);" % fma[0][1], body).group(1)
-    assert "TTS_LOG2E" not in maximum and re.fullmatch(r"\w+\[rb\]", maximum), maximum
-    assert len(re.findall(r"__builtin_amdgcn_exp2f\(\w+\[rb\]\[nb\]\[i\] \* TTS_LOG2E\)", body)) == 1
+    assert fma[0].startswith("from") and re.search(r"%s\[rb\] = (\w+)\[rb\] == nothing \? 0\.f : \1\[rb\];" % fma[0], body)
 
 
 def test_add_only_loops_keep_the_order_of_their_grid(native, tmp_path):

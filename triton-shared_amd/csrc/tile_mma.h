@@ -646,7 +646,8 @@ struct MmaGen : Gen {
   // Scores that a positive scalar scales before such an exponential are held as the product left them (factor_of), and so are
   // they behind a select that puts -infinity in the place of some: the factor is in the exponential's fma, and a maximum
   // over them is scaled once it is taken (rounding keeps the order, so it is the same maximum).  A scalar outside of [2^-60,
-  // 2^60] -- nothing that scales scores -- is multiplied in at once, and the factor is one.
+  // 1] is multiplied in at once, and the factor is one: one above could take finite scores to infinity, whose difference is not a number, but
+  // not in the fma.
   bool minus_infinity(int v) const {
     const SOp *d = def_of(v);
     while (d && (d->kind == SK::Splat || d->kind == SK::Broadcast)) d = def_of(d->operands.at(0));
@@ -671,7 +672,7 @@ struct MmaGen : Gen {
     if (!scaled(s.result, &x, &by) || !tile_of.count(x) || factor_of.count(x) || !read_by_such_an_exponential(s.result)) return false;
     const std::string n = declare_tile(s.result), f = "f" + std::to_string(s.result);
     line("const float s" + f + " = " + at(by, "0", "0") + ";");
-    line("const bool fits_" + f + " = s" + f + " >= 0x1p-60f && s" + f + " <= 0x1p60f;");
+    line("const bool fits_" + f + " = s" + f + " >= 0x1p-60f && s" + f + " <= 1.0f;");
     line("const float " + f + " = fits_" + f + " ? s" + f + " : 1.0f;");
     tile_loop(s.result, n + "[rb][nb][i] = " + el(x, TILE) + ";");
     line("if (!fits_" + f + ") {");
@@ -684,38 +685,17 @@ struct MmaGen : Gen {
     return true;
   }
   // The same with the difference written where it is read.  It is taken before the factor log2 e, from scores that are held without
-  // their factor as one fma, fma(x, factor, -m), where no row's maximum is infinite or NaN (every wavefront asks: a factor that takes finite
-  // scores to infinity leaves not-a-number behind, which the fma would not).  With both factors in the fma, exp2(fma(x, factor log2 e,
-  // -(m log2 e))), an instruction less a score, m log2 e rounds by up to 2^-19 of a row's probabilities, by another amount in every block
-  // that raises the maximum: rms error of the row sums against 64 bits, largest scores of 26, 6.7e-7 against 9.7e-8 here and with
-  // the scaled score rounded first, of the results 2.2e-7 against 1.3e-7.
+  // their factor as one fma, fma(x, factor, -m).  With both factors in the fma, exp2(fma(x, factor log2 e, -(m log2 e))), an instruction
+  // less a score, m log2 e rounds by up to 2^-19 of a row's probabilities, by another amount in every block that raises the maximum: rms
+  // error of the row sums against 64 bits, largest scores of 26, 6.7e-7 against 9.7e-8 here and with the scaled score rounded
+  // first, of the results 2.2e-7 against 1.3e-7.
   bool emit_exp_of_difference(const SOp &s) {
     int scalar = -1;
     const SOp *d = difference_against_maximum(s, &scalar);
     if (!d) return false;
-    const std::string n = declare_tile(s.result), x = "(" + el(d->operands[0], TILE) + " - " + el(d->operands[1], TILE) + ")";
-    const SOp *b = def_of(d->operands[1]);
-    if (factor_of.count(d->operands[0]) && b && b->kind == SK::Broadcast && val(b->operands[0]).shape.size() == 2 && val(b->operands[0]).shape[1] == 1) {
-      const std::string m = "m" + std::to_string(s.result);
-      line("float " + m + "[" + std::to_string(R) + "];");
-      line("bool finite_" + m + " = true;");
-      row_loop("{");
-      line("  " + m + "[rb] = " + el(d->operands[1], TILE) + ";");
-      line("  finite_" + m + " = finite_" + m + " && fabsf(" + m + "[rb]) < __builtin_inff();");
-      line("}");
-      line("if (!__builtin_amdgcn_ballot_w64(!finite_" + m + ")) {");
-      indent++;
-      tile_loop(s.result, n + "[rb][nb][i] = __builtin_fmaf(" + tile_of[d->operands[0]] + "[rb][nb][i], " + factor_of[d->operands[0]] + ", -" + m + "[rb]);");
-      indent--;
-      line("} else {");
-      indent++;
-      tile_loop(s.result, n + "[rb][nb][i] = " + x + ";");
-      indent--;
-      line("}");
-      tile_loop(s.result, n + "[rb][nb][i] = " + hardware_exp(s, n + "[rb][nb][i]") + ";");
-      tile_of[s.result] = n;
-      return true;
-    }
+    const std::string n = declare_tile(s.result), m = el(d->operands[1], TILE);
+    const std::string x = factor_of.count(d->operands[0]) ? "__builtin_fmaf(" + tile_of[d->operands[0]] + "[rb][nb][i], " + factor_of[d->operands[0]] + ", -(" + m + "))"
+                                                          : "(" + el(d->operands[0], TILE) + " - " + m + ")";
     if (scalar >= 0) {
       line("if (" + at(scalar, "0", "0") + " >= 0.f) {");
       indent++;
