@@ -18,7 +18,7 @@
 //     Blocks that stick out of their tensor or are not 16-byte aligned are staged through registers instead.
 // What the ordinary form of the family spends its time on -- operands, products and every reduced row going through LDS
 // element by element between some twenty barriers per iteration -- does not exist here: causal attention of 32 heads x
-// 4096 x 128 in bf16 (64 x 64 blocks) 12.4 ms -> 170 us, 810 TFLOP/s; 32 x 4096 x 64 in fp16, no mask, 2.7 ms -> 200 us.
+// 4096 x 128 in bf16 (64 x 64 blocks) 12.4 ms -> 170 us, 810 TFLOP/s; 32 x 4096 x 64 in fp16, no mask, 2.7 ms -> 205 us.
 // What bounds it is the chain of an iteration, of which a SIMD holds two at most: the copies' way to LDS (a quarter of it while every
 // wavefront sent its copies at once: with the next blocks' copies among the first product's instructions, fragments read four
 // instructions ahead, the loop's tests in 32 bits and the row sums among the second product's instructions, 8 heads x 4096 x 128

@@ -229,8 +229,8 @@ def block_cumsum(x_ptr, y_ptr, n, BLOCK: tl.constexpr):
 
 @triton.jit
 def matmul_leaky_relu(a_ptr, b_ptr, c_ptr, M, N, K, s_am, s_bk, s_cm, slope, BM: tl.constexpr, BN: tl.constexpr, BK: tl.constexpr):
-    """C = leaky_relu(A @ B): a tiled matmul with an activation fused before the narrowing store.  Not the shape the
-    hand-written MFMA kernels take: it runs on the generic family (operands staged in LDS, 32x32 MFMA blocks)."""
+    """C = leaky_relu(A @ B): a tiled matmul with an activation fused before the narrowing store.  The matrix-product
+    kernels take it with the activation as the functor of their epilogue, compiled at run time."""
     tm = tl.program_id(0)
     tn = tl.program_id(1)
     rm = tm * BM + tl.arange(0, BM)
